@@ -99,6 +99,12 @@ int shk_gate_mul(const void* x, const void* gate, void* out, int dtype, long lon
 int shk_gemm(const void* a, const void* w, const float* bias, void* out, int n, int m, int k,
              int lda, int ldo, int in_dtype, int out_dtype, int accumulate, void* stream);
 
+// The same for float32 with the weights in tiles of 16 rows x 16 k (shk_retile_f32: ceil(m/16) *
+// ceil(k/16) tiles of 1 KiB); the sum's order is shk_gemm's.
+int shk_retile_f32(const void* w, int m, int k, void* wt, void* stream);
+int shk_gemm_f32_tiled_weight(const void* a, const void* wt, const float* bias, void* out, int n, int m, int k, int lda,
+                              int ldo, int accumulate, void* stream);
+
 // wt = the tiled layout of the row-major bfloat16 matrix w[m, k] (see
 // gemm_bf16.hip): ceil(m/16) * ceil(k/32) tiles of 1 KiB.
 int shk_retile_weight(const void* w, int m, int k, void* wt, void* stream);

@@ -65,6 +65,7 @@ const Launcher kLaunchers[] = {
     SHK_LAUNCHER(shk_add_normed_rmsnorm),
     SHK_LAUNCHER(shk_act_mul_rows),
     SHK_LAUNCHER(shk_gemm),
+    SHK_LAUNCHER(shk_gemm_f32_tiled_weight),
     SHK_LAUNCHER(shk_gemm_bf16_tiled_weight),
     SHK_LAUNCHER(shk_rope_kv_store),
     SHK_LAUNCHER(shk_attention),

@@ -1,10 +1,9 @@
 // out[n, m] = a[n, k] @ w[m, k]^T + bias: the matrix products of the model
 // (projections, feed-forward, output matrix).
 //
-// gemm_tiled_kernel is the general kernel: every size, float32 or bfloat16
-// storage, float32 fused-multiply-add accumulation in ascending k for every
-// output element.  It is the whole of the float32 path (no matrix mode of
-// reduced precision is involved) and the fallback of the bfloat16 path.
+// gemm_tiled_kernel is the general kernel of bfloat16 operands: every size, float32
+// fused-multiply-add accumulation in ascending k for every output element; the
+// fallback of the bfloat16 path.  float32 operands go to gemm_f32.hip.
 #include "api.h"
 #include "common.h"
 
@@ -107,6 +106,11 @@ __global__ void __launch_bounds__(256)
   }
 }
 
+// gemm_f32.hip
+void gemm_f32(const float* a, const float* w, bool tiled, const float* bias, float* out, int n, int m, int k, int lda,
+              int ldo, int accumulate, int batch, long long a_batch, long long w_batch, long long out_batch,
+              hipStream_t s);
+
 template <typename TI, typename TO>
 static int launch_tiled(const void* a, const void* w, const float* bias, void* out, int n, int m,
                         int k, int lda, int ldo, int accumulate, hipStream_t s, int batch = 1,
@@ -139,7 +143,8 @@ extern "C" int shk_gemm(const void* a, const void* w, const float* bias, void* o
   SHK_REQUIRE((n + kTM - 1) / kTM <= 65535, "gemm: too many rows (%d)", n);
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (in_dtype == kF32)
-    launch_tiled<float, float>(a, w, bias, out, n, m, k, lda, ldo, accumulate, s);
+    gemm_f32(static_cast<const float*>(a), static_cast<const float*>(w), false, bias, static_cast<float*>(out), n, m, k, lda,
+             ldo, accumulate, 1, 0, 0, 0, s);
   else if (out_dtype == kF32)
     launch_tiled<bf16, float>(a, w, bias, out, n, m, k, lda, ldo, accumulate, s);
   else
@@ -230,7 +235,7 @@ extern "C" int shk_gemm_batched(const void* a, const void* w, void* out, int n, 
                                                           static_cast<bf16*>(out), n, m, k, lda, ldo, a_batch, w_batch,
                                                           out_batch);
   } else if (n <= 2 * kSkinnyRows && dtype == kBF16) {
-    // (float32 keeps one order of summation whatever the number of rows: the tiled kernel's ascending k)
+    // (float32 keeps one order of summation whatever the number of rows: gemm_f32.hip)
     dim3 grid((m + 3) / 4, batch);
     if (out_dtype == kF32)
       gemm_batched_skinny_kernel<bf16, float><<<grid, 256, 0, s>>>(static_cast<const bf16*>(a), static_cast<const bf16*>(w),
@@ -241,7 +246,8 @@ extern "C" int shk_gemm_batched(const void* a, const void* w, void* out, int n, 
                                                                   static_cast<bf16*>(out), n, m, k, lda, ldo, a_batch,
                                                                   w_batch, out_batch);
   } else if (dtype == kF32)
-    launch_tiled<float, float>(a, w, nullptr, out, n, m, k, lda, ldo, 0, s, batch, a_batch, w_batch, out_batch);
+    gemm_f32(static_cast<const float*>(a), static_cast<const float*>(w), false, nullptr, static_cast<float*>(out), n, m, k,
+             lda, ldo, 0, batch, a_batch, w_batch, out_batch, s);
   else if (out_dtype == kF32)
     launch_tiled<bf16, float>(a, w, nullptr, out, n, m, k, lda, ldo, 0, s, batch, a_batch, w_batch, out_batch);
   else

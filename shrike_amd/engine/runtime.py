@@ -1,8 +1,8 @@
 """The runtime a model is loaded into: device, compute dtype, how matrices are
 held, and the choice of kernel for each matrix product.
 
-float32: every product runs in the general float32 kernel (fused multiply-add,
-no matrix mode of reduced precision).  bfloat16: weights are held in the MFMA
+float32: every product runs in the float32 kernel (full float32 arithmetic, one
+order of summation whatever the number of rows), weights in tiles of 16 x 16.  bfloat16: weights are held in the MFMA
 operand layout; products with at most 64 rows stream them once through the
 skinny MFMA kernel, larger ones run the LDS-staged MFMA kernel.  What a mixer
 does between its products is the mixer's own business.
@@ -18,11 +18,11 @@ from ..kernels import ops
 class LinearWeight:
     """A weight matrix [rows, cols] as the kernels want it."""
 
-    __slots__ = ("rows", "cols", "dense", "tiled", "gate_args")
+    __slots__ = ("rows", "cols", "tiled_f32", "tiled", "gate_args")
 
-    def __init__(self, shape, dense: torch.Tensor | None, tiled: torch.Tensor | None, gate_args=None):
+    def __init__(self, shape, tiled_f32: torch.Tensor | None, tiled: torch.Tensor | None, gate_args=None):
         self.rows, self.cols = shape
-        self.dense = dense  # row-major (float32 path)
+        self.tiled_f32 = tiled_f32  # tiles of 16 x 16 (float32 path)
         self.tiled = tiled  # MFMA operand layout (bfloat16 path)
         self.gate_args = gate_args  # (limit, up_shift) on the device, for a gate with constants
 
@@ -39,7 +39,7 @@ class Runtime:
         w = w.contiguous()
         if self.dtype == torch.bfloat16:
             return LinearWeight(w.shape, None, ops.retile_weight(w))
-        return LinearWeight(w.shape, w, None)
+        return LinearWeight(w.shape, ops.retile_f32(w), None)
 
     def gated_weight(self, gate: torch.Tensor, up: torch.Tensor, activation: str = "silu", limit=None,
                      up_shift: float = 0.0):
@@ -76,7 +76,7 @@ class Runtime:
             return
         if activation not in (None, "relu_squared"):
             raise ValueError(f"activation {activation!r} is not built for float32 products")
-        ops.gemm(x, w.dense, out, bias=bias, accumulate=accumulate)
+        ops.gemm_f32_tiled_weight(x, w.tiled_f32, w.rows, w.cols, out, bias=bias, accumulate=accumulate)
         if activation is not None:
             ops.activate(out, out, activation)
 

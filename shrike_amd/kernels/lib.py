@@ -40,6 +40,8 @@ _SIGNATURES = {
     "shk_activate": [_P, _P, _I, c_longlong, _I, _P],
     "shk_gate_mul": [_P, _P, _P, _I, c_longlong, _P],
     "shk_gemm": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P],
+    "shk_retile_f32": [_P, _I, _I, _P, _P],
+    "shk_gemm_f32_tiled_weight": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
     "shk_retile_weight": [_P, _I, _I, _P, _P],
     "shk_interleave_gate_up": [_P, _P, _I, _I, _P, _P],
     "shk_gemm_bf16_tiled_weight": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P],

@@ -343,6 +343,33 @@ def gemm(a, w, out, bias=None, accumulate=False) -> None:
     )
 
 
+def retile_f32(w: torch.Tensor) -> torch.Tensor:
+    """A row-major float32 [m, k] matrix in tiles of 16 rows x 16 k (a flat tensor)."""
+    if w.dim() != 2 or not w.is_contiguous() or w.dtype != torch.float32:
+        raise KernelError("retile_f32: expected a contiguous float32 matrix")
+    m, k = w.shape
+    wt = torch.empty(-(-m // 16) * -(-k // 16) * 256, dtype=torch.float32, device=w.device)
+    check(load().shk_retile_f32(_dev(w, "w"), m, k, _dev(wt, "wt"), _stream()))
+    return wt
+
+
+def gemm_f32_tiled_weight(a, wt, m: int, k: int, out, bias=None, accumulate=False) -> None:
+    """gemm() of float32 tensors with the weights in tiles (retile_f32); the same bits as gemm()."""
+    _rows(a, "gemm_f32_tiled_weight a")
+    _rows(out, "gemm_f32_tiled_weight out")
+    n = a.shape[0]
+    if a.shape[1] != k or out.shape != (n, m):
+        raise KernelError(f"gemm_f32_tiled_weight: a is {tuple(a.shape)}, out {tuple(out.shape)} for a [{m}, {k}] matrix")
+    if wt.numel() != -(-m // 16) * -(-k // 16) * 256 or not wt.is_contiguous():
+        raise KernelError(f"gemm_f32_tiled_weight: the tiled weights do not belong to a [{m}, {k}] matrix")
+    if bias is not None and bias.numel() != m:
+        raise KernelError(f"gemm_f32_tiled_weight: bias has {bias.numel()} elements, m is {m}")
+    check(load().shk_gemm_f32_tiled_weight(
+        _dev(a, "a", torch.float32), _dev(wt, "wt", torch.float32),
+        None if bias is None else _dev(bias, "bias", torch.float32), _dev(out, "out", torch.float32), n, m, k,
+        a.stride(0), out.stride(0), int(bool(accumulate)), _stream()))
+
+
 def tiled_numel(m: int, k: int) -> int:
     """bfloat16 elements of the tiled layout of an [m, k] matrix."""
     return -(-m // 16) * -(-k // 32) * 512

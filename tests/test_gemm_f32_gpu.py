@@ -1,0 +1,60 @@
+"""Float32 products on the matrix units: against float64 at the edges of every tile shape, and the same
+bits for a row whatever shape the number of rows selects, tiled weights or not."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from shrike_amd.kernels import ops
+
+    return ops
+
+
+# k: one element, a step and one more, a segment's edge, many steps a segment; m and n around 16, 32 and 64
+@pytest.mark.parametrize("m, k", [(1, 1), (17, 16), (64, 17), (130, 70), (896, 896), (2052, 257), (333, 4864), (33000, 40)])
+@pytest.mark.parametrize("aligned", [True, False])
+def test_against_float64_and_the_same_bits_for_any_number_of_rows(ops, m, k, aligned):
+    torch.manual_seed(m + k)
+    n_max = 70 if m > 20000 else 1100 if m == 896 else 260
+    wide = torch.randn(n_max, k + 5, device="cuda")
+    a = wide[:, :k] if not aligned else wide[:, :k].contiguous()
+    w, bias = torch.randn(m, k, device="cuda"), torch.randn(m, device="cuda")
+    wt = ops.retile_f32(w)
+    full = None
+    for n in [n_max, 1, 2, 15, 16, 17, 31, 33, 64, 65, 129]:
+        if n > n_max:
+            continue
+        rows, tiled = torch.full((n, m + 3), 7.0, device="cuda"), torch.full((n, m), 7.0, device="cuda")
+        ops.gemm(a[:n], w, rows[:, :m], bias=bias)
+        ops.gemm_f32_tiled_weight(a[:n], wt, m, k, tiled, bias=bias)
+        assert bool((rows[:, m:] == 7.0).all())
+        assert torch.equal(rows[:, :m], tiled)
+        if full is None:
+            full = tiled
+            exact = a.double() @ w.double().t() + bias.double()
+            # at most k / 16 + 40 roundings on the way of a product into its sum, each of half an ulp of a partial
+            # sum that the sum of the products' sizes bounds
+            size = a.double().abs() @ w.double().abs().t() + bias.double().abs()
+            assert bool(((tiled.double() - exact).abs() <= (k / 16 + 40) * 2.0**-24 * size).all())
+        assert torch.equal(tiled, full[:n])
+        again = tiled.clone()
+        ops.gemm_f32_tiled_weight(a[:n], wt, m, k, again, accumulate=True)
+        plain = torch.empty_like(tiled)
+        ops.gemm_f32_tiled_weight(a[:n], wt, m, k, plain)
+        assert torch.equal(again, plain + tiled)
+
+
+def test_what_does_not_fit_is_refused(ops):
+    from shrike_amd.kernels import KernelError
+
+    a, wt = torch.zeros(2, 8, device="cuda"), ops.retile_f32(torch.zeros(4, 8, device="cuda"))
+    with pytest.raises(KernelError, match="tiled weights"):
+        ops.gemm_f32_tiled_weight(a, wt, 17, 8, torch.zeros(2, 17, device="cuda"))
+    with pytest.raises(KernelError):
+        ops.gemm_f32_tiled_weight(a, wt, 4, 8, torch.zeros(2, 5, device="cuda"))
+    with pytest.raises(KernelError):
+        ops.retile_f32(torch.zeros(4, 8, device="cuda", dtype=torch.bfloat16))
