@@ -1,6 +1,7 @@
 // Causal grouped-query attention over paged key/value caches.
 //
-// attention_generic_kernel: one workgroup per (query token, query head), for
+// attention_generic_kernel: what the kernels on the matrix units (attention_mfma.hip,
+// attention_f32.hip) do not take; one workgroup per (query token, query head), for
 // any head size up to 256, any page size, any number of heads and groups,
 // float32 or bfloat16 storage.  Scores, softmax and the weighted sum of values
 // are float32.  It walks the keys of the token's sequence in tiles of 256
@@ -12,6 +13,7 @@
 // term per head, exp(sinks[head]), that has no key and no value.  A learned bias by
 // distance, dist_bias[head][min(i - j, rows - 1)], may be added to the (capped) score.
 #include "api.h"
+#include "attention_f32.h"
 #include "common.h"
 
 namespace shk {
@@ -126,7 +128,8 @@ extern "C" int shk_attention(const void* q, int q_stride, void* out, int dtype, 
                              const int32_t* token_seq, const int32_t* tables, int table_stride,
                              int num_seqs, const void* k_pool, const void* v_pool, int page_size,
                              int num_pages, int window, int chunk, float scale, int v_dim, float softcap,
-                             const float* sinks, const float* dist_bias, int bias_rows, void* stream) {
+                             const float* sinks, const float* dist_bias, int bias_rows, float* partial, int splits,
+                             void* stream) {
   SHK_REQUIRE(dtype == kF32 || dtype == kBF16, "attention: unknown dtype %d", dtype);
   SHK_REQUIRE(!dist_bias || bias_rows > 0, "attention: a distance bias needs a table of at least one row");
   SHK_REQUIRE(n >= 0 && heads > 0 && kv_heads > 0 && heads % kv_heads == 0,
@@ -146,9 +149,17 @@ extern "C" int shk_attention(const void* q, int q_stride, void* out, int dtype, 
   SHK_REQUIRE(n <= 65535, "attention: at most 65535 tokens a call, got %d", n);
   SHK_REQUIRE(q && out && positions && token_seq && tables && k_pool && v_pool,
               "attention: null pointer");
+  SHK_REQUIRE(splits >= 1 && splits <= 65535, "attention: splits %d is outside 1..65535", splits);
   hipStream_t s = static_cast<hipStream_t>(stream);
   dim3 grid(heads, n);
-  if (dtype == kF32)
+  if (dtype == kF32 && attention_f32_takes(head_dim, v_dim, page_size, k_pool, v_pool)) {
+    const long long blocks = (static_cast<long long>(table_stride) * page_size + kKeyBlock - 1) / kKeyBlock;
+    attention_f32({static_cast<const float*>(q), static_cast<const float*>(k_pool), static_cast<const float*>(v_pool), sinks,
+                   dist_bias, static_cast<float*>(out), partial, positions, token_seq, tables, q_stride, heads, kv_heads,
+                   head_dim, v_dim, table_stride, page_size, num_pages, window, chunk, bias_rows, static_cast<int>(blocks),
+                   scale, softcap},
+                  n, partial ? splits : 1, s);
+  } else if (dtype == kF32)
     attention_generic_kernel<float><<<grid, kAttnThreads, 0, s>>>(
         static_cast<const float*>(q), q_stride, static_cast<float*>(out), heads, kv_heads, head_dim, v_dim,
         positions, token_seq, tables, table_stride, static_cast<const float*>(k_pool),

@@ -1,0 +1,261 @@
+// Causal grouped-query attention over the paged cache in float32 on the matrix units
+// (v_mfma_f32_16x16x4_f32): one workgroup of four wavefronts per (token, key/value head, 16 of its
+// query heads), the heads being the columns of both products, S^T = K Q^T and O^T = V^T P^T.
+//
+// A float32 result has the same bits however a prompt is cut, so the order of every sum follows from
+// the key's position alone: keys are taken in blocks of 256 counted from position 0, a wavefront has
+// the same 64 of each; a block has a maximum and sums of its own (the wavefronts' in order), and the
+// blocks are joined in order with a running maximum.  A masked key has weight 0 and values that are
+// read as 0 (its slot may hold anything), which changes no sum, so nothing depends on where a window
+// begins within a block.  Single tokens may have their blocks formed by workgroups of their own
+// (kSplit), whose results attention_f32_join_kernel joins by the same arithmetic.
+//
+// A lane of the first product's result holds four neighbouring keys of one head, which is the second
+// product's operand as it stands: weights never pass through LDS.  What bounds it: a block is 64 + 64
+// instructions of 32 cycles per wavefront (head size 64) and three barriers, about 3 us; the general
+// kernel's one workgroup per query head with one key per thread took 560 us for 14 heads of 64 over
+// 509 tokens, and 50 us for four single tokens at 400 (whole passes: a 509-token prompt of the 0.5B model
+// 18.9 ms then, 6.5 now; a decode step of four requests 2.43 ms, 1.67 now).
+#include "api.h"
+#include "attention_f32.h"
+#include "common.h"
+
+namespace shk {
+
+typedef float af4 __attribute__((ext_vector_type(4)));
+
+constexpr int kBlockWaves = 4, kWaveKeys = kKeyBlock / kBlockWaves;
+
+// (m, l) joins (M, L); e0 and e1 are the factors of what has been summed and of what joins.
+__device__ __forceinline__ void join_block(float& M, float& L, float m, float l, float& e0, float& e1) {
+  const float top = fmaxf(M, m);
+  e0 = M == -INFINITY ? 0.f : expf(M - top);
+  e1 = m == -INFINITY ? 0.f : expf(m - top);
+  L = __fmaf_rn(L, e0, __fmul_rn(l, e1));
+  M = top;
+}
+
+__device__ __forceinline__ float joined(float sum, float e0, float block, float e1) {
+  return __fmaf_rn(sum, e0, __fmul_rn(block, e1));
+}
+
+// the sink joins the denominator alone
+__device__ __forceinline__ float keys_share(float M, float& L, const float* sinks, int head) {
+  if (!sinks) return 1.f;
+  const float sink = sinks[head], top = fmaxf(M, sink), share = expf(M - top);
+  L = L * share + expf(sink - top);
+  return share;
+}
+
+// D: sixteens of the larger of head_dim and v_dim
+template <int D, bool kSplit>
+__global__ void __launch_bounds__(kWave * kBlockWaves) attention_f32_kernel(F32Attention p) {
+  __shared__ af4 sums[kBlockWaves][D][kWave];
+  __shared__ float tops[kBlockWaves][16], weights[kBlockWaves][16];
+  const int lane = threadIdx.x % kWave, i = lane % 16, kg = lane / 16;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int per = p.heads / p.kv_heads, parts = (per + 15) / 16;
+  const int kvh = blockIdx.x / parts, in_group = blockIdx.x % parts * 16 + i;
+  const bool row = in_group < per;
+  const int head = kvh * per + (row ? in_group : 0);
+  const int t = blockIdx.y;
+  const int pos = p.positions[t], lo = first_key(pos, p.window, p.chunk);
+  const int32_t* table = p.tables + static_cast<size_t>(p.token_seq[t]) * p.table_stride;
+  int first = lo / kKeyBlock, last = pos / kKeyBlock, step = 1;
+  if (kSplit) {
+    first += blockIdx.z;
+    step = gridDim.z;
+    if (first > last) return;
+  }
+
+  const float* qr = p.q + static_cast<size_t>(t) * p.q_stride + head * p.head_dim;
+  af4 qv[D];
+#pragma unroll
+  for (int s = 0; s < D; ++s)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int d = 16 * s + 4 * kg + e;
+      const float x = qr[d < p.head_dim ? d : 0];
+      qv[s][e] = row && d < p.head_dim ? x : 0.f;
+    }
+
+  constexpr int kOwn = (D + kBlockWaves - 1) / kBlockWaves;  // tiles of values that this wavefront joins: wave, wave + 4, ..
+  af4 own[kOwn];
+#pragma unroll
+  for (int o = 0; o < kOwn; ++o) own[o] = af4{0.f, 0.f, 0.f, 0.f};
+  float M = -INFINITY, L = 0.f;
+  const int slab = key_slab(p.head_dim), ps = p.page_size;
+  const size_t k_page = static_cast<size_t>(ps) * p.head_dim, v_page = static_cast<size_t>(ps) * p.v_dim;
+  auto page_of = [&](int key) {  // -1 where no key may be read
+    const int page = key >= lo && key <= pos ? table[key / ps] : -1;
+    return page < p.num_pages ? page : -1;
+  };
+
+  for (int b = first; b <= last; b += step) {
+    const int key0 = b * kKeyBlock + wave * kWaveKeys;
+    // scores: this lane loads key key0 + 16 u + i, and gets keys key0 + 16 u + 4 kg + 0..3 of head i
+    af4 s[kWaveKeys / 16];
+    int v_at[kWaveKeys / 16];  // page of the keys whose values this lane loads
+#pragma unroll
+    for (int u = 0; u < kWaveKeys / 16; ++u) {
+      s[u] = af4{0.f, 0.f, 0.f, 0.f};
+      const int key = key0 + 16 * u + i, vkey = key0 + 16 * u + 4 * kg;
+      const int page = max(page_of(key), 0);
+      // (page sizes are multiples of four: the four keys share a page; the first or the last of them is
+      // one that may be read, if any is)
+      v_at[u] = max(page_of(vkey), page_of(min(vkey + 3, pos)));
+      const float* kr = p.k_pool + (static_cast<size_t>(page) * p.kv_heads + kvh) * k_page + static_cast<size_t>(key % ps) * slab;
+      af4 kv[D];
+#pragma unroll
+      for (int x = 0; x < D; ++x) {
+        const int d = 16 * x + 4 * kg;
+        const bool have = d < p.head_dim;
+        const size_t at = have ? static_cast<size_t>(d / slab) * ps * slab + d % slab : 0;
+        kv[x] = *reinterpret_cast<const af4*>(kr + at);
+        if (!have) kv[x] = af4{0.f, 0.f, 0.f, 0.f};
+      }
+#pragma unroll
+      for (int x = 0; x < D; ++x)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[x][e], qv[x][e], s[u], 0, 0, 0);
+    }
+    float top = -INFINITY;
+#pragma unroll
+    for (int u = 0; u < kWaveKeys / 16; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int key = key0 + 16 * u + 4 * kg + e;
+        float x = s[u][e] * p.scale;
+        if (p.softcap > 0.f) x = p.softcap * tanhf(x / p.softcap);
+        const bool have = key >= lo && key <= pos && v_at[u] >= 0;
+        if (p.dist_bias && have) x += p.dist_bias[static_cast<size_t>(head) * p.bias_rows + min(pos - key, p.bias_rows - 1)];
+        s[u][e] = have ? x : -INFINITY;
+        top = fmaxf(top, s[u][e]);
+      }
+    top = fmaxf(top, __shfl_xor(top, 16));
+    top = fmaxf(top, __shfl_xor(top, 32));
+    if (kg == 0) tops[wave][i] = top;
+    __syncthreads();
+    float m = tops[0][i];
+#pragma unroll
+    for (int w = 1; w < kBlockWaves; ++w) m = fmaxf(m, tops[w][i]);
+
+    float l = 0.f;
+    af4 acc[D];
+#pragma unroll
+    for (int x = 0; x < D; ++x) acc[x] = af4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < kWaveKeys / 16; ++u) {
+      const int vkey = key0 + 16 * u + 4 * kg;
+      const float* vr = p.v_pool + (static_cast<size_t>(max(v_at[u], 0)) * p.kv_heads + kvh) * v_page + vkey % ps;
+      af4 vv[D];
+#pragma unroll
+      for (int x = 0; x < D; ++x) {
+        const int d = 16 * x + i;
+        vv[x] = *reinterpret_cast<const af4*>(vr + static_cast<size_t>(d < p.v_dim ? d : 0) * ps);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const bool have = vkey + e >= lo && vkey + e <= pos && v_at[u] >= 0;
+        const float w = have ? expf(s[u][e] - m) : 0.f;
+        l += w;
+        s[u][e] = w;
+#pragma unroll
+        for (int x = 0; x < D; ++x) vv[x][e] = have ? vv[x][e] : 0.f;
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int x = 0; x < D; ++x) acc[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[x][e], s[u][e], acc[x], 0, 0, 0);
+    }
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
+    if (kg == 0) weights[wave][i] = l;
+#pragma unroll
+    for (int x = 0; x < D; ++x) sums[wave][x][lane] = acc[x];
+    __syncthreads();
+    l = weights[0][i];
+#pragma unroll
+    for (int w = 1; w < kBlockWaves; ++w) l += weights[w][i];
+    float e0 = 0.f, e1 = 1.f;
+    if (!kSplit) join_block(M, L, m, l, e0, e1);
+    float* mine = kSplit ? p.partial + ((static_cast<size_t>(t) * p.heads + head) * p.blocks + b) * (p.v_dim + 2) : nullptr;
+    if (kSplit && row && wave == 0 && kg == 0) {
+      mine[p.v_dim] = m;
+      mine[p.v_dim + 1] = l;
+    }
+#pragma unroll
+    for (int o = 0; o < kOwn; ++o) {
+      const int x = wave + o * kBlockWaves;
+      if (x >= D) continue;
+      af4 v = sums[0][x][lane];
+#pragma unroll
+      for (int w = 1; w < kBlockWaves; ++w) v += sums[w][x][lane];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int d = 16 * x + 4 * kg + e;
+        if (!kSplit)
+          own[o][e] = joined(own[o][e], e0, v[e], e1);
+        else if (row && d < p.v_dim)
+          mine[d] = v[e];
+      }
+    }
+    __syncthreads();  // the next block writes tops, weights and sums again
+  }
+  if (kSplit || !row) return;
+  const float share = keys_share(M, L, p.sinks, head);
+#pragma unroll
+  for (int o = 0; o < kOwn; ++o)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int d = 16 * (wave + o * kBlockWaves) + 4 * kg + e;
+      if (d < p.v_dim) p.out[(static_cast<size_t>(t) * p.heads + head) * p.v_dim + d] = own[o][e] * share / L;
+    }
+}
+
+// a workgroup per (head, token), a thread per element of the value
+__global__ void __launch_bounds__(256) attention_f32_join_kernel(F32Attention p) {
+  const int head = blockIdx.x, t = blockIdx.y, d = threadIdx.x;
+  const int pos = p.positions[t], lo = first_key(pos, p.window, p.chunk);
+  if (d >= p.v_dim) return;
+  float M = -INFINITY, L = 0.f, sum = 0.f;
+  for (int b = lo / kKeyBlock; b <= pos / kKeyBlock; ++b) {
+    const float* block = p.partial + ((static_cast<size_t>(t) * p.heads + head) * p.blocks + b) * (p.v_dim + 2);
+    float e0, e1;
+    join_block(M, L, block[p.v_dim], block[p.v_dim + 1], e0, e1);
+    sum = joined(sum, e0, block[d], e1);
+  }
+  const float share = keys_share(M, L, p.sinks, head);
+  p.out[(static_cast<size_t>(t) * p.heads + head) * p.v_dim + d] = sum * share / L;
+}
+
+bool attention_f32_takes(int head_dim, int v_dim, int page_size, const void* k_pool, const void* v_pool) {
+  return head_dim % 4 == 0 && page_size % 4 == 0 && reinterpret_cast<uintptr_t>(k_pool) % 16 == 0 &&
+         reinterpret_cast<uintptr_t>(v_pool) % 16 == 0;
+}
+
+template <int D>
+static void launch(const F32Attention& p, int n, int splits, hipStream_t s) {
+  const int per = p.heads / p.kv_heads;
+  const dim3 grid(p.kv_heads * ((per + 15) / 16), n, splits);
+  if (splits > 1) {
+    attention_f32_kernel<D, true><<<grid, kWave * kBlockWaves, 0, s>>>(p);
+    attention_f32_join_kernel<<<dim3(p.heads, n), (p.v_dim + kWave - 1) / kWave * kWave, 0, s>>>(p);
+  } else {
+    attention_f32_kernel<D, false><<<grid, kWave * kBlockWaves, 0, s>>>(p);
+  }
+}
+
+void attention_f32(const F32Attention& p, int n, int splits, hipStream_t s) {
+  const int d = p.head_dim > p.v_dim ? p.head_dim : p.v_dim;
+  if (d <= 32)
+    launch<2>(p, n, splits, s);
+  else if (d <= 64)
+    launch<4>(p, n, splits, s);
+  else if (d <= 128)
+    launch<8>(p, n, splits, s);
+  else
+    launch<16>(p, n, splits, s);
+}
+
+}  // namespace shk

@@ -547,8 +547,11 @@ def rope_kv_store(qkv, heads, kv_heads, head_dim, rot_dim, inv_freq, positions, 
 
 
 def attention(q, out, heads, kv_heads, head_dim, positions, token_seq, tables, k_pool, v_pool,
-              page_size, window, scale, chunk=None, v_dim=None, softcap=None, sinks=None, dist_bias=None) -> None:
+              page_size, window, scale, chunk=None, v_dim=None, softcap=None, sinks=None, dist_bias=None, partial=None,
+              splits=1) -> None:
     """q: [n, >= heads*head_dim] rows (a view into qkv is fine); out [n, heads*v_dim].
+    partial: float32 scratch of attention_partial_floats() with which float32 attention may form a token's
+    blocks of 256 keys in up to `splits` workgroups (the same bits).
     v_dim: size of a value (None: head_dim); softcap: scores become cap * tanh(score / cap);
     sinks: float32 [heads], one more term exp(sinks[h]) in each head's softmax denominator;
     dist_bias: float32 [heads, rows], dist_bias[h, min(i - j, rows - 1)] joins the (capped) score."""
@@ -561,6 +564,8 @@ def attention(q, out, heads, kv_heads, head_dim, positions, token_seq, tables, k
         raise KernelError(f"attention: sinks must hold one value per head ({heads})")
     _dist_bias(dist_bias, heads, "attention")
     _check_pools("attention", q, tables, k_pool, v_pool, kv_heads, head_dim, page_size, v_dim)
+    if partial is not None and partial.numel() < attention_partial_floats(n, heads, v_dim, tables.shape[1], page_size):
+        raise KernelError("attention: the scratch for the blocks' results is too small")
     check(
         load().shk_attention(
             _dev(q, "q"), q.stride(0), _dev(out, "out"), dtype_code(q.dtype), n, heads, kv_heads,
@@ -570,9 +575,18 @@ def attention(q, out, heads, kv_heads, head_dim, positions, token_seq, tables, k
             page_size, k_pool.shape[0], int(window or 0), int(chunk or 0), float(scale), v_dim,
             float(softcap or 0.0), None if sinks is None else _dev(sinks, "sinks", torch.float32),
             None if dist_bias is None else _dev(dist_bias, "dist_bias", torch.float32),
-            0 if dist_bias is None else dist_bias.shape[1], _stream(),
+            0 if dist_bias is None else dist_bias.shape[1],
+            None if partial is None else _dev(partial, "partial", torch.float32), int(splits), _stream(),
         )
     )
+
+
+ATTENTION_KEY_BLOCK = 256  # keys whose maximum and sums float32 attention forms together
+
+
+def attention_partial_floats(n: int, heads: int, v_dim: int, table_width: int, page_size: int) -> int:
+    """Scratch for attention(partial=...): one result per token, head and block of keys."""
+    return n * heads * -(-table_width * page_size // ATTENTION_KEY_BLOCK) * (v_dim + 2)
 
 
 def _dist_bias_args(dist_bias, heads, who):

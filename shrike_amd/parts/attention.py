@@ -466,10 +466,19 @@ class PagedAttention(Mixer):
                                   sink=getattr(s, "fixed_sink", None), nshare=plan.nsplit)
             return
         if not plan.mfma:
+            partial, splits = None, 1
+            if self.dtype == torch.float32 and ctx.num_decode == ctx.num_tokens:
+                # few single tokens: their blocks of keys side by side (as many as the tables are wide: what a
+                # replayed launch must serve; the result is the same bits)
+                blocks = -(-tables.shape[1] * cache.page_size // ops.ATTENTION_KEY_BLOCK)
+                if blocks > 1 and ctx.num_tokens * hkv < 2 * compute_units():
+                    splits = min(blocks, MAX_KEY_SPLITS)
+                    floats = ops.attention_partial_floats(ctx.num_tokens, h, self.value_dim, tables.shape[1], cache.page_size)
+                    partial = ctx.buffer("attn_f32_partial", (floats,), torch.float32)
             ops.attention(q, out, h, hkv, d, ctx.positions, ctx.token_seq, tables, cache.pools["k"],
                           cache.pools["v"], cache.page_size, s.window, s.scale, chunk=s.chunk,
                           v_dim=self.value_dim, softcap=getattr(s, "softcap", None), sinks=self.sinks,
-                          dist_bias=self.dist_bias)
+                          dist_bias=self.dist_bias, partial=partial, splits=splits)
             return
         if ctx.num_decode:
             partial = ctx.buffer("attn_partial", (ctx.num_decode * h * plan.nsplit * (d + 2),),
