@@ -522,10 +522,13 @@ int shk_moe_experts(const void* x, const int32_t* chosen, const float* weights, 
 // expert) pairs that chose it (built on the device).  width and ff in multiples of 8; scratch:
 // shk_moe_grouped_scratch_bytes(...) bytes, 16-byte aligned.
 long long shk_moe_grouped_scratch_bytes(int n, int width, int experts, int top);
+// tiled: w_gate, w_up and w_down are the stacked matrices as shk_retile_weight lays them out (width and ff in
+// multiples of 64).
 int shk_moe_experts_grouped(const void* x, const int32_t* chosen, const float* weights, const void* w_gate,
                             const void* w_up, const void* w_down, const void* add, const float* add_gate,
                             int gate_ld, void* act_buf, void* out, void* scratch, int n, int width, int ff, int experts, int top,
-                            int identity, int act, float limit, float shift, void* stream);
+                            int identity, int act, float limit, float shift, int tiled,
+                            void* stream);
 
 // out = a_pos z^2 + z / 2 where z > 0, a_neg (exp(z) - 1 - z) + z / 2 elsewhere; elementwise.
 int shk_xielu(const void* x, void* out, int dtype, long long numel, float a_pos, float a_neg, void* stream);

@@ -284,11 +284,14 @@ __global__ void __launch_bounds__(256)
 // The two products for lists of few pairs, where what counts is how fast the experts' matrices stream: a
 // workgroup takes 32 pairs and 32 weight rows (of both matrices where there is a gate), its four wavefronts
 // a quarter of k each, so that even one token's experts are read by hundreds of wavefronts; a lane asks for
-// four steps' operands at once.  The quarters' sums meet in LDS and are added in order.
+// four steps' operands at once.  The quarters' sums meet in LDS and are added in order.  The weights' stream is
+// what bounds it: with row-major weights (16 pieces of 64 bytes a load) eight tokens' experts (two of eight, 4736
+// features of width 3584) took 99 and 56 us, in tiles 83 and 45 (680 MB: 113 us at the memory's rate).
 constexpr int kQuarters = 4;
 
-// acc[m][a][b] += W_m[row b] . x[pair a] over this wavefront's quarter of k
-template <int MATRICES>
+// acc[m][a][b] += W_m[row b] . x[pair a] over this wavefront's quarter of k.  TILED: the weights lie in tiles of
+// 16 rows x 32 k (512 elements; wr points at the lane's 8 of the row block's first tile), one run of 1 KiB a load
+template <int MATRICES, bool TILED>
 __device__ __forceinline__ void moe_quarter(const bf16* const (&xr)[2], const bool (&have_pair)[2],
                                             const bf16* const (&wr)[MATRICES][2], int k, int quarter, int kg,
                                             mf32x4 (&acc)[MATRICES][2][2]) {
@@ -306,7 +309,7 @@ __device__ __forceinline__ void moe_quarter(const bf16* const (&xr)[2], const bo
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
           wv[u][m][b] = make_uint4(0, 0, 0, 0);
-          if (have) wv[u][m][b] = *reinterpret_cast<const uint4*>(wr[m][b] + kk);
+          if (have) wv[u][m][b] = *reinterpret_cast<const uint4*>(wr[m][b] + (TILED ? kk * 16 : kk));
         }
 #pragma unroll
       for (int a = 0; a < 2; ++a) {
@@ -352,7 +355,7 @@ __device__ __forceinline__ void moe_join_quarters(const mf32x4 (&acc)[MATRICES][
 
 // act[pair, f] = act(W_gate_e[f] . x_t) * (W_up_e[f] . x_t) for the pairs of expert e's list.  SINGLE: experts
 // without a gate, the one product is both factors.
-template <bool SINGLE>
+template <bool SINGLE, bool TILED>
 __global__ void __launch_bounds__(256)
     moe_gate_up_mfma_kernel(const bf16* __restrict__ x, const int32_t* __restrict__ order,
                             const int32_t* __restrict__ counts, const bf16* __restrict__ wg,
@@ -378,9 +381,11 @@ __global__ void __launch_bounds__(256)
     have[a] = pair[a] >= 0;
     const int t = have[a] ? min(pair[a] / top, n - 1) : 0;
     xr[a] = x + static_cast<size_t>(t) * width + kg * 8;
-    const size_t f = static_cast<size_t>(e) * ff + min(f0 + a * 16 + i, ff - 1);
-    wr[0][a] = wg + f * width + kg * 8;
-    if (!SINGLE) wr[M - 1][a] = wu + f * width + kg * 8;
+    // (in tiles: ff is a multiple of 64)
+    const size_t f = static_cast<size_t>(e) * ff + (TILED ? f0 + a * 16 : min(f0 + a * 16 + i, ff - 1));
+    const size_t at = f * width + (TILED ? lane * 8 : kg * 8);
+    wr[0][a] = wg + at;
+    if (!SINGLE) wr[M - 1][a] = wu + at;
   }
   mf32x4 acc[M][2][2], total[M];
 #pragma unroll
@@ -389,7 +394,7 @@ __global__ void __launch_bounds__(256)
     for (int a = 0; a < 2; ++a)
 #pragma unroll
       for (int b = 0; b < 2; ++b) acc[m][a][b] = mf32x4{0.f, 0.f, 0.f, 0.f};
-  moe_quarter<M>(xr, have, wr, width, wave, kg, acc);
+  moe_quarter<M, TILED>(xr, have, wr, width, wave, kg, acc);
   moe_join_quarters<M>(acc, wave, lane, sums, total);
   // features were the rows of the products: this lane holds features f0 + 16 b + 4 kg + r of pair row a * 16 + i
   const int p = wave / 2 ? pair[1] : pair[0];
@@ -402,6 +407,7 @@ __global__ void __launch_bounds__(256)
 }
 
 // pair_out[pair, c] = W_down_e[c] . act[pair]
+template <bool TILED>
 __global__ void __launch_bounds__(256)
     moe_down_mfma_kernel(const bf16* __restrict__ act_in, const int32_t* __restrict__ order,
                          const int32_t* __restrict__ counts, const bf16* __restrict__ wd,
@@ -424,14 +430,15 @@ __global__ void __launch_bounds__(256)
     pair[a] = r < count ? order[static_cast<size_t>(e) * n + r] : -1;
     have[a] = pair[a] >= 0;
     ar[a] = act_in + static_cast<size_t>(have[a] ? min(pair[a], n * top - 1) : 0) * ff + kg * 8;
-    wr[0][a] = wd + (static_cast<size_t>(e) * width + min(c0 + a * 16 + i, width - 1)) * ff + kg * 8;
+    wr[0][a] = wd + (static_cast<size_t>(e) * width + (TILED ? c0 + a * 16 : min(c0 + a * 16 + i, width - 1))) * ff +
+               (TILED ? lane * 8 : kg * 8);
   }
   mf32x4 acc[1][2][2], total[1];
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
     for (int b = 0; b < 2; ++b) acc[0][a][b] = mf32x4{0.f, 0.f, 0.f, 0.f};
-  moe_quarter<1>(ar, have, wr, ff, wave, kg, acc);
+  moe_quarter<1, TILED>(ar, have, wr, ff, wave, kg, acc);
   moe_join_quarters<1>(acc, wave, lane, sums, total);
   const int p = wave / 2 ? pair[1] : pair[0];
   if (p < 0) return;
@@ -578,23 +585,237 @@ __global__ void __launch_bounds__(256)
   }
 }
 
+// The same two products for weights in tiles (k and m multiples of 64): 256 weight rows (gate/up: 128
+// features of each) x 128 pairs a workgroup of eight wavefronts, each 64 x 64, in stages of 64 along k that go
+// from memory straight into LDS (global_load_lds), 1 KiB a load: a weight tile of 16 rows x 32, which
+// is the matrix instruction's operand as it lies, or 8 pairs' rows x 128 bytes, whole cache lines, gathered on
+// the way since a lane gives its own address.  Three stage buffers: two stages' loads are in flight while one is
+// multiplied, one barrier a stage.  Lane l of a pairs' load brings chunk l / 8 (of 8 elements) of row l % 8;
+// the operand of step ks takes rows j from unit j / 8 at place j % 8 + 8 * (kg + 4 ks): eight lanes read 128
+// consecutive bytes.
+// The grid is one row of workgroups and the lists' lengths are only known on the device: workgroup p takes the
+// p / 8-th tile of die p % 8's share of all live tiles, counted expert by expert, features outside, the
+// expert's pairs inside, so that the 32 compute units of a die read a matrix from memory once and its pairs'
+// rows stay in the die's L2.
+// 1,501 tokens, two of eight experts of 4736 features and width 3584: gate/up 360 us and down 227 in the
+// kernel above, 262 and 157 here; with row-major weights (8 rows x 128 bytes a load) this kernel
+// took 350 and 213, through registers 449 and 276: what it waits for is memory that is read 128 bytes at a time.
+// Pairs' rows laid out in tiles first (19 us a layer) changed nothing, nor did leaving out the multiplications
+// for the empty half of a list's last tile: the loads are what takes the time, about 42 GB/s a compute unit.
+constexpr int kBigPairs = 128, kBigRows = 256, kBigWaves = 8;
+
+#define SHK_MOE_TO_LDS(gptr, lptr)                                                                             \
+  __builtin_amdgcn_global_load_lds(                                                                           \
+      reinterpret_cast<const __attribute__((address_space(1))) void*>(reinterpret_cast<uintptr_t>(gptr)),     \
+      (__attribute__((address_space(3))) void*)(lptr), 16, 0, 0)
+// s_waitcnt vmcnt(n) alone
+#define SHK_MOE_WAIT(n) __builtin_amdgcn_s_waitcnt(0x0f70 | ((n) & 15) | (((n) >> 4) << 14))
+
+// Tile `index` of all experts' live tiles (features x ceil(count / kBigPairs) each): expert, first feature
+// tile, first pair; false beyond the last.  `index` < 0 asks for none and returns their number in `total`.
+__device__ __forceinline__ bool moe_tile(const int32_t* counts, int experts, int n, int features, int index, int lane,
+                                         int& total, int& e, int& within, int& row_tiles) {
+  total = 0;
+  for (int e0 = 0; e0 < experts; e0 += kWave) {
+    const int mine = e0 + lane < experts ? (min(counts[e0 + lane], n) + kBigPairs - 1) / kBigPairs : 0;
+    int before = mine;  // inclusive prefix over the lanes
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) {
+      const int up = __shfl_up(before, d, kWave);
+      if (lane >= d) before += up;
+    }
+    const int all = __shfl(before, kWave - 1, kWave);
+    if (index >= 0 && index < total + all * features) {
+      const int first = total + (before - mine) * features;
+      const unsigned long long hit = __ballot(mine > 0 && index >= first && index < first + mine * features);
+      const int at = __ffsll(hit) - 1;
+      e = e0 + at;
+      row_tiles = __shfl(mine, at, kWave);
+      within = index - __shfl(first, at, kWave);
+      return true;
+    }
+    total += all * features;
+  }
+  return false;
+}
+
+enum MoeProduct : int { kMoeGated = 0, kMoeSingle = 1, kMoeDown = 2 };
+
+template <int PRODUCT>
+__global__ void __launch_bounds__(kBigWaves* kWave)
+    moe_big_mfma_kernel(const bf16* __restrict__ a, const int32_t* __restrict__ order,
+                        const int32_t* __restrict__ counts, const bf16* __restrict__ w0, const bf16* __restrict__ w1,
+                        bf16* __restrict__ act_out, float* __restrict__ pair_out, int n, int k, int m, int experts, int top,
+                        GateForm form) {
+  constexpr int GN = 2, WM = 4, WN = 4;                         // wavefronts along the pairs; tiles of 16 x 16 a wavefront
+  constexpr int kWUnits = kBigRows / 8, kUnits = kWUnits + kBigPairs / 8, kLoads = kUnits / kBigWaves, kWLoads = kWUnits / kBigWaves;
+  constexpr int kFeatures = PRODUCT == kMoeGated ? kBigRows / 2 : kBigRows;
+  typedef unsigned int u4 __attribute__((ext_vector_type(4)));
+  __shared__ u4 stage0[kUnits][kWave], stage1[kUnits][kWave], stage2[kUnits][kWave];
+  const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int features = (m + kFeatures - 1) / kFeatures;
+  int total, e, within, row_tiles;
+  moe_tile(counts, experts, n, features, -1, lane, total, e, within, row_tiles);
+  const int per_die = (total + 7) / 8, turn = blockIdx.x / 8;
+  if (turn >= per_die) return;
+  if (!moe_tile(counts, experts, n, features, blockIdx.x % 8 * per_die + turn, lane, total, e, within, row_tiles)) return;
+  e = __builtin_amdgcn_readfirstlane(e);
+  within = __builtin_amdgcn_readfirstlane(within);
+  row_tiles = __builtin_amdgcn_readfirstlane(row_tiles);
+  const int count = min(counts[e], n), row0 = within % row_tiles * kBigPairs, f0 = within / row_tiles * kFeatures;
+  const int32_t* list = order + static_cast<size_t>(e) * n;
+  const int wm = wave / GN, wn = wave % GN;
+
+  // what this wavefront loads: units wave, wave + 8, ..: weight tiles first (block u / 2, step u % 2), then
+  // pairs' rows; rows beyond either matrix are read as its last (their products are not stored)
+  const bf16* src[kLoads];
+#pragma unroll
+  for (int i = 0; i < kLoads; ++i) {
+    const int u = wave + kBigWaves * i;
+    if (i < kWLoads) {
+      const int block = u / 2;  // wavefront block / 4's tile block % 4
+      // (gated: tiles 0 and 1 are gate features, 2 and 3 the same features of up)
+      const int f = PRODUCT == kMoeGated ? f0 + block / 4 * 32 + block % 2 * 16 : f0 + block * 16;
+      src[i] = (PRODUCT == kMoeGated && block % 4 >= 2 ? w1 : w0) +
+               ((static_cast<size_t>(e) * m + min(f, m - 16)) / 16 * (k / 32) + u % 2) * 512 + lane * 8;
+    } else {
+      const int at = row0 + (u - kWUnits) * 8 + lane % 8;
+      const int pair = list[at < count ? at : row0];
+      src[i] = a + static_cast<size_t>(PRODUCT == kMoeDown ? min(max(pair, 0), n * top - 1) : min(max(pair, 0) / top, n - 1)) * k +
+               lane / 8 * 8;
+    }
+  }
+  const int stages = k / 64;
+  auto load = [&](u4 (&buf)[kUnits][kWave], int st) {
+    const size_t at = static_cast<size_t>(st < stages ? st : 0) * 64;  // past the end: any stage, never multiplied
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) SHK_MOE_TO_LDS(src[i] + (i < kWLoads ? at * 16 : at), &buf[wave + kBigWaves * i][0]);
+  };
+  mf32x4 acc[WM][WN];
+#pragma unroll
+  for (int i = 0; i < WM; ++i)
+#pragma unroll
+    for (int jn = 0; jn < WN; ++jn) acc[i][jn] = mf32x4{0.f, 0.f, 0.f, 0.f};
+  const int unit = lane % 16 / 8, place = lane % 8 + 8 * (lane / 16);
+  auto multiply = [&](const u4 (&buf)[kUnits][kWave]) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      u4 wf[WM], af[WN];
+#pragma unroll
+      for (int jn = 0; jn < WN; ++jn) af[jn] = buf[kWUnits + (wn * WN + jn) * 2 + unit][place + 32 * ks];
+#pragma unroll
+      for (int i = 0; i < WM; ++i) wf[i] = buf[(wm * WM + i) * 2 + ks][lane];
+#pragma unroll
+      for (int i = 0; i < WM; ++i)
+#pragma unroll
+        for (int jn = 0; jn < WN; ++jn)
+          acc[i][jn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(mbf16x8, wf[i]),
+                                                               __builtin_bit_cast(mbf16x8, af[jn]), acc[i][jn], 0, 0, 0);
+    }
+  };
+  // a stage has landed for every wavefront once each has waited for its own loads of it (the younger stage's
+  // may stay in flight) and met the others; after the barrier nobody reads the stage before any more
+#define SHK_MOE_STEP(now, refill, st_refill) \
+  SHK_MOE_WAIT(kLoads);                      \
+  asm volatile("" ::: "memory");             \
+  __builtin_amdgcn_s_barrier();              \
+  asm volatile("" ::: "memory");             \
+  load(refill, st_refill);                   \
+  __builtin_amdgcn_sched_barrier(0);         \
+  multiply(now);
+  load(stage0, 0);
+  load(stage1, 1);
+  int st = 0;
+  for (; st + 2 < stages; st += 3) {
+    SHK_MOE_STEP(stage0, stage2, st + 2)
+    SHK_MOE_STEP(stage1, stage0, st + 3)
+    SHK_MOE_STEP(stage2, stage1, st + 4)
+  }
+  if (st < stages) { SHK_MOE_STEP(stage0, stage2, st + 2) }
+  if (st + 1 < stages) { SHK_MOE_STEP(stage1, stage0, st + 3) }
+#undef SHK_MOE_STEP
+  SHK_MOE_WAIT(0);  // no load may arrive in LDS that the workgroup has given back
+
+  // lane (j, kg) holds weight rows 4 kg + r of a tile for pair j
+  const int j = lane % 16, kg = lane / 16;
+#pragma unroll
+  for (int jn = 0; jn < WN; ++jn) {
+    const int at = row0 + (wn * WN + jn) * 16 + j;
+    if (at >= count) continue;
+    const size_t pair = min(max(list[at], 0), n * top - 1);
+#pragma unroll
+    for (int i = 0; i < (PRODUCT == kMoeGated ? WM / 2 : WM); ++i) {
+      const int f = f0 + (PRODUCT == kMoeGated ? wm * 32 + i * 16 : (wm * WM + i) * 16) + 4 * kg;
+      if (f >= m) continue;  // (m is a multiple of 8: four features are inside or outside together)
+      if (PRODUCT == kMoeDown) {
+        *reinterpret_cast<mf32x4*>(pair_out + pair * m + f) = acc[i][jn];
+      } else {
+        uint16_t h[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          h[r] = bf16_bits(gate_times_up(acc[i][jn][r], PRODUCT == kMoeGated ? acc[(i + WM / 2) % WM][jn][r] : acc[i][jn][r], form));
+        *reinterpret_cast<uint2*>(act_out + pair * m + f) =
+            make_uint2(h[0] | static_cast<uint32_t>(h[1]) << 16, h[2] | static_cast<uint32_t>(h[3]) << 16);
+      }
+    }
+  }
+}
+
+template <int PRODUCT>
+static void launch_big(const bf16* a, const int32_t* order, const int32_t* counts, const void* w0, const void* w1, bf16* act_out,
+                       float* pair_out, int n, int k, int m, int experts, int top, GateForm form, hipStream_t s) {
+  const long long features = PRODUCT == kMoeGated ? (m + kBigRows / 2 - 1) / (kBigRows / 2) : (m + kBigRows - 1) / kBigRows;
+  const long long pairs = static_cast<long long>(n) * top;
+  const long long tiles = features * (pairs / kBigPairs + (experts < pairs ? experts : pairs));  // live ones at most
+  moe_big_mfma_kernel<PRODUCT><<<static_cast<unsigned>((tiles + 7) / 8 * 8), kBigWaves * kWave, 0, s>>>(
+      a, order, counts, static_cast<const bf16*>(w0), static_cast<const bf16*>(w1), act_out, pair_out, n, k, m, experts, top,
+      form);
+}
+
 // out[t, c] = add[t, c] + sum_k weights[t, k] * pair_out[t * top + k, c], k in the order chosen; an identity
-// expert's output is x[t, c]
+// expert's output is x[t, c].  Eight columns a thread (width is a multiple of 8): 16-byte loads and stores, 25 us
+// at 1,501 tokens of 3584 with one column a thread, 13 so.
 __global__ void __launch_bounds__(256)
     moe_join_kernel(const float* __restrict__ pair_out, const int32_t* __restrict__ chosen, const bf16* __restrict__ x,
                     const float* __restrict__ weights, const bf16* __restrict__ add, const float* __restrict__ add_gate,
                     int gate_ld, bf16* __restrict__ out, int width, int top, int experts) {
+  union Eight {
+    uint4 u;
+    bf16 h[8];
+  };
   const int t = blockIdx.y;
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
+  const int c = (blockIdx.x * blockDim.x + threadIdx.x) * 8;
   if (c >= width) return;
-  float total = 0.f;
+  const size_t at = static_cast<size_t>(t) * width + c;
+  float total[8] = {};
   for (int k = 0; k < top; ++k) {
     const size_t pair = static_cast<size_t>(t) * top + k;
-    const float y = chosen[pair] < experts ? pair_out[pair * width + c] : to_float(x[static_cast<size_t>(t) * width + c]);
-    total = fmaf(weights[pair], y, total);
+    const float weight = weights[pair];
+    if (chosen[pair] < experts) {
+      const float4 *y = reinterpret_cast<const float4*>(pair_out + pair * width + c);
+      const float4 y0 = y[0], y1 = y[1];
+      total[0] = fmaf(weight, y0.x, total[0]), total[1] = fmaf(weight, y0.y, total[1]);
+      total[2] = fmaf(weight, y0.z, total[2]), total[3] = fmaf(weight, y0.w, total[3]);
+      total[4] = fmaf(weight, y1.x, total[4]), total[5] = fmaf(weight, y1.y, total[5]);
+      total[6] = fmaf(weight, y1.z, total[6]), total[7] = fmaf(weight, y1.w, total[7]);
+    } else {
+      Eight v;
+      v.u = *reinterpret_cast<const uint4*>(x + at);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) total[i] = fmaf(weight, to_float(v.h[i]), total[i]);
+    }
   }
-  if (add) total += shared_share(add_gate, gate_ld, t) * to_float(add[static_cast<size_t>(t) * width + c]);
-  out[static_cast<size_t>(t) * width + c] = from_float<bf16>(total);
+  if (add) {
+    Eight v;
+    v.u = *reinterpret_cast<const uint4*>(add + at);
+    const float share = shared_share(add_gate, gate_ld, t);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) total[i] += share * to_float(v.h[i]);
+  }
+  Eight v;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v.h[i] = from_float<bf16>(total[i]);
+  *reinterpret_cast<uint4*>(out + at) = v.u;
 }
 
 }  // namespace shk
@@ -663,19 +884,22 @@ extern "C" long long shk_moe_grouped_scratch_bytes(int n, int width, int experts
 extern "C" int shk_moe_experts_grouped(const void* x, const int32_t* chosen, const float* weights, const void* w_gate,
                                        const void* w_up, const void* w_down, const void* add, const float* add_gate,
                                        int gate_ld, void* act_buf, void* out, void* scratch, int n, int width, int ff, int experts, int top,
-                                       int identity, int act, float limit, float shift, void* stream) {
+                                       int identity, int act, float limit, float shift, int tiled, void* stream) {
   SHK_REQUIRE(n >= 0 && width > 0 && ff > 0 && experts > 0 && experts <= 65535 && identity >= 0 && top >= 1 && top <= experts + identity,
               "moe_experts_grouped: bad sizes n=%d width=%d ff=%d experts=%d top=%d", n, width, ff, experts, top);
   SHK_REQUIRE(act >= 1 && act <= 4, "moe_experts_grouped: unknown activation %d", act);
   SHK_REQUIRE(!add_gate || (add && gate_ld >= 1),
               "moe_experts_grouped: a gate of the added rows needs those rows and a stride");
   SHK_REQUIRE(width % 8 == 0 && ff % 8 == 0, "moe_experts_grouped: width %d and ff %d must be multiples of 8", width, ff);
+  SHK_REQUIRE(!tiled || (width % 64 == 0 && ff % 64 == 0),
+              "moe_experts_grouped: weights in tiles need a width %d and ff %d in multiples of 64", width, ff);
   if (n == 0) return 0;
   SHK_REQUIRE(static_cast<long long>(n) * top < (1LL << 30) && (n + 31) / 32 <= 65535,
               "moe_experts_grouped: too many (token, expert) pairs");
   SHK_REQUIRE(x && chosen && weights && w_gate && w_up && w_down && act_buf && out && scratch,
               "moe_experts_grouped: null pointer");
-  for (const void* p : {x, w_gate, w_up, w_down, static_cast<const void*>(act_buf), static_cast<const void*>(scratch)})
+  for (const void* p : {x, w_gate, w_up, w_down, add, static_cast<const void*>(act_buf), static_cast<const void*>(scratch),
+                        static_cast<const void*>(out)})
     SHK_REQUIRE(reinterpret_cast<uintptr_t>(p) % 16 == 0, "moe_experts_grouped: operands must be 16-byte aligned");
   hipStream_t s = static_cast<hipStream_t>(stream);
   const GateForm form{act, limit, shift};
@@ -684,8 +908,15 @@ extern "C" int shk_moe_experts_grouped(const void* x, const int32_t* chosen, con
   const long long ints = static_cast<long long>(experts) * n + experts;
   float* pair_out = reinterpret_cast<float*>(static_cast<char*>(scratch) + ((ints * 4 + 15) / 16) * 16);
   moe_lists_kernel<<<experts, 256, 0, s>>>(chosen, n, top, order, counts);
-  if (static_cast<long long>(n) * top >= 64LL * experts) {
-    // lists of 64 pairs and more on average: tiles of 128 pairs through LDS
+  const bf16 *xb = static_cast<const bf16*>(x), *actb = static_cast<const bf16*>(act_buf);
+  const bool many = static_cast<long long>(n) * top >= 64LL * experts;  // lists of 64 pairs and more on average
+  if (many && tiled) {
+    if (w_gate == w_up)
+      launch_big<kMoeSingle>(xb, order, counts, w_gate, w_up, static_cast<bf16*>(act_buf), nullptr, n, width, ff, experts, top, form, s);
+    else
+      launch_big<kMoeGated>(xb, order, counts, w_gate, w_up, static_cast<bf16*>(act_buf), nullptr, n, width, ff, experts, top, form, s);
+    launch_big<kMoeDown>(actb, order, counts, w_down, nullptr, nullptr, pair_out, n, ff, width, experts, top, form, s);
+  } else if (many) {
     const int row_tiles = (n + kTileRows - 1) / kTileRows;
     if (w_gate == w_up)
       moe_tiled_mfma_kernel<true, true><<<dim3((ff + 127) / 128, row_tiles, experts), 256, 0, s>>>(
@@ -700,19 +931,17 @@ extern "C" int shk_moe_experts_grouped(const void* x, const int32_t* chosen, con
         ff, width, top, form);
   } else {
     const int row_tiles = (n + 31) / 32;
-    const dim3 features((ff + 31) / 32, row_tiles, experts);
-    if (w_gate == w_up)
-      moe_gate_up_mfma_kernel<true><<<features, 256, 0, s>>>(
-          static_cast<const bf16*>(x), order, counts, static_cast<const bf16*>(w_gate), static_cast<const bf16*>(w_up),
-          static_cast<bf16*>(act_buf), n, width, ff, top, form);
-    else
-      moe_gate_up_mfma_kernel<false><<<features, 256, 0, s>>>(
-          static_cast<const bf16*>(x), order, counts, static_cast<const bf16*>(w_gate), static_cast<const bf16*>(w_up),
-          static_cast<bf16*>(act_buf), n, width, ff, top, form);
-    moe_down_mfma_kernel<<<dim3((width + 31) / 32, row_tiles, experts), 256, 0, s>>>(
-        static_cast<const bf16*>(act_buf), order, counts, static_cast<const bf16*>(w_down), pair_out, n, width, ff, top);
+    const dim3 features((ff + 31) / 32, row_tiles, experts), columns((width + 31) / 32, row_tiles, experts);
+    const bool single = w_gate == w_up;
+    auto gate_up = tiled ? (single ? moe_gate_up_mfma_kernel<true, true> : moe_gate_up_mfma_kernel<false, true>)
+                         : (single ? moe_gate_up_mfma_kernel<true, false> : moe_gate_up_mfma_kernel<false, false>);
+    gate_up<<<features, 256, 0, s>>>(xb, order, counts, static_cast<const bf16*>(w_gate), static_cast<const bf16*>(w_up),
+                                     static_cast<bf16*>(act_buf), n, width, ff, top, form);
+    auto down = tiled ? moe_down_mfma_kernel<true> : moe_down_mfma_kernel<false>;
+    down<<<columns, 256, 0, s>>>(actb, order, counts, static_cast<const bf16*>(w_down), pair_out, n, width, ff, top);
   }
-  moe_join_kernel<<<dim3((width + 255) / 256, n), 256, 0, s>>>(pair_out, chosen, static_cast<const bf16*>(x), weights,
+  const int join_threads = width >= 2048 ? 256 : kWave;
+  moe_join_kernel<<<dim3((width / 8 + join_threads - 1) / join_threads, n), join_threads, 0, s>>>(pair_out, chosen, static_cast<const bf16*>(x), weights,
                                                                static_cast<const bf16*>(add), add_gate, gate_ld,
                                                                static_cast<bf16*>(out), width, top, experts);
   SHK_LAUNCH_CHECK("moe_experts_grouped");

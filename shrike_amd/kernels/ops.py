@@ -1225,8 +1225,29 @@ def moe_grouped_scratch_bytes(n: int, width: int, experts: int, top: int) -> int
     return int(load().shk_moe_grouped_scratch_bytes(n, width, experts, top))
 
 
+def moe_tiles(width: int, ff: int, dtype) -> bool:
+    """Whether stacked experts' matrices may be held in tiles: bfloat16, whole tiles and stages of every kernel."""
+    return dtype == torch.bfloat16 and width % 64 == 0 and ff % 64 == 0
+
+
+def tile_experts(matrices) -> torch.Tensor:
+    """The experts' [m, k] matrices (a list, or stacked), one behind the other in tiles of 16 rows x 32 columns, as
+    retile_weight() lays them out (m and k multiples of 64: no padding between them): [experts, m, k]."""
+    m, k = matrices[0].shape
+    if m % 64 or k % 64:
+        raise KernelError(f"tile_experts: matrices of {m} x {k} are not whole tiles")
+    out = torch.empty(len(matrices), m, k, dtype=torch.bfloat16, device=matrices[0].device)
+    for e in range(len(matrices)):
+        w = matrices[e]
+        if tuple(w.shape) != (m, k) or not w.is_contiguous():
+            raise KernelError("tile_experts: expected contiguous matrices of one shape")
+        check(load().shk_retile_weight(_dev(w, "w", torch.bfloat16), m, k, _dev(out[e], "out"), _stream()))
+    return out
+
+
 def moe_experts(x, chosen, weights, w_gate, w_up, w_down, act_buf, out, activation: str = "silu", add=None,
-                scratch=None, add_gate=None, identity: int = 0, limit: float | None = None, up_shift: float = 0.0) -> None:
+                scratch=None, add_gate=None, identity: int = 0, limit: float | None = None, up_shift: float = 0.0,
+                tiled: bool = False) -> None:
     """out = add + sum_k weights[:, k] * down_e(act(gate_e x) * (up_e x + up_shift)), e = chosen[:, k]; with `limit`
     the gate's product is bounded from above and the other one from both sides first; the `identity` indices
     behind the stacked experts stand for x itself; matrices
@@ -1234,7 +1255,8 @@ def moe_experts(x, chosen, weights, w_gate, w_up, w_down, act_buf, out, activati
     moe_grouped_scratch_bytes): the products run per expert on the matrix units (see moe_grouped).
     add_gate: a float32 column (a view [n] with any stride): add[t] is multiplied by
     sigmoid(add_gate[t]).  Experts without a gate whose activation is the square of ReLU pass
-    their one matrix as both w_gate and w_up with activation "relu"."""
+    their one matrix as both w_gate and w_up with activation "relu".  tiled: the matrices are what
+    tile_experts() made of the stacked ones (needs scratch)."""
     n, width = x.shape
     experts, ff, _ = w_gate.shape
     top = chosen.shape[1]
@@ -1261,8 +1283,10 @@ def moe_experts(x, chosen, weights, w_gate, w_up, w_down, act_buf, out, activati
             _dev(x, "x"), _dev(chosen, "chosen"), _dev(weights, "weights"), _dev(w_gate, "w_gate"), _dev(w_up, "w_up"),
             _dev(w_down, "w_down"), None if add is None else _dev(add, "add"), gate_ptr, gate_ld,
             _dev(act_buf, "act_buf"), _dev(out, "out"), _dev(scratch, "scratch"), n, width, ff, experts, top, *form,
-            _stream()))
+            int(bool(tiled)), _stream()))
         return
+    if tiled:
+        raise KernelError("moe_experts: matrices in tiles are for steps with scratch")
     check(load().shk_moe_experts(_dev(x, "x"), _dev(chosen, "chosen"), _dev(weights, "weights"), _dev(w_gate, "w_gate"),
                                  _dev(w_up, "w_up"), _dev(w_down, "w_down"), None if add is None else _dev(add, "add"),
                                  gate_ptr, gate_ld, _dev(act_buf, "act_buf"), _dev(out, "out"), dtype_code(x.dtype), n, width, ff, experts,

@@ -85,7 +85,14 @@ class MixtureOfExperts(FeedForward):
 
     def load(self, tensors, runtime):
         s = self.spec
-        stack = lambda role: torch.stack([tensors[self._expert(e, role)] for e in range(s.experts)]).contiguous()  # noqa: E731
+        # (in tiles: every bfloat16 step takes the kernels that read them, MOE_GROUPED_FROM is one token)
+        self.tiled = ops.moe_tiles(self.width, s.expert_size, runtime.dtype) and ops.moe_grouped(
+            1, self.width, s.expert_size, runtime.dtype)
+
+        def stack(role):
+            matrices = [tensors[self._expert(e, role)].contiguous() for e in range(s.experts)]
+            return ops.tile_experts(matrices) if self.tiled else torch.stack(matrices)
+
         self.w_up, self.w_down = stack("up"), stack("down")
         # experts without a gate: relu(u) * u is the square of relu(u), so the gated kernels take the one
         # matrix in both places (they form its product once where the two are the same)
@@ -142,7 +149,7 @@ class MixtureOfExperts(FeedForward):
         ops.moe_experts(x, chosen, weights, self.w_gate, self.w_up, self.w_down, act_buf, out, self.activation,
                         add=shared_out, scratch=scratch,
                         add_gate=logits[:, self.choices] if self.shared_gate else None, identity=s.identity,
-                        limit=s.limit, up_shift=s.up_shift)
+                        limit=s.limit, up_shift=s.up_shift, tiled=self.tiled)
         return out
 
 
