@@ -188,6 +188,10 @@ __device__ __forceinline__ void skinny_load_aligned(SkinnyBatch<NB, RB>& b,
 // silu(gate) * up: out[token][16b + row], `m` being the width of that output.
 // MODE kPair: a workgroup owns two consecutive blocks of rows, so that every
 // activation it loads feeds two multiplications.
+// blockIdx.z: which NB * 16 tokens.  More than one such group comes with matrices of up to 64
+// rows (a router, a low-rank pair's first matrix) and many tokens: the large kernels would give
+// 1,501 tokens to 12 workgroups that each walk all of k alone (10 x 3584: 37 us); here 94
+// workgroups share each group's k among 16 wavefronts (9.8 us).
 constexpr int kSingle = 0, kGated = 1, kPair = 2;
 
 template <int NB, int WAVES, int MODE>
@@ -203,6 +207,9 @@ __global__ void __launch_bounds__(WAVES* kWave)
   const int mb = blockIdx.x;  // block of 16 output rows (kPair: of 32)
   const int z = blockIdx.y;   // which share of k (ksplit workgroups per block)
   const int j = lane % 16, kg = lane / 16;
+  const int tok0 = blockIdx.z * NB * 16;
+  a += static_cast<size_t>(tok0) * lda;
+  n -= tok0;
   const uint4* wrow = wt + static_cast<size_t>(mb) * RB * ktiles * kWave + lane;
   // weight blocks of 16 rows that exist for this workgroup (the last pair may be half)
   const int blocks = MODE == kPair ? ((m + 15) / 16 - mb * 2 >= 2 ? 2 : 1) : RB;
@@ -308,7 +315,7 @@ __global__ void __launch_bounds__(WAVES* kWave)
     if (GATED) v = gate_times_up(v, up, accumulate, bias);
     if (!GATED && bias) v += bias[row];
     if (!GATED) v = plain_act(v, accumulate, row);
-    const size_t idx = static_cast<size_t>(token) * ldo + row;
+    const size_t idx = static_cast<size_t>(tok0 + token) * ldo + row;
     if (out_f32) {
       float* o = static_cast<float*>(out);
       o[idx] = (accumulate == 1 && !GATED) ? o[idx] + v : v;
@@ -1323,6 +1330,9 @@ static int big_shape(int split, int n, int wblocks, int m, int k) {
 
 extern "C" int shk_gemm_bf16_splits(int n, int m, int k);
 
+// Matrices of so few rows that many tokens go to gemm_skinny_kernel, group by group.
+static bool few_rows(int m) { return m <= 64; }
+
 // 256 x 256 tiles that do not make whole rounds of the 256 compute units (296 of them:
 // two rounds, the second nearly empty) are better run as two products: the row tiles
 // that make whole rounds, then the remaining rows with the tile shape that suits them.
@@ -1345,13 +1355,14 @@ static int big_main_blocks(int shape, int n, int wblocks, int m, int k, int gate
 
 // Products that a call with these sizes is made of (1, or 2: see big_main_blocks).
 extern "C" int shk_gemm_bf16_parts(int n, int m, int k, int gated) {
-  if (n <= 64 || shk_gemm_bf16_splits(n, m, k) > 1) return 1;
+  if (n <= 64 || (few_rows(m) && !gated) || shk_gemm_bf16_splits(n, m, k) > 1) return 1;
   const int wblocks = (gated ? 2 : 1) * ((m + 15) / 16);
   return big_main_blocks(big_shape(1, n, wblocks, m, k), n, wblocks, m, k, gated) ? 2 : 1;
 }
 
 extern "C" int shk_gemm_bf16_splits(int n, int m, int k) {
   const int mblocks = (m + 15) / 16, ktiles = (k + 31) / 32;
+  if (n > 64 && few_rows(m)) return 1;
   if (n > 64) {
     // many tokens: the number of shares, each of at least 8 stages of 64, that
     // big_estimate() expects to be fastest with the tile shape that suits it
@@ -1435,6 +1446,12 @@ extern "C" int shk_gemm_bf16_tiled_weight(const void* a, const void* wt, const f
   const bf16* ap = static_cast<const bf16*>(a);
   const uint4* wp = static_cast<const uint4*>(wt);
   const int of = out_dtype == kF32;
+  if (n > 64 && few_rows(m) && !gated && ksplit == 1 && n <= 65535 * 16) {
+    gemm_skinny_kernel<1, 16, kSingle><<<dim3(mb, 1, (n + 15) / 16), 16 * kWave, 0, s>>>(
+        ap, lda, n, k, wp, kt, m, bias, out, ldo, of, accumulate, vec, 1);
+    SHK_LAUNCH_CHECK("gemm_bf16");
+    return 0;
+  }
   if (n > 64) {
     SHK_REQUIRE(reinterpret_cast<uintptr_t>(out) % 8 == 0, "gemm_bf16: out is not 8-byte aligned");
     const int wblocks = (gated ? 2 : 1) * mb;  // blocks of 16 weight rows

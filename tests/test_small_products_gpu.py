@@ -1,0 +1,55 @@
+"""Products with matrices of few rows over many tokens, and batched products in each of their shapes, against
+float64, at the edges of tiles and with ends of k that are no whole step."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n", [65, 80, 1501])
+@pytest.mark.parametrize("m, k", [(1, 64), (10, 3584), (16, 896), (17, 72), (64, 520), (65, 512)])
+def test_few_rows_many_tokens(n, m, k):
+    from shrike_amd.kernels import ops
+
+    torch.manual_seed(n + m + k)
+    a, w = torch.randn(n, k, device="cuda").bfloat16(), torch.randn(m, k, device="cuda").bfloat16()
+    bias, wt = torch.randn(m, device="cuda"), ops.retile_weight(w)
+    want = a.double() @ w.double().t() + bias.double()
+    out = torch.full((n, m + 3), 7.0, device="cuda")
+    ops.gemm_tiled_weight(a, wt, m, k, out[:, :m], bias=bias)
+    # float32 sums: at most k / 32 + 40 roundings of half an ulp of a partial sum each
+    size = a.double().abs() @ w.double().abs().t() + bias.double().abs()
+    assert bool(((out[:, :m].double() - want).abs() <= (k / 32 + 40) * 2.0**-24 * size).all())
+    assert bool((out[:, m:] == 7.0).all())
+    half = torch.empty(n, m, device="cuda", dtype=torch.bfloat16)
+    ops.gemm_tiled_weight(a, wt, m, k, half, bias=bias)
+    assert torch.equal(half, out[:, :m].bfloat16())
+    few = torch.empty(n - 3, m, device="cuda", dtype=torch.bfloat16)
+    if n - 3 > 64:
+        ops.gemm_tiled_weight(a[3:], wt, m, k, few, bias=bias)
+        assert torch.equal(few, half[3:])
+
+
+@pytest.mark.parametrize("batch, m, k", [(3, 40, 8), (28, 448, 128), (5, 130, 200), (14, 512, 256), (2, 3, 40), (1, 64, 24)])
+def test_batched_products_of_every_shape(batch, m, k):
+    from shrike_amd.kernels import ops
+
+    torch.manual_seed(batch + m + k)
+    n_max = 300
+    a = torch.randn(n_max, batch * k + 8, device="cuda").bfloat16()
+    w = torch.randn(batch, m, k, device="cuda").bfloat16()
+    per = a[:, : batch * k].view(n_max, batch, k).transpose(0, 1).double()
+    want = (per @ w.transpose(1, 2).contiguous().double()).transpose(0, 1).reshape(n_max, batch * m)
+    size = (per.abs() @ w.transpose(1, 2).contiguous().double().abs()).transpose(0, 1).reshape(n_max, batch * m)
+    whole = None
+    for n in (n_max, 1, 15, 16, 17, 65, 129):
+        out = torch.full((n, batch * m + 4), 7.0, device="cuda")
+        ops.gemm_batched(a[:n, : batch * k], w, out[:, : batch * m], batch, k, m)
+        assert bool(((out[:, : batch * m].double() - want[:n]).abs() <= (k / 32 + 40) * 2.0**-24 * size[:n]).all())
+        assert bool((out[:, batch * m :] == 7.0).all())
+        whole = out if whole is None else whole
+        assert torch.equal(out, whole[:n]), "the same bits in every shape"
+        odd = torch.full((n, batch * m + 3), 7.0, device="cuda", dtype=torch.bfloat16)  # rows no multiple of 4 elements apart
+        ops.gemm_batched(a[:n, : batch * k], w, odd[:, 1 : 1 + batch * m], batch, k, m)
+        assert torch.equal(odd[:, 1 : 1 + batch * m], out[:, : batch * m].bfloat16())
