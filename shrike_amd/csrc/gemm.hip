@@ -155,57 +155,127 @@ extern "C" int shk_gemm(const void* a, const void* w, const float* bias, void* o
 
 // The same batch on the matrix units for bfloat16: both operands are row-major with k innermost, which
 // is the operand layout of v_mfma_f32_16x16x32_bf16 as it stands (a lane's 8 consecutive k of one row
-// are one 16-byte load), so nothing passes through LDS.  A wavefront forms 16 rows x 64 features (four
-// tiles that share the rows' operand); a workgroup of four wavefronts 64 x 64.  k in multiples of 8
-// and 16-byte aligned rows; a wavefront's result does not depend on what else is in the step.
+// are one 16-byte load), so nothing passes through LDS.  A wavefront forms RT x CT tiles of 16 rows x
+// 16 features, a workgroup RW x CW of that; the next U steps' operands are in flight while U are
+// multiplied.  k in multiples of 8 and 16-byte aligned rows; sums run over k in ascending order in every
+// shape, so a row's result depends neither on the shape nor on what else is in the step.
+// What bounds it is the compute units' intake: 64 x 64 a wavefront needs 8 KiB for 16 instructions.
+// 28 heads, 1,501 rows: k = 128 to 448 features 74 us with 16 x 64 a wavefront, no load ahead and 2-byte
+// stores, 41 so; k = 448 to 128 features 58, now 35; 14 blocks of 256 to 512 float32 68, now 35.  Eight rows: 6.0,
+// 11.7 and 7.5 us with 64-row workgroups, 5.0, 5.9 and 4.7 now.
 typedef __bf16 gbf16x8 __attribute__((ext_vector_type(8)));
 typedef float gf32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int gu32x4 __attribute__((ext_vector_type(4)));
 
-template <typename TO>
-__global__ void __launch_bounds__(256)
+template <int RT, int CT, int RW, int CW, int U, typename TO>
+__global__ void __launch_bounds__(kWave* RW* CW)
     gemm_batched_mfma_kernel(const bf16* __restrict__ a, const bf16* __restrict__ w, TO* __restrict__ out, int n,
-                             int m, int k, int lda, int ldo, long long a_batch, long long w_batch,
+                             int m, int k, int lda, int ldo, int vec_out, long long a_batch, long long w_batch,
                              long long out_batch) {
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   const int i = lane % 16, kg = lane / 16;
   const int b = blockIdx.z;
-  const int row = (blockIdx.y * 4 + wave) * 16 + i;  // the row of a whose operand this lane loads
-  const int col0 = blockIdx.x * 64;
-  const bf16* ar = a + b * a_batch + static_cast<size_t>(row < n ? row : 0) * lda + kg * 8;
-  const bf16* wr[4];
+  const int row0 = (blockIdx.y * RW + wave / CW) * RT * 16, col0 = (blockIdx.x * CW + wave % CW) * CT * 16;
+  if (row0 >= n || col0 >= m) return;  // (no barrier in this kernel)
+  // rows beyond either matrix are read as its last and not stored
+  const bf16 *ar[RT], *wr[CT];
 #pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    const int c = col0 + t * 16 + i;  // the feature whose weights this lane loads for tile t
-    wr[t] = w + b * w_batch + static_cast<size_t>(c < m ? c : 0) * k + kg * 8;
-  }
-  gf32x4 acc[4];
+  for (int r = 0; r < RT; ++r) ar[r] = a + b * a_batch + static_cast<size_t>(min(row0 + r * 16 + i, n - 1)) * lda + kg * 8;
 #pragma unroll
-  for (int t = 0; t < 4; ++t) acc[t] = gf32x4{0.f, 0.f, 0.f, 0.f};
-  for (int k0 = 0; k0 < k; k0 += 32) {
-    const bool have = k0 + kg * 8 < k;  // (k is a multiple of 8: a piece is whole or absent)
-    uint4 av = make_uint4(0, 0, 0, 0), wv[4];
-    if (have && row < n) av = *reinterpret_cast<const uint4*>(ar + k0);
+  for (int c = 0; c < CT; ++c) wr[c] = w + b * w_batch + static_cast<size_t>(min(col0 + c * 16 + i, m - 1)) * k + kg * 8;
+  gf32x4 acc[RT][CT];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      wv[t] = make_uint4(0, 0, 0, 0);
-      if (have && col0 + t * 16 + i < m) wv[t] = *reinterpret_cast<const uint4*>(wr[t] + k0);
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int c = 0; c < CT; ++c) acc[r][c] = gf32x4{0.f, 0.f, 0.f, 0.f};
+  // the products are formed transposed (features as rows): a lane gets features 4 kg + 0..3 of a tile for row i
+  auto multiply = [&](const gu32x4(&av)[RT], const gu32x4(&wv)[CT]) {
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int c = 0; c < CT; ++c)
+        acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gbf16x8, wv[c]),
+                                                            __builtin_bit_cast(gbf16x8, av[r]), acc[r][c], 0, 0, 0);
+  };
+  const int steps = k / 32;
+  if (steps > 0) {
+    gu32x4 av[2][U][RT], wv[2][U][CT];
+    auto load = [&](int set, int s0) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {  // (unconditional: a step beyond the last is the last again)
+        const int kk = min(s0 + u, steps - 1) * 32;
+#pragma unroll
+        for (int r = 0; r < RT; ++r) av[set][u][r] = *reinterpret_cast<const gu32x4*>(ar[r] + kk);
+#pragma unroll
+        for (int c = 0; c < CT; ++c) wv[set][u][c] = *reinterpret_cast<const gu32x4*>(wr[c] + kk);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    load(0, 0);
+    for (int s = 0; s < steps; s += 2 * U) {
+      load(1, s + U);
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (s + u < steps) multiply(av[0][u], wv[0][u]);
+      load(0, s + 2 * U);
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (s + U + u < steps) multiply(av[1][u], wv[1][u]);
     }
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gbf16x8, wv[t]), __builtin_bit_cast(gbf16x8, av),
-                                                       acc[t], 0, 0, 0);
   }
-  // the products were formed transposed (features as rows): this lane holds features 4 kg + r of tile t for row i
-  const int orow = (blockIdx.y * 4 + wave) * 16 + i;
-  if (orow >= n) return;
-  TO* dst = out + b * out_batch + static_cast<size_t>(orow) * ldo;
+  if (steps * 32 < k) {  // (k is a multiple of 8: a lane's piece is whole or absent)
+    const bool have = steps * 32 + kg * 8 < k;
+    const int kk = have ? steps * 32 : -kg * 8;
+    const uint32_t keep = have ? 0xffffffffu : 0u;
+    gu32x4 av[RT], wv[CT];
 #pragma unroll
-  for (int t = 0; t < 4; ++t)
+    for (int r = 0; r < RT; ++r) av[r] = *reinterpret_cast<const gu32x4*>(ar[r] + kk) & keep;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int c = col0 + t * 16 + 4 * kg + r;
-      if (c < m) dst[c] = from_float<TO>(acc[t][r]);
+    for (int c = 0; c < CT; ++c) wv[c] = *reinterpret_cast<const gu32x4*>(wr[c] + kk) & keep;
+    multiply(av, wv);
+  }
+#pragma unroll
+  for (int r = 0; r < RT; ++r) {
+    const int row = row0 + r * 16 + i;
+    if (row >= n) continue;
+    TO* dst = out + b * out_batch + static_cast<size_t>(row) * ldo;
+#pragma unroll
+    for (int t = 0; t < CT; ++t) {
+      const int c = col0 + t * 16 + 4 * kg;
+      if (vec_out && c + 3 < m) {
+        if constexpr (sizeof(TO) == 4) {
+          *reinterpret_cast<gf32x4*>(dst + c) = acc[r][t];
+        } else {
+          const uint32_t lo = bf16_bits(acc[r][t][0]) | static_cast<uint32_t>(bf16_bits(acc[r][t][1])) << 16;
+          const uint32_t hi = bf16_bits(acc[r][t][2]) | static_cast<uint32_t>(bf16_bits(acc[r][t][3])) << 16;
+          *reinterpret_cast<uint2*>(dst + c) = make_uint2(lo, hi);
+        }
+        continue;
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (c + e < m) dst[c + e] = from_float<TO>(acc[r][t][e]);
     }
+  }
+}
+
+// Shapes: up to 16 rows 16 x 16 a wavefront, side by side along the features (the weights' latency is all
+// there is); 64 x 64 a wavefront where such workgroups fill the compute units, else 32 x 32.
+template <typename TO>
+static void launch_batched_mfma(const bf16* a, const bf16* w, TO* out, int n, int m, int k, int lda, int ldo, int batch,
+                                long long a_batch, long long w_batch, long long out_batch, hipStream_t s) {
+  const int vec_out = ldo % 4 == 0 && out_batch % 4 == 0 && reinterpret_cast<uintptr_t>(out) % (4 * sizeof(TO)) == 0;
+  auto grid = [&](int rows, int cols) { return dim3((m + cols - 1) / cols, (n + rows - 1) / rows, batch); };
+  const dim3 large = grid(128, 128);
+  if (n <= 16)
+    gemm_batched_mfma_kernel<1, 1, 1, 4, 4, TO>
+        <<<grid(16, 64), 256, 0, s>>>(a, w, out, n, m, k, lda, ldo, vec_out, a_batch, w_batch, out_batch);
+  else if (static_cast<long long>(large.x) * large.y * batch >= 256)
+    gemm_batched_mfma_kernel<4, 4, 2, 2, 1, TO>
+        <<<large, 256, 0, s>>>(a, w, out, n, m, k, lda, ldo, vec_out, a_batch, w_batch, out_batch);
+  else
+    gemm_batched_mfma_kernel<2, 2, 2, 2, 2, TO>
+        <<<grid(64, 64), 256, 0, s>>>(a, w, out, n, m, k, lda, ldo, vec_out, a_batch, w_batch, out_batch);
 }
 
 // A batch of products of one shape (one per head, say): product b reads a + b * a_batch
@@ -225,15 +295,11 @@ extern "C" int shk_gemm_batched(const void* a, const void* w, void* out, int n, 
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (dtype == kBF16 && k % 8 == 0 && lda % 8 == 0 && a_batch % 8 == 0 && reinterpret_cast<uintptr_t>(a) % 16 == 0 &&
       reinterpret_cast<uintptr_t>(w) % 16 == 0 && (n + 63) / 64 <= 65535) {
-    dim3 grid((m + 63) / 64, (n + 63) / 64, batch);
+    const bf16 *ab = static_cast<const bf16*>(a), *wb = static_cast<const bf16*>(w);
     if (out_dtype == kF32)
-      gemm_batched_mfma_kernel<float><<<grid, 256, 0, s>>>(static_cast<const bf16*>(a), static_cast<const bf16*>(w),
-                                                           static_cast<float*>(out), n, m, k, lda, ldo, a_batch, w_batch,
-                                                           out_batch);
+      launch_batched_mfma(ab, wb, static_cast<float*>(out), n, m, k, lda, ldo, batch, a_batch, w_batch, out_batch, s);
     else
-      gemm_batched_mfma_kernel<bf16><<<grid, 256, 0, s>>>(static_cast<const bf16*>(a), static_cast<const bf16*>(w),
-                                                          static_cast<bf16*>(out), n, m, k, lda, ldo, a_batch, w_batch,
-                                                          out_batch);
+      launch_batched_mfma(ab, wb, static_cast<bf16*>(out), n, m, k, lda, ldo, batch, a_batch, w_batch, out_batch, s);
   } else if (n <= 2 * kSkinnyRows && dtype == kBF16) {
     // (float32 keeps one order of summation whatever the number of rows: gemm_f32.hip)
     dim3 grid((m + 3) / 4, batch);
