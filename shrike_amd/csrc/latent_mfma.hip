@@ -17,6 +17,8 @@
 // results (O, maximum, sum) latent_merge_kernel joins in order (single tokens with thousands
 // of rows would otherwise leave the chip idle).  Rows of up to 640 elements in multiples of 8,
 // up to 128 heads; other shapes are served by latent_attention_kernel (latent.hip).
+#include <type_traits>
+
 #include "api.h"
 #include "common.h"
 
@@ -248,6 +250,209 @@ __global__ void __launch_bounds__(kLatentWaves* kWave)
   }
 }
 
+// Prompt portions: a workgroup of eight wavefronts serves `tpw` tokens that follow each other, all heads of
+// each: up to 16 NC columns (token, head) of both products.  Wavefront w < NC forms the scores and weights of
+// column tile w over a chunk of 32 rows and leaves the weights in LDS as operands, beside the factor by which
+// its columns' sums shrink; all eight then form O^T += V^T P^T, wavefront w the value elements of tiles w, w + 8,
+// .. for every column.  A value operand (eight 2-byte reads, transposing on the way out of LDS) thus serves NC
+// matrix instructions where the kernel above uses it once, and a chunk is staged once for tpw tokens.  Two
+// buffers for the rows and for the weights: two barriers a chunk.
+// What bounded the kernel above over a prompt was its LDS reads, 288 for 60 matrix instructions a chunk and
+// wavefront: 28 heads over rows of 512, 1,501 tokens, 483 us a layer, 266 here; rows straight into LDS instead
+// of through registers took 437 (more addresses than registers are left: spills).
+constexpr int kPromptWaves = 8;
+
+template <int KS, int DBW, int NC>  // rows of up to 32 KS elements, values of up to 128 DBW, 16 NC columns
+__global__ void __launch_bounds__(kPromptWaves* kWave)
+    latent_prompt_kernel(const bf16* __restrict__ q, bf16* __restrict__ out, int heads, int key_dim, int v_dim,
+                         const int32_t* __restrict__ positions, const int32_t* __restrict__ token_seq,
+                         const int32_t* __restrict__ tables, int table_stride, const bf16* __restrict__ pool,
+                         int page_size, int num_pages, int window, int chunk, float scale,
+                         float* __restrict__ partial, int nsplit, int n, int tpw) {
+  // (rows in LDS are padded as above)
+  constexpr int STRIDE = KS * 32 + 32, kRows = 32 * STRIDE + 64;
+  auto at = [](int kk) { return kk * STRIDE + (kk >> 3) * 16; };
+  constexpr int kThreads = kPromptWaves * kWave, kPieces = (32 * 4 * KS + kThreads - 1) / kThreads;
+  __shared__ __attribute__((aligned(16))) uint16_t rows0[2 * kRows];
+  __shared__ uint4 weights0[2 * NC * kWave];
+  __shared__ float shrink0[2 * NC * 16];
+  const int tid = threadIdx.x, lane = tid % kWave, j = lane % 16, g = lane / 16;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int t0 = (gridDim.x - 1 - blockIdx.x) * tpw, z = blockIdx.y;  // (the last tokens read the most rows: they start first)
+  const int t_last = min(t0 + tpw, n) - 1;
+  const int dtiles = (v_dim + 15) / 16;
+
+  // this lane's column of tile `wave`
+  const int col = wave * 16 + j, t = t0 + col / heads;
+  const bool scores = wave < NC, col_ok = scores && col < tpw * heads && t <= t_last;
+  const int pos = positions[min(t, t_last)], lo = first_key(pos, window, chunk);
+  LFrag qf[KS];
+  const bf16* qrow = q + (static_cast<size_t>(t0) * heads + (col_ok ? col : 0)) * key_dim;
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    qf[ks].u = make_uint4(0, 0, 0, 0);
+    const int d0 = ks * 32 + g * 8;
+    if (col_ok && d0 < key_dim) qf[ks].u = *reinterpret_cast<const uint4*>(qrow + d0);
+  }
+  // what lies behind a row's elements stays zero for the whole kernel
+  for (int i = tid; i < 2 * kRows / 8; i += kThreads) reinterpret_cast<uint4*>(rows0)[i] = make_uint4(0, 0, 0, 0);
+  __syncthreads();
+
+  bool same = true;
+  for (int i = t0 + 1; i <= t_last; ++i) same = same && token_seq[i] == token_seq[t0];
+  const int passes = same ? 1 : t_last - t0 + 1;
+  const int npieces = key_dim / 8;
+  const float scale2 = scale * 1.4426950408889634f;
+  float m = -INFINITY, l = 0.f;  // l: the lane's share of its column's sum until the end
+  lf32x4 o[DBW][NC];             // element 16 (wave + 8 x) + 4 g + r of column 16 c + j
+#pragma unroll
+  for (int x = 0; x < DBW; ++x)
+#pragma unroll
+    for (int c = 0; c < NC; ++c) o[x][c] = lf32x4{0.f, 0.f, 0.f, 0.f};
+
+  uint4 staged[kPieces];
+  int piece_row[kPieces], piece_col[kPieces];
+#pragma unroll
+  for (int u = 0; u < kPieces; ++u) {
+    const int idx = tid + u * kThreads;
+    piece_row[u] = idx < 32 * npieces ? idx / npieces : -1;
+    piece_col[u] = (idx % npieces) * 8;
+  }
+  const int page_shift = (page_size & (page_size - 1)) == 0 ? __ffs(page_size) - 1 : -1;
+  int buf = 0;
+  for (int pass = 0; pass < passes; ++pass) {
+    const int ta = same ? t0 : t0 + pass, tb = same ? t_last : t0 + pass;
+    const int stage_hi = positions[tb], stage_lo = first_key(positions[ta], window, chunk);
+    const int32_t* table = tables + static_cast<size_t>(token_seq[ta]) * table_stride;
+    const bool mine = col_ok && t >= ta && t <= tb;
+    const int key_begin = stage_lo & ~31;
+    const int nchunks = (stage_hi - key_begin) / 32 + 1;
+    const int per_split = (nchunks + nsplit - 1) / nsplit;
+    const int c_first = z * per_split, c_end = min(c_first + per_split, nchunks);
+    auto fetch = [&](int c) {
+      const int kb = key_begin + c * 32;
+#pragma unroll
+      for (int u = 0; u < kPieces; ++u) {
+        const int key = kb + piece_row[u];
+        staged[u] = make_uint4(0, 0, 0, 0);
+        if (piece_row[u] >= 0 && key >= stage_lo && key <= stage_hi) {
+          const int entry = page_shift >= 0 ? key >> page_shift : key / page_size;
+          const int slot = page_shift >= 0 ? key & (page_size - 1) : key % page_size;
+          const int page = table[entry];
+          if (page >= 0 && page < num_pages)
+            staged[u] = *reinterpret_cast<const uint4*>(
+                pool + (static_cast<size_t>(page) * page_size + slot) * key_dim + piece_col[u]);
+        }
+      }
+    };
+    if (c_first < c_end) fetch(c_first);
+    for (int c = c_first; c < c_end; ++c, buf ^= 1) {
+      const int kb = key_begin + c * 32;
+      uint16_t* const rows = rows0 + buf * kRows;
+      uint4* const weights = weights0 + buf * NC * kWave;
+      float* const shrink = shrink0 + buf * NC * 16;
+#pragma unroll
+      for (int u = 0; u < kPieces; ++u)
+        if (piece_row[u] >= 0) *reinterpret_cast<uint4*>(rows + at(piece_row[u]) + piece_col[u]) = staged[u];
+      __syncthreads();
+      if (scores) {
+        // row i of tile tt is row 8 (i / 4) + 4 tt + i % 4 of the chunk: the lane's eight scores belong to rows 8 g + e
+        lf32x4 s[2];
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt) {
+          s[tt] = lf32x4{0.f, 0.f, 0.f, 0.f};
+          const int kk = 8 * (j / 4) + 4 * tt + (j % 4);
+#pragma unroll
+          for (int ks = 0; ks < KS; ++ks) {
+            LFrag a;
+            a.u = *reinterpret_cast<const uint4*>(rows + at(kk) + ks * 32 + g * 8);
+            s[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.v, qf[ks].v, s[tt], 0, 0, 0);
+            if (ks % 8 == 7) __builtin_amdgcn_sched_barrier(0);  // (else operands of all steps are held at once)
+          }
+        }
+        float sc[8], mx = -INFINITY;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int key = kb + 8 * g + e;
+          sc[e] = (mine && key >= lo && key <= pos) ? s[e / 4][e % 4] * scale2 : -INFINITY;
+          mx = fmaxf(mx, sc[e]);
+        }
+        mx = quad_lanes_max(mx);
+        const float m_new = fmaxf(m, mx);
+        const float m_safe = (m_new == -INFINITY) ? 0.f : m_new;
+        const float alpha = __builtin_amdgcn_exp2f(m - m_safe);
+        float pr[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) pr[e] = __builtin_amdgcn_exp2f(sc[e] - m_safe);
+        l = l * alpha + (((pr[0] + pr[1]) + (pr[2] + pr[3])) + ((pr[4] + pr[5]) + (pr[6] + pr[7])));
+        m = m_new;
+        LFrag pf;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) pf.v[e] = static_cast<__bf16>(pr[e]);
+        weights[wave * kWave + lane] = pf.u;
+        if (g == 0) shrink[col] = alpha;
+      }
+      if (c + 1 < c_end) fetch(c + 1);  // (behind the scores: their operands leave no registers for it)
+      __syncthreads();
+      lu32x4 vw[DBW];
+      const uint16_t* vrows = rows + at(8 * g) + j;  // rows 8 g .. 8 g + 7 lie STRIDE apart
+#pragma unroll
+      for (int x = 0; x < DBW; ++x)
+#pragma unroll
+        for (int e2 = 0; e2 < 4; ++e2)
+          vw[x][e2] = static_cast<uint32_t>(vrows[(2 * e2) * STRIDE + (wave + 8 * x) * 16]) |
+                      (static_cast<uint32_t>(vrows[(2 * e2 + 1) * STRIDE + (wave + 8 * x) * 16]) << 16);
+#pragma unroll
+      for (int cc = 0; cc < NC; ++cc) {
+        LFrag pf;
+        pf.u = weights[cc * kWave + lane];
+        const float alpha = shrink[cc * 16 + j];
+        if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {  // some column's maximum rose
+#pragma unroll
+          for (int x = 0; x < DBW; ++x) o[x][cc] *= alpha;
+        }
+#pragma unroll
+        for (int x = 0; x < DBW; ++x)
+          o[x][cc] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(lbf16x8, vw[x]), pf.v, o[x][cc], 0, 0, 0);
+      }
+    }
+  }
+  l = quad_lanes_sum(l);
+  __syncthreads();
+  float* const sums = shrink0;  // [16 NC], and behind them the maxima
+  if (scores && g == 0) {
+    sums[col] = l;
+    sums[NC * 16 + col] = m;
+  }
+  __syncthreads();
+  const size_t all_rows = static_cast<size_t>(n) * heads;
+#pragma unroll
+  for (int cc = 0; cc < NC; ++cc) {
+    const int c = cc * 16 + j;
+    if (c >= tpw * heads || t0 + c / heads > t_last) continue;
+    const size_t row = static_cast<size_t>(t0) * heads + c;
+    const float inv = 1.f / sums[c];
+#pragma unroll
+    for (int x = 0; x < DBW; ++x) {
+      const int d = (wave + 8 * x) * 16 + 4 * g;
+      if (wave + 8 * x >= dtiles) continue;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        if (d + r >= v_dim) continue;
+        if (nsplit == 1)
+          out[row * v_dim + d + r] = from_float<bf16>(o[x][cc][r] * inv);
+        else
+          partial[(row * nsplit + z) * v_dim + d + r] = o[x][cc][r];
+      }
+    }
+    if (nsplit > 1 && wave == 0 && g == 0) {
+      float* ml = partial + all_rows * nsplit * v_dim + (row * nsplit + z) * 2;
+      ml[0] = sums[NC * 16 + c];
+      ml[1] = sums[c];
+    }
+  }
+}
+
 // out[row][:] = sum_z 2^(m_z - M) O_z / sum_z 2^(m_z - M) l_z, shares in order; one wavefront a row.
 __global__ void __launch_bounds__(kWave)
     latent_merge_kernel(const float* __restrict__ partial, bf16* __restrict__ out, int nsplit, int v_dim) {
@@ -286,6 +491,51 @@ static void launch_latent(dim3 grid, hipStream_t s, const bf16* q, bf16* out, in
 }  // namespace shk
 
 using namespace shk;
+
+// Tokens a workgroup of latent_prompt_kernel serves, 0 where it does not take the shape: rows of up to 512
+// elements, and as many whole tokens as fit into its columns.
+extern "C" int shk_latent_prompt_tokens(int heads, int key_dim, int v_dim) {
+  if (!shk_latent_attention_supports_mfma(heads, key_dim, v_dim) || key_dim > 512) return 0;
+  return (v_dim > 256 ? 112 : 128) / heads;
+}
+
+// The same for tokens of prompt portions, `positions` rising along each.
+extern "C" int shk_latent_prompt_bf16(const void* q, void* out, int n, int heads, int key_dim, int v_dim,
+                                      const int32_t* positions, const int32_t* token_seq, const int32_t* tables,
+                                      int table_stride, const void* pool, int page_size, int num_pages, int window, int chunk,
+                                      float scale, float* partial, int nsplit, void* stream) {
+  const int tpw = shk_latent_prompt_tokens(heads, key_dim, v_dim);
+  SHK_REQUIRE(tpw > 0, "latent_prompt_bf16: %d heads over rows of %d with values of %d are not served", heads, key_dim, v_dim);
+  SHK_REQUIRE(n >= 0 && n <= 1 << 30 && nsplit >= 1 && nsplit <= 64, "latent_prompt_bf16: bad sizes n=%d nsplit=%d", n, nsplit);
+  SHK_REQUIRE(page_size > 0 && num_pages > 0 && table_stride > 0,
+              "latent_prompt_bf16: bad cache sizes page_size=%d num_pages=%d table_stride=%d", page_size, num_pages, table_stride);
+  if (n == 0) return 0;
+  SHK_REQUIRE(q && out && positions && token_seq && tables && pool && (partial || nsplit == 1), "latent_prompt_bf16: null pointer");
+  SHK_REQUIRE(reinterpret_cast<uintptr_t>(q) % 16 == 0 && reinterpret_cast<uintptr_t>(pool) % 16 == 0,
+              "latent_prompt_bf16: q and the pool must be 16-byte aligned");
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const dim3 grid((n + tpw - 1) / tpw, nsplit);
+  auto go = [&](auto ks, auto dbw, auto nc) {
+    constexpr int KS = decltype(ks)::value, DBW = decltype(dbw)::value, NC = decltype(nc)::value;
+    latent_prompt_kernel<KS, DBW, NC><<<grid, kPromptWaves * kWave, 0, s>>>(
+        static_cast<const bf16*>(q), static_cast<bf16*>(out), heads, key_dim, v_dim, positions, token_seq, tables, table_stride,
+        static_cast<const bf16*>(pool), page_size, num_pages, window, chunk, scale, partial, nsplit, n, tpw);
+  };
+  using std::integral_constant;
+  const int ks = (key_dim + 31) / 32, db = (v_dim + 15) / 16;
+  if (ks <= 8 && db <= 8)
+    go(integral_constant<int, 8>{}, integral_constant<int, 1>{}, integral_constant<int, 8>{});
+  else if (ks <= 8)
+    go(integral_constant<int, 8>{}, integral_constant<int, 2>{}, integral_constant<int, 8>{});
+  else if (db <= 16)
+    go(integral_constant<int, 16>{}, integral_constant<int, 2>{}, integral_constant<int, 8>{});
+  else
+    go(integral_constant<int, 16>{}, integral_constant<int, 4>{}, integral_constant<int, 7>{});
+  if (nsplit > 1)
+    latent_merge_kernel<<<static_cast<unsigned>(n) * heads, kWave, 0, s>>>(partial, static_cast<bf16*>(out), nsplit, v_dim);
+  SHK_LAUNCH_CHECK("latent_prompt_bf16");
+  return 0;
+}
 
 // 1 if the matrix-instruction kernel takes the shape: rows of up to 640 elements in multiples of
 // 8, values no larger than rows, up to 128 heads.

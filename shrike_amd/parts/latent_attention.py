@@ -83,28 +83,38 @@ class LatentAttention(Mixer):
         key = ("latent_attention", s.num_heads, s.kv_rank, s.rot_dim, s.window, s.chunk)
         if key in shape.notes:
             return
-        nsplit = 1
-        if self.mfma:
-            tokens, reach = 1, int(shape.ctx_lens.max())
-            while tokens < shape.num_tokens:
+        bounds = [int(b) for b in (s.window, s.chunk) if b]
+
+        def shares(workgroups, rows, least):
+            """Workgroups a token's rows are shared among: twice the compute units in all, `least` rows each."""
+            tokens, keys = 1, 64
+            while tokens < workgroups:
                 tokens *= 2
-            for bound in (s.window, s.chunk):
-                if bound:
-                    reach = min(reach, bound)
-            keys = 64
-            while keys < reach:
+            while keys < min([rows, *bounds]):
                 keys *= 2
-            nsplit = max(1, min(2 * compute_units() // tokens, keys // 128, 64))
-        # a step with prompt portions: neighbouring tokens may share a workgroup (and what it stages)
-        group = 1 if shape.num_decode == shape.num_seqs else 4
-        shape.notes[key] = (nsplit, group)
-        shape.launch_key.append((key, nsplit, group))
+            return max(1, min(2 * compute_units() // tokens, keys // least, 64))
+
+        # prompt portions in a kernel of their own where it takes the shape; else every token alike
+        # (neighbouring tokens of a step with portions may share a workgroup and what it stages)
+        nsplit, group, first, prompt_split = 1, 1, shape.num_tokens, 1
+        if self.mfma:
+            if self.prompt_tokens and shape.num_decode < shape.num_seqs:
+                first = shape.num_decode
+                prompt_split = shares(-(-(shape.num_tokens - first) // self.prompt_tokens), int(shape.ctx_lens[first:].max()), 512)
+                if first:
+                    nsplit = shares(first, int(shape.ctx_lens[:first].max()), 128)
+            else:
+                nsplit = shares(shape.num_tokens, int(shape.ctx_lens.max()), 128)
+                group = 1 if shape.num_decode == shape.num_seqs else 4
+        shape.notes[key] = (nsplit, group, first, prompt_split)
+        shape.launch_key.append((key, nsplit, group, first, prompt_split))
 
     def load(self, tensors, runtime):
         s = self.spec
         H = s.num_heads
         self.mfma = runtime.dtype == torch.bfloat16 and ops.latent_attention_supports_mfma(
             H, s.kv_rank + s.rot_dim, s.kv_rank)
+        self.prompt_tokens = ops.latent_prompt_tokens(H, s.kv_rank + s.rot_dim, s.kv_rank) if self.mfma else 0
         self.w_down = runtime.weight(torch.cat([tensors[self._t("dq")], tensors[self._t("dkv")]], dim=0))
         self.q_norm = tensors[self._t("dq.norm")]
         self.kv_norm = tensors[self._t("dkv.norm")]
@@ -153,13 +163,20 @@ class LatentAttention(Mixer):
                          ctx.positions, magnitude=self.magnitude)
         mixed = ctx.buffer("latent_mixed", (n, H * s.kv_rank), ctx.dtype)
         if self.mfma:
-            nsplit, group = ctx.notes[("latent_attention", H, s.kv_rank, s.rot_dim, s.window, s.chunk)]
-            partial = None
-            if nsplit > 1:
-                partial = ctx.buffer("latent_partial", (n * H * nsplit * (s.kv_rank + 2),), torch.float32)
-            ops.latent_attention_mfma(folded, mixed, H, key_dim, s.kv_rank, ctx.positions, ctx.token_seq, tables,
-                                      cache.pools["latent"], cache.page_size, s.window, s.scale, chunk=s.chunk,
-                                      partial=partial, nsplit=nsplit, tokens_per_group=group)
+            nsplit, group, first, prompt_split = ctx.notes[("latent_attention", H, s.kv_rank, s.rot_dim, s.window, s.chunk)]
+
+            def attend(kernel, lo, hi, shares, **more):
+                partial = None
+                if shares > 1:
+                    partial = ctx.buffer("latent_partial" if lo == 0 else "latent_prompt_partial", ((hi - lo) * H * shares * (s.kv_rank + 2),), torch.float32)
+                kernel(folded[lo:hi], mixed[lo:hi], H, key_dim, s.kv_rank, ctx.positions[lo:hi], ctx.token_seq[lo:hi], tables,
+                       cache.pools["latent"], cache.page_size, s.window, s.scale, chunk=s.chunk, partial=partial, nsplit=shares,
+                       **more)
+
+            if first:
+                attend(ops.latent_attention_mfma, 0, first, nsplit, tokens_per_group=group)
+            if first < n:
+                attend(ops.latent_prompt, first, n, prompt_split)
         else:
             ops.latent_attention(folded, mixed, H, key_dim, s.kv_rank, ctx.positions, ctx.token_seq, tables,
                                  cache.pools["latent"], cache.page_size, s.window, s.scale, chunk=s.chunk)

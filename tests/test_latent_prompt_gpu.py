@@ -1,0 +1,48 @@
+"""Latent attention of prompt portions: portions of several sequences whose ends fall within a workgroup's
+tokens, rows and values of every size class, windows and block-local masks, rows shared among workgroups,
+not-numbers wherever nothing may be read."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("heads, key_dim, v_dim, page, window, chunk", [
+    (28, 512, 448, 16, None, None), (14, 160, 128, 16, None, None), (3, 40, 24, 4, None, 64), (64, 264, 200, 32, 70, None),
+    (112, 512, 500, 16, None, None), (1, 8, 3, 8, 33, None), (17, 256, 256, 64, None, None), (128, 320, 250, 16, 100, 128),
+])
+@pytest.mark.parametrize("nsplit", [1, 3])
+def test_against_float64(heads, key_dim, v_dim, page, window, chunk, nsplit):
+    from shrike_amd.kernels import ops
+
+    assert ops.latent_prompt_tokens(heads, key_dim, v_dim) >= 1
+    torch.manual_seed(heads + key_dim)
+    starts, lengths = [0, 61, 0, 130], [45, 7, 1, 35]  # (one-token portions are served too)
+    n, ctx = sum(lengths), [s + k for s, k in zip(starts, lengths)]
+    per = -(-max(ctx) // page)
+    pool = torch.full((4 * per + 1, page, key_dim), float("nan"), device="cuda", dtype=torch.bfloat16)
+    tables = torch.randperm(4 * per + 1)[: 4 * per].view(4, per).int()
+    rows = [torch.randn(c, key_dim).bfloat16() for c in ctx]
+    for s, r in enumerate(rows):
+        at = torch.arange(r.shape[0])
+        pool[tables[s].long()[at // page].cuda(), (at % page).cuda()] = r.cuda()
+    q = torch.randn(n, heads, key_dim).bfloat16()
+    positions = torch.cat([torch.arange(s, s + k) for s, k in zip(starts, lengths)])
+    seqs = torch.repeat_interleave(torch.arange(4), torch.tensor(lengths))
+    scale = 0.7 / key_dim**0.5
+    out = torch.full((n, heads * v_dim), float("nan"), device="cuda", dtype=torch.bfloat16)
+    partial = torch.full((n * heads * nsplit * (v_dim + 2),), float("nan"), device="cuda")
+    ops.latent_prompt(q.view(n, -1).cuda(), out, heads, key_dim, v_dim, positions.int().cuda(), seqs.int().cuda(), tables.cuda(),
+                      pool, page, window, scale, chunk=chunk, partial=partial, nsplit=nsplit)
+    got = out.view(n, heads, v_dim).double().cpu()
+    for t in range(n):
+        p = int(positions[t])
+        lo = max(0, p - window + 1) if window else 0
+        lo = max(lo, p // chunk * chunk) if chunk else lo
+        r = rows[int(seqs[t])][lo : p + 1].double()
+        w = torch.softmax(q[t].double() @ r.T * scale, -1)
+        want = w @ r[:, :v_dim]
+        # weights and the result are rounded to bfloat16 (2^-9 each, the weights' sizes adding up to one)
+        bound = 2.0**-7 * (w @ r[:, :v_dim].abs()) + 1e-3
+        assert bool(((got[t] - want).abs() <= bound).all()), t
