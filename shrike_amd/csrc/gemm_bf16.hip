@@ -915,6 +915,96 @@ __global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per
 }
 
 
+// gemm_direct_kernel: for small matrices (cached by the time that a few hundred wavefronts ask for them) and
+// from 17 tokens on: nothing is staged.  A wavefront forms RT x CT tiles of 16 weight rows x 16 tokens with both
+// operands straight from memory, U tiles of k asked for ahead; KW wavefronts share a tile's k, each a run of it, and
+// meet in LDS once at the end (in order); MW x NW such groups make a workgroup.  Such products are a matter of
+// latency: 896 x 896 at 128 / 512 / 1,119 tokens took 16.6 / 16.5 / 17.0 us in the LDS-staged kernel, whose 7
+// to 63 workgroups met at 14 barriers, and takes 4.7 / 8.1 / 11.8; 64 tokens 7.5 us in three shares of the
+// streaming kernel, 4.6 whole.  896 x 4864 at 64 / 128 tokens: 9.4 in eight shares and 17.5 in nine against 7.4 in
+// two and 10.3 whole.  With larger matrices it loses by far (7B gate/up at 512 tokens 370 us against 161):
+// every tile fetches its operands for itself.
+template <int RT, int CT, int KW, int U>
+__global__ void __launch_bounds__(kWave* KW)
+    gemm_direct_kernel(const bf16* __restrict__ a, int lda, int n, int k, const uint4* __restrict__ wt, int ktiles, int m,
+                       const float* __restrict__ bias, void* __restrict__ out, int ldo, int out_f32, int accumulate,
+                       int ksplit) {
+  constexpr int kTiles = RT * CT;
+  const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int j = lane % 16, kg = lane / 16;
+  const int mblocks = (m + 15) / 16;
+  // workgroup -> tile: each die takes a run of tiles, the tokens innermost
+  const int rows = (n + 16 * CT - 1) / (16 * CT), cols = (mblocks + RT - 1) / RT;
+  const int per_die = (rows * cols + kDies - 1) / kDies;
+  const int tile = blockIdx.x % kDies * per_die + blockIdx.x / kDies;
+  if (blockIdx.x / kDies >= per_die || tile >= rows * cols) return;
+  const int mb0 = tile / rows * RT, tok0 = tile % rows * CT * 16;
+  // this wavefront's k tiles: of the workgroup's share a run of its own
+  const int share = (ktiles + ksplit - 1) / ksplit, sbegin = min(static_cast<int>(blockIdx.y) * share, ktiles);
+  const int send = min(sbegin + share, ktiles);
+  const int per = (send - sbegin + KW - 1) / KW, begin = min(sbegin + wave * per, send), end = min(begin + per, send);
+
+  const u32x4* wr[RT];
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+    wr[r] = reinterpret_cast<const u32x4*>(wt) + static_cast<size_t>(min(mb0 + r, mblocks - 1)) * ktiles * kWave + lane;
+  const bf16* ar[CT];
+#pragma unroll
+  for (int c = 0; c < CT; ++c) ar[c] = a + static_cast<size_t>(min(tok0 + c * 16 + j, n - 1)) * lda;
+  f32x4 acc[RT][CT];
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int c = 0; c < CT; ++c) acc[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (begin < end) {
+    u32x4 wv[2][U][RT], av[2][U][CT];
+    auto load = [&](int set, int t0) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {  // (unconditional: a tile beyond the run's last is the last again)
+        const int t = min(t0 + u, end - 1), col = t * 32 + kg * 8;
+#pragma unroll
+        for (int r = 0; r < RT; ++r) wv[set][u][r] = wr[r][static_cast<size_t>(t) * kWave];
+#pragma unroll
+        // (a piece beyond k: the row's first 16 bytes, numbers that meet the weight tiles' zeros)
+        for (int c = 0; c < CT; ++c) av[set][u][c] = *reinterpret_cast<const u32x4*>(ar[c] + (col < k ? col : 0));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto multiply = [&](const u32x4(&w)[RT], const u32x4(&x)[CT]) {
+#pragma unroll
+      for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int c = 0; c < CT; ++c)
+          acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w[r]), __builtin_bit_cast(bf16x8, x[c]),
+                                                              acc[r][c], 0, 0, 0);
+    };
+    load(0, begin);
+    for (int t = begin; t < end; t += 2 * U) {
+      load(1, t + U);
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (t + u < end) multiply(wv[0][u], av[0][u]);
+      load(0, t + 2 * U);
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (t + U + u < end) multiply(wv[1][u], av[1][u]);
+    }
+  }
+  __shared__ f32x4 sums[KW][kTiles][kWave];
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int c = 0; c < CT; ++c) sums[wave][r * CT + c][lane] = acc[r][c];
+  __syncthreads();
+  for (int p = wave; p < kTiles; p += KW) {
+    f32x4 one[1][1];
+    one[0][0] = sums[0][p][lane];
+#pragma unroll
+    for (int x = 1; x < KW; ++x) one[0][0] += sums[x][p][lane];
+    big_store<1, 1, false>(one, lane, tok0 + p % CT * 16, mb0 + p / CT, n, m, bias, out, ldo, out_f32, accumulate, blockIdx.y);
+  }
+}
+
 // gemm_stream_kernel: for 17 to 64 tokens whose rows are 16-byte aligned with
 // k % 8 == 0.  Such a product is bound by the stream of weights, like the skinny
 // one, but its activations (up to 64 x k) are too many to fetch once per block of
@@ -1330,6 +1420,37 @@ static int big_shape(int split, int n, int wblocks, int m, int k) {
 
 extern "C" int shk_gemm_bf16_splits(int n, int m, int k);
 
+// Which gemm_direct_kernel serves a product of n > 16 tokens (0: none): the smallest tile of which a launch has no
+// more than the 256 compute units (64 x 64: two a unit).  Limits as measured with k = 896 and 4864: matrices of 256
+// to 2,048 rows (more of them fill the staged kernels' larger tiles) and up to 10 MB; the two larger tiles only for a short k (4864 at 300 tokens: 23.5 us against 20.7).  Up to 256 tokens n counts as
+// the power of two above it: the choice is then the same for every number of tokens that a captured decode step may
+// stand for.
+struct DirectTile {
+  int rows, tokens, most;
+};
+static const DirectTile kDirect[5] = {{0, 0, 0}, {32, 16, 256}, {32, 32, 256}, {32, 64, 256}, {64, 64, 512}};
+
+static int direct_shape(int n, int m, int k, int ksplit) {
+  if (n <= 16 || m < 256 || m > 2048 || static_cast<long long>(m) * k > 5 * 1000 * 1000) return 0;
+  int tokens = n;
+  if (n <= 256)
+    for (tokens = 32; tokens < n;) tokens *= 2;
+  for (int shape = 1; shape <= (k <= 2048 ? 4 : 2); ++shape) {
+    const DirectTile& t = kDirect[shape];
+    const long long count = static_cast<long long>((m + t.rows - 1) / t.rows) * ((tokens + t.tokens - 1) / t.tokens);
+    if (count * ksplit <= t.most) return shape;
+  }
+  return 0;
+}
+
+template <int RT, int CT, int KW, int U>
+static void launch_direct(hipStream_t s, const bf16* ap, int lda, int n, int k, const uint4* wp, int kt, int m, const float* bias,
+                          void* out, int ldo, int of, int accumulate, int ksplit) {
+  const int tiles = ((n + 16 * CT - 1) / (16 * CT)) * (((m + 15) / 16 + RT - 1) / RT);
+  gemm_direct_kernel<RT, CT, KW, U><<<dim3((tiles + kDies - 1) / kDies * kDies, ksplit), KW * kWave, 0, s>>>(
+      ap, lda, n, k, wp, kt, m, bias, out, ldo, of, accumulate, ksplit);
+}
+
 // Matrices of so few rows that many tokens go to gemm_skinny_kernel, group by group.
 static bool few_rows(int m) { return m <= 64; }
 
@@ -1355,7 +1476,7 @@ static int big_main_blocks(int shape, int n, int wblocks, int m, int k, int gate
 
 // Products that a call with these sizes is made of (1, or 2: see big_main_blocks).
 extern "C" int shk_gemm_bf16_parts(int n, int m, int k, int gated) {
-  if (n <= 64 || (few_rows(m) && !gated) || shk_gemm_bf16_splits(n, m, k) > 1) return 1;
+  if (n <= 64 || (!gated && (few_rows(m) || direct_shape(n, m, k, 1))) || shk_gemm_bf16_splits(n, m, k) > 1) return 1;
   const int wblocks = (gated ? 2 : 1) * ((m + 15) / 16);
   return big_main_blocks(big_shape(1, n, wblocks, m, k), n, wblocks, m, k, gated) ? 2 : 1;
 }
@@ -1363,6 +1484,10 @@ extern "C" int shk_gemm_bf16_parts(int n, int m, int k, int gated) {
 extern "C" int shk_gemm_bf16_splits(int n, int m, int k) {
   const int mblocks = (m + 15) / 16, ktiles = (k + 31) / 32;
   if (n > 64 && few_rows(m)) return 1;
+  // (a long k in two shares up to 64 tokens: 896 x 4864 7.4 us against 10.0 whole, the second share costs its reader
+  // half a microsecond)
+  const int direct = n <= 64 && k > 2048 ? 2 : 1;
+  if (direct_shape(n, m, k, direct)) return direct;
   if (n > 64) {
     // many tokens: the number of shares, each of at least 8 stages of 64, that
     // big_estimate() expects to be fastest with the tile shape that suits it
@@ -1449,6 +1574,16 @@ extern "C" int shk_gemm_bf16_tiled_weight(const void* a, const void* wt, const f
   if (n > 64 && few_rows(m) && !gated && ksplit == 1 && n <= 65535 * 16) {
     gemm_skinny_kernel<1, 16, kSingle><<<dim3(mb, 1, (n + 15) / 16), 16 * kWave, 0, s>>>(
         ap, lda, n, k, wp, kt, m, bias, out, ldo, of, accumulate, vec, 1);
+    SHK_LAUNCH_CHECK("gemm_bf16");
+    return 0;
+  }
+  const int direct = !gated && vec && reinterpret_cast<uintptr_t>(out) % 8 == 0 ? direct_shape(n, m, k, ksplit) : 0;
+  if (direct) {
+    const auto go = direct == 1   ? launch_direct<2, 1, 8, 2>
+                    : direct == 2 ? launch_direct<2, 2, 4, 2>
+                    : direct == 3 ? launch_direct<2, 4, 8, 1>
+                                  : launch_direct<4, 4, 4, 1>;
+    go(s, ap, lda, n, k, wp, kt, m, bias, out, ldo, of, accumulate, ksplit);
     SHK_LAUNCH_CHECK("gemm_bf16");
     return 0;
   }

@@ -31,6 +31,36 @@ def test_few_rows_many_tokens(n, m, k):
         assert torch.equal(few, half[3:])
 
 
+@pytest.mark.parametrize("m, k", [(896, 896), (1152, 896), (256, 40), (896, 4864), (1000, 2056), (300, 8192)])
+def test_small_matrices_without_staging(m, k):
+    """Every tile that serves small matrices from 17 tokens on (and what serves them beyond), whole and in shares."""
+    from shrike_amd.kernels import ops
+
+    torch.manual_seed(m + k)
+    n_max = 1200
+    a, w = torch.randn(n_max, k, device="cuda").bfloat16(), torch.randn(m, k, device="cuda").bfloat16()
+    bias, wt = torch.randn(m, device="cuda"), ops.retile_weight(w)
+    want = a.double() @ w.double().t()
+    size = a.double().abs() @ w.double().abs().t()
+    bound = (k / 32 + 48) * 2.0**-24
+    for n in (17, 32, 33, 64, 65, 128, 129, 256, 300, 511, 1200):
+        out = torch.full((n, m), 7.0, device="cuda")
+        ops.gemm_tiled_weight(a[:n], wt, m, k, out, bias=bias)
+        off = (out.double() - want[:n] - bias.double()).abs()
+        assert bool((off <= bound * (size[:n] + bias.double().abs())).all()), n
+        half = torch.empty(n, m, device="cuda", dtype=torch.bfloat16)
+        ops.gemm_tiled_weight(a[:n], wt, m, k, half, bias=bias)
+        assert torch.equal(half, out.bfloat16()), n
+        splits = max(2, ops.gemm_splits(n, m, k))
+        parts = torch.full((splits, n, m), float("nan"), device="cuda")
+        ops.gemm_tiled_weight(a[:n], wt, m, k, parts, splits=splits)
+        assert bool(((parts.double().sum(0) - want[:n]).abs() <= bound * size[:n]).all()), n
+        if n == 64:  # a captured step stands for every batch up to its own size
+            few = torch.empty(41, m, device="cuda")
+            ops.gemm_tiled_weight(a[:41], wt, m, k, few, bias=bias)
+            assert torch.equal(few, out[:41])
+
+
 @pytest.mark.parametrize("batch, m, k", [(3, 40, 8), (28, 448, 128), (5, 130, 200), (14, 512, 256), (2, 3, 40), (1, 64, 24)])
 def test_batched_products_of_every_shape(batch, m, k):
     from shrike_amd.kernels import ops
