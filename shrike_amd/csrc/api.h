@@ -213,13 +213,14 @@ int shk_attention_supports_mfma(int heads, int kv_heads, int head_dim, int page_
 // `partial` is float32 scratch of num_seqs * heads * nsplit * (head_dim + 2).
 // streaming != 0: keys and values are fetched with non-temporal loads (faster when a
 // launch reads tens of megabytes of them, slightly slower below; the result is the same).
+// waves: wavefronts a workgroup, 4, or 8 for heads of up to 64 elements.
 // softcap / sinks / dist_bias as in shk_attention (0 and null: none).
 int shk_attention_decode_bf16(const void* q, int q_stride, void* out, int num_seqs, int heads,
                               int kv_heads, int head_dim, const int32_t* positions,
                               const int32_t* tables, int table_stride, const void* k_pool,
                               const void* v_pool, int page_size, int window, int chunk, float scale,
-                              float* partial, int nsplit, int streaming, float softcap, const float* sinks,
-                              const float* dist_bias, int bias_rows, void* stream);
+                              float* partial, int nsplit, int streaming, int waves, float softcap,
+                              const float* sinks, const float* dist_bias, int bias_rows, void* stream);
 
 // bfloat16 attention for prompt portions, in tiles of 16 queries: tile i covers
 // queries tile_q0[i] .. +16 of sequence tile_seq[i]'s portion.  cu_q[s] is the

@@ -285,11 +285,12 @@ __device__ __forceinline__ void attend_tile(const TileArgs& ta, const AFrag (&qf
 }
 
 // ------------------------------------------------------------------- decode
-// grid (kv_heads, sequences, splits), kDecodeWaves wavefronts per workgroup.  A
+// grid (kv_heads, sequences, splits), WAVES wavefronts per workgroup.  A
 // single wavefront needs about 1,700 cycles for a chunk of 32 keys whatever the
 // memory does, so a workgroup's key range is dealt out to its wavefronts chunk
 // by chunk, and their results are combined through LDS before anything is
-// written.
+// written.  Four wavefronts, or eight for up to 512 keys of a short context
+// that would else be two splits (the caller's rule).
 //
 // The two products are formed transposed, so that a lane owns one query head
 // throughout and nothing passes through LDS:
@@ -309,7 +310,6 @@ __device__ __forceinline__ void attend_tile(const TileArgs& ta, const AFrag (&qf
 // the caller says which it wants.
 
 constexpr int kMaxSplits = 64;
-constexpr int kDecodeWaves = 4;
 
 template <int D>
 struct DecodeChunk {
@@ -317,8 +317,8 @@ struct DecodeChunk {
   AFrag v[D / 16];
 };
 
-template <int D, bool NT>
-__global__ void __launch_bounds__(kDecodeWaves* kWave)
+template <int D, bool NT, int WAVES>
+__global__ void __launch_bounds__(WAVES* kWave)
     attention_decode_kernel(const bf16* __restrict__ q, int q_stride, bf16* __restrict__ out,
                             int heads, int kv_heads, const int32_t* __restrict__ positions,
                             const int32_t* __restrict__ tables, int table_stride,
@@ -326,9 +326,9 @@ __global__ void __launch_bounds__(kDecodeWaves* kWave)
                             int page_size, uint32_t page_magic, int window, int block, float scale,
                             float* __restrict__ partial, int nsplit, ScoreOpts so) {
   constexpr int NBUF = 2;  // chunk buffers: one computed, one in flight
-  constexpr int kStep = 32 * kDecodeWaves;  // keys between two chunks of one wavefront
-  __shared__ float m_lds[kDecodeWaves][16], l_lds[kDecodeWaves][16];
-  __shared__ float4 o_lds[kDecodeWaves - 1][D / 16][kWave];
+  constexpr int kStep = 32 * WAVES;  // keys between two chunks of one wavefront
+  __shared__ float m_lds[WAVES][16], l_lds[WAVES][16];
+  __shared__ float4 o_lds[WAVES - 1][D / 16][kWave];
   const int kvh = blockIdx.x, seq = blockIdx.y, z = blockIdx.z;
   const int wave = threadIdx.x / kWave;
   const int lane = threadIdx.x % kWave, j = lane % 16, g = lane / 16;
@@ -516,11 +516,11 @@ __global__ void __launch_bounds__(kDecodeWaves* kWave)
   __syncthreads();
   float m_all = m_lds[0][j];
 #pragma unroll
-  for (int w = 1; w < kDecodeWaves; ++w) m_all = fmaxf(m_all, m_lds[w][j]);
+  for (int w = 1; w < WAVES; ++w) m_all = fmaxf(m_all, m_lds[w][j]);
   const float m_ref = (m_all == -INFINITY) ? 0.f : m_all;
   l = 0.f;
 #pragma unroll
-  for (int w = 0; w < kDecodeWaves; ++w)
+  for (int w = 0; w < WAVES; ++w)
     l += l_lds[w][j] * __builtin_amdgcn_exp2f(m_lds[w][j] - m_ref);  // 2^-inf = 0: nothing seen
   const float mine = __builtin_amdgcn_exp2f(m - m_ref);
   m = m_all;
@@ -534,7 +534,7 @@ __global__ void __launch_bounds__(kDecodeWaves* kWave)
   __syncthreads();
   if (wave > 0 || j >= group) return;
 #pragma unroll
-  for (int w = 0; w < kDecodeWaves - 1; ++w)
+  for (int w = 0; w < WAVES - 1; ++w)
 #pragma unroll
     for (int db = 0; db < D / 16; ++db) {
       const float4 x = o_lds[w][db][lane];
@@ -1000,16 +1000,14 @@ static void launch_decode(dim3 grid, hipStream_t s, const bf16* q, int q_stride,
                           int heads, int kv_heads, const int32_t* positions, const int32_t* tables,
                           int table_stride, const bf16* k_pool, const bf16* v_pool, int page_size,
                           int window, int block, float scale, float* partial, int nsplit, int streaming,
-                          ScoreOpts so) {
+                          int waves, ScoreOpts so) {
   const uint32_t magic = static_cast<uint32_t>(((1ull << 32) + page_size - 1) / page_size);
-  if (streaming)
-    attention_decode_kernel<D, true><<<grid, kDecodeWaves * kWave, 0, s>>>(
-        q, q_stride, out, heads, kv_heads, positions, tables, table_stride, k_pool, v_pool, page_size,
-        magic, window, block, scale, partial, nsplit, so);
-  else
-    attention_decode_kernel<D, false><<<grid, kDecodeWaves * kWave, 0, s>>>(
-        q, q_stride, out, heads, kv_heads, positions, tables, table_stride, k_pool, v_pool, page_size,
-        magic, window, block, scale, partial, nsplit, so);
+  auto kernel = streaming ? attention_decode_kernel<D, true, 4> : attention_decode_kernel<D, false, 4>;
+  if constexpr (D <= 64)
+    if (waves == 8) kernel = streaming ? attention_decode_kernel<D, true, 8> : attention_decode_kernel<D, false, 8>;
+  kernel<<<grid, waves * kWave, 0, s>>>(q, q_stride, out, heads, kv_heads, positions, tables, table_stride,
+                                                         k_pool, v_pool, page_size, magic, window, block, scale, partial,
+                                                         nsplit, so);
   if (nsplit > 1)
     attention_merge_kernel<D><<<grid.y * heads, kWave, 0, s>>>(partial, out, nsplit, so.sinks, heads);
 }
@@ -1098,8 +1096,10 @@ extern "C" int shk_attention_decode_bf16(const void* q, int q_stride, void* out,
                                          const int32_t* positions, const int32_t* tables,
                                          int table_stride, const void* k_pool, const void* v_pool,
                                          int page_size, int window, int block, float scale, float* partial,
-                                         int nsplit, int streaming, float softcap, const float* sinks,
-                                         const float* dist_bias, int bias_rows, void* stream) {
+                                         int nsplit, int streaming, int waves, float softcap,
+                                         const float* sinks, const float* dist_bias, int bias_rows, void* stream) {
+  SHK_REQUIRE(waves == 4 || (waves == 8 && head_dim <= 64),
+              "attention_decode: workgroups of 4 wavefronts, or of 8 for heads of up to 64 elements; got %d for %d", waves, head_dim);
   SHK_REQUIRE(softcap >= 0.f, "attention_decode: a score cap must be positive (0: none), got %g", softcap);
   SHK_REQUIRE(!dist_bias || bias_rows > 0, "attention_decode: a distance bias needs a table of at least one row");
   const ScoreOpts so = score_opts(scale, softcap, sinks, dist_bias, bias_rows);
@@ -1123,7 +1123,7 @@ extern "C" int shk_attention_decode_bf16(const void* q, int q_stride, void* out,
   launch_decode<D>(grid, s, static_cast<const bf16*>(q), q_stride, static_cast<bf16*>(out), heads, \
                    kv_heads, positions, tables, table_stride, static_cast<const bf16*>(k_pool),    \
                    static_cast<const bf16*>(v_pool), page_size, window, block, scale, partial, nsplit,    \
-                   streaming, so)
+                   streaming, waves, so)
   SHK_DISPATCH_D(head_dim, CALL)
 #undef CALL
   SHK_LAUNCH_CHECK("attention_decode");

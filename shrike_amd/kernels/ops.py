@@ -1358,8 +1358,9 @@ def _sinks(sinks, heads, who):
 
 def attention_decode(q, out, num_seqs, heads, kv_heads, head_dim, positions, tables, k_pool, v_pool,
                      page_size, window, scale, partial, nsplit, streaming=False, chunk=None, softcap=None,
-                     sinks=None, dist_bias=None) -> None:
+                     sinks=None, dist_bias=None, waves: int = 4) -> None:
     """bfloat16 MFMA attention for the first num_seqs rows of q, one token per sequence.
+    `waves`: wavefronts a workgroup, 4 or (heads of up to 64 elements) 8.
     `streaming`: fetch keys and values with non-temporal loads (same result; faster when
     the launch reads tens of megabytes of them)."""
     _rows(q, "attention_decode q")
@@ -1378,7 +1379,7 @@ def attention_decode(q, out, num_seqs, heads, kv_heads, head_dim, positions, tab
             _dev(positions, "positions", torch.int32), _dev(tables, "tables", torch.int32),
             tables.shape[1], _dev(k_pool, "k_pool"), _dev(v_pool, "v_pool"), page_size,
             int(window or 0), int(chunk or 0), float(scale), _dev(partial, "partial", torch.float32), nsplit,
-            int(bool(streaming)), float(softcap or 0.0), _sinks(sinks, heads, "attention_decode"),
+            int(bool(streaming)), int(waves), float(softcap or 0.0), _sinks(sinks, heads, "attention_decode"),
             *_dist_bias_args(dist_bias, heads, "attention_decode"), _stream(),
         )
     )

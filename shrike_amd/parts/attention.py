@@ -87,6 +87,18 @@ def decode_splits(num_seqs: int, kv_heads: int, max_ctx: int) -> int:
     return max(1, min(want, most, MAX_KEY_SPLITS))
 
 
+def decode_shares(num_seqs: int, kv_heads: int, head_dim: int, max_ctx: int) -> tuple[int, int]:
+    """(key splits, wavefronts a workgroup) of decode attention.  Where a few short sequences of small heads
+    would share up to 512 keys among two workgroups of four wavefronts, one of eight walks them as fast, and the kernel
+    that joins two splits, which takes as long as either, goes (14 heads of 64 over 2, one sequence at 333: 4.4 + 2.5
+    us against 5.0).  Elsewhere eight wavefronts gain nothing: 8 sequences at 2,060 with 28 heads of 128 over 4 a step of
+    3.24 ms against 3.18, 64 at 61 to 1,203 4.43 against 4.35.  Rounded up as in decode_splits()."""
+    splits = decode_splits(num_seqs, kv_heads, max_ctx)
+    if splits > 1 and head_dim <= 64 and _pow2(max_ctx, KEYS_PER_WORKGROUP) <= 2 * KEYS_PER_WORKGROUP:
+        return 1, 8
+    return splits, 4
+
+
 def decode_streams(num_seqs: int, kv_heads: int, head_dim: int, max_ctx: int, window: int | None = None) -> bool:
     """Whether a decode launch reads so many keys and values that non-temporal
     loads pay (measured with 4 key/value heads of 128: a tenth faster from 64
@@ -105,6 +117,7 @@ class AttentionPlan:
 
     mfma: bool = False
     nsplit: int = 1  # key splits of the single-token rows
+    waves: int = 4  # wavefronts of their workgroups
     streaming: bool = False  # single-token rows: non-temporal loads of keys and values
     kernel: str = ""  # for prompt portions: "shared", "tiles" or "" (none in the step)
     small: bool = False  # "shared" with half as many wavefronts per workgroup
@@ -396,10 +409,10 @@ class PagedAttention(Mixer):
         if not plan.mfma:
             return  # the general kernel takes every token alike
         if shape.num_decode:
-            plan.nsplit = decode_splits(shape.num_decode, hkv, min(shape.max_decode_ctx, reach))
+            plan.nsplit, plan.waves = decode_shares(shape.num_decode, hkv, d, min(shape.max_decode_ctx, reach))
             plan.streaming = decode_streams(shape.num_decode, hkv, d, shape.max_decode_ctx,
                                             reach if s.window or s.chunk else None)
-            shape.launch_key.append((key, plan.nsplit, plan.streaming))
+            shape.launch_key.append((key, plan.nsplit, plan.waves, plan.streaming))
         portions = shape.q_lens[shape.num_decode:]
         if portions.size == 0:
             return
@@ -485,7 +498,7 @@ class PagedAttention(Mixer):
                                  torch.float32)
             ops.attention_decode(q, out, ctx.num_decode, h, hkv, d, ctx.positions, tables,
                                  cache.pools["k"], cache.pools["v"], cache.page_size, s.window, s.scale,
-                                 partial, plan.nsplit, plan.streaming, chunk=s.chunk,
+                                 partial, plan.nsplit, plan.streaming, chunk=s.chunk, waves=plan.waves,
                                  softcap=getattr(s, "softcap", None), sinks=self.sinks, dist_bias=self.dist_bias)
         if plan.kernel == "shared":
             partial = None
