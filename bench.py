@@ -322,7 +322,7 @@ def kernel_breakdown(engine, steps: int = 3, before_step=None) -> dict:
 
     from shrike_amd.kernels import ops
 
-    names = ["embed", "add_rmsnorm", "act_mul", "gemm", "gemm_f32_tiled_weight", "gemm_tiled_weight", "rope_kv_store", "attention",
+    names = ["embed", "add_rmsnorm", "act_mul", "gemm", "gemm_f32_tiled_weight", "latent_prompt", "gemm_tiled_weight", "rope_kv_store", "attention",
              "attention_decode", "attention_prefill", "attention_prefill_shared", "argmax", "sample",
              "add_deltas", "add_normed_rmsnorm", "act_mul_rows", "add_rows", "embed_pairs", "qkv_store",
              "latent_prepare", "rotate_heads", "latent_attention", "latent_attention_mfma", "gemm_batched", "mlstm_scan", "headnorm_gate",

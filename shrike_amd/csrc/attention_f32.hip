@@ -12,10 +12,10 @@
 //
 // A lane of the first product's result holds four neighbouring keys of one head, which is the second
 // product's operand as it stands: weights never pass through LDS.  What bounds it: a block is 64 + 64
-// instructions of 32 cycles per wavefront (head size 64) and three barriers, about 3 us; the general
-// kernel's one workgroup per query head with one key per thread took 560 us for 14 heads of 64 over
-// 509 tokens, and 50 us for four single tokens at 400 (whole passes: a 509-token prompt of the 0.5B model
-// 18.9 ms then, 6.5 now; a decode step of four requests 2.43 ms, 1.67 now).
+// instructions of 32 cycles per wavefront (head size 64: 4,096 cycles) and three barriers.  14 heads of 64
+// over 2, 509 tokens: 560 us a layer in the general kernel, whose one workgroup per query head had one key
+// per thread, 40 here; four single tokens at about 400: 50 us, here 16 and 4.6 for the join (whole passes: a
+// prompt of 24 such layers 18.9 ms then, 6.5 now; a decode step of four requests 2.43 ms, 1.67 now).
 #include "api.h"
 #include "attention_f32.h"
 #include "common.h"

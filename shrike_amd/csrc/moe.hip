@@ -21,9 +21,10 @@
 //
 // On the matrix units (bfloat16, many tokens): the (token, expert) pairs are listed per expert
 // in the order of the tokens (moe_lists_kernel, a workgroup per expert), and the two products
-// run per expert over its list in tiles of 32 pairs (v_mfma_f32_16x16x32_bf16, both operands
-// row-major with k innermost and loaded as operands straight from memory).  Workgroups beyond
-// an expert's list leave at once, so the grid depends on the step's size alone.  A pair's
+// run per expert over its list (v_mfma_f32_16x16x32_bf16): short lists in tiles of 32 pairs, operands
+// straight from memory, longer ones in tiles of 128 pairs through LDS.  Matrices whose sides are multiples
+// of 64 lie in tiles of 16 rows x 32, others row-major with k innermost.  Workgroups beyond
+// an expert's list leave at once or take none, so the grid depends on the step's size alone.  A pair's
 // sums run over k in one fixed order wherever the pair stands in its list; the pairs' outputs
 // are kept in float32 and joined per token in the order the experts were chosen.
 #include "api.h"

@@ -89,9 +89,9 @@ def decode_splits(num_seqs: int, kv_heads: int, max_ctx: int) -> int:
 
 def decode_shares(num_seqs: int, kv_heads: int, head_dim: int, max_ctx: int) -> tuple[int, int]:
     """(key splits, wavefronts a workgroup) of decode attention.  Where a few short sequences of small heads
-    would share up to 512 keys among two workgroups of four wavefronts, one of eight walks them as fast, and the kernel
-    that joins two splits, which takes as long as either, goes (14 heads of 64 over 2, one sequence at 333: 4.4 + 2.5
-    us against 5.0).  Elsewhere eight wavefronts gain nothing: 8 sequences at 2,060 with 28 heads of 128 over 4 a step of
+    would share up to 512 keys among two workgroups of four wavefronts, one of eight takes longer than either but less
+    than both and the kernel that joins them (14 heads of 64 over 2, one sequence at 333: 6.2 us a layer against
+    4.4 + 2.5 in two launches; a decode step of 24 such layers 815 us against 848).  Elsewhere eight wavefronts gain nothing: 8 sequences at 2,060 with 28 heads of 128 over 4 a step of
     3.24 ms against 3.18, 64 at 61 to 1,203 4.43 against 4.35.  Rounded up as in decode_splits()."""
     splits = decode_splits(num_seqs, kv_heads, max_ctx)
     if splits > 1 and head_dim <= 64 and _pow2(max_ctx, KEYS_PER_WORKGROUP) <= 2 * KEYS_PER_WORKGROUP:
