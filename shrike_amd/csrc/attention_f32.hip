@@ -14,8 +14,12 @@
 // product's operand as it stands: weights never pass through LDS.  What bounds it: a block is 64 + 64
 // instructions of 32 cycles per wavefront (head size 64: 4,096 cycles) and three barriers.  14 heads of 64
 // over 2, 509 tokens: 560 us a layer in the general kernel, whose one workgroup per query head had one key
-// per thread, 40 here; four single tokens at about 400: 50 us, here 16 and 4.6 for the join (whole passes: a
-// prompt of 24 such layers 18.9 ms then, 6.5 now; a decode step of four requests 2.43 ms, 1.67 now).
+// per thread, 40 here; four single tokens at about 400: 50 us, here 12 and 4.4 for the join (whole passes: a
+// prompt of 24 such layers 18.9 ms then, 6.5 now; a decode step of four requests 2.43 ms, 1.56 now).  A
+// single token's block is one chain from the page numbers over keys and values to the join, so all page
+// numbers are read first, without a branch, then as many steps' keys and values as registers hold before the
+// first product (head size 64: all of them; with each step's loads next to its products 16 us for the 12).  A
+// prompt's tokens, with workgroups enough to cover one another's waits, take 6.5 ms either way.
 #include "api.h"
 #include "attention_f32.h"
 #include "common.h"
@@ -86,42 +90,72 @@ __global__ void __launch_bounds__(kWave * kBlockWaves) attention_f32_kernel(F32A
   float M = -INFINITY, L = 0.f;
   const int slab = key_slab(p.head_dim), ps = p.page_size;
   const size_t k_page = static_cast<size_t>(ps) * p.head_dim, v_page = static_cast<size_t>(ps) * p.v_dim;
-  auto page_of = [&](int key) {  // -1 where no key may be read
-    const int page = key >= lo && key <= pos ? table[key / ps] : -1;
+  constexpr int kSteps = kWaveKeys / 16, kAhead = D <= 4 ? kSteps : D == 8 ? 2 : 1;  // steps of 16 keys, and how many are loaded at once
+  auto page_of = [&](int key) {  // of `key`, or of the nearest key that is read; -1 where there is none
+    const int page = table[min(max(key, lo), pos) / ps];
     return page < p.num_pages ? page : -1;
   };
 
   for (int b = first; b <= last; b += step) {
     const int key0 = b * kKeyBlock + wave * kWaveKeys;
+    const bool any = key0 <= pos && key0 + kWaveKeys > lo;  // of this wavefront's keys is read
     // scores: this lane loads key key0 + 16 u + i, and gets keys key0 + 16 u + 4 kg + 0..3 of head i
-    af4 s[kWaveKeys / 16];
-    int v_at[kWaveKeys / 16];  // page of the keys whose values this lane loads
-#pragma unroll
-    for (int u = 0; u < kWaveKeys / 16; ++u) {
-      s[u] = af4{0.f, 0.f, 0.f, 0.f};
-      const int key = key0 + 16 * u + i, vkey = key0 + 16 * u + 4 * kg;
-      const int page = max(page_of(key), 0);
-      // (page sizes are multiples of four: the four keys share a page; the first or the last of them is
-      // one that may be read, if any is)
-      v_at[u] = max(page_of(vkey), page_of(min(vkey + 3, pos)));
-      const float* kr = p.k_pool + (static_cast<size_t>(page) * p.kv_heads + kvh) * k_page + static_cast<size_t>(key % ps) * slab;
-      af4 kv[D];
+    af4 s[kSteps];
+    int k_at[kSteps], v_at[kSteps];  // pages of the keys, and of the values, that this lane loads
+    af4 kv[kAhead][D], vv[kAhead][D];
+    auto load_keys = [&](int u) {
+      const int key = key0 + 16 * u + i;
+      const float* kr = p.k_pool + (static_cast<size_t>(max(k_at[u], 0)) * p.kv_heads + kvh) * k_page + static_cast<size_t>(key % ps) * slab;
 #pragma unroll
       for (int x = 0; x < D; ++x) {
         const int d = 16 * x + 4 * kg;
-        const bool have = d < p.head_dim;
-        const size_t at = have ? static_cast<size_t>(d / slab) * ps * slab + d % slab : 0;
-        kv[x] = *reinterpret_cast<const af4*>(kr + at);
-        if (!have) kv[x] = af4{0.f, 0.f, 0.f, 0.f};
+        const size_t at = d < p.head_dim ? static_cast<size_t>(d / slab) * ps * slab + d % slab : 0;
+        kv[u % kAhead][x] = *reinterpret_cast<const af4*>(kr + at);
+      }
+    };
+    auto load_values = [&](int u) {
+      const int key = key0 + 16 * u + 4 * kg;
+      const float* vr = p.v_pool + (static_cast<size_t>(max(v_at[u], 0)) * p.kv_heads + kvh) * v_page + key % ps;
+#pragma unroll
+      for (int x = 0; x < D; ++x) {
+        const int d = 16 * x + i;
+        vv[u % kAhead][x] = *reinterpret_cast<const af4*>(vr + static_cast<size_t>(d < p.v_dim ? d : 0) * ps);
+      }
+    };
+#pragma unroll
+    for (int u = 0; u < kSteps; ++u) {
+      s[u] = af4{0.f, 0.f, 0.f, 0.f};
+      v_at[u] = -1;
+    }
+    if (any) {
+#pragma unroll
+      for (int u = 0; u < kSteps; ++u) {
+        // (page sizes are multiples of four: a lane's four keys share a page, and where any of them is read
+        // the nearest to the first that is read is one of them)
+        k_at[u] = page_of(key0 + 16 * u + i);
+        v_at[u] = page_of(key0 + 16 * u + 4 * kg);
       }
 #pragma unroll
-      for (int x = 0; x < D; ++x)
+      for (int u0 = 0; u0 < kSteps; u0 += kAhead) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) s[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[x][e], qv[x][e], s[u], 0, 0, 0);
+        for (int u = u0; u < u0 + kAhead; ++u) load_keys(u);
+        if (u0 + kAhead == kSteps)
+#pragma unroll
+          for (int u = 0; u < kAhead; ++u) load_values(u);
+#pragma unroll
+        for (int x = 0; x < D; ++x)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int u = u0; u < u0 + kAhead; ++u) {
+              const float key = 16 * x + 4 * kg < p.head_dim ? kv[u % kAhead][x][e] : 0.f;
+              s[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(key, qv[x][e], s[u], 0, 0, 0);
+            }
+      }
     }
     float top = -INFINITY;
 #pragma unroll
-    for (int u = 0; u < kWaveKeys / 16; ++u)
+    for (int u = 0; u < kSteps; ++u)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int key = key0 + 16 * u + 4 * kg + e;
@@ -144,29 +178,23 @@ __global__ void __launch_bounds__(kWave * kBlockWaves) attention_f32_kernel(F32A
     af4 acc[D];
 #pragma unroll
     for (int x = 0; x < D; ++x) acc[x] = af4{0.f, 0.f, 0.f, 0.f};
+    if (any) {
 #pragma unroll
-    for (int u = 0; u < kWaveKeys / 16; ++u) {
-      const int vkey = key0 + 16 * u + 4 * kg;
-      const float* vr = p.v_pool + (static_cast<size_t>(max(v_at[u], 0)) * p.kv_heads + kvh) * v_page + vkey % ps;
-      af4 vv[D];
+      for (int u = 0; u < kSteps; ++u) {
+        if (u >= kAhead && u % kAhead == 0)
 #pragma unroll
-      for (int x = 0; x < D; ++x) {
-        const int d = 16 * x + i;
-        vv[x] = *reinterpret_cast<const af4*>(vr + static_cast<size_t>(d < p.v_dim ? d : 0) * ps);
+          for (int ahead = u; ahead < u + kAhead; ++ahead) load_values(ahead);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int key = key0 + 16 * u + 4 * kg + e;
+          const bool have = key >= lo && key <= pos && v_at[u] >= 0;
+          const float w = have ? expf(s[u][e] - m) : 0.f;
+          l += w;
+#pragma unroll
+          for (int x = 0; x < D; ++x)
+            acc[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(have ? vv[u % kAhead][x][e] : 0.f, w, acc[x], 0, 0, 0);
+        }
       }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const bool have = vkey + e >= lo && vkey + e <= pos && v_at[u] >= 0;
-        const float w = have ? expf(s[u][e] - m) : 0.f;
-        l += w;
-        s[u][e] = w;
-#pragma unroll
-        for (int x = 0; x < D; ++x) vv[x][e] = have ? vv[x][e] : 0.f;
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-#pragma unroll
-        for (int x = 0; x < D; ++x) acc[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[x][e], s[u][e], acc[x], 0, 0, 0);
     }
     l += __shfl_xor(l, 16);
     l += __shfl_xor(l, 32);
