@@ -14,7 +14,7 @@
 // product's operand as it stands: weights never pass through LDS.  What bounds it: a block is 64 + 64
 // instructions of 32 cycles per wavefront (head size 64: 4,096 cycles) and three barriers.  14 heads of 64
 // over 2, 509 tokens: 560 us a layer in the general kernel, whose one workgroup per query head had one key
-// per thread, 40 here; four single tokens at about 400: 50 us, here 12 and 4.4 for the join (whole passes: a
+// per thread, 39 here; four single tokens at about 400: 50 us, here 12 and 4.4 for the join (whole passes: a
 // prompt of 24 such layers 18.9 ms then, 6.5 now; a decode step of four requests 2.43 ms, 1.56 now).  A
 // single token's block is one chain from the page numbers over keys and values to the join, so all page
 // numbers are read first, without a branch, then as many steps' keys and values as registers hold before the
