@@ -83,3 +83,27 @@ def test_batched_products_of_every_shape(batch, m, k):
         odd = torch.full((n, batch * m + 3), 7.0, device="cuda", dtype=torch.bfloat16)  # rows no multiple of 4 elements apart
         ops.gemm_batched(a[:n, : batch * k], w, odd[:, 1 : 1 + batch * m], batch, k, m)
         assert torch.equal(odd[:, 1 : 1 + batch * m], out[:, : batch * m].bfloat16())
+
+
+@pytest.mark.parametrize("m, k", [(4080, 896), (4096, 24), (4100, 896), (4864, 1024), (4864, 1032), (8176, 264)])
+def test_gated_products_of_a_short_k(m, k):
+    """Where 16 wavefronts share k and where four do: up to 16 tokens beside what serves each token alone."""
+    from shrike_amd.kernels import ops
+
+    torch.manual_seed(m + k)
+    a = torch.randn(16, k, device="cuda").bfloat16()
+    gate, up = ((torch.randn(m, k, device="cuda") / k**0.5).bfloat16() for _ in range(2))
+    wt = ops.interleave_gate_up(gate, up)
+    g, u = a.double() @ gate.double().t(), a.double() @ up.double().t()
+    sized = [a.double().abs() @ w.double().abs().t() for w in (gate, up)]
+    act = g * torch.sigmoid(g)
+    # float32 sums as above, SiLU's slope is at most 1.1; bfloat16 results (half an ulp is 2^-9, the rest for the exponential)
+    each = (k / 32 + 40) * 2.0**-24
+    bound = 2.0**-8 * (act * u).abs() + 2 * each * (1.1 * sized[0] * u.abs() + sized[1] * act.abs())
+    whole = torch.empty(16, m, device="cuda", dtype=torch.bfloat16)
+    ops.gemm_tiled_weight(a, wt, m, k, whole, gated=True)
+    assert bool(((whole.double() - act * u).abs() <= bound + 1e-7).all())
+    for n in (1, 5):
+        out = torch.full((n, m + 8), 7.0, device="cuda", dtype=torch.bfloat16)
+        ops.gemm_tiled_weight(a[16 - n:], wt, m, k, out[:, :m], gated=True)
+        assert torch.equal(out[:, :m], whole[16 - n:]) and bool((out[:, m:] == 7.0).all())
