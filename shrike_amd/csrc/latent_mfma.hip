@@ -258,9 +258,26 @@ __global__ void __launch_bounds__(kLatentWaves* kWave)
 // matrix instructions where the kernel above uses it once, and a chunk is staged once for tpw tokens.  Two
 // buffers for the rows and for the weights: two barriers a chunk.
 // What bounded the kernel above over a prompt was its LDS reads, 288 for 60 matrix instructions a chunk and
-// wavefront: 28 heads over rows of 512, 1,501 tokens, 483 us a layer, 266 here; rows straight into LDS instead
-// of through registers took 437 (more addresses than registers are left: spills).
+// wavefront: 28 heads over rows of 512, 1,501 tokens, 468 us a layer, 200 here; rows straight into LDS instead
+// of through registers took 437.  Queries (64 registers) and sums (112) leave so little that addresses kept from chunk to
+// chunk were spilled: 261 us with 21 such registers; worked out anew (here()) three remain.
+//
+// A column takes nothing but rows that its own token reads, not even 0 times a number that is none: the products run
+// over all columns, so tokens of several sequences in a workgroup are served one sequence after the other, each from
+// sums of zero, and where a staged row that some of a sequence's tokens do not read holds an infinity or a NaN, those
+// tokens are served again, one after the other.
 constexpr int kPromptWaves = 8;
+
+// whether either of two bfloat16 values is an infinity or not a number
+__device__ __forceinline__ bool not_number(uint32_t two) {
+  return (two & 0x7f80u) == 0x7f80u || (two & 0x7f800000u) == 0x7f800000u;
+}
+
+// x, but what follows from it is worked out where it is used, not kept in registers (or spilled) from chunk to chunk
+__device__ __forceinline__ int here(int x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
 
 template <int KS, int DBW, int NC>  // rows of up to 32 KS elements, values of up to 128 DBW, 16 NC columns
 __global__ void __launch_bounds__(kPromptWaves* kWave)
@@ -276,6 +293,7 @@ __global__ void __launch_bounds__(kPromptWaves* kWave)
   __shared__ __attribute__((aligned(16))) uint16_t rows0[2 * kRows];
   __shared__ uint4 weights0[2 * NC * kWave];
   __shared__ float shrink0[2 * NC * 16];
+  __shared__ int unsafe[2];  // by a pass's parity: the pass that met a number that is none in a row not read by all
   const int tid = threadIdx.x, lane = tid % kWave, j = lane % 16, g = lane / 16;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int t0 = (gridDim.x - 1 - blockIdx.x) * tpw, z = blockIdx.y;  // (the last tokens read the most rows: they start first)
@@ -296,52 +314,58 @@ __global__ void __launch_bounds__(kPromptWaves* kWave)
   }
   // what lies behind a row's elements stays zero for the whole kernel
   for (int i = tid; i < 2 * kRows / 8; i += kThreads) reinterpret_cast<uint4*>(rows0)[i] = make_uint4(0, 0, 0, 0);
+  if (tid < 2) unsafe[tid] = 0;
   __syncthreads();
 
-  bool same = true;
-  for (int i = t0 + 1; i <= t_last; ++i) same = same && token_seq[i] == token_seq[t0];
-  const int passes = same ? 1 : t_last - t0 + 1;
   const int npieces = key_dim / 8;
   const float scale2 = scale * 1.4426950408889634f;
-  float m = -INFINITY, l = 0.f;  // l: the lane's share of its column's sum until the end
-  lf32x4 o[DBW][NC];             // element 16 (wave + 8 x) + 4 g + r of column 16 c + j
-#pragma unroll
-  for (int x = 0; x < DBW; ++x)
-#pragma unroll
-    for (int c = 0; c < NC; ++c) o[x][c] = lf32x4{0.f, 0.f, 0.f, 0.f};
-
   uint4 staged[kPieces];
-  int piece_row[kPieces], piece_col[kPieces];
+  int piece[kPieces];  // row and first element of what this thread stages; negative: nothing
 #pragma unroll
   for (int u = 0; u < kPieces; ++u) {
     const int idx = tid + u * kThreads;
-    piece_row[u] = idx < 32 * npieces ? idx / npieces : -1;
-    piece_col[u] = (idx % npieces) * 8;
+    piece[u] = idx < 32 * npieces ? idx / npieces << 16 | idx % npieces * 8 : -1;
   }
   const int page_shift = (page_size & (page_size - 1)) == 0 ? __ffs(page_size) - 1 : -1;
-  int buf = 0;
-  for (int pass = 0; pass < passes; ++pass) {
-    const int ta = same ? t0 : t0 + pass, tb = same ? t_last : t0 + pass;
+  int buf = 0, pass = 0;
+  int seq_end = t0 - 1, ta = t0, tb = t0 - 1;  // the last token of the sequence that is served; the pass's tokens
+  int key_begin = 0, c_first = 0, c_end = 0;
+  while (tb < t_last) {
+    if (tb == seq_end) {
+      for (ta = tb + 1, tb = ta; tb < t_last && token_seq[tb + 1] == token_seq[ta];) ++tb;
+      seq_end = tb;
+      // the chunks of this share are the same ones however the sequence's tokens are served
+      key_begin = first_key(positions[ta], window, chunk) & ~31;
+      const int nchunks = (positions[tb] - key_begin) / 32 + 1, per_split = (nchunks + nsplit - 1) / nsplit;
+      c_first = z * per_split, c_end = min(c_first + per_split, nchunks);
+    } else {
+      ta = ++tb;
+    }
+  again:
+    ++pass;
     const int stage_hi = positions[tb], stage_lo = first_key(positions[ta], window, chunk);
+    const int all_hi = positions[ta], all_lo = first_key(positions[tb], window, chunk);  // rows that each token reads
     const int32_t* table = tables + static_cast<size_t>(token_seq[ta]) * table_stride;
     const bool mine = col_ok && t >= ta && t <= tb;
-    const int key_begin = stage_lo & ~31;
-    const int nchunks = (stage_hi - key_begin) / 32 + 1;
-    const int per_split = (nchunks + nsplit - 1) / nsplit;
-    const int c_first = z * per_split, c_end = min(c_first + per_split, nchunks);
+    float m = -INFINITY, l = 0.f;  // l: the lane's share of its column's sum until the end
+    lf32x4 o[DBW][NC];             // element 16 (wave + 8 x) + 4 g + r of column 16 c + j
+#pragma unroll
+    for (int x = 0; x < DBW; ++x)
+#pragma unroll
+      for (int c = 0; c < NC; ++c) o[x][c] = lf32x4{0.f, 0.f, 0.f, 0.f};
     auto fetch = [&](int c) {
       const int kb = key_begin + c * 32;
 #pragma unroll
       for (int u = 0; u < kPieces; ++u) {
-        const int key = kb + piece_row[u];
+        const int place = here(piece[u]), key = kb + (place >> 16);
         staged[u] = make_uint4(0, 0, 0, 0);
-        if (piece_row[u] >= 0 && key >= stage_lo && key <= stage_hi) {
+        if (place >= 0 && key >= stage_lo && key <= stage_hi) {
           const int entry = page_shift >= 0 ? key >> page_shift : key / page_size;
           const int slot = page_shift >= 0 ? key & (page_size - 1) : key % page_size;
           const int page = table[entry];
           if (page >= 0 && page < num_pages)
             staged[u] = *reinterpret_cast<const uint4*>(
-                pool + (static_cast<size_t>(page) * page_size + slot) * key_dim + piece_col[u]);
+                pool + (static_cast<size_t>(page) * page_size + slot) * key_dim + (place & 0xffff));
         }
       }
     };
@@ -352,8 +376,18 @@ __global__ void __launch_bounds__(kPromptWaves* kWave)
       uint4* const weights = weights0 + buf * NC * kWave;
       float* const shrink = shrink0 + buf * NC * 16;
 #pragma unroll
-      for (int u = 0; u < kPieces; ++u)
-        if (piece_row[u] >= 0) *reinterpret_cast<uint4*>(rows + at(piece_row[u]) + piece_col[u]) = staged[u];
+      for (int u = 0; u < kPieces; ++u) {
+        const int place = here(piece[u]);
+        if (place >= 0) *reinterpret_cast<uint4*>(rows + at(place >> 16) + (place & 0xffff)) = staged[u];
+      }
+      if (kb < all_lo || kb + 31 > all_hi) {
+        asm volatile("");  // (a branch, not instructions that every chunk passes)
+        bool none = false;  // (pieces of no row are zeros)
+#pragma unroll
+        for (int u = 0; u < kPieces; ++u)
+          none = none || not_number(staged[u].x) || not_number(staged[u].y) || not_number(staged[u].z) || not_number(staged[u].w);
+        if (none) unsafe[pass & 1] = pass;
+      }
       __syncthreads();
       if (scores) {
         // row i of tile tt is row 8 (i / 4) + 4 tt + i % 4 of the chunk: the lane's eight scores belong to rows 8 g + e
@@ -416,39 +450,44 @@ __global__ void __launch_bounds__(kPromptWaves* kWave)
           o[x][cc] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(lbf16x8, vw[x]), pf.v, o[x][cc], 0, 0, 0);
       }
     }
-  }
-  l = quad_lanes_sum(l);
-  __syncthreads();
-  float* const sums = shrink0;  // [16 NC], and behind them the maxima
-  if (scores && g == 0) {
-    sums[col] = l;
-    sums[NC * 16 + col] = m;
-  }
-  __syncthreads();
-  const size_t all_rows = static_cast<size_t>(n) * heads;
-#pragma unroll
-  for (int cc = 0; cc < NC; ++cc) {
-    const int c = cc * 16 + j;
-    if (c >= tpw * heads || t0 + c / heads > t_last) continue;
-    const size_t row = static_cast<size_t>(t0) * heads + c;
-    const float inv = 1.f / sums[c];
-#pragma unroll
-    for (int x = 0; x < DBW; ++x) {
-      const int d = (wave + 8 * x) * 16 + 4 * g;
-      if (wave + 8 * x >= dtiles) continue;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        if (d + r >= v_dim) continue;
-        if (nsplit == 1)
-          out[row * v_dim + d + r] = from_float<bf16>(o[x][cc][r] * inv);
-        else
-          partial[(row * nsplit + z) * v_dim + d + r] = o[x][cc][r];
-      }
+    l = quad_lanes_sum(l);
+    __syncthreads();
+    float* const sums = shrink0;  // [16 NC], and behind them the maxima
+    if (scores && g == 0) {
+      sums[col] = l;
+      sums[NC * 16 + col] = m;
     }
-    if (nsplit > 1 && wave == 0 && g == 0) {
-      float* ml = partial + all_rows * nsplit * v_dim + (row * nsplit + z) * 2;
-      ml[0] = sums[NC * 16 + c];
-      ml[1] = sums[c];
+    __syncthreads();
+    if (tb > ta && unsafe[pass & 1] == pass) {  // (the same for all; the next pass writes the other place)
+      tb = ta;
+      goto again;
+    }
+    const int column = here(j), tile = __builtin_amdgcn_readfirstlane(here(wave));
+    const size_t all_rows = static_cast<size_t>(n) * heads;
+#pragma unroll
+    for (int cc = 0; cc < NC; ++cc) {
+      const int c = cc * 16 + column;
+      if (c < (ta - t0) * heads || c >= (tb - t0 + 1) * heads) continue;
+      const size_t row = static_cast<size_t>(t0) * heads + c;
+      const float inv = 1.f / sums[c];
+#pragma unroll
+      for (int x = 0; x < DBW; ++x) {
+        const int d = (tile + 8 * x) * 16 + 4 * g;
+        if (tile + 8 * x >= dtiles) continue;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          if (d + r >= v_dim) continue;
+          if (nsplit == 1)
+            out[row * v_dim + d + r] = from_float<bf16>(o[x][cc][r] * inv);
+          else
+            partial[(row * nsplit + z) * v_dim + d + r] = o[x][cc][r];
+        }
+      }
+      if (nsplit > 1 && wave == 0 && g == 0) {
+        float* ml = partial + all_rows * nsplit * v_dim + (row * nsplit + z) * 2;
+        ml[0] = sums[NC * 16 + c];
+        ml[1] = sums[c];
+      }
     }
   }
 }

@@ -46,3 +46,49 @@ def test_against_float64(heads, key_dim, v_dim, page, window, chunk, nsplit):
         # weights and the result are rounded to bfloat16 (2^-9 each, the weights' sizes adding up to one)
         bound = 2.0**-7 * (w @ r[:, :v_dim].abs()) + 1e-3
         assert bool(((got[t] - want).abs() <= bound).all()), t
+
+
+@pytest.mark.parametrize("heads, key_dim, v_dim, window, chunk", [
+    (28, 512, 448, None, None), (14, 160, 128, None, None), (3, 40, 24, None, 64), (64, 264, 200, 70, None), (1, 8, 8, 33, None),
+    (17, 256, 256, None, None), (9, 320, 250, 100, 128),
+])
+@pytest.mark.parametrize("nsplit", [1, 3])
+def test_a_row_that_is_no_number_stays_with_the_tokens_that_read_it(heads, key_dim, v_dim, window, chunk, nsplit):
+    """Infinities and NaN in one sequence's rows, from some position on: tokens of other sequences in the same
+    workgroups, earlier ones of the same sequence and later ones whose window has passed them keep their bits."""
+    from shrike_amd.kernels import ops
+
+    page = 16
+    torch.manual_seed(heads + key_dim)
+    starts, lengths = [0, 61, 0, 130, 3], [45, 7, 1, 35, 150]
+    n, ctx = sum(lengths), [s + k for s, k in zip(starts, lengths)]
+    per = -(-max(ctx) // page)
+    tables = torch.randperm(5 * per).view(5, per).int().cuda()
+    clean = torch.randn(5 * per, page, key_dim, device="cuda").bfloat16()
+    q = torch.randn(n, heads * key_dim, device="cuda").bfloat16()
+    positions = torch.cat([torch.arange(s, s + k) for s, k in zip(starts, lengths)]).int().cuda()
+    seqs = torch.repeat_interleave(torch.arange(5), torch.tensor(lengths)).int().cuda()
+
+    def run(pool):
+        out = torch.full((n, heads * v_dim), 9.0, device="cuda", dtype=torch.bfloat16)
+        partial = torch.full((n * heads * nsplit * (v_dim + 2),), float("nan"), device="cuda")
+        ops.latent_prompt(q, out, heads, key_dim, v_dim, positions, seqs, tables, pool, page, window, 0.7 / key_dim**0.5,
+                          chunk=chunk, partial=partial, nsplit=nsplit)
+        return out
+
+    want = run(clean)
+    assert bool(torch.isfinite(want.float()).all())
+    p = positions.long()
+    lo = torch.zeros_like(p)
+    if window:
+        lo = torch.maximum(lo, p - window + 1)
+    if chunk:
+        lo = torch.maximum(lo, p // chunk * chunk)
+    for seq, at, what in ((0, 17, float("nan")), (1, 67, float("inf")), (3, 140, float("-inf")), (4, 40, float("nan"))):
+        pool = clean.clone()
+        pool[tables[seq, at // page].long(), at % page, v_dim // 2] = what
+        got = run(pool)
+        reads = (seqs == seq) & (lo <= at) & (at <= p)
+        assert bool(reads.any())
+        assert torch.equal(got[~reads], want[~reads]), (seq, at)
+        assert not bool(torch.isfinite(got[reads].float()).view(-1, heads, v_dim)[:, :, v_dim // 2].any()), (seq, at)
