@@ -1481,13 +1481,9 @@ extern "C" int shk_gemm_bf16_parts(int n, int m, int k, int gated) {
   return big_main_blocks(big_shape(1, n, wblocks, m, k), n, wblocks, m, k, gated) ? 2 : 1;
 }
 
-extern "C" int shk_gemm_bf16_splits(int n, int m, int k) {
+// Shares of k for the kernels that stage operands or stream the weights.
+static int staged_splits(int n, int m, int k) {
   const int mblocks = (m + 15) / 16, ktiles = (k + 31) / 32;
-  if (n > 64 && few_rows(m)) return 1;
-  // (a long k in two shares up to 64 tokens: 896 x 4864 7.4 us against 10.0 whole, the second share costs its reader
-  // half a microsecond)
-  const int direct = n <= 64 && k > 2048 ? 2 : 1;
-  if (direct_shape(n, m, k, direct)) return direct;
   if (n > 64) {
     // many tokens: the number of shares, each of at least 8 stages of 64, that
     // big_estimate() expects to be fastest with the tile shape that suits it
@@ -1544,6 +1540,21 @@ extern "C" int shk_gemm_bf16_splits(int n, int m, int k) {
   }
   if (split > most) split = most;
   return split > 1 ? split : 1;
+}
+
+extern "C" int shk_gemm_bf16_splits(int n, int m, int k) {
+  if (n > 64 && few_rows(m)) return 1;
+  // (a long k in two shares up to 64 tokens: 896 x 4864 7.4 us against 10.0 whole, the second share costs its reader
+  // half a microsecond)
+  const int direct = n <= 64 && k > 2048 ? 2 : 1;
+  return direct_shape(n, m, k, direct) ? direct : staged_splits(n, m, k);
+}
+
+// Whether a reader that adds up shares gets an unsplit product as one float32 share all the same: where
+// gemm_direct_kernel, or gemm_skinny_kernel group by group, form whole what the staged kernels would leave in shares.  In bfloat16
+// it would be rounded once more than a product in shares, before the residual or the rotation.
+extern "C" int shk_gemm_bf16_keeps_float32(int n, int m, int k) {
+  return shk_gemm_bf16_splits(n, m, k) == 1 && staged_splits(n, m, k) > 1;
 }
 
 extern "C" int shk_gemm_bf16_tiled_weight(const void* a, const void* wt, const float* bias,

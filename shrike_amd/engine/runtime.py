@@ -90,11 +90,13 @@ class Runtime:
         reader "rows": a kernel that adds the parts of any width (ops.act_mul_rows).
         keep_float32: a product that is not split comes as a SplitSum of one float32
         part instead of a tensor in the compute dtype (for a reader that takes parts
-        and is sensitive to the rounding of its input)."""
+        and is sensitive to the rounding of its input); small matrices that are formed
+        whole where larger ones would be split (gemm_keeps_float32) always do."""
         n = x.shape[0]
-        splits = ops.gemm_splits(n, w.rows, w.cols) if w.tiled is not None else 1
-        if reader == "norm" and (bias is not None or w.rows % 4 or w.rows > 8192):
-            splits = 1
+        splits = 1
+        if w.tiled is not None and not (reader == "norm" and (bias is not None or w.rows % 4 or w.rows > 8192)):
+            splits = ops.gemm_splits(n, w.rows, w.cols)
+            keep_float32 = keep_float32 or ops.gemm_keeps_float32(n, w.rows, w.cols)
         if splits > 1:
             parts = ctx.buffer(name + "_parts", (splits, n, w.rows), torch.float32)
             ops.gemm_tiled_weight(x, w.tiled, w.rows, w.cols, parts, splits=splits)

@@ -403,6 +403,11 @@ def gemm_splits(n: int, m: int, k: int) -> int:
     return int(load().shk_gemm_bf16_splits(n, m, k))
 
 
+def gemm_keeps_float32(n: int, m: int, k: int) -> bool:
+    """Whether an [n, k] x [m, k]^T product that is not split reaches a reader of partial sums as one float32 part."""
+    return bool(load().shk_gemm_bf16_keeps_float32(n, m, k))
+
+
 def gemm_parts(n: int, m: int, k: int, gated: bool = False) -> int:
     """Launches that an [n, k] x [m, k]^T product is made of (2: rows whose tiles
     fill whole rounds of the compute units, then the rest)."""

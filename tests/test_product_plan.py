@@ -27,6 +27,28 @@ def test_shares_keep_enough_of_k(m, k):
         assert s == 1 or -(-k // 32) // s >= 16
 
 
+SMALL = [(896, 896), (1152, 896), (896, 4864), (1000, 2056), (512, 3584), (2048, 2048), (1536, 1536), (256, 40), (10, 3584), (64, 520),
+         (1, 64), (300, 8192)]
+
+
+@pytest.mark.parametrize("m, k", SMALL)
+def test_small_matrices_are_planned_alike_for_every_row_count_of_a_graph_bucket(m, k):
+    for lo, hi in ((1, 16), (17, 32), (33, 64), (65, 128), (129, 256)):
+        assert len({(ops.gemm_splits(n, m, k), ops.gemm_keeps_float32(n, m, k), ops.gemm_parts(n, m, k))
+                    for n in range(lo, hi + 1)}) == 1, f"rows {lo}..{hi}"
+
+
+def test_small_matrices_formed_whole_reach_their_reader_in_float32():
+    """What the staged kernels would leave as float32 shares is not rounded to bfloat16 for being formed whole."""
+    for m, k, ns in ((896, 896, (17, 64)), (1152, 896, (17, 64)), (896, 4864, (65, 256)), (512, 3584, (65, 300))):
+        for n in ns:
+            assert ops.gemm_splits(n, m, k) == 1 and ops.gemm_keeps_float32(n, m, k), (m, k, n)
+    assert ops.gemm_splits(64, 896, 4864) == 2 and not ops.gemm_keeps_float32(64, 896, 4864)  # shares are float32 anyway
+    # never split, never kept: one token, large matrices, a short k
+    for m, k, n in ((896, 896, 1), (152064, 3584, 8), (18944, 3584, 4096), (896, 128, 64)):
+        assert ops.gemm_splits(n, m, k) == 1 and not ops.gemm_keeps_float32(n, m, k), (m, k, n)
+
+
 def test_matrices_that_fill_the_chip_are_not_split():
     assert ops.gemm_splits(8, 152064, 3584) == 1      # 9504 row blocks
     assert ops.gemm_splits(4096, 18944, 3584) == 1    # 592 tiles of 256 x 256

@@ -107,3 +107,31 @@ def test_gated_products_of_a_short_k(m, k):
         out = torch.full((n, m + 8), 7.0, device="cuda", dtype=torch.bfloat16)
         ops.gemm_tiled_weight(a[16 - n:], wt, m, k, out[:, :m], gated=True)
         assert torch.equal(out[:, :m], whole[16 - n:]) and bool((out[:, m:] == 7.0).all())
+
+
+@pytest.mark.parametrize("m, k, n", [(896, 896, 17), (896, 896, 64), (1152, 896, 40), (896, 4864, 65), (896, 4864, 256), (512, 3584, 300),
+                                     (64, 3584, 200), (896, 4864, 33)])
+def test_a_reader_of_shares_gets_small_products_unrounded(m, k, n):
+    """The residual after the reading norm is off by float32 roundings only, whether k was shared or not."""
+    from shrike_amd.engine.context import Workspace
+    from shrike_amd.engine.runtime import Runtime
+    from shrike_amd.kernels import ops
+
+    torch.manual_seed(m + k + n)
+    runtime, space = Runtime("cuda:0", torch.bfloat16), Workspace("cuda:0")
+
+    class Context:
+        buffer = staticmethod(space.get)
+
+    a, w = torch.randn(n, k, device="cuda").bfloat16(), torch.randn(m, k, device="cuda").bfloat16()
+    bias = torch.randn(m, device="cuda")
+    exact, size = a.double() @ w.double().t(), a.double().abs() @ w.double().abs().t()
+    bound = (k / 32 + 48) * 2.0**-24  # (as above, and one more for the residual's own sum)
+    resid = torch.randn(n, m, device="cuda")
+    want = resid.double() + exact
+    product = runtime.linear_deferred(Context, "p", a, runtime.weight(w))
+    ops.add_rmsnorm(resid, product, torch.ones(m, device="cuda"), 1e-6, torch.empty(n, m, device="cuda").bfloat16())
+    assert bool(((resid.double() - want).abs() <= bound * size + 2.0**-24 * want.abs()).all())
+    product = runtime.linear_deferred(Context, "q", a, runtime.weight(w), bias=bias, reader="position")
+    got = product.parts.double().sum(0) + (0 if product.bias is None else product.bias.double())
+    assert bool(((got - exact - bias.double()).abs() <= bound * (size + bias.double().abs())).all())
