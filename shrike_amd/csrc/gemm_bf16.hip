@@ -1420,27 +1420,57 @@ static int big_shape(int split, int n, int wblocks, int m, int k) {
 
 extern "C" int shk_gemm_bf16_splits(int n, int m, int k);
 
+// Up to 256 tokens n counts as the power of two above it: a choice made by it is then the same for every number
+// of tokens that a captured decode step may stand for.
+static int counted_tokens(int n) {
+  if (n > 256) return n;
+  int tokens = 32;
+  while (tokens < n) tokens *= 2;
+  return tokens;
+}
+
 // Which gemm_direct_kernel serves a product of n > 16 tokens (0: none): the smallest tile of which a launch has no
-// more than the 256 compute units (64 x 64: two a unit).  Limits as measured with k = 896 and 4864: matrices of 256
-// to 2,048 rows (more of them fill the staged kernels' larger tiles) and up to 10 MB; the two larger tiles only for a short k (4864 at 300 tokens: 23.5 us against 20.7).  Up to 256 tokens n counts as
-// the power of two above it: the choice is then the same for every number of tokens that a captured decode step may
-// stand for.
+// more than the 256 compute units, for matrices of 256 to 2,048 rows (more of them fill the staged kernels' larger
+// tiles), up to 10 MB and rows that are whole 16-byte pieces; in shares of k up to 64 tokens.  Against the staged kernels,
+// product and reading norm, over ten widths of 256 to 2,048, k from 128 to 14,336 and 17 to 4,096 tokens: 0.36 to 1.0 of
+// their time with up to 8,192 of k in the two smaller tiles (to 1.4 beyond), up to 2,048 in the two larger ones (k = 4864 at 300
+// tokens 23.5 us against 20.7).  64 x 64 with two workgroups a unit 0.81 to 1.0 up to k = 512, up to 352 of them 0.88 to
+// 1.0 up to k = 1024; beyond, 1024 x 2048 at 1,119 tokens 30 us against 27, 512 x 1024 at 4,096 30.3 against 26.5.
 struct DirectTile {
-  int rows, tokens, most;
+  int rows, tokens, most_k, waves;
 };
-static const DirectTile kDirect[5] = {{0, 0, 0}, {32, 16, 256}, {32, 32, 256}, {32, 64, 256}, {64, 64, 512}};
+static const DirectTile kDirect[5] = {{0, 0, 0, 0}, {32, 16, 8192, 8}, {32, 32, 8192, 4}, {32, 64, 2048, 8}, {64, 64, 2048, 4}};
 
 static int direct_shape(int n, int m, int k, int ksplit) {
-  if (n <= 16 || m < 256 || m > 2048 || static_cast<long long>(m) * k > 5 * 1000 * 1000) return 0;
-  int tokens = n;
-  if (n <= 256)
-    for (tokens = 32; tokens < n;) tokens *= 2;
-  for (int shape = 1; shape <= (k <= 2048 ? 4 : 2); ++shape) {
+  if (n <= 16 || (n > 64 && ksplit > 1) || m < 256 || m > 2048 || k % 8 || static_cast<long long>(m) * k > 5 * 1000 * 1000)
+    return 0;
+  const int tokens = counted_tokens(n);
+  for (int shape = 1; shape <= (ksplit > 1 ? 2 : 4); ++shape) {
     const DirectTile& t = kDirect[shape];
-    const long long count = static_cast<long long>((m + t.rows - 1) / t.rows) * ((tokens + t.tokens - 1) / t.tokens);
-    if (count * ksplit <= t.most) return shape;
+    long long count = static_cast<long long>((m + t.rows - 1) / t.rows) * ((tokens + t.tokens - 1) / t.tokens);
+    if (ksplit > 1) count = (count + kDies - 1) / kDies * kDies;  // (as launched)
+    const int most = shape < 4 || k > 1024 ? 256 : k > 512 ? 352 : 512;
+    if (k / ksplit <= t.most_k && count * ksplit <= most) return shape;
   }
   return 0;
+}
+
+// Shares of k for gemm_direct_kernel, 0 where it does not serve the product.  Up to 64 tokens: a wavefront of the
+// smaller tiles takes four tiles of k a step, about a microsecond, a share costs its reader 0.15.  Product and
+// reading norm at 17 / 64 tokens: 512 x 2048 8.2 / 8.2 us in two shares against 9.1 whole and 8.0 / 10.5 in the streaming kernel's
+// eight, 512 x 3584 8.1 / 8.3 in four (9.4 in two; 8.9 / 11.8), 896 x 4864 9.6 / 10.9 in three and two (10.4 / 13.8), 256
+// x 8192 8.8 / 8.9 in eight (12.1 in two; 10.8 / 14.4).
+static int direct_splits(int n, int m, int k) {
+  int best = 0;
+  double least = 0.0;
+  for (int shares = 1; shares <= (n <= 64 ? 8 : 1); ++shares) {
+    const int shape = direct_shape(n, m, k, shares);
+    if (!shape) continue;
+    const int tiles = ((k + 31) / 32 + shares - 1) / shares, a_wave = (tiles + kDirect[shape].waves - 1) / kDirect[shape].waves;
+    const double us = (a_wave + 3) / 4 + 0.15 * shares;
+    if (!best || us < least) least = us, best = shares;
+  }
+  return best;
 }
 
 template <int RT, int CT, int KW, int U>
@@ -1453,6 +1483,15 @@ static void launch_direct(hipStream_t s, const bf16* ap, int lda, int n, int k, 
 
 // Matrices of so few rows that many tokens go to gemm_skinny_kernel, group by group.
 static bool few_rows(int m) { return m <= 64; }
+
+// Whether it also beats the staged kernels' shares of k with the kernel that adds them up: up to k = 4096 with two
+// workgroups a compute unit (64 x 3584 at 2,048 tokens 0.85 of their time, 48 x 3584 at 3,000 27 us against 22), up to
+// 8,192 where they are neither few nor more than one a unit (32 x 8192 at 256 tokens 0.92; 16 x 8192 at 65 17.5 us
+// against 13, 64 x 8192 at 1,119 27 against 21); 48 x 14336 28 to 32 us against 22 to 24.
+static bool few_rows_whole(int n, int m, int k) {
+  const int groups = (m + 15) / 16 * ((counted_tokens(n) + 15) / 16);
+  return k <= 4096 ? groups <= 512 : k <= 8192 && m > 16 && groups >= 32 && groups <= 256;
+}
 
 // 256 x 256 tiles that do not make whole rounds of the 256 compute units (296 of them:
 // two rounds, the second nearly empty) are better run as two products: the row tiles
@@ -1543,11 +1582,9 @@ static int staged_splits(int n, int m, int k) {
 }
 
 extern "C" int shk_gemm_bf16_splits(int n, int m, int k) {
-  if (n > 64 && few_rows(m)) return 1;
-  // (a long k in two shares up to 64 tokens: 896 x 4864 7.4 us against 10.0 whole, the second share costs its reader
-  // half a microsecond)
-  const int direct = n <= 64 && k > 2048 ? 2 : 1;
-  return direct_shape(n, m, k, direct) ? direct : staged_splits(n, m, k);
+  if (n > 64 && few_rows(m) && few_rows_whole(n, m, k)) return 1;
+  const int direct = direct_splits(n, m, k);
+  return direct ? direct : staged_splits(n, m, k);
 }
 
 // Whether a reader that adds up shares gets an unsplit product as one float32 share all the same: where
@@ -1732,7 +1769,8 @@ extern "C" int shk_gemm_bf16_tiled_weight(const void* a, const void* wt, const f
   }
   // wavefronts per workgroup: matrices with few row blocks get more of them
   // (but a gated matrix whose blocks alone fill the 256 compute units and whose k is a tile or two for each of 16
-  // takes four: 2 x 4864 rows of 896 at 1 / 8 / 16 tokens 5.8 / 6.2 / 6.9 us against 6.5 / 6.8 / 7.3)
+  // takes four: 2 x 4864 rows of 896 at 1 / 8 / 16 tokens 5.8 / 6.2 / 6.9 us against 6.5 / 6.8 / 7.3; 0.58 to 0.98 of the
+  // time over 4,096 to 8,176 rows of 256 to 1,024)
   const bool short_gated = gated && mb >= 256 && mb < 512 && kt <= 32;
   const int waves = (mb >= 512) ? 8 : (ksplit > 1 || short_gated) ? 4 : 16;
   const int max_waves = 16;

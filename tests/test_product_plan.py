@@ -43,10 +43,23 @@ def test_small_matrices_formed_whole_reach_their_reader_in_float32():
     for m, k, ns in ((896, 896, (17, 64)), (1152, 896, (17, 64)), (896, 4864, (65, 256)), (512, 3584, (65, 300))):
         for n in ns:
             assert ops.gemm_splits(n, m, k) == 1 and ops.gemm_keeps_float32(n, m, k), (m, k, n)
-    assert ops.gemm_splits(64, 896, 4864) == 2 and not ops.gemm_keeps_float32(64, 896, 4864)  # shares are float32 anyway
+    assert ops.gemm_splits(64, 896, 4864) > 1 and not ops.gemm_keeps_float32(64, 896, 4864)  # shares are float32 anyway
     # never split, never kept: one token, large matrices, a short k
     for m, k, n in ((896, 896, 1), (152064, 3584, 8), (18944, 3584, 4096), (896, 128, 64)):
         assert ops.gemm_splits(n, m, k) == 1 and not ops.gemm_keeps_float32(n, m, k), (m, k, n)
+
+
+def test_a_long_k_is_shared_where_one_walk_along_it_takes_longer():
+    for n in (17, 64):
+        assert ops.gemm_splits(n, 512, 1024) == 1 and ops.gemm_splits(n, 512, 2048) == 2 and ops.gemm_splits(n, 512, 3584) == 4
+        assert ops.gemm_splits(n, 256, 8192) == 8 and ops.gemm_splits(n, 896, 4864) >= 2
+    # few rows: whole, but not a long k in a handful of workgroups or in more than the compute units take at once
+    assert ops.gemm_splits(1501, 10, 3584) == 1 and ops.gemm_splits(256, 32, 8192) == 1
+    assert ops.gemm_splits(65, 16, 8192) > 1 and ops.gemm_splits(1501, 64, 8192) > 1 and ops.gemm_splits(4096, 64, 3584) > 1
+    # small matrices: not where the staged kernels' larger tiles fill the chip
+    assert ops.gemm_splits(1119, 1024, 2048) == 2 and ops.gemm_splits(640, 256, 14336) > 8
+    # rows that are no whole 16-byte pieces keep the shares of the kernels that take them
+    assert ops.gemm_splits(64, 896, 4860) == ops.gemm_splits(64, 896, 4861) > 1
 
 
 def test_matrices_that_fill_the_chip_are_not_split():
