@@ -775,11 +775,11 @@ static void launch_big(const bf16* a, const int32_t* order, const int32_t* count
 
 // out[t, c] = add[t, c] + sum_k weights[t, k] * pair_out[t * top + k, c], k in the order chosen; an identity
 // expert's output is x[t, c].  Eight columns a thread (width is a multiple of 8): 16-byte loads and stores, 25 us
-// at 1,501 tokens of 3584 with one column a thread, 13 so.
+// at 1,501 tokens of 3584 with one column a thread, 13 so.  wide: add and out are 16-byte aligned, else element by element.
 __global__ void __launch_bounds__(256)
     moe_join_kernel(const float* __restrict__ pair_out, const int32_t* __restrict__ chosen, const bf16* __restrict__ x,
                     const float* __restrict__ weights, const bf16* __restrict__ add, const float* __restrict__ add_gate,
-                    int gate_ld, bf16* __restrict__ out, int width, int top, int experts) {
+                    int gate_ld, bf16* __restrict__ out, int width, int top, int experts, int wide) {
   union Eight {
     uint4 u;
     bf16 h[8];
@@ -808,7 +808,11 @@ __global__ void __launch_bounds__(256)
   }
   if (add) {
     Eight v;
-    v.u = *reinterpret_cast<const uint4*>(add + at);
+    if (wide)
+      v.u = *reinterpret_cast<const uint4*>(add + at);
+    else
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v.h[i] = add[at + i];
     const float share = shared_share(add_gate, gate_ld, t);
 #pragma unroll
     for (int i = 0; i < 8; ++i) total[i] += share * to_float(v.h[i]);
@@ -816,7 +820,11 @@ __global__ void __launch_bounds__(256)
   Eight v;
 #pragma unroll
   for (int i = 0; i < 8; ++i) v.h[i] = from_float<bf16>(total[i]);
-  *reinterpret_cast<uint4*>(out + at) = v.u;
+  if (wide)
+    *reinterpret_cast<uint4*>(out + at) = v.u;
+  else
+#pragma unroll
+    for (int i = 0; i < 8; ++i) out[at + i] = v.h[i];
 }
 
 }  // namespace shk
@@ -899,8 +907,7 @@ extern "C" int shk_moe_experts_grouped(const void* x, const int32_t* chosen, con
               "moe_experts_grouped: too many (token, expert) pairs");
   SHK_REQUIRE(x && chosen && weights && w_gate && w_up && w_down && act_buf && out && scratch,
               "moe_experts_grouped: null pointer");
-  for (const void* p : {x, w_gate, w_up, w_down, add, static_cast<const void*>(act_buf), static_cast<const void*>(scratch),
-                        static_cast<const void*>(out)})
+  for (const void* p : {x, w_gate, w_up, w_down, static_cast<const void*>(act_buf), static_cast<const void*>(scratch)})
     SHK_REQUIRE(reinterpret_cast<uintptr_t>(p) % 16 == 0, "moe_experts_grouped: operands must be 16-byte aligned");
   hipStream_t s = static_cast<hipStream_t>(stream);
   const GateForm form{act, limit, shift};
@@ -942,9 +949,10 @@ extern "C" int shk_moe_experts_grouped(const void* x, const int32_t* chosen, con
     down<<<columns, 256, 0, s>>>(actb, order, counts, static_cast<const bf16*>(w_down), pair_out, n, width, ff, top);
   }
   const int join_threads = width >= 2048 ? 256 : kWave;
-  moe_join_kernel<<<dim3((width / 8 + join_threads - 1) / join_threads, n), join_threads, 0, s>>>(pair_out, chosen, static_cast<const bf16*>(x), weights,
-                                                               static_cast<const bf16*>(add), add_gate, gate_ld,
-                                                               static_cast<bf16*>(out), width, top, experts);
+  const int wide = reinterpret_cast<uintptr_t>(add) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
+  moe_join_kernel<<<dim3((width / 8 + join_threads - 1) / join_threads, n), join_threads, 0, s>>>(
+      pair_out, chosen, static_cast<const bf16*>(x), weights, static_cast<const bf16*>(add), add_gate, gate_ld,
+      static_cast<bf16*>(out), width, top, experts, wide);
   SHK_LAUNCH_CHECK("moe_experts_grouped");
   return 0;
 }

@@ -68,3 +68,32 @@ def test_lists_of_every_length(width, ff, counts, form):
     assert torch.equal(*both)
     # the activations are rounded to bfloat16 (2^-9 of each), the result once more; float32 sums add little
     assert bool(((out.double() - want).abs() <= 2.0**-8 * size + 1e-3).all())
+
+
+@pytest.mark.parametrize("off_add, off_out", [(1, 0), (0, 1), (3, 5)])
+@pytest.mark.parametrize("n, width, ff, tiled", [(6, 128, 64, True), (300, 64, 64, True), (6, 72, 40, False)])
+def test_added_rows_and_results_anywhere_in_memory(n, width, ff, tiled, off_add, off_out):
+    """`add` and `out` need not be 16-byte aligned: the same bits as where they are."""
+    from shrike_amd.kernels import ops
+
+    torch.manual_seed(n + width)
+    experts, top = 4, 2
+    x = torch.randn(n, width, device="cuda").bfloat16()
+    matrices = [torch.randn(experts, r, c, device="cuda").bfloat16() for r, c in ((ff, width), (ff, width), (width, ff))]
+    if tiled:
+        matrices = [ops.tile_experts(w) for w in matrices]
+    chosen, weights = torch.randint(0, experts + 1, (n, top), device="cuda").int(), torch.rand(n, top, device="cuda")
+    added = torch.randn(n, width, device="cuda").bfloat16()
+    scratch = torch.empty(ops.moe_grouped_scratch_bytes(n, width, experts, top), device="cuda", dtype=torch.uint8)
+    act_buf = torch.empty(n * top, ff, device="cuda", dtype=torch.bfloat16)
+
+    def run(off_add, off_out):
+        add = torch.zeros(n * width + 16, device="cuda", dtype=torch.bfloat16)[off_add : off_add + n * width].view(n, width)
+        add.copy_(added)
+        flat = torch.full((n * width + 16,), 5.0, device="cuda", dtype=torch.bfloat16)
+        out = flat[off_out : off_out + n * width].view(n, width)
+        ops.moe_experts(x, chosen, weights, *matrices, act_buf, out, "silu", add=add, scratch=scratch, identity=1, tiled=tiled)
+        assert bool((flat[:off_out] == 5.0).all()) and bool((flat[off_out + n * width :] == 5.0).all())
+        return out
+
+    assert torch.equal(run(off_add, off_out), run(0, 0))
