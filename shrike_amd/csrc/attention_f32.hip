@@ -173,6 +173,8 @@ __global__ void __launch_bounds__(kWave * kBlockWaves) attention_f32_kernel(F32A
     float m = tops[0][i];
 #pragma unroll
     for (int w = 1; w < kBlockWaves; ++w) m = fmaxf(m, tops[w][i]);
+    // (scores may be -infinity by themselves, from a table of distances or an overflow: a block of them has weights of 0)
+    const float origin = m == -INFINITY ? 0.f : m;
 
     float l = 0.f;
     af4 acc[D];
@@ -188,7 +190,7 @@ __global__ void __launch_bounds__(kWave * kBlockWaves) attention_f32_kernel(F32A
         for (int e = 0; e < 4; ++e) {
           const int key = key0 + 16 * u + 4 * kg + e;
           const bool have = key >= lo && key <= pos && v_at[u] >= 0;
-          const float w = have ? expf(s[u][e] - m) : 0.f;
+          const float w = have ? expf(s[u][e] - origin) : 0.f;
           l += w;
 #pragma unroll
           for (int x = 0; x < D; ++x)

@@ -71,3 +71,42 @@ def test_edges_of_the_blocks(heads, kv_heads, head_dim, v_dim, page, window, chu
             # a score of size ~10 is off by some ulp, a weight by as much relatively; the sums add half an ulp
             # of values of order one a term, a few hundred terms weighted to one
             assert torch.allclose(whole[t, h * v_dim : (h + 1) * v_dim].double(), want, atol=2e-5, rtol=0), (t, h)
+
+
+@pytest.mark.parametrize("splits", [1, 3])
+@pytest.mark.parametrize("sinks", [False, True])
+def test_scores_of_minus_infinity(splits, sinks):
+    """A table of distances that rules out the nearest keys, whole blocks of them, or the far ones: what is left is the
+    softmax; where nothing is left, nothing beside the sink, or no number without one."""
+    from shrike_amd.kernels import ops
+
+    torch.manual_seed(3)
+    heads, dim, page, ctx = 4, 32, 16, 1024
+    k_pool = torch.randn(ctx // page, 1, dim // ops.key_slab(dim), page, ops.key_slab(dim), device="cuda")
+    v_pool = torch.randn(ctx // page, 1, dim, page, device="cuda")
+    tables = torch.arange(ctx // page, device="cuda").int().view(1, -1)
+    keys = k_pool.permute(0, 3, 1, 2, 4).reshape(ctx, dim)
+    values = v_pool.permute(0, 3, 1, 2).reshape(ctx, dim)
+    positions = torch.tensor([5, 255, 256, 700, 1023], dtype=torch.int32, device="cuda")
+    n = positions.numel()
+    q = torch.randn(n, heads * dim, device="cuda")
+    bias = torch.randn(heads, 1024, device="cuda")
+    bias[0, :300] = -float("inf")  # the nearest block and more
+    bias[1, 10:] = -float("inf")  # all but the nearest ten: whole blocks in front
+    bias[2, 100:900] = -float("inf")
+    sink = torch.randn(heads, device="cuda") if sinks else None
+    out = torch.full((n, heads * dim), 9.0, device="cuda")
+    partial = torch.full((ops.attention_partial_floats(n, heads, dim, ctx // page, page),), float("nan"), device="cuda")
+    ops.attention(q, out, heads, 1, dim, positions, torch.zeros(n, dtype=torch.int32, device="cuda"), tables, k_pool, v_pool, page, None,
+                  dim**-0.5, dist_bias=bias, sinks=sink, **(dict(partial=partial, splits=splits) if splits > 1 else {}))
+    got = out.view(n, heads, dim).double()
+    for t, pos in enumerate(positions.tolist()):
+        for h in range(heads):
+            s = keys[: pos + 1].double() @ q[t, h * dim : (h + 1) * dim].double() * dim**-0.5
+            s = s + bias[h, pos - torch.arange(pos + 1, device="cuda")].double()
+            top = torch.cat([s, sink[h : h + 1].double()]) if sinks else s
+            if bool(torch.isinf(top).all()):
+                assert bool(torch.isnan(got[t, h]).all())
+                continue
+            want = torch.exp(s - torch.logsumexp(top, 0)) @ values[: pos + 1].double()
+            assert torch.allclose(got[t, h], want, atol=2e-5, rtol=0), (t, h)
