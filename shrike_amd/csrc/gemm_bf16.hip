@@ -16,6 +16,7 @@
 
 #include "api.h"
 #include "common.h"
+#include "to_lds.h"
 
 namespace shk {
 
@@ -766,15 +767,6 @@ __global__ void __launch_bounds__(GM* GN* kWave)
 // loads issued since) before the barrier.  Each buffer is an LDS array of its
 // own, so that the compiler's own bookkeeping tells the buffers apart and adds
 // no wait for loads into another one.
-#define SHK_LOAD_TO_LDS(gptr, lptr)                                                        \
-  __builtin_amdgcn_global_load_lds(                                                       \
-      reinterpret_cast<const __attribute__((address_space(1))) void*>(                    \
-          reinterpret_cast<uintptr_t>(gptr)),                                             \
-      (__attribute__((address_space(3))) void*)(lptr), 16, 0, 0)
-
-// s_waitcnt vmcnt(n) alone (gfx9 encoding: vmcnt in bits 3:0 and 15:14, the other counters at their maxima)
-#define SHK_WAIT_LOADS(n) __builtin_amdgcn_s_waitcnt(0x0f70 | ((n) & 15) | (((n) >> 4) << 14))
-
 template <int GM, int GN, int WM, int WN, int KS, bool GATED>
 __global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per_eu(GM * GN >= 16 ? 4 : 2)))
     gemm_big_lds_kernel(const bf16* __restrict__ a, int lda, int n, int k,
@@ -875,10 +867,7 @@ __global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per
   // own loads (the younger stages may stay in flight) and met the others; after the
   // barrier nobody reads the stage before any more, so its buffer takes new loads.
 #define SHK_LDS_STEP(now, refill, st_refill)  \
-  SHK_WAIT_LOADS((NS - 2) * kLoads);          \
-  asm volatile("" ::: "memory");              \
-  __builtin_amdgcn_s_barrier();               \
-  asm volatile("" ::: "memory");              \
+  SHK_MEET_WITH_LOADS((NS - 2) * kLoads);     \
   load(refill, st_refill);                    \
   __builtin_amdgcn_sched_barrier(0);          \
   multiply(now);
@@ -1125,10 +1114,7 @@ __global__ void __launch_bounds__(16 * kWave)
   // the barrier nobody reads the stage before any more, so its buffer and its
   // registers take the loads of the stage after next.
 #define SHK_STREAM_STEP(buf_now, w_now, buf_fill, w_fill, st_fill, tiles) \
-  SHK_WAIT_LOADS(kLoads);                                                  \
-  asm volatile("" ::: "memory");                                           \
-  __builtin_amdgcn_s_barrier();                                            \
-  asm volatile("" ::: "memory");                                           \
+  SHK_MEET_WITH_LOADS(kLoads);                                             \
   fetch(buf_fill, w_fill, st_fill);                                        \
   __builtin_amdgcn_sched_barrier(0);                                       \
   multiply(buf_now, w_now, tiles);

@@ -29,6 +29,7 @@
 // are kept in float32 and joined per token in the order the experts were chosen.
 #include "api.h"
 #include "common.h"
+#include "to_lds.h"
 
 namespace shk {
 
@@ -605,13 +606,6 @@ __global__ void __launch_bounds__(256)
 // for the empty half of a list's last tile: the loads are what takes the time, about 42 GB/s a compute unit.
 constexpr int kBigPairs = 128, kBigRows = 256, kBigWaves = 8;
 
-#define SHK_MOE_TO_LDS(gptr, lptr)                                                                             \
-  __builtin_amdgcn_global_load_lds(                                                                           \
-      reinterpret_cast<const __attribute__((address_space(1))) void*>(reinterpret_cast<uintptr_t>(gptr)),     \
-      (__attribute__((address_space(3))) void*)(lptr), 16, 0, 0)
-// s_waitcnt vmcnt(n) alone
-#define SHK_MOE_WAIT(n) __builtin_amdgcn_s_waitcnt(0x0f70 | ((n) & 15) | (((n) >> 4) << 14))
-
 // Tile `index` of all experts' live tiles (features x ceil(count / kBigPairs) each): expert, first feature
 // tile, first pair; false beyond the last.  `index` < 0 asks for none and returns their number in `total`.
 __device__ __forceinline__ bool moe_tile(const int32_t* counts, int experts, int n, int features, int index, int lane,
@@ -690,7 +684,7 @@ __global__ void __launch_bounds__(kBigWaves* kWave)
   auto load = [&](u4 (&buf)[kUnits][kWave], int st) {
     const size_t at = static_cast<size_t>(st < stages ? st : 0) * 64;  // past the end: any stage, never multiplied
 #pragma unroll
-    for (int i = 0; i < kLoads; ++i) SHK_MOE_TO_LDS(src[i] + (i < kWLoads ? at * 16 : at), &buf[wave + kBigWaves * i][0]);
+    for (int i = 0; i < kLoads; ++i) SHK_LOAD_TO_LDS(src[i] + (i < kWLoads ? at * 16 : at), &buf[wave + kBigWaves * i][0]);
   };
   mf32x4 acc[WM][WN];
 #pragma unroll
@@ -717,10 +711,7 @@ __global__ void __launch_bounds__(kBigWaves* kWave)
   // a stage has landed for every wavefront once each has waited for its own loads of it (the younger stage's
   // may stay in flight) and met the others; after the barrier nobody reads the stage before any more
 #define SHK_MOE_STEP(now, refill, st_refill) \
-  SHK_MOE_WAIT(kLoads);                      \
-  asm volatile("" ::: "memory");             \
-  __builtin_amdgcn_s_barrier();              \
-  asm volatile("" ::: "memory");             \
+  SHK_MEET_WITH_LOADS(kLoads);               \
   load(refill, st_refill);                   \
   __builtin_amdgcn_sched_barrier(0);         \
   multiply(now);
@@ -735,7 +726,7 @@ __global__ void __launch_bounds__(kBigWaves* kWave)
   if (st < stages) { SHK_MOE_STEP(stage0, stage2, st + 2) }
   if (st + 1 < stages) { SHK_MOE_STEP(stage1, stage0, st + 3) }
 #undef SHK_MOE_STEP
-  SHK_MOE_WAIT(0);  // no load may arrive in LDS that the workgroup has given back
+  SHK_WAIT_LOADS(0);  // no load may arrive in LDS that the workgroup has given back
 
   // lane (j, kg) holds weight rows 4 kg + r of a tile for pair j
   const int j = lane % 16, kg = lane / 16;
