@@ -63,6 +63,9 @@ class LLMEngine:
             reserve = workspace_reserve(model, runtime, cfg)
             free, _total = torch.cuda.mem_get_info(runtime.device)
             per_page = max(1, probe.bytes_per_page(elem))
+            # the longest context that the pool or the model could hold makes some buffers larger
+            keys = int(max(0, free - reserve) * cfg.gpu_mem_util) // per_page * cfg.block_size
+            reserve += context_reserve(model, cfg, min(keys, model.spec.max_position_embeddings or keys))
             num_blocks = max(1, int(max(0, free - reserve) * cfg.gpu_mem_util) // per_page)
         self.cache = CacheManager(specs, cfg.block_size, num_blocks, max_slots=cfg.max_running,
                                   enable_prefix_caching=cfg.enable_prefix_caching)
@@ -282,6 +285,17 @@ def workspace_reserve(model, runtime, cfg: EngineConfig) -> int:
                                             model.spec.vocab_size)
     slack = 64 << 20  # graph objects, page-locked staging
     return 2 * sizes[0] + sizes[1] + sampler + slack
+
+
+def context_reserve(model, cfg: EngineConfig, keys: int) -> int:
+    """Bytes that single-token steps' buffers take beyond workspace_reserve() once contexts have grown to `keys`
+    tokens: each batch bucket's graphs keep what they have outgrown (sizes go up in powers of two), steps outside of
+    graphs have one buffer more."""
+    from .runner import GRAPH_BATCH_BUCKETS
+
+    rows = min(cfg.max_running, cfg.max_tokens_per_step, GRAPH_BATCH_BUCKETS[-1])
+    sizes = [model.context_scratch_bytes(b, max(1, keys)) for b in GRAPH_BATCH_BUCKETS if b < 2 * rows]
+    return 2 * sum(sizes) + max(sizes)
 
 
 class LLM:

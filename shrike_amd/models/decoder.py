@@ -81,6 +81,10 @@ class DecoderModel:
         list of launches for any later step of the same shape."""
         return all(part.launches_follow_shape for part in self.parts())
 
+    def context_scratch_bytes(self, rows: int, keys: int) -> int:
+        """The largest of its mixers': layers share a step's buffers."""
+        return max((block.mixer.context_scratch_bytes(rows, keys) for block in self.blocks), default=0)
+
     def cache_specs(self) -> list:
         """Cache need of every schedule position (for a position that reads another
         position's cache, what its mixer keeps beside that; None where nothing is kept), and after

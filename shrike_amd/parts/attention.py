@@ -99,6 +99,20 @@ def decode_shares(num_seqs: int, kv_heads: int, head_dim: int, max_ctx: int) -> 
     return splits, 4
 
 
+F32_SPLIT_SCRATCH = 512 << 20  # bytes: the most that single tokens' blocks of keys side by side may take
+
+
+def f32_split_floats(rows: int, heads: int, kv_heads: int, value_dim: int, keys: int) -> int:
+    """Scratch (float32 numbers) with which float32 attention forms `rows` single tokens' blocks of keys in workgroups
+    of their own, for tables of up to `keys` keys; 0 where a workgroup takes all of a token's blocks: one block, or
+    rows enough to fill the chip, or more scratch than F32_SPLIT_SCRATCH.  Counted for a power of two of blocks: a
+    workspace that keeps what it has outgrown then holds at most twice the newest buffer however a context
+    grows."""
+    blocks = -(-keys // ops.ATTENTION_KEY_BLOCK)
+    floats = rows * heads * _pow2(blocks) * (value_dim + 2)
+    return 0 if blocks <= 1 or rows * kv_heads >= 2 * compute_units() or 4 * floats > F32_SPLIT_SCRATCH else floats
+
+
 def decode_streams(num_seqs: int, kv_heads: int, head_dim: int, max_ctx: int, window: int | None = None) -> bool:
     """Whether a decode launch reads so many keys and values that non-temporal
     loads pay (measured with 4 key/value heads of 128: a tenth faster from 64
@@ -354,6 +368,12 @@ class PagedAttention(Mixer):
                 self.talking, self.value_dim, self._qkv_width(), bool(getattr(s, "bucket_bias", None)),
                 bool(getattr(s, "softcap", None)), bool(getattr(s, "sinks", False)))
 
+    def context_scratch_bytes(self, rows: int, keys: int) -> int:
+        s = self.spec
+        if self.dtype != torch.float32 or self.talking:
+            return 0
+        return 4 * f32_split_floats(rows, s.num_heads, s.num_kv_heads, self.value_dim, keys)
+
     def prepare(self, shape) -> None:
         """Decides once per step and head geometry how attention is launched:
         the key splits of single-token rows, and for prompt portions the kernel
@@ -483,10 +503,10 @@ class PagedAttention(Mixer):
             if self.dtype == torch.float32 and ctx.num_decode == ctx.num_tokens:
                 # few single tokens: their blocks of keys side by side (as many as the tables are wide: what a
                 # replayed launch must serve; the result is the same bits)
-                blocks = -(-tables.shape[1] * cache.page_size // ops.ATTENTION_KEY_BLOCK)
-                if blocks > 1 and ctx.num_tokens * hkv < 2 * compute_units():
-                    splits = min(blocks, MAX_KEY_SPLITS)
-                    floats = ops.attention_partial_floats(ctx.num_tokens, h, self.value_dim, tables.shape[1], cache.page_size)
+                keys = tables.shape[1] * cache.page_size
+                floats = f32_split_floats(ctx.num_tokens, h, hkv, self.value_dim, keys)
+                if floats:
+                    splits = min(-(-keys // ops.ATTENTION_KEY_BLOCK), MAX_KEY_SPLITS)
                     partial = ctx.buffer("attn_f32_partial", (floats,), torch.float32)
             ops.attention(q, out, h, hkv, d, ctx.positions, ctx.token_seq, tables, cache.pools["k"],
                           cache.pools["v"], cache.page_size, s.window, s.scale, chunk=s.chunk,

@@ -267,6 +267,11 @@ class Mixer(Part):
         CompositeSpec whose entries join those that are read in the LayerCache's `parts`."""
         return None
 
+    def context_scratch_bytes(self, rows: int, keys: int) -> int:
+        """Bytes of the buffer that a step of `rows` single tokens takes beyond what a step of short contexts does,
+        once one of them has `keys` tokens in the cache."""
+        return 0
+
     def forward(self, ctx, x: torch.Tensor, cache) -> torch.Tensor:
         raise NotImplementedError
 

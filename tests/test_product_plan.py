@@ -204,3 +204,51 @@ def test_where_a_product_runs_in_two_parts():
     assert ops.gemm_parts(2048, 18944, 3584, True) == 1   # 1,184 tiles: the rest would take a round of its own anyway
     assert ops.gemm_parts(512, 3584, 18944) == 1          # shares of k instead
     assert ops.gemm_parts(2048, 13824, 5120, True) == 2   # 864 tiles: three whole rounds, then 96 tiles' rows in smaller tiles
+
+
+def test_scratch_of_float32_decode_attention_stays_near_what_is_in_use():
+    """A context that crosses every table width up to 128k tokens, in a workspace whose graphs keep what it outgrew."""
+    import torch
+
+    from shrike_amd.engine.context import Workspace
+    from shrike_amd.engine.runner import GRAPH_TABLE_QUANTUM
+    from shrike_amd.kernels import ops
+    from shrike_amd.parts.attention import F32_SPLIT_SCRATCH, f32_split_floats
+
+    page, heads, kv_heads, dim = 16, 14, 2, 64
+    for rows in (1, 4):
+        space, live = Workspace("cpu", keep_outgrown=True), 0
+        for width in range(GRAPH_TABLE_QUANTUM, 8192 + 1, GRAPH_TABLE_QUANTUM):
+            floats = f32_split_floats(rows, heads, kv_heads, dim, width * page)
+            assert floats >= ops.attention_partial_floats(rows, heads, dim, width, page)
+            live = max(live, 4 * space.get("p", (floats,), torch.float32).numel())
+        assert live == 4 * rows * heads * 512 * (dim + 2)
+        assert space.nbytes() <= 2 * live and space.generation <= 10
+    # none for one block, for rows that fill the chip, or beyond the limit
+    assert f32_split_floats(1, heads, kv_heads, dim, 256) == 0 and f32_split_floats(1, heads, kv_heads, dim, 257) > 0
+    assert f32_split_floats(256, heads, kv_heads, dim, 4096) == 0
+    for rows in (1, 8, 64, 255):
+        for keys in (1 << 12, 1 << 17, 1 << 20, 1 << 24):
+            assert 4 * f32_split_floats(rows, 28, 1, 128, keys) <= F32_SPLIT_SCRATCH
+
+
+def test_the_reserve_counts_scratch_that_grows_with_the_context():
+    import torch
+
+    from shrike_amd.config import AttentionSpec, BlockSpec, EngineConfig, ModelSpec, RMSNormSpec, SwiGLUSpec
+    from shrike_amd.engine.llm_engine import context_reserve
+    from shrike_amd.models import DecoderModel
+
+    norm = RMSNormSpec(eps=1e-6)
+    mixer = AttentionSpec(num_heads=14, num_kv_heads=2, head_dim=64, qkv_bias=True, out_bias=False, scale=0.1)
+    block = BlockSpec(name="model.layers.0", mixer=mixer, ffn=SwiGLUSpec(intermediate_size=64), mixer_norm=norm, ffn_norm=norm)
+    model = DecoderModel(ModelSpec(architecture="t", hidden_size=896, vocab_size=100, blocks=(block,), final_norm=norm,
+                                   tie_word_embeddings=False))
+    cfg = EngineConfig(max_running=100)
+    model.blocks[0].mixer.dtype = torch.bfloat16
+    assert context_reserve(model, cfg, 32768) == 0
+    model.blocks[0].mixer.dtype = torch.float32
+    row = 14 * 128 * 66 * 4  # bytes a row at 32,768 keys
+    assert context_reserve(model, cfg, 32768) == 2 * 255 * row + 128 * row  # buckets 1 to 128, the largest once more
+    assert context_reserve(model, EngineConfig(max_running=1), 32768) == 3 * row
+    assert context_reserve(model, cfg, 100) == 0
