@@ -297,11 +297,11 @@ int shk_latent_attention_bf16(const void* q, void* out, int n, int heads, int ke
                               int chunk, float scale, float* partial, int nsplit, int tokens_per_group,
                               void* stream);
 // The same for the tokens of prompt portions (n tokens, positions rising along each sequence's) where
-// shk_latent_prompt_tokens, the tokens a workgroup serves, is not 0.
+// shk_latent_prompt_tokens, the most tokens that a workgroup serves, is not 0; `tokens`: as many a workgroup (0: the most).
 int shk_latent_prompt_tokens(int heads, int key_dim, int v_dim);
 int shk_latent_prompt_bf16(const void* q, void* out, int n, int heads, int key_dim, int v_dim, const int32_t* positions,
                            const int32_t* token_seq, const int32_t* tables, int table_stride, const void* pool,
-                           int page_size, int num_pages, int window, int chunk, float scale, float* partial, int nsplit,
+                           int page_size, int num_pages, int window, int chunk, float scale, float* partial, int nsplit, int tokens,
                            void* stream);
 
 // A batch of products of one shape: out_b[n, m] = a_b[n, k] @ w_b[m, k]^T for b < batch, with

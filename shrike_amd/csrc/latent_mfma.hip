@@ -258,7 +258,7 @@ __global__ void __launch_bounds__(kLatentWaves* kWave)
 // matrix instructions where the kernel above uses it once, and a chunk is staged once for tpw tokens.  Two
 // buffers for the rows and for the weights: two barriers a chunk.
 // What bounded the kernel above over a prompt was its LDS reads, 288 for 60 matrix instructions a chunk and
-// wavefront: 28 heads over rows of 512, 1,501 tokens, 468 us a layer, 200 here; rows straight into LDS instead
+// wavefront: 28 heads over rows of 512, 1,501 tokens, 468 us a layer, 186 here (202 with results of two bytes a store); rows straight into LDS instead
 // of through registers took 437.  Queries (64 registers) and sums (112) leave so little that addresses kept from chunk to
 // chunk were spilled: 261 us with 21 such registers; worked out anew (here()) three remain.
 //
@@ -280,12 +280,12 @@ __device__ __forceinline__ int here(int x) {
 }
 
 template <int KS, int DBW, int NC>  // rows of up to 32 KS elements, values of up to 128 DBW, 16 NC columns
-__global__ void __launch_bounds__(kPromptWaves* kWave)
+__global__ void __launch_bounds__(kPromptWaves* kWave) __attribute__((amdgpu_waves_per_eu(KS == 8 && DBW == 1 ? 4 : 2)))
     latent_prompt_kernel(const bf16* __restrict__ q, bf16* __restrict__ out, int heads, int key_dim, int v_dim,
                          const int32_t* __restrict__ positions, const int32_t* __restrict__ token_seq,
                          const int32_t* __restrict__ tables, int table_stride, const bf16* __restrict__ pool,
                          int page_size, int num_pages, int window, int chunk, float scale,
-                         float* __restrict__ partial, int nsplit, int n, int tpw) {
+                         float* __restrict__ partial, int nsplit, int n, int tpw, int wide) {
   // (rows in LDS are padded as above)
   constexpr int STRIDE = KS * 32 + 32, kRows = 32 * STRIDE + 64;
   auto at = [](int kk) { return kk * STRIDE + (kk >> 3) * 16; };
@@ -298,11 +298,10 @@ __global__ void __launch_bounds__(kPromptWaves* kWave)
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int t0 = (gridDim.x - 1 - blockIdx.x) * tpw, z = blockIdx.y;  // (the last tokens read the most rows: they start first)
   const int t_last = min(t0 + tpw, n) - 1;
-  const int dtiles = (v_dim + 15) / 16;
 
   // this lane's column of tile `wave`
   const int col = wave * 16 + j, t = t0 + col / heads;
-  const bool scores = wave < NC, col_ok = scores && col < tpw * heads && t <= t_last;
+  const bool scores = wave < NC && wave * 16 < tpw * heads, col_ok = scores && col < tpw * heads && t <= t_last;
   const int pos = positions[min(t, t_last)], lo = first_key(pos, window, chunk);
   LFrag qf[KS];
   const bf16* qrow = q + (static_cast<size_t>(t0) * heads + (col_ok ? col : 0)) * key_dim;
@@ -473,7 +472,17 @@ __global__ void __launch_bounds__(kPromptWaves* kWave)
 #pragma unroll
       for (int x = 0; x < DBW; ++x) {
         const int d = (tile + 8 * x) * 16 + 4 * g;
-        if (tile + 8 * x >= dtiles) continue;
+        if (d >= v_dim) continue;
+        if (wide) {  // (v_dim is a multiple of four)
+          if (nsplit == 1) {
+            const uint32_t low = bf16_bits(o[x][cc][0] * inv) | static_cast<uint32_t>(bf16_bits(o[x][cc][1] * inv)) << 16;
+            const uint32_t high = bf16_bits(o[x][cc][2] * inv) | static_cast<uint32_t>(bf16_bits(o[x][cc][3] * inv)) << 16;
+            *reinterpret_cast<uint2*>(out + row * v_dim + d) = make_uint2(low, high);
+          } else {
+            *reinterpret_cast<lf32x4*>(partial + (row * nsplit + z) * v_dim + d) = o[x][cc];
+          }
+          continue;
+        }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           if (d + r >= v_dim) continue;
@@ -531,20 +540,21 @@ static void launch_latent(dim3 grid, hipStream_t s, const bf16* q, bf16* out, in
 
 using namespace shk;
 
-// Tokens a workgroup of latent_prompt_kernel serves, 0 where it does not take the shape: rows of up to 512
+// The most tokens that a workgroup of latent_prompt_kernel serves, 0 where it does not take the shape: rows of up to 512
 // elements, and as many whole tokens as fit into its columns.
 extern "C" int shk_latent_prompt_tokens(int heads, int key_dim, int v_dim) {
   if (!shk_latent_attention_supports_mfma(heads, key_dim, v_dim) || key_dim > 512) return 0;
   return (v_dim > 256 ? 112 : 128) / heads;
 }
 
-// The same for tokens of prompt portions, `positions` rising along each.
+// The same for tokens of prompt portions, `positions` rising along each; tokens: of them a workgroup (0: the most).
 extern "C" int shk_latent_prompt_bf16(const void* q, void* out, int n, int heads, int key_dim, int v_dim,
                                       const int32_t* positions, const int32_t* token_seq, const int32_t* tables,
                                       int table_stride, const void* pool, int page_size, int num_pages, int window, int chunk,
-                                      float scale, float* partial, int nsplit, void* stream) {
-  const int tpw = shk_latent_prompt_tokens(heads, key_dim, v_dim);
-  SHK_REQUIRE(tpw > 0, "latent_prompt_bf16: %d heads over rows of %d with values of %d are not served", heads, key_dim, v_dim);
+                                      float scale, float* partial, int nsplit, int tokens, void* stream) {
+  const int most = shk_latent_prompt_tokens(heads, key_dim, v_dim), tpw = tokens > 0 ? tokens : most;
+  SHK_REQUIRE(most > 0, "latent_prompt_bf16: %d heads over rows of %d with values of %d are not served", heads, key_dim, v_dim);
+  SHK_REQUIRE(tokens >= 0 && tokens <= most, "latent_prompt_bf16: %d tokens a workgroup, at most %d", tokens, most);
   SHK_REQUIRE(n >= 0 && n <= 1 << 30 && nsplit >= 1 && nsplit <= 64, "latent_prompt_bf16: bad sizes n=%d nsplit=%d", n, nsplit);
   SHK_REQUIRE(page_size > 0 && num_pages > 0 && table_stride > 0,
               "latent_prompt_bf16: bad cache sizes page_size=%d num_pages=%d table_stride=%d", page_size, num_pages, table_stride);
@@ -554,11 +564,12 @@ extern "C" int shk_latent_prompt_bf16(const void* q, void* out, int n, int heads
               "latent_prompt_bf16: q and the pool must be 16-byte aligned");
   hipStream_t s = static_cast<hipStream_t>(stream);
   const dim3 grid((n + tpw - 1) / tpw, nsplit);
+  const int wide = v_dim % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 8 == 0 && reinterpret_cast<uintptr_t>(partial) % 16 == 0;
   auto go = [&](auto ks, auto dbw, auto nc) {
     constexpr int KS = decltype(ks)::value, DBW = decltype(dbw)::value, NC = decltype(nc)::value;
     latent_prompt_kernel<KS, DBW, NC><<<grid, kPromptWaves * kWave, 0, s>>>(
         static_cast<const bf16*>(q), static_cast<bf16*>(out), heads, key_dim, v_dim, positions, token_seq, tables, table_stride,
-        static_cast<const bf16*>(pool), page_size, num_pages, window, chunk, scale, partial, nsplit, n, tpw);
+        static_cast<const bf16*>(pool), page_size, num_pages, window, chunk, scale, partial, nsplit, n, tpw, wide);
   };
   using std::integral_constant;
   const int ks = (key_dim + 31) / 32, db = (v_dim + 15) / 16;

@@ -761,20 +761,21 @@ def latent_attention_mfma(q, out, heads, key_dim, v_dim, positions, token_seq, t
 
 
 def latent_prompt_tokens(heads: int, key_dim: int, v_dim: int) -> int:
-    """Tokens a workgroup of latent_prompt() serves; 0: it does not take the shape."""
+    """The most tokens that a workgroup of latent_prompt() serves; 0: it does not take the shape."""
     return int(load().shk_latent_prompt_tokens(heads, key_dim, v_dim))
 
 
 def latent_prompt(q, out, heads, key_dim, v_dim, positions, token_seq, tables, pool, page_size, window, scale, chunk=None,
-                  partial=None, nsplit: int = 1) -> None:
-    """latent_attention_mfma() for the tokens of prompt portions, where latent_prompt_tokens() is not 0."""
+                  partial=None, nsplit: int = 1, tokens: int = 0) -> None:
+    """latent_attention_mfma() for the tokens of prompt portions, where latent_prompt_tokens() is not 0; `tokens` of
+    them a workgroup (0: the most)."""
     n = _check_latent("latent_prompt", q, out, heads, key_dim, v_dim, positions, token_seq, tables, pool, page_size, partial,
                       nsplit)
     check(load().shk_latent_prompt_bf16(
         _dev(q, "q"), _dev(out, "out"), n, heads, key_dim, v_dim, _dev(positions, "positions", torch.int32),
         _dev(token_seq, "token_seq", torch.int32), _dev(tables, "tables", torch.int32), tables.shape[1],
         _dev(pool, "pool"), page_size, pool.shape[0], int(window or 0), int(chunk or 0), float(scale),
-        _dev(partial, "partial", torch.float32) if nsplit > 1 else None, int(nsplit), _stream()))
+        _dev(partial, "partial", torch.float32) if nsplit > 1 else None, int(nsplit), int(tokens), _stream()))
 
 
 def gemm_batched(a, w, out, batch: int, a_step: int, out_step: int) -> None:

@@ -85,29 +85,42 @@ class LatentAttention(Mixer):
             return
         bounds = [int(b) for b in (s.window, s.chunk) if b]
 
-        def shares(workgroups, rows, least):
-            """Workgroups a token's rows are shared among: twice the compute units in all, `least` rows each."""
-            tokens, keys = 1, 64
-            while tokens < workgroups:
-                tokens *= 2
+        def most_shares(rows):
+            """Shares of 128 rows that a token's rows make."""
+            keys = 64
             while keys < min([rows, *bounds]):
                 keys *= 2
-            return max(1, min(2 * compute_units() // tokens, keys // least, 64))
+            return min(max(1, keys // 128), 64)
+
+        def shares(workgroups, rows):
+            """Workgroups a token's rows are shared among: twice the compute units in all."""
+            tokens = 1
+            while tokens < workgroups:
+                tokens *= 2
+            return max(1, min(2 * compute_units() // tokens, most_shares(rows)))
 
         # prompt portions in a kernel of their own where it takes the shape; else every token alike
         # (neighbouring tokens of a step with portions may share a workgroup and what it stages)
-        nsplit, group, first, prompt_split = 1, 1, shape.num_tokens, 1
+        nsplit, group, first, prompt_split, tokens = 1, 1, shape.num_tokens, 1, 0
         if self.mfma:
             if self.prompt_tokens and shape.num_decode < shape.num_seqs:
                 first = shape.num_decode
-                prompt_split = shares(-(-(shape.num_tokens - first) // self.prompt_tokens), int(shape.ctx_lens[first:].max()), 512)
+                # fewer tokens a workgroup where short contexts would leave compute units without one (28 heads over
+                # rows of 512, 64 tokens from 0 on 37 us with four tokens a workgroup, 14 with one; 16 tokens at 2,000
+                # 87 and 38, in 16 shares instead of 4; the kernel for single tokens 27 and 55), and no more than a
+                # portion has on average: tokens of two sequences take their turns (30 portions of 9 tokens at 700, 8
+                # heads over 320, 143 us with 16 a workgroup, 42 with 8)
+                count, longest = shape.num_tokens - first, int(shape.ctx_lens[first:].max())
+                tokens = count * most_shares(longest) // compute_units()
+                tokens = max(1, min(tokens, count // (shape.num_seqs - first), self.prompt_tokens))
+                prompt_split = shares(-(-count // tokens), longest)
                 if first:
-                    nsplit = shares(first, int(shape.ctx_lens[:first].max()), 128)
+                    nsplit = shares(first, int(shape.ctx_lens[:first].max()))
             else:
-                nsplit = shares(shape.num_tokens, int(shape.ctx_lens.max()), 128)
+                nsplit = shares(shape.num_tokens, int(shape.ctx_lens.max()))
                 group = 1 if shape.num_decode == shape.num_seqs else 4
-        shape.notes[key] = (nsplit, group, first, prompt_split)
-        shape.launch_key.append((key, nsplit, group, first, prompt_split))
+        shape.notes[key] = (nsplit, group, first, prompt_split, tokens)
+        shape.launch_key.append((key, nsplit, group, first, prompt_split, tokens))
 
     def load(self, tensors, runtime):
         s = self.spec
@@ -163,7 +176,7 @@ class LatentAttention(Mixer):
                          ctx.positions, magnitude=self.magnitude)
         mixed = ctx.buffer("latent_mixed", (n, H * s.kv_rank), ctx.dtype)
         if self.mfma:
-            nsplit, group, first, prompt_split = ctx.notes[("latent_attention", H, s.kv_rank, s.rot_dim, s.window, s.chunk)]
+            nsplit, group, first, prompt_split, tokens = ctx.notes[("latent_attention", H, s.kv_rank, s.rot_dim, s.window, s.chunk)]
 
             def attend(kernel, lo, hi, shares, **more):
                 partial = None
@@ -176,7 +189,7 @@ class LatentAttention(Mixer):
             if first:
                 attend(ops.latent_attention_mfma, 0, first, nsplit, tokens_per_group=group)
             if first < n:
-                attend(ops.latent_prompt, first, n, prompt_split)
+                attend(ops.latent_prompt, first, n, prompt_split, tokens=tokens)
         else:
             ops.latent_attention(folded, mixed, H, key_dim, s.kv_rank, ctx.positions, ctx.token_seq, tables,
                                  cache.pools["latent"], cache.page_size, s.window, s.scale, chunk=s.chunk)

@@ -92,3 +92,63 @@ def test_a_row_that_is_no_number_stays_with_the_tokens_that_read_it(heads, key_d
         assert bool(reads.any())
         assert torch.equal(got[~reads], want[~reads]), (seq, at)
         assert not bool(torch.isfinite(got[reads].float()).view(-1, heads, v_dim)[:, :, v_dim // 2].any()), (seq, at)
+
+
+@pytest.mark.parametrize("heads, key_dim, v_dim, window", [(28, 512, 448, None), (14, 160, 128, 70), (1, 64, 62, None), (8, 320, 256, None)])
+def test_any_number_of_tokens_a_workgroup(heads, key_dim, v_dim, window):
+    """The same bits with one token a workgroup, a few, and as many as fit; results at any address."""
+    from shrike_amd.kernels import KernelError, ops
+
+    page, most = 16, ops.latent_prompt_tokens(heads, key_dim, v_dim)
+    torch.manual_seed(heads)
+    starts, lengths = [0, 61, 200, 0], [45, 7, 130, 2]
+    n, ctx = sum(lengths), [s + k for s, k in zip(starts, lengths)]
+    per = -(-max(ctx) // page)
+    tables = torch.randperm(4 * per).view(4, per).int().cuda()
+    pool = torch.randn(4 * per, page, key_dim, device="cuda").bfloat16()
+    q = torch.randn(n, heads * key_dim, device="cuda").bfloat16()
+    positions = torch.cat([torch.arange(s, s + k) for s, k in zip(starts, lengths)]).int().cuda()
+    seqs = torch.repeat_interleave(torch.arange(4), torch.tensor(lengths)).int().cuda()
+
+    def run(tokens, offset=0):
+        flat = torch.full((n * heads * v_dim + 8,), 9.0, device="cuda", dtype=torch.bfloat16)
+        out = flat[offset : offset + n * heads * v_dim].view(n, heads * v_dim)
+        ops.latent_prompt(q, out, heads, key_dim, v_dim, positions, seqs, tables, pool, page, window, 0.1, tokens=tokens)
+        assert bool((flat[:offset] == 9.0).all()) and bool((flat[offset + n * heads * v_dim :] == 9.0).all())
+        return out
+
+    want = run(0)
+    assert bool(torch.isfinite(want.float()).all())
+    for tokens in {1, max(1, most // 2), max(1, most - 1), most}:
+        assert torch.equal(run(tokens), want)
+    assert torch.equal(run(0, offset=1), want)
+    with pytest.raises(KernelError):
+        run(most + 1)
+
+
+def test_tokens_and_shares_of_a_step():
+    """Short portions spread over the chip, long prompts fill workgroups, shares stop at twice the compute units."""
+    from types import SimpleNamespace
+
+    import numpy as np
+
+    from shrike_amd.engine.context import StepShape
+    from shrike_amd.parts.attention import compute_units
+    from shrike_amd.parts.latent_attention import LatentAttention
+
+    part = LatentAttention.__new__(LatentAttention)
+    part.spec = SimpleNamespace(num_heads=28, kv_rank=448, rot_dim=64, window=None, chunk=None)
+    part.mfma, part.prompt_tokens = True, 4
+
+    def plan(lens, starts):
+        shape = StepShape(np.array(lens), np.array(starts), 16)
+        part.prepare(shape)
+        (note,) = shape.notes.values()
+        return note
+
+    assert compute_units() == 256
+    assert plan([1501], [0]) == (1, 1, 0, 1, 4)
+    assert plan([64], [0]) == (1, 1, 0, 1, 1)
+    assert plan([16], [2000]) == (1, 1, 0, 16, 1)
+    assert plan([2] * 60, [300] * 60)[4] == 1
+    assert plan([1, 1, 300], [900, 40, 0]) == (8, 1, 2, 4, 4)
