@@ -11,7 +11,8 @@
 //   in order to the result.
 // What differs between shapes is which wavefront walks which segments: all 16 wavefronts of a
 // workgroup one each (few rows: a chain of k is then k / 16 long, and 16 KiB of weights are in
-// flight per workgroup), or four a group each with 64 x 64 results per workgroup (many rows).
+// flight per workgroup), four a group each with 64 x 64 results per workgroup (many rows), or every one all
+// of them (many rows and a k of up to 256).
 // Operands go straight from memory to registers: an instruction takes 32 cycles of its SIMD, a 2 x 2
 // arrangement of tiles needs 4 KiB of operands every 512 cycles and SIMD, which L1 and L2 deliver.
 // The model's weights are held in tiles of 16 rows x 16 k (retile_f32_kernel): a wavefront's load is
@@ -236,7 +237,10 @@ static void launch_f32(const F32Product& p, hipStream_t s) {
 //     k), 896 x 4864 13 (37); 9728 x 896 10.7 with four row blocks (12), 151936 x 896 98 with eight (113);
 //   more: the largest tile that still leaves the 256 compute units evenly loaded.  896 x 896 at 64 / 128 / 509 /
 //     1024 rows 5.7 / 7.3 / 17 / 26 (16 x 16, 32 x 16, 32 x 64, 64 x 64), 9728 x 896 at 64 / 509 25 / 124
-//     (32 x 32, 64 x 64: 70 TFLOP/s of the 150 that the instruction reaches alone).
+//     (32 x 32, 64 x 64: 70 TFLOP/s of the 150 that the instruction reaches alone).  A k of up to 256 is one step
+//     a segment, and a shorter one leaves the later of four groups without any: there a wavefront walks all of k and
+//     four lie side by side along the rows.  1,501 rows: 28 products of 448 x 128 160 us shared by four groups, 77 so
+//     (95 with vector instructions), 14 of 128 x 64 27, 13 (14), 40 of 256 x 192 132, 86 (105), 4864 x 256 73, 55 (66).
 template <bool TILED>
 static void run_f32(const F32Product& p, hipStream_t s) {
   auto tiles = [&](int rows, int cols) {
@@ -251,7 +255,10 @@ static void run_f32(const F32Product& p, hipStream_t s) {
     else
       launch_f32<2, 1, 4, 4, 1, 2, TILED>(p, s);
   } else if (tiles(64, 64) >= 640 || one_round(tiles(64, 64))) {
-    launch_f32<4, 4, 4, 1, 1, 1, TILED>(p, s);
+    if (p.k <= 256)
+      launch_f32<4, 2, 1, 1, 4, 1, TILED>(p, s);
+    else
+      launch_f32<4, 4, 4, 1, 1, 1, TILED>(p, s);
   } else if (one_round(tiles(32, 64))) {
     launch_f32<2, 4, 4, 1, 1, 2, TILED>(p, s);
   } else if (tiles(16, 16) <= 256) {

@@ -48,6 +48,24 @@ def test_against_float64_and_the_same_bits_for_any_number_of_rows(ops, m, k, ali
         assert torch.equal(again, plain + tiled)
 
 
+@pytest.mark.parametrize("batch, m, k", [(28, 448, 128), (14, 128, 64), (40, 250, 192), (16, 96, 77), (3, 900, 256), (5, 512, 260), (9, 700, 16)])
+def test_many_rows_of_a_short_k_in_batches(ops, batch, m, k):
+    torch.manual_seed(batch + k)
+    n_max = 700
+    a, w = torch.randn(n_max, batch * k, device="cuda"), torch.randn(batch, m, k, device="cuda")
+    per = a.view(n_max, batch, k).transpose(0, 1).double()
+    exact = torch.stack([per[b] @ w[b].double().t() for b in range(batch)], 1).view(n_max, batch * m)
+    size = torch.stack([per[b].abs() @ w[b].double().abs().t() for b in range(batch)], 1).view(n_max, batch * m)
+    full = None
+    for n in (n_max, 1, 17, 100, 300, 511):
+        out = torch.full((n, batch * m + 4), 7.0, device="cuda")
+        ops.gemm_batched(a[:n], w, out[:, : batch * m], batch, k, m)
+        assert bool((out[:, batch * m :] == 7.0).all())
+        full = out if full is None else full
+        assert torch.equal(out, full[:n]), "the same bits in every shape"
+    assert bool(((full[:, : batch * m].double() - exact).abs() <= (k / 16 + 40) * 2.0**-24 * size).all())
+
+
 def test_what_does_not_fit_is_refused(ops):
     from shrike_amd.kernels import KernelError
 
