@@ -99,6 +99,10 @@ __global__ void __launch_bounds__(kWave * kBlockWaves) attention_f32_kernel(F32A
   for (int b = first; b <= last; b += step) {
     const int key0 = b * kKeyBlock + wave * kWaveKeys;
     const bool any = key0 <= pos && key0 + kWaveKeys > lo;  // of this wavefront's keys is read
+    // whether a step holds a key that is read: heads of more than 128 alone, whose steps are long and loaded one at a time
+    // (six heads of 256, a prompt of 17 tokens 27 us, 20 so; with a branch for heads of 128 a second workgroup no
+    // longer fits on a compute unit)
+    auto read = [&](int u) { return kAhead > 1 || (key0 + 16 * u <= pos && key0 + 16 * (u + kAhead) > lo); };
     // scores: this lane loads key key0 + 16 u + i, and gets keys key0 + 16 u + 4 kg + 0..3 of head i
     af4 s[kSteps];
     int k_at[kSteps], v_at[kSteps];  // pages of the keys, and of the values, that this lane loads
@@ -137,11 +141,14 @@ __global__ void __launch_bounds__(kWave * kBlockWaves) attention_f32_kernel(F32A
       }
 #pragma unroll
       for (int u0 = 0; u0 < kSteps; u0 += kAhead) {
+        const bool reads = read(u0);
+        if (reads)
 #pragma unroll
-        for (int u = u0; u < u0 + kAhead; ++u) load_keys(u);
+          for (int u = u0; u < u0 + kAhead; ++u) load_keys(u);
         if (u0 + kAhead == kSteps)
 #pragma unroll
           for (int u = 0; u < kAhead; ++u) load_values(u);
+        if (reads)
 #pragma unroll
         for (int x = 0; x < D; ++x)
 #pragma unroll
@@ -183,6 +190,7 @@ __global__ void __launch_bounds__(kWave * kBlockWaves) attention_f32_kernel(F32A
     if (any) {
 #pragma unroll
       for (int u = 0; u < kSteps; ++u) {
+        if (!read(u / kAhead * kAhead)) continue;
         if (u >= kAhead && u % kAhead == 0)
 #pragma unroll
           for (int ahead = u; ahead < u + kAhead; ++ahead) load_values(ahead);
