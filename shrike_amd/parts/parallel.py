@@ -62,6 +62,10 @@ class ParallelMixers(Mixer):
                         for sub, _ in self.branches]
         self.eps = float(self.spec.eps)
 
+    def context_scratch_bytes(self, rows: int, keys: int) -> int:
+        # (one step's buffers serve the branches in turn, as they serve the layers)
+        return max((m.context_scratch_bytes(rows, keys) for _, m in self.branches), default=0)
+
     def forward(self, ctx, x: torch.Tensor, cache):
         n = x.shape[0]
         total = ctx.buffer("parallel_sum", (1, n, self.width), torch.float32)

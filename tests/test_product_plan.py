@@ -252,3 +252,19 @@ def test_the_reserve_counts_scratch_that_grows_with_the_context():
     assert context_reserve(model, cfg, 32768) == 2 * 255 * row + 128 * row  # buckets 1 to 128, the largest once more
     assert context_reserve(model, EngineConfig(max_running=1), 32768) == 3 * row
     assert context_reserve(model, cfg, 100) == 0
+
+
+def test_the_reserve_counts_mixers_side_by_side():
+    import torch
+
+    from shrike_amd.config import AttentionSpec
+    from shrike_amd.config.specs import ParallelMixerSpec
+    from shrike_amd.parts.base import build_part
+
+    small = AttentionSpec(num_heads=2, num_kv_heads=1, head_dim=32, qkv_bias=False, out_bias=False, scale=0.1)
+    large = AttentionSpec(num_heads=14, num_kv_heads=2, head_dim=64, qkv_bias=False, out_bias=False, scale=0.1)
+    both = build_part("mixer", ParallelMixerSpec(branches=(("left", small), ("right", large)), eps=1e-6, scale=1.0), 896, "m")
+    for _, mixer in both.branches:
+        mixer.dtype = torch.float32
+    assert both.context_scratch_bytes(3, 32768) == 3 * 14 * 128 * 66 * 4
+    assert both.context_scratch_bytes(3, 200) == 0
