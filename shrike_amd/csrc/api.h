@@ -216,7 +216,7 @@ int shk_attention_supports_mfma(int heads, int kv_heads, int head_dim, int page_
 // `partial` is float32 scratch of num_seqs * heads * nsplit * (head_dim + 2).
 // streaming != 0: keys and values are fetched with non-temporal loads (faster when a
 // launch reads tens of megabytes of them, slightly slower below; the result is the same).
-// waves: wavefronts a workgroup, 4, or 8 for heads of up to 64 elements.
+// waves: wavefronts a workgroup, 4, or 8 (plain loads always) for heads of up to 64 elements.
 // softcap / sinks / dist_bias as in shk_attention (0 and null: none).
 int shk_attention_decode_bf16(const void* q, int q_stride, void* out, int num_seqs, int heads,
                               int kv_heads, int head_dim, const int32_t* positions,

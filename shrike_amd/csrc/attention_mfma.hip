@@ -1004,10 +1004,9 @@ static void launch_decode(dim3 grid, hipStream_t s, const bf16* q, int q_stride,
   const uint32_t magic = static_cast<uint32_t>(((1ull << 32) + page_size - 1) / page_size);
   auto kernel = streaming ? attention_decode_kernel<D, true, 4> : attention_decode_kernel<D, false, 4>;
   if constexpr (D <= 64)
-    if (waves == 8) kernel = streaming ? attention_decode_kernel<D, true, 8> : attention_decode_kernel<D, false, 8>;
-  kernel<<<grid, waves * kWave, 0, s>>>(q, q_stride, out, heads, kv_heads, positions, tables, table_stride,
-                                                         k_pool, v_pool, page_size, magic, window, block, scale, partial,
-                                                         nsplit, so);
+    if (waves == 8) kernel = attention_decode_kernel<D, false, 8>;  // (contexts too short to stream)
+  kernel<<<grid, waves * kWave, 0, s>>>(q, q_stride, out, heads, kv_heads, positions, tables, table_stride, k_pool, v_pool,
+                                        page_size, magic, window, block, scale, partial, nsplit, so);
   if (nsplit > 1)
     attention_merge_kernel<D><<<grid.y * heads, kWave, 0, s>>>(partial, out, nsplit, so.sinks, heads);
 }
