@@ -135,3 +135,53 @@ def test_a_reader_of_shares_gets_small_products_unrounded(m, k, n):
     product = runtime.linear_deferred(Context, "q", a, runtime.weight(w), bias=bias, reader="position")
     got = product.parts.double().sum(0) + (0 if product.bias is None else product.bias.double())
     assert bool(((got - exact - bias.double()).abs() <= bound * (size + bias.double().abs())).all())
+
+
+@pytest.mark.parametrize("m, k", [(300, 64), (1152, 896), (896, 4864), (2000, 264), (37, 72)])
+@pytest.mark.parametrize("n", [17, 64, 100, 200, 300, 700, 1200])
+def test_small_matrices_add_to_their_output_and_activate(m, k, n):
+    """Sums onto what is there, the square of ReLU and SiLU of the first columns, with a bias, in the kernels that stage nothing."""
+    from shrike_amd.kernels import ops
+
+    torch.manual_seed(m + k + n)
+    a, w = torch.randn(n, k, device="cuda").bfloat16(), (torch.randn(m, k, device="cuda") / k**0.5).bfloat16()
+    bias, wt = torch.randn(m, device="cuda"), ops.retile_weight(w)
+    v = a.double() @ w.double().t() + bias.double()
+    off = (k / 32 + 48) * 2.0**-24 * (a.double().abs() @ w.double().abs().t() + bias.double().abs())  # of a float32 sum
+    there = torch.randn(n, m + 8, device="cuda")
+    for dtype, ulp in ((torch.float32, 2.0**-23), (torch.bfloat16, 2.0**-8)):
+        out = there.to(dtype, copy=True)
+        if dtype == torch.float32:
+            ops.gemm_tiled_weight(a, wt, m, k, out[:, :m], bias=bias, accumulate=True)
+            want = there[:, :m].double() + v
+            assert bool(((out[:, :m].double() - want).abs() <= off + ulp * (want.abs() + off)).all())
+        ops.gemm_tiled_weight(a, wt, m, k, out[:, :m], bias=bias, activation="relu_squared")
+        want = v.clamp(min=0) ** 2
+        assert bool(((out[:, :m].double() - want).abs() <= 2.2 * off * (v.abs() + off) + ulp * want).all())
+        for rows in (1, 37, m - 3, m):
+            ops.gemm_tiled_weight(a, wt, m, k, out[:, :m], bias=bias, activation=("silu", min(rows, m)))
+            want = v.clone()
+            want[:, :rows] = v[:, :rows] * torch.sigmoid(v[:, :rows])
+            # (the slope of SiLU is at most 1.1; its float32 exponential and quotient: a few roundings of the result, or of
+            # an exponent of up to 40, 2^-18)
+            assert bool(((out[:, :m].double() - want).abs() <= 1.1 * off + (ulp + 2.0**-18) * want.abs() + 1e-12).all()), rows
+        assert torch.equal(out[:, m:], there[:, m:].to(dtype))
+
+
+@pytest.mark.parametrize("m, k", [(896, 896), (1152, 896), (896, 4864), (1000, 2056), (512, 3584), (2048, 1024), (10, 3584), (64, 520), (32, 8192)])
+def test_small_products_keep_their_bits_within_a_batch_bucket(m, k):
+    """A captured step of 32, 64, 128 or 256 rows stands for every smaller batch down to the next."""
+    from shrike_amd.kernels import ops
+
+    torch.manual_seed(m + k)
+    a, w = torch.randn(256, k, device="cuda").bfloat16(), torch.randn(m, k, device="cuda").bfloat16()
+    wt = ops.retile_weight(w)
+    for end, fewer in ((32, (17, 21)), (64, (33, 41)), (128, (65, 97)), (256, (129, 201))):
+        splits = ops.gemm_splits(end, m, k)
+        whole = torch.full((splits, end, m), float("nan"), device="cuda")
+        ops.gemm_tiled_weight(a[:end], wt, m, k, whole if splits > 1 else whole[0], splits=splits)
+        assert not bool(torch.isnan(whole).any())
+        for n in fewer:
+            part = torch.full((splits, n, m), float("nan"), device="cuda")
+            ops.gemm_tiled_weight(a[:n], wt, m, k, part if splits > 1 else part[0], splits=splits)
+            assert torch.equal(part, whole[:, :n]), (n, end)
