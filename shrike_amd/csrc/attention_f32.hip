@@ -90,7 +90,8 @@ __global__ void __launch_bounds__(kWave * kBlockWaves) attention_f32_kernel(F32A
   float M = -INFINITY, L = 0.f;
   const int slab = key_slab(p.head_dim), ps = p.page_size;
   const size_t k_page = static_cast<size_t>(ps) * p.head_dim, v_page = static_cast<size_t>(ps) * p.v_dim;
-  constexpr int kSteps = kWaveKeys / 16, kAhead = D <= 4 ? kSteps : D == 8 ? 2 : 1;  // steps of 16 keys, and how many are loaded at once
+  // steps of 16 keys, how many are loaded at once, and how many are multiplied side by side
+  constexpr int kSteps = kWaveKeys / 16, kAhead = D <= 4 ? kSteps : D <= 8 ? 2 : 1, kGroup = D <= 3 ? 2 : kAhead;
   auto page_of = [&](int key) {  // of `key`, or of the nearest key that is read; -1 where there is none
     const int page = table[min(max(key, lo), pos) / ps];
     return page < p.num_pages ? page : -1;
@@ -99,10 +100,11 @@ __global__ void __launch_bounds__(kWave * kBlockWaves) attention_f32_kernel(F32A
   for (int b = first; b <= last; b += step) {
     const int key0 = b * kKeyBlock + wave * kWaveKeys;
     const bool any = key0 <= pos && key0 + kWaveKeys > lo;  // of this wavefront's keys is read
-    // whether a step holds a key that is read: heads of more than 128 alone, whose steps are long and loaded one at a time
-    // (six heads of 256, a prompt of 17 tokens 27 us, 20 so; with a branch for heads of 128 a second workgroup no
-    // longer fits on a compute unit)
-    auto read = [&](int u) { return kAhead > 1 || (key0 + 16 * u <= pos && key0 + 16 * (u + kAhead) > lo); };
+    // whether a group of steps holds a key that is read, for heads of up to 48 and of more than 128 (a prompt of 17 tokens,
+    // heads of 32 7.2 us with all products, 6.4 so, of 256 27 and 20).  Those between lose more by the branch
+    // than they gain (64: 500 tokens 37.6 us, 38.5 with it; 128: a second workgroup no longer fits on a compute
+    // unit) and take up to 0.6 (64) and 1.9 us (16 heads of 128) longer than the general kernel for 17 tokens
+    auto read = [&](int u) { return (D > 3 && D <= 8) || (key0 + 16 * u <= pos && key0 + 16 * (u + kGroup) > lo); };
     // scores: this lane loads key key0 + 16 u + i, and gets keys key0 + 16 u + 4 kg + 0..3 of head i
     af4 s[kSteps];
     int k_at[kSteps], v_at[kSteps];  // pages of the keys, and of the values, that this lane loads
@@ -141,23 +143,26 @@ __global__ void __launch_bounds__(kWave * kBlockWaves) attention_f32_kernel(F32A
       }
 #pragma unroll
       for (int u0 = 0; u0 < kSteps; u0 += kAhead) {
-        const bool reads = read(u0);
-        if (reads)
+        const bool loads = D <= 4 || read(u0);
+        if (loads)
 #pragma unroll
           for (int u = u0; u < u0 + kAhead; ++u) load_keys(u);
         if (u0 + kAhead == kSteps)
 #pragma unroll
           for (int u = 0; u < kAhead; ++u) load_values(u);
-        if (reads)
 #pragma unroll
-        for (int x = 0; x < D; ++x)
+        for (int g = u0; g < u0 + kAhead; g += kGroup) {
+          if (!read(g)) continue;
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
+          for (int x = 0; x < D; ++x)
 #pragma unroll
-            for (int u = u0; u < u0 + kAhead; ++u) {
-              const float key = 16 * x + 4 * kg < p.head_dim ? kv[u % kAhead][x][e] : 0.f;
-              s[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(key, qv[x][e], s[u], 0, 0, 0);
-            }
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+              for (int u = g; u < g + kGroup; ++u) {
+                const float key = 16 * x + 4 * kg < p.head_dim ? kv[u % kAhead][x][e] : 0.f;
+                s[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(key, qv[x][e], s[u], 0, 0, 0);
+              }
+        }
       }
     }
     float top = -INFINITY;
@@ -190,7 +195,7 @@ __global__ void __launch_bounds__(kWave * kBlockWaves) attention_f32_kernel(F32A
     if (any) {
 #pragma unroll
       for (int u = 0; u < kSteps; ++u) {
-        if (!read(u / kAhead * kAhead)) continue;
+        if (!read(u / kGroup * kGroup)) continue;
         if (u >= kAhead && u % kAhead == 0)
 #pragma unroll
           for (int ahead = u; ahead < u + kAhead; ++ahead) load_values(ahead);
@@ -286,10 +291,15 @@ static void launch(const F32Attention& p, int n, int splits, hipStream_t s) {
 
 void attention_f32(const F32Attention& p, int n, int splits, hipStream_t s) {
   const int d = p.head_dim > p.v_dim ? p.head_dim : p.v_dim;
+  // (heads of 40 in the kernel for 64, of 96 in that for 128: 500 tokens 34.7 us and 35.0 instead of 29.8 and 28.9)
   if (d <= 32)
     launch<2>(p, n, splits, s);
+  else if (d <= 48)
+    launch<3>(p, n, splits, s);
   else if (d <= 64)
     launch<4>(p, n, splits, s);
+  else if (d <= 96)
+    launch<6>(p, n, splits, s);
   else if (d <= 128)
     launch<8>(p, n, splits, s);
   else

@@ -132,6 +132,7 @@ class AttentionPlan:
     mfma: bool = False
     nsplit: int = 1  # key splits of the single-token rows
     waves: int = 4  # wavefronts of their workgroups
+    blocks_apart: bool = False  # float32: workgroups of their own for a single token's blocks of keys
     streaming: bool = False  # single-token rows: non-temporal loads of keys and values
     kernel: str = ""  # for prompt portions: "shared", "tiles" or "" (none in the step)
     small: bool = False  # "shared" with half as many wavefronts per workgroup
@@ -427,7 +428,11 @@ class PagedAttention(Mixer):
         # the most keys that any query reads, where the mask bounds them
         reach = min(x for x in (s.window, s.chunk, 1 << 40) if x)
         if not plan.mfma:
-            return  # the general kernel takes every token alike
+            # the general kernels take every token alike, but float32 single tokens of more than one block of keys
+            # (a longer step's launches serve them side by side and join them: two kernels instead of one)
+            plan.blocks_apart = self.dtype == torch.float32 and shape.max_decode_ctx > ops.ATTENTION_KEY_BLOCK
+            shape.launch_key.append((key, plan.blocks_apart))
+            return
         if shape.num_decode:
             plan.nsplit, plan.waves = decode_shares(shape.num_decode, hkv, d, min(shape.max_decode_ctx, reach))
             plan.streaming = decode_streams(shape.num_decode, hkv, d, shape.max_decode_ctx,
@@ -500,7 +505,7 @@ class PagedAttention(Mixer):
             return
         if not plan.mfma:
             partial, splits = None, 1
-            if self.dtype == torch.float32 and ctx.num_decode == ctx.num_tokens:
+            if plan.blocks_apart and ctx.num_decode == ctx.num_tokens:
                 # few single tokens: their blocks of keys side by side (as many as the tables are wide: what a
                 # replayed launch must serve; the result is the same bits)
                 keys = tables.shape[1] * cache.page_size

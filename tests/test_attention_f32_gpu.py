@@ -110,3 +110,30 @@ def test_scores_of_minus_infinity(splits, sinks):
                 continue
             want = torch.exp(s - torch.logsumexp(top, 0)) @ values[: pos + 1].double()
             assert torch.allclose(got[t, h], want, atol=2e-5, rtol=0), (t, h)
+
+
+@pytest.mark.parametrize("heads, kv_heads, dim, page, window", [(4, 1, 32, 16, None), (4, 2, 40, 4, None), (14, 2, 64, 16, 20), (5, 5, 48, 8, 33),
+                                                              (3, 1, 80, 16, None), (6, 2, 132, 16, 17)])
+def test_steps_without_a_key_that_is_read(heads, kv_heads, dim, page, window):
+    """Prompts of up to 100 tokens: every number of steps of 16 keys, and of pairs of them, that hold one."""
+    from shrike_amd.kernels import ops
+
+    torch.manual_seed(dim)
+    n, slab = 100, ops.key_slab(dim)
+    pages = -(-n // page)
+    k_pool = torch.full((pages + 1, kv_heads, dim // slab, page, slab), float("nan"), device="cuda")
+    v_pool = torch.full((pages + 1, kv_heads, dim, page), float("nan"), device="cuda")
+    tables = torch.randperm(pages + 1, device="cuda")[:pages].int().view(1, -1)
+    keys, values = torch.randn(n, kv_heads, dim, device="cuda"), torch.randn(n, kv_heads, dim, device="cuda")
+    at = torch.arange(n, device="cuda")
+    k_pool[tables[0].long()[at // page], :, :, at % page] = keys.view(n, kv_heads, dim // slab, slab)
+    v_pool[tables[0].long()[at // page], :, :, at % page] = values
+    q, out = torch.randn(n, heads * dim, device="cuda"), torch.empty(n, heads * dim, device="cuda")
+    ops.attention(q, out, heads, kv_heads, dim, at.int(), torch.zeros(n, dtype=torch.int32, device="cuda"), tables, k_pool, v_pool, page,
+                  window, dim**-0.5)
+    s = torch.einsum("thd,khd->htk", q.view(n, heads, dim).double(), keys.repeat_interleave(heads // kv_heads, 1).double()) * dim**-0.5
+    far = at.view(-1, 1) - at
+    s = s.masked_fill((far < 0) | (far >= (window or n)), -float("inf"))
+    want = torch.einsum("htk,khd->thd", torch.softmax(s, -1), values.repeat_interleave(heads // kv_heads, 1).double())
+    # (scores of a few units off by some ulp, weights by as much; half an ulp of values of order one a term)
+    assert torch.allclose(out.view(n, heads, dim).double(), want, atol=1e-5, rtol=0)

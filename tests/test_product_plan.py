@@ -268,3 +268,32 @@ def test_the_reserve_counts_mixers_side_by_side():
         mixer.dtype = torch.float32
     assert both.context_scratch_bytes(3, 32768) == 3 * 14 * 128 * 66 * 4
     assert both.context_scratch_bytes(3, 200) == 0
+
+
+def test_float32_single_tokens_of_one_block_of_keys_are_one_launch():
+    """A graph of 64 pages' tables stands for contexts of up to 1,024 tokens: those of one block have one of their own."""
+    import torch
+
+    from shrike_amd.cache import CacheManager
+    from shrike_amd.config import AttentionSpec, BlockSpec, ModelSpec, RMSNormSpec, SwiGLUSpec
+    from shrike_amd.engine.runner import ModelRunner, StepEntry
+    from shrike_amd.engine.runtime import Runtime
+    from shrike_amd.models import DecoderModel
+
+    norm = RMSNormSpec(eps=1e-6)
+    mixer = AttentionSpec(num_heads=14, num_kv_heads=2, head_dim=64, qkv_bias=True, out_bias=False, scale=0.1)
+    block = BlockSpec(name="model.layers.0", mixer=mixer, ffn=SwiGLUSpec(intermediate_size=64), mixer_norm=norm, ffn_norm=norm)
+    model = DecoderModel(ModelSpec(architecture="t", hidden_size=896, vocab_size=100, blocks=(block,), final_norm=norm,
+                                   tie_word_embeddings=False))
+    model.blocks[0].mixer.dtype = torch.float32
+    cache = CacheManager(model.cache_specs(), 16, 1 << 10)
+    runner = ModelRunner(model, cache, Runtime("cuda:0", torch.float32))
+    keys = {}
+    for ctx in (1, 200, 256, 257, 300, 1024, 1025):
+        seqs = [cache.new_sequence() for _ in range(2)]
+        cache.append(seqs[0], 0, ctx)
+        cache.append(seqs[1], 0, 1)
+        keys[ctx] = runner._graph_key([StepEntry(seqs[0], [0], ctx - 1, [0]), StepEntry(seqs[1], [0], 0, [0])])
+        for s in seqs:
+            cache.free(s)
+    assert keys[1] == keys[200] == keys[256] != keys[257] == keys[300] == keys[1024] != keys[1025]
