@@ -260,19 +260,28 @@ __global__ void __launch_bounds__(kWave* RW* CW)
 }
 
 // Shapes: up to 16 rows 16 x 16 a wavefront, side by side along the features (the weights' latency is all
-// there is); 64 x 64 a wavefront where such workgroups fill the compute units, else 32 x 32.
+// there is); 64 x 64 a wavefront where such workgroups fill the compute units, else 32 x 32.  A k of one or two steps
+// is loaded a step at a time: eight steps' loads, most of them the last step's again, took 4.1 us for 8 products
+// of 256 x 64 at 16 rows, two 2.4 (3.1 with 64-row workgroups).
 template <typename TO>
 static void launch_batched_mfma(const bf16* a, const bf16* w, TO* out, int n, int m, int k, int lda, int ldo, int batch,
                                 long long a_batch, long long w_batch, long long out_batch, hipStream_t s) {
   const int vec_out = ldo % 4 == 0 && out_batch % 4 == 0 && reinterpret_cast<uintptr_t>(out) % (4 * sizeof(TO)) == 0;
   auto grid = [&](int rows, int cols) { return dim3((m + cols - 1) / cols, (n + rows - 1) / rows, batch); };
   const dim3 large = grid(128, 128);
-  if (n <= 16)
+  const bool short_k = k <= 64;
+  if (n <= 16 && short_k)
+    gemm_batched_mfma_kernel<1, 1, 1, 4, 1, TO>
+        <<<grid(16, 64), 256, 0, s>>>(a, w, out, n, m, k, lda, ldo, vec_out, a_batch, w_batch, out_batch);
+  else if (n <= 16)
     gemm_batched_mfma_kernel<1, 1, 1, 4, 4, TO>
         <<<grid(16, 64), 256, 0, s>>>(a, w, out, n, m, k, lda, ldo, vec_out, a_batch, w_batch, out_batch);
   else if (static_cast<long long>(large.x) * large.y * batch >= 256)
     gemm_batched_mfma_kernel<4, 4, 2, 2, 1, TO>
         <<<large, 256, 0, s>>>(a, w, out, n, m, k, lda, ldo, vec_out, a_batch, w_batch, out_batch);
+  else if (short_k)
+    gemm_batched_mfma_kernel<2, 2, 2, 2, 1, TO>
+        <<<grid(64, 64), 256, 0, s>>>(a, w, out, n, m, k, lda, ldo, vec_out, a_batch, w_batch, out_batch);
   else
     gemm_batched_mfma_kernel<2, 2, 2, 2, 2, TO>
         <<<grid(64, 64), 256, 0, s>>>(a, w, out, n, m, k, lda, ldo, vec_out, a_batch, w_batch, out_batch);
