@@ -764,9 +764,29 @@ static void launch_big(const bf16* a, const int32_t* order, const int32_t* count
       form);
 }
 
+// Whether lists of 64 pairs and more keep moe_big_mfma_kernel's few, long workgroups busy for longer than they take to start and end,
+// or the kernels for short lists, at about 200 TFLOP/s, are done before.  Both products and the join at 64 / 128 / 300 pairs a list, short lists'
+// kernels against this one: 8 experts of 64 x 64 12 / 13 / 15 us against 22 / 24 / 26 (21 to 23 in the kernel for row-major
+// weights), of 512 x 512 22 / 24 / 35 against 36 / 39 / 42, of 1024 x 1024 35 / 44 / 73 against 48 / 53 / 57, of 3584 x 1024
+// 69 / 104 / 201 against 79 / 88 / 113; 32 of 512 x 512 35 / 51 / 92 against 40 / 46 / 69.  Up to 256 tokens the next power of two counts,
+// so that a captured step decides as those it stands for.
+static bool fills_long_lists(int n, int top, int width, int ff, bool single) {
+  long long tokens = n;
+  for (int end = 32; end <= 256 && n <= 256; end *= 2)
+    if (n <= end) {
+      tokens = end;
+      break;
+    }
+  const double flops = (single ? 4.0 : 6.0) * static_cast<double>(tokens * top) * width * ff;
+  return flops / 2e8 >= 7.0 + 0.0125 * (width + ff);  // microseconds
+}
+
 // out[t, c] = add[t, c] + sum_k weights[t, k] * pair_out[t * top + k, c], k in the order chosen; an identity
 // expert's output is x[t, c].  Eight columns a thread (width is a multiple of 8): 16-byte loads and stores, 25 us
-// at 1,501 tokens of 3584 with one column a thread, 13 so.  wide: add and out are 16-byte aligned, else element by element.
+// at 1,501 tokens of 3584 with one column a thread, 13 so.  Without identity experts there is no branch between the pairs'
+// loads (8 of 32 experts of 64 features, width 128: all four launches 14.5 us at 8 tokens, 12.1 so).  wide: add and out are
+// 16-byte aligned, else element by element.
+template <bool IDENTITY>
 __global__ void __launch_bounds__(256)
     moe_join_kernel(const float* __restrict__ pair_out, const int32_t* __restrict__ chosen, const bf16* __restrict__ x,
                     const float* __restrict__ weights, const bf16* __restrict__ add, const float* __restrict__ add_gate,
@@ -780,16 +800,19 @@ __global__ void __launch_bounds__(256)
   if (c >= width) return;
   const size_t at = static_cast<size_t>(t) * width + c;
   float total[8] = {};
+  auto join = [&](float weight, float4 y0, float4 y1) {
+    total[0] = fmaf(weight, y0.x, total[0]), total[1] = fmaf(weight, y0.y, total[1]);
+    total[2] = fmaf(weight, y0.z, total[2]), total[3] = fmaf(weight, y0.w, total[3]);
+    total[4] = fmaf(weight, y1.x, total[4]), total[5] = fmaf(weight, y1.y, total[5]);
+    total[6] = fmaf(weight, y1.z, total[6]), total[7] = fmaf(weight, y1.w, total[7]);
+  };
+#pragma unroll 4
   for (int k = 0; k < top; ++k) {
     const size_t pair = static_cast<size_t>(t) * top + k;
     const float weight = weights[pair];
-    if (chosen[pair] < experts) {
-      const float4 *y = reinterpret_cast<const float4*>(pair_out + pair * width + c);
-      const float4 y0 = y[0], y1 = y[1];
-      total[0] = fmaf(weight, y0.x, total[0]), total[1] = fmaf(weight, y0.y, total[1]);
-      total[2] = fmaf(weight, y0.z, total[2]), total[3] = fmaf(weight, y0.w, total[3]);
-      total[4] = fmaf(weight, y1.x, total[4]), total[5] = fmaf(weight, y1.y, total[5]);
-      total[6] = fmaf(weight, y1.z, total[6]), total[7] = fmaf(weight, y1.w, total[7]);
+    if (!IDENTITY || chosen[pair] < experts) {
+      const float4* y = reinterpret_cast<const float4*>(pair_out + pair * width + c);
+      join(weight, y[0], y[1]);
     } else {
       Eight v;
       v.u = *reinterpret_cast<const uint4*>(x + at);
@@ -909,13 +932,13 @@ extern "C" int shk_moe_experts_grouped(const void* x, const int32_t* chosen, con
   moe_lists_kernel<<<experts, 256, 0, s>>>(chosen, n, top, order, counts);
   const bf16 *xb = static_cast<const bf16*>(x), *actb = static_cast<const bf16*>(act_buf);
   const bool many = static_cast<long long>(n) * top >= 64LL * experts;  // lists of 64 pairs and more on average
-  if (many && tiled) {
+  if (many && tiled && fills_long_lists(n, top, width, ff, w_gate == w_up)) {
     if (w_gate == w_up)
       launch_big<kMoeSingle>(xb, order, counts, w_gate, w_up, static_cast<bf16*>(act_buf), nullptr, n, width, ff, experts, top, form, s);
     else
       launch_big<kMoeGated>(xb, order, counts, w_gate, w_up, static_cast<bf16*>(act_buf), nullptr, n, width, ff, experts, top, form, s);
     launch_big<kMoeDown>(actb, order, counts, w_down, nullptr, nullptr, pair_out, n, ff, width, experts, top, form, s);
-  } else if (many) {
+  } else if (many && !tiled) {
     const int row_tiles = (n + kTileRows - 1) / kTileRows;
     if (w_gate == w_up)
       moe_tiled_mfma_kernel<true, true><<<dim3((ff + 127) / 128, row_tiles, experts), 256, 0, s>>>(
@@ -941,9 +964,9 @@ extern "C" int shk_moe_experts_grouped(const void* x, const int32_t* chosen, con
   }
   const int join_threads = width >= 2048 ? 256 : kWave;
   const int wide = reinterpret_cast<uintptr_t>(add) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
-  moe_join_kernel<<<dim3((width / 8 + join_threads - 1) / join_threads, n), join_threads, 0, s>>>(
-      pair_out, chosen, static_cast<const bf16*>(x), weights, static_cast<const bf16*>(add), add_gate, gate_ld,
-      static_cast<bf16*>(out), width, top, experts, wide);
+  auto join = identity ? moe_join_kernel<true> : moe_join_kernel<false>;
+  join<<<dim3((width / 8 + join_threads - 1) / join_threads, n), join_threads, 0, s>>>(
+      pair_out, chosen, xb, weights, static_cast<const bf16*>(add), add_gate, gate_ld, static_cast<bf16*>(out), width, top, experts, wide);
   SHK_LAUNCH_CHECK("moe_experts_grouped");
   return 0;
 }

@@ -12,6 +12,10 @@ pytestmark = pytest.mark.gpu
     (192, 320, [700, 0, 0]),
     (1344, 448, [131, 255, 257, 5, 0, 96, 512, 1]),
     (128, 192, [0] * 70 + [900, 127] + [64] * 75),  # more experts than a wavefront has lanes
+    # (small matrices take the kernels for short lists up to here, see fills_long_lists)
+    (64, 64, [0, 1, 128, 129, 385, 64, 36000]),
+    (192, 320, [4000, 0, 0]),
+    (128, 192, [0] * 70 + [900, 127] + [64] * 75 + [5000]),
 ])
 @pytest.mark.parametrize("form", ["silu", "bounded", "single"])
 def test_lists_of_every_length(width, ff, counts, form):
@@ -66,8 +70,9 @@ def test_lists_of_every_length(width, ff, counts, form):
                         up_shift=shift, tiled=tiled)
         both.append(small)
     assert torch.equal(*both)
-    # the activations are rounded to bfloat16 (2^-9 of each), the result once more; float32 sums add little
-    assert bool(((out.double() - want).abs() <= 2.0**-8 * size + 1e-3).all())
+    # the activations are rounded to bfloat16, the result once more: eight significant bits, so 2^-8 of each at most, together
+    # 2^-7 where one activation makes the result (a few in a million elements come above 2^-8); float32 sums add little
+    assert bool(((out.double() - want).abs() <= 2.0**-7 * size + 1e-3).all())
 
 
 @pytest.mark.parametrize("off_add, off_out", [(1, 0), (0, 1), (3, 5)])
