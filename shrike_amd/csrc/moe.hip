@@ -770,7 +770,8 @@ static void launch_big(const bf16* a, const int32_t* order, const int32_t* count
 // weights), of 512 x 512 22 / 24 / 35 against 36 / 39 / 42, of 1024 x 1024 35 / 44 / 73 against 48 / 53 / 57, of 3584 x 1024
 // 69 / 104 / 201 against 79 / 88 / 113; 32 of 512 x 512 35 / 51 / 92 against 40 / 46 / 69.  Up to 256 tokens the next power of two counts,
 // so that a captured step decides as those it stands for.
-static bool fills_long_lists(int n, int top, int width, int ff, bool single) {
+// The short lists' grid has a place for every 32 tokens of each expert; those beyond a list's end, about 3,000 a microsecond, count too.
+static bool fills_long_lists(int n, int top, int width, int ff, int experts, bool single) {
   long long tokens = n;
   for (int end = 32; end <= 256 && n <= 256; end *= 2)
     if (n <= end) {
@@ -778,14 +779,17 @@ static bool fills_long_lists(int n, int top, int width, int ff, bool single) {
       break;
     }
   const double flops = (single ? 4.0 : 6.0) * static_cast<double>(tokens * top) * width * ff;
-  return flops / 2e8 >= 7.0 + 0.0125 * (width + ff);  // microseconds
+  const double empty = top < experts ? (tokens + 31) / 32 * static_cast<double>(experts - top) * ((width + 31) / 32 + (ff + 31) / 32) : 0.0;
+  return flops / 2e8 + empty / 3e3 >= 7.0 + 0.0125 * (width + ff);  // microseconds
 }
 
 // out[t, c] = add[t, c] + sum_k weights[t, k] * pair_out[t * top + k, c], k in the order chosen; an identity
 // expert's output is x[t, c].  Eight columns a thread (width is a multiple of 8): 16-byte loads and stores, 25 us
-// at 1,501 tokens of 3584 with one column a thread, 13 so.  Without identity experts there is no branch between the pairs'
-// loads (8 of 32 experts of 64 features, width 128: all four launches 14.5 us at 8 tokens, 12.1 so).  wide: add and out are
-// 16-byte aligned, else element by element.
+// at 1,501 tokens of 3584 with one column a thread, 13 so.  wide: add and out are 16-byte aligned,
+// else element by element.  IDENTITY: a pair may be an identity expert's; the branch lets a token wait for each pair's output
+// before it asks for the next (8 of 32 experts of 64 features, width 128, 8 tokens: all four launches 14.5 us, 12.1
+// without).  From some 500 tokens on others cover that wait and the loop with the branch, which holds less in registers, is as fast
+// or faster (128,000 tokens of one expert each, width 512: 780 us against 842).
 template <bool IDENTITY>
 __global__ void __launch_bounds__(256)
     moe_join_kernel(const float* __restrict__ pair_out, const int32_t* __restrict__ chosen, const bf16* __restrict__ x,
@@ -800,25 +804,28 @@ __global__ void __launch_bounds__(256)
   if (c >= width) return;
   const size_t at = static_cast<size_t>(t) * width + c;
   float total[8] = {};
-  auto join = [&](float weight, float4 y0, float4 y1) {
-    total[0] = fmaf(weight, y0.x, total[0]), total[1] = fmaf(weight, y0.y, total[1]);
-    total[2] = fmaf(weight, y0.z, total[2]), total[3] = fmaf(weight, y0.w, total[3]);
-    total[4] = fmaf(weight, y1.x, total[4]), total[5] = fmaf(weight, y1.y, total[5]);
-    total[6] = fmaf(weight, y1.z, total[6]), total[7] = fmaf(weight, y1.w, total[7]);
-  };
-#pragma unroll 4
-  for (int k = 0; k < top; ++k) {
+  auto join = [&](int k) {
     const size_t pair = static_cast<size_t>(t) * top + k;
     const float weight = weights[pair];
     if (!IDENTITY || chosen[pair] < experts) {
-      const float4* y = reinterpret_cast<const float4*>(pair_out + pair * width + c);
-      join(weight, y[0], y[1]);
+      const float4 *y = reinterpret_cast<const float4*>(pair_out + pair * width + c);
+      const float4 y0 = y[0], y1 = y[1];
+      total[0] = fmaf(weight, y0.x, total[0]), total[1] = fmaf(weight, y0.y, total[1]);
+      total[2] = fmaf(weight, y0.z, total[2]), total[3] = fmaf(weight, y0.w, total[3]);
+      total[4] = fmaf(weight, y1.x, total[4]), total[5] = fmaf(weight, y1.y, total[5]);
+      total[6] = fmaf(weight, y1.z, total[6]), total[7] = fmaf(weight, y1.w, total[7]);
     } else {
       Eight v;
       v.u = *reinterpret_cast<const uint4*>(x + at);
 #pragma unroll
       for (int i = 0; i < 8; ++i) total[i] = fmaf(weight, to_float(v.h[i]), total[i]);
     }
+  };
+  if (IDENTITY) {
+    for (int k = 0; k < top; ++k) join(k);
+  } else {
+#pragma unroll 4
+    for (int k = 0; k < top; ++k) join(k);
   }
   if (add) {
     Eight v;
@@ -932,7 +939,7 @@ extern "C" int shk_moe_experts_grouped(const void* x, const int32_t* chosen, con
   moe_lists_kernel<<<experts, 256, 0, s>>>(chosen, n, top, order, counts);
   const bf16 *xb = static_cast<const bf16*>(x), *actb = static_cast<const bf16*>(act_buf);
   const bool many = static_cast<long long>(n) * top >= 64LL * experts;  // lists of 64 pairs and more on average
-  if (many && tiled && fills_long_lists(n, top, width, ff, w_gate == w_up)) {
+  if (many && tiled && fills_long_lists(n, top, width, ff, experts, w_gate == w_up)) {
     if (w_gate == w_up)
       launch_big<kMoeSingle>(xb, order, counts, w_gate, w_up, static_cast<bf16*>(act_buf), nullptr, n, width, ff, experts, top, form, s);
     else
@@ -964,7 +971,7 @@ extern "C" int shk_moe_experts_grouped(const void* x, const int32_t* chosen, con
   }
   const int join_threads = width >= 2048 ? 256 : kWave;
   const int wide = reinterpret_cast<uintptr_t>(add) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
-  auto join = identity ? moe_join_kernel<true> : moe_join_kernel<false>;
+  auto join = identity || top == 1 || n > 512 ? moe_join_kernel<true> : moe_join_kernel<false>;
   join<<<dim3((width / 8 + join_threads - 1) / join_threads, n), join_threads, 0, s>>>(
       pair_out, chosen, xb, weights, static_cast<const bf16*>(add), add_gate, gate_ld, static_cast<bf16*>(out), width, top, experts, wide);
   SHK_LAUNCH_CHECK("moe_experts_grouped");
