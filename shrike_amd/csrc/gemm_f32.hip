@@ -19,8 +19,9 @@
 // then one run of 1 KiB instead of 16 pieces of 64 bytes (four rows of a 9728 x 896 matrix 10.7 us
 // against 14, of 896 x 4864 13 against 18).  Operands of other callers are row-major.
 // What bounds it: with few rows the latency of one round of loads and a reduction through LDS; with
-// many the matrix instruction (150 TFLOP/s alone), of which loads that are only one step ahead and
-// the ends of workgroups leave half.  Before, one workgroup per 64 x 64 results with vector
+// many the supply of operands and the last round of workgroups, which leave half of the matrix instruction's rate
+// (150 TFLOP/s alone; 9728 x 896 at 509 rows 75): a workgroup's wavefronts walk different parts of k and so share no operand,
+// and loads are one step ahead.  At the full rate that would be 38 GB/s a compute unit, about what one takes in.  Before, one workgroup per 64 x 64 results with vector
 // instructions: a 0.5B decode step of four requests 23.9 ms (2.4 with this kernel, 1.56 with attention_f32.hip as
 // well), a 509-token prompt 42.6 ms (18.9, 6.5); the logits' error against 64 bits 6.4e-7 (2.5e-7).
 #include "api.h"

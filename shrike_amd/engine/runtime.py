@@ -3,8 +3,10 @@ held, and the choice of kernel for each matrix product.
 
 float32: every product runs in the float32 kernel (full float32 arithmetic, one
 order of summation whatever the number of rows), weights in tiles of 16 x 16.  bfloat16: weights are held in the MFMA
-operand layout; products with at most 64 rows stream them once through the
-skinny MFMA kernel, larger ones run the LDS-staged MFMA kernel.  What a mixer
+operand layout; products with at most 16 rows stream them once through the
+skinny kernel, up to 64 through the streaming one, more rows run the LDS-staged one; from 17 rows on matrices of 256 to 2,048
+weight rows (as far as they are quicker so) run without staging, and from 65 on matrices of up to 64 weight rows in the
+skinny kernel, 16 rows a workgroup.  What a mixer
 does between its products is the mixer's own business.
 """
 

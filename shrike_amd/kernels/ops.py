@@ -430,7 +430,8 @@ def gemm_tiled_weight(a, wt, m: int, k: int, out, bias=None, accumulate=False, g
                       splits: int = 1, gate_args=None, activation=None) -> None:
     """out (+)= a @ w.T + bias with wt = retile_weight(w): up to 64 rows of a
     stream the weights once; more rows run the LDS-staged MFMA kernel (tiles of
-    128 x 128 to 256 x 256, chosen by how many the product has).
+    128 x 128 to 256 x 256, chosen by how many the product has); small matrices run
+    without staging.
     splits > 1: out is float32 [splits, n, m] and receives partial sums.
     gated: False, or the gate's activation (one of GATE_ACTIVATIONS; True is "silu") for
     an interleaved gate/up weight.  gate_args: float32 [2] on the device, (limit, up_shift) of
