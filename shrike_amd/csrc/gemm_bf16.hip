@@ -14,17 +14,10 @@
 // The weights are read exactly once from HBM; accumulation is float32.
 #include <cstdlib>
 
-#include "api.h"
-#include "common.h"
+#include "gemm_bf16.h"
 #include "to_lds.h"
 
 namespace shk {
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-// 16 bytes as the compiler's own vector type: copies of it are loads and stores,
-// where copies of HIP's uint4 struct can end up as memcpy through scratch memory
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 union Frag {
   uint4 u;
@@ -61,57 +54,6 @@ struct SkinnyBatch {
   Frag x[kSkinnyBatch][NB];
   uint32_t keep[kSkinnyBatch];  // all ones, or zero where x[u] lies beyond the matrix
 };
-
-__device__ __forceinline__ float silu(float g) { return g / (1.f + __expf(-g)); }
-
-// The activation of a gated product's gate: kActSilu, or the tanh form of GELU,
-// 0.5 g (1 + tanh(sqrt(2/pi) (g + 0.044715 g^3))) = g / (1 + exp(-2 u)).  Gated
-// kernels get the code in the argument that other products use for `accumulate`
-// (a gated product never accumulates).
-// kActRelu is max(g, 0), kActQuickGelu g / (1 + exp(-1.702 g)).
-constexpr int kActSilu = 1, kActGeluTanh = 2, kActRelu = 3, kActQuickGelu = 4;
-__device__ __forceinline__ float gate_act(float g, int act) {
-  if (act == kActGeluTanh) {
-    const float u = 0.7978845608028654f * (g + 0.044715f * g * g * g);
-    return g / (1.f + __expf(-2.f * u));
-  }
-  if (act == kActRelu) return fmaxf(g, 0.f);
-  if (act == kActQuickGelu) return g / (1.f + __expf(-1.702f * g));
-  return silu(g);
-}
-
-// The activation of a plain product: such a product's `accumulate` argument is 0 (store), 1 (add to a
-// float32 output), kPlainReluSquared: the square of max(v, 0) is stored, v the sum with its bias, or 4 *
-// rows: the first `rows` output rows (weight rows) pass SiLU, the others are stored as they are.
-constexpr int kPlainReluSquared = 2, kPlainSiluRows = 4;
-__device__ __forceinline__ float plain_act(float v, int accumulate, int row) {
-  if (accumulate == kPlainReluSquared) {
-    const float r = fmaxf(v, 0.f);
-    return r * r;
-  }
-  return accumulate >= kPlainSiluRows && row < accumulate / kPlainSiluRows ? silu(v) : v;
-}
-// the same argument for the rows from `first` on
-inline int plain_act_from(int accumulate, int first) {
-  if (accumulate < kPlainSiluRows) return accumulate;
-  const int left = accumulate / kPlainSiluRows - first;
-  return left > 0 ? left * kPlainSiluRows : 0;
-}
-
-// act(g) * u of a gated product.  A gate with constants brings them where other products bring their bias
-// (a gated product has none): args[0] > 0 bounds the gate from above and the other factor from both sides
-// before anything else, args[1] is added to that factor.
-__device__ __forceinline__ float gate_times_up(float g, float u, int act, const float* __restrict__ args) {
-  if (args) {
-    const float limit = args[0];
-    if (limit > 0.f) {
-      g = fminf(g, limit);
-      u = fminf(fmaxf(u, -limit), limit);
-    }
-    u += args[1];
-  }
-  return gate_act(g, act) * u;
-}
 
 template <int NB, int RB>
 __device__ __forceinline__ void skinny_load(SkinnyBatch<NB, RB>& b, const uint4* __restrict__ wrow,
@@ -537,45 +479,14 @@ __device__ __forceinline__ void big_store(const f32x4 (&acc)[WM][WN], int lane, 
   }
 }
 
-// gemm_big_kernel: for many tokens (prompt portions).  A workgroup of 4 or 8
-// wavefronts computes a tile of weight rows x tokens, each wavefront a part of
+// gemm_big_kernel: for many tokens whose rows are not 16-byte aligned (gemm_wide.hip serves the others).  A
+// workgroup of 4 to 16 wavefronts computes a tile of weight rows x tokens, each wavefront a part of
 // it as WM x WN MFMA tiles.  Per stage of k, the weights' tiles (already in
 // operand layout) and the activations (re-laid on the way) are staged in LDS
 // "fragment-major": the 16 bytes of lane l of a fragment sit at l * 16, so every
 // LDS access is a conflict-free 128-bit access.  Two LDS buffers alternate, and
-// the loads of the next two stages are in flight (in registers) while a stage is
+// the loads of the next stage are in flight (in registers) while a stage is
 // multiplied.
-
-constexpr int kDies = 8;        // accelerator dies (XCDs), each with an L2 of its own
-constexpr int kDieUnits = 32;  // compute units per die
-
-// The tile of a workgroup of the large kernels; false: none (the grid is padded).
-__device__ __forceinline__ bool big_tile(int tiles_x, int tiles_y, int by_die, int& tile_x, int& tile_y) {
-  // Which tile: workgroups are handed to the chip's eight dies (each with its own
-  // L2) in turn, workgroup p to die p % 8.  The tiles are therefore dealt out in
-  // blocks of 32 (up to 8 token tiles of 32 / that many weight tiles) and block B goes to
-  // die B % 8, whose 32 compute units then work on tiles that share their
-  // operands: the die's L2 serves most of their loads.
-  // With fewer tiles (by_die == 2 * dx) the grid of tiles is cut into dx x 8/dx
-  // rectangles, one for each die, where the numbers of tiles allow that; else
-  // (by_die == 0) the tiles are taken in plain order.
-  tile_x = blockIdx.x % tiles_x, tile_y = blockIdx.x / tiles_x;
-  if (by_die > 1) {
-    const int die = blockIdx.x % kDies, turn = blockIdx.x / kDies;
-    const int dx = by_die / 2, wide = tiles_x / dx, high = tiles_y / (kDies / dx);
-    tile_x = (die % dx) * wide + turn % wide;
-    tile_y = (die / dx) * high + turn / wide;
-  } else if (by_die) {
-    const int die = blockIdx.x % kDies, turn = blockIdx.x / kDies;
-    const int block_y = tiles_y < 8 ? tiles_y : 8, block_x = kDieUnits / block_y;
-    const int blocks_x = (tiles_x + block_x - 1) / block_x;
-    const int block = (turn / kDieUnits) * kDies + die, within = turn % kDieUnits;
-    tile_x = (block % blocks_x) * block_x + within / block_y;
-    tile_y = (block / blocks_x) * block_y + within % block_y;
-    if (within >= block_x * block_y) return false;
-  }
-  return tile_x < tiles_x && tile_y < tiles_y;
-}
 
 // GM x GN wavefronts per workgroup, each with WM x WN MFMA tiles (16 x 16): the
 // workgroup covers 16*GM*WM weight rows x 16*GN*WN tokens.  KS: MFMA steps (32 of
@@ -666,243 +577,20 @@ __global__ void __launch_bounds__(GM* GN* kWave)
               acc[i][jn], 0, 0, 0);
   };
 
-  if (vec && kWFrags % kWaves == 0 && kAFrags % kWaves == 0) {
-    // Aligned rows: every load is unconditional, its address clamped into the
-    // matrices (what an activation row holds past k meets the zeros that pad the
-    // weight tiles), and the loads of two stages are in flight while a stage is
-    // multiplied.
-    const uint4* wsrc[kWPer];
-    const bf16* asrc[kAPer];
-#pragma unroll
-    for (int i = 0; i < kWPer; ++i) {
-      const int rb = (wave + kWaves * i) / KS;
-      const int block = mb0 + rb < mblocks ? mb0 + rb : mblocks - 1;
-      wsrc[i] = wt + static_cast<size_t>(block) * ktiles * kWave + lane;
-    }
-#pragma unroll
-    for (int i = 0; i < kAPer; ++i) {
-      const int rb = (wave + kWaves * i) / KS;
-      const int token = tok0 + rb * 16 + lane % 16;
-      asrc[i] = a + static_cast<size_t>(token < n ? token : n - 1) * lda;  // + (lane / 16) * 8 where that lies in the row
-    }
-    // Two named sets of registers, not an array of two: an array indexed by the
-    // loop's step would live in scratch memory.
-    u32x4 even_w[kWPer], even_x[kAPer], odd_w[kWPer], odd_x[kAPer];
-    auto fetch = [&](u32x4 (&hw)[kWPer], u32x4 (&hx)[kAPer], int st) {
-#pragma unroll
-      for (int i = 0; i < kAPer; ++i) {
-        // (columns beyond k: the row's first 16 bytes, numbers that meet the weight tiles' zeros)
-        const int col = (st * KS + (wave + kWaves * i) % KS) * 32 + (lane / 16) * 8;
-        hx[i] = *reinterpret_cast<const u32x4*>(asrc[i] + (col < k ? col : 0));
-      }
-#pragma unroll
-      for (int i = 0; i < kWPer; ++i) {
-        const int kt = st * KS + (wave + kWaves * i) % KS;
-        hw[i] = *reinterpret_cast<const u32x4*>(wsrc[i] + static_cast<size_t>(kt < ktiles ? kt : 0) * kWave);
-      }
-      __builtin_amdgcn_sched_barrier(0);  // the loads go out before the multiplications
-    };
-    auto put = [&](const u32x4 (&hw)[kWPer], const u32x4 (&hx)[kAPer], int st, int buf) {
-#pragma unroll
-      for (int i = 0; i < kWPer; ++i)
-        *reinterpret_cast<u32x4*>(stage(buf, wave + kWaves * i) + lane) = hw[i];
-#pragma unroll
-      for (int i = 0; i < kAPer; ++i) {
-        // a k-tile past the last one (the stage is not full) must contribute nothing
-        const uint32_t keep = st * KS + (wave + kWaves * i) % KS < ktiles ? ~0u : 0u;
-        *reinterpret_cast<u32x4*>(stage(buf, kWFrags + wave + kWaves * i) + lane) = hx[i] & keep;
-      }
-    };
-    // stage st is multiplied from LDS buffer st % 2 while the loads of stages
-    // st + 1 (issued a step ago) and st + 2 (issued now) are in flight
-    fetch(even_w, even_x, st_first);
-    fetch(odd_w, odd_x, st_first + 1);
-    put(even_w, even_x, st_first, 0);
+  load_stage(st_first);
+  store_stage(0);
+  __syncthreads();
+  for (int st = st_first; st < nstages; ++st) {
+    const int buf = (st - st_first) & 1;
+    if (st + 1 < nstages) load_stage(st + 1);
+    multiply(buf);
+    if (st + 1 < nstages) store_stage(buf ^ 1);
     __syncthreads();
-    // The loop's body has no branch: with one, the compiler moves loads behind it,
-    // next to their use, and nothing is in flight any more.
-    int st = st_first;
-    for (; st + 2 < nstages; st += 2) {
-      fetch(even_w, even_x, st + 2);
-      multiply(0);
-      put(odd_w, odd_x, st + 1, 1);
-      __syncthreads();
-      fetch(odd_w, odd_x, st + 3);
-      multiply(1);
-      put(even_w, even_x, st + 2, 0);
-      __syncthreads();
-    }
-    if (st < nstages) multiply(0);
-    if (st + 1 < nstages) {
-      put(odd_w, odd_x, st + 1, 1);
-      __syncthreads();
-      multiply(1);
-    }
-  } else {
-    load_stage(st_first);
-    store_stage(0);
-    __syncthreads();
-    for (int st = st_first; st < nstages; ++st) {
-      const int buf = (st - st_first) & 1;
-      if (st + 1 < nstages) load_stage(st + 1);
-      multiply(buf);
-      if (st + 1 < nstages) store_stage(buf ^ 1);
-      __syncthreads();
-    }
   }
 
   big_store<WM, WN, GATED>(acc, lane, tok0 + wn * WN * 16, mb0 + wm * WM, n, m, bias, out, ldo, out_f32,
                            accumulate, blockIdx.y);
 }
-
-// gemm_big_lds_kernel: the same tiles, for aligned activations and whole stages
-// of k, with the operands loaded from global memory straight into LDS
-// (global_load_lds_dwordx4: lane l's 16 bytes land at l * 16 of the fragment, the
-// layout above) instead of through registers.  Four stage buffers (three for the
-// largest stages); the loads of the next two stages (one) are in flight while a
-// stage is multiplied, and one barrier
-// per stage both publishes a stage and frees the buffer of the stage before.
-// The compiler cannot see when another wavefront's load has landed: every
-// wavefront waits for its own loads of the stage (s_waitcnt vmcnt, counting the
-// loads issued since) before the barrier.  Each buffer is an LDS array of its
-// own, so that the compiler's own bookkeeping tells the buffers apart and adds
-// no wait for loads into another one.
-template <int GM, int GN, int WM, int WN, int KS, bool GATED>
-__global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per_eu(GM * GN >= 16 ? 4 : 2)))
-    gemm_big_lds_kernel(const bf16* __restrict__ a, int lda, int n, int k,
-                        const uint4* __restrict__ wt, int ktiles, int m,
-                        const float* __restrict__ bias, void* __restrict__ out, int ldo,
-                        int out_f32, int accumulate, int ksplit, int tiles_x, int tiles_y,
-                        int by_die) {
-  constexpr int kWaves = GM * GN;
-  constexpr int kWFrags = GM * WM * KS, kAFrags = GN * WN * KS, kFrags = kWFrags + kAFrags;
-  constexpr int kWPer = kWFrags / kWaves, kAPer = kAFrags / kWaves;
-  constexpr int kLoads = kWPer + kAPer;  // per wavefront and stage
-  static_assert(kWFrags % kWaves == 0 && kAFrags % kWaves == 0, "fragments must divide among the wavefronts");
-  // four stage buffers where they fit into the 160 KiB of LDS, else three
-  constexpr int NS = 4 * kFrags * kWave * 16 <= 160 * 1024 ? 4 : 3;
-  static_assert(NS * kFrags * kWave * 16 <= 160 * 1024, "three stages must fit in LDS");
-  __shared__ u32x4 stage0[kFrags][kWave], stage1[kFrags][kWave], stage2[kFrags][kWave],
-      stage3[NS == 4 ? kFrags : 1][kWave];
-  const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
-  const int wm = wave / GN, wn = wave % GN;
-  int tile_x, tile_y;
-  if (!big_tile(tiles_x, tiles_y, by_die, tile_x, tile_y)) return;
-  const int mb0 = tile_x * (GM * WM);
-  const int tok0 = tile_y * (16 * GN * WN);
-  const int mblocks = (GATED ? 2 : 1) * ((m + 15) / 16);
-  const int all_stages = ktiles / KS;  // the host sends only whole stages here
-  const int per_split = (all_stages + ksplit - 1) / ksplit;
-  const int st_first = blockIdx.y * per_split;
-  const int nstages = st_first + per_split < all_stages ? st_first + per_split : all_stages;
-
-  f32x4 acc[WM][WN];
-#pragma unroll
-  for (int i = 0; i < WM; ++i)
-#pragma unroll
-    for (int jn = 0; jn < WN; ++jn) acc[i][jn] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  // what this wavefront loads: fragments wave, wave + kWaves, ... of either operand,
-  // from rows clamped into the matrices (their products are never stored)
-  const uint4* wsrc[kWPer];
-  const bf16* asrc[kAPer];
-#pragma unroll
-  for (int i = 0; i < kWPer; ++i) {
-    const int rb = (wave + kWaves * i) / KS;
-    const int block = mb0 + rb < mblocks ? mb0 + rb : mblocks - 1;
-    wsrc[i] = wt + static_cast<size_t>(block) * ktiles * kWave + lane;
-  }
-  // Activations, 1 KiB per load.  With stages of 64 of k (KS == 2) a load takes 8
-  // tokens x 128 bytes, lane l the 16 bytes at (token l % 8, chunk l / 8): whole cache
-  // lines, where a fragment of 16 tokens x 64 bytes uses half of each line it touches
-  // and asks the L2 twice as often.  Unit u holds tokens (u / 2) * 16 + (u % 2) * 8 ...
-  // in lane order; lane (j, kg) of the operand of step ks finds its 16 bytes in unit
-  // 2 * block + j / 8 at place j % 8 + 8 * (kg + 4 * ks): groups of 8 lanes read 128
-  // contiguous bytes, without bank conflicts.
-  constexpr bool kUnits = KS == 2;
-#pragma unroll
-  for (int i = 0; i < kAPer; ++i) {
-    const int f = wave + kWaves * i;
-    const int token = kUnits ? tok0 + (f / 2) * 16 + (f % 2) * 8 + lane % 8 : tok0 + (f / KS) * 16 + lane % 16;
-    asrc[i] = a + static_cast<size_t>(token < n ? token : n - 1) * lda;  // + the lane's chunk where it lies in the row
-  }
-  const int xunit = (lane % 16) / 8, xplace = lane % 8 + 8 * (lane / 16);
-  auto load = [&](u32x4 (&buf)[kFrags][kWave], int st) {
-    const int stage = st < all_stages ? st : 0;  // past the end: any stage, never multiplied
-#pragma unroll
-    for (int i = 0; i < kAPer; ++i) {
-      // (a chunk beyond k: the row's first 16 bytes, numbers that meet the weight tiles' zeros)
-      const int col = (kUnits ? stage * 64 : (stage * KS + (wave + kWaves * i) % KS) * 32) +
-                      (kUnits ? lane / 8 : lane / 16) * 8;
-      SHK_LOAD_TO_LDS(asrc[i] + (col < k ? col : 0), &buf[kWFrags + wave + kWaves * i][0]);
-    }
-#pragma unroll
-    for (int i = 0; i < kWPer; ++i) {
-      const int kt = stage * KS + (wave + kWaves * i) % KS;
-      SHK_LOAD_TO_LDS(wsrc[i] + static_cast<size_t>(kt) * kWave, &buf[wave + kWaves * i][0]);
-    }
-  };
-  auto multiply = [&](const u32x4 (&buf)[kFrags][kWave]) {
-    u32x4 af[KS][WN], wf[KS][WM];
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-#pragma unroll
-      for (int jn = 0; jn < WN; ++jn)
-        af[ks][jn] = kUnits ? buf[kWFrags + (wn * WN + jn) * 2 + xunit][xplace + 32 * ks]
-                            : buf[kWFrags + (wn * WN + jn) * KS + ks][lane];
-#pragma unroll
-      for (int i = 0; i < WM; ++i) wf[ks][i] = buf[(wm * WM + i) * KS + ks][lane];
-    }
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-      for (int i = 0; i < WM; ++i)
-#pragma unroll
-        for (int jn = 0; jn < WN; ++jn)
-          acc[i][jn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              __builtin_bit_cast(bf16x8, wf[ks][i]), __builtin_bit_cast(bf16x8, af[ks][jn]),
-              acc[i][jn], 0, 0, 0);
-  };
-  // The stage in `now` has landed for every wavefront once each has waited for its
-  // own loads (the younger stages may stay in flight) and met the others; after the
-  // barrier nobody reads the stage before any more, so its buffer takes new loads.
-#define SHK_LDS_STEP(now, refill, st_refill)  \
-  SHK_MEET_WITH_LOADS((NS - 2) * kLoads);     \
-  load(refill, st_refill);                    \
-  __builtin_amdgcn_sched_barrier(0);          \
-  multiply(now);
-  int st = st_first;
-  if constexpr (NS == 4) {
-    load(stage0, st_first);
-    load(stage1, st_first + 1);
-    load(stage2, st_first + 2);
-    for (; st + 3 < nstages; st += 4) {
-      SHK_LDS_STEP(stage0, stage3, st + 3)
-      SHK_LDS_STEP(stage1, stage0, st + 4)
-      SHK_LDS_STEP(stage2, stage1, st + 5)
-      SHK_LDS_STEP(stage3, stage2, st + 6)
-    }
-    if (st < nstages) { SHK_LDS_STEP(stage0, stage3, st + 3) }
-    if (st + 1 < nstages) { SHK_LDS_STEP(stage1, stage0, st + 4) }
-    if (st + 2 < nstages) { SHK_LDS_STEP(stage2, stage1, st + 5) }
-  } else {
-    load(stage0, st_first);
-    load(stage1, st_first + 1);
-    for (; st + 2 < nstages; st += 3) {
-      SHK_LDS_STEP(stage0, stage2, st + 2)
-      SHK_LDS_STEP(stage1, stage0, st + 3)
-      SHK_LDS_STEP(stage2, stage1, st + 4)
-    }
-    if (st < nstages) { SHK_LDS_STEP(stage0, stage2, st + 2) }
-    if (st + 1 < nstages) { SHK_LDS_STEP(stage1, stage0, st + 3) }
-  }
-#undef SHK_LDS_STEP
-  SHK_WAIT_LOADS(0);  // no load may arrive in LDS that the workgroup has given back
-
-  big_store<WM, WN, GATED>(acc, lane, tok0 + wn * WN * 16, mb0 + wm * WM, n, m, bias, out, ldo, out_f32,
-                           accumulate, blockIdx.y);
-}
-
 
 // gemm_direct_kernel: for small matrices (cached by the time that a few hundred wavefronts ask for them) and
 // from 17 tokens on: nothing is staged.  A wavefront forms RT x CT tiles of 16 weight rows x 16 tokens with both
@@ -1309,42 +997,8 @@ static void launch_big(hipStream_t s, const bf16* ap, int lda, int n, int k, con
                        int gated, int wblocks, int ksplit) {
   constexpr int lds = 2 * (GM * WM + GN * WN) * KS * kWave * 16;
   const int tiles_x = (wblocks + GM * WM - 1) / (GM * WM), tiles_y = (n + 16 * GN * WN - 1) / (16 * GN * WN);
-  // one-dimensional, in whole rounds of the eight dies' blocks of 32 tiles (see the kernel)
-  const int block_y = tiles_y < 8 ? tiles_y : 8, block_x = kDieUnits / block_y;
-  const long long blocks = static_cast<long long>((tiles_x + block_x - 1) / block_x) *
-                           ((tiles_y + block_y - 1) / block_y);
-  // worth it from four rounds of workgroups on: below that, whole dies would stay idle
-  int by_die = static_cast<long long>(tiles_x) * tiles_y >= 4 * kDies * kDieUnits;
-  if (!by_die) {
-    // one rectangle of tiles per die, cut so that a die's tiles share the most
-    // operands (the fewest rows of weights and activations to read per die)
-    long long least = 0;
-    for (int dx = 1; dx <= kDies; dx *= 2) {
-      const int dy = kDies / dx;
-      if (tiles_x % dx || tiles_y % dy) continue;
-      const long long rows = static_cast<long long>(tiles_x / dx) * (16 * GM * WM) +
-                             static_cast<long long>(tiles_y / dy) * (16 * GN * WN);
-      if (!least || rows < least) least = rows, by_die = 2 * dx;
-    }
-  }
-  dim3 grid(by_die == 1 ? static_cast<unsigned>((blocks + kDies - 1) / kDies * kDies * kDieUnits)
-                   : static_cast<unsigned>(tiles_x * tiles_y),
-            ksplit);
-  // The kernel that loads straight into LDS, for workgroups that have a compute unit
-  // to themselves anyway (its three or four stage buffers leave no room for a
-  // second) and at least 128 tokens (with 64 it measured 3 % slower).
-  if constexpr (GM * GN >= 8 && GN * WN >= 8 &&
-                3 * (GM * WM + GN * WN) * KS * kWave * 16 <= 160 * 1024) {
-    if (vec && kt % KS == 0) {
-      if (gated)
-        gemm_big_lds_kernel<GM, GN, WM, WN, KS, true><<<grid, GM * GN * kWave, 0, s>>>(
-            ap, lda, n, k, wp, kt, m, bias, out, ldo, of, accumulate, ksplit, tiles_x, tiles_y, by_die);
-      else
-        gemm_big_lds_kernel<GM, GN, WM, WN, KS, false><<<grid, GM * GN * kWave, 0, s>>>(
-            ap, lda, n, k, wp, kt, m, bias, out, ldo, of, accumulate, ksplit, tiles_x, tiles_y, by_die);
-      return;
-    }
-  }
+  int by_die;
+  const dim3 grid(big_grid(tiles_x, tiles_y, 16 * GM * WM, 16 * GN * WN, &by_die), ksplit);
   if (gated) {
     auto kernel = gemm_big_kernel<GM, GN, WM, WN, KS, true>;
     if (lds > 65536)
@@ -1405,15 +1059,6 @@ static int big_shape(int split, int n, int wblocks, int m, int k) {
 }
 
 extern "C" int shk_gemm_bf16_splits(int n, int m, int k);
-
-// Up to 256 tokens n counts as the power of two above it: a choice made by it is then the same for every number
-// of tokens that a captured decode step may stand for.
-static int counted_tokens(int n) {
-  if (n > 256) return n;
-  int tokens = 32;
-  while (tokens < n) tokens *= 2;
-  return tokens;
-}
 
 // Which gemm_direct_kernel serves a product of n > 16 tokens (0: none): the smallest tile of which a launch has no
 // more than the 256 compute units, for matrices of 256 to 2,048 rows (more of them fill the staged kernels' larger
@@ -1502,6 +1147,7 @@ static int big_main_blocks(int shape, int n, int wblocks, int m, int k, int gate
 // Products that a call with these sizes is made of (1, or 2: see big_main_blocks).
 extern "C" int shk_gemm_bf16_parts(int n, int m, int k, int gated) {
   if (n <= 64 || (!gated && (few_rows(m) || direct_shape(n, m, k, 1))) || shk_gemm_bf16_splits(n, m, k) > 1) return 1;
+  if (k % 8 == 0) return wide_parts(n, m, k, gated);
   const int wblocks = (gated ? 2 : 1) * ((m + 15) / 16);
   return big_main_blocks(big_shape(1, n, wblocks, m, k), n, wblocks, m, k, gated) ? 2 : 1;
 }
@@ -1570,7 +1216,9 @@ static int staged_splits(int n, int m, int k) {
 extern "C" int shk_gemm_bf16_splits(int n, int m, int k) {
   if (n > 64 && few_rows(m) && few_rows_whole(n, m, k)) return 1;
   const int direct = direct_splits(n, m, k);
-  return direct ? direct : staged_splits(n, m, k);
+  if (direct) return direct;
+  const int staged = staged_splits(n, m, k);
+  return n > 64 && k % 8 == 0 ? wide_splits(n, m, k, staged > 1 ? 4 : 2) : staged;
 }
 
 // Whether a reader that adds up shares gets an unsplit product as one float32 share all the same: where
@@ -1623,6 +1271,11 @@ extern "C" int shk_gemm_bf16_tiled_weight(const void* a, const void* wt, const f
   }
   if (n > 64) {
     SHK_REQUIRE(reinterpret_cast<uintptr_t>(out) % 8 == 0, "gemm_bf16: out is not 8-byte aligned");
+    if (vec && wide_serves(lda, k)) {
+      wide_product(s, ap, lda, n, k, wp, m, bias, out, ldo, of, accumulate, gated, ksplit);
+      SHK_LAUNCH_CHECK("gemm_bf16");
+      return 0;
+    }
     const int wblocks = (gated ? 2 : 1) * mb;  // blocks of 16 weight rows
     // Tile of the workgroup: 256 x 256, 256 x 128 or 128 x 128 (weight rows x
     // tokens), whichever big_estimate() expects to finish first.

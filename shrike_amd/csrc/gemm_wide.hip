@@ -1,0 +1,434 @@
+// bfloat16 products of more than 64 tokens, with weights in the tiled layout that gemm_bf16.hip describes: both operands
+// go from global memory straight into LDS, and the instructions that feed the matrix units are laid out between the
+// multiplications by hand.
+//
+// A workgroup of GM x GN wavefronts forms 32*GM*RM weight rows x 32*GN*RN tokens, each wavefront RM x RN tiles of 32 x 32
+// (v_mfma_f32_32x32x16_bf16: half the operand reads of the 16 x 16 form for the same product, and the same sums).
+//
+// k is walked in substeps of 32 (a weight tile) and stages of 64 (whole cache lines of activations).  Weights live in a
+// ring of four substeps, activations in a ring of three stages, so that what is loaded has three substeps to arrive.
+// A wavefront multiplies half a substep (16 of k) while it reads the operands of the next half from LDS: one read behind
+// each of the first multiplications, then the loads that refill what the barrier has just freed.  The barrier stands
+// in the middle of a substep, where all its operands have been read.
+//
+// What bounds it: at 2,048 tokens the power limit.  A stage of the 256 x 256 tile takes 2,180 cycles, the multiplications
+// alone 2,048 to 2,110, at 1.55 to 1.6 GHz where every compute unit works.  What it took to get there from 2,600 and
+// more, measured on the 7B sizes:
+//  * Activations: a load into LDS takes 8 tokens x 128 bytes.  Neighbouring lanes on one token's line cost what a
+//    contiguous load costs; a lane a token, as the kernel before had it, 20 % of the loop (2,634 cycles a stage against 2,155).
+//    The pieces of a line are stored rotated by token (piece c at place c ^ (token % 8)), so that the reads of the
+//    operands, 32 tokens at one piece, meet no bank conflicts.
+//  * The results leave through LDS in whole 16-byte pieces along the rows, by straight-line code without a
+//    branch per value: 2 to 5 us a workgroup, 20 to 30 before.
+// Against the kernel before (16 wavefronts, tiles of 16 x 16, 256 x 256, 256 x 128 and 128 x 128): 7B QKV at 2,048
+// tokens 101 us -> 62, output 67 -> 49, gate/up 500 -> 443 (1.26 PFLOP/s), down 276 -> 235; at 512 tokens QKV 45 -> 25, down
+// 121 -> 74, the 14B QKV 65 -> 42, output 61 -> 34, gate/up 169 -> 130, down 98 -> 69.
+#include "gemm_bf16.h"
+#include "to_lds.h"
+
+#include <type_traits>
+
+namespace shk {
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+
+// 16 bytes a lane from base + offset into LDS at `lds` + 16 * lane.  Not the builtin: for that the compiler
+// waits, before a read of LDS, for loads into any part of the same array.  The kernel waits by itself.
+__device__ __forceinline__ void load_to_lds(unsigned lds, unsigned offset, const char* base) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(offset), "s"(base) : "memory");
+}
+
+template <int GM, int GN, int RM, int RN>
+struct WideShape {
+  static constexpr int kWaves = GM * GN;
+  static constexpr int kTiles = 2 * GM * RM, kUnits = 4 * GN * RN;      // KiB of a substep's weights, of a stage's activations
+  static constexpr int kWLoads = kTiles / kWaves, kXLoads = kUnits / kWaves / 2;  // of a wavefront, a substep
+  static constexpr int kDepth = 3, kWRing = kDepth + 1, kXRing = kDepth;          // substeps; substeps; stages
+  static constexpr int kWBytes = kTiles * 1024, kXBytes = kUnits * 1024;
+  static constexpr int kLds = kWRing * kWBytes + kXRing * kXBytes;
+  static_assert(kWLoads * kWaves == kTiles && 2 * kXLoads * kWaves == kUnits, "loads divide evenly among the wavefronts");
+  static_assert(kLds <= 160 * 1024 && kDepth * (kWLoads + kXLoads) <= 63, "fits LDS and the load counter");
+  static_assert(kWaves * 32 * (32 * RM * 4 + 16) <= kLds, "the results of 32 tokens a wavefront fit LDS");
+};
+
+template <int GM, int GN, int RM, int RN, bool GATED>
+__global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per_eu(GM * GN / 4, GM * GN / 4)))
+    gemm_wide_kernel(const bf16* __restrict__ a, int lda, int n, int k, const uint4* __restrict__ wt, int ktiles, int m,
+                     const float* __restrict__ bias, void* __restrict__ out, int ldo, int out_f32, int accumulate, int whole,
+                     int ksplit, int tiles_x, int tiles_y, int by_die) {
+  using S = WideShape<GM, GN, RM, RN>;
+  constexpr int N = RM * RN, R = RM + RN, WL = S::kWLoads, XL = S::kXLoads;
+  static_assert(N >= R || (RM == 2 && RN == 2), "a multiplication for every read");
+  __shared__ u32x4 mem[S::kLds / 16];
+  const int tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int wm = wave / GN, wn = wave % GN;
+  int tile_x, tile_y;
+  if (!big_tile(tiles_x, tiles_y, by_die, tile_x, tile_y)) return;
+  const int mb0 = tile_x * S::kTiles, tok0 = tile_y * (32 * GN * RN);
+  // blocks of 16 weight rows; a gated weight has two per 16 output rows
+  const int mblocks = (GATED ? 2 : 1) * ((m + 15) / 16);
+  // this share's stages of k; the last stage of k may be half a one
+  const int all = (ktiles + 1) / 2;
+  const int first = static_cast<int>(static_cast<long long>(all) * blockIdx.y / ksplit);
+  const int stages = static_cast<int>(static_cast<long long>(all) * (blockIdx.y + 1) / ksplit) - first;
+  if (stages == 0) {  // more shares than stages: zeros
+    float* o = static_cast<float*>(out) + static_cast<size_t>(blockIdx.y) * n * ldo;
+    for (int i = tid; i < 32 * GN * RN * 16 * S::kTiles; i += S::kWaves * kWave) {
+      const int token = tok0 + i / (16 * S::kTiles), row = mb0 * 16 + i % (16 * S::kTiles);
+      if (token < n && row < m) o[static_cast<size_t>(token) * ldo + row] = 0.f;
+    }
+    return;
+  }
+  const int left = ktiles - 2 * first, subs = 2 * stages < left ? 2 * stages : left;
+
+  // What a wavefront loads: weight tiles and units of 8 tokens wave, wave + kWaves, ..., from rows clamped into the
+  // matrices (their products are never stored).  In the last stage of k a piece beyond k is replaced by the
+  // stage's first (numbers that meet the zeros which pad the weight tiles).
+  unsigned woff[WL], xoff[2 * XL];
+#pragma unroll
+  for (int i = 0; i < WL; ++i) {
+    const int rb = wave + S::kWaves * i;
+    const int block = mb0 + rb < mblocks ? rb : mblocks - 1 - mb0;
+    woff[i] = (static_cast<unsigned>(block) * ktiles * kWave + lane) * 16u;
+  }
+  const unsigned piece = (lane % 8) ^ (lane / 8);
+#pragma unroll
+  for (int i = 0; i < 2 * XL; ++i) {
+    const int t = (wave + S::kWaves * i) * 8 + lane / 8;
+    const int token = tok0 + t < n ? t : n - 1 - tok0;
+    xoff[i] = static_cast<unsigned>(token) * lda * 2u + piece * 16u;
+  }
+  const unsigned beyond = (all - 1) * 64 + static_cast<int>(piece) * 8 < k ? 0u : piece * 16u;
+  const char* wsrc = reinterpret_cast<const char*>(wt) + (static_cast<size_t>(mb0) * ktiles + 2 * first) * 1024;
+  const char* xsrc = reinterpret_cast<const char*>(a) + static_cast<size_t>(tok0) * lda * 2 + static_cast<size_t>(first) * 128;
+  const unsigned base =
+      static_cast<unsigned>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)&mem[0])) + wave * 1024;
+  constexpr int kX0 = S::kWRing * S::kWBytes;  // where the activations' ring begins
+
+  // (past the share's end: substep or stage 0 again, never multiplied)
+  auto load_w = [&](int at, int sub, int i) {
+    load_to_lds(base + at + i * S::kWaves * 1024, woff[i], wsrc + static_cast<size_t>(sub < subs ? sub : 0) * 1024);
+  };
+  auto load_x = [&](int at, int st, int half, int i) {
+    st = st < stages ? st : 0;
+    const unsigned cut = first + st == all - 1 ? ~0u : 0u;
+    load_to_lds(base + kX0 + at + (half * XL + i) * S::kWaves * 1024, xoff[half * XL + i] - (beyond & cut),
+                xsrc + static_cast<size_t>(st) * 128);
+  };
+
+  f32x16 acc[RM][RN];
+#pragma unroll
+  for (int i = 0; i < RM; ++i)
+#pragma unroll
+    for (int jn = 0; jn < RN; ++jn)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][jn][r] = 0.f;
+
+  // Operands of 16 of k: lane l holds row (or token) l % 32, k (l / 32) * 8 .. + 8 of them.
+  const char* lds = reinterpret_cast<const char*>(&mem[0]);
+  const int wat = (wm * RM * 2 + (lane % 32) / 16) * 1024 + ((lane / 32) * 16 + lane % 16) * 16;
+  int xat[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+    xat[c] = kX0 + (wn * RN * 32 + lane % 32) * 128 + ((2 * c + lane / 32) ^ (lane % 8)) * 16;
+  struct Operands {
+    u32x4 w[RM], x[RN];
+  } even, odd;
+  // operand i of half h of a substep in the weights' ring at `watp`, the stage's substep p in the activations' at `xatp`
+  auto read = [&](Operands& f, int watp, int xatp, int p, int h, int i) {
+    if (i < RM)
+      f.w[i] = *reinterpret_cast<const u32x4*>(lds + wat + watp + i * 2048 + 512 * h);
+    else
+      f.x[i - RM] = *reinterpret_cast<const u32x4*>(lds + xat[2 * p + h] + xatp + (i - RM) * 4096);
+  };
+  auto multiply = [&](const Operands& f, int q) {
+    const int i = q / RN, jn = q % RN;
+    acc[i][jn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, f.w[i]),
+                                                         __builtin_bit_cast(bf16x8, f.x[jn]), acc[i][jn], 0, 0, 0);
+  };
+  auto after_w = [](int at, int by) {
+    return at + by * S::kWBytes < S::kWRing * S::kWBytes ? at + by * S::kWBytes : at + (by - S::kWRing) * S::kWBytes;
+  };
+  auto after_x = [](int at, int by) {
+    return at + by * S::kXBytes < S::kXRing * S::kXBytes ? at + by * S::kXBytes : at + (by - S::kXRing) * S::kXBytes;
+  };
+
+  // Loads go out in the order in which they are waited for: per substep its weights and half a stage of activations.
+#pragma unroll
+  for (int i = 0; i < XL; ++i) load_x(0, 0, 0, i);
+#pragma unroll
+  for (int sub = 0; sub < S::kWRing; ++sub) {
+#pragma unroll
+    for (int i = 0; i < WL; ++i) load_w(sub * S::kWBytes, sub, i);
+#pragma unroll
+    for (int i = 0; i < XL; ++i) load_x((sub + 1) / 2 * S::kXBytes, (sub + 1) / 2, (sub + 1) % 2, i);
+  }
+  SHK_MEET_WITH_LOADS(S::kDepth * (WL + XL));
+#pragma unroll
+  for (int i = 0; i < R; ++i) read(even, 0, 0, 0, 0, i);
+// Half a substep: its multiplications, and behind each of the first a read for the next half and one of the loads.
+// Nothing is moved across sched_barrier, so this is the order in which they are issued.
+#define SHK_WIDE_HALF(now, next, watp, xatp, p, h, loads, LOAD) \
+  _Pragma("unroll") for (int q = 0; q < (N > R ? N : R); ++q) { \
+    if (q < N) multiply(now, q);                                \
+    if (q < R) read(next, watp, xatp, p, h, q);                 \
+    if (q >= 1 && q <= loads) {                                 \
+      const int i = q - 1;                                      \
+      LOAD;                                                     \
+    }                                                           \
+    __builtin_amdgcn_sched_barrier(0);                          \
+  }
+// The stage's first substep from its second half on, its second substep's first half.
+#define SHK_WIDE_STAGE()                                                             \
+  SHK_MEET_WITH_LOADS((S::kDepth - 1) * (WL + XL));                                  \
+  const int w1 = after_w(wp, 1), xlast = after_x(xp, S::kXRing - 1);                 \
+  SHK_WIDE_HALF(odd, even, w1, xp, 1, 0, WL, load_w(wp, 2 * s + S::kWRing, i))       \
+  SHK_WIDE_HALF(even, odd, w1, xp, 1, 1, XL, load_x(xlast, s + S::kXRing - 1, 1, i))
+  int s = 0, wp = 0, xp = 0;  // stage; where its first substep and its activations lie in the rings
+  SHK_WIDE_HALF(even, odd, 0, 0, 0, 1, 0, (void)i)
+  for (; s + 1 < stages; ++s) {
+    SHK_WIDE_STAGE()
+    SHK_MEET_WITH_LOADS((S::kDepth - 1) * (WL + XL));
+    const int w2 = after_w(wp, 2), x1 = after_x(xp, 1);
+    SHK_WIDE_HALF(odd, even, w2, x1, 0, 0, WL, load_w(w1, 2 * s + 1 + S::kWRing, i))
+    SHK_WIDE_HALF(even, odd, w2, x1, 0, 1, XL, load_x(xp, s + S::kXRing, 0, i))
+    wp = w2, xp = x1;
+  }
+  if (2 * s + 1 < subs) {
+    SHK_WIDE_STAGE()
+  }
+#pragma unroll
+  for (int q = 0; q < N; ++q) multiply(odd, q);
+#undef SHK_WIDE_HALF
+#undef SHK_WIDE_STAGE
+  SHK_WAIT_LOADS(0);
+  __syncthreads();  // nothing more is loaded into LDS or read from the rings
+
+  // Accumulator register g * 4 + r of lane (j, half): token j, row g * 8 + half * 4 + r.  Gated: rows 0 to 15 of a tile
+  // belong to the gate, 16 to 31 are the same rows of the other factor.
+  constexpr int kRows = (GATED ? 16 : 32) * RM;  // output rows of a wavefront
+  const int half = lane / 32, j = lane % 32;
+  const int row0 = (GATED ? mb0 / 2 : mb0) * 16 + wm * kRows, tok = tok0 + wn * RN * 32;
+  const size_t plane = static_cast<size_t>(blockIdx.y) * n;
+  if (row0 >= m) return;  // (no barrier follows)
+  char* mine = reinterpret_cast<char*>(&mem[0]) + wave * (32 * (32 * RM * 4 + 16));
+#define SHK_WIDE_LANDED() asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory")
+  if (whole) {
+    // Rows in whole 16-byte pieces and at most a bias or SiLU's gate: finished in registers.
+    auto finish = [&](auto f32) {
+      constexpr bool F32 = decltype(f32)::value;
+      constexpr int E = F32 ? 4 : 2, kPitch = kRows * E + 16, kPieces = kRows * E / 16;
+      auto put = [&](const f32x16 (&c)[RN], int jn, int i) {
+#pragma unroll
+        for (int g = 0; g < (GATED ? 2 : 4); ++g) {
+          const int row = (GATED ? 16 : 32) * i + g * 8 + half * 4;
+          f32x4 v;
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            v[r] = GATED ? gate_times_up(c[jn][g * 4 + r], c[jn][(GATED ? 8 : 0) + g * 4 + r], kActSilu, nullptr) : c[jn][g * 4 + r];
+          if (!GATED && bias && row0 + row < m) {
+            const f32x4 b = *reinterpret_cast<const f32x4*>(bias + row0 + row);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] += b[r];
+          }
+          if constexpr (F32) {
+            *reinterpret_cast<f32x4*>(mine + j * kPitch + row * 4) = v;
+          } else {
+            bf16x4 o;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[r] = static_cast<__bf16>(v[r]);
+            *reinterpret_cast<bf16x4*>(mine + j * kPitch + row * 2) = o;
+          }
+        }
+      };
+#pragma unroll
+      for (int jn = 0; jn < RN; ++jn) {
+        put(acc[0], jn, 0);
+        put(acc[1], jn, 1);
+        if constexpr (RM > 2) put(acc[2], jn, 2);
+        if constexpr (RM > 3) put(acc[3], jn, 3);
+        SHK_WIDE_LANDED();
+#pragma unroll
+        for (int q = 0; q < 32 * kPieces / kWave; ++q) {
+          const int at = q * kWave + lane, t = at / kPieces, p = at % kPieces, token = tok + jn * 32 + t, row = row0 + p * (16 / E);
+          const u32x4 v = *reinterpret_cast<const u32x4*>(mine + t * kPitch + p * 16);
+          if (token < n && row < m)
+            *reinterpret_cast<u32x4*>(static_cast<char*>(out) + ((plane + token) * ldo + row) * E) = v;
+        }
+        SHK_WIDE_LANDED();
+      }
+    };
+    if (out_f32)
+      finish(std::true_type{});
+    else
+      finish(std::false_type{});
+    return;
+  }
+  // Anything else: the sums go through LDS as they are, and a loop of single values finishes them.
+  constexpr int kPitch = 32 * RM * 4 + 16;
+  auto put = [&](const f32x16 (&c)[RN], int jn, int i) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      f32x4 v;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = c[jn][g * 4 + r];
+      *reinterpret_cast<f32x4*>(mine + j * kPitch + (i * 32 + g * 8 + half * 4) * 4) = v;
+    }
+  };
+#pragma unroll
+  for (int jn = 0; jn < RN; ++jn) {
+    put(acc[0], jn, 0);
+    put(acc[1], jn, 1);
+    if constexpr (RM > 2) put(acc[2], jn, 2);
+    if constexpr (RM > 3) put(acc[3], jn, 3);
+    SHK_WIDE_LANDED();
+#pragma unroll 1
+    for (int at = lane; at < 32 * kRows; at += kWave) {
+      const int t = at / kRows, p = at % kRows, token = tok + jn * 32 + t, row = row0 + p;
+      if (token >= n || row >= m) continue;
+      const float* sums = reinterpret_cast<const float*>(mine + t * kPitch);
+      const size_t idx = (plane + token) * ldo + row;
+      float v;
+      if (GATED)
+        v = gate_times_up(sums[p / 16 * 32 + p % 16], sums[p / 16 * 32 + 16 + p % 16], accumulate, bias);
+      else
+        v = plain_act(sums[p] + (bias ? bias[row] : 0.f), accumulate, row);
+      if (out_f32) {
+        float* o = static_cast<float*>(out) + idx;
+        *o = (accumulate == 1 && !GATED) ? *o + v : v;
+      } else {
+        static_cast<bf16*>(out)[idx] = from_float<bf16>(v);
+      }
+    }
+    SHK_WIDE_LANDED();
+  }
+#undef SHK_WIDE_LANDED
+}
+
+// The tiles, and what they were measured to take: a workgroup's start and end, a stage of 64 of k with the chip nearly
+// empty (its loads' latency) and what is added when all its compute units work (the power limit), in us; workgroups that
+// fit on the chip.  From 13 products of 512 to 8,192 tokens in one to three shares: within 15 % of nearly all.
+struct WideTile {
+  int rows, tokens, units;
+  double ends, alone, full;
+};
+static const WideTile kWide[] = {{256, 256, 256, 5.0, 0.897, 0.663}, {256, 192, 256, 7.0, 0.720, 0.460}, {192, 256, 256, 7.0, 0.791, 0.400},
+                                 {192, 192, 256, 7.0, 0.524, 0.405}, {256, 128, 256, 3.5, 0.718, 0.167}, {128, 256, 256, 5.0, 0.631, 0.205},
+                                 {128, 192, 256, 5.0, 0.428, 0.224}, {128, 128, 512, 3.5, 0.360, 0.620}};
+constexpr int kWideTiles = sizeof(kWide) / sizeof(kWide[0]);
+
+static double wide_estimate(const WideTile& t, int split, int n, int wblocks, int k) {
+  const long long groups = static_cast<long long>((wblocks * 16 + t.rows - 1) / t.rows) * ((n + t.tokens - 1) / t.tokens) * split;
+  const double stages = static_cast<double>(((k + 63) / 64 + split - 1) / split);
+  const double rounds = static_cast<double>(groups / t.units), rest = static_cast<double>(groups % t.units) / t.units;
+  double us = 2.0 + rounds * (t.ends + stages * (t.alone + t.full));
+  if (rest > 0.0) us += t.ends + stages * (t.alone + t.full * rest);
+  return us;
+}
+
+// The tile of the least estimate.
+static int wide_tile(int split, int n, int wblocks, int k, double* least) {
+  int best = 0;
+  *least = wide_estimate(kWide[0], split, n, wblocks, k);
+  for (int i = 1; i < kWideTiles; ++i) {
+    const double us = wide_estimate(kWide[i], split, n, wblocks, k);
+    if (us < *least) *least = us, best = i;
+  }
+  return best;
+}
+
+// Tiles that do not make whole rounds of the compute units (256 x 256 tiles of the 7B gate/up matrix at 512 tokens: 296) are
+// better run as two products: the rows whose tiles make whole rounds, then the others with the tile that suits them.
+struct WidePlan {
+  int tile, main_blocks, rest_tile;  // main_blocks: blocks of 16 weight rows of the first product, 0: one product
+};
+static WidePlan wide_plan(int split, int n, int wblocks, int k, double* us) {
+  n = counted_tokens(n);
+  WidePlan plan = {0, 0, 0};
+  plan.tile = wide_tile(split, n, wblocks, k, us);
+  if (split > 1) return plan;
+  const double whole = *us;
+  for (int i = 0; i < kWideTiles; ++i) {
+    const WideTile& t = kWide[i];
+    const int tiles_x = (wblocks * 16 + t.rows - 1) / t.rows, tiles_y = (n + t.tokens - 1) / t.tokens;
+    const long long total = static_cast<long long>(tiles_x) * tiles_y;
+    const int main_x = static_cast<int>(total / t.units * t.units / tiles_y);
+    if (total <= t.units || main_x <= 0 || main_x >= tiles_x) continue;
+    const int main_blocks = main_x * (t.rows / 16);
+    double rest;
+    const int rest_tile = wide_tile(1, n, wblocks - main_blocks, k, &rest);
+    const double both = wide_estimate(t, 1, n, main_blocks, k) + rest;
+    if (both < 0.97 * whole && both < *us) *us = both, plan = {i, main_blocks, rest_tile};
+  }
+  return plan;
+}
+
+// Shares of k: at most 16, of at least 16 tiles of 32, that the estimate expects to be the fastest with what writing and
+// reading the output costs: float32 parts, or `whole_bytes` a value of an unsplit product (3 TB/s).
+int wide_splits(int n, int m, int k, int whole_bytes) {
+  const int mblocks = (m + 15) / 16, ktiles = (k + 31) / 32;
+  const int most = ktiles / 16 < 16 ? ktiles / 16 : 16;
+  int best = 1;
+  double least;
+  wide_plan(1, n, mblocks, k, &least);
+  const double values = static_cast<double>(counted_tokens(n)) * m;
+  least += 2.0 * values * whole_bytes / 3e6;
+  for (int split = 2; split <= most; ++split) {
+    double us;
+    wide_plan(split, n, mblocks, k, &us);
+    us += 2.0 * values * split * 4.0 / 3e6;
+    if (us < 0.97 * least) least = us, best = split;  // more shares only for a clear gain
+  }
+  return best;
+}
+
+int wide_parts(int n, int m, int k, int gated) {
+  double us;
+  return wide_plan(1, n, (gated ? 2 : 1) * ((m + 15) / 16), k, &us).main_blocks ? 2 : 1;
+}
+
+// Whether offsets within a tile fit 32 bits.
+bool wide_serves(int lda, int k) { return lda <= 4 * 1024 * 1024 && k <= 4 * 1024 * 1024; }
+
+template <int GM, int GN, int RM, int RN>
+static void launch_wide(hipStream_t s, const bf16* a, int lda, int n, int k, const uint4* wt, int m, int wblocks, const float* bias,
+                        void* out, int ldo, int out_f32, int accumulate, int gated, int ksplit) {
+  using S = WideShape<GM, GN, RM, RN>;
+  const int tiles_x = (wblocks + S::kTiles - 1) / S::kTiles, tiles_y = (n + 32 * GN * RN - 1) / (32 * GN * RN);
+  int by_die;
+  const unsigned groups = big_grid(tiles_x, tiles_y, 16 * S::kTiles, 32 * GN * RN, &by_die);
+  const int per = out_f32 ? 4 : 8;  // values of 16 bytes
+  const int whole = m % per == 0 && ldo % per == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0 &&
+                    reinterpret_cast<uintptr_t>(bias) % 16 == 0 && (gated ? accumulate == kActSilu && !bias : accumulate == 0);
+  const int ktiles = (k + 31) / 32;
+  if (gated)
+    gemm_wide_kernel<GM, GN, RM, RN, true><<<dim3(groups, ksplit), S::kWaves * kWave, 0, s>>>(
+        a, lda, n, k, wt, ktiles, m, bias, out, ldo, out_f32, accumulate, whole, ksplit, tiles_x, tiles_y, by_die);
+  else
+    gemm_wide_kernel<GM, GN, RM, RN, false><<<dim3(groups, ksplit), S::kWaves * kWave, 0, s>>>(
+        a, lda, n, k, wt, ktiles, m, bias, out, ldo, out_f32, accumulate, whole, ksplit, tiles_x, tiles_y, by_die);
+}
+
+void wide_product(hipStream_t s, const bf16* a, int lda, int n, int k, const uint4* wt, int m, const float* bias, void* out,
+                  int ldo, int out_f32, int accumulate, int gated, int ksplit) {
+  static decltype(&launch_wide<2, 2, 2, 2>) const launch[kWideTiles] = {
+      launch_wide<2, 4, 4, 2>, launch_wide<2, 2, 4, 3>, launch_wide<2, 2, 3, 4>, launch_wide<2, 2, 3, 3>,
+      launch_wide<4, 2, 2, 2>, launch_wide<2, 2, 2, 4>, launch_wide<2, 2, 2, 3>, launch_wide<2, 2, 2, 2>};
+  const int wblocks = (gated ? 2 : 1) * ((m + 15) / 16);
+  double us;
+  const WidePlan plan = wide_plan(ksplit, n, wblocks, k, &us);
+  if (!plan.main_blocks) {
+    launch[plan.tile](s, a, lda, n, k, wt, m, wblocks, bias, out, ldo, out_f32, accumulate, gated, ksplit);
+    return;
+  }
+  const int main_rows = plan.main_blocks * 16 / (gated ? 2 : 1);
+  launch[plan.tile](s, a, lda, n, k, wt, main_rows, plan.main_blocks, bias, out, ldo, out_f32, accumulate, gated, 1);
+  // (a gated product's `bias` is its gate's two constants, the same for every row)
+  launch[plan.rest_tile](s, a, lda, n, k, wt + static_cast<size_t>(plan.main_blocks) * ((k + 31) / 32) * kWave, m - main_rows,
+                            wblocks - plan.main_blocks, bias && !gated ? bias + main_rows : bias,
+                            static_cast<char*>(out) + static_cast<size_t>(main_rows) * (out_f32 ? 4 : 2), ldo, out_f32,
+                            gated ? accumulate : plain_act_from(accumulate, main_rows), gated, 1);
+}
+
+}  // namespace shk
