@@ -1,56 +1,17 @@
-// bfloat16 products of more than 64 tokens, with weights in the tiled layout that gemm_bf16.hip describes: both operands
-// go from global memory straight into LDS, and the instructions that feed the matrix units are laid out between the
-// multiplications by hand.
+// bfloat16 products of more than 64 tokens, with weights in the tiled layout that gemm_bf16.hip describes: wide_loop()
+// of gemm_wide.h in eight tile sizes.
 //
-// A workgroup of GM x GN wavefronts forms 32*GM*RM weight rows x 32*GN*RN tokens, each wavefront RM x RN tiles of 32 x 32
-// (v_mfma_f32_32x32x16_bf16: half the operand reads of the 16 x 16 form for the same product, and the same sums).
-//
-// k is walked in substeps of 32 (a weight tile) and stages of 64 (whole cache lines of activations).  Weights live in a
-// ring of four substeps, activations in a ring of three stages, so that what is loaded has three substeps to arrive.
-// A wavefront multiplies half a substep (16 of k) while it reads the operands of the next half from LDS: one read behind
-// each of the first multiplications, then the loads that refill what the barrier has just freed.  The barrier stands
-// in the middle of a substep, where all its operands have been read.
-//
-// What bounds it: at 2,048 tokens the power limit.  A stage of the 256 x 256 tile takes 2,180 cycles, the multiplications
-// alone 2,048 to 2,110, at 1.55 to 1.6 GHz where every compute unit works.  What it took to get there from 2,600 and
-// more, measured on the 7B sizes:
-//  * Activations: a load into LDS takes 8 tokens x 128 bytes.  Neighbouring lanes on one token's line cost what a
-//    contiguous load costs; a lane a token, as the kernel before had it, 20 % of the loop (2,634 cycles a stage against 2,155).
-//    The pieces of a line are stored rotated by token (piece c at place c ^ (token % 8)), so that the reads of the
-//    operands, 32 tokens at one piece, meet no bank conflicts.
-//  * The results leave through LDS in whole 16-byte pieces along the rows, by straight-line code without a
-//    branch per value: 2 to 5 us a workgroup, 20 to 30 before.
+// The results leave through LDS in whole 16-byte pieces along the rows, by straight-line code without a branch per
+// value: 2 to 5 us a workgroup, 20 to 30 where every value was tested and stored for itself.
 // Against the kernel before (16 wavefronts, tiles of 16 x 16, 256 x 256, 256 x 128 and 128 x 128): 7B QKV at 2,048
 // tokens 101 us -> 62, output 67 -> 49, gate/up 500 -> 443 (1.26 PFLOP/s), down 276 -> 235; at 512 tokens QKV 45 -> 25, down
 // 121 -> 74, the 14B QKV 65 -> 42, output 61 -> 34, gate/up 169 -> 130, down 98 -> 69.
 #include "gemm_bf16.h"
-#include "to_lds.h"
+#include "gemm_wide.h"
 
 #include <type_traits>
 
 namespace shk {
-
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-
-// 16 bytes a lane from base + offset into LDS at `lds` + 16 * lane.  Not the builtin: for that the compiler
-// waits, before a read of LDS, for loads into any part of the same array.  The kernel waits by itself.
-__device__ __forceinline__ void load_to_lds(unsigned lds, unsigned offset, const char* base) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(offset), "s"(base) : "memory");
-}
-
-template <int GM, int GN, int RM, int RN>
-struct WideShape {
-  static constexpr int kWaves = GM * GN;
-  static constexpr int kTiles = 2 * GM * RM, kUnits = 4 * GN * RN;      // KiB of a substep's weights, of a stage's activations
-  static constexpr int kWLoads = kTiles / kWaves, kXLoads = kUnits / kWaves / 2;  // of a wavefront, a substep
-  static constexpr int kDepth = 3, kWRing = kDepth + 1, kXRing = kDepth;          // substeps; substeps; stages
-  static constexpr int kWBytes = kTiles * 1024, kXBytes = kUnits * 1024;
-  static constexpr int kLds = kWRing * kWBytes + kXRing * kXBytes;
-  static_assert(kWLoads * kWaves == kTiles && 2 * kXLoads * kWaves == kUnits, "loads divide evenly among the wavefronts");
-  static_assert(kLds <= 160 * 1024 && kDepth * (kWLoads + kXLoads) <= 63, "fits LDS and the load counter");
-  static_assert(kWaves * 32 * (32 * RM * 4 + 16) <= kLds, "the results of 32 tokens a wavefront fit LDS");
-};
 
 template <int GM, int GN, int RM, int RN, bool GATED>
 __global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per_eu(GM * GN / 4, GM * GN / 4)))
@@ -58,8 +19,7 @@ __global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per
                      const float* __restrict__ bias, void* __restrict__ out, int ldo, int out_f32, int accumulate, int whole,
                      int ksplit, int tiles_x, int tiles_y, int by_die) {
   using S = WideShape<GM, GN, RM, RN>;
-  constexpr int N = RM * RN, R = RM + RN, WL = S::kWLoads, XL = S::kXLoads;
-  static_assert(N >= R || (RM == 2 && RN == 2), "a multiplication for every read");
+  constexpr int WL = S::kWLoads, XL = S::kXLoads;
   __shared__ u32x4 mem[S::kLds / 16];
   const int tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int wm = wave / GN, wn = wave % GN;
@@ -102,108 +62,9 @@ __global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per
   const unsigned beyond = (all - 1) * 64 + static_cast<int>(piece) * 8 < k ? 0u : piece * 16u;
   const char* wsrc = reinterpret_cast<const char*>(wt) + (static_cast<size_t>(mb0) * ktiles + 2 * first) * 1024;
   const char* xsrc = reinterpret_cast<const char*>(a) + static_cast<size_t>(tok0) * lda * 2 + static_cast<size_t>(first) * 128;
-  const unsigned base =
-      static_cast<unsigned>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)&mem[0])) + wave * 1024;
-  constexpr int kX0 = S::kWRing * S::kWBytes;  // where the activations' ring begins
-
-  // (past the share's end: substep or stage 0 again, never multiplied)
-  auto load_w = [&](int at, int sub, int i) {
-    load_to_lds(base + at + i * S::kWaves * 1024, woff[i], wsrc + static_cast<size_t>(sub < subs ? sub : 0) * 1024);
-  };
-  auto load_x = [&](int at, int st, int half, int i) {
-    st = st < stages ? st : 0;
-    const unsigned cut = first + st == all - 1 ? ~0u : 0u;
-    load_to_lds(base + kX0 + at + (half * XL + i) * S::kWaves * 1024, xoff[half * XL + i] - (beyond & cut),
-                xsrc + static_cast<size_t>(st) * 128);
-  };
 
   f32x16 acc[RM][RN];
-#pragma unroll
-  for (int i = 0; i < RM; ++i)
-#pragma unroll
-    for (int jn = 0; jn < RN; ++jn)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][jn][r] = 0.f;
-
-  // Operands of 16 of k: lane l holds row (or token) l % 32, k (l / 32) * 8 .. + 8 of them.
-  const char* lds = reinterpret_cast<const char*>(&mem[0]);
-  const int wat = (wm * RM * 2 + (lane % 32) / 16) * 1024 + ((lane / 32) * 16 + lane % 16) * 16;
-  int xat[4];
-#pragma unroll
-  for (int c = 0; c < 4; ++c)
-    xat[c] = kX0 + (wn * RN * 32 + lane % 32) * 128 + ((2 * c + lane / 32) ^ (lane % 8)) * 16;
-  struct Operands {
-    u32x4 w[RM], x[RN];
-  } even, odd;
-  // operand i of half h of a substep in the weights' ring at `watp`, the stage's substep p in the activations' at `xatp`
-  auto read = [&](Operands& f, int watp, int xatp, int p, int h, int i) {
-    if (i < RM)
-      f.w[i] = *reinterpret_cast<const u32x4*>(lds + wat + watp + i * 2048 + 512 * h);
-    else
-      f.x[i - RM] = *reinterpret_cast<const u32x4*>(lds + xat[2 * p + h] + xatp + (i - RM) * 4096);
-  };
-  auto multiply = [&](const Operands& f, int q) {
-    const int i = q / RN, jn = q % RN;
-    acc[i][jn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, f.w[i]),
-                                                         __builtin_bit_cast(bf16x8, f.x[jn]), acc[i][jn], 0, 0, 0);
-  };
-  auto after_w = [](int at, int by) {
-    return at + by * S::kWBytes < S::kWRing * S::kWBytes ? at + by * S::kWBytes : at + (by - S::kWRing) * S::kWBytes;
-  };
-  auto after_x = [](int at, int by) {
-    return at + by * S::kXBytes < S::kXRing * S::kXBytes ? at + by * S::kXBytes : at + (by - S::kXRing) * S::kXBytes;
-  };
-
-  // Loads go out in the order in which they are waited for: per substep its weights and half a stage of activations.
-#pragma unroll
-  for (int i = 0; i < XL; ++i) load_x(0, 0, 0, i);
-#pragma unroll
-  for (int sub = 0; sub < S::kWRing; ++sub) {
-#pragma unroll
-    for (int i = 0; i < WL; ++i) load_w(sub * S::kWBytes, sub, i);
-#pragma unroll
-    for (int i = 0; i < XL; ++i) load_x((sub + 1) / 2 * S::kXBytes, (sub + 1) / 2, (sub + 1) % 2, i);
-  }
-  SHK_MEET_WITH_LOADS(S::kDepth * (WL + XL));
-#pragma unroll
-  for (int i = 0; i < R; ++i) read(even, 0, 0, 0, 0, i);
-// Half a substep: its multiplications, and behind each of the first a read for the next half and one of the loads.
-// Nothing is moved across sched_barrier, so this is the order in which they are issued.
-#define SHK_WIDE_HALF(now, next, watp, xatp, p, h, loads, LOAD) \
-  _Pragma("unroll") for (int q = 0; q < (N > R ? N : R); ++q) { \
-    if (q < N) multiply(now, q);                                \
-    if (q < R) read(next, watp, xatp, p, h, q);                 \
-    if (q >= 1 && q <= loads) {                                 \
-      const int i = q - 1;                                      \
-      LOAD;                                                     \
-    }                                                           \
-    __builtin_amdgcn_sched_barrier(0);                          \
-  }
-// The stage's first substep from its second half on, its second substep's first half.
-#define SHK_WIDE_STAGE()                                                             \
-  SHK_MEET_WITH_LOADS((S::kDepth - 1) * (WL + XL));                                  \
-  const int w1 = after_w(wp, 1), xlast = after_x(xp, S::kXRing - 1);                 \
-  SHK_WIDE_HALF(odd, even, w1, xp, 1, 0, WL, load_w(wp, 2 * s + S::kWRing, i))       \
-  SHK_WIDE_HALF(even, odd, w1, xp, 1, 1, XL, load_x(xlast, s + S::kXRing - 1, 1, i))
-  int s = 0, wp = 0, xp = 0;  // stage; where its first substep and its activations lie in the rings
-  SHK_WIDE_HALF(even, odd, 0, 0, 0, 1, 0, (void)i)
-  for (; s + 1 < stages; ++s) {
-    SHK_WIDE_STAGE()
-    SHK_MEET_WITH_LOADS((S::kDepth - 1) * (WL + XL));
-    const int w2 = after_w(wp, 2), x1 = after_x(xp, 1);
-    SHK_WIDE_HALF(odd, even, w2, x1, 0, 0, WL, load_w(w1, 2 * s + 1 + S::kWRing, i))
-    SHK_WIDE_HALF(even, odd, w2, x1, 0, 1, XL, load_x(xp, s + S::kXRing, 0, i))
-    wp = w2, xp = x1;
-  }
-  if (2 * s + 1 < subs) {
-    SHK_WIDE_STAGE()
-  }
-#pragma unroll
-  for (int q = 0; q < N; ++q) multiply(odd, q);
-#undef SHK_WIDE_HALF
-#undef SHK_WIDE_STAGE
-  SHK_WAIT_LOADS(0);
-  __syncthreads();  // nothing more is loaded into LDS or read from the rings
+  wide_loop<GM, GN, RM, RN>(acc, mem, wsrc, woff, xsrc, xoff, beyond, all - 1 - first, subs, stages);
 
   // Accumulator register g * 4 + r of lane (j, half): token j, row g * 8 + half * 4 + r.  Gated: rows 0 to 15 of a tile
   // belong to the gate, 16 to 31 are the same rows of the other factor.
@@ -213,7 +74,6 @@ __global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per
   const size_t plane = static_cast<size_t>(blockIdx.y) * n;
   if (row0 >= m) return;  // (no barrier follows)
   char* mine = reinterpret_cast<char*>(&mem[0]) + wave * (32 * (32 * RM * 4 + 16));
-#define SHK_WIDE_LANDED() asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory")
   if (whole) {
     // Rows in whole 16-byte pieces and at most a bias or SiLU's gate: finished in registers.
     auto finish = [&](auto f32) {
@@ -248,7 +108,7 @@ __global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per
         put(acc[1], jn, 1);
         if constexpr (RM > 2) put(acc[2], jn, 2);
         if constexpr (RM > 3) put(acc[3], jn, 3);
-        SHK_WIDE_LANDED();
+        SHK_LDS_DONE();
 #pragma unroll
         for (int q = 0; q < 32 * kPieces / kWave; ++q) {
           const int at = q * kWave + lane, t = at / kPieces, p = at % kPieces, token = tok + jn * 32 + t, row = row0 + p * (16 / E);
@@ -256,7 +116,7 @@ __global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per
           if (token < n && row < m)
             *reinterpret_cast<u32x4*>(static_cast<char*>(out) + ((plane + token) * ldo + row) * E) = v;
         }
-        SHK_WIDE_LANDED();
+        SHK_LDS_DONE();
       }
     };
     if (out_f32)
@@ -282,7 +142,7 @@ __global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per
     put(acc[1], jn, 1);
     if constexpr (RM > 2) put(acc[2], jn, 2);
     if constexpr (RM > 3) put(acc[3], jn, 3);
-    SHK_WIDE_LANDED();
+    SHK_LDS_DONE();
 #pragma unroll 1
     for (int at = lane; at < 32 * kRows; at += kWave) {
       const int t = at / kRows, p = at % kRows, token = tok + jn * 32 + t, row = row0 + p;
@@ -301,9 +161,8 @@ __global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per
         static_cast<bf16*>(out)[idx] = from_float<bf16>(v);
       }
     }
-    SHK_WIDE_LANDED();
+    SHK_LDS_DONE();
   }
-#undef SHK_WIDE_LANDED
 }
 
 // The tiles, and what they were measured to take: a workgroup's start and end, a stage of 64 of k with the chip nearly

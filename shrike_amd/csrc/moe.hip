@@ -29,7 +29,7 @@
 // are kept in float32 and joined per token in the order the experts were chosen.
 #include "api.h"
 #include "common.h"
-#include "to_lds.h"
+#include "gemm_wide.h"
 
 namespace shk {
 
@@ -637,16 +637,15 @@ __device__ __forceinline__ bool moe_tile(const int32_t* counts, int experts, int
 enum MoeProduct : int { kMoeGated = 0, kMoeSingle = 1, kMoeDown = 2 };
 
 template <int PRODUCT>
-__global__ void __launch_bounds__(kBigWaves* kWave)
+__global__ void __launch_bounds__(kBigWaves* kWave) __attribute__((amdgpu_waves_per_eu(2, 2)))
     moe_big_mfma_kernel(const bf16* __restrict__ a, const int32_t* __restrict__ order,
                         const int32_t* __restrict__ counts, const bf16* __restrict__ w0, const bf16* __restrict__ w1,
                         bf16* __restrict__ act_out, float* __restrict__ pair_out, int n, int k, int m, int experts, int top,
                         GateForm form) {
-  constexpr int GN = 2, WM = 4, WN = 4;                         // wavefronts along the pairs; tiles of 16 x 16 a wavefront
-  constexpr int kWUnits = kBigRows / 8, kUnits = kWUnits + kBigPairs / 8, kLoads = kUnits / kBigWaves, kWLoads = kWUnits / kBigWaves;
+  using S = WideShape<4, 2, 2, 2>;
+  static_assert(S::kWaves == kBigWaves && 16 * S::kTiles == kBigRows && 8 * S::kUnits == kBigPairs, "one tile of wide_loop()");
   constexpr int kFeatures = PRODUCT == kMoeGated ? kBigRows / 2 : kBigRows;
-  typedef unsigned int u4 __attribute__((ext_vector_type(4)));
-  __shared__ u4 stage0[kUnits][kWave], stage1[kUnits][kWave], stage2[kUnits][kWave];
+  __shared__ u32x4 mem[S::kLds / 16];
   const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int features = (m + kFeatures - 1) / kFeatures;
   int total, e, within, row_tiles;
@@ -659,97 +658,63 @@ __global__ void __launch_bounds__(kBigWaves* kWave)
   row_tiles = __builtin_amdgcn_readfirstlane(row_tiles);
   const int count = min(counts[e], n), row0 = within % row_tiles * kBigPairs, f0 = within / row_tiles * kFeatures;
   const int32_t* list = order + static_cast<size_t>(e) * n;
-  const int wm = wave / GN, wn = wave % GN;
 
-  // what this wavefront loads: units wave, wave + 8, ..: weight tiles first (block u / 2, step u % 2), then
-  // pairs' rows; rows beyond either matrix are read as its last (their products are not stored)
-  const bf16* src[kLoads];
+  // What this wavefront loads: weight tiles and units of 8 pairs wave, wave + 8; rows beyond either matrix are read as its
+  // last (their products are not stored).  Gated: even tiles are the gate's features, odd ones the same features of up.
+  const bool up = PRODUCT == kMoeGated && wave % 2;
+  unsigned woff[S::kWLoads], xoff[2 * S::kXLoads];
 #pragma unroll
-  for (int i = 0; i < kLoads; ++i) {
-    const int u = wave + kBigWaves * i;
-    if (i < kWLoads) {
-      const int block = u / 2;  // wavefront block / 4's tile block % 4
-      // (gated: tiles 0 and 1 are gate features, 2 and 3 the same features of up)
-      const int f = PRODUCT == kMoeGated ? f0 + block / 4 * 32 + block % 2 * 16 : f0 + block * 16;
-      src[i] = (PRODUCT == kMoeGated && block % 4 >= 2 ? w1 : w0) +
-               ((static_cast<size_t>(e) * m + min(f, m - 16)) / 16 * (k / 32) + u % 2) * 512 + lane * 8;
-    } else {
-      const int at = row0 + (u - kWUnits) * 8 + lane % 8;
-      const int pair = list[at < count ? at : row0];
-      src[i] = a + static_cast<size_t>(PRODUCT == kMoeDown ? min(max(pair, 0), n * top - 1) : min(max(pair, 0) / top, n - 1)) * k +
-               lane / 8 * 8;
-    }
+  for (int i = 0; i < S::kWLoads; ++i) {
+    const int tile = wave + kBigWaves * i, f = f0 + (PRODUCT == kMoeGated ? tile / 2 : tile) * 16;
+    woff[i] = (static_cast<unsigned>(min(f, m - 16) / 16) * (k / 32) * kWave + lane) * 16u;
   }
-  const int stages = k / 64;
-  auto load = [&](u4 (&buf)[kUnits][kWave], int st) {
-    const size_t at = static_cast<size_t>(st < stages ? st : 0) * 64;  // past the end: any stage, never multiplied
 #pragma unroll
-    for (int i = 0; i < kLoads; ++i) SHK_LOAD_TO_LDS(src[i] + (i < kWLoads ? at * 16 : at), &buf[wave + kBigWaves * i][0]);
-  };
-  mf32x4 acc[WM][WN];
-#pragma unroll
-  for (int i = 0; i < WM; ++i)
-#pragma unroll
-    for (int jn = 0; jn < WN; ++jn) acc[i][jn] = mf32x4{0.f, 0.f, 0.f, 0.f};
-  const int unit = lane % 16 / 8, place = lane % 8 + 8 * (lane / 16);
-  auto multiply = [&](const u4 (&buf)[kUnits][kWave]) {
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      u4 wf[WM], af[WN];
-#pragma unroll
-      for (int jn = 0; jn < WN; ++jn) af[jn] = buf[kWUnits + (wn * WN + jn) * 2 + unit][place + 32 * ks];
-#pragma unroll
-      for (int i = 0; i < WM; ++i) wf[i] = buf[(wm * WM + i) * 2 + ks][lane];
-#pragma unroll
-      for (int i = 0; i < WM; ++i)
-#pragma unroll
-        for (int jn = 0; jn < WN; ++jn)
-          acc[i][jn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(mbf16x8, wf[i]),
-                                                               __builtin_bit_cast(mbf16x8, af[jn]), acc[i][jn], 0, 0, 0);
-    }
-  };
-  // a stage has landed for every wavefront once each has waited for its own loads of it (the younger stage's
-  // may stay in flight) and met the others; after the barrier nobody reads the stage before any more
-#define SHK_MOE_STEP(now, refill, st_refill) \
-  SHK_MEET_WITH_LOADS(kLoads);               \
-  load(refill, st_refill);                   \
-  __builtin_amdgcn_sched_barrier(0);         \
-  multiply(now);
-  load(stage0, 0);
-  load(stage1, 1);
-  int st = 0;
-  for (; st + 2 < stages; st += 3) {
-    SHK_MOE_STEP(stage0, stage2, st + 2)
-    SHK_MOE_STEP(stage1, stage0, st + 3)
-    SHK_MOE_STEP(stage2, stage1, st + 4)
+  for (int i = 0; i < 2 * S::kXLoads; ++i) {
+    const int at = row0 + (wave + kBigWaves * i) * 8 + lane / 8;
+    const int pair = max(list[at < count ? at : row0], 0);
+    const int row = PRODUCT == kMoeDown ? min(pair, n * top - 1) : min(pair / top, n - 1);
+    xoff[i] = static_cast<unsigned>(row) * k * 2u + ((lane % 8) ^ (lane / 8)) * 16u;
   }
-  if (st < stages) { SHK_MOE_STEP(stage0, stage2, st + 2) }
-  if (st + 1 < stages) { SHK_MOE_STEP(stage1, stage0, st + 3) }
-#undef SHK_MOE_STEP
-  SHK_WAIT_LOADS(0);  // no load may arrive in LDS that the workgroup has given back
+  f32x16 acc[2][2];
+  wide_loop<4, 2, 2, 2>(acc, mem, reinterpret_cast<const char*>((up ? w1 : w0) + static_cast<size_t>(e) * m * k), woff,
+                        reinterpret_cast<const char*>(a), xoff, 0u, -1, k / 32, k / 64);
 
-  // lane (j, kg) holds weight rows 4 kg + r of a tile for pair j
-  const int j = lane % 16, kg = lane / 16;
+  // Register g * 4 + r of lane (j, half) of a tile of 32 x 32 holds weight row g * 8 + half * 4 + r for pair j.  32 pairs'
+  // sums at a time go through LDS and leave in 16-byte pieces along the pairs' rows.
+  constexpr int kRows = PRODUCT == kMoeGated ? 32 : 64;           // output features of a wavefront
+  constexpr int kPitch = 64 * 4 + 16, kValues = PRODUCT == kMoeDown ? 4 : 8, kPieces = kRows / kValues;
+  const int half = lane / 32, j = lane % 32, first = f0 + wave / 2 * kRows;
+  char* mine = reinterpret_cast<char*>(mem) + wave * 32 * kPitch;
 #pragma unroll
-  for (int jn = 0; jn < WN; ++jn) {
-    const int at = row0 + (wn * WN + jn) * 16 + j;
-    if (at >= count) continue;
-    const size_t pair = min(max(list[at], 0), n * top - 1);
+  for (int jn = 0; jn < 2; ++jn) {
 #pragma unroll
-    for (int i = 0; i < (PRODUCT == kMoeGated ? WM / 2 : WM); ++i) {
-      const int f = f0 + (PRODUCT == kMoeGated ? wm * 32 + i * 16 : (wm * WM + i) * 16) + 4 * kg;
-      if (f >= m) continue;  // (m is a multiple of 8: four features are inside or outside together)
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<f32x4*>(mine + j * kPitch + (i * 32 + g * 8 + half * 4) * 4) =
+            f32x4{acc[i][jn][g * 4], acc[i][jn][g * 4 + 1], acc[i][jn][g * 4 + 2], acc[i][jn][g * 4 + 3]};
+    SHK_LDS_DONE();
+#pragma unroll 1
+    for (int q = lane; q < 32 * kPieces; q += kWave) {
+      const int t = q / kPieces, row = q % kPieces * kValues, at = row0 + (wave % 2 * 2 + jn) * 32 + t, f = first + row;
+      if (at >= count || f >= m) continue;  // (m is a multiple of 64: a piece is inside or outside as a whole)
+      const size_t pair = min(max(list[at], 0), n * top - 1);
+      const float* sums = reinterpret_cast<const float*>(mine + t * kPitch);
       if (PRODUCT == kMoeDown) {
-        *reinterpret_cast<mf32x4*>(pair_out + pair * m + f) = acc[i][jn];
+        *reinterpret_cast<f32x4*>(pair_out + pair * m + f) = *reinterpret_cast<const f32x4*>(sums + row);
       } else {
-        uint16_t h[4];
+        const float* gate = sums + (PRODUCT == kMoeGated ? row / 16 * 32 + row % 16 : row);
+        u32x4 v;
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          h[r] = bf16_bits(gate_times_up(acc[i][jn][r], PRODUCT == kMoeGated ? acc[(i + WM / 2) % WM][jn][r] : acc[i][jn][r], form));
-        *reinterpret_cast<uint2*>(act_out + pair * m + f) =
-            make_uint2(h[0] | static_cast<uint32_t>(h[1]) << 16, h[2] | static_cast<uint32_t>(h[3]) << 16);
+        for (int r = 0; r < 4; ++r) {
+          const int apart = PRODUCT == kMoeGated ? 16 : 0;
+          v[r] = bf16_bits(gate_times_up(gate[2 * r], gate[2 * r + apart], form)) |
+                 static_cast<uint32_t>(bf16_bits(gate_times_up(gate[2 * r + 1], gate[2 * r + 1 + apart], form))) << 16;
+        }
+        *reinterpret_cast<u32x4*>(act_out + pair * m + f) = v;
       }
     }
+    SHK_LDS_DONE();
   }
 }
 
@@ -939,7 +904,10 @@ extern "C" int shk_moe_experts_grouped(const void* x, const int32_t* chosen, con
   moe_lists_kernel<<<experts, 256, 0, s>>>(chosen, n, top, order, counts);
   const bf16 *xb = static_cast<const bf16*>(x), *actb = static_cast<const bf16*>(act_buf);
   const bool many = static_cast<long long>(n) * top >= 64LL * experts;  // lists of 64 pairs and more on average
-  if (many && tiled && fills_long_lists(n, top, width, ff, experts, w_gate == w_up)) {
+  // (offsets within an operand of moe_big_mfma_kernel are 32 bits wide)
+  const bool near = static_cast<long long>(n) * (width > static_cast<long long>(top) * ff ? width : static_cast<long long>(top) * ff) < (1LL << 31) &&
+                    static_cast<long long>(width) * ff < (1LL << 31);
+  if (many && tiled && near && fills_long_lists(n, top, width, ff, experts, w_gate == w_up)) {
     if (w_gate == w_up)
       launch_big<kMoeSingle>(xb, order, counts, w_gate, w_up, static_cast<bf16*>(act_buf), nullptr, n, width, ff, experts, top, form, s);
     else
