@@ -747,14 +747,13 @@ __global__ void __launch_bounds__(16 * kWave)
 
   // What a wavefront fetches of the stage's activations, 1 KiB at a time: unit f is
   // (token block f / KT, pair of tiles (f % KT) / 2, half of the block's tokens
-  // f % 2): 8 tokens x 128 bytes, lane l taking the 16 bytes at (token l % 8,
-  // chunk l / 8) - whole cache lines, where a fragment of 16 tokens x 64 bytes
-  // would use half of each line it touches.  In LDS the unit lies in lane order;
-  // lane (j, kg) of the operand of tile t finds its 16 bytes in unit (j / 8) at
-  // place j % 8 + 8 * (kg + 4 * (t % 2)): groups of 8 lanes read 128 contiguous
-  // bytes, without bank conflicts.  Beyond the last unit the first ones are
+  // f % 2): 8 tokens x 128 bytes, lane l taking piece (l % 8) ^ (l / 8) of token l / 8: whole cache lines, eight
+  // neighbouring lanes on one (a lane a token: a 7B step of 64 sequences 4.39 ms, 4.25 so).  In LDS the unit lies in lane order, so a
+  // token's pieces lie rotated by its number, and lane (j, kg) of the operand of tile t finds its 16 bytes in unit
+  // (j / 8), piece 4 * (t % 2) + kg of token j % 8: without bank conflicts.  Beyond the last unit the first ones are
   // fetched again.
   static_assert(KT % 2 == 0, "tiles are fetched in pairs");
+  const int piece = (lane % 8) ^ (lane / 8);
   const bf16* asrc[APER];
   int afrag[APER];
 #pragma unroll
@@ -762,8 +761,8 @@ __global__ void __launch_bounds__(16 * kWave)
     int f = wave + waves * i;
     f = f < kFrags ? f : f % kFrags;
     afrag[i] = f;
-    const int token = (f / KT) * 16 + (f % 2) * 8 + lane % 8;
-    asrc[i] = a + static_cast<size_t>(token < n ? token : n - 1) * lda;  // + (lane / 8) * 8 where that lies in the row
+    const int token = (f / KT) * 16 + (f % 2) * 8 + lane / 8;
+    asrc[i] = a + static_cast<size_t>(token < n ? token : n - 1) * lda;  // + piece * 8 where that lies in the row
   }
   auto fetch = [&](u32x4 (&buf)[kFrags][kWave], u32x4 (&w)[KT], int st) {
     // past the share's end: some stage that exists, never multiplied
@@ -773,7 +772,7 @@ __global__ void __launch_bounds__(16 * kWave)
     for (int i = 0; i < APER; ++i) {
       // a chunk beyond k is fetched from the row's first 16 bytes instead (it meets zeros of the
       // weight tiles' padding, so it must be numbers, not whatever lies behind the matrix)
-      const int col = (stage * KT + ((afrag[i] % KT) / 2) * 2) * 32 + (lane / 8) * 8;
+      const int col = (stage * KT + ((afrag[i] % KT) / 2) * 2) * 32 + piece * 8;
       SHK_LOAD_TO_LDS(asrc[i] + (col < k ? col : 0), &buf[afrag[i]][0]);
     }
 #pragma unroll
@@ -782,7 +781,8 @@ __global__ void __launch_bounds__(16 * kWave)
       w[t] = __builtin_nontemporal_load(wrow + static_cast<size_t>(tt < ktiles ? tt : ktiles - 1) * kWave);
     }
   };
-  const int xunit = j / 8, xplace = j % 8 + 8 * kg;  // where this lane's operands lie
+  // where this lane's operands of even and odd tiles lie
+  const int xunit = j / 8, xplace[2] = {j % 8 * 8 + (kg ^ j % 8), j % 8 * 8 + ((4 + kg) ^ j % 8)};
   auto multiply = [&](const u32x4 (&buf)[kFrags][kWave], const u32x4 (&w)[KT], int tiles) {
 #pragma unroll
     for (int t = 0; t < KT; ++t) {
@@ -791,7 +791,7 @@ __global__ void __launch_bounds__(16 * kWave)
         for (int b = 0; b < NB; ++b)
           acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
               __builtin_bit_cast(bf16x8, w[t]),
-              __builtin_bit_cast(bf16x8, buf[b * KT + (t / 2) * 2 + xunit][xplace + 32 * (t % 2)]), acc[b],
+              __builtin_bit_cast(bf16x8, buf[b * KT + (t / 2) * 2 + xunit][xplace[t % 2]]), acc[b],
               0, 0, 0);
       }
     }
