@@ -167,6 +167,26 @@ __device__ __forceinline__ void wide_loop(f32x16 (&acc)[RM][RN], u32x4* mem, con
   __syncthreads();
 }
 
+// The tiles, and what they were measured to take: a workgroup's start and end, a stage of 64 of k with the chip nearly
+// empty (its loads' latency) and what is added when all its compute units work (the power limit), in us; workgroups that
+// fit on the chip.  From 13 products of 512 to 8,192 tokens in one to three shares: within 15 % of nearly all.
+struct WideTile {
+  int rows, tokens, units;
+  double ends, alone, full;
+};
+constexpr WideTile kWide[] = {{256, 256, 256, 5.0, 0.897, 0.663}, {256, 192, 256, 7.0, 0.720, 0.460}, {192, 256, 256, 7.0, 0.791, 0.400},
+                                 {192, 192, 256, 7.0, 0.524, 0.405}, {256, 128, 256, 3.5, 0.718, 0.167}, {128, 256, 256, 5.0, 0.631, 0.205},
+                                 {128, 192, 256, 5.0, 0.428, 0.224}, {128, 128, 512, 3.5, 0.360, 0.620}};
+constexpr int kWideTiles = sizeof(kWide) / sizeof(kWide[0]);
+
+// Microseconds of `groups` workgroups of a tile, each walking `stages` stages of k.
+inline double wide_time(const WideTile& t, double groups, int stages) {
+  const double rounds = static_cast<double>(static_cast<long long>(groups) / t.units), rest = (groups - rounds * t.units) / t.units;
+  double us = 2.0 + rounds * (t.ends + stages * (t.alone + t.full));
+  if (rest > 0.0) us += t.ends + stages * (t.alone + t.full * rest);
+  return us;
+}
+
 // Until this wavefront's accesses to LDS are done.
 #define SHK_LDS_DONE() asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory")
 

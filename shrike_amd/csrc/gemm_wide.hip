@@ -165,25 +165,9 @@ __global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per
   }
 }
 
-// The tiles, and what they were measured to take: a workgroup's start and end, a stage of 64 of k with the chip nearly
-// empty (its loads' latency) and what is added when all its compute units work (the power limit), in us; workgroups that
-// fit on the chip.  From 13 products of 512 to 8,192 tokens in one to three shares: within 15 % of nearly all.
-struct WideTile {
-  int rows, tokens, units;
-  double ends, alone, full;
-};
-static const WideTile kWide[] = {{256, 256, 256, 5.0, 0.897, 0.663}, {256, 192, 256, 7.0, 0.720, 0.460}, {192, 256, 256, 7.0, 0.791, 0.400},
-                                 {192, 192, 256, 7.0, 0.524, 0.405}, {256, 128, 256, 3.5, 0.718, 0.167}, {128, 256, 256, 5.0, 0.631, 0.205},
-                                 {128, 192, 256, 5.0, 0.428, 0.224}, {128, 128, 512, 3.5, 0.360, 0.620}};
-constexpr int kWideTiles = sizeof(kWide) / sizeof(kWide[0]);
-
 static double wide_estimate(const WideTile& t, int split, int n, int wblocks, int k) {
   const long long groups = static_cast<long long>((wblocks * 16 + t.rows - 1) / t.rows) * ((n + t.tokens - 1) / t.tokens) * split;
-  const double stages = static_cast<double>(((k + 63) / 64 + split - 1) / split);
-  const double rounds = static_cast<double>(groups / t.units), rest = static_cast<double>(groups % t.units) / t.units;
-  double us = 2.0 + rounds * (t.ends + stages * (t.alone + t.full));
-  if (rest > 0.0) us += t.ends + stages * (t.alone + t.full * rest);
-  return us;
+  return wide_time(t, static_cast<double>(groups), ((k + 63) / 64 + split - 1) / split);
 }
 
 // The tile of the least estimate.

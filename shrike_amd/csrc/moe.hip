@@ -604,15 +604,14 @@ __global__ void __launch_bounds__(256)
 // took 350 and 213, through registers 449 and 276: what it waits for is memory that is read 128 bytes at a time.
 // Pairs' rows laid out in tiles first (19 us a layer) changed nothing, nor did leaving out the multiplications
 // for the empty half of a list's last tile: the loads are what takes the time, about 42 GB/s a compute unit.
-constexpr int kBigPairs = 128, kBigRows = 256, kBigWaves = 8;
-
-// Tile `index` of all experts' live tiles (features x ceil(count / kBigPairs) each): expert, first feature
+// Tile `index` of all experts' live tiles (features x ceil(count / PAIRS) each): expert, first feature
 // tile, first pair; false beyond the last.  `index` < 0 asks for none and returns their number in `total`.
+template <int PAIRS>
 __device__ __forceinline__ bool moe_tile(const int32_t* counts, int experts, int n, int features, int index, int lane,
                                          int& total, int& e, int& within, int& row_tiles) {
   total = 0;
   for (int e0 = 0; e0 < experts; e0 += kWave) {
-    const int mine = e0 + lane < experts ? (min(counts[e0 + lane], n) + kBigPairs - 1) / kBigPairs : 0;
+    const int mine = e0 + lane < experts ? (min(counts[e0 + lane], n) + PAIRS - 1) / PAIRS : 0;
     int before = mine;  // inclusive prefix over the lanes
 #pragma unroll
     for (int d = 1; d < kWave; d <<= 1) {
@@ -636,59 +635,59 @@ __device__ __forceinline__ bool moe_tile(const int32_t* counts, int experts, int
 
 enum MoeProduct : int { kMoeGated = 0, kMoeSingle = 1, kMoeDown = 2 };
 
-template <int PRODUCT>
-__global__ void __launch_bounds__(kBigWaves* kWave) __attribute__((amdgpu_waves_per_eu(2, 2)))
+template <int PRODUCT, int GM, int GN, int RM, int RN>
+__global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per_eu(GM * GN / 4, GM * GN / 4)))
     moe_big_mfma_kernel(const bf16* __restrict__ a, const int32_t* __restrict__ order,
                         const int32_t* __restrict__ counts, const bf16* __restrict__ w0, const bf16* __restrict__ w1,
                         bf16* __restrict__ act_out, float* __restrict__ pair_out, int n, int k, int m, int experts, int top,
                         GateForm form) {
-  using S = WideShape<4, 2, 2, 2>;
-  static_assert(S::kWaves == kBigWaves && 16 * S::kTiles == kBigRows && 8 * S::kUnits == kBigPairs, "one tile of wide_loop()");
-  constexpr int kFeatures = PRODUCT == kMoeGated ? kBigRows / 2 : kBigRows;
+  using S = WideShape<GM, GN, RM, RN>;
+  constexpr int kRows = 32 * GM * RM, kPairs = 32 * GN * RN, kFeatures = PRODUCT == kMoeGated ? kRows / 2 : kRows;
+  static_assert(PRODUCT != kMoeGated || S::kWaves % 2 == 0, "a wavefront loads tiles of one of the two matrices");
   __shared__ u32x4 mem[S::kLds / 16];
   const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int features = (m + kFeatures - 1) / kFeatures;
   int total, e, within, row_tiles;
-  moe_tile(counts, experts, n, features, -1, lane, total, e, within, row_tiles);
+  moe_tile<kPairs>(counts, experts, n, features, -1, lane, total, e, within, row_tiles);
   const int per_die = (total + 7) / 8, turn = blockIdx.x / 8;
   if (turn >= per_die) return;
-  if (!moe_tile(counts, experts, n, features, blockIdx.x % 8 * per_die + turn, lane, total, e, within, row_tiles)) return;
+  if (!moe_tile<kPairs>(counts, experts, n, features, blockIdx.x % 8 * per_die + turn, lane, total, e, within, row_tiles)) return;
   e = __builtin_amdgcn_readfirstlane(e);
   within = __builtin_amdgcn_readfirstlane(within);
   row_tiles = __builtin_amdgcn_readfirstlane(row_tiles);
-  const int count = min(counts[e], n), row0 = within % row_tiles * kBigPairs, f0 = within / row_tiles * kFeatures;
+  const int count = min(counts[e], n), row0 = within % row_tiles * kPairs, f0 = within / row_tiles * kFeatures;
   const int32_t* list = order + static_cast<size_t>(e) * n;
 
-  // What this wavefront loads: weight tiles and units of 8 pairs wave, wave + 8; rows beyond either matrix are read as its
+  // What this wavefront loads: weight tiles and units of 8 pairs wave, wave + kWaves, ..; rows beyond either matrix are read as its
   // last (their products are not stored).  Gated: even tiles are the gate's features, odd ones the same features of up.
   const bool up = PRODUCT == kMoeGated && wave % 2;
   unsigned woff[S::kWLoads], xoff[2 * S::kXLoads];
 #pragma unroll
   for (int i = 0; i < S::kWLoads; ++i) {
-    const int tile = wave + kBigWaves * i, f = f0 + (PRODUCT == kMoeGated ? tile / 2 : tile) * 16;
+    const int tile = wave + S::kWaves * i, f = f0 + (PRODUCT == kMoeGated ? tile / 2 : tile) * 16;
     woff[i] = (static_cast<unsigned>(min(f, m - 16) / 16) * (k / 32) * kWave + lane) * 16u;
   }
 #pragma unroll
   for (int i = 0; i < 2 * S::kXLoads; ++i) {
-    const int at = row0 + (wave + kBigWaves * i) * 8 + lane / 8;
+    const int at = row0 + (wave + S::kWaves * i) * 8 + lane / 8;
     const int pair = max(list[at < count ? at : row0], 0);
     const int row = PRODUCT == kMoeDown ? min(pair, n * top - 1) : min(pair / top, n - 1);
     xoff[i] = static_cast<unsigned>(row) * k * 2u + ((lane % 8) ^ (lane / 8)) * 16u;
   }
-  f32x16 acc[2][2];
-  wide_loop<4, 2, 2, 2>(acc, mem, reinterpret_cast<const char*>((up ? w1 : w0) + static_cast<size_t>(e) * m * k), woff,
+  f32x16 acc[RM][RN];
+  wide_loop<GM, GN, RM, RN>(acc, mem, reinterpret_cast<const char*>((up ? w1 : w0) + static_cast<size_t>(e) * m * k), woff,
                         reinterpret_cast<const char*>(a), xoff, 0u, -1, k / 32, k / 64);
 
   // Register g * 4 + r of lane (j, half) of a tile of 32 x 32 holds weight row g * 8 + half * 4 + r for pair j.  32 pairs'
   // sums at a time go through LDS and leave in 16-byte pieces along the pairs' rows.
-  constexpr int kRows = PRODUCT == kMoeGated ? 32 : 64;           // output features of a wavefront
-  constexpr int kPitch = 64 * 4 + 16, kValues = PRODUCT == kMoeDown ? 4 : 8, kPieces = kRows / kValues;
-  const int half = lane / 32, j = lane % 32, first = f0 + wave / 2 * kRows;
+  constexpr int kMine = kFeatures / GM;  // output features of a wavefront
+  constexpr int kPitch = 32 * RM * 4 + 16, kValues = PRODUCT == kMoeDown ? 4 : 8, kPieces = kMine / kValues;
+  const int half = lane / 32, j = lane % 32, first = f0 + wave / GN * kMine;
   char* mine = reinterpret_cast<char*>(mem) + wave * 32 * kPitch;
 #pragma unroll
-  for (int jn = 0; jn < 2; ++jn) {
+  for (int jn = 0; jn < RN; ++jn) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < RM; ++i)
 #pragma unroll
       for (int g = 0; g < 4; ++g)
         *reinterpret_cast<f32x4*>(mine + j * kPitch + (i * 32 + g * 8 + half * 4) * 4) =
@@ -696,7 +695,7 @@ __global__ void __launch_bounds__(kBigWaves* kWave) __attribute__((amdgpu_waves_
     SHK_LDS_DONE();
 #pragma unroll 1
     for (int q = lane; q < 32 * kPieces; q += kWave) {
-      const int t = q / kPieces, row = q % kPieces * kValues, at = row0 + (wave % 2 * 2 + jn) * 32 + t, f = first + row;
+      const int t = q / kPieces, row = q % kPieces * kValues, at = row0 + (wave % GN * RN + jn) * 32 + t, f = first + row;
       if (at >= count || f >= m) continue;  // (m is a multiple of 64: a piece is inside or outside as a whole)
       const size_t pair = min(max(list[at], 0), n * top - 1);
       const float* sums = reinterpret_cast<const float*>(mine + t * kPitch);
@@ -718,15 +717,39 @@ __global__ void __launch_bounds__(kBigWaves* kWave) __attribute__((amdgpu_waves_
   }
 }
 
-template <int PRODUCT>
+template <int PRODUCT, int GM, int GN, int RM, int RN>
 static void launch_big(const bf16* a, const int32_t* order, const int32_t* counts, const void* w0, const void* w1, bf16* act_out,
                        float* pair_out, int n, int k, int m, int experts, int top, GateForm form, hipStream_t s) {
-  const long long features = PRODUCT == kMoeGated ? (m + kBigRows / 2 - 1) / (kBigRows / 2) : (m + kBigRows - 1) / kBigRows;
-  const long long pairs = static_cast<long long>(n) * top;
-  const long long tiles = features * (pairs / kBigPairs + (experts < pairs ? experts : pairs));  // live ones at most
-  moe_big_mfma_kernel<PRODUCT><<<static_cast<unsigned>((tiles + 7) / 8 * 8), kBigWaves * kWave, 0, s>>>(
+  constexpr int kPairs = 32 * GN * RN, kFeatures = 32 * GM * RM / (PRODUCT == kMoeGated ? 2 : 1);
+  const long long features = (m + kFeatures - 1) / kFeatures, pairs = static_cast<long long>(n) * top;
+  const long long tiles = features * (pairs / kPairs + (experts < pairs ? experts : pairs));  // live ones at most
+  moe_big_mfma_kernel<PRODUCT, GM, GN, RM, RN><<<static_cast<unsigned>((tiles + 7) / 8 * 8), GM * GN * kWave, 0, s>>>(
       a, order, counts, static_cast<const bf16*>(w0), static_cast<const bf16*>(w1), act_out, pair_out, n, k, m, experts, top,
       form);
+}
+
+// A product per expert in the tile that wide_time() expects to be done first, as far as that can be known here: every
+// list ends in half a tile, and `identity` of the router's outputs take their share of the pairs.  (Which tile makes no
+// difference to the sums.)  A lane's values of the activation take 0.12 us each.  8 experts of 3584 x 4736, 1,501 tokens
+// of two choices in 256 x 128, 256 x 192, 128 x 192: gate and up 232 / 254 / 260 us, down 142 / 105 / 122.
+template <int PRODUCT>
+static void big_product(const bf16* a, const int32_t* order, const int32_t* counts, const void* w0, const void* w1, bf16* act_out,
+                        float* pair_out, int n, int k, int m, int experts, int identity, int top, GateForm form, hipStream_t s) {
+  const double pairs = static_cast<double>(n) * top * experts / (experts + identity);
+  const int rows = PRODUCT == kMoeGated ? 2 * m : m;
+  constexpr int kTried[] = {4, 1, 6};  // 256 x 128, 256 x 192, 128 x 192
+  int best = 0;
+  double least = 0.0;
+  for (int i = 0; i < 3; ++i) {
+    WideTile t = kWide[kTried[i]];
+    if (PRODUCT != kMoeDown) t.ends += 0.12 * (PRODUCT == kMoeGated ? t.rows / 2 : t.rows) * t.tokens / (i ? 256 : 512);
+    const double us = wide_time(t, ((rows + t.rows - 1) / t.rows) * (pairs / t.tokens + 0.5 * (experts < pairs ? experts : pairs)), k / 64);
+    if (!i || us < least) least = us, best = i;
+  }
+  const auto launch = best == 0   ? launch_big<PRODUCT, 4, 2, 2, 2>
+                      : best == 1 ? launch_big<PRODUCT, 2, 2, 4, 3>
+                                  : launch_big<PRODUCT, 2, 2, 2, 3>;
+  launch(a, order, counts, w0, w1, act_out, pair_out, n, k, m, experts, top, form, s);
 }
 
 // Whether lists of 64 pairs and more keep moe_big_mfma_kernel's few, long workgroups busy for longer than they take to start and end,
@@ -909,10 +932,10 @@ extern "C" int shk_moe_experts_grouped(const void* x, const int32_t* chosen, con
                     static_cast<long long>(width) * ff < (1LL << 31);
   if (many && tiled && near && fills_long_lists(n, top, width, ff, experts, w_gate == w_up)) {
     if (w_gate == w_up)
-      launch_big<kMoeSingle>(xb, order, counts, w_gate, w_up, static_cast<bf16*>(act_buf), nullptr, n, width, ff, experts, top, form, s);
+      big_product<kMoeSingle>(xb, order, counts, w_gate, w_up, static_cast<bf16*>(act_buf), nullptr, n, width, ff, experts, identity, top, form, s);
     else
-      launch_big<kMoeGated>(xb, order, counts, w_gate, w_up, static_cast<bf16*>(act_buf), nullptr, n, width, ff, experts, top, form, s);
-    launch_big<kMoeDown>(actb, order, counts, w_down, nullptr, nullptr, pair_out, n, ff, width, experts, top, form, s);
+      big_product<kMoeGated>(xb, order, counts, w_gate, w_up, static_cast<bf16*>(act_buf), nullptr, n, width, ff, experts, identity, top, form, s);
+    big_product<kMoeDown>(actb, order, counts, w_down, nullptr, nullptr, pair_out, n, ff, width, experts, identity, top, form, s);
   } else if (many && !tiled) {
     const int row_tiles = (n + kTileRows - 1) / kTileRows;
     if (w_gate == w_up)
