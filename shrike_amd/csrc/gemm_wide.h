@@ -181,7 +181,10 @@ constexpr int kWideTiles = sizeof(kWide) / sizeof(kWide[0]);
 
 // Microseconds of `groups` workgroups of a tile, each walking `stages` stages of k.
 inline double wide_time(const WideTile& t, double groups, int stages) {
-  const double rounds = static_cast<double>(static_cast<long long>(groups) / t.units), rest = (groups - rounds * t.units) / t.units;
+  const double rounds = static_cast<double>(static_cast<long long>(groups) / t.units);
+  double rest = (groups - rounds * t.units) / t.units;
+  // (two on some compute units take as long as two on all: 296 of 128 x 128 x 3584 at 128 tokens 78 us, 148 of 256 x 128 66)
+  if (t.units > 256 && rest > 0.5) rest = 1.0;
   double us = 2.0 + rounds * (t.ends + stages * (t.alone + t.full));
   if (rest > 0.0) us += t.ends + stages * (t.alone + t.full * rest);
   return us;
