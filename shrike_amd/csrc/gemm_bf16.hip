@@ -1063,25 +1063,24 @@ extern "C" int shk_gemm_bf16_splits(int n, int m, int k);
 // Which gemm_direct_kernel serves a product of n > 16 tokens (0: none): the smallest tile of which a launch has no
 // more than the 256 compute units, for matrices of 256 to 2,048 rows (more of them fill the staged kernels' larger
 // tiles), up to 10 MB and rows that are whole 16-byte pieces; in shares of k up to 64 tokens.  Against the staged kernels,
-// product and reading norm, over ten widths of 256 to 2,048, k from 128 to 14,336 and 17 to 4,096 tokens: 0.36 to 1.0 of
-// their time with up to 8,192 of k in the two smaller tiles (to 1.4 beyond), up to 2,048 in the two larger ones (k = 4864 at 300
-// tokens 23.5 us against 20.7).  64 x 64 with two workgroups a unit 0.81 to 1.0 up to k = 512, up to 352 of them 0.88 to
-// 1.0 up to k = 1024; beyond, 1024 x 2048 at 1,119 tokens 30 us against 27, 512 x 1024 at 4,096 30.3 against 26.5.
+// product and reading norm, over six widths of 256 to 2,048, k from 128 to 8,192 and 65 to 4,096 tokens: 0.65 to 0.98 of
+// their time with up to 2,048 of k in the two smaller tiles, 0.93 to 1.24 up to 4,864, 1.16 to 1.63 with 8,192; the largest
+// tile 0.91 to 1.0 up to 896 of k and 1.08 to 1.3 from 1,024 on.  (64 x 64 tiles took 1.14 to 1.5 of the staged kernels' time.)
 struct DirectTile {
   int rows, tokens, most_k, waves;
 };
-static const DirectTile kDirect[5] = {{0, 0, 0, 0}, {32, 16, 8192, 8}, {32, 32, 8192, 4}, {32, 64, 2048, 8}, {64, 64, 2048, 4}};
+static const DirectTile kDirect[4] = {{0, 0, 0, 0}, {32, 16, 8192, 8}, {32, 32, 8192, 4}, {32, 64, 960, 8}};
 
 static int direct_shape(int n, int m, int k, int ksplit) {
   if (n <= 16 || (n > 64 && ksplit > 1) || m < 256 || m > 2048 || k % 8 || static_cast<long long>(m) * k > 5 * 1000 * 1000)
     return 0;
   const int tokens = counted_tokens(n);
-  for (int shape = 1; shape <= (ksplit > 1 ? 2 : 4); ++shape) {
+  for (int shape = 1; shape <= (ksplit > 1 ? 2 : 3); ++shape) {
     const DirectTile& t = kDirect[shape];
     long long count = static_cast<long long>((m + t.rows - 1) / t.rows) * ((tokens + t.tokens - 1) / t.tokens);
     if (ksplit > 1) count = (count + kDies - 1) / kDies * kDies;  // (as launched)
-    const int most = shape < 4 || k > 1024 ? 256 : k > 512 ? 352 : 512;
-    if (k / ksplit <= t.most_k && count * ksplit <= most) return shape;
+    const int most_k = n > 64 && t.most_k > 4864 ? 4864 : t.most_k;
+    if (k / ksplit <= most_k && count * ksplit <= 256) return shape;
   }
   return 0;
 }
@@ -1263,8 +1262,7 @@ extern "C" int shk_gemm_bf16_tiled_weight(const void* a, const void* wt, const f
   if (direct) {
     const auto go = direct == 1   ? launch_direct<2, 1, 8, 2>
                     : direct == 2 ? launch_direct<2, 2, 4, 2>
-                    : direct == 3 ? launch_direct<2, 4, 8, 1>
-                                  : launch_direct<4, 4, 4, 1>;
+                                  : launch_direct<2, 4, 8, 1>;
     go(s, ap, lda, n, k, wp, kt, m, bias, out, ldo, of, accumulate, ksplit);
     SHK_LAUNCH_CHECK("gemm_bf16");
     return 0;
