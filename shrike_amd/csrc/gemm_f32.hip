@@ -19,13 +19,13 @@
 // then one run of 1 KiB instead of 16 pieces of 64 bytes (four rows of a 9728 x 896 matrix 10.7 us
 // against 14, of 896 x 4864 13 against 18).  Operands of other callers are row-major.
 // What bounds it: with few rows the latency of one round of loads and a reduction through LDS; with
-// many the supply of operands and the last round of workgroups, which leave half of the matrix instruction's rate
-// (150 TFLOP/s alone; 9728 x 896 at 509 rows 75): a workgroup's wavefronts walk different parts of k and so share no operand,
-// and loads are one step ahead.  At the full rate that would be 38 GB/s a compute unit, about what one takes in.  Before, one workgroup per 64 x 64 results with vector
+// many the supply of operands: a workgroup's wavefronts walk different parts of k and so share no operand (9728 x 896 at 509
+// rows 75 TFLOP/s; gemm_f32_lds_kernel, which shares them, 97).  Before, one workgroup per 64 x 64 results with vector
 // instructions: a 0.5B decode step of four requests 23.9 ms (2.4 with this kernel, 1.56 with attention_f32.hip as
-// well), a 509-token prompt 42.6 ms (18.9, 6.5); the logits' error against 64 bits 6.4e-7 (2.5e-7).
+// well), a 509-token prompt 42.6 ms (18.9, 6.5; 5.4 with operands shared); the logits' error against 64 bits 6.4e-7 (2.5e-7).
 #include "api.h"
 #include "common.h"
+#include "gemm_wide.h"
 
 namespace shk {
 
@@ -212,6 +212,137 @@ __global__ void __launch_bounds__(kWave * KW * MW * NW)
   }
 }
 
+// The same product, in the same order, for many rows and more than 256 of k in whole stages of 32: four wavefronts, 2 x 2 of
+// RT x CT tiles, share their operands through LDS, loaded straight into it two stages ahead.  A wavefront walks all of
+// k, the tiles' sums of segment, group and all in its registers.  The operands of an instruction's 32 cycles are then a
+// quarter of what they are where every wavefront walks a part of k of its own and none shares with another.
+// Eight lanes load a row's 128 bytes of a stage, piece c at place c ^ (row / 2 % 8): the 16 lanes that read one piece of 16
+// rows meet no bank conflicts.
+// What bounds it: the matrix units where workgroups fill the chip several times (3584 x 3584 at 1,501 rows 119 TFLOP/s of
+// the 150 that the instruction reaches alone, 9728 x 896 at 509 97).  64 x 64, 128 x 64 and 128 x 128 results a workgroup
+// were 4 % slower to twice as slow: fewer wavefronts to cover each other's barriers.
+template <int RT, int CT>
+__global__ void __launch_bounds__(4 * kWave)
+    gemm_f32_lds_kernel(const float* __restrict__ a, const float* __restrict__ w, const float* __restrict__ bias,
+                        float* __restrict__ out, int n, int m, int k, int lda, int ldo, int accumulate, int vec_out) {
+  constexpr int kRing = 3, kW = 4 * RT, kA = 4 * CT;  // stages; KiB of a stage's weights and rows
+  __shared__ mf4 mem[kRing * (kW + kA)][kWave];
+  const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int mw = wave / 2, nw = wave % 2, i = lane % 16, kg = lane / 16;
+  // workgroup -> tile as in gemm_f32_kernel
+  const int rows = (n + 32 * CT - 1) / (32 * CT), cols = (m + 32 * RT - 1) / (32 * RT);
+  const int per_die = (rows * cols + kDies - 1) / kDies;
+  const int tile = blockIdx.x % kDies * per_die + blockIdx.x / kDies;
+  if (blockIdx.x / kDies >= per_die || tile >= rows * cols) return;
+  const int f0 = tile / rows * 2 * RT, t0 = tile % rows * 32 * CT;  // first block of 16 features, first row
+  const int ktiles = k / 16, stages = k / 32, blocks = (m + 15) / 16;
+
+  // what a wavefront loads: units wave, wave + 4, ..; rows beyond the last are read as the last and not stored
+  unsigned woff[RT], aoff[CT];
+#pragma unroll
+  for (int u = 0; u < RT; ++u) {
+    const int unit = wave + 4 * u, block = min(f0 + unit / 2, blocks - 1) - f0;
+    woff[u] = (static_cast<unsigned>(block) * ktiles + unit % 2) * 1024u + lane * 16u;
+  }
+#pragma unroll
+  for (int u = 0; u < CT; ++u)
+    aoff[u] = static_cast<unsigned>(min(t0 + (wave + 4 * u) * 8 + lane / 8, n - 1) - t0) * lda * 4u + ((lane % 8) ^ (wave % 2 * 4 + lane / 16)) * 16u;
+  const char* wsrc = reinterpret_cast<const char*>(w) + static_cast<size_t>(f0) * ktiles * 1024;
+  const char* asrc = reinterpret_cast<const char*>(a) + static_cast<size_t>(t0) * lda * 4;
+  const unsigned base =
+      static_cast<unsigned>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)&mem[0][0])) + wave * 1024;
+  auto load = [&](int slot, int stage) {
+    const int st = stage < stages ? stage : 0;  // past the end: stage 0 again, never multiplied
+#pragma unroll
+    for (int u = 0; u < RT; ++u) load_to_lds(base + (slot * (kW + kA) + 4 * u) * 1024, woff[u], wsrc + static_cast<size_t>(st) * 2048);
+#pragma unroll
+    for (int u = 0; u < CT; ++u) load_to_lds(base + (slot * (kW + kA) + kW + 4 * u) * 1024, aoff[u], asrc + static_cast<size_t>(st) * 128);
+  };
+
+  mf4 acc[RT][CT], group[RT][CT], total[RT][CT];
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int c = 0; c < CT; ++c) acc[r][c] = group[r][c] = total[r][c] = mf4{0.f, 0.f, 0.f, 0.f};
+  const int seg_steps = (k + 16 * kF32Segments - 1) / (16 * kF32Segments);
+  int in_seg = 0, in_group = 0;
+  load(0, 0);
+  load(1, 1);
+  int slot = 0;
+  for (int st = 0; st < stages; ++st) {
+    SHK_MEET_WITH_LOADS(RT + CT);
+    load(slot ? slot - 1 : kRing - 1, st + 2);
+    const mf4(*now)[kWave] = mem + slot * (kW + kA);
+    mf4 wv[2][RT], av[2][CT];
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+#pragma unroll
+      for (int r = 0; r < RT; ++r) wv[half][r] = now[(mw * RT + r) * 2 + half][lane];
+#pragma unroll
+      for (int c = 0; c < CT; ++c)  // row i of 16: unit i / 8, its row i % 8
+        av[half][c] = now[kW + (nw * CT + c) * 2 + i / 8][i % 8 * 8 + ((half * 4 + kg) ^ (i / 2))];
+    }
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+#pragma unroll
+          for (int c = 0; c < CT; ++c)
+            acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[half][r][j], av[half][c][j], acc[r][c], 0, 0, 0);
+      if (++in_seg == seg_steps) {  // a segment ends
+        in_seg = 0;
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+#pragma unroll
+          for (int c = 0; c < CT; ++c) {
+            group[r][c] += acc[r][c];
+            acc[r][c] = mf4{0.f, 0.f, 0.f, 0.f};
+          }
+        if (++in_group == kF32Group) {
+          in_group = 0;
+#pragma unroll
+          for (int r = 0; r < RT; ++r)
+#pragma unroll
+            for (int c = 0; c < CT; ++c) {
+              total[r][c] += group[r][c];
+              group[r][c] = mf4{0.f, 0.f, 0.f, 0.f};
+            }
+        }
+      }
+    }
+    slot = slot + 1 < kRing ? slot + 1 : 0;
+  }
+  SHK_WAIT_LOADS(0);  // no load may arrive in LDS that the workgroup has given back
+
+#pragma unroll
+  for (int c = 0; c < CT; ++c) {
+    const int row = t0 + (nw * CT + c) * 16 + i;  // the matrix instruction's columns
+    if (row >= n) continue;
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+      const int col = (f0 + mw * RT + r) * 16 + kg * 4;
+      mf4 v = total[r][c] + (group[r][c] + acc[r][c]);
+      float* dst = out + static_cast<size_t>(row) * ldo + col;
+      if (vec_out && col + 3 < m) {
+        if (bias) v += mf4{bias[col], bias[col + 1], bias[col + 2], bias[col + 3]};
+        if (accumulate) v += *reinterpret_cast<const mf4*>(dst);
+        *reinterpret_cast<mf4*>(dst) = v;
+        continue;
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (col + e >= m) continue;
+        float x = v[e];
+        if (bias) x += bias[col + e];
+        if (accumulate) x += dst[e];
+        dst[e] = x;
+      }
+    }
+  }
+}
+
 struct F32Product {
   const float *a, *w, *bias;
   float* out;
@@ -240,14 +371,30 @@ static void launch_f32(const F32Product& p, hipStream_t s) {
 //     1024 rows 5.7 / 7.3 / 17 / 26 (16 x 16, 32 x 16, 32 x 64, 64 x 64), 9728 x 896 at 64 / 509 25 / 124
 //     (32 x 32, 64 x 64: 70 TFLOP/s of the 150 that the instruction reaches alone).  A k of up to 256 is one step
 //     a segment, and a shorter one leaves the later of four groups without any: there a wavefront walks all of k and
-//     four lie side by side along the rows.  1,501 rows: 28 products of 448 x 128 160 us shared by four groups, 77 so
+//     four lie side by side along the rows.
+//   tiled weights of a k in whole stages, enough of them: gemm_f32_lds_kernel with 32 features x 64 rows, or 32 x 32 where those
+//     are few and k is short.  9728 x 896 at 64 / 200 / 509 / 1,024 rows 18.8 / 45.7 / 91.8 / 163 (24 / 62.6 / 120.6 / 229.5
+//     without it), 1152 x 896 at 509 / 2,000 18.7 / 43.9 (23.7 / 63.1), 3584 x 3584 at 1,501 325 (414), 896 x 4864 at 1,024 97.7
+//     (100.8), but at 509 (224 workgroups of 32 x 64) 61 against 57, 1152 x 896 at 200 (252 of 32 x 32) 10.7 against 9.3.
+//    1,501 rows: 28 products of 448 x 128 160 us shared by four groups, 77 so
 //     (95 with vector instructions), 14 of 128 x 64 27, 13 (14), 40 of 256 x 192 132, 86 (105), 4864 x 256 73, 55 (66).
+template <int RT, int CT>
+static void launch_f32_lds(const F32Product& p, hipStream_t s) {
+  const int tiles = (p.m + 32 * RT - 1) / (32 * RT) * ((p.n + 32 * CT - 1) / (32 * CT));
+  const int vec_out = p.ldo % 4 == 0 && reinterpret_cast<uintptr_t>(p.out) % 16 == 0;
+  gemm_f32_lds_kernel<RT, CT><<<(tiles + kDies - 1) / kDies * kDies, 4 * kWave, 0, s>>>(p.a, p.w, p.bias, p.out, p.n, p.m, p.k, p.lda,
+                                                                                    p.ldo, p.accumulate, vec_out);
+}
+
 template <bool TILED>
 static void run_f32(const F32Product& p, hipStream_t s) {
   auto tiles = [&](int rows, int cols) {
     return static_cast<long long>((p.m + rows - 1) / rows) * ((p.n + cols - 1) / cols) * p.batch;
   };
   auto one_round = [](long long count) { return count >= 192 && count <= 256; };
+  // whole stages of aligned rows, offsets within a tile of 32 bits
+  const bool staged = TILED && p.batch == 1 && p.k % 32 == 0 && p.k > 256 && p.k <= 1 << 20 && p.lda % 4 == 0 && p.lda <= 1 << 20 &&
+                      reinterpret_cast<uintptr_t>(p.a) % 16 == 0;
   if (p.n <= 16) {
     if (p.m <= 2048)
       launch_f32<1, 1, 16, 1, 1, 2, TILED>(p, s);
@@ -255,6 +402,10 @@ static void run_f32(const F32Product& p, hipStream_t s) {
       launch_f32<1, 1, 4, 4, 1, 4, TILED>(p, s);
     else
       launch_f32<2, 1, 4, 4, 1, 2, TILED>(p, s);
+  } else if (staged && (tiles(32, 64) >= 1536 || (p.k > 1024 && tiles(32, 64) >= 440))) {
+    launch_f32_lds<1, 2>(p, s);
+  } else if (staged && p.k <= 1024 && tiles(32, 32) > kDies * 32) {
+    launch_f32_lds<1, 1>(p, s);
   } else if (tiles(64, 64) >= 640 || one_round(tiles(64, 64))) {
     if (p.k <= 256)
       launch_f32<4, 2, 1, 1, 4, 1, TILED>(p, s);
