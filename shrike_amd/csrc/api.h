@@ -249,6 +249,7 @@ int shk_attention_prefill_bf16(const void* q, int q_stride, void* out, int num_t
 // first_token: the index of the step's first prompt token (prompt tokens follow
 // the single tokens); prompt_tokens: how many there are.
 int shk_attention_prefill_shared_tiles(int heads, int kv_heads, int head_dim, int small);
+int shk_attention_prefill_rows_queries(int heads, int kv_heads, int head_dim);
 int shk_attention_prefill_shared_bf16(const void* q, int q_stride, void* out, int num_wgs,
                                       int heads, int kv_heads, int head_dim, const int32_t* cu_q,
                                       const int32_t* ctx_lens, const int32_t* wg_seq,

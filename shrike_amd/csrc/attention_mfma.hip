@@ -19,6 +19,7 @@
 // multiples of 16; up to 16 query heads per key/value head.  Other shapes are
 // served by the general kernel.
 #include "api.h"
+#include "attention_rows.h"
 #include "common.h"
 #include "mfma_tile.h"
 
@@ -1138,6 +1139,13 @@ extern "C" int shk_attention_prefill_shared_tiles(int heads, int kv_heads, int h
   return units / group;
 }
 
+// Queries that one workgroup of attention_rows_kernel (small == 2) serves; 0: not served.  Groups of fewer than four heads
+// would make runs of 128 queries and more, which is coarse for causal prompts.
+extern "C" int shk_attention_prefill_rows_queries(int heads, int kv_heads, int head_dim) {
+  const int group = heads / kv_heads;
+  return group >= 4 && group <= kAttentionRows && (head_dim == 64 || head_dim == 128) ? kAttentionRows / group : 0;
+}
+
 extern "C" int shk_attention_prefill_shared_bf16(const void* q, int q_stride, void* out,
                                                  int num_wgs, int heads, int kv_heads,
                                                  int head_dim, const int32_t* cu_q,
@@ -1155,7 +1163,9 @@ extern "C" int shk_attention_prefill_shared_bf16(const void* q, int q_stride, vo
   const ScoreOpts so = score_opts(scale, softcap, sinks, dist_bias, bias_rows);
   if (check_mfma_shapes("attention_prefill_shared", heads, kv_heads, head_dim, page_size, q_stride))
     return 1;
-  const int tiles = shk_attention_prefill_shared_tiles(heads, kv_heads, head_dim, small);
+  const int tiles = small == 2 ? shk_attention_prefill_rows_queries(heads, kv_heads, head_dim)
+                               : shk_attention_prefill_shared_tiles(heads, kv_heads, head_dim, small);
+  SHK_REQUIRE(small != 2 || (softcap == 0.f && !dist_bias), "attention_prefill_shared: rows of 32 take no score cap and no distance bias");
   SHK_REQUIRE(tiles > 0, "attention_prefill_shared: %d query heads per key/value head or head_dim %d "
               "is not served", heads / kv_heads, head_dim);
   SHK_REQUIRE(nsplit >= 1 && nsplit <= kMaxSplits, "attention_prefill_shared: %d key splits (at most %d)",
@@ -1178,6 +1188,19 @@ extern "C" int shk_attention_prefill_shared_bf16(const void* q, int q_stride, vo
               table_stride, page_size);
   hipStream_t s = static_cast<hipStream_t>(stream);
   dim3 grid(num_wgs * kv_heads * nsplit);
+  if (small == 2) {
+    const int rows = prompt_tokens * heads;
+    bf16* dst = static_cast<bf16*>(out);
+    launch_attention_rows(head_dim, grid.x, s, static_cast<const bf16*>(q), q_stride, dst, heads, kv_heads, tiles, cu_q, ctx_lens, wg_seq,
+                          wg_q0, tables, table_stride, static_cast<const bf16*>(k_pool), static_cast<const bf16*>(v_pool), page_size,
+                          window, block, scale, partial, nsplit, first_token, rows, sinks);
+    if (nsplit > 1) {
+      auto merge = head_dim == 64 ? attention_merge_kernel<64> : attention_merge_kernel<128>;
+      merge<<<rows, kWave, 0, s>>>(partial, dst + static_cast<size_t>(first_token) * heads * head_dim, nsplit, sinks, heads);
+    }
+    SHK_LAUNCH_CHECK("attention_prefill_shared");
+    return 0;
+  }
 #define CALL(D)                                                                                \
   launch_prefill_shared<D>(grid, s, static_cast<const bf16*>(q), q_stride, static_cast<bf16*>(out), \
                            heads, kv_heads, tiles, cu_q, ctx_lens, wg_seq, wg_q0, tables,      \

@@ -105,6 +105,7 @@ _SIGNATURES = {
                                   _P, _I, _P],
     "shk_attention_prefill_bf16": [_P, _I, _P, _I, _I, _I, _I, _P, _P, _P, _P, _P, _I, _P, _P, _I, _I, _I, _F, _P],
     "shk_attention_prefill_shared_tiles": [_I, _I, _I, _I],
+    "shk_attention_prefill_rows_queries": [_I, _I, _I],
     "shk_attention_prefill_shared_bf16": [_P, _I, _P, _I, _I, _I, _I, _P, _P, _P, _P, _P, _I, _P, _P, _I, _I, _I, _F,
                                           _I, _P, _I, _I, _I, _F, _P, _P, _I, _P],
     "shk_argmax": [_P, _P, _I, _I, _I, _P, _P],

@@ -1420,6 +1420,11 @@ def attention_prefill_shared_tiles(heads, kv_heads, head_dim, small=False) -> in
     return int(load().shk_attention_prefill_shared_tiles(heads, kv_heads, head_dim, int(small)))
 
 
+def attention_prefill_rows_queries(heads, kv_heads, head_dim) -> int:
+    """Queries per workgroup of attention_prefill_shared(..., small=2); 0 if the shape is not served."""
+    return int(load().shk_attention_prefill_rows_queries(heads, kv_heads, head_dim))
+
+
 def attention_prefill_shared(q, out, num_wgs, heads, kv_heads, head_dim, cu_q, ctx_lens, wg_seq, wg_q0,
                              tables, k_pool, v_pool, page_size, window, scale, small=False,
                              partial=None, nsplit: int = 1, first_token: int = 0, chunk=None, softcap=None,
@@ -1427,7 +1432,8 @@ def attention_prefill_shared(q, out, num_wgs, heads, kv_heads, head_dim, cu_q, c
     """bfloat16 MFMA attention for prompt portions; one workgroup per (run of query
     tiles, key/value head) shares each chunk of keys among its query heads.
     wg_seq / wg_q0 are in steps of 16 * attention_prefill_shared_tiles(..., small),
-    launched in the list's order.  nsplit > 1 shares every entry's keys among
+    launched in the list's order.  small=2: the kernel with 32 rows a wavefront, in steps of
+    attention_prefill_rows_queries (no score cap, no distance bias).  nsplit > 1 shares every entry's keys among
     that many workgroups, whose results pass through `partial` (float32, (rows
     of q from first_token on) * heads * nsplit * (head_dim + 2) values)."""
     _rows(q, "attention_prefill_shared q")

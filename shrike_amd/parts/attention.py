@@ -135,7 +135,7 @@ class AttentionPlan:
     blocks_apart: bool = False  # float32: workgroups of their own for a single token's blocks of keys
     streaming: bool = False  # single-token rows: non-temporal loads of keys and values
     kernel: str = ""  # for prompt portions: "shared", "tiles" or "" (none in the step)
-    small: bool = False  # "shared" with half as many wavefronts per workgroup
+    small: int = 0  # "shared" with half as many wavefronts per workgroup (1), with 32 rows a wavefront (2)
     portion_splits: int = 1  # "shared": workgroups that share an entry's keys
     first_token: int = 0  # index of the step's first prompt token
     count: int = 0  # workgroups ("shared") or tiles ("tiles")
@@ -166,6 +166,18 @@ def portion_splits(workgroups: int, mean_keys: int) -> int:
     if workgroups <= 0:
         return 1
     return max(1, min(2 * compute_units() // workgroups, mean_keys // KEYS_PER_WORKGROUP, MAX_KEY_SPLITS))
+
+
+# Keys that a query reads on average from which the prompt kernel with 32 rows a wavefront is the faster one, if its workgroups
+# have most compute units to do: 28 heads over 4, 512 queries at 12,001 167 us -> 137, at 1,536 42 -> 41, at 0 21 -> 26; 500 at
+# 6,000 beside 300 at 3,000 (184 workgroups) 117 -> 123.
+ROWS_FROM_KEYS = 1800
+
+
+def portion_mean_keys(q_lens, starts, reach: int) -> float:
+    """Keys that a query of the step's prompt portions reads on average, at most `reach` each."""
+    keys = np.minimum(np.asarray(starts, dtype=np.int64) + np.asarray(q_lens, dtype=np.int64) / 2.0, float(reach))
+    return float((keys * q_lens).sum() / max(1, int(np.sum(q_lens))))
 
 
 def heavy_first(work):
@@ -441,8 +453,23 @@ class PagedAttention(Mixer):
         portions = shape.q_lens[shape.num_decode:]
         if portions.size == 0:
             return
+        rows = 0 if getattr(s, "softcap", None) or self.dist_bias is not None else ops.attention_prefill_rows_queries(h, hkv, d)
+        if rows:
+            seqs, q0 = portion_runs(portions, shape.num_decode, rows)
+            keys = np.minimum(shape.starts[seqs] + q0 + rows, reach + rows)
+            count = int(seqs.size) * hkv
+            splits = portion_splits(2 * count, int(keys.mean()))  # (one workgroup on a compute unit)
+            # enough keys for a query, and workgroups for most compute units
+            if (portion_mean_keys(portions, shape.starts[shape.num_decode:], reach) < ROWS_FROM_KEYS
+                    or 4 * count * splits < 3 * compute_units()):
+                rows = 0
         tiles = ops.attention_prefill_shared_tiles(h, hkv, d)
-        if tiles:
+        if rows:
+            plan.kernel, plan.small, plan.portion_splits = "shared", 2, splits
+            order = heavy_first(keys)
+            seqs, q0 = seqs[order], q0[order]
+            plan.first_token = shape.num_decode
+        elif tiles:
             plan.kernel = "shared"
             small_tiles = ops.attention_prefill_shared_tiles(h, hkv, d, small=True)
             if small_tiles:
@@ -454,7 +481,7 @@ class PagedAttention(Mixer):
                 small_count = int((-(-portions // (QUERY_TILE * small_tiles))).sum())
                 # (two workgroups of 8 wavefronts fit on a compute unit)
                 if small_count * hkv <= 2 * compute_units():
-                    plan.small, tiles = True, small_tiles
+                    plan.small, tiles = 1, small_tiles
             seqs, q0 = portion_runs(portions, shape.num_decode, QUERY_TILE * tiles)
             # the keys an entry's last query reads: where its portion starts plus its queries
             keys = shape.starts[seqs] + q0 + QUERY_TILE * tiles
