@@ -240,7 +240,9 @@ int shk_attention_prefill_bf16(const void* q, int q_stride, void* out, int num_t
 // one sequence (wg_seq, wg_q0 in steps of 16 * tiles) and stages each chunk of
 // keys once in LDS.  small != 0: workgroups of 8 wavefronts instead of 16, with
 // half as many tiles each, for portions that would otherwise make too few
-// workgroups for the chip.  tiles == 0: the shape is not served (more query
+// workgroups for the chip.  small == 2: attention_rows.hip, a workgroup for
+// shk_attention_prefill_rows_queries(...) consecutive queries (wg_q0 in steps of that; 0:
+// not served), without a score cap or distance bias.  tiles == 0: the shape is not served (more query
 // heads per key/value head than a workgroup has wavefronts, head_dim > 128).
 // Entries are launched in the order of the list.  nsplit > 1 shares every entry's
 // keys among nsplit workgroups (for a few queries far into a sequence, which alone

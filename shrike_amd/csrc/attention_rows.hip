@@ -124,12 +124,12 @@ __global__ void __launch_bounds__(8 * kWave) __attribute__((amdgpu_waves_per_eu(
   auto load_k = [&](int slot, Group g) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < kLoads; ++i)
-      load_to_lds(base + slot * kBytes + (wave * kLoads + i) * 1024, koff[i], reinterpret_cast<const char*>(k_pool) + g.at + g.slot * 64);
+      SHK_LOAD_TO_LDS(base + slot * kBytes + (wave * kLoads + i) * 1024, koff[i], reinterpret_cast<const char*>(k_pool) + g.at + g.slot * 64);
   };
   auto load_v = [&](int slot, Group g) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < kLoads; ++i)
-      load_to_lds(base + (kRing + slot) * kBytes + (wave * kLoads + i) * 1024, voff[i], reinterpret_cast<const char*>(v_pool) + g.at + g.slot * 2);
+      SHK_LOAD_TO_LDS(base + (kRing + slot) * kBytes + (wave * kLoads + i) * 1024, voff[i], reinterpret_cast<const char*>(v_pool) + g.at + g.slot * 2);
   };
 
   // ---- where this lane's operands lie

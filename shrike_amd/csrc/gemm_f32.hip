@@ -254,9 +254,9 @@ __global__ void __launch_bounds__(4 * kWave)
   auto load = [&](int slot, int stage) {
     const int st = stage < stages ? stage : 0;  // past the end: stage 0 again, never multiplied
 #pragma unroll
-    for (int u = 0; u < RT; ++u) load_to_lds(base + (slot * (kW + kA) + 4 * u) * 1024, woff[u], wsrc + static_cast<size_t>(st) * 2048);
+    for (int u = 0; u < RT; ++u) SHK_LOAD_TO_LDS(base + (slot * (kW + kA) + 4 * u) * 1024, woff[u], wsrc + static_cast<size_t>(st) * 2048);
 #pragma unroll
-    for (int u = 0; u < CT; ++u) load_to_lds(base + (slot * (kW + kA) + kW + 4 * u) * 1024, aoff[u], asrc + static_cast<size_t>(st) * 128);
+    for (int u = 0; u < CT; ++u) SHK_LOAD_TO_LDS(base + (slot * (kW + kA) + kW + 4 * u) * 1024, aoff[u], asrc + static_cast<size_t>(st) * 128);
   };
 
   mf4 acc[RT][CT], group[RT][CT], total[RT][CT];

@@ -30,12 +30,6 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 
-// 16 bytes a lane from base + offset into LDS at `lds` + 16 * lane.  Not the builtin: for that the compiler
-// waits, before a read of LDS, for loads into any part of the same array.  The kernel waits by itself.
-__device__ __forceinline__ void load_to_lds(unsigned lds, unsigned offset, const char* base) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(offset), "s"(base) : "memory");
-}
-
 template <int GM, int GN, int RM, int RN>
 struct WideShape {
   static constexpr int kWaves = GM * GN;
@@ -70,12 +64,12 @@ __device__ __forceinline__ void wide_loop(f32x16 (&acc)[RM][RN], u32x4* mem, con
 
   // (past the share's end: substep or stage 0 again, never multiplied)
   auto load_w = [&](int at, int sub, int i) {
-    load_to_lds(base + at + i * S::kWaves * 1024, woff[i], wsrc + static_cast<size_t>(sub < subs ? sub : 0) * 1024);
+    SHK_LOAD_TO_LDS(base + at + i * S::kWaves * 1024, woff[i], wsrc + static_cast<size_t>(sub < subs ? sub : 0) * 1024);
   };
   auto load_x = [&](int at, int st, int half, int i) {
     st = st < stages ? st : 0;
     const unsigned cut = st == last ? ~0u : 0u;
-    load_to_lds(base + kX0 + at + (half * XL + i) * S::kWaves * 1024, xoff[half * XL + i] - (beyond & cut),
+    SHK_LOAD_TO_LDS(base + kX0 + at + (half * XL + i) * S::kWaves * 1024, xoff[half * XL + i] - (beyond & cut),
                 xsrc + static_cast<size_t>(st) * 128);
   };
 

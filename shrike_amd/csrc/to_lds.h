@@ -3,17 +3,29 @@
 
 #include <hip/hip_runtime.h>
 
-// 16 bytes a lane: lane l's land at l * 16 behind lptr (the same for the whole wavefront)
-#define SHK_LOAD_TO_LDS(gptr, lptr)                                                                        \
+// SHK_LOAD_TO_LDS(gptr, lptr): 16 bytes a lane: lane l's land at l * 16 behind lptr (the same for the whole wavefront)
+#define SHK_LOAD_TO_LDS_PTR(gptr, lptr)                                                                    \
   __builtin_amdgcn_global_load_lds(                                                                       \
       reinterpret_cast<const __attribute__((address_space(1))) void*>(reinterpret_cast<uintptr_t>(gptr)), \
       (__attribute__((address_space(3))) void*)(lptr), 16, 0, 0)
+
+// SHK_LOAD_TO_LDS(lds, offset, base): the same from base + offset to the byte `lds` of LDS.  Not the builtin: for that the
+// compiler waits, before a read of LDS, for loads into any part of the same array; here the kernel waits by itself.
+#define SHK_LOAD_TO_LDS_AT(lds, offset, base) shk::load_to_lds(lds, offset, base)
+
+#define SHK_LOAD_TO_LDS_PICK(a, b, c, name, ...) name
+#define SHK_LOAD_TO_LDS(...) \
+  SHK_LOAD_TO_LDS_PICK(__VA_ARGS__, SHK_LOAD_TO_LDS_AT, SHK_LOAD_TO_LDS_PTR, )(__VA_ARGS__)
 
 namespace shk {
 
 // s_waitcnt's operand (gfx9 encoding): vmcnt in bits 3:0 and 15:14, expcnt in 6:4, lgkmcnt in 11:8; a counter at
 // its maximum is not waited for.
 constexpr int wait_counts(int vmcnt, int lgkmcnt) { return (vmcnt & 15) | (vmcnt >> 4) << 14 | 7 << 4 | lgkmcnt << 8; }
+
+__device__ __forceinline__ void load_to_lds(unsigned lds, unsigned offset, const char* base) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(offset), "s"(base) : "memory");
+}
 
 }  // namespace shk
 
