@@ -453,15 +453,17 @@ class PagedAttention(Mixer):
         portions = shape.q_lens[shape.num_decode:]
         if portions.size == 0:
             return
-        rows = 0 if getattr(s, "softcap", None) or self.dist_bias is not None else ops.attention_prefill_rows_queries(h, hkv, d)
+        # enough keys for a query, and workgroups for most compute units (a prompt too short for it is not looked at further)
+        rows, starts = 0, shape.starts[shape.num_decode:]
+        if ((starts + portions).max() >= ROWS_FROM_KEYS and portion_mean_keys(portions, starts, reach) >= ROWS_FROM_KEYS
+                and not getattr(s, "softcap", None) and self.dist_bias is None):
+            rows = ops.attention_prefill_rows_queries(h, hkv, d)
         if rows:
             seqs, q0 = portion_runs(portions, shape.num_decode, rows)
             keys = np.minimum(shape.starts[seqs] + q0 + rows, reach + rows)
             count = int(seqs.size) * hkv
             splits = portion_splits(2 * count, int(keys.mean()))  # (one workgroup on a compute unit)
-            # enough keys for a query, and workgroups for most compute units
-            if (portion_mean_keys(portions, shape.starts[shape.num_decode:], reach) < ROWS_FROM_KEYS
-                    or 4 * count * splits < 3 * compute_units()):
+            if 4 * count * splits < 3 * compute_units():
                 rows = 0
         tiles = ops.attention_prefill_shared_tiles(h, hkv, d)
         if rows:
