@@ -70,7 +70,7 @@ __device__ __forceinline__ void wide_loop(f32x16 (&acc)[RM][RN], u32x4* mem, con
     st = st < stages ? st : 0;
     const unsigned cut = st == last ? ~0u : 0u;
     SHK_LOAD_TO_LDS(base + kX0 + at + (half * XL + i) * S::kWaves * 1024, xoff[half * XL + i] - (beyond & cut),
-                xsrc + static_cast<size_t>(st) * 128);
+                    xsrc + static_cast<size_t>(st) * 128);
   };
 
 #pragma unroll
