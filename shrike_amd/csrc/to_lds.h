@@ -23,8 +23,10 @@ namespace shk {
 // its maximum is not waited for.
 constexpr int wait_counts(int vmcnt, int lgkmcnt) { return (vmcnt & 15) | (vmcnt >> 4) << 14 | 7 << 4 | lgkmcnt << 8; }
 
+// (m0, the place in LDS, is an operand: written inside the statement, the builtin's next load would take what it had put
+// there before, and a clobbered reserved register is no promise of the compiler's.  s_nop: m0 may be written right before.)
 __device__ __forceinline__ void load_to_lds(unsigned lds, unsigned offset, const char* base) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(offset), "s"(base) : "memory");
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"{m0}"(lds), "v"(offset), "s"(base) : "memory");
 }
 
 }  // namespace shk

@@ -54,3 +54,38 @@ def test_the_barrier_waits_for_reads_of_lds(tmp_path):
         for i, count in zip(barriers, (n, 0)):
             assert re.fullmatch(rf"s_waitcnt vmcnt\({count}\) lgkmcnt\(0\)", lines[i - 1]), lines[i - 1]
         assert f"s_waitcnt vmcnt({n})" in lines[barriers[1] :]  # (the wait alone leaves reads of LDS in flight)
+
+
+def test_both_forms_of_the_load_in_one_kernel(tmp_path):
+    """Each of three loads (builtin, base + offset, builtin) goes where it should: m0 is written anew before it."""
+    hipcc = find_hipcc()
+    if hipcc is None:
+        pytest.skip("no hipcc")
+    source = tmp_path / "both.hip"
+    source.write_text("""
+        #include "to_lds.h"
+        __global__ void both(float* p) {
+          __shared__ float a[256];
+          const unsigned at = static_cast<unsigned>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)&a[0]));
+          SHK_LOAD_TO_LDS(p + threadIdx.x * 4, a);
+          SHK_LOAD_TO_LDS(at + 512u, threadIdx.x * 16u, reinterpret_cast<const char*>(p + 4096));
+          SHK_LOAD_TO_LDS(p + 8192 + threadIdx.x * 4, a);
+          SHK_MEET_WITH_LOADS(0);
+          p[threadIdx.x] = a[threadIdx.x];
+        }
+    """)
+    out = tmp_path / "both.s"
+    run = subprocess.run([hipcc, *HIPCC_FLAGS, f"-I{CSRC}", "--cuda-device-only", "-S", str(source), "-o", str(out)], check=True,
+                         capture_output=True, text=True)
+    assert "reserved register" not in run.stderr
+    text = out.read_text()
+    body = text[text.index("_Z4bothPf:") :]
+    seen = re.findall(r"(m0, \S+)|(global_load_lds_dwordx4)", body[: body.index("s_endpgm")])
+    places = []
+    for place, load in seen:
+        if place:
+            last = place
+        if load:
+            places.append(last)
+            last = None  # (a load leaves m0 as it was, but the next one's place differs)
+    assert places == ["m0, 0", "m0, 0x200", "m0, 0"]
