@@ -168,10 +168,70 @@ def portion_splits(workgroups: int, mean_keys: int) -> int:
     return max(1, min(2 * compute_units() // workgroups, mean_keys // KEYS_PER_WORKGROUP, MAX_KEY_SPLITS))
 
 
-# Keys that a query reads on average from which the prompt kernel with 32 rows a wavefront is the faster one, if its workgroups
-# have most compute units to do: 28 heads over 4, 512 queries at 12,001 167 us -> 137, at 1,536 42 -> 41, at 0 21 -> 26; 500 at
-# 6,000 beside 300 at 3,000 (184 workgroups) 117 -> 123.
+# Keys that a query reads on average from which the prompt kernel with 32 rows a wavefront (small == 2) is looked at: 28 heads
+# over 4, 512 queries at 1,536 42 us -> 41, at 0 21 -> 26.
 ROWS_FROM_KEYS = 1800
+
+# What a launch of the prompt kernels takes, by AttentionPlan.small, in us: to start and end, then for heads of 128 (64: 0.7 of
+# it) a key of its heaviest workgroup, a key of the workgroup that has to share or follow on that one's compute unit, and
+# a key of a compute unit's part of them all.  Over thirteen forms (4 to 16 heads a key/value head, heads of 64 and 128) and
+# twenty steps (8 to 8,192 queries, 1 to 64 portions) 6 % from the time in the mean.
+PORTION_COSTS = ((10.8, 0.031, 0.027, 0.040), (7.3, 0.024, 0.017, 0.022), (8.3, 0.035, 0.007, 0.036))
+
+
+def portion_us(small: int, keys, kv_heads: int, head_dim: int, splits: int, queries: int, heads: int) -> float:
+    """Estimated time of a step's prompt portions in one of the kernels: `keys` that its workgroups read, for one key/value
+    head, which `splits` of them share."""
+    ends, heaviest, second, each = PORTION_COSTS[small]
+    units, same = compute_units(), kv_heads * splits  # workgroups that read alike
+    keys = np.sort(keys)[::-1]
+    at = units // same
+    walk = max(heaviest * float(keys[0]) + (second * float(keys[at]) if at < keys.size else 0.0),
+               each * float(keys.sum()) * same / units) / splits
+    us = ends + (0.7 if head_dim == 64 else 1.0) * walk
+    if splits > 1:  # the kernel that joins the shares
+        us += 3.0 + 0.35e-6 * 4 * queries * heads * splits * head_dim
+    return us
+
+
+def portion_plan(portions, starts, first_seq: int, heads: int, kv_heads: int, head_dim: int, tiles: int, small_tiles: int, rows: int,
+                 reach: int):
+    """How a step's prompt portions are launched: (AttentionPlan.small, shares of keys, sequence and first query of each
+    workgroup).  tiles, small_tiles: of the kernels with 16 queries a wavefront; rows: queries a workgroup of the
+    kernel with 32, 0 where it does not serve the portions; reach: the most keys that a query reads."""
+    small = 0
+    if small_tiles:
+        # Workgroups of half the size while all of them find room on the chip at
+        # once (two on a compute unit): the step then takes as long as the
+        # heaviest of them, which has half the queries.  Measured at 28 heads
+        # over 4: 2,048 queries in 67 to 77 us against 92, 4,096 the same either way;
+        # at 40 over 8: 1,024 in 37 against 48, 2,048 in 118 against 98.
+        small_count = int((-(-portions // (QUERY_TILE * small_tiles))).sum())
+        # (two workgroups of 8 wavefronts fit on a compute unit)
+        if small_count * kv_heads <= 2 * compute_units():
+            small, tiles = 1, small_tiles
+
+    def listed(run):
+        seqs, q0 = portion_runs(portions, first_seq, run)
+        # the keys an entry's last query reads: where its portion starts plus its queries
+        return seqs, q0, np.minimum(starts[seqs - first_seq] + q0 + run, reach + run)
+
+    seqs, q0, keys = listed(QUERY_TILE * tiles)
+    splits = portion_splits(int(seqs.size) * kv_heads, int(keys.mean()))
+    # enough keys for a query, and workgroups for most compute units (a prompt too short for it is not looked at further)
+    if rows and (starts + portions).max() >= ROWS_FROM_KEYS and portion_mean_keys(portions, starts, reach) >= ROWS_FROM_KEYS:
+        row_seqs, row_q0, row_keys = listed(rows)
+        count = int(row_seqs.size) * kv_heads
+        row_splits = portion_splits(2 * count, int(row_keys.mean()))  # (one workgroup on a compute unit)
+        # Workgroups of 256 rows lose where the portions fill few of them (64 portions of 8 queries at 2,000, 28 heads over 4:
+        # 60 us against 80) or where their heaviest one walks alone (4,096 queries at 0, 14 over 2: 95 against 108).
+        queries = int(portions.sum())
+        if 4 * count * row_splits >= 3 * compute_units() and (
+                1.03 * portion_us(2, row_keys, kv_heads, head_dim, row_splits, queries, heads)
+                <= portion_us(small, keys, kv_heads, head_dim, splits, queries, heads)):
+            small, splits, seqs, q0, keys = 2, row_splits, row_seqs, row_q0, row_keys
+    order = heavy_first(keys)
+    return small, splits, seqs[order], q0[order]
 
 
 def portion_mean_keys(q_lens, starts, reach: int) -> float:
@@ -453,46 +513,15 @@ class PagedAttention(Mixer):
         portions = shape.q_lens[shape.num_decode:]
         if portions.size == 0:
             return
-        # enough keys for a query, and workgroups for most compute units (a prompt too short for it is not looked at further)
-        rows, starts = 0, shape.starts[shape.num_decode:]
-        if ((starts + portions).max() >= ROWS_FROM_KEYS and portion_mean_keys(portions, starts, reach) >= ROWS_FROM_KEYS
-                and not getattr(s, "softcap", None) and self.dist_bias is None):
-            rows = ops.attention_prefill_rows_queries(h, hkv, d)
-        if rows:
-            seqs, q0 = portion_runs(portions, shape.num_decode, rows)
-            keys = np.minimum(shape.starts[seqs] + q0 + rows, reach + rows)
-            count = int(seqs.size) * hkv
-            splits = portion_splits(2 * count, int(keys.mean()))  # (one workgroup on a compute unit)
-            if 4 * count * splits < 3 * compute_units():
-                rows = 0
         tiles = ops.attention_prefill_shared_tiles(h, hkv, d)
-        if rows:
-            plan.kernel, plan.small, plan.portion_splits = "shared", 2, splits
-            order = heavy_first(keys)
-            seqs, q0 = seqs[order], q0[order]
-            plan.first_token = shape.num_decode
-        elif tiles:
-            plan.kernel = "shared"
-            small_tiles = ops.attention_prefill_shared_tiles(h, hkv, d, small=True)
-            if small_tiles:
-                # Workgroups of half the size while all of them find room on the chip at
-                # once (two on a compute unit): the step then takes as long as the
-                # heaviest of them, which has half the queries.  Measured at 28 heads
-                # over 4: 2,048 queries in 67 to 77 us against 92, 4,096 the same either way;
-                # at 40 over 8: 1,024 in 37 against 48, 2,048 in 118 against 98.
-                small_count = int((-(-portions // (QUERY_TILE * small_tiles))).sum())
-                # (two workgroups of 8 wavefronts fit on a compute unit)
-                if small_count * hkv <= 2 * compute_units():
-                    plan.small, tiles = 1, small_tiles
-            seqs, q0 = portion_runs(portions, shape.num_decode, QUERY_TILE * tiles)
-            # the keys an entry's last query reads: where its portion starts plus its queries
-            keys = shape.starts[seqs] + q0 + QUERY_TILE * tiles
-            if s.window or s.chunk:
-                keys = np.minimum(keys, reach + QUERY_TILE * tiles)
-            order = heavy_first(keys)
-            seqs, q0 = seqs[order], q0[order]
-            plan.portion_splits = portion_splits(int(seqs.size) * hkv, int(keys.mean()))
-            plan.first_token = shape.num_decode
+        if tiles:
+            plan.kernel, plan.first_token = "shared", shape.num_decode
+            rows = 0
+            if not getattr(s, "softcap", None) and self.dist_bias is None:
+                rows = ops.attention_prefill_rows_queries(h, hkv, d)
+            plan.small, plan.portion_splits, seqs, q0 = portion_plan(
+                portions, shape.starts[shape.num_decode:], shape.num_decode, h, hkv, d, tiles,
+                ops.attention_prefill_shared_tiles(h, hkv, d, small=True), rows, reach)
         else:
             plan.kernel = "tiles"
             seqs, q0 = portion_runs(portions, shape.num_decode, QUERY_TILE)

@@ -297,3 +297,56 @@ def test_float32_single_tokens_of_one_block_of_keys_are_one_launch():
         for s in seqs:
             cache.free(s)
     assert keys[1] == keys[200] == keys[256] != keys[257] == keys[300] == keys[1024] != keys[1025]
+
+
+# (query heads, key/value heads, head size, portions [(queries, position)], whether the kernel with 32 rows a wavefront serves
+# them; us of the other kernel and of it)
+PROMPT_KERNELS = [
+    (28, 4, 128, [(512, 6000)], True),         # 98 -> 84
+    (28, 4, 128, [(512, 2000)], True),         # 50 -> 47
+    (28, 4, 128, [(8192, 0)], True),           # 682 -> 575
+    (28, 4, 128, [(100, 8000)] * 4, True),     # 100 -> 76
+    (40, 8, 128, [(170, 5000)] * 3, True),     # 202 -> 103
+    (16, 1, 128, [(12, 6000)] * 32, True),     # 59 -> 46
+    (14, 2, 64, [(512, 16000)], True),         # 77 -> 68
+    (16, 4, 64, [(8192, 0)], True),            # 282 -> 231
+    # portions that fill few of a workgroup's rows
+    (28, 4, 128, [(8, 2000)] * 64, False),     # 60 / 80
+    (28, 4, 128, [(12, 6000)] * 32, False),    # 94 / 140
+    (40, 8, 128, [(8, 2000)] * 16, False),     # 33 / 46
+    (32, 8, 128, [(20, 2000)] * 16, False),    # 38 / 50
+    (32, 8, 128, [(30, 4000)] * 16, False),    # 69 / 95
+    (32, 8, 128, [(17, 16000), (9, 14000)], False),  # 34 / 46
+    (14, 2, 64, [(12, 6000)] * 32, False),     # 35 / 49
+    (16, 4, 64, [(30, 4000)] * 16, False),     # 29 / 37
+    # the last queries of one prompt in one workgroup, one to a compute unit
+    (16, 4, 128, [(4096, 0)], False),          # 130 / 140
+    (16, 1, 128, [(4096, 0)], False),          # 125 / 139
+    (14, 2, 64, [(4096, 0)], False),           # 95 / 108
+    # few keys, or few workgroups
+    (28, 4, 128, [(512, 0)], False), (28, 4, 128, [(40, 3000)], False),
+]
+
+
+@pytest.mark.parametrize("heads, kv_heads, head_dim, steps, rows", PROMPT_KERNELS)
+def test_prompt_portions_take_the_kernel_that_serves_them_sooner(heads, kv_heads, head_dim, steps, rows):
+    import numpy as np
+    import torch
+
+    from shrike_amd.config import AttentionSpec
+    from shrike_amd.engine.context import StepShape
+    from shrike_amd.parts.attention import QUERY_TILE, PagedAttention
+
+    mixer = PagedAttention(AttentionSpec(num_heads=heads, num_kv_heads=kv_heads, head_dim=head_dim, qkv_bias=False, out_bias=False,
+                                         scale=0.1), 256, "m")
+    mixer.dtype, mixer.dist_bias = torch.bfloat16, None
+    queries, starts = (np.array(x) for x in zip(*steps))
+    shape = StepShape(np.concatenate([[1, 1], queries]), np.concatenate([[5, 70], starts]), 16)
+    mixer.prepare(shape)
+    plan = shape.notes[mixer.plan_key]
+    assert plan.kernel == "shared" and (plan.small == 2) == rows and plan.first_token == 2
+    # every query once, whichever kernel it is
+    run = (ops.attention_prefill_rows_queries(heads, kv_heads, head_dim) if rows
+           else QUERY_TILE * ops.attention_prefill_shared_tiles(heads, kv_heads, head_dim, small=bool(plan.small)))
+    listed = sorted(zip(shape.extras[plan.seq_name].tolist(), shape.extras[plan.q0_name].tolist()))
+    assert listed == [(2 + i, q) for i, n in enumerate(queries) for q in range(0, int(n), run)] and len(listed) == plan.count
