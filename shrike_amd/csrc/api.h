@@ -538,6 +538,9 @@ int shk_moe_experts(const void* x, const int32_t* chosen, const float* weights, 
 long long shk_moe_grouped_scratch_bytes(int n, int width, int experts, int top);
 // tiled: w_gate, w_up and w_down are the stacked matrices as shk_retile_weight lays them out (width and ff in
 // multiples of 64).
+// shk_moe_experts_plan: 8 * the tile of gate and up + the tile of down (numbers of kWide, gemm_wide.h) where tiled matrices and
+// long lists take the large kernel, -1: the kernel for long lists of row-major matrices, -2: those for short lists.
+int shk_moe_experts_plan(int n, int width, int ff, int experts, int top, int identity, int single, int tiled);
 int shk_moe_experts_grouped(const void* x, const int32_t* chosen, const float* weights, const void* w_gate,
                             const void* w_up, const void* w_down, const void* add, const float* add_gate,
                             int gate_ld, void* act_buf, void* out, void* scratch, int n, int width, int ff, int experts, int top,

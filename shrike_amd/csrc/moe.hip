@@ -665,7 +665,7 @@ __global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per
 #pragma unroll
   for (int i = 0; i < S::kWLoads; ++i) {
     const int tile = wave + S::kWaves * i, f = f0 + (PRODUCT == kMoeGated ? tile / 2 : tile) * 16;
-    woff[i] = (static_cast<unsigned>(min(f, m - 16) / 16) * (k / 32) * kWave + lane) * 16u;
+    woff[i] = (static_cast<unsigned>((min(f, m - 16) - f0) / 16) * (k / 32) * kWave + lane) * 16u;  // (from row f0 on)
   }
 #pragma unroll
   for (int i = 0; i < 2 * S::kXLoads; ++i) {
@@ -675,7 +675,7 @@ __global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per
     xoff[i] = static_cast<unsigned>(row) * k * 2u + ((lane % 8) ^ (lane / 8)) * 16u;
   }
   f32x16 acc[RM][RN];
-  wide_loop<GM, GN, RM, RN>(acc, mem, reinterpret_cast<const char*>((up ? w1 : w0) + static_cast<size_t>(e) * m * k), woff,
+  wide_loop<GM, GN, RM, RN>(acc, mem, reinterpret_cast<const char*>((up ? w1 : w0) + (static_cast<size_t>(e) * m + f0) * k), woff,
                         reinterpret_cast<const char*>(a), xoff, 0u, -1, k / 32, k / 64);
 
   // Register g * 4 + r of lane (j, half) of a tile of 32 x 32 holds weight row g * 8 + half * 4 + r for pair j.  32 pairs'
@@ -732,22 +732,27 @@ static void launch_big(const bf16* a, const int32_t* order, const int32_t* count
 // list ends in half a tile, and `identity` of the router's outputs take their share of the pairs.  (Which tile makes no
 // difference to the sums.)  A lane's values of the activation take 0.12 us each.  8 experts of 3584 x 4736, 1,501 tokens
 // of two choices in 256 x 128, 256 x 192, 128 x 192: gate and up 232 / 254 / 260 us, down 142 / 105 / 122.
-template <int PRODUCT>
-static void big_product(const bf16* a, const int32_t* order, const int32_t* counts, const void* w0, const void* w1, bf16* act_out,
-                        float* pair_out, int n, int k, int m, int experts, int identity, int top, GateForm form, hipStream_t s) {
+constexpr int kBigTiles[] = {4, 1, 6};  // of kWide: 256 x 128, 256 x 192, 128 x 192
+static int big_tile_of(int product, int n, int k, int m, int experts, int identity, int top) {
   const double pairs = static_cast<double>(n) * top * experts / (experts + identity);
-  const int rows = PRODUCT == kMoeGated ? 2 * m : m;
-  constexpr int kTried[] = {4, 1, 6};  // 256 x 128, 256 x 192, 128 x 192
+  const int rows = product == kMoeGated ? 2 * m : m;
   int best = 0;
   double least = 0.0;
   for (int i = 0; i < 3; ++i) {
-    WideTile t = kWide[kTried[i]];
-    if (PRODUCT != kMoeDown) t.ends += 0.12 * (PRODUCT == kMoeGated ? t.rows / 2 : t.rows) * t.tokens / (i ? 256 : 512);
+    WideTile t = kWide[kBigTiles[i]];
+    if (product != kMoeDown) t.ends += 0.12 * (product == kMoeGated ? t.rows / 2 : t.rows) * t.tokens / (i ? 256 : 512);
     const double us = wide_time(t, ((rows + t.rows - 1) / t.rows) * (pairs / t.tokens + 0.5 * (experts < pairs ? experts : pairs)), k / 64);
     if (!i || us < least) least = us, best = i;
   }
-  const auto launch = best == 0   ? launch_big<PRODUCT, 4, 2, 2, 2>
-                      : best == 1 ? launch_big<PRODUCT, 2, 2, 4, 3>
+  return best;
+}
+
+template <int PRODUCT>
+static void big_product(const bf16* a, const int32_t* order, const int32_t* counts, const void* w0, const void* w1, bf16* act_out,
+                        float* pair_out, int n, int k, int m, int experts, int identity, int top, GateForm form, hipStream_t s) {
+  const int tile = big_tile_of(PRODUCT, n, k, m, experts, identity, top);
+  const auto launch = tile == 0   ? launch_big<PRODUCT, 4, 2, 2, 2>
+                      : tile == 1 ? launch_big<PRODUCT, 2, 2, 4, 3>
                                   : launch_big<PRODUCT, 2, 2, 2, 3>;
   launch(a, order, counts, w0, w1, act_out, pair_out, n, k, m, experts, top, form, s);
 }
@@ -769,6 +774,23 @@ static bool fills_long_lists(int n, int top, int width, int ff, int experts, boo
   const double flops = (single ? 4.0 : 6.0) * static_cast<double>(tokens * top) * width * ff;
   const double empty = top < experts ? (tokens + 31) / 32 * static_cast<double>(experts - top) * ((width + 31) / 32 + (ff + 31) / 32) : 0.0;
   return flops / 2e8 + empty / 3e3 >= 7.0 + 0.0125 * (width + ff);  // microseconds
+}
+
+// Tokens of one call with lists for moe_big_mfma_kernel, whose offsets within the tokens' rows, and within the pairs', are 32 bits
+// wide; more of them are taken in several turns.
+static int big_tokens(int n, int width, int ff, int top) {
+  const long long row = width > static_cast<long long>(top) * ff ? width : static_cast<long long>(top) * ff;
+  const long long most = ((1LL << 31) - 1) / row, turns = most ? (n + most - 1) / most : 1;
+  return static_cast<int>((n + turns - 1) / turns);
+}
+
+// Which kernels take a step's products: 0 moe_big_mfma_kernel, 1 moe_tiled_mfma_kernel, 2 those for short lists.
+static int experts_kernel(int n, int width, int ff, int experts, int top, bool single, bool tiled) {
+  const bool many = static_cast<long long>(n) * top >= 64LL * experts;  // lists of 64 pairs and more on average
+  if (many && !tiled) return 1;
+  // (offsets within 256 rows of a matrix, and within a token's, are 32 bits wide)
+  const bool near = width <= 1 << 22 && static_cast<long long>(top) * ff < 1LL << 31 && ff <= 1 << 22;
+  return many && near && fills_long_lists(n, top, width, ff, experts, single) ? 0 : 2;
 }
 
 // out[t, c] = add[t, c] + sum_k weights[t, k] * pair_out[t * top + k, c], k in the order chosen; an identity
@@ -899,6 +921,14 @@ extern "C" long long shk_moe_grouped_scratch_bytes(int n, int width, int experts
   return ((ints * 4 + 15) / 16) * 16 + static_cast<long long>(n) * top * width * 4;
 }
 
+extern "C" int shk_moe_experts_plan(int n, int width, int ff, int experts, int top, int identity, int single, int tiled) {
+  const int kernel = experts_kernel(n, width, ff, experts, top, single, tiled);
+  if (kernel) return -kernel;
+  n = big_tokens(n, width, ff, top);
+  return 8 * kBigTiles[big_tile_of(single ? kMoeSingle : kMoeGated, n, width, ff, experts, identity, top)] +
+         kBigTiles[big_tile_of(kMoeDown, n, ff, width, experts, identity, top)];
+}
+
 extern "C" int shk_moe_experts_grouped(const void* x, const int32_t* chosen, const float* weights, const void* w_gate,
                                        const void* w_up, const void* w_down, const void* add, const float* add_gate,
                                        int gate_ld, void* act_buf, void* out, void* scratch, int n, int width, int ff, int experts, int top,
@@ -918,6 +948,20 @@ extern "C" int shk_moe_experts_grouped(const void* x, const int32_t* chosen, con
               "moe_experts_grouped: null pointer");
   for (const void* p : {x, w_gate, w_up, w_down, static_cast<const void*>(act_buf), static_cast<const void*>(scratch)})
     SHK_REQUIRE(reinterpret_cast<uintptr_t>(p) % 16 == 0, "moe_experts_grouped: operands must be 16-byte aligned");
+  const int kernel = experts_kernel(n, width, ff, experts, top, w_gate == w_up, tiled);
+  const int turn = kernel ? n : big_tokens(n, width, ff, top);
+  if (turn < n) {
+    for (int t = 0; t < n; t += turn) {
+      const size_t at = t;
+      const int failed = shk_moe_experts_grouped(
+          static_cast<const bf16*>(x) + at * width, chosen + at * top, weights + at * top, w_gate, w_up, w_down,
+          add ? static_cast<const bf16*>(add) + at * width : nullptr, add_gate ? add_gate + at * gate_ld : nullptr, gate_ld, act_buf,
+          static_cast<bf16*>(out) + at * width, scratch, turn < n - t ? turn : n - t, width, ff, experts, top, identity, act, limit,
+          shift, tiled, stream);
+      if (failed) return failed;
+    }
+    return 0;
+  }
   hipStream_t s = static_cast<hipStream_t>(stream);
   const GateForm form{act, limit, shift};
   int32_t* order = static_cast<int32_t*>(scratch);
@@ -926,17 +970,13 @@ extern "C" int shk_moe_experts_grouped(const void* x, const int32_t* chosen, con
   float* pair_out = reinterpret_cast<float*>(static_cast<char*>(scratch) + ((ints * 4 + 15) / 16) * 16);
   moe_lists_kernel<<<experts, 256, 0, s>>>(chosen, n, top, order, counts);
   const bf16 *xb = static_cast<const bf16*>(x), *actb = static_cast<const bf16*>(act_buf);
-  const bool many = static_cast<long long>(n) * top >= 64LL * experts;  // lists of 64 pairs and more on average
-  // (offsets within an operand of moe_big_mfma_kernel are 32 bits wide)
-  const bool near = static_cast<long long>(n) * (width > static_cast<long long>(top) * ff ? width : static_cast<long long>(top) * ff) < (1LL << 31) &&
-                    static_cast<long long>(width) * ff < (1LL << 31);
-  if (many && tiled && near && fills_long_lists(n, top, width, ff, experts, w_gate == w_up)) {
+  if (kernel == 0) {
     if (w_gate == w_up)
       big_product<kMoeSingle>(xb, order, counts, w_gate, w_up, static_cast<bf16*>(act_buf), nullptr, n, width, ff, experts, identity, top, form, s);
     else
       big_product<kMoeGated>(xb, order, counts, w_gate, w_up, static_cast<bf16*>(act_buf), nullptr, n, width, ff, experts, identity, top, form, s);
     big_product<kMoeDown>(actb, order, counts, w_down, nullptr, nullptr, pair_out, n, ff, width, experts, identity, top, form, s);
-  } else if (many && !tiled) {
+  } else if (kernel == 1) {
     const int row_tiles = (n + kTileRows - 1) / kTileRows;
     if (w_gate == w_up)
       moe_tiled_mfma_kernel<true, true><<<dim3((ff + 127) / 128, row_tiles, experts), 256, 0, s>>>(

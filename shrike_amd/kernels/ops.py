@@ -1275,6 +1275,14 @@ def tile_experts(matrices) -> torch.Tensor:
     return out
 
 
+def moe_experts_tiles(n: int, width: int, ff: int, experts: int, top: int, identity: int = 0, single: bool = False):
+    """Tiles (weight rows x pairs; gate and up, down) in which the products of long lists of experts in tiles run, None where
+    the kernels for short lists take them."""
+    plan = int(load().shk_moe_experts_plan(n, width, ff, experts, top, identity, int(single), 1))
+    sizes = {4: (256, 128), 1: (256, 192), 6: (128, 192)}
+    return None if plan < 0 else (sizes[plan // 8], sizes[plan % 8])
+
+
 def moe_experts(x, chosen, weights, w_gate, w_up, w_down, act_buf, out, activation: str = "silu", add=None,
                 scratch=None, add_gate=None, identity: int = 0, limit: float | None = None, up_shift: float = 0.0,
                 tiled: bool = False) -> None:

@@ -102,3 +102,62 @@ def test_added_rows_and_results_anywhere_in_memory(n, width, ff, tiled, off_add,
         return out
 
     assert torch.equal(run(off_add, off_out), run(0, 0))
+
+
+# width, features, lists (the edges of tiles of 128 and of 192 pairs; matrices that end within a tile) and the tiles of both products
+TILES = [
+    (576, 192, [191, 192, 193, 384, 385, 1, 0, 7654], ("silu", "bounded"), ((256, 192), (256, 128))),
+    (1344, 64, [191, 193, 0, 385, 3200], ("silu", "bounded"), ((128, 192), (256, 192))),
+    (64, 704, [127, 128, 129, 191, 192, 193, 385, 2700], ("silu",), ((256, 128), (128, 192))),
+    (1344, 320, [191, 192, 193, 384, 385, 1, 0, 7654], ("single",), ((256, 192), (256, 128))),
+    (1344, 64, [191, 192, 193, 385, 0, 257, 63, 2719], ("single",), ((128, 192), (256, 192))),
+]
+
+
+@pytest.mark.parametrize("width, ff, counts, form, tiles", [(w, f, c, form, t) for w, f, c, forms, t in TILES for form in forms])
+def test_every_tile(width, ff, counts, form, tiles):
+    from shrike_amd.kernels import ops
+
+    n = max(sum(counts), 32 * len(counts))
+    assert ops.moe_experts_tiles(n, width, ff, len(counts), 2, 1, form == "single") == tiles
+    test_lists_of_every_length(width, ff, counts, form)
+
+
+def test_more_than_two_to_the_31_activations():
+    """Offsets that no longer fit 32 bits: the tokens are taken in turns, by the kernel that takes fewer of them, and a token's
+    result is the same bits whatever the call holds beside it."""
+    from shrike_amd.kernels import ops
+
+    width, ff, experts, top, n, few = 64, 8192, 2, 2, 131200, 20000
+    assert n * top * ff > 1 << 31 and ops.moe_experts_tiles(n, width, ff, experts, top, 1) and ops.moe_experts_tiles(few, width, ff, experts, top, 1)
+    gen = torch.Generator("cuda").manual_seed(1)
+    x = torch.randn(n, width, generator=gen, device="cuda").bfloat16()
+    w_gate, w_up = ((torch.randn(experts, ff, width, generator=gen, device="cuda") / 8).bfloat16() for _ in range(2))
+    w_down = (torch.randn(experts, width, ff, generator=gen, device="cuda") / 90).bfloat16()
+    tiled = [ops.tile_experts(w) for w in (w_gate, w_up, w_down)]
+    chosen = torch.rand(n, experts + 1, generator=gen, device="cuda").argsort(1)[:, :top].int().contiguous()  # (no expert twice)
+    weights, add = torch.rand(n, top, generator=gen, device="cuda"), torch.randn(n, width, generator=gen, device="cuda").bfloat16()
+    share = torch.randn(n, 3, generator=gen, device="cuda")
+
+    def run(lo, hi):
+        rows, out = slice(lo, hi), torch.full((hi - lo, width), 5.0, device="cuda", dtype=torch.bfloat16)
+        act_buf = torch.empty((hi - lo) * top, ff, device="cuda", dtype=torch.bfloat16)
+        scratch = torch.empty(ops.moe_grouped_scratch_bytes(hi - lo, width, experts, top), device="cuda", dtype=torch.uint8)
+        ops.moe_experts(x[rows], chosen[rows], weights[rows], *tiled, act_buf, out, "silu", scratch=scratch, add=add[rows],
+                        add_gate=share[rows, 1], identity=1, tiled=True)
+        return out
+
+    out = run(0, n)
+    for lo in (0, n // 2 - few // 2, n - few):
+        assert torch.equal(out[lo : lo + few], run(lo, lo + few))
+    for t in (0, n // 2 - 1, n // 2, n - 1):
+        want = torch.sigmoid(share[t, 1].double()) * add[t].double()
+        for k in range(top):
+            e = int(chosen[t, k])
+            y = x[t].double()
+            if e < experts:
+                g, u = w_gate[e].double() @ y, w_up[e].double() @ y
+                y = w_down[e].double() @ (g * torch.sigmoid(g) * u)
+            want += weights[t, k].double() * y
+        # 2^-8 of the result and of each of 8,192 activations, whose errors add as their squares do
+        assert float((out[t].double() - want).norm()) <= 2.0**-7 * float(want.norm())

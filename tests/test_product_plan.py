@@ -350,3 +350,10 @@ def test_prompt_portions_take_the_kernel_that_serves_them_sooner(heads, kv_heads
            else QUERY_TILE * ops.attention_prefill_shared_tiles(heads, kv_heads, head_dim, small=bool(plan.small)))
     listed = sorted(zip(shape.extras[plan.seq_name].tolist(), shape.extras[plan.q0_name].tolist()))
     assert listed == [(2 + i, q) for i, n in enumerate(queries) for q in range(0, int(n), run)] and len(listed) == plan.count
+
+
+def test_experts_of_any_size_keep_the_kernel_for_long_lists():
+    assert ops.moe_experts_tiles(131200, 64, 8192, 2, 2)  # 2^31 activations and more
+    assert ops.moe_experts_tiles(70000, 32768, 64, 8, 2)  # elements of the tokens' rows
+    assert ops.moe_experts_tiles(128, 32768, 65536, 1, 1)  # of a matrix
+    assert ops.moe_experts_tiles(64, 64, 64, 8, 2) is None and ops.moe_experts_tiles(1501, 3584, 4736, 8, 2, 2) == ((256, 128), (256, 192))
