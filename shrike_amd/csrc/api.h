@@ -136,6 +136,9 @@ int shk_gemm_bf16_splits(int n, int m, int k);
 // 1 where a product that is not split reaches a reader of partial sums as one float32 part (what the kernels for large
 // matrices would have split).
 int shk_gemm_bf16_keeps_float32(int n, int m, int k);
+// the same for activations whose rows are not 16-byte aligned
+int shk_gemm_bf16_splits_unaligned(int n, int m, int k);
+int shk_gemm_bf16_keeps_float32_unaligned(int n, int m, int k);
 // 2 where a product of many tokens runs as two (the weight rows whose tiles make whole
 // rounds of the compute units, then the rest with tiles of its own), else 1.
 int shk_gemm_bf16_parts(int n, int m, int k, int gated);

@@ -1212,19 +1212,28 @@ static int staged_splits(int n, int m, int k) {
   return split > 1 ? split : 1;
 }
 
-extern "C" int shk_gemm_bf16_splits(int n, int m, int k) {
+// Shares of k that the kernel for a product wants.  Rows that are not 16-byte aligned are taken by others than aligned
+// ones (gemm_big_kernel instead of gemm_wide_kernel: 1000 x 5120 x 13824 522 us in its three shares, 747 whole).
+static int splits_of(int n, int m, int k, bool aligned) {
   if (n > 64 && few_rows(m) && few_rows_whole(n, m, k)) return 1;
+  const int staged = staged_splits(n, m, k);
+  if (!aligned || k % 8) return staged;
   const int direct = direct_splits(n, m, k);
   if (direct) return direct;
-  const int staged = staged_splits(n, m, k);
-  return n > 64 && k % 8 == 0 ? wide_splits(n, m, k, staged > 1 ? 4 : 2) : staged;
+  return n > 64 ? wide_splits(n, m, k, staged > 1 ? 4 : 2) : staged;
 }
+
+extern "C" int shk_gemm_bf16_splits(int n, int m, int k) { return splits_of(n, m, k, true); }
+extern "C" int shk_gemm_bf16_splits_unaligned(int n, int m, int k) { return splits_of(n, m, k, false); }
 
 // Whether a reader that adds up shares gets an unsplit product as one float32 share all the same: where
 // gemm_direct_kernel, or gemm_skinny_kernel group by group, form whole what the staged kernels would leave in shares.  In bfloat16
 // it would be rounded once more than a product in shares, before the residual or the rotation.
 extern "C" int shk_gemm_bf16_keeps_float32(int n, int m, int k) {
-  return shk_gemm_bf16_splits(n, m, k) == 1 && staged_splits(n, m, k) > 1;
+  return splits_of(n, m, k, true) == 1 && staged_splits(n, m, k) > 1;
+}
+extern "C" int shk_gemm_bf16_keeps_float32_unaligned(int n, int m, int k) {
+  return splits_of(n, m, k, false) == 1 && staged_splits(n, m, k) > 1;
 }
 
 extern "C" int shk_gemm_bf16_tiled_weight(const void* a, const void* wt, const float* bias,

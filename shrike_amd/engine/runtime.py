@@ -97,8 +97,9 @@ class Runtime:
         n = x.shape[0]
         splits = 1
         if w.tiled is not None and not (reader == "norm" and (bias is not None or w.rows % 4 or w.rows > 8192)):
-            splits = ops.gemm_splits(n, w.rows, w.cols)
-            keep_float32 = keep_float32 or ops.gemm_keeps_float32(n, w.rows, w.cols)
+            aligned = ops.rows_aligned(x)
+            splits = ops.gemm_splits(n, w.rows, w.cols, aligned)
+            keep_float32 = keep_float32 or ops.gemm_keeps_float32(n, w.rows, w.cols, aligned)
         if splits > 1:
             parts = ctx.buffer(name + "_parts", (splits, n, w.rows), torch.float32)
             ops.gemm_tiled_weight(x, w.tiled, w.rows, w.cols, parts, splits=splits)

@@ -398,14 +398,22 @@ def interleave_gate_up(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     return wt
 
 
-def gemm_splits(n: int, m: int, k: int) -> int:
-    """Shares of k that fill the chip for an [n, k] x [m, k]^T product (1: do not split)."""
-    return int(load().shk_gemm_bf16_splits(n, m, k))
+def rows_aligned(x) -> bool:
+    """Whether the rows of a bfloat16 matrix begin at multiples of 16 bytes."""
+    return x.data_ptr() % 16 == 0 and x.stride(0) % 8 == 0
 
 
-def gemm_keeps_float32(n: int, m: int, k: int) -> bool:
+def gemm_splits(n: int, m: int, k: int, aligned: bool = True) -> int:
+    """Shares of k that fill the chip for an [n, k] x [m, k]^T product (1: do not split); `aligned`: rows_aligned()
+    of the first factor, other kernels take it where it is not."""
+    lib = load()
+    return int((lib.shk_gemm_bf16_splits if aligned else lib.shk_gemm_bf16_splits_unaligned)(n, m, k))
+
+
+def gemm_keeps_float32(n: int, m: int, k: int, aligned: bool = True) -> bool:
     """Whether an [n, k] x [m, k]^T product that is not split reaches a reader of partial sums as one float32 part."""
-    return bool(load().shk_gemm_bf16_keeps_float32(n, m, k))
+    lib = load()
+    return bool((lib.shk_gemm_bf16_keeps_float32 if aligned else lib.shk_gemm_bf16_keeps_float32_unaligned)(n, m, k))
 
 
 def gemm_parts(n: int, m: int, k: int, gated: bool = False) -> int:

@@ -357,3 +357,31 @@ def test_experts_of_any_size_keep_the_kernel_for_long_lists():
     assert ops.moe_experts_tiles(70000, 32768, 64, 8, 2)  # elements of the tokens' rows
     assert ops.moe_experts_tiles(128, 32768, 65536, 1, 1)  # of a matrix
     assert ops.moe_experts_tiles(64, 64, 64, 8, 2) is None and ops.moe_experts_tiles(1501, 3584, 4736, 8, 2, 2) == ((256, 128), (256, 192))
+
+
+def test_rows_that_are_not_aligned_take_the_shares_of_their_own_kernels():
+    """As many as for a k that is no whole number of 16-byte pieces, which the same kernels take."""
+    for n, m, k in ((1000, 5120, 13824), (512, 3584, 18944), (100, 3584, 3584), (300, 896, 4864), (64, 896, 4864), (8, 3584, 18944),
+                    (1501, 10, 3584), (2048, 4608, 3584)):
+        assert ops.gemm_splits(n, m, k, aligned=False) == ops.gemm_splits(n, m, k - 4)
+        assert ops.gemm_keeps_float32(n, m, k, aligned=False) == ops.gemm_keeps_float32(n, m, k - 4)
+    assert ops.gemm_splits(1000, 5120, 13824) == 1 and ops.gemm_splits(1000, 5120, 13824, aligned=False) == 3
+
+
+def test_a_deferred_product_is_planned_for_the_rows_that_it_gets(monkeypatch):
+    from types import SimpleNamespace
+
+    import torch
+
+    from shrike_amd.engine.runtime import Runtime
+
+    runtime, calls = Runtime("cpu", torch.bfloat16), []
+    monkeypatch.setattr(ops, "gemm_tiled_weight", lambda x, wt, m, k, out, **more: calls.append(more["splits"]))
+    ctx = SimpleNamespace(buffer=lambda name, shape, dtype: torch.empty(shape, dtype=dtype))
+    weight = SimpleNamespace(tiled=1, rows=5120, cols=13824)
+    rows = torch.empty(512, 13824 + 8, dtype=torch.bfloat16)
+    for x, aligned in ((rows[:, :13824], True), (rows[:, 4:13828], False), (rows.flatten()[: 512 * 13828].view(512, 13828)[:, :13824], False)):
+        assert ops.rows_aligned(x) == aligned
+        out = runtime.linear_deferred(ctx, "p", x, weight)
+        assert out.parts.shape[0] == calls[-1] == ops.gemm_splits(512, 5120, 13824, aligned)
+    assert len(set(calls)) == 2
