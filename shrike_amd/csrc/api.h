@@ -142,6 +142,8 @@ int shk_gemm_bf16_keeps_float32_unaligned(int n, int m, int k);
 // 2 where a product of many tokens runs as two (the weight rows whose tiles make whole
 // rounds of the compute units, then the rest with tiles of its own), else 1.
 int shk_gemm_bf16_parts(int n, int m, int k, int gated);
+// tiles of a product of more than 64 tokens: their number (0: not served in tiles), (weight rows, tokens) of up to two
+int shk_gemm_bf16_tiles(int n, int m, int k, int gated, int ksplit, int aligned, int* sizes);
 
 // The matrix instruction alone, for measuring its rate on operands of a given kind:
 // workgroups x 4 wavefronts each multiply, iters times, a 64 x 64 x 32 block

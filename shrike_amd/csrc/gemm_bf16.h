@@ -111,6 +111,8 @@ inline unsigned big_grid(int tiles_x, int tiles_y, int tile_rows, int tile_token
 // Products of more than 64 tokens whose activations are 16-byte aligned with k % 8 == 0 (gemm_wide.hip).
 int wide_splits(int n, int m, int k, int whole_bytes);
 int wide_parts(int n, int m, int k, int gated);
+int wide_tiles(int n, int m, int k, int gated, int ksplit);
+void wide_tile_size(int tile, int* rows, int* tokens);
 bool wide_serves(int lda, int k);
 void wide_product(hipStream_t s, const bf16* a, int lda, int n, int k, const uint4* wt, int m, const float* bias, void* out,
                   int ldo, int out_f32, int accumulate, int gated, int ksplit);

@@ -988,9 +988,6 @@ extern "C" int shk_interleave_gate_up(const void* gate_t, const void* up_t, int 
   return 0;
 }
 
-// Workgroups per block of 16 weight rows that a product with at most 64 rows
-// should be split into along k so that the chip is full (about 8192 wavefronts
-// with 4 k-tiles or more each): 1 for matrices with many row blocks.
 template <int GM, int GN, int WM, int WN, int KS>
 static void launch_big(hipStream_t s, const bf16* ap, int lda, int n, int k, const uint4* wp, int kt,
                        int m, const float* bias, void* out, int ldo, int of, int accumulate, int vec,
@@ -1019,15 +1016,15 @@ static void launch_big(hipStream_t s, const bf16* ap, int lda, int n, int k, con
 // Estimated time in microseconds of a product of many tokens with workgroup tiles
 // of `shape` (0: 256 weight rows x 256 tokens, 1: 256 x 128, 2: 128 x 128) and
 // `split` shares of k: rounds of workgroups over the chip's 256 compute units
-// times the time of one workgroup, at the rates measured for each shape
-// (TFLOP/s per compute unit: 4.75, 4.0, and for the smallest tile 3.0 with the
-// compute unit to itself or 1.5 for each of two), plus what a kernel costs
-// anyway, plus writing and reading the float32 parts of a split product at
-// 3 TB/s (at 4 TB/s the estimate took shares that lost with their reader: the
-// 14B down matrix at 4,096 tokens 701 us in two shares against 553 whole, the 14B
-// QKV matrix at 768 tokens 100 us in three against 87, the 7B QKV matrix at 512
-// tokens 54 in three against 51).  It reproduces the measured times of the 7B
-// and 14B matrices at 512 tokens within 10 %.
+// times the time of one workgroup at the shape's rate (TFLOP/s per compute unit: 4.75,
+// 4.0, and for the smallest tile 3.0 with the compute unit to itself or 1.5 for each
+// of two), plus what a kernel costs anyway, plus writing and reading the float32 parts
+// of a split product at 3 TB/s.  The rates are those of loads in whole 16-byte pieces.
+// gemm_big_kernel, which takes the rows that are not aligned, reaches a quarter to a half
+// of them (512 x 4608 x 3588 in two shares 124 us, 2048 x 18944 x 3588 gated 2,107), in about
+// the same proportion: over 17 such products the shape taken is within 11 % of the fastest
+// of the three.  The shares that it expects for aligned rows say which products reach their
+// reader in float32 (shk_gemm_bf16_keeps_float32).
 static double big_estimate(int shape, int split, int n, int wblocks, int m, int k) {
   const int rows = shape == 2 ? 128 : 256, tokens = shape == 0 ? 256 : 128;
   const long long tiles =
@@ -1057,8 +1054,6 @@ static int big_shape(int split, int n, int wblocks, int m, int k) {
       best = shape;
   return best;
 }
-
-extern "C" int shk_gemm_bf16_splits(int n, int m, int k);
 
 // Which gemm_direct_kernel serves a product of n > 16 tokens (0: none): the smallest tile of which a launch has no
 // more than the 256 compute units, for matrices of 256 to 2,048 rows (more of them fill the staged kernels' larger
@@ -1143,12 +1138,42 @@ static int big_main_blocks(int shape, int n, int wblocks, int m, int k, int gate
   return parts < 0.93 * whole ? main_blocks : 0;
 }
 
+struct BigPlan {
+  int shape, main_blocks, rest_shape;  // main_blocks: blocks of 16 weight rows of the first product, 0: one product
+};
+static BigPlan big_plan(int ksplit, int n, int wblocks, int m, int k, int gated) {
+  BigPlan plan = {big_shape(ksplit, n, wblocks, m, k), 0, 0};
+  if (ksplit == 1) plan.main_blocks = big_main_blocks(plan.shape, n, wblocks, m, k, gated);
+  if (!plan.main_blocks) return plan;
+  plan.shape = 0;
+  plan.rest_shape = big_shape(1, n, wblocks - plan.main_blocks, m - plan.main_blocks * 16 / (gated ? 2 : 1), k);
+  return plan;
+}
+
 // Products that a call with these sizes is made of (1, or 2: see big_main_blocks).
 extern "C" int shk_gemm_bf16_parts(int n, int m, int k, int gated) {
   if (n <= 64 || (!gated && (few_rows(m) || direct_shape(n, m, k, 1))) || shk_gemm_bf16_splits(n, m, k) > 1) return 1;
   if (k % 8 == 0) return wide_parts(n, m, k, gated);
   const int wblocks = (gated ? 2 : 1) * ((m + 15) / 16);
-  return big_main_blocks(big_shape(1, n, wblocks, m, k), n, wblocks, m, k, gated) ? 2 : 1;
+  return big_plan(1, n, wblocks, m, k, gated).main_blocks ? 2 : 1;
+}
+
+// Tiles (weight rows, tokens, twice where a product runs as two) of a product of more than 64 tokens, in gemm_wide.hip or for
+// unaligned rows in gemm_big_kernel; returns their number, 0 where another kernel serves it.
+extern "C" int shk_gemm_bf16_tiles(int n, int m, int k, int gated, int ksplit, int aligned, int* sizes) {
+  aligned = aligned && k % 8 == 0;
+  if (n <= 64 || (!gated && ((few_rows(m) && ksplit == 1) || (aligned && direct_shape(n, m, k, ksplit))))) return 0;
+  if (aligned && wide_serves(k, k)) {
+    const int tiles = wide_tiles(n, m, k, gated, ksplit);
+    wide_tile_size(tiles % 16, &sizes[0], &sizes[1]);
+    if (tiles < 16) return 1;
+    wide_tile_size(tiles / 16 - 1, &sizes[2], &sizes[3]);
+    return 2;
+  }
+  const BigPlan plan = big_plan(ksplit, n, (gated ? 2 : 1) * ((m + 15) / 16), m, k, gated);
+  sizes[0] = plan.shape == 2 ? 128 : 256, sizes[1] = plan.shape == 0 ? 256 : 128;
+  sizes[2] = plan.rest_shape == 2 ? 128 : 256, sizes[3] = plan.rest_shape == 0 ? 256 : 128;
+  return plan.main_blocks ? 2 : 1;
 }
 
 // Shares of k for the kernels that stage operands or stream the weights.
@@ -1286,49 +1311,22 @@ extern "C" int shk_gemm_bf16_tiled_weight(const void* a, const void* wt, const f
     const int wblocks = (gated ? 2 : 1) * mb;  // blocks of 16 weight rows
     // Tile of the workgroup: 256 x 256, 256 x 128 or 128 x 128 (weight rows x
     // tokens), whichever big_estimate() expects to finish first.
-    const int shape = big_shape(ksplit, n, wblocks, m, k);
-    int main_blocks = 0;
-    if (ksplit == 1) main_blocks = big_main_blocks(shape, n, wblocks, m, k, gated);
-    if (main_blocks) {
-      const int rest_blocks = wblocks - main_blocks;
-      const int main_rows = main_blocks * 16 / (gated ? 2 : 1), rest_rows = m - main_rows;
-      const int rest_shape = big_shape(1, n, rest_blocks, rest_rows, k);
-      launch_big<4, 4, 4, 4, 1>(s, ap, lda, n, k, wp, kt, main_rows, bias, out, ldo, of, accumulate,
-                                vec, gated, main_blocks, 1);
-      const uint4* rest_w = wp + static_cast<size_t>(main_blocks) * kt * kWave;
-      const int rest_act = gated ? accumulate : plain_act_from(accumulate, main_rows);
-      // (a gated product's `bias` is its gate's two constants, the same for every row)
-      const float* rest_bias = (bias && !gated) ? bias + main_rows : bias;
-      void* rest_out = of ? static_cast<void*>(static_cast<float*>(out) + main_rows)
-                          : static_cast<void*>(static_cast<bf16*>(out) + main_rows);
-      if (rest_shape == 0)
-        launch_big<4, 4, 4, 4, 1>(s, ap, lda, n, k, rest_w, kt, rest_rows, rest_bias, rest_out, ldo,
-                                  of, rest_act, vec, gated, rest_blocks, 1);
-      else if (rest_shape == 1)
-        launch_big<4, 4, 4, 2, 2>(s, ap, lda, n, k, rest_w, kt, rest_rows, rest_bias, rest_out, ldo,
-                                  of, rest_act, vec, gated, rest_blocks, 1);
-      else if (static_cast<long long>((rest_blocks + 7) / 8) * ((n + 127) / 128) <= 256)
-        launch_big<4, 2, 2, 4, 2>(s, ap, lda, n, k, rest_w, kt, rest_rows, rest_bias, rest_out, ldo,
-                                  of, rest_act, vec, gated, rest_blocks, 1);
-      else
-        launch_big<2, 2, 4, 4, 2>(s, ap, lda, n, k, rest_w, kt, rest_rows, rest_bias, rest_out, ldo,
-                                  of, rest_act, vec, gated, rest_blocks, 1);
-      SHK_LAUNCH_CHECK("gemm_bf16");
-      return 0;
-    }
-    if (shape == 0)
-      launch_big<4, 4, 4, 4, 1>(s, ap, lda, n, k, wp, kt, m, bias, out, ldo, of, accumulate, vec,
-                                gated, wblocks, ksplit);
-    else if (shape == 1)
-      launch_big<4, 4, 4, 2, 2>(s, ap, lda, n, k, wp, kt, m, bias, out, ldo, of, accumulate, vec,
-                                gated, wblocks, ksplit);
-    else if (static_cast<long long>((wblocks + 7) / 8) * ((n + 127) / 128) * ksplit <= 256)
-      // every workgroup has a compute unit to itself: eight wavefronts, loads straight into LDS
-      launch_big<4, 2, 2, 4, 2>(s, ap, lda, n, k, wp, kt, m, bias, out, ldo, of, accumulate, vec,
-                                gated, wblocks, ksplit);
-    else  // four wavefronts and two LDS buffers: two workgroups fit on a compute unit
-      launch_big<2, 2, 4, 4, 2>(s, ap, lda, n, k, wp, kt, m, bias, out, ldo, of, accumulate, vec,
-                                gated, wblocks, ksplit);
+    const BigPlan plan = big_plan(ksplit, n, wblocks, m, k, gated);
+    auto go = [&](int shape, const uint4* weights, int rows, int blocks, const float* b, void* dst, int act) {
+      const long long small = static_cast<long long>((blocks + 7) / 8) * ((n + 127) / 128) * ksplit;
+      const auto launch = shape == 0     ? launch_big<4, 4, 4, 4, 1>
+                          : shape == 1   ? launch_big<4, 4, 4, 2, 2>
+                          : small <= 256 ? launch_big<4, 2, 2, 4, 2>   // (a compute unit each: eight wavefronts)
+                                         : launch_big<2, 2, 4, 4, 2>;  // (four, two workgroups on a compute unit)
+      launch(s, ap, lda, n, k, weights, kt, rows, b, dst, ldo, of, act, vec, gated, blocks, ksplit);
+    };
+    const int main_rows = plan.main_blocks * 16 / (gated ? 2 : 1);
+    go(plan.shape, wp, main_rows ? main_rows : m, main_rows ? plan.main_blocks : wblocks, bias, out, accumulate);
+    // (a gated product's `bias` is its gate's two constants, the same for every row)
+    if (main_rows)
+      go(plan.rest_shape, wp + static_cast<size_t>(plan.main_blocks) * kt * kWave, m - main_rows, wblocks - plan.main_blocks,
+         bias && !gated ? bias + main_rows : bias, static_cast<char*>(out) + static_cast<size_t>(main_rows) * (of ? 4 : 2),
+         gated ? accumulate : plain_act_from(accumulate, main_rows));
     SHK_LAUNCH_CHECK("gemm_bf16");
     return 0;
   }

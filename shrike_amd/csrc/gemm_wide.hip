@@ -231,6 +231,15 @@ int wide_parts(int n, int m, int k, int gated) {
   return wide_plan(1, n, (gated ? 2 : 1) * ((m + 15) / 16), k, &us).main_blocks ? 2 : 1;
 }
 
+// The tile of a product's only or first launch, and 16 * (1 + the tile of its second, where there is one).
+int wide_tiles(int n, int m, int k, int gated, int ksplit) {
+  double us;
+  const WidePlan plan = wide_plan(ksplit, n, (gated ? 2 : 1) * ((m + 15) / 16), k, &us);
+  return plan.tile + (plan.main_blocks ? 16 * (1 + plan.rest_tile) : 0);
+}
+
+void wide_tile_size(int tile, int* rows, int* tokens) { *rows = kWide[tile].rows, *tokens = kWide[tile].tokens; }
+
 // Whether offsets within a tile fit 32 bits.
 bool wide_serves(int lda, int k) { return lda <= 4 * 1024 * 1024 && k <= 4 * 1024 * 1024; }
 

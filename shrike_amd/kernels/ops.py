@@ -4,6 +4,8 @@ the current HIP stream to libshrike_hip.  Nothing here computes anything."""
 
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
 from .lib import KernelError, check, load
@@ -420,6 +422,13 @@ def gemm_parts(n: int, m: int, k: int, gated: bool = False) -> int:
     """Launches that an [n, k] x [m, k]^T product is made of (2: rows whose tiles
     fill whole rounds of the compute units, then the rest)."""
     return int(load().shk_gemm_bf16_parts(n, m, k, int(gated)))
+
+
+def gemm_tiles(n: int, m: int, k: int, gated: bool = False, splits: int = 1, aligned: bool = True) -> tuple:
+    """Tiles (weight rows, tokens) of the launches of a product of more than 64 tokens, () where kernels without them serve it."""
+    sizes = (ctypes.c_int * 4)()
+    count = int(load().shk_gemm_bf16_tiles(n, m, k, int(gated), splits, int(aligned), sizes))
+    return tuple((sizes[2 * i], sizes[2 * i + 1]) for i in range(count))
 
 
 def mfma_alone(operands: torch.Tensor, workgroups: int, iters: int) -> float:

@@ -1,5 +1,5 @@
-"""bfloat16 products of more than 64 tokens with aligned rows: every tile, the ends of k, of the rows and of the
-tokens, shares of k, and every way in which results leave."""
+"""bfloat16 products of more than 64 tokens: every tile, the ends of k, of the rows and of the tokens, shares of k, and
+every way in which results leave; rows that are not aligned, which a kernel of their own takes."""
 
 import math
 
@@ -33,20 +33,20 @@ def check(out, want, k):
     assert not bad.any(), f"{int(bad.sum())} values off, the most by {float((out.double() - want).abs().max())}"
 
 
-# (the tiles that the plan takes: weight rows x tokens)
+# (the tiles that the plan takes, weight rows x tokens: TILES below)
 SIZES = [
-    (65, 200, 136),       # 128 x 128
-    (640, 9000, 136),     # 256 x 128
-    (1665, 4616, 136),    # 256 x 256
-    (513, 9000, 520),     # 128 x 192
-    (1665, 4616, 520),    # 192 x 192
-    (1282, 7000, 520),    # 256 x 192
-    (961, 9000, 1096),    # 192 x 256
-    (2048, 3584, 128),    # 128 x 256
-    (1281, 12000, 136),   # two products: 256 x 256, then 128 x 128
-    (1281, 12000, 520),   # 192 x 192, then 256 x 128
-    (1921, 9000, 1096),   # 192 x 256, then 128 x 192
-    (2561, 7000, 1096),   # 256 x 192, then 128 x 128
+    (65, 200, 136),
+    (640, 9000, 136),
+    (1665, 4616, 136),
+    (513, 9000, 520),
+    (1665, 4616, 520),
+    (1282, 7000, 520),
+    (961, 9000, 1096),
+    (2048, 3584, 128),
+    (1281, 12000, 136),   # (two products each)
+    (1281, 12000, 520),
+    (1921, 9000, 1096),
+    (2561, 7000, 1096),
     # k: one piece, less than a tile, a tile, a stage, a stage and a piece, three tiles, five stages and a half
     (70, 2064, 8), (70, 2064, 24), (129, 2064, 32), (129, 2064, 64), (200, 2064, 72), (300, 2064, 96), (130, 2064, 352),
     # rows that are no whole pieces, fewer than a block, one block
@@ -118,3 +118,107 @@ def test_rows_do_not_depend_on_the_others_or_on_the_tile(ops):
     part = torch.empty(513, m, device="cuda")
     ops.gemm_tiled_weight(apart[:, :k], wt, m, k, part)
     assert torch.equal(part, whole[:513])
+
+
+# every tile as a plan takes it: (n, m, k, gated, shares): tiles of the one or two launches
+TILES = {
+    (65, 200, 136, False, 1): ((128, 128),),
+    (640, 9000, 136, False, 1): ((256, 128),),
+    (1665, 4616, 136, False, 1): ((256, 256),),
+    (513, 9000, 520, False, 1): ((128, 192),),
+    (1665, 4616, 520, False, 1): ((192, 192),),
+    (1282, 7000, 520, False, 1): ((256, 192),),
+    (961, 9000, 1096, False, 1): ((192, 256),),
+    (2048, 3584, 128, False, 1): ((256, 128),),
+    (1281, 12000, 136, False, 1): ((256, 256), (128, 128)),
+    (1281, 12000, 520, False, 1): ((192, 192), (256, 128)),
+    (1921, 9000, 1096, False, 1): ((192, 256), (128, 192)),
+    (2561, 7000, 1096, False, 1): ((256, 192), (256, 128)),
+    (65, 200, 136, True, 1): ((128, 128),),
+    (640, 4500, 136, True, 1): ((256, 128),),
+    (1665, 2308, 136, True, 1): ((256, 256),),
+    (513, 4500, 520, True, 1): ((128, 192),),
+    (961, 4500, 1096, True, 1): ((192, 256),),
+    (1282, 3500, 520, True, 1): ((256, 192),),
+    (1665, 2308, 520, True, 1): ((192, 192),),
+    (512, 4608, 1032, False, 2): ((128, 192),),
+    (513, 2060, 520, False, 16): ((256, 256),),
+    # 128 x 256: rows that are and are no whole pieces, half a last stage of k; alone, as the second of two, with shares
+    (1181, 4616, 2056, False, 1): ((128, 256),),
+    (1181, 4615, 2056, False, 1): ((128, 256),),
+    (2049, 9003, 2056, False, 1): ((256, 192), (128, 256)),
+    (158, 9008, 2056, True, 1): ((128, 256),),
+    (158, 9003, 2056, True, 1): ((128, 256),),
+    (1925, 4616, 2056, True, 1): ((256, 192), (128, 256)),
+    (158, 9003, 3592, False, 2): ((128, 256),),
+    (1181, 2060, 2056, False, 3): ((128, 256),),
+    # the others in shares of k
+    (778, 4616, 72, False, 2): ((256, 256),),
+    (158, 9003, 72, False, 2): ((256, 128),),
+    (778, 5125, 1048, False, 2): ((256, 192),),
+    (406, 9003, 2056, False, 2): ((192, 256),),
+    (1026, 3589, 520, False, 2): ((192, 192),),
+    (778, 2309, 1048, False, 2): ((128, 192),),
+    # the tiles left that a second product may have
+    (1801, 7001, 2056, True, 1): ((256, 256), (256, 192)),
+    (1026, 9003, 2056, True, 1): ((256, 192), (192, 192)),
+}
+
+
+@pytest.mark.parametrize("n, m, k, gated, splits", TILES)
+def test_every_tile(ops, n, m, k, gated, splits):
+    assert ops.gemm_tiles(n, m, k, gated, splits) == TILES[n, m, k, gated, splits]
+    if gated:
+        test_gated_products(ops, n, m, k)
+    elif splits > 1:
+        test_shares_of_k(ops, n, m, k, splits)
+    elif (n, m, k) not in SIZES:
+        test_plain_products(ops, n, m, k)
+
+
+# rows that begin anywhere: (n, m, k, gated), elements between rows beyond k; every tile of their kernel, also with more
+# workgroups of 128 x 128 than compute units (four wavefronts instead of eight)
+UNALIGNED = {
+    (65, 130, 36, False, 0): ((128, 128),),
+    (129, 516, 333, False, 0): ((128, 128),),
+    (300, 1000, 520, False, 3): ((128, 128),),
+    (769, 4616, 36, True, 0): ((128, 128),),
+    (257, 12003, 36, False, 0): ((256, 128),),
+    (129, 9003, 100, True, 4): ((256, 128),),
+    (2199, 1100, 12, False, 0): ((128, 128),),  # (486 of 128 x 128 in its three shares)
+    (641, 12003, 37, False, 0): ((256, 256),),
+    (257, 12003, 72, True, 1): ((256, 256),),
+    (1281, 12003, 1100, False, 0): ((256, 256), (128, 128)),
+    (641, 12003, 1100, True, 0): ((256, 256), (128, 128)),
+    (2049, 9003, 2052, True, 0): ((256, 256), (256, 128)),
+}
+
+
+@pytest.mark.parametrize("n, m, k, gated, apart", UNALIGNED)
+def test_rows_that_are_not_aligned(ops, n, m, k, gated, apart):
+    assert ops.gemm_tiles(n, m, k, gated, 1, aligned=False) == UNALIGNED[n, m, k, gated, apart]
+    x, ws = operands(n, m, k, matrices=2 if gated else 1)
+    rows = torch.full((n, k + apart), float("nan"), device="cuda", dtype=BF16)  # (NaN between the rows)
+    rows[:, :k] = x
+    rows = rows[:, :k]
+    assert not ops.rows_aligned(rows) or k % 8
+    first, *second = (x.double() @ w.double().T for w in ws)
+    out, bias = torch.full((n, m), float("nan"), device="cuda", dtype=BF16), torch.randn(m, device="cuda")
+    if gated:
+        wt = ops.interleave_gate_up(*ws)
+        ops.gemm_tiled_weight(rows, wt, m, k, out, gated=True)
+        check(out, torch.nn.functional.silu(first) * second[0], 4 * k)
+        args = torch.tensor([0.5, 1.0], device="cuda")
+        ops.gemm_tiled_weight(rows, wt, m, k, out, gated="quick_gelu", gate_args=args)
+        g, u = first.clamp(max=0.5), second[0].clamp(-0.5, 0.5) + 1.0
+        check(out, g * torch.sigmoid(1.702 * g) * u, 4 * k)
+        return
+    wt = ops.retile_weight(ws[0])
+    ops.gemm_tiled_weight(rows, wt, m, k, out, bias=bias)
+    check(out, first + bias.double(), k)
+    edge = m - 7  # (in the second of two products)
+    ops.gemm_tiled_weight(rows, wt, m, k, out, activation=("silu", edge))
+    check(out, torch.cat([torch.nn.functional.silu(first[:, :edge]), first[:, edge:]], 1), 2 * k)
+    parts = torch.full((3, n, m), float("nan"), device="cuda")
+    ops.gemm_tiled_weight(rows, wt, m, k, parts, splits=3)
+    check(parts.sum(0), first, 2 * k)
