@@ -10,14 +10,19 @@ from shrike_amd.csrc.build import CSRC, HIPCC_FLAGS, find_hipcc
 
 
 def test_no_stage_is_freed_by_another_barrier():
-    users = 0
-    for path in sorted(CSRC.glob("*.hip")):
+    """In every source and header but the one that defines the loads and the barrier."""
+    users = set()
+    for path in sorted([*CSRC.glob("*.hip"), *CSRC.glob("*.h")]):
+        if path.name == "to_lds.h":
+            continue
         text = path.read_text()
-        assert "__builtin_amdgcn_s_barrier" not in text and "__builtin_amdgcn_s_waitcnt" not in text, path.name
+        for name in ("__builtin_amdgcn_s_barrier", "__builtin_amdgcn_s_waitcnt", "__builtin_amdgcn_global_load_lds", "global_load_lds_dword",
+                     "load_to_lds(", "s_barrier", "vmcnt"):
+            assert name not in text, (path.name, name)
         if "SHK_LOAD_TO_LDS(" in text:
-            users += 1
+            users.add(path.name)
             assert "SHK_MEET_WITH_LOADS(" in text, path.name
-    assert users >= 2
+    assert {"gemm_wide.h", "gemm_bf16.hip", "gemm_f32.hip", "attention_rows.hip"} <= users
 
 
 def test_the_barrier_waits_for_reads_of_lds(tmp_path):
@@ -57,7 +62,8 @@ def test_the_barrier_waits_for_reads_of_lds(tmp_path):
 
 
 def test_both_forms_of_the_load_in_one_kernel(tmp_path):
-    """Each of three loads (builtin, base + offset, builtin) goes where it should: m0 is written anew before it."""
+    """Each of three loads (builtin, base + offset, builtin) goes where it should: m0 is written anew before it; the barrier
+    behind a load from base + offset waits for those before it and for reads of LDS."""
     hipcc = find_hipcc()
     if hipcc is None:
         pytest.skip("no hipcc")
@@ -71,7 +77,11 @@ def test_both_forms_of_the_load_in_one_kernel(tmp_path):
           SHK_LOAD_TO_LDS(at + 512u, threadIdx.x * 16u, reinterpret_cast<const char*>(p + 4096));
           SHK_LOAD_TO_LDS(p + 8192 + threadIdx.x * 4, a);
           SHK_MEET_WITH_LOADS(0);
-          p[threadIdx.x] = a[threadIdx.x];
+          const float x = a[threadIdx.x ^ 1];
+          SHK_LOAD_TO_LDS(at, threadIdx.x * 16u, reinterpret_cast<const char*>(p));
+          SHK_LOAD_TO_LDS(at + 256u, threadIdx.x * 16u, reinterpret_cast<const char*>(p));
+          SHK_MEET_WITH_LOADS(1);
+          p[threadIdx.x] = a[threadIdx.x] + x;
         }
     """)
     out = tmp_path / "both.s"
@@ -87,5 +97,8 @@ def test_both_forms_of_the_load_in_one_kernel(tmp_path):
             last = place
         if load:
             places.append(last)
-            last = None  # (a load leaves m0 as it was, but the next one's place differs)
-    assert places == ["m0, 0", "m0, 0x200", "m0, 0"]
+    assert places == ["m0, 0", "m0, 0x200", "m0, 0", "m0, 0", "m0, 0x100"]
+    lines = [line.strip() for line in body[: body.index("s_endpgm")].splitlines()]
+    lines = [line for line in lines if line and not line.startswith((";", "."))]
+    waits = [lines[i - 1] for i, line in enumerate(lines) if line == "s_barrier"]
+    assert [re.fullmatch(r"s_waitcnt vmcnt\((\d)\) lgkmcnt\(0\)", w).group(1) for w in waits] == ["0", "1"], waits
