@@ -52,7 +52,7 @@ __global__ void __launch_bounds__(8 * kWave) __attribute__((amdgpu_waves_per_eu(
   constexpr int kSide = 4 * DB, kLoads = kSide / 8;  // units of a chunk's keys (and of its values); a wavefront's of each
   constexpr int kRing = 4, kBytes = kSide * 1024;  // chunks; bytes of a chunk's keys
   static_assert(kLoads >= 1 && kSide % 8 == 0, "a wavefront loads whole units");
-  __shared__ u32x4 mem[2 * kRing * kBytes / 16];
+  __shared__ u32x4 mem[(2 * kRing * kBytes + 2 * DB * 1024) / 16];  // keys, values, a tile's values of zero
   const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int col = lane % 32, half = lane / 32;
   const PageDiv pd{page_size, page_magic};
@@ -169,8 +169,11 @@ __global__ void __launch_bounds__(8 * kWave) __attribute__((amdgpu_waves_per_eu(
     }
   };
 
-  bf16x8 weights[2];  // of the tile before, whose values begin at `before`
-  int before = 0;
+  // Of the tile before, whose values begin at `before`.  The first tile's product with it is 0 times 0: with values that are
+  // there, infinities among them, 0 times those would be NaN.
+  bf16x8 weights[2];
+  int before = kRing * kBytes;
+  for (int i = threadIdx.x; i < 2 * DB * kWave; i += 8 * kWave) mem[2 * kRing * kBytes / 16 + i] = u32x4{0, 0, 0, 0};
 #pragma unroll
   for (int e = 0; e < 8; ++e) weights[0][e] = weights[1][e] = static_cast<__bf16>(0.f);
 

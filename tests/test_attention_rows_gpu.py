@@ -89,3 +89,24 @@ def test_sinks_join_the_sum(ops):
                 for out in outs:
                     close(out[at + i, h].double(), (plain[at + i, h].double() * share).cpu(), torch.bfloat16, scale=1.0)
         at += length
+
+
+@pytest.mark.parametrize("heads, kv_heads, head_dim, nsplit, at", [(14, 2, 64, 1, 3), (28, 4, 128, 1, 31), (28, 4, 128, 3, 200), (28, 4, 128, 1, 400)])
+def test_an_infinite_value_is_an_infinite_result_and_no_other(ops, heads, kv_heads, head_dim, nsplit, at, monkeypatch):
+    """One element of the value of a key that every query reads is infinity, in the first tile that a workgroup reads or a
+    later one: each gets infinity for that element, and nothing else changes."""
+    import sys
+
+    element, page_size, seq_lens, starts = 5, 16, [30], [500]
+    plain, _ = run(ops, heads, kv_heads, head_dim, page_size, None, None, nsplit, 0, seq_lens, starts)
+    fill = fill_pools
+
+    def fill_and_spoil(tables, k_pool, v_pool, ctx, page_size):
+        fill(tables, k_pool, v_pool, ctx, page_size)
+        v_pool[int(tables[0, at // page_size]), :, element, at % page_size] = float("inf")
+
+    monkeypatch.setattr(sys.modules[__name__], "fill_pools", fill_and_spoil)
+    got, _ = run(ops, heads, kv_heads, head_dim, page_size, None, None, nsplit, 0, seq_lens, starts)
+    assert bool((got[..., element] == float("inf")).all())
+    others = [e for e in range(head_dim) if e != element]
+    assert torch.equal(got[..., others], plain[..., others])
