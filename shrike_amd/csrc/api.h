@@ -124,7 +124,7 @@ int shk_interleave_gate_up(const void* gate_t, const void* up_t, int m, int k, v
 // `bias` is null or two floats, the gate's constants: with bias[0] > 0 the gate is bounded
 // from above and the other factor from both sides by it before anything else, and bias[1]
 // is added to that factor (as in shk_act_mul).
-// ksplit > 1 (at most 64 rows, float32 output, no bias): the k range is shared
+// ksplit > 1 (float32 output, no bias): the k range is shared
 // by ksplit workgroups per block of weight rows and out is [ksplit][n][m], the
 // partial sums, which the kernel that reads the product adds up in order
 // (shk_add_rmsnorm, shk_rope_kv_store).  shk_gemm_bf16_splits says how many

@@ -1057,10 +1057,13 @@ static int big_shape(int split, int n, int wblocks, int m, int k) {
 
 // Which gemm_direct_kernel serves a product of n > 16 tokens (0: none): the smallest tile of which a launch has no
 // more than the 256 compute units, for matrices of 256 to 2,048 rows (more of them fill the staged kernels' larger
-// tiles), up to 10 MB and rows that are whole 16-byte pieces; in shares of k up to 64 tokens.  Against the staged kernels,
-// product and reading norm, over six widths of 256 to 2,048, k from 128 to 8,192 and 65 to 4,096 tokens: 0.65 to 0.98 of
-// their time with up to 2,048 of k in the two smaller tiles, 0.93 to 1.24 up to 4,864, 1.16 to 1.63 with 8,192; the largest
-// tile 0.91 to 1.0 up to 896 of k and 1.08 to 1.3 from 1,024 on.  (64 x 64 tiles took 1.14 to 1.5 of the staged kernels' time.)
+// tiles), up to 10 MB and rows that are whole 16-byte pieces; in shares of k up to 64 tokens.  Its share of the time
+// of gemm_wide_kernel (with the norm that reads the product) over nine widths of 256 to 2,048, fourteen k of 256 to 12,288 and
+// 65 to 2,048 tokens: 32 x 16 tiles 0.64 to 0.96 up to 3,072 of k, 0.93 to 1.06 at 3,584 and 4,096, 0.98 to 1.14 at 4,864,
+// 1.05 to 1.7 beyond; 32 x 32 tiles 0.71 to 1.0 up to 2,048, 0.95 to 1.14 to 3,072, 1.05 to 1.31 from 3,584 to 4,864, 1.33 to
+// 1.84 beyond; 32 x 64 tiles 0.91 to 0.99 up to 896, 1.05 to 1.15 at 1,280.  More than 64 tokens: up to 960 of k in
+// the largest tile, and up to 4,864 in the others, which is further than they are the faster ones: readers of products of up
+// to that k get them whole, in one float32 part.
 struct DirectTile {
   int rows, tokens, most_k, waves;
 };

@@ -363,6 +363,14 @@ static void launch_f32(const F32Product& p, hipStream_t s) {
                                                p.a_batch, p.w_batch, p.out_batch);
 }
 
+template <int RT, int CT>
+static void launch_f32_lds(const F32Product& p, hipStream_t s) {
+  const int tiles = (p.m + 32 * RT - 1) / (32 * RT) * ((p.n + 32 * CT - 1) / (32 * CT));
+  const int vec_out = p.ldo % 4 == 0 && reinterpret_cast<uintptr_t>(p.out) % 16 == 0;
+  gemm_f32_lds_kernel<RT, CT><<<(tiles + kDies - 1) / kDies * kDies, 4 * kWave, 0, s>>>(p.a, p.w, p.bias, p.out, p.n, p.m, p.k, p.lda,
+                                                                                    p.ldo, p.accumulate, vec_out);
+}
+
 // The shape of the kernel for a size (results are the same bits in all of them).  Measured on the 0.5B
 // model's matrices, tiled weights, microseconds:
 //   up to 16 rows: 896 x 896 5 in one-tile workgroups of 16 segments (9 with four row blocks and four groups of
@@ -372,20 +380,12 @@ static void launch_f32(const F32Product& p, hipStream_t s) {
 //     (32 x 32, 64 x 64: 70 TFLOP/s of the 150 that the instruction reaches alone).  A k of up to 256 is one step
 //     a segment, and a shorter one leaves the later of four groups without any: there a wavefront walks all of k and
 //     four lie side by side along the rows.
+//     1,501 rows: 28 products of 448 x 128 160 us shared by four groups, 77 so
+//     (95 with vector instructions), 14 of 128 x 64 27, 13 (14), 40 of 256 x 192 132, 86 (105), 4864 x 256 73, 55 (66).
 //   tiled weights of a k in whole stages, enough of them: gemm_f32_lds_kernel with 32 features x 64 rows, or 32 x 32 where those
 //     are few and k is short.  9728 x 896 at 64 / 200 / 509 / 1,024 rows 18.8 / 45.7 / 91.8 / 163 (24 / 62.6 / 120.6 / 229.5
 //     without it), 1152 x 896 at 509 / 2,000 18.7 / 43.9 (23.7 / 63.1), 3584 x 3584 at 1,501 325 (414), 896 x 4864 at 1,024 97.7
 //     (100.8), but at 509 (224 workgroups of 32 x 64) 61 against 57, 1152 x 896 at 200 (252 of 32 x 32) 10.7 against 9.3.
-//    1,501 rows: 28 products of 448 x 128 160 us shared by four groups, 77 so
-//     (95 with vector instructions), 14 of 128 x 64 27, 13 (14), 40 of 256 x 192 132, 86 (105), 4864 x 256 73, 55 (66).
-template <int RT, int CT>
-static void launch_f32_lds(const F32Product& p, hipStream_t s) {
-  const int tiles = (p.m + 32 * RT - 1) / (32 * RT) * ((p.n + 32 * CT - 1) / (32 * CT));
-  const int vec_out = p.ldo % 4 == 0 && reinterpret_cast<uintptr_t>(p.out) % 16 == 0;
-  gemm_f32_lds_kernel<RT, CT><<<(tiles + kDies - 1) / kDies * kDies, 4 * kWave, 0, s>>>(p.a, p.w, p.bias, p.out, p.n, p.m, p.k, p.lda,
-                                                                                    p.ldo, p.accumulate, vec_out);
-}
-
 template <bool TILED>
 static void run_f32(const F32Product& p, hipStream_t s) {
   auto tiles = [&](int rows, int cols) {

@@ -39,6 +39,9 @@ struct WideShape {
   static constexpr int kWBytes = kTiles * 1024, kXBytes = kUnits * 1024;
   static constexpr int kLds = kWRing * kWBytes + kXRing * kXBytes;
   static_assert(kWLoads * kWaves == kTiles && 2 * kXLoads * kWaves == kUnits, "loads divide evenly among the wavefronts");
+  // (a load stands behind each of a half's multiplications or reads but the first)
+  static_assert(kWLoads < (RM * RN > RM + RN ? RM * RN : RM + RN) && kXLoads < (RM * RN > RM + RN ? RM * RN : RM + RN),
+                "a half substep has a place for each of its loads");
   static_assert(kLds <= 160 * 1024 && kDepth * (kWLoads + kXLoads) <= 63, "fits LDS and the load counter");
   static_assert(kWaves * 32 * (32 * RM * 4 + 16) <= kLds, "the results of 32 tokens a wavefront fit LDS");
 };

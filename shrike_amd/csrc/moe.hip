@@ -587,23 +587,19 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// The same two products for weights in tiles (k and m multiples of 64): 256 weight rows (gate/up: 128
-// features of each) x 128 pairs a workgroup of eight wavefronts, each 64 x 64, in stages of 64 along k that go
-// from memory straight into LDS (global_load_lds), 1 KiB a load: a weight tile of 16 rows x 32, which
-// is the matrix instruction's operand as it lies, or 8 pairs' rows x 128 bytes, whole cache lines, gathered on
-// the way since a lane gives its own address.  Three stage buffers: two stages' loads are in flight while one is
-// multiplied, one barrier a stage.  Lane l of a pairs' load brings chunk l / 8 (of 8 elements) of row l % 8;
-// the operand of step ks takes rows j from unit j / 8 at place j % 8 + 8 * (kg + 4 ks): eight lanes read 128
-// consecutive bytes.
+// The same two products for weights in tiles (k and m multiples of 64): wide_loop() of gemm_wide.h over a tile of weight rows (gate/up:
+// half of them of each) x pairs, 256 x 128, 256 x 192 or 128 x 192.  A unit of the loop's activations is 8 pairs' rows
+// x 128 bytes, gathered on the way into LDS, since a lane gives its own address.
 // The grid is one row of workgroups and the lists' lengths are only known on the device: workgroup p takes the
 // p / 8-th tile of die p % 8's share of all live tiles, counted expert by expert, features outside, the
 // expert's pairs inside, so that the 32 compute units of a die read a matrix from memory once and its pairs'
 // rows stay in the die's L2.
-// 1,501 tokens, two of eight experts of 4736 features and width 3584: gate/up 360 us and down 227 in the
-// kernel above, 262 and 157 here; with row-major weights (8 rows x 128 bytes a load) this kernel
-// took 350 and 213, through registers 449 and 276: what it waits for is memory that is read 128 bytes at a time.
-// Pairs' rows laid out in tiles first (19 us a layer) changed nothing, nor did leaving out the multiplications
-// for the empty half of a list's last tile: the loads are what takes the time, about 42 GB/s a compute unit.
+// What bounds it: as the loop, the multiplications' power limit, and the pairs that a list's last tile lacks.  1,501 tokens, two of
+// eight experts of 4736 features and width 3584: gate/up 232 us, down 101 (262 and 157 with 16 x 16 multiplications and
+// a pair's row per lane; 360 and 227 in the kernel above; with row-major weights that loop took 350 and 213).  Pairs'
+// rows laid out in tiles first (19 us a layer) changed nothing, nor did leaving out the multiplications
+// for the empty half of a list's last tile.
+
 // Tile `index` of all experts' live tiles (features x ceil(count / PAIRS) each): expert, first feature
 // tile, first pair; false beyond the last.  `index` < 0 asks for none and returns their number in `total`.
 template <int PAIRS>

@@ -1,4 +1,4 @@
-"""Experts' products in tiles of 256 weight rows x 128 pairs: lists of no pair, one, a whole tile and one
+"""Experts' products in tiles of 128 or 256 weight rows x 128 or 192 pairs: lists of no pair, one, a whole tile and one
 more, features that end within a tile, every form of expert, against float64."""
 
 import pytest
