@@ -108,6 +108,17 @@ inline unsigned big_grid(int tiles_x, int tiles_y, int tile_rows, int tile_token
   return static_cast<unsigned>(tiles_x * tiles_y);
 }
 
+// Weight rows and tokens that the tiles of each die need, summed over the dies, where the tiles are taken in plain order (every
+// eighth one on a die); 0 in the other orders, whose dies share.
+inline double big_operands(int tiles_x, int tiles_y, int tile_rows, int tile_tokens) {
+  int by_die;
+  big_grid(tiles_x, tiles_y, tile_rows, tile_tokens, &by_die);
+  if (by_die) return 0.0;
+  const double tiles = static_cast<double>(tiles_x) * tiles_y, dies = tiles < kDies ? tiles : kDies, each = tiles / dies;
+  const int columns = tiles_x / (tiles_x % 4 == 0 ? 4 : tiles_x % 2 == 0 ? 2 : 1);  // of tiles that a die meets
+  return dies * ((each < columns ? each : columns) * tile_rows + (each < tiles_y ? each : tiles_y) * tile_tokens);
+}
+
 // Products of more than 64 tokens whose activations are 16-byte aligned with k % 8 == 0 (gemm_wide.hip).
 int wide_splits(int n, int m, int k, int whole_bytes);
 int wide_parts(int n, int m, int k, int gated);

@@ -9,6 +9,7 @@
 #include "gemm_bf16.h"
 #include "gemm_wide.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace shk {
@@ -165,9 +166,21 @@ __global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per
   }
 }
 
+// The least time that the dies' fetches take, at 7 TB/s, where tiles are taken in plain order (big_grid): each die then needs most
+// operands of every share.  896 x 18944 at 2,048 tokens with its norm: 128 us in three shares of 128 x 192 tiles (8.4 MB a stage),
+// which wide_time() alone prefers, 75 in four of 128 x 256.  One or two rows of tiles read their weights as often in any order; with
+// less than 8,192 of k the shares' start and end weigh more (896 x 4864 at 1,119 tokens in a prompt: 25 us in the three
+// shares of 128 x 128 without this, 31 in the two of 128 x 192 that it would take).
+static double wide_fetch(const WideTile& t, int n, int wblocks, int k) {
+  const int tiles_x = (wblocks * 16 + t.rows - 1) / t.rows, tiles_y = (n + t.tokens - 1) / t.tokens;
+  if (tiles_y <= 2 || k < 8192) return 0.0;
+  return 2.0 + t.ends + ((k + 63) / 64) * 128.0 * big_operands(tiles_x, tiles_y, t.rows, t.tokens) / 7e6;
+}
+
 static double wide_estimate(const WideTile& t, int split, int n, int wblocks, int k) {
   const long long groups = static_cast<long long>((wblocks * 16 + t.rows - 1) / t.rows) * ((n + t.tokens - 1) / t.tokens) * split;
-  return wide_time(t, static_cast<double>(groups), ((k + 63) / 64 + split - 1) / split);
+  const double us = wide_time(t, static_cast<double>(groups), ((k + 63) / 64 + split - 1) / split);
+  return split > 1 ? std::max(us, wide_fetch(t, n, wblocks, k)) : us;
 }
 
 // The tile of the least estimate.
@@ -214,7 +227,8 @@ int wide_splits(int n, int m, int k, int whole_bytes) {
   const int most = ktiles / 16 < 16 ? ktiles / 16 : 16;
   int best = 1;
   double least;
-  wide_plan(1, n, mblocks, k, &least);
+  const WidePlan whole = wide_plan(1, n, mblocks, k, &least);
+  if (!whole.main_blocks) least = std::max(least, wide_fetch(kWide[whole.tile], counted_tokens(n), mblocks, k));
   const double values = static_cast<double>(counted_tokens(n)) * m;
   least += 2.0 * values * whole_bytes / 3e6;
   for (int split = 2; split <= most; ++split) {
