@@ -16,11 +16,12 @@
 //
 // What bounds it: the vector units' issue, about 170 instructions a wavefront and tile, 64 of them the rescaling of o in
 // every tile (a branch around it costs as much in copies), beside 16 multiplications: the matrix units are busy 40 % of
-// the time.  Weights relative to a reference that rarely moves would need no rescaling (118 us instead of 137 for 512
+// the time.  Weights relative to a reference that rarely moves would need no rescaling (118 us where this kernel took 137, 512
 // queries at 12,001), but are a tenth less exact: the largest would no longer be 1.
-// Against the kernel with 16 queries a wavefront, which reads every operand from LDS twice as often: 28 heads over 4, 512
-// queries at 12,001 167 us -> 137, at 31,000 341 -> 287, at 3,584 63 -> 57, at 1,536 42 -> 41, at 0 21 -> 26 (fewer,
-// longer workgroups); 4,096 from 0 183 -> 154, 2,048 76 -> 79.  The bits are the same with the same shares.
+// Against the kernel with 16 queries a wavefront, which reads every operand from LDS twice as often, 28 heads over 4: 512
+// queries at 12,001 148 us -> 123 alone and 156 -> 144 a layer in a model's pass; alone, at 31,000 335 -> 279, at 3,584 61 -> 55, at
+// 1,536 40 -> 40, at 0 21 -> 25 (fewer, longer workgroups); 4,096 from 0 183 -> 151, 2,048 69 -> 74.  Where portions fill few
+// of a workgroup's rows it loses (64 of 8 queries at 2,000: 60 -> 80).  The bits are the same with the same shares.
 #include "attention_rows.h"
 #include "gemm_wide.h"
 #include "mfma_tile.h"

@@ -3,9 +3,10 @@
 //
 // The results leave through LDS in whole 16-byte pieces along the rows, by straight-line code without a branch per
 // value: 2 to 5 us a workgroup, 20 to 30 where every value was tested and stored for itself.
-// Against the kernel before (16 wavefronts, tiles of 16 x 16, 256 x 256, 256 x 128 and 128 x 128): 7B QKV at 2,048
-// tokens 101 us -> 62, output 67 -> 49, gate/up 500 -> 443 (1.26 PFLOP/s), down 276 -> 235; at 512 tokens QKV 45 -> 25, down
-// 121 -> 74, the 14B QKV 65 -> 42, output 61 -> 34, gate/up 169 -> 130, down 98 -> 69.
+// Against the kernel before (16 wavefronts, tiles of 16 x 16, 256 x 256, 256 x 128 and 128 x 128), both in the passes of whole models on
+// one card: 7B at 2,048 tokens QKV 100 us -> 72, output and down 168 -> 146 on average, gate/up 507 -> 462 (1.20 PFLOP/s); at 512
+// QKV 46 -> 26, output 33 -> 25, gate/up 156 -> 133 (two launches), down 104 -> 78; 14B at 512 QKV 64 -> 60, output and down
+// 72 -> 58, gate/up 156 -> 126.  Alone, replayed on the same operands, a product takes 2 to 10 % less.
 #include "gemm_bf16.h"
 #include "gemm_wide.h"
 

@@ -169,7 +169,7 @@ def portion_splits(workgroups: int, mean_keys: int) -> int:
 
 
 # Keys that a query reads on average from which the prompt kernel with 32 rows a wavefront (small == 2) is looked at: 28 heads
-# over 4, 512 queries at 1,536 42 us -> 41, at 0 21 -> 26.
+# over 4, 512 queries at 1,536 40 us -> 40, at 0 21 -> 25.
 ROWS_FROM_KEYS = 1800
 
 # What a launch of the prompt kernels takes, by AttentionPlan.small, in us: to start and end, then for heads of 128 (64: 0.7 of
