@@ -2,7 +2,9 @@
 // of gemm_wide.h in eight tile sizes.
 //
 // The results leave through LDS in whole 16-byte pieces along the rows, by straight-line code without a branch per
-// value: 2 to 5 us a workgroup, 20 to 30 where every value was tested and stored for itself.
+// value: 2 to 5 us a workgroup, 20 to 30 where every value was tested and stored for itself.  Other epilogues and rows that are no
+// whole pieces finish eight rows at a time: 4864 x 896 at 1,119 tokens with bounded gates 33 us in the kernel before, 46 one value at a
+// time, 29 so; 4737 x 896 at 2,048 47, 63, 36; added to 9472 x 3584 float32 results at 2,048 199, 256, 142.
 // Against the kernel before (16 wavefronts, tiles of 16 x 16, 256 x 256, 256 x 128 and 128 x 128), both in the passes of whole models on
 // one card: 7B at 2,048 tokens QKV 100 us -> 72, output and down 168 -> 146 on average, gate/up 507 -> 462 (1.20 PFLOP/s); at 512
 // QKV 46 -> 26, output 33 -> 25, gate/up 156 -> 133 (two launches), down 104 -> 78; 14B at 512 QKV 64 -> 60, output and down
@@ -15,10 +17,12 @@
 
 namespace shk {
 
-template <int GM, int GN, int RM, int RN, bool GATED>
+// WHOLE: rows in whole 16-byte pieces and at most a bias or SiLU's gate, finished in registers.  Anything else is a kernel of its
+// own, which keeps both short.  pieces: its results leave in 16-byte pieces too.
+template <int GM, int GN, int RM, int RN, bool GATED, bool WHOLE>
 __global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per_eu(GM * GN / 4, GM * GN / 4)))
     gemm_wide_kernel(const bf16* __restrict__ a, int lda, int n, int k, const uint4* __restrict__ wt, int ktiles, int m,
-                     const float* __restrict__ bias, void* __restrict__ out, int ldo, int out_f32, int accumulate, int whole,
+                     const float* __restrict__ bias, void* __restrict__ out, int ldo, int out_f32, int accumulate, int pieces,
                      int ksplit, int tiles_x, int tiles_y, int by_die) {
   using S = WideShape<GM, GN, RM, RN>;
   constexpr int WL = S::kWLoads, XL = S::kXLoads;
@@ -76,10 +80,20 @@ __global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per
   const size_t plane = static_cast<size_t>(blockIdx.y) * n;
   if (row0 >= m) return;  // (no barrier follows)
   char* mine = reinterpret_cast<char*>(&mem[0]) + wave * (32 * (32 * RM * 4 + 16));
-  if (whole) {
-    // Rows in whole 16-byte pieces and at most a bias or SiLU's gate: finished in registers.
-    auto finish = [&](auto f32) {
-      constexpr bool F32 = decltype(f32)::value;
+  if constexpr (WHOLE) {
+    auto finish = [&](auto f32, auto biased) {
+      constexpr bool F32 = decltype(f32)::value, BIASED = decltype(biased)::value;
+      // (asked for together: one by one, each group of rows waits for its own)
+      f32x4 add[RM][4];
+      if constexpr (BIASED) {
+#pragma unroll
+        for (int i = 0; i < RM; ++i)
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            const int row = row0 + 32 * i + g * 8 + half * 4;
+            add[i][g] = *reinterpret_cast<const f32x4*>(bias + (row < m ? row : m - 4));
+          }
+      }
       constexpr int E = F32 ? 4 : 2, kPitch = kRows * E + 16, kPieces = kRows * E / 16;
       auto put = [&](const f32x16 (&c)[RN], int jn, int i) {
 #pragma unroll
@@ -89,11 +103,7 @@ __global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per
 #pragma unroll
           for (int r = 0; r < 4; ++r)
             v[r] = GATED ? gate_times_up(c[jn][g * 4 + r], c[jn][(GATED ? 8 : 0) + g * 4 + r], kActSilu, nullptr) : c[jn][g * 4 + r];
-          if (!GATED && bias && row0 + row < m) {
-            const f32x4 b = *reinterpret_cast<const f32x4*>(bias + row0 + row);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) v[r] += b[r];
-          }
+          if constexpr (BIASED) v += add[i][g];
           if constexpr (F32) {
             *reinterpret_cast<f32x4*>(mine + j * kPitch + row * 4) = v;
           } else {
@@ -121,14 +131,23 @@ __global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per
         SHK_LDS_DONE();
       }
     };
+    auto leave = [&](auto f32) {
+      if (!GATED && bias)
+        finish(f32, std::bool_constant<!GATED>{});
+      else
+        finish(f32, std::false_type{});
+    };
     if (out_f32)
-      finish(std::true_type{});
+      leave(std::true_type{});
     else
-      finish(std::false_type{});
+      leave(std::false_type{});
     return;
   }
-  // Anything else: the sums go through LDS as they are, and a loop of single values finishes them.
+  // Anything else: the sums go through LDS as they are; a lane finishes eight neighbouring rows of a token at a time, so that
+  // what is the same for all of them is asked once, and stores them as 16-byte pieces where rows allow.  Others go
+  // back to their place and leave as single values, neighbouring lanes on neighbouring rows.
   constexpr int kPitch = 32 * RM * 4 + 16;
+  auto place = [&](int t, int p) { return reinterpret_cast<float*>(mine + t * kPitch) + (GATED ? p / 16 * 32 + p % 16 : p); };
   auto put = [&](const f32x16 (&c)[RN], int jn, int i) {
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
@@ -136,6 +155,48 @@ __global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per
 #pragma unroll
       for (int r = 0; r < 4; ++r) v[r] = c[jn][g * 4 + r];
       *reinterpret_cast<f32x4*>(mine + j * kPitch + (i * 32 + g * 8 + half * 4) * 4) = v;
+    }
+  };
+  const int done = pieces ? m & ~7 : 0;  // rows below it leave in pieces
+  const float limit = GATED && bias ? bias[0] : 0.f, shift = GATED && bias ? bias[1] : 0.f;
+  const bool near_bias = reinterpret_cast<uintptr_t>(bias) % 16 == 0;
+  auto finish = [&](float (&v)[8], const float (&u)[8], int row) {
+    if constexpr (GATED) {
+      float g[8], f[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        g[e] = v[e], f[e] = u[e];
+        if (limit > 0.f) g[e] = fminf(g[e], limit), f[e] = fminf(fmaxf(f[e], -limit), limit);
+        if (bias) f[e] += shift;
+      }
+      auto all = [&](auto act) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = gate_times_up(g[e], f[e], decltype(act)::value, nullptr);
+      };
+      if (accumulate == kActSilu)
+        all(std::integral_constant<int, kActSilu>{});
+      else if (accumulate == kActGeluTanh)
+        all(std::integral_constant<int, kActGeluTanh>{});
+      else if (accumulate == kActRelu)
+        all(std::integral_constant<int, kActRelu>{});
+      else
+        all(std::integral_constant<int, kActQuickGelu>{});
+    } else {
+      if (bias && row + 8 <= m && near_bias) {
+        const f32x4 lo = *reinterpret_cast<const f32x4*>(bias + row), hi = *reinterpret_cast<const f32x4*>(bias + row + 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] += lo[e], v[4 + e] += hi[e];
+      } else if (bias) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] += bias[row + e < m ? row + e : m - 1];
+      }
+      if (accumulate == kPlainReluSquared) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = plain_act(v[e], kPlainReluSquared, row + e);
+      } else if (accumulate >= kPlainSiluRows && row < accumulate / kPlainSiluRows) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = plain_act(v[e], accumulate, row + e);
+      }
     }
   };
 #pragma unroll
@@ -146,21 +207,57 @@ __global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per
     if constexpr (RM > 3) put(acc[3], jn, 3);
     SHK_LDS_DONE();
 #pragma unroll 1
-    for (int at = lane; at < 32 * kRows; at += kWave) {
-      const int t = at / kRows, p = at % kRows, token = tok + jn * 32 + t, row = row0 + p;
+    for (int at = lane; at < 4 * kRows; at += kWave) {
+      const int t = at / (kRows / 8), p = at % (kRows / 8) * 8, token = tok + jn * 32 + t, row = row0 + p;
       if (token >= n || row >= m) continue;
-      const float* sums = reinterpret_cast<const float*>(mine + t * kPitch);
+      f32x4* from = reinterpret_cast<f32x4*>(place(t, p));
+      const f32x4 lo = from[0], hi = from[1];
+      float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]}, u[8] = {};
+      if constexpr (GATED) {
+        const f32x4 ulo = from[4], uhi = from[5];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) u[e] = ulo[e], u[4 + e] = uhi[e];
+      }
+      finish(v, u, row);
       const size_t idx = (plane + token) * ldo + row;
-      float v;
-      if (GATED)
-        v = gate_times_up(sums[p / 16 * 32 + p % 16], sums[p / 16 * 32 + 16 + p % 16], accumulate, bias);
-      else
-        v = plain_act(sums[p] + (bias ? bias[row] : 0.f), accumulate, row);
-      if (out_f32) {
-        float* o = static_cast<float*>(out) + idx;
-        *o = (accumulate == 1 && !GATED) ? *o + v : v;
+      if (row >= done) {
+        from[0] = f32x4{v[0], v[1], v[2], v[3]}, from[1] = f32x4{v[4], v[5], v[6], v[7]};
+      } else if (out_f32) {
+        f32x4* o = reinterpret_cast<f32x4*>(static_cast<float*>(out) + idx);
+        f32x4 x = {v[0], v[1], v[2], v[3]}, y = {v[4], v[5], v[6], v[7]};
+        if (accumulate == 1 && !GATED) x = o[0] + x, y = o[1] + y;
+        o[0] = x, o[1] = y;
       } else {
-        static_cast<bf16*>(out)[idx] = from_float<bf16>(v);
+        bf16x8 o;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = static_cast<__bf16>(v[e]);
+        *reinterpret_cast<bf16x8*>(static_cast<bf16*>(out) + idx) = o;
+      }
+    }
+    SHK_LDS_DONE();
+    const int tokens = n - (tok + jn * 32) < 32 ? n - (tok + jn * 32) : 32;
+    if (row0 + kRows > done && done < m) {
+#pragma unroll
+      for (int q = 0; q < (kRows + kWave - 1) / kWave; ++q) {
+        const int p = q * kWave + lane, row = row0 + p;
+        if (p >= kRows || row < done || row >= m) continue;
+        const float* from = place(0, p);
+        const size_t idx = (plane + tok + jn * 32) * ldo + row;
+        auto leave = [&](auto* o, auto added) {
+#pragma unroll 8
+          for (int t = 0; t < tokens; ++t, o += ldo, from += kPitch / 4) {
+            if constexpr (decltype(added)::value)
+              *o = *o + *from;
+            else
+              *o = from_float<std::remove_pointer_t<decltype(o)>>(*from);
+          }
+        };
+        if (!out_f32)
+          leave(static_cast<bf16*>(out) + idx, std::false_type{});
+        else if (accumulate == 1 && !GATED)
+          leave(static_cast<float*>(out) + idx, std::true_type{});
+        else
+          leave(static_cast<float*>(out) + idx, std::false_type{});
       }
     }
     SHK_LDS_DONE();
@@ -266,15 +363,14 @@ static void launch_wide(hipStream_t s, const bf16* a, int lda, int n, int k, con
   int by_die;
   const unsigned groups = big_grid(tiles_x, tiles_y, 16 * S::kTiles, 32 * GN * RN, &by_die);
   const int per = out_f32 ? 4 : 8;  // values of 16 bytes
-  const int whole = m % per == 0 && ldo % per == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0 &&
-                    reinterpret_cast<uintptr_t>(bias) % 16 == 0 && (gated ? accumulate == kActSilu && !bias : accumulate == 0);
+  const int pieces = ldo % per == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
+  const bool whole = pieces && m % per == 0 && reinterpret_cast<uintptr_t>(bias) % 16 == 0 &&
+                     (gated ? accumulate == kActSilu && !bias : accumulate == 0);
   const int ktiles = (k + 31) / 32;
-  if (gated)
-    gemm_wide_kernel<GM, GN, RM, RN, true><<<dim3(groups, ksplit), S::kWaves * kWave, 0, s>>>(
-        a, lda, n, k, wt, ktiles, m, bias, out, ldo, out_f32, accumulate, whole, ksplit, tiles_x, tiles_y, by_die);
-  else
-    gemm_wide_kernel<GM, GN, RM, RN, false><<<dim3(groups, ksplit), S::kWaves * kWave, 0, s>>>(
-        a, lda, n, k, wt, ktiles, m, bias, out, ldo, out_f32, accumulate, whole, ksplit, tiles_x, tiles_y, by_die);
+  const auto kernel = gated ? (whole ? gemm_wide_kernel<GM, GN, RM, RN, true, true> : gemm_wide_kernel<GM, GN, RM, RN, true, false>)
+                            : (whole ? gemm_wide_kernel<GM, GN, RM, RN, false, true> : gemm_wide_kernel<GM, GN, RM, RN, false, false>);
+  kernel<<<dim3(groups, ksplit), S::kWaves * kWave, 0, s>>>(a, lda, n, k, wt, ktiles, m, bias, out, ldo, out_f32, accumulate, pieces,
+                                                            ksplit, tiles_x, tiles_y, by_die);
 }
 
 void wide_product(hipStream_t s, const bf16* a, int lda, int n, int k, const uint4* wt, int m, const float* bias, void* out,

@@ -222,3 +222,45 @@ def test_rows_that_are_not_aligned(ops, n, m, k, gated, apart):
     parts = torch.full((3, n, m), float("nan"), device="cuda")
     ops.gemm_tiled_weight(rows, wt, m, k, parts, splits=3)
     check(parts.sum(0), first, 2 * k)
+
+
+@pytest.mark.parametrize("m", [2312, 2308, 2311])  # whole pieces, half a piece left, rows that begin anywhere
+@pytest.mark.parametrize("n, k", [(70, 136), (513, 520)])
+def test_results_are_the_same_bits_however_they_leave(ops, n, m, k):
+    """In pieces straight from registers, in pieces behind the loop that finishes them, as single values."""
+    x, (g, u) = operands(n, m, k, matrices=2)
+    pair, plain = ops.interleave_gate_up(g, u), ops.retile_weight(g)
+    wide, odd = (torch.full((n, m + extra), 3.0, device="cuda", dtype=BF16) for extra in (-m % 8 + 8, 8 + (m + 1) % 2))
+    bias = torch.randn(m + 1, device="cuda")
+    a, b = x.double() @ g.double().T, x.double() @ u.double().T
+    gates = {"silu": lambda v: v * torch.sigmoid(v), "gelu_tanh": lambda v: torch.nn.functional.gelu(v, approximate="tanh"),
+             "relu": torch.relu, "quick_gelu": lambda v: v * torch.sigmoid(1.702 * v)}
+
+    def same(want, bound, **how):
+        outs = []
+        for rows in (torch.empty(n, m, device="cuda", dtype=BF16), wide[:, :m], odd[:, 4 : m + 4]):
+            rows.fill_(float("nan"))
+            ops.gemm_tiled_weight(x, pair if "gated" in how else plain, m, k, rows, **how)
+            outs.append(rows)
+        check(outs[0], want, bound)
+        assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+        assert (wide[:, m:] == 3).all() and (odd[:, :4] == 3).all() and (odd[:, m + 4 :] == 3).all()
+
+    for name, act in gates.items():
+        same(act(a) * b, 4 * k, gated=name)
+        limit = torch.tensor([0.25, 0.0], device="cuda")
+        same(act(a.clamp(max=0.25)) * b.clamp(-0.25, 0.25), 4 * k, gated=name, gate_args=limit)
+        same(act(a) * (b + 1.5), 4 * k, gated=name, gate_args=torch.tensor([0.0, 1.5], device="cuda"))
+    for shift in (0, 1):  # (a bias that is and is not 16-byte aligned)
+        add = bias[shift : shift + m]
+        same(a + add.double(), k, bias=add)
+        same((a + add.double()).relu().square(), 4 * k, bias=add, activation="relu_squared")
+    same(torch.cat([gates["silu"](a[:, :1003]), a[:, 1003:]], 1), 2 * k, activation=("silu", 1003))
+    sums = []
+    for rows in (torch.empty(n, m, device="cuda"), torch.empty(n, m + 6 + (m + 1) % 2, device="cuda")[:, 2 : m + 2]):
+        rows.fill_(2.0)
+        ops.gemm_tiled_weight(x, plain, m, k, rows, accumulate=True)
+        ops.gemm_tiled_weight(x, plain, m, k, rows, bias=bias[:m], accumulate=True)
+        sums.append(rows)
+    check(sums[0], 2 * a + 2.0 + bias[:m].double(), 2 * k)
+    assert torch.equal(*sums)
