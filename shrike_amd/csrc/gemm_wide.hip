@@ -6,8 +6,8 @@
 // whole pieces finish eight rows at a time: 4864 x 896 at 1,119 tokens with bounded gates 33 us in the kernel before, 46 one value at a
 // time, 29 so; 4737 x 896 at 2,048 47, 63, 36; added to 9472 x 3584 float32 results at 2,048 199, 256, 142.
 // Against the kernel before (16 wavefronts, tiles of 16 x 16, 256 x 256, 256 x 128 and 128 x 128), both in the passes of whole models on
-// one card: 7B at 2,048 tokens QKV 100 us -> 72, output and down 168 -> 146 on average, gate/up 507 -> 462 (1.20 PFLOP/s); at 512
-// QKV 46 -> 26, output 33 -> 25, gate/up 156 -> 133 (two launches), down 104 -> 78; 14B at 512 QKV 64 -> 60, output and down
+// one card: 7B at 2,048 tokens QKV 100 us -> 67, output and down 168 -> 146 on average, gate/up 507 -> 462 (1.20 PFLOP/s); at 512
+// QKV 46 -> 26, output 33 -> 25, gate/up 156 -> 133 (two launches), down 104 -> 78; 14B at 512 QKV 64 -> 58, output and down
 // 72 -> 58, gate/up 156 -> 126.  Alone, replayed on the same operands, a product takes 2 to 10 % less.
 #include "gemm_bf16.h"
 #include "gemm_wide.h"
