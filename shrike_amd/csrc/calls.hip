@@ -67,6 +67,9 @@ const Launcher kLaunchers[] = {
     SHK_LAUNCHER(shk_gemm),
     SHK_LAUNCHER(shk_gemm_f32_tiled_weight),
     SHK_LAUNCHER(shk_gemm_bf16_tiled_weight),
+    SHK_LAUNCHER(shk_few_stream),
+    SHK_LAUNCHER(shk_few_gated),
+    SHK_LAUNCHER(shk_few_heads),
     SHK_LAUNCHER(shk_rope_kv_store),
     SHK_LAUNCHER(shk_attention),
     SHK_LAUNCHER(shk_attention_decode_bf16),

@@ -1,0 +1,425 @@
+// Products of up to 16 tokens that finish what the kernels between two products would do, so that a decode step has
+// fewer dependent kernels: five a layer instead of eight.  A step of a small model is a chain of kernels of 2.5 to 6 us each,
+// most of which start, wait for memory once and end (weights already in the caches make the 7B output projection 6.3 us
+// instead of 6.8).
+//
+// An output or down projection (few_stream) adds its result to the float32 residual stream and leaves the stream times
+// the next norm's weight in bfloat16, with the sums of squares of every workgroup's rows beside it.  The product
+// that reads those rows multiplies its sums by 1 / rms at the end: rsqrt(mean(x^2) + eps) is the same for a whole row,
+// and W (x w) / rms = W (x w / rms).  So the norm between two products is no kernel of its own, and nobody waits for
+// a row to be whole before multiplying.  (Forming the norm at the head of every workgroup of the next product was
+// slower than the kernel it replaced.)
+// A query/key/value projection (few_heads) rotates what it has formed and writes keys and values into their pages.
+//
+// Rows travel between these kernels as [k / 8][n][8]: sixteen neighbouring lanes of a matrix operand then read
+// neighbouring pieces of 16 bytes, where rows of their own would cost a cache line a lane (896 x 4864 at 16 tokens 9.6 us,
+// 7.8 so; 3584 x 18944 at 8 tokens 25.7, 23.2).
+//
+// Weights cold, chains of one kind of call, us at 1 / 8 / 16 tokens.  Product and norm against few_stream: 896 x 896
+// 5.6 / 6.0 / 6.4 -> 3.0 / 3.3 / 3.6, 896 x 4864 6.9 / 7.3 / 7.5 -> 6.0 / 6.0 / 6.7, 3584 x 3584 9.6 / 9.5 / 10.4 -> 6.1 / 7.4 / 8.3,
+// 3584 x 18944 26.4 / 26.7 / 29.6 -> 21.9 / 24.1 / 27.0.  Projections, rotation and cache write against few_heads: 1152 x 896
+// 5.5 / 6.1 / 6.4 -> 4.1 / 4.3 / 4.4, 4608 x 3584 10.7 / 11.1 / 12.2 -> 10.4 / 11.2 / 12.3, 7168 x 5120 16.4 / 16.2 / 18.2 -> 14.2 / 15.4 /
+// 17.2.  few_gated against the product without the division: 9728 x 896 5.6 / 6.2 / 6.9 -> 5.9 / 6.1 / 6.4, 37888 x 3584 40.6 /
+// 40.6 / 45.1 -> 40.9 / 40.9 / 42.1.  Steps: 0.5B at 1 / 4 / 16 sequences 755 / 814 / 917 -> 653 / 692 / 757, 7B at 1 / 8 / 16
+// 2,883 / 3,174 / 3,366 -> 2,686 / 3,000 / 3,158.
+#include <type_traits>
+
+#include "gemm_bf16.h"
+
+namespace shk {
+
+// Rows of up to 16 tokens: piece `col` (a multiple of 8) of a token lies at token * token_step + col * col_step.
+struct FewRows {
+  const bf16* a;
+  int token_step, col_step, n, k;
+};
+
+// What divides them: the squares' sums [count][n], null for rows that are normed already.
+struct FewScale {
+  const float* sums;
+  int count;
+  float inv_width, eps;
+};
+
+// A thread adds up every (threads / 16)th sum of one token.  They are asked for before the weights, all at once ...
+template <int LOADS>
+struct FewSquares {
+  float v[LOADS > 0 ? LOADS : 1];
+  __device__ __forceinline__ void load(const FewScale& s, int n) {
+    const int token = threadIdx.x % 16, first = threadIdx.x / 16, step = blockDim.x / 16;
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      const int c = first + i * step;
+      const float x = s.sums[static_cast<size_t>(c < s.count ? c : 0) * n + (token < n ? token : 0)];
+      v[i] = c < s.count ? x : 0.f;
+    }
+  }
+  // ... and left by wavefront while the weights travel
+  __device__ __forceinline__ void leave(float* part) {
+    float t = 0.f;
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) t += v[i];
+    t += __shfl_xor(t, 16, kWave);
+    t += __shfl_xor(t, 32, kWave);
+    if (threadIdx.x % kWave < 16) part[threadIdx.x / kWave * 16 + threadIdx.x % kWave] = t;
+  }
+  __device__ __forceinline__ float scale(const FewScale& s, const float* part, int token, int waves) const {
+    if (LOADS == 0) return 1.f;
+    float t = 0.f;
+    for (int w = 0; w < waves; ++w) t += part[w * 16 + token];
+    return rsqrtf(t * s.inv_width + s.eps);
+  }
+};
+
+// A wavefront asks for everything before it waits for anything: its k-tiles at once where they fit its registers.
+// acc += the wavefront's k-tiles (wave, wave + waves, ...) of RB blocks of 16 weight rows by up to 16 tokens.  wrow[]: the lane's
+// weight row at its piece of the first tile.  C > 0: a wavefront has at most C tiles, which are all asked for at once;
+// C = 0: batches of B tiles, two in flight.  Addresses are clamped into the matrices and what lies beyond k is
+// zeroed when it is used: no load stands under a condition.
+template <int C, int B, int RB, typename Between>
+__device__ __forceinline__ void few_multiply(f32x4 (&acc)[RB], const u32x4* const (&wrow)[RB], const FewRows& x, int ktiles, int wave,
+                                             int waves, Between between) {
+  const int lane = threadIdx.x % kWave, j = lane % 16, kg = lane / 16;
+  const bf16* arow = x.a + static_cast<size_t>(j < x.n ? j : x.n - 1) * x.token_step;
+  constexpr int kTiles = C > 0 ? C : B;
+  struct Batch {
+    u32x4 w[kTiles][RB], x[kTiles];
+    uint32_t keep[kTiles];
+  };
+  auto load = [&](Batch& b, int t) {
+#pragma unroll
+    for (int u = 0; u < kTiles; ++u) {
+      const int tt = t + u * waves, col = tt * 32 + kg * 8;
+#pragma unroll
+      for (int r = 0; r < RB; ++r)
+        b.w[u][r] = __builtin_nontemporal_load(wrow[r] + static_cast<size_t>(tt < ktiles ? tt : ktiles - 1) * kWave);
+      const bool inside = col < x.k;
+      b.keep[u] = inside ? ~0u : 0u;
+      b.x[u] = *reinterpret_cast<const u32x4*>(arow + (inside ? static_cast<size_t>(col) * x.col_step : 0));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto multiply = [&](const Batch& b) {
+#pragma unroll
+    for (int u = 0; u < kTiles; ++u) {
+      const u32x4 v = b.x[u] & b.keep[u];
+#pragma unroll
+      for (int r = 0; r < RB; ++r)
+        acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, b.w[u][r]), __builtin_bit_cast(bf16x8, v),
+                                                         acc[r], 0, 0, 0);
+    }
+  };
+#pragma unroll
+  for (int r = 0; r < RB; ++r) acc[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+  Batch ping;
+  load(ping, wave);
+  if constexpr (C > 0) {
+    between();
+    multiply(ping);
+  } else {
+    Batch pong;
+    const int step = B * waves, batches = (ktiles + step - 1) / step;
+    load(pong, wave + step);
+    between();
+    int b = 0;
+    for (; b + 3 < batches; b += 2) {
+      multiply(ping);
+      load(ping, wave + (b + 2) * step);
+      multiply(pong);
+      load(pong, wave + (b + 3) * step);
+    }
+    multiply(ping);
+    if (b + 2 < batches) {
+      load(ping, wave + (b + 2) * step);
+      multiply(pong);
+      multiply(ping);
+    } else {
+      multiply(pong);
+    }
+  }
+}
+
+constexpr int kFewWaves = 9;  // wavefronts of a workgroup at most
+constexpr int kFewTiles = 10, kFewPairs = 7;  // k-tiles of a wavefront that are held at once: of one block of weight rows, of two
+
+// Element (row, token) of the 16 x 16 results that `waves` wavefronts have left in LDS, added in their order.
+__device__ __forceinline__ float few_sum(const f32x4* red, int stride, int row, int token, int waves) {
+  const float* p = reinterpret_cast<const float*>(red + row / 4 * 16 + token) + row % 4;
+  float v = 0.f;
+#pragma unroll 4
+  for (int w = 0; w < waves; ++w) v += p[static_cast<size_t>(w) * stride * 4];
+  return v;
+}
+
+// ROWS = 16: a workgroup for a block of 16 weight rows.  ROWS = 8: for half of one (a tile's pieces of 8 rows are whole
+// lines of 128 bytes), where whole blocks leave compute units idle; the other half of the matrix instruction does the same again.
+template <int C, int ROWS>
+__global__ void __launch_bounds__(kFewWaves* kWave)
+    few_stream_kernel(FewRows x, const u32x4* __restrict__ wt, int ktiles, int m, const float* __restrict__ bias,
+                      float* __restrict__ resid, const float* __restrict__ weight, bf16* __restrict__ rows,
+                      float* __restrict__ sums) {
+  extern __shared__ f32x4 red[];  // [waves][64]
+  const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), waves = blockDim.x / kWave;
+  const int wr = blockIdx.x * ROWS + lane % ROWS;
+  const int token = threadIdx.x / ROWS, r = threadIdx.x % ROWS, row = blockIdx.x * ROWS + r;
+  const bool mine = token < x.n;
+  const size_t at = static_cast<size_t>(mine ? token : 0) * m + row;
+  float old = 0.f, w = 0.f;
+  if (mine) {
+    old = resid[at];
+    w = weight[row];
+    if (bias) old += bias[row];
+  }
+  const u32x4* const wrow[1] = {wt + static_cast<size_t>(wr / 16) * ktiles * kWave + wr % 16 + lane / 16 * 16};
+  f32x4 acc[1];
+  few_multiply<C, 4, 1>(acc, wrow, x, ktiles, wave, waves, [] {});
+  red[wave * kWave + lane] = acc[0];
+  __syncthreads();
+  if (threadIdx.x >= 16 * ROWS) return;
+  const float v = few_sum(red, kWave, r, token, waves) + old;
+  float square = v * v;
+#pragma unroll
+  for (int off = 1; off < ROWS; off <<= 1) square += __shfl_xor(square, off, kWave);
+  if (!mine) return;
+  resid[at] = v;
+  rows[(static_cast<size_t>(row / 8) * x.n + token) * 8 + row % 8] = from_float<bf16>(v * w);
+  if (r == 0) sums[static_cast<size_t>(blockIdx.x) * x.n + token] = square;
+}
+
+// A gated product: a workgroup for a gate block and its up block.
+template <int C, int LOADS>
+__global__ void __launch_bounds__(kFewWaves* kWave)
+    few_gated_kernel(FewRows x, const u32x4* __restrict__ wt, int ktiles, int m, FewScale scaled, const float* __restrict__ args,
+                     bf16* __restrict__ out, int ldo, int act) {
+  extern __shared__ f32x4 red[];  // [waves][2][64], then the squares' sums by wavefront [waves][16]
+  const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), waves = blockDim.x / kWave;
+  float* part = reinterpret_cast<float*>(red + waves * 2 * kWave);
+  FewSquares<LOADS> squares;
+  squares.load(scaled, x.n);
+  const u32x4* first = wt + static_cast<size_t>(blockIdx.x) * 2 * ktiles * kWave + lane;
+  const u32x4* const wrow[2] = {first, first + static_cast<size_t>(ktiles) * kWave};
+  f32x4 acc[2];
+  few_multiply<C, 2, 2>(acc, wrow, x, ktiles, wave, waves, [&] { if (LOADS) squares.leave(part); });
+  red[(wave * 2) * kWave + lane] = acc[0];
+  red[(wave * 2 + 1) * kWave + lane] = acc[1];
+  __syncthreads();
+  const int token = threadIdx.x / 16, r = threadIdx.x % 16, row = blockIdx.x * 16 + r;
+  if (token >= x.n || row >= m) return;
+  const float s = squares.scale(scaled, part, token, waves);
+  const float g = few_sum(red, 2 * kWave, r, token, waves) * s, u = few_sum(red + kWave, 2 * kWave, r, token, waves) * s;
+  const size_t at = ldo ? static_cast<size_t>(token) * ldo + row : (static_cast<size_t>(row / 8) * x.n + token) * 8 + row % 8;
+  out[at] = from_float<bf16>(gate_times_up(g, u, act, args));
+}
+
+// Projections to queries, keys and values.  A workgroup forms 16 rows of the stacked matrix: of a query or key head 8 elements
+// of the first half and their partners of the second, so that the rotation finds both, of the values 16 elements in a
+// row.  The last wavefront multiplies nothing: it looks up pages and forms cosines and sines meanwhile.
+template <int C, int LOADS>
+__global__ void __launch_bounds__(kFewWaves* kWave)
+    few_heads_kernel(FewRows x, const u32x4* __restrict__ wt, int ktiles, FewScale scaled, const float* __restrict__ bias,
+                     bf16* __restrict__ out, int heads, int kv_heads, int head_dim, const float* __restrict__ inv_freq,
+                     const int32_t* __restrict__ positions, const int32_t* __restrict__ token_seq,
+                     const int32_t* __restrict__ tables, int table_stride, bf16* __restrict__ k_pool, bf16* __restrict__ v_pool,
+                     int page_size, int num_pages, int write_kv, float magnitude) {
+  extern __shared__ f32x4 red[];  // [waves][64], then the squares' sums by wavefront [waves + 1][16]
+  __shared__ float cosine[16][8], sine[16][8];
+  __shared__ int page_of[16], slot_of[16];
+  const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), waves = blockDim.x / kWave - 1;
+  float* part = reinterpret_cast<float*>(red + waves * kWave);
+  const int per_head = head_dim / 16, head = blockIdx.x / per_head, group = blockIdx.x % per_head;
+  const bool turned = head < heads + kv_heads;
+  // this workgroup's first row and, eight rows on, where the other eight begin
+  const int first = head * head_dim + group * (turned ? 8 : 16), second = first + (turned ? head_dim / 2 : 8);
+  FewSquares<LOADS> squares;
+  squares.load(scaled, x.n);
+  if (wave == waves) {
+    if (LOADS) squares.leave(part);
+    if (lane < x.n) {
+      const int pos = positions[lane];
+      int page = -1;
+      if (write_kv && head >= heads) page = tables[static_cast<size_t>(token_seq[lane]) * table_stride + pos / page_size];
+      page_of[lane] = page >= 0 && page < num_pages ? page : -1;  // (outside: a host bug; never dereferenced)
+      slot_of[lane] = pos % page_size;
+    }
+    if (turned) {
+#pragma unroll
+      for (int e = lane; e < 128; e += kWave) {  // (angles as in rope_kv.hip)
+        const int token = e / 8 < x.n ? e / 8 : x.n - 1;
+        const float angle = static_cast<float>(positions[token]) * inv_freq[group * 8 + e % 8];
+        const double wide = static_cast<double>(angle);
+        const double turns = rint(wide * 0.15915494309189535);
+        const float reduced = static_cast<float>(fma(turns, -6.283185307179586, wide));
+        float sv, cv;
+        sincosf(reduced, &sv, &cv);
+        cosine[e / 8][e % 8] = cv * magnitude;
+        sine[e / 8][e % 8] = sv * magnitude;
+      }
+    }
+  } else {
+    const int wr = lane % 16 < 8 ? first + lane % 16 : second + lane % 16 - 8;
+    const u32x4* const wrow[1] = {wt + static_cast<size_t>(wr / 16) * ktiles * kWave + wr % 16 + lane / 16 * 16};
+    f32x4 acc[1];
+    few_multiply<C, 4, 1>(acc, wrow, x, ktiles, wave, waves, [&] { if (LOADS) squares.leave(part); });
+    red[wave * kWave + lane] = acc[0];
+  }
+  const int token = threadIdx.x / 8, i = threadIdx.x % 8;
+  float b1 = 0.f, b2 = 0.f;
+  if (bias) b1 = bias[first + i], b2 = bias[second + i];
+  __syncthreads();
+  if (token >= x.n) return;
+  const float s = squares.scale(scaled, part, token, waves + 1);
+  const float x1 = few_sum(red, kWave, i, token, waves) * s + b1, x2 = few_sum(red, kWave, i + 8, token, waves) * s + b2;
+  const float c = turned ? cosine[token][i] : 1.f, t = turned ? sine[token][i] : 0.f;
+  const float o1 = turned ? x1 * c - x2 * t : x1, o2 = turned ? x2 * c + x1 * t : x2;
+  if (head < heads) {
+    bf16* row = out + static_cast<size_t>(token) * (heads + 2 * kv_heads) * head_dim;
+    row[first + i] = from_float<bf16>(o1);
+    row[second + i] = from_float<bf16>(o2);
+    return;
+  }
+  if (page_of[token] < 0) return;
+  const int kv = turned ? head - heads : head - heads - kv_heads;
+  const size_t base = (static_cast<size_t>(page_of[token]) * kv_heads + kv) * page_size * head_dim;
+  const int slot = slot_of[token], e1 = first - head * head_dim + i, e2 = second - head * head_dim + i;
+  if (turned) {
+    k_pool[base + key_offset(slot, e1, page_size, head_dim)] = from_float<bf16>(o1);
+    k_pool[base + key_offset(slot, e2, page_size, head_dim)] = from_float<bf16>(o2);
+  } else {
+    v_pool[base + static_cast<size_t>(e1) * page_size + slot] = from_float<bf16>(o1);
+    v_pool[base + static_cast<size_t>(e2) * page_size + slot] = from_float<bf16>(o2);
+  }
+}
+
+}  // namespace shk
+
+using namespace shk;
+
+static bool few_rows_of(FewRows* x, const void* a, int lda, int n, int k) {
+  const bool pieces = lda == 0;  // [k / 8][n][8]
+  *x = FewRows{static_cast<const bf16*>(a), pieces ? 8 : lda, pieces ? n : 1, n, k};
+  return n >= 0 && n <= 16 && k > 0 && k % 8 == 0 && (pieces || (lda >= k && lda % 8 == 0));
+}
+
+// Wavefronts that share k: where four to eight of them hold all their tiles at once, the number that holds the fewest
+// beyond k, else four or five.  Few, because each more is another sum to add at the end: 896 x 896 with one token 2.97 us in 4,
+// 3.10 in 7, 3.21 in 15; 3584 x 18944 at 1 / 8 / 16 tokens 22.2 / 23.2 / 27.0 in 4, 22.0 / 24.1 / 28.4 in 5, 23.1 / 24.5 / 27.8
+// in 16; 1536 x 8960, whose 280 tiles five share without loads beyond k, 9.7 / 9.8 / 10.6 in 4 and 9.0 / 9.2 / 11.0 in 5.
+// (Whatever the tokens: a row's bits do not depend on those beside it.)
+static int few_waves(int ktiles, int most) {
+  int best = 0, least = 0;
+  for (int waves = 4; waves <= 8; ++waves) {
+    const int tiles = (ktiles + waves - 1) / waves;
+    if (tiles <= most && (!best || tiles * waves < least)) best = waves, least = tiles * waves;
+  }
+  const auto whole = [&](int waves) { return (ktiles + 4 * waves - 1) / (4 * waves) * 4 * waves; };
+  return best ? best : whole(5) <= whole(4) ? 5 : 4;
+}
+
+// fn with the number of k-tiles of a wavefront as a constant, 0 for more than MOST.
+template <int MOST, int C = 1, typename Fn>
+static void with_tiles(int tiles, Fn fn) {
+  if constexpr (C > MOST) {
+    fn(std::integral_constant<int, 0>{});
+  } else {
+    if (tiles == C) fn(std::integral_constant<int, C>{});
+    else with_tiles<MOST, C + 1>(tiles, fn);
+  }
+}
+
+// and with the loads of a thread that adds up squares
+template <typename Fn>
+static void with_loads(int count, int threads, Fn fn) {
+  const int loads = (count + threads / 16 - 1) / (threads / 16);
+  if (loads == 0) fn(std::integral_constant<int, 0>{});
+  else if (loads <= 4) fn(std::integral_constant<int, 4>{});
+  else if (loads <= 8) fn(std::integral_constant<int, 8>{});
+  else fn(std::integral_constant<int, 16>{});
+}
+constexpr int kFewMostLoads = 16;
+
+// Half blocks where whole ones would be one for every second compute unit or fewer: 896 x 4864 at 8 tokens 6.6 us whole, 6.0 in
+// halves, 2048 x 11008 12.7 and 11.1; 3584 x 18944 23.2 and 32.1.
+static int few_stream_rows(int m) { return m <= 2048 ? 8 : 16; }
+
+// Not where a second round of workgroups would be nearly empty: 320 of them (5120 x 5120 at 8 tokens 14.3 us for product in shares
+// and norm, 15.1 here; 5120 x 13824 28.0 and 31.4).  256 are a round: 4096 x 14336 23.7 -> 20.0.
+extern "C" int shk_few_stream_sums(int m, int k) {
+  return m > 0 && m <= 4096 && m % 16 == 0 && k > 0 && k % 8 == 0 ? m / few_stream_rows(m) : 0;
+}
+
+extern "C" int shk_few_stream(const void* a, int lda, int n, int k, const void* wt, int m, const float* bias, float* resid,
+                              const float* weight, void* rows, float* sums, void* stream) {
+  FewRows x;
+  SHK_REQUIRE(few_rows_of(&x, a, lda, n, k) && m > 0 && m % 16 == 0, "few_stream: bad sizes n=%d m=%d k=%d lda=%d", n, m, k, lda);
+  if (n == 0) return 0;
+  SHK_REQUIRE(a && wt && resid && weight && rows && sums, "few_stream: null pointer");
+  SHK_REQUIRE(reinterpret_cast<uintptr_t>(a) % 16 == 0, "few_stream: rows are not 16-byte aligned");
+  const int kt = (k + 31) / 32, waves = few_waves(kt, kFewTiles), rows_each = few_stream_rows(m);
+  with_tiles<kFewTiles>((kt + waves - 1) / waves, [&](auto c) {
+    const auto kernel = rows_each == 8 ? few_stream_kernel<c.value, 8> : few_stream_kernel<c.value, 16>;
+    kernel<<<m / rows_each, waves * kWave, waves * kWave * sizeof(f32x4), static_cast<hipStream_t>(stream)>>>(
+        x, static_cast<const u32x4*>(wt), kt, m, bias, resid, weight, static_cast<bf16*>(rows), sums);
+  });
+  SHK_LAUNCH_CHECK("few_stream");
+  return 0;
+}
+
+extern "C" int shk_few_gated(const void* a, int lda, int n, int k, const void* wt, const float* sums, int count, float eps,
+                             const float* args, void* out, int m, int ldo, int gated, void* stream) {
+  FewRows x;
+  SHK_REQUIRE(few_rows_of(&x, a, lda, n, k) && m > 0 && (ldo ? ldo >= m : m % 8 == 0),
+              "few_gated: bad sizes n=%d m=%d k=%d lda=%d ldo=%d", n, m, k, lda, ldo);
+  SHK_REQUIRE(gated > 0 && gated <= kActQuickGelu, "few_gated: unknown gate activation %d", gated);
+  SHK_REQUIRE(sums && count > 0 && eps > 0.f, "few_gated: rows come with the sums of their squares");
+  if (n == 0) return 0;
+  SHK_REQUIRE(a && wt && out, "few_gated: null pointer");
+  SHK_REQUIRE(reinterpret_cast<uintptr_t>(a) % 16 == 0, "few_gated: rows are not 16-byte aligned");
+  const FewScale scaled = {sums, count, 1.f / static_cast<float>(k), eps};
+  // four wavefronts where they hold their tiles at once (9728 x 896: 5.8 us with one token, 5.9 in eight), else eight
+  // (22016 x 2048 15.6, 15.9 in four)
+  const int kt = (k + 31) / 32, waves = kt <= 4 * kFewPairs ? 4 : 8;
+  SHK_REQUIRE(count <= kFewMostLoads * waves * 4, "few_gated: too many sums (%d)", count);
+  with_loads(count, waves * kWave, [&](auto loads) {
+    with_tiles<kFewPairs>((kt + waves - 1) / waves, [&](auto c) {
+      const size_t lds = waves * (2 * kWave * sizeof(f32x4) + 16 * sizeof(float));
+      few_gated_kernel<c.value, loads.value><<<(m + 15) / 16, waves * kWave, lds, static_cast<hipStream_t>(stream)>>>(
+          x, static_cast<const u32x4*>(wt), kt, m, scaled, args, static_cast<bf16*>(out), ldo, gated);
+    });
+  });
+  SHK_LAUNCH_CHECK("few_gated");
+  return 0;
+}
+
+extern "C" int shk_few_heads(const void* a, int lda, int n, int k, const void* wt, const float* sums, int count, float eps,
+                             const float* bias, void* out, int heads, int kv_heads, int head_dim, const float* inv_freq,
+                             const int32_t* positions, const int32_t* token_seq, const int32_t* tables, int table_stride,
+                             void* k_pool, void* v_pool, int page_size, int num_pages, int write_kv, float magnitude,
+                             void* stream) {
+  FewRows x;
+  SHK_REQUIRE(few_rows_of(&x, a, lda, n, k), "few_heads: bad sizes n=%d k=%d lda=%d", n, k, lda);
+  SHK_REQUIRE(heads > 0 && kv_heads > 0 && head_dim > 0 && head_dim % 16 == 0, "few_heads: bad heads %d %d %d", heads, kv_heads, head_dim);
+  if (n == 0) return 0;
+  SHK_REQUIRE(a && wt && out && inv_freq && positions, "few_heads: null pointer");
+  SHK_REQUIRE(reinterpret_cast<uintptr_t>(a) % 16 == 0, "few_heads: rows are not 16-byte aligned");
+  SHK_REQUIRE(!sums || (count > 0 && eps > 0.f), "few_heads: bad sums");
+  if (write_kv) {
+    SHK_REQUIRE(token_seq && tables && k_pool && v_pool, "few_heads: null cache pointer");
+    SHK_REQUIRE(page_size > 0 && num_pages > 0 && table_stride > 0, "few_heads: bad cache sizes page_size=%d num_pages=%d table_stride=%d",
+                page_size, num_pages, table_stride);
+  }
+  const FewScale scaled = {sums, count, 1.f / static_cast<float>(k), eps};
+  const int groups = (heads + 2 * kv_heads) * (head_dim / 16);
+  const int kt = (k + 31) / 32, waves = few_waves(kt, kFewTiles);
+  SHK_REQUIRE(!sums || count <= kFewMostLoads * (waves + 1) * 4, "few_heads: too many sums (%d)", count);
+  with_loads(sums ? count : 0, (waves + 1) * kWave, [&](auto loads) {
+    with_tiles<kFewTiles>((kt + waves - 1) / waves, [&](auto c) {
+      const size_t lds = waves * kWave * sizeof(f32x4) + (waves + 1) * 16 * sizeof(float);
+      few_heads_kernel<c.value, loads.value><<<groups, (waves + 1) * kWave, lds, static_cast<hipStream_t>(stream)>>>(
+          x, static_cast<const u32x4*>(wt), kt, scaled, bias, static_cast<bf16*>(out), heads, kv_heads, head_dim, inv_freq, positions,
+          token_seq, tables, table_stride, static_cast<bf16*>(k_pool), static_cast<bf16*>(v_pool), page_size, num_pages, write_kv,
+          magnitude);
+    });
+  });
+  SHK_LAUNCH_CHECK("few_heads");
+  return 0;
+}

@@ -149,6 +149,8 @@ class StepContext:
     # what the parts' prepare() added: device arrays, and host-side decisions
     extras: dict = field(default_factory=dict)
     notes: dict = field(default_factory=dict)
+    # (HiddenState, norm): the stream that a sublayer's last product may add to, leaving the norm's rows (Runtime.linear_onto)
+    onto: tuple | None = None
     # everything a step's launches may depend on, for parts that say launches_follow_shape
     shape_key: tuple = ()
 

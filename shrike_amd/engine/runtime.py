@@ -61,6 +61,9 @@ class Runtime:
         """out = act(g) * (u + up_shift), g = x @ gate.T, u = x @ up.T, both bounded by `limit` first
         where one is given.  bfloat16: one product whose epilogue applies the gate (its constants are
         those the weight was made with); float32: product, then activation."""
+        if isinstance(x, ops.ScaledRows):
+            ops.few_gated(x, w.tiled, w.rows, w.cols, out, activation, w.gate_args)
+            return
         if w.tiled is not None:
             ops.gemm_tiled_weight(x, w.tiled, w.rows, w.cols, out, gated=activation, gate_args=w.gate_args)
             return
@@ -81,6 +84,29 @@ class Runtime:
         ops.gemm_f32_tiled_weight(x, w.tiled_f32, w.rows, w.cols, out, bias=bias, accumulate=accumulate)
         if activation is not None:
             ops.activate(out, out, activation)
+
+    def linear_onto(self, ctx, name: str, x, w: LinearWeight, bias=None):
+        """linear_deferred() for a sublayer's last product.  Where the block has said which stream it joins and which norm
+        comes next (ctx.onto) and the tokens are few, the product adds to the stream itself and leaves the norm's rows
+        in hidden.scaled, and nothing is pending: None."""
+        count = self.onto_sums(ctx, w) if x.dim() == 3 or ops.rows_aligned(x) else 0
+        target, ctx.onto = ctx.onto, None
+        if not count:
+            return self.linear_deferred(ctx, name, x, w, bias=bias)
+        hidden, norm = target
+        n = hidden.resid.shape[0]
+        rows = ctx.buffer("stream_rows", (w.rows // 8, n, 8), self.dtype)
+        sums = ctx.buffer("stream_sums", (count, n), torch.float32)
+        ops.few_stream(x, w.tiled, w.rows, w.cols, hidden.resid, norm.weight, rows, sums, bias=bias)
+        hidden.scaled = (norm, ops.ScaledRows(rows, sums, norm.eps))
+        hidden.cast = None
+        return None
+
+    def onto_sums(self, ctx, w: LinearWeight) -> int:
+        """Groups of sums that linear_onto() leaves of its product with `w` in this step, 0 where it leaves it pending."""
+        if ctx.onto is None or w.tiled is None or ctx.num_tokens > ops.FEW_TOKENS or w.cols % 8:
+            return 0
+        return ops.few_stream_sums(w.rows, w.cols)
 
     def linear_deferred(self, ctx, name: str, x, w: LinearWeight, bias=None, reader="norm",
                         keep_float32: bool = False):

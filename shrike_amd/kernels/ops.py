@@ -494,6 +494,112 @@ def gemm_tiled_weight(a, wt, m: int, k: int, out, bias=None, accumulate=False, g
     )
 
 
+class ScaledRows:
+    """Rows x * w of a stream x in bfloat16 that a norm's weight w has multiplied and that still have to be divided by
+    sqrt(mean(x^2) + eps): `rows` [k / 8, n, 8], `sums` float32 [count, n] the squares of x, summed by groups of columns."""
+
+    __slots__ = ("rows", "sums", "eps")
+
+    def __init__(self, rows: torch.Tensor, sums: torch.Tensor, eps: float):
+        self.rows, self.sums, self.eps = rows, sums, eps
+
+    @property
+    def shape(self):
+        return (self.rows.shape[1], 8 * self.rows.shape[0])
+
+
+FEW_TOKENS = 16  # the most that few_stream, few_gated and few_heads take
+
+
+def few_stream_sums(m: int, k: int) -> int:
+    """Groups of columns that few_stream sums the squares of (0: it does not take an [m, k] matrix, or not as well as a
+    product and a norm do)."""
+    return int(load().shk_few_stream_sums(m, k))
+
+
+def _few_rows(who, x, k, wt, numel):
+    """(address, row stride, tokens) of rows [n, k], or [k / 8, n, 8] with the stride 0."""
+    pieces = x.dim() == 3
+    if pieces:
+        fits = x.is_contiguous() and x.shape[0] * 8 == k and x.shape[2] == 8
+    else:
+        _rows(x, f"{who} rows")
+        fits = x.shape[1] == k
+    n = x.shape[1] if pieces else x.shape[0]
+    if not fits or x.dtype != torch.bfloat16 or n > FEW_TOKENS:
+        raise KernelError(f"{who}: rows must be bfloat16 [up to {FEW_TOKENS}, {k}] or pieces of them, got {tuple(x.shape)}")
+    if wt.numel() != numel or wt.dtype != torch.bfloat16:
+        raise KernelError(f"{who}: the tiled weights do not belong to the product")
+    return _dev(x, "rows"), 0 if pieces else x.stride(0), n
+
+
+def _few_sums(who, x):
+    """(rows, address of the sums, their number, eps) of ScaledRows, or of rows that are normed already."""
+    if not isinstance(x, ScaledRows):
+        return x, None, 0, 0.0
+    if x.sums.dim() != 2 or x.sums.shape[1] != x.shape[0] or not x.sums.is_contiguous():
+        raise KernelError(f"{who}: sums must be contiguous [count, {x.shape[0]}]")
+    return x.rows, _dev(x.sums, "sums", torch.float32), x.sums.shape[0], float(x.eps)
+
+
+def few_stream(a, wt, m: int, k: int, resid, weight, rows, sums, bias=None) -> None:
+    """resid += a @ w.T + bias; rows [m / 8, n, 8] = resid * weight in bfloat16 and sums its squares by groups of columns
+    (ScaledRows).  `a` [n, k], or pieces [k / 8, n, 8]."""
+    p, lda, n = _few_rows("few_stream", a, k, wt, tiled_numel(m, k))
+    if tuple(resid.shape) != (n, m) or not resid.is_contiguous() or weight.numel() != m or (bias is not None and bias.numel() != m):
+        raise KernelError(f"few_stream: resid must be contiguous [{n}, {m}], weight and bias as wide")
+    if m % 8 or tuple(rows.shape) != (m // 8, n, 8) or not rows.is_contiguous() or rows.dtype != torch.bfloat16:
+        raise KernelError(f"few_stream: rows must be contiguous bfloat16 [{m // 8}, {n}, 8]")
+    if tuple(sums.shape) != (few_stream_sums(m, k), n) or not sums.is_contiguous():
+        raise KernelError(f"few_stream: sums must be contiguous [{few_stream_sums(m, k)}, {n}]")
+    check(load().shk_few_stream(
+        p, lda, n, k, _dev(wt, "wt"), m, None if bias is None else _dev(bias, "bias", torch.float32),
+        _dev(resid, "resid", torch.float32), _dev(weight, "weight", torch.float32), _dev(rows, "rows"),
+        _dev(sums, "sums", torch.float32), _stream()))
+
+
+def few_gated(x: ScaledRows, wt, m: int, k: int, out, activation, gate_args=None) -> None:
+    """The gated product of gemm_tiled_weight of up to 16 rows that are still to be divided by their root mean square;
+    `out` [n, m], or pieces [m / 8, n, 8]."""
+    rows, sums, count, eps = _few_sums("few_gated", x)
+    p, lda, n = _few_rows("few_gated", rows, k, wt, 2 * tiled_numel(m, k))
+    pieces = out.dim() == 3
+    if tuple(out.shape) != ((m // 8, n, 8) if pieces else (n, m)) or out.dtype != torch.bfloat16 or out.stride(-1) != 1 \
+            or (pieces and (m % 8 or not out.is_contiguous())):
+        raise KernelError(f"few_gated: out must be bfloat16 [{n}, {m}] or pieces of it")
+    if gate_args is not None and (gate_args.numel() != 2 or gate_args.dtype != torch.float32):
+        raise KernelError("few_gated: gate_args are two float32 numbers")
+    check(load().shk_few_gated(p, lda, n, k, _dev(wt, "wt"), sums, count, eps,
+                               None if gate_args is None else _dev(gate_args, "gate_args"), _dev(out, "out"), m,
+                               0 if pieces else out.stride(0), activation_code(activation), _stream()))
+
+
+def few_heads(x, wt, k: int, out, heads, kv_heads, head_dim, inv_freq, positions, token_seq, tables, k_pool, v_pool,
+              page_size, write_kv=True, bias=None, magnitude: float = 1.0) -> None:
+    """The projections of up to 16 rows (normed, or ScaledRows) to queries, keys and values, rotated whole as in
+    rope_kv_store: queries into out's query columns, keys and values into their pages."""
+    rows, sums, count, eps = _few_sums("few_heads", x)
+    width = (heads + 2 * kv_heads) * head_dim
+    p, lda, n = _few_rows("few_heads", rows, k, wt, tiled_numel(width, k))
+    if tuple(out.shape) != (n, width) or not out.is_contiguous() or out.dtype != torch.bfloat16:
+        raise KernelError(f"few_heads: out must be contiguous bfloat16 [{n}, {width}]")
+    if bias is not None and bias.numel() != width:
+        raise KernelError(f"few_heads: bias has {bias.numel()} elements, not {width}")
+    if inv_freq.numel() < head_dim // 2:
+        raise KernelError("few_heads: heads are rotated whole")
+    if positions.shape[0] < n or (write_kv and token_seq.shape[0] < n):
+        raise KernelError(f"few_heads: {n} rows but positions / token_seq are shorter")
+    if write_kv:
+        _check_pools("few_heads", out, tables, k_pool, v_pool, kv_heads, head_dim, page_size)
+    check(load().shk_few_heads(
+        p, lda, n, k, _dev(wt, "wt"), sums, count, eps, None if bias is None else _dev(bias, "bias", torch.float32),
+        _dev(out, "out"), heads, kv_heads, head_dim, _dev(inv_freq, "inv_freq", torch.float32),
+        _dev(positions, "positions", torch.int32), _dev(token_seq, "token_seq", torch.int32) if write_kv else None,
+        _dev(tables, "tables", torch.int32) if write_kv else None, tables.shape[1] if write_kv else 0,
+        _dev(k_pool, "k_pool") if write_kv else None, _dev(v_pool, "v_pool") if write_kv else None, page_size,
+        k_pool.shape[0] if write_kv else 0, int(bool(write_kv)), float(magnitude), _stream()))
+
+
 def key_slab(head_dim: int) -> int:
     """Elements per slab of the cached keys: 32, or the whole row where head_dim
     is no multiple of 32 (csrc/common.h: key_slab)."""

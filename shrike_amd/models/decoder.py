@@ -7,6 +7,7 @@ from __future__ import annotations
 import torch
 
 from ..config.specs import ModelSpec
+from ..parts.block import PreNormResidualBlock
 from ..parts.base import CompositeSpec, HiddenState, ParamSpec, Part, StateSpec, build_part
 
 
@@ -34,6 +35,12 @@ class DecoderModel:
         # every run's result is kept and the stream that goes on is a weighted sum of them
         self._averaged = bool(spec.schedule) and spec.schedule[0].depth_average is not None
         self.depth_coefficients: list = []
+        # of every run, (norm, mixer) that the next one begins with, where nothing comes between them
+        self._following: list = [None] * len(spec.schedule)
+        for pos, entry in enumerate(spec.schedule[1:]):
+            block = self.blocks[entry.block]
+            if type(block).forward is PreNormResidualBlock.forward and not entry.add_embedding and entry.add_vector is None:
+                self._following[pos] = (block.mixer_norm, block.mixer)
         # the parts whose prepare() does something, in the order they run
         self._preparers = [p for p in self.parts() if type(p).prepare is not Part.prepare]
 
@@ -152,6 +159,7 @@ class DecoderModel:
                     vector = self.stream_vectors[entry.add_vector[0]][entry.add_vector[1]]
                 ops.add_rows(hidden.resid, embedded if entry.add_embedding else None, vector)
                 hidden.cast = None
+            hidden.following = self._following[pos] if history is None else None
             self.blocks[entry.block].forward(ctx, hidden, caches[pos])
             if history is not None:
                 # the run's result is its stream plus what is pending; a pending output with a

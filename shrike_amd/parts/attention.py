@@ -429,7 +429,7 @@ class PagedAttention(Mixer):
         if self.position is not None:
             self.position.load(tensors, runtime)
         self.linear = runtime.linear
-        self.linear_deferred = runtime.linear_deferred
+        self.linear_deferred, self.linear_onto = runtime.linear_deferred, runtime.linear_onto
         self.dtype = runtime.dtype
 
     # ------------------------------------------------------------ launch plans
@@ -610,6 +610,19 @@ class PagedAttention(Mixer):
             return (s.num_heads + s.num_kv_heads) * s.head_dim
         return (s.num_heads + s.num_kv_heads) * s.head_dim + s.num_kv_heads * self.value_dim
 
+    @property
+    def ends_onto(self) -> bool:
+        return type(self).forward is PagedAttention.forward
+
+    def takes_scaled(self, ctx) -> bool:
+        """Whether the step's projections, their rotation and the cache write are one kernel (ops.few_heads)."""
+        s = self.spec
+        if not self.ends_onto or self.plain_store or s.values_from_keys or self.position is None or getattr(self.position, "adjacent_pairs", False):
+            return False
+        table = self.position.rotary_table()
+        return (table is not None and table[1] == s.head_dim and s.head_dim % 16 == 0 and self.w_qkv.tiled is not None
+                and ctx.num_tokens <= ops.FEW_TOKENS and self.width % 8 == 0)
+
     def forward(self, ctx, x: torch.Tensor, cache) -> torch.Tensor:
         s = self.spec
         n = x.shape[0]
@@ -630,8 +643,17 @@ class PagedAttention(Mixer):
                           has_kv=not self.shared_kv)
             attn = ctx.buffer("attn_out", (n, s.num_heads * self.value_dim), ctx.dtype)
             self.attend(ctx, qkv, attn, tables, cache)
-            return self.linear_deferred(ctx, "attn_proj", attn, self.w_o, bias=self.b_o)
+            return self.linear_onto(ctx, "attn_proj", attn, self.w_o, bias=self.b_o)
         table = self.position.rotary_table() if self.position is not None else None
+        tables = ctx.block_tables[cache.group]
+        if self.takes_scaled(ctx) and (isinstance(x, ops.ScaledRows) or ops.rows_aligned(x)):
+            qkv = ctx.buffer("attn_qkv", (n, qkv_width), ctx.dtype)
+            ops.few_heads(x, self.w_qkv.tiled, self.width, qkv, s.num_heads, s.num_kv_heads, s.head_dim, table[0], ctx.positions,
+                          ctx.token_seq, tables, cache.pools["k"], cache.pools["v"], cache.page_size, write_kv=cache.owned,
+                          bias=self.b_qkv, magnitude=float(getattr(self.position, "magnitude", 1.0)))
+            attn = ctx.buffer("attn_out", (n, s.num_heads * s.head_dim), ctx.dtype)
+            self.attend(ctx, qkv, attn, tables, cache)
+            return self.linear_onto(ctx, "attn_proj", attn, self.w_o, bias=self.b_o)
         fused_position = self.position is None or table is not None
         split_sum = None
         if fused_position:
@@ -645,7 +667,6 @@ class PagedAttention(Mixer):
             self.linear(x, self.w_qkv, qkv, bias=self.b_qkv)
             self.position.apply(ctx, qkv, s.num_heads, s.num_kv_heads, s.head_dim)
         inv_freq, rot_dim = table if table is not None else (None, 0)
-        tables = ctx.block_tables[cache.group]
         ops.rope_kv_store(
             qkv, s.num_heads, s.num_kv_heads, s.head_dim, rot_dim, inv_freq, ctx.positions,
             ctx.token_seq, tables, cache.pools["k"], cache.pools["v"], cache.page_size,
@@ -657,7 +678,7 @@ class PagedAttention(Mixer):
         attn = ctx.buffer("attn_out", (n, s.num_heads * s.head_dim), ctx.dtype)
         self.attend(ctx, qkv, attn, tables, cache)
         # the norm that follows adds the output to the residual stream and can add up parts
-        return self.linear_deferred(ctx, "attn_proj", attn, self.w_o, bias=self.b_o)
+        return self.linear_onto(ctx, "attn_proj", attn, self.w_o, bias=self.b_o)
 
 
 register_mixer("paged_attention", PagedAttention)

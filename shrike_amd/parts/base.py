@@ -161,9 +161,11 @@ class HiddenState:
     (weight, bias, eps) that it joins as its layer norm, (pending - mean) /
     sqrt(var + eps) * weight + bias.  `pending_scale`: what `pending` (without a norm of its
     own) is multiplied by as it joins.  `cast`: the stream as it stands (nothing pending) in the
-    compute dtype, where the kernel that wrote `resid` last left such a copy."""
+    compute dtype, where the kernel that wrote `resid` last left such a copy.  `scaled`: (norm, ops.ScaledRows), what the
+    product that added to `resid` last has left for the norm that comes next.  `following`: (norm, mixer) of the
+    block after the one that runs, where it begins with them."""
 
-    __slots__ = ("resid", "pending", "pending_norm", "pending_scale", "cast")
+    __slots__ = ("resid", "pending", "pending_norm", "pending_scale", "cast", "scaled", "following")
 
     def __init__(self, resid: torch.Tensor, pending: torch.Tensor | None = None, pending_norm=None):
         self.resid = resid
@@ -171,6 +173,7 @@ class HiddenState:
         self.pending_norm = pending_norm
         self.pending_scale = 1.0
         self.cast = None
+        self.scaled = self.following = None
 
     def settle(self, ctx) -> None:
         """Adds what is pending to `resid` now (for a reader that is no norm)."""
@@ -206,6 +209,12 @@ class Part:
     # run such a model's forward from a recorded list of launches.  A part that
     # decides anything else on the host per step must put it into the launch key.
     launches_follow_shape = False
+    # whether a sublayer's last product goes through Runtime.linear_onto
+    ends_onto = False
+
+    def takes_scaled(self, ctx) -> bool:
+        """Whether forward takes ops.ScaledRows in this step in the place of normed rows."""
+        return False
 
     def __init__(self, spec, width: int, name: str):
         self.spec = spec
@@ -235,6 +244,10 @@ class Part:
 
 
 class Norm(Part):
+    # whether forward's rows are the stream's times `weight` over the root of their mean square plus `eps`, and it takes
+    # hidden.scaled in their place
+    leaves_scaled = False
+
     def forward(self, ctx, hidden: HiddenState, rows=None, write_resid=True) -> torch.Tensor:
         raise NotImplementedError
 

@@ -43,14 +43,28 @@ class PreNormResidualBlock(Block):
 
     def forward(self, ctx, hidden: HiddenState, cache) -> None:
         scale = float(getattr(self.spec, "residual_scale", 1.0))
+        following = hidden.following or (None, None)
+        after_mixer = (self.ffn_norm, self.ffn) if self.ffn is not None else following
         x = self.mixer_norm.forward(ctx, hidden)
+        ctx.onto = self._onto(ctx, hidden, scale, self.mixer, *after_mixer)
         hidden.pending = self.mixer.forward(ctx, x, cache)
         hidden.pending_scale = scale
+        ctx.onto = None
         if self.ffn is None:
             return
         x = self.ffn_norm.forward(ctx, hidden)
+        ctx.onto = self._onto(ctx, hidden, scale, self.ffn, *following)
         hidden.pending = self.ffn.forward(ctx, x)
         hidden.pending_scale = scale
+        ctx.onto = None
+
+    @staticmethod
+    def _onto(ctx, hidden, scale, part, norm, reader):
+        """What `part`'s last product may add to (StepContext.onto): the stream, where the next norm and its reader take
+        what such a product leaves."""
+        if scale != 1.0 or norm is None or not part.ends_onto or not norm.leaves_scaled or not reader.takes_scaled(ctx):
+            return None
+        return hidden, norm
 
 
 register_block("prenorm_residual", PreNormResidualBlock)

@@ -4,6 +4,7 @@ from __future__ import annotations
 
 import torch
 
+from ..kernels import ops
 from .base import FeedForward, ParamSpec, register_ffn
 
 
@@ -14,6 +15,13 @@ class SwiGLU(FeedForward):
     activated values."""
 
     launches_follow_shape = True
+
+    @property
+    def ends_onto(self) -> bool:
+        return type(self).forward is SwiGLU.forward
+
+    def takes_scaled(self, ctx) -> bool:
+        return self.ends_onto and self.w_gate_up.tiled is not None and ctx.num_tokens <= ops.FEW_TOKENS and self.width % 8 == 0
 
     def params(self):
         inter, h = self.spec.intermediate_size, self.width
@@ -41,15 +49,16 @@ class SwiGLU(FeedForward):
             self.activation, self.limit, self.up_shift,
         )
         self.w_down = runtime.weight(tensors[self.tensor_name("down", "down_proj.weight")])
-        self.linear_deferred = runtime.linear_deferred
+        self.linear_onto, self.onto_sums = runtime.linear_onto, runtime.onto_sums
         self.gated_linear = runtime.gated_linear
 
     def forward(self, ctx, x: torch.Tensor) -> torch.Tensor:
         n = x.shape[0]
-        act = ctx.buffer("ffn_act", (n, self.inter), ctx.dtype)
+        pieces = isinstance(x, ops.ScaledRows) and self.inter % 8 == 0 and self.onto_sums(ctx, self.w_down)
+        act = ctx.buffer("ffn_act", (self.inter // 8, n, 8) if pieces else (n, self.inter), ctx.dtype)
         self.gated_linear(ctx, x, self.w_gate_up, act, self.activation, self.limit, self.up_shift)
         # the norm that follows adds the output to the residual stream and can add up parts
-        return self.linear_deferred(ctx, "ffn_out", act, self.w_down)
+        return self.linear_onto(ctx, "ffn_out", act, self.w_down)
 
 
 register_ffn("swiglu", SwiGLU)

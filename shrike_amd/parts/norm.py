@@ -15,6 +15,10 @@ class RMSNorm(Norm):
 
     launches_follow_shape = True
 
+    @property
+    def leaves_scaled(self) -> bool:
+        return type(self).forward is RMSNorm.forward
+
     def params(self):
         offset = float(getattr(self.spec, "offset", 0.0))
         return [ParamSpec(self.tensor_name("weight"), (self.width,), init="norm" if offset == 0.0 else "norm_zero",
@@ -28,6 +32,11 @@ class RMSNorm(Norm):
         self.eps = float(self.spec.eps)
 
     def forward(self, ctx, hidden: HiddenState, rows=None, write_resid=True) -> torch.Tensor:
+        if hidden.scaled is not None:
+            (norm, scaled), hidden.scaled = hidden.scaled, None
+            if norm is not self or rows is not None:
+                raise RuntimeError(f"{self.name}: the rows that a product has left belong to another norm")
+            return scaled  # the norm's reader divides what it forms
         n = hidden.resid.shape[0] if rows is None else rows.shape[0]
         out = ctx.buffer(f"normed", (n, self.width), ctx.dtype)
         if hidden.pending is not None and (hidden.pending_scale != 1.0 or (
