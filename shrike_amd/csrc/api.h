@@ -145,17 +145,19 @@ int shk_gemm_bf16_parts(int n, int m, int k, int gated);
 // tiles of a product of more than 64 tokens: their number (0: not served in tiles), (weight rows, tokens) of up to two
 int shk_gemm_bf16_tiles(int n, int m, int k, int gated, int ksplit, int aligned, int* sizes);
 
-// Products of up to 16 tokens (bfloat16, rows 16-byte aligned, k a multiple of 8) that spare the kernels around them.
-// lda 0: the rows come as [k / 8][n][8].
+// Products of up to 64 tokens (bfloat16, rows 16-byte aligned, k a multiple of 8) that spare the kernels around them; the
+// queries say for which sizes they are the faster ones (shk_few_stream_sums: 0 where not).  lda 0: the rows come as [k / 8][n][8].
 // shk_few_stream: resid[n, m] += a @ w^T + bias (float32 [m] or null); rows [m / 8][n][8] = the new resid * weight in
-// bfloat16 and sums[shk_few_stream_sums()][n] its squares summed by workgroup: what the next two calls take in the place of
+// bfloat16 and sums[shk_few_stream_sums(n, m, k)][n] its squares summed by workgroup: what the next two calls take in the place of
 // normed rows, dividing by sqrt(mean(resid^2) + eps) what they form.  m a multiple of 16.
 // shk_few_gated: out = act((a @ gate^T) / rms) * ((a @ up^T) / rms), wt and args (bias) as in shk_gemm_bf16_tiled_weight;
 // ldo 0: out is [m / 8][n][8], m a multiple of 8.
 // shk_few_heads: (a @ w^T) / rms + bias as the [n, (heads + 2 kv_heads) * head_dim] projections of shk_rope_kv_store, which
 // are rotated whole (pairs (i, i + head_dim / 2)): queries go to out's query columns (its others are left alone), keys and
 // values to their pages as there.  sums null: rows that are normed already.  head_dim a multiple of 16.
-int shk_few_stream_sums(int m, int k);
+int shk_few_stream_sums(int n, int m, int k);
+int shk_few_gated_takes(int n, int m, int k);
+int shk_few_heads_takes(int n, int m, int k);
 int shk_few_stream(const void* a, int lda, int n, int k, const void* wt, int m, const float* bias, float* resid,
                    const float* weight, void* rows, float* sums, void* stream);
 int shk_few_gated(const void* a, int lda, int n, int k, const void* wt, const float* sums, int count, float eps,

@@ -1,4 +1,4 @@
-// Products of up to 16 tokens that finish what the kernels between two products would do, so that a decode step has
+// Products of up to 16 tokens, with small matrices of up to 64, that finish what the kernels between two products would do, so that a decode step has
 // fewer dependent kernels: five a layer instead of eight.  A step of a small model is a chain of kernels of 2.5 to 6 us each,
 // most of which start, wait for memory once and end (weights already in the caches make the 7B output projection 6.3 us
 // instead of 6.8).
@@ -28,7 +28,13 @@
 
 namespace shk {
 
-// Rows of up to 16 tokens: piece `col` (a multiple of 8) of a token lies at token * token_step + col * col_step.
+// A workgroup takes NB blocks of 16 tokens; blockIdx.y says which.
+template <int NB>
+__device__ __forceinline__ int few_first() {
+  return blockIdx.y * 16 * NB;
+}
+
+// Rows: piece `col` (a multiple of 8) of a token lies at token * token_step + col * col_step.
 struct FewRows {
   const bf16* a;
   int token_step, col_step, n, k;
@@ -41,12 +47,13 @@ struct FewScale {
   float inv_width, eps;
 };
 
-// A thread adds up every (threads / 16)th sum of one token.  They are asked for before the weights, all at once ...
-template <int LOADS>
+// A thread adds up some of the sums of one token.  They are asked for before the weights, all at once ...
+template <int LOADS, int NB>
 struct FewSquares {
+  static constexpr int kTokens = 16 * NB;
   float v[LOADS > 0 ? LOADS : 1];
   __device__ __forceinline__ void load(const FewScale& s, int n) {
-    const int token = threadIdx.x % 16, first = threadIdx.x / 16, step = blockDim.x / 16;
+    const int token = few_first<NB>() + threadIdx.x % kTokens, first = threadIdx.x / kTokens, step = blockDim.x / kTokens;
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
       const int c = first + i * step;
@@ -59,31 +66,33 @@ struct FewSquares {
     float t = 0.f;
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) t += v[i];
-    t += __shfl_xor(t, 16, kWave);
-    t += __shfl_xor(t, 32, kWave);
-    if (threadIdx.x % kWave < 16) part[threadIdx.x / kWave * 16 + threadIdx.x % kWave] = t;
+#pragma unroll
+    for (int off = kTokens; off < kWave; off <<= 1) t += __shfl_xor(t, off, kWave);
+    if (threadIdx.x % kWave < kTokens) part[threadIdx.x / kWave * kTokens + threadIdx.x % kWave] = t;
   }
   __device__ __forceinline__ float scale(const FewScale& s, const float* part, int token, int waves) const {
     if (LOADS == 0) return 1.f;
     float t = 0.f;
-    for (int w = 0; w < waves; ++w) t += part[w * 16 + token];
+    for (int w = 0; w < waves; ++w) t += part[w * kTokens + token];
     return rsqrtf(t * s.inv_width + s.eps);
   }
 };
 
 // A wavefront asks for everything before it waits for anything: its k-tiles at once where they fit its registers.
-// acc += the wavefront's k-tiles (wave, wave + waves, ...) of RB blocks of 16 weight rows by up to 16 tokens.  wrow[]: the lane's
+// acc += the wavefront's k-tiles (wave, wave + waves, ...) of RB blocks of 16 weight rows by NB blocks of 16 tokens.  wrow[]: the lane's
 // weight row at its piece of the first tile.  C > 0: a wavefront has at most C tiles, which are all asked for at once;
 // C = 0: batches of B tiles, two in flight.  Addresses are clamped into the matrices and what lies beyond k is
 // zeroed when it is used: no load stands under a condition.
-template <int C, int B, int RB, typename Between>
-__device__ __forceinline__ void few_multiply(f32x4 (&acc)[RB], const u32x4* const (&wrow)[RB], const FewRows& x, int ktiles, int wave,
+template <int C, int B, int RB, int NB, typename Between>
+__device__ __forceinline__ void few_multiply(f32x4 (&acc)[RB][NB], const u32x4* const (&wrow)[RB], const FewRows& x, int ktiles, int wave,
                                              int waves, Between between) {
   const int lane = threadIdx.x % kWave, j = lane % 16, kg = lane / 16;
-  const bf16* arow = x.a + static_cast<size_t>(j < x.n ? j : x.n - 1) * x.token_step;
+  const bf16* arow[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) arow[b] = x.a + static_cast<size_t>(min(few_first<NB>() + b * 16 + j, x.n - 1)) * x.token_step;
   constexpr int kTiles = C > 0 ? C : B;
   struct Batch {
-    u32x4 w[kTiles][RB], x[kTiles];
+    u32x4 w[kTiles][RB], x[kTiles][NB];
     uint32_t keep[kTiles];
   };
   auto load = [&](Batch& b, int t) {
@@ -95,22 +104,28 @@ __device__ __forceinline__ void few_multiply(f32x4 (&acc)[RB], const u32x4* cons
         b.w[u][r] = __builtin_nontemporal_load(wrow[r] + static_cast<size_t>(tt < ktiles ? tt : ktiles - 1) * kWave);
       const bool inside = col < x.k;
       b.keep[u] = inside ? ~0u : 0u;
-      b.x[u] = *reinterpret_cast<const u32x4*>(arow + (inside ? static_cast<size_t>(col) * x.col_step : 0));
+#pragma unroll
+      for (int c = 0; c < NB; ++c)
+        b.x[u][c] = *reinterpret_cast<const u32x4*>(arow[c] + (inside ? static_cast<size_t>(col) * x.col_step : 0));
     }
     __builtin_amdgcn_sched_barrier(0);
   };
   auto multiply = [&](const Batch& b) {
 #pragma unroll
-    for (int u = 0; u < kTiles; ++u) {
-      const u32x4 v = b.x[u] & b.keep[u];
+    for (int u = 0; u < kTiles; ++u)
 #pragma unroll
-      for (int r = 0; r < RB; ++r)
-        acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, b.w[u][r]), __builtin_bit_cast(bf16x8, v),
-                                                         acc[r], 0, 0, 0);
-    }
+      for (int c = 0; c < NB; ++c) {
+        const u32x4 v = b.x[u][c] & b.keep[u];
+#pragma unroll
+        for (int r = 0; r < RB; ++r)
+          acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, b.w[u][r]), __builtin_bit_cast(bf16x8, v),
+                                                              acc[r][c], 0, 0, 0);
+      }
   };
 #pragma unroll
-  for (int r = 0; r < RB; ++r) acc[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int r = 0; r < RB; ++r)
+#pragma unroll
+    for (int c = 0; c < NB; ++c) acc[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
   Batch ping;
   load(ping, wave);
   if constexpr (C > 0) {
@@ -153,62 +168,80 @@ __device__ __forceinline__ float few_sum(const f32x4* red, int stride, int row, 
 
 // ROWS = 16: a workgroup for a block of 16 weight rows.  ROWS = 8: for half of one (a tile's pieces of 8 rows are whole
 // lines of 128 bytes), where whole blocks leave compute units idle; the other half of the matrix instruction does the same again.
-template <int C, int ROWS>
+template <int C, int ROWS, int NB>
 __global__ void __launch_bounds__(kFewWaves* kWave)
     few_stream_kernel(FewRows x, const u32x4* __restrict__ wt, int ktiles, int m, const float* __restrict__ bias,
                       float* __restrict__ resid, const float* __restrict__ weight, bf16* __restrict__ rows,
                       float* __restrict__ sums) {
-  extern __shared__ f32x4 red[];  // [waves][64]
+  extern __shared__ f32x4 red[];  // [waves][NB][64]
   const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), waves = blockDim.x / kWave;
   const int wr = blockIdx.x * ROWS + lane % ROWS;
-  const int token = threadIdx.x / ROWS, r = threadIdx.x % ROWS, row = blockIdx.x * ROWS + r;
-  const bool mine = token < x.n;
-  const size_t at = static_cast<size_t>(mine ? token : 0) * m + row;
-  float old = 0.f, w = 0.f;
-  if (mine) {
-    old = resid[at];
+  const int inside = threadIdx.x / ROWS, r = threadIdx.x % ROWS, row = blockIdx.x * ROWS + r;
+  float old[NB], w = 0.f;
+#pragma unroll
+  for (int c = 0; c < NB; ++c) {
+    const int token = few_first<NB>() + c * 16 + inside;
+    old[c] = inside < 16 && token < x.n ? resid[static_cast<size_t>(token) * m + row] : 0.f;
+  }
+  if (inside < 16) {
     w = weight[row];
-    if (bias) old += bias[row];
+    if (bias) {
+      const float add = bias[row];
+#pragma unroll
+      for (int c = 0; c < NB; ++c) old[c] += add;
+    }
   }
   const u32x4* const wrow[1] = {wt + static_cast<size_t>(wr / 16) * ktiles * kWave + wr % 16 + lane / 16 * 16};
-  f32x4 acc[1];
-  few_multiply<C, 4, 1>(acc, wrow, x, ktiles, wave, waves, [] {});
-  red[wave * kWave + lane] = acc[0];
-  __syncthreads();
-  if (threadIdx.x >= 16 * ROWS) return;
-  const float v = few_sum(red, kWave, r, token, waves) + old;
-  float square = v * v;
+  f32x4 acc[1][NB];
+  few_multiply<C, 4, 1, NB>(acc, wrow, x, ktiles, wave, waves, [] {});
 #pragma unroll
-  for (int off = 1; off < ROWS; off <<= 1) square += __shfl_xor(square, off, kWave);
-  if (!mine) return;
-  resid[at] = v;
-  rows[(static_cast<size_t>(row / 8) * x.n + token) * 8 + row % 8] = from_float<bf16>(v * w);
-  if (r == 0) sums[static_cast<size_t>(blockIdx.x) * x.n + token] = square;
+  for (int c = 0; c < NB; ++c) red[(wave * NB + c) * kWave + lane] = acc[0][c];
+  __syncthreads();
+  if (inside >= 16) return;
+#pragma unroll
+  for (int c = 0; c < NB; ++c) {
+    const int token = few_first<NB>() + c * 16 + inside;
+    const float v = few_sum(red + c * kWave, NB * kWave, r, inside, waves) + old[c];
+    float square = v * v;
+#pragma unroll
+    for (int off = 1; off < ROWS; off <<= 1) square += __shfl_xor(square, off, kWave);
+    if (token >= x.n) continue;
+    resid[static_cast<size_t>(token) * m + row] = v;
+    rows[(static_cast<size_t>(row / 8) * x.n + token) * 8 + row % 8] = from_float<bf16>(v * w);
+    if (r == 0) sums[static_cast<size_t>(blockIdx.x) * x.n + token] = square;
+  }
 }
 
 // A gated product: a workgroup for a gate block and its up block.
-template <int C, int LOADS>
+template <int C, int LOADS, int NB>
 __global__ void __launch_bounds__(kFewWaves* kWave)
     few_gated_kernel(FewRows x, const u32x4* __restrict__ wt, int ktiles, int m, FewScale scaled, const float* __restrict__ args,
                      bf16* __restrict__ out, int ldo, int act) {
-  extern __shared__ f32x4 red[];  // [waves][2][64], then the squares' sums by wavefront [waves][16]
+  extern __shared__ f32x4 red[];  // [waves][2][NB][64], then the squares' sums by wavefront [waves][16 NB]
   const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), waves = blockDim.x / kWave;
-  float* part = reinterpret_cast<float*>(red + waves * 2 * kWave);
-  FewSquares<LOADS> squares;
+  float* part = reinterpret_cast<float*>(red + waves * 2 * NB * kWave);
+  FewSquares<LOADS, NB> squares;
   squares.load(scaled, x.n);
   const u32x4* first = wt + static_cast<size_t>(blockIdx.x) * 2 * ktiles * kWave + lane;
   const u32x4* const wrow[2] = {first, first + static_cast<size_t>(ktiles) * kWave};
-  f32x4 acc[2];
-  few_multiply<C, 2, 2>(acc, wrow, x, ktiles, wave, waves, [&] { if (LOADS) squares.leave(part); });
-  red[(wave * 2) * kWave + lane] = acc[0];
-  red[(wave * 2 + 1) * kWave + lane] = acc[1];
+  f32x4 acc[2][NB];
+  few_multiply<C, 2, 2, NB>(acc, wrow, x, ktiles, wave, waves, [&] { squares.leave(part); });
+#pragma unroll
+  for (int c = 0; c < NB; ++c) {
+    red[(wave * 2 * NB + c) * kWave + lane] = acc[0][c];
+    red[((wave * 2 + 1) * NB + c) * kWave + lane] = acc[1][c];
+  }
   __syncthreads();
-  const int token = threadIdx.x / 16, r = threadIdx.x % 16, row = blockIdx.x * 16 + r;
-  if (token >= x.n || row >= m) return;
-  const float s = squares.scale(scaled, part, token, waves);
-  const float g = few_sum(red, 2 * kWave, r, token, waves) * s, u = few_sum(red + kWave, 2 * kWave, r, token, waves) * s;
-  const size_t at = ldo ? static_cast<size_t>(token) * ldo + row : (static_cast<size_t>(row / 8) * x.n + token) * 8 + row % 8;
-  out[at] = from_float<bf16>(gate_times_up(g, u, act, args));
+  for (int e = threadIdx.x; e < NB * 256; e += blockDim.x) {
+    const int inside = e / 16, token = few_first<NB>() + inside, r = e % 16, row = blockIdx.x * 16 + r;
+    if (token >= x.n || row >= m) continue;
+    const float s = squares.scale(scaled, part, inside, waves);
+    const f32x4* mine = red + inside / 16 * kWave;
+    const float g = few_sum(mine, 2 * NB * kWave, r, inside % 16, waves) * s;
+    const float u = few_sum(mine + NB * kWave, 2 * NB * kWave, r, inside % 16, waves) * s;
+    const size_t at = ldo ? static_cast<size_t>(token) * ldo + row : (static_cast<size_t>(row / 8) * x.n + token) * 8 + row % 8;
+    out[at] = from_float<bf16>(gate_times_up(g, u, act, args));
+  }
 }
 
 // Projections to queries, keys and values.  A workgroup forms 16 rows of the stacked matrix: of a query or key head 8 elements
@@ -230,21 +263,22 @@ __global__ void __launch_bounds__(kFewWaves* kWave)
   const bool turned = head < heads + kv_heads;
   // this workgroup's first row and, eight rows on, where the other eight begin
   const int first = head * head_dim + group * (turned ? 8 : 16), second = first + (turned ? head_dim / 2 : 8);
-  FewSquares<LOADS> squares;
+  FewSquares<LOADS, 1> squares;
   squares.load(scaled, x.n);
   if (wave == waves) {
     if (LOADS) squares.leave(part);
-    if (lane < x.n) {
-      const int pos = positions[lane];
+    if (lane < 16 && few_first<1>() + lane < x.n) {
+      const int pos = positions[few_first<1>() + lane];
       int page = -1;
-      if (write_kv && head >= heads) page = tables[static_cast<size_t>(token_seq[lane]) * table_stride + pos / page_size];
+      if (write_kv && head >= heads)
+        page = tables[static_cast<size_t>(token_seq[few_first<1>() + lane]) * table_stride + pos / page_size];
       page_of[lane] = page >= 0 && page < num_pages ? page : -1;  // (outside: a host bug; never dereferenced)
       slot_of[lane] = pos % page_size;
     }
     if (turned) {
 #pragma unroll
       for (int e = lane; e < 128; e += kWave) {  // (angles as in rope_kv.hip)
-        const int token = e / 8 < x.n ? e / 8 : x.n - 1;
+        const int token = min(few_first<1>() + e / 8, x.n - 1);
         const float angle = static_cast<float>(positions[token]) * inv_freq[group * 8 + e % 8];
         const double wide = static_cast<double>(angle);
         const double turns = rint(wide * 0.15915494309189535);
@@ -258,18 +292,18 @@ __global__ void __launch_bounds__(kFewWaves* kWave)
   } else {
     const int wr = lane % 16 < 8 ? first + lane % 16 : second + lane % 16 - 8;
     const u32x4* const wrow[1] = {wt + static_cast<size_t>(wr / 16) * ktiles * kWave + wr % 16 + lane / 16 * 16};
-    f32x4 acc[1];
-    few_multiply<C, 4, 1>(acc, wrow, x, ktiles, wave, waves, [&] { if (LOADS) squares.leave(part); });
-    red[wave * kWave + lane] = acc[0];
+    f32x4 acc[1][1];
+    few_multiply<C, 4, 1, 1>(acc, wrow, x, ktiles, wave, waves, [&] { if (LOADS) squares.leave(part); });
+    red[wave * kWave + lane] = acc[0][0];
   }
-  const int token = threadIdx.x / 8, i = threadIdx.x % 8;
+  const int inside = threadIdx.x / 8, token = few_first<1>() + inside, i = threadIdx.x % 8;
   float b1 = 0.f, b2 = 0.f;
   if (bias) b1 = bias[first + i], b2 = bias[second + i];
   __syncthreads();
-  if (token >= x.n) return;
-  const float s = squares.scale(scaled, part, token, waves + 1);
-  const float x1 = few_sum(red, kWave, i, token, waves) * s + b1, x2 = few_sum(red, kWave, i + 8, token, waves) * s + b2;
-  const float c = turned ? cosine[token][i] : 1.f, t = turned ? sine[token][i] : 0.f;
+  if (inside >= 16 || token >= x.n) return;
+  const float s = squares.scale(scaled, part, inside, waves + 1);
+  const float x1 = few_sum(red, kWave, i, inside, waves) * s + b1, x2 = few_sum(red, kWave, i + 8, inside, waves) * s + b2;
+  const float c = turned ? cosine[inside][i] : 1.f, t = turned ? sine[inside][i] : 0.f;
   const float o1 = turned ? x1 * c - x2 * t : x1, o2 = turned ? x2 * c + x1 * t : x2;
   if (head < heads) {
     bf16* row = out + static_cast<size_t>(token) * (heads + 2 * kv_heads) * head_dim;
@@ -277,10 +311,10 @@ __global__ void __launch_bounds__(kFewWaves* kWave)
     row[second + i] = from_float<bf16>(o2);
     return;
   }
-  if (page_of[token] < 0) return;
+  if (page_of[inside] < 0) return;
   const int kv = turned ? head - heads : head - heads - kv_heads;
-  const size_t base = (static_cast<size_t>(page_of[token]) * kv_heads + kv) * page_size * head_dim;
-  const int slot = slot_of[token], e1 = first - head * head_dim + i, e2 = second - head * head_dim + i;
+  const size_t base = (static_cast<size_t>(page_of[inside]) * kv_heads + kv) * page_size * head_dim;
+  const int slot = slot_of[inside], e1 = first - head * head_dim + i, e2 = second - head * head_dim + i;
   if (turned) {
     k_pool[base + key_offset(slot, e1, page_size, head_dim)] = from_float<bf16>(o1);
     k_pool[base + key_offset(slot, e2, page_size, head_dim)] = from_float<bf16>(o2);
@@ -297,7 +331,7 @@ using namespace shk;
 static bool few_rows_of(FewRows* x, const void* a, int lda, int n, int k) {
   const bool pieces = lda == 0;  // [k / 8][n][8]
   *x = FewRows{static_cast<const bf16*>(a), pieces ? 8 : lda, pieces ? n : 1, n, k};
-  return n >= 0 && n <= 16 && k > 0 && k % 8 == 0 && (pieces || (lda >= k && lda % 8 == 0));
+  return n >= 0 && n <= 64 && k > 0 && k % 8 == 0 && (pieces || (lda >= k && lda % 8 == 0));
 }
 
 // Wavefronts that share k: where four to eight of them hold all their tiles at once, the number that holds the fewest
@@ -341,11 +375,27 @@ constexpr int kFewMostLoads = 16;
 // halves, 2048 x 11008 12.7 and 11.1; 3584 x 18944 23.2 and 32.1.
 static int few_stream_rows(int m) { return m <= 2048 ? 8 : 16; }
 
+// The most rows * k for which 17 to 64 tokens go this way: every 16 of them read the weights again, from the caches.
+// At 17 / 32 / 64 tokens, with the norm: 896 x 896 7.6 / 7.6 / 7.6 -> 3.6 / 3.6 / 4.7, 896 x 4864 10.3 / 11.0 / 12.2 -> 6.3 / 6.6 / 9.5,
+// but 1536 x 8960 12.7 / 13.5 / 16.9 -> 17.5 / 18.6 / 26.6.  Heads, with the position kernel: 1152 x 896 7.7 / 7.7 / 7.8 -> 4.4 / 4.6 /
+// 5.3, 2560 x 2048 9.9 / 11.1 / 14.0 -> 9.2 / 9.7 / 13.3, 4608 x 3584 13.7 / 14.4 / 18.1 -> 16.9 / 17.8 / 29.  Gated, without the norm
+// that it spares: 9728 x 896 7.2 / 7.4 / 10.0 -> 7.5 / 7.9 / 10.4, 17920 x 1536 12.9 / 13.5 / 16.8 -> 13.7 / 15.0 / 23.2.
+constexpr long long kFewStreamMost = 5 * 1000 * 1000, kFewHeadsMost = 6 * 1000 * 1000, kFewGatedMost = 10 * 1000 * 1000;
+
+static bool few_takes(int n, int m, int k, long long most) {
+  return n <= 16 || (n <= 64 && static_cast<long long>(m) * k <= most);
+}
+
 // Not where a second round of workgroups would be nearly empty: 320 of them (5120 x 5120 at 8 tokens 14.3 us for product in shares
 // and norm, 15.1 here; 5120 x 13824 28.0 and 31.4).  256 are a round: 4096 x 14336 23.7 -> 20.0.
-extern "C" int shk_few_stream_sums(int m, int k) {
-  return m > 0 && m <= 4096 && m % 16 == 0 && k > 0 && k % 8 == 0 ? m / few_stream_rows(m) : 0;
+extern "C" int shk_few_stream_sums(int n, int m, int k) {
+  return m > 0 && m <= 4096 && m % 16 == 0 && k > 0 && k % 8 == 0 && few_takes(n, m, k, kFewStreamMost) ? m / few_stream_rows(m) : 0;
 }
+
+// `m` rows of the gate and as many of the other matrix; the k columns may come with as many sums as few_stream leaves.
+extern "C" int shk_few_gated_takes(int n, int m, int k) { return m > 0 && k > 0 && k % 8 == 0 && few_takes(n, 2 * m, k, kFewGatedMost); }
+
+extern "C" int shk_few_heads_takes(int n, int m, int k) { return m > 0 && k > 0 && k % 8 == 0 && few_takes(n, m, k, kFewHeadsMost); }
 
 extern "C" int shk_few_stream(const void* a, int lda, int n, int k, const void* wt, int m, const float* bias, float* resid,
                               const float* weight, void* rows, float* sums, void* stream) {
@@ -355,9 +405,13 @@ extern "C" int shk_few_stream(const void* a, int lda, int n, int k, const void* 
   SHK_REQUIRE(a && wt && resid && weight && rows && sums, "few_stream: null pointer");
   SHK_REQUIRE(reinterpret_cast<uintptr_t>(a) % 16 == 0, "few_stream: rows are not 16-byte aligned");
   const int kt = (k + 31) / 32, waves = few_waves(kt, kFewTiles), rows_each = few_stream_rows(m);
+  // two blocks of tokens in a workgroup where many tokens would have a long k read four times over (896 x 4864 at 64
+  // tokens 10.4 us in one, 9.5; at 32 6.6 in one, 10.0)
+  const int nb = n > 32 && kt > kFewTiles * waves ? 2 : 1;
   with_tiles<kFewTiles>((kt + waves - 1) / waves, [&](auto c) {
-    const auto kernel = rows_each == 8 ? few_stream_kernel<c.value, 8> : few_stream_kernel<c.value, 16>;
-    kernel<<<m / rows_each, waves * kWave, waves * kWave * sizeof(f32x4), static_cast<hipStream_t>(stream)>>>(
+    const auto kernel = nb == 2 ? rows_each == 8 ? few_stream_kernel<c.value, 8, 2> : few_stream_kernel<c.value, 16, 2>
+                        : rows_each == 8 ? few_stream_kernel<c.value, 8, 1> : few_stream_kernel<c.value, 16, 1>;
+    kernel<<<dim3(m / rows_each, (n + 16 * nb - 1) / (16 * nb)), waves * kWave, nb * waves * kWave * sizeof(f32x4), static_cast<hipStream_t>(stream)>>>(
         x, static_cast<const u32x4*>(wt), kt, m, bias, resid, weight, static_cast<bf16*>(rows), sums);
   });
   SHK_LAUNCH_CHECK("few_stream");
@@ -378,11 +432,13 @@ extern "C" int shk_few_gated(const void* a, int lda, int n, int k, const void* w
   // four wavefronts where they hold their tiles at once (9728 x 896: 5.8 us with one token, 5.9 in eight), else eight
   // (22016 x 2048 15.6, 15.9 in four)
   const int kt = (k + 31) / 32, waves = kt <= 4 * kFewPairs ? 4 : 8;
-  SHK_REQUIRE(count <= kFewMostLoads * waves * 4, "few_gated: too many sums (%d)", count);
-  with_loads(count, waves * kWave, [&](auto loads) {
+  SHK_REQUIRE(count <= kFewMostLoads * waves * 4 / (n > 16 ? 2 : 1), "few_gated: too many sums (%d)", count);
+  const int nb = n > 16 ? 2 : 1;  // (9728 x 896 at 17 / 32 / 64 tokens 8.2 / 8.5 / 12.4 us in one, 7.5 / 7.9 / 10.4)
+  with_loads(count, waves * kWave / nb, [&](auto loads) {
     with_tiles<kFewPairs>((kt + waves - 1) / waves, [&](auto c) {
-      const size_t lds = waves * (2 * kWave * sizeof(f32x4) + 16 * sizeof(float));
-      few_gated_kernel<c.value, loads.value><<<(m + 15) / 16, waves * kWave, lds, static_cast<hipStream_t>(stream)>>>(
+      const size_t lds = nb * waves * (2 * kWave * sizeof(f32x4) + 16 * sizeof(float));
+      const auto kernel = nb == 2 ? few_gated_kernel<c.value, loads.value, 2> : few_gated_kernel<c.value, loads.value, 1>;
+      kernel<<<dim3((m + 15) / 16, (n + 16 * nb - 1) / (16 * nb)), waves * kWave, lds, static_cast<hipStream_t>(stream)>>>(
           x, static_cast<const u32x4*>(wt), kt, m, scaled, args, static_cast<bf16*>(out), ldo, gated);
     });
   });
@@ -414,7 +470,7 @@ extern "C" int shk_few_heads(const void* a, int lda, int n, int k, const void* w
   with_loads(sums ? count : 0, (waves + 1) * kWave, [&](auto loads) {
     with_tiles<kFewTiles>((kt + waves - 1) / waves, [&](auto c) {
       const size_t lds = waves * kWave * sizeof(f32x4) + (waves + 1) * 16 * sizeof(float);
-      few_heads_kernel<c.value, loads.value><<<groups, (waves + 1) * kWave, lds, static_cast<hipStream_t>(stream)>>>(
+      few_heads_kernel<c.value, loads.value><<<dim3(groups, (n + 15) / 16), (waves + 1) * kWave, lds, static_cast<hipStream_t>(stream)>>>(
           x, static_cast<const u32x4*>(wt), kt, scaled, bias, static_cast<bf16*>(out), heads, kv_heads, head_dim, inv_freq, positions,
           token_seq, tables, table_stride, static_cast<bf16*>(k_pool), static_cast<bf16*>(v_pool), page_size, num_pages, write_kv,
           magnitude);

@@ -104,9 +104,9 @@ class Runtime:
 
     def onto_sums(self, ctx, w: LinearWeight) -> int:
         """Groups of sums that linear_onto() leaves of its product with `w` in this step, 0 where it leaves it pending."""
-        if ctx.onto is None or w.tiled is None or ctx.num_tokens > ops.FEW_TOKENS or w.cols % 8:
+        if ctx.onto is None or w.tiled is None:
             return 0
-        return ops.few_stream_sums(w.rows, w.cols)
+        return ops.few_stream_sums(ctx.num_tokens, w.rows, w.cols)
 
     def linear_deferred(self, ctx, name: str, x, w: LinearWeight, bias=None, reader="norm",
                         keep_float32: bool = False):

@@ -51,7 +51,9 @@ _SIGNATURES = {
     "shk_gemm_bf16_keeps_float32_unaligned": [_I, _I, _I],
     "shk_gemm_bf16_parts": [_I, _I, _I, _I],
     "shk_gemm_bf16_tiles": [_I, _I, _I, _I, _I, _I, _P],
-    "shk_few_stream_sums": [_I, _I],
+    "shk_few_stream_sums": [_I, _I, _I],
+    "shk_few_gated_takes": [_I, _I, _I],
+    "shk_few_heads_takes": [_I, _I, _I],
     "shk_few_stream": [_P, _I, _I, _I, _P, _I, _P, _P, _P, _P, _P, _P],
     "shk_few_gated": [_P, _I, _I, _I, _P, _P, _I, _F, _P, _P, _I, _I, _I, _P],
     "shk_few_heads": [_P, _I, _I, _I, _P, _P, _I, _F, _P, _P, _I, _I, _I, _P, _P, _P, _P, _I, _P, _P, _I, _I, _I, _F, _P],

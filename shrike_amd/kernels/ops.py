@@ -508,13 +508,23 @@ class ScaledRows:
         return (self.rows.shape[1], 8 * self.rows.shape[0])
 
 
-FEW_TOKENS = 16  # the most that few_stream, few_gated and few_heads take
+FEW_TOKENS = 64  # the most that few_stream, few_gated and few_heads take
 
 
-def few_stream_sums(m: int, k: int) -> int:
-    """Groups of columns that few_stream sums the squares of (0: it does not take an [m, k] matrix, or not as well as a
-    product and a norm do)."""
-    return int(load().shk_few_stream_sums(m, k))
+def few_stream_sums(n: int, m: int, k: int) -> int:
+    """Groups of columns that few_stream sums the squares of for n rows and an [m, k] matrix (0: it does not take them, or
+    not as well as a product and a norm do)."""
+    return int(load().shk_few_stream_sums(n, m, k))
+
+
+def few_gated_takes(n: int, m: int, k: int) -> bool:
+    """Whether few_gated takes n rows and two [m, k] matrices as well as a product of normed rows."""
+    return bool(load().shk_few_gated_takes(n, m, k))
+
+
+def few_heads_takes(n: int, m: int, k: int) -> bool:
+    """Whether few_heads takes n rows and an [m, k] matrix, and better than a product and the position kernel."""
+    return bool(load().shk_few_heads_takes(n, m, k))
 
 
 def _few_rows(who, x, k, wt, numel):
@@ -550,8 +560,8 @@ def few_stream(a, wt, m: int, k: int, resid, weight, rows, sums, bias=None) -> N
         raise KernelError(f"few_stream: resid must be contiguous [{n}, {m}], weight and bias as wide")
     if m % 8 or tuple(rows.shape) != (m // 8, n, 8) or not rows.is_contiguous() or rows.dtype != torch.bfloat16:
         raise KernelError(f"few_stream: rows must be contiguous bfloat16 [{m // 8}, {n}, 8]")
-    if tuple(sums.shape) != (few_stream_sums(m, k), n) or not sums.is_contiguous():
-        raise KernelError(f"few_stream: sums must be contiguous [{few_stream_sums(m, k)}, {n}]")
+    if tuple(sums.shape) != (few_stream_sums(n, m, k), n) or not sums.is_contiguous():
+        raise KernelError(f"few_stream: sums must be contiguous [{few_stream_sums(n, m, k)}, {n}]")
     check(load().shk_few_stream(
         p, lda, n, k, _dev(wt, "wt"), m, None if bias is None else _dev(bias, "bias", torch.float32),
         _dev(resid, "resid", torch.float32), _dev(weight, "weight", torch.float32), _dev(rows, "rows"),
@@ -559,7 +569,7 @@ def few_stream(a, wt, m: int, k: int, resid, weight, rows, sums, bias=None) -> N
 
 
 def few_gated(x: ScaledRows, wt, m: int, k: int, out, activation, gate_args=None) -> None:
-    """The gated product of gemm_tiled_weight of up to 16 rows that are still to be divided by their root mean square;
+    """The gated product of gemm_tiled_weight of up to 64 rows that are still to be divided by their root mean square;
     `out` [n, m], or pieces [m / 8, n, 8]."""
     rows, sums, count, eps = _few_sums("few_gated", x)
     p, lda, n = _few_rows("few_gated", rows, k, wt, 2 * tiled_numel(m, k))
@@ -576,7 +586,7 @@ def few_gated(x: ScaledRows, wt, m: int, k: int, out, activation, gate_args=None
 
 def few_heads(x, wt, k: int, out, heads, kv_heads, head_dim, inv_freq, positions, token_seq, tables, k_pool, v_pool,
               page_size, write_kv=True, bias=None, magnitude: float = 1.0) -> None:
-    """The projections of up to 16 rows (normed, or ScaledRows) to queries, keys and values, rotated whole as in
+    """The projections of up to 64 rows (normed, or ScaledRows) to queries, keys and values, rotated whole as in
     rope_kv_store: queries into out's query columns, keys and values into their pages."""
     rows, sums, count, eps = _few_sums("few_heads", x)
     width = (heads + 2 * kv_heads) * head_dim

@@ -621,7 +621,7 @@ class PagedAttention(Mixer):
             return False
         table = self.position.rotary_table()
         return (table is not None and table[1] == s.head_dim and s.head_dim % 16 == 0 and self.w_qkv.tiled is not None
-                and ctx.num_tokens <= ops.FEW_TOKENS and self.width % 8 == 0)
+                and ops.few_heads_takes(ctx.num_tokens, self.w_qkv.rows, self.width))
 
     def forward(self, ctx, x: torch.Tensor, cache) -> torch.Tensor:
         s = self.spec

@@ -21,7 +21,8 @@ class SwiGLU(FeedForward):
         return type(self).forward is SwiGLU.forward
 
     def takes_scaled(self, ctx) -> bool:
-        return self.ends_onto and self.w_gate_up.tiled is not None and ctx.num_tokens <= ops.FEW_TOKENS and self.width % 8 == 0
+        return (self.ends_onto and self.w_gate_up.tiled is not None
+                and ops.few_gated_takes(ctx.num_tokens, self.inter, self.width))
 
     def params(self):
         inter, h = self.spec.intermediate_size, self.width
