@@ -105,6 +105,16 @@ int shk_retile_f32(const void* w, int m, int k, void* wt, void* stream);
 int shk_gemm_f32_tiled_weight(const void* a, const void* wt, const float* bias, void* out, int n, int m, int k, int lda,
                               int ldo, int accumulate, void* stream);
 
+// Up to 16 rows (16-byte aligned, k a multiple of 16), the same bits.  shk_gemm_f32_groups: out [4][n][m] receives the sum's four
+// groups, whose sum in order is the product (shk_add_rmsnorm adds them); shk_gemm_f32_splits: 4 where that is worth it, else 1.
+// shk_gemm_f32_gated: out[n, m] = act(g) * (u + up_shift) of the product [g | u] with 2 m features, as shk_act_mul forms it
+// (m a multiple of 16).
+int shk_gemm_f32_splits(int n, int m, int k);
+int shk_gemm_f32_groups(const void* a, const void* wt, void* out, int n, int m, int k, int lda, void* stream);
+int shk_gemm_f32_gated_takes(int n, int m, int k);
+int shk_gemm_f32_gated(const void* a, const void* wt, void* out, int n, int m, int k, int lda, int act, float limit,
+                       float up_shift, void* stream);
+
 // wt = the tiled layout of the row-major bfloat16 matrix w[m, k] (see
 // gemm_bf16.hip): ceil(m/16) * ceil(k/32) tiles of 1 KiB.
 int shk_retile_weight(const void* w, int m, int k, void* wt, void* stream);

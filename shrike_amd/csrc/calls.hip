@@ -67,6 +67,8 @@ const Launcher kLaunchers[] = {
     SHK_LAUNCHER(shk_gemm),
     SHK_LAUNCHER(shk_gemm_f32_tiled_weight),
     SHK_LAUNCHER(shk_gemm_bf16_tiled_weight),
+    SHK_LAUNCHER(shk_gemm_f32_groups),
+    SHK_LAUNCHER(shk_gemm_f32_gated),
     SHK_LAUNCHER(shk_few_stream),
     SHK_LAUNCHER(shk_few_gated),
     SHK_LAUNCHER(shk_few_heads),

@@ -491,8 +491,8 @@ extern "C" int shk_add_rmsnorm(float* resid, const void* delta, const float* wei
   const auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
   const bool vec = hidden % 4 == 0 && hidden <= 1024 * 4 * kNormVecs && aligned(resid) &&
                    aligned(weight) && aligned(out) && (!delta || aligned(delta));
-  SHK_REQUIRE(delta_splits == 0 || (delta && vec && dtype == kBF16 && resid_rows > 0),
-              "add_rmsnorm: partial sums need bfloat16 output, hidden %% 4 == 0 and at most 8192");
+  SHK_REQUIRE(delta_splits == 0 || (delta && vec && resid_rows > 0),
+              "add_rmsnorm: partial sums need hidden %% 4 == 0 and at most 8192");
   const size_t stride = static_cast<size_t>(resid_rows) * hidden;
   const int splits = delta_splits > 0 ? delta_splits : 1;
 #define SHK_NORM(T, TD, THREADS)                                                              \
@@ -506,7 +506,7 @@ extern "C" int shk_add_rmsnorm(float* resid, const void* delta, const float* wei
     else                                 \
       SHK_NORM(T, TD, 1024);             \
   } while (0)
-  if (delta_splits > 0) {
+  if (delta_splits > 0 && dtype == kBF16) {
     SHK_NORM_T(bf16, float);
   } else if (vec && dtype == kF32) {
     SHK_NORM_T(float, float);

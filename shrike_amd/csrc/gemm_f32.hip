@@ -23,6 +23,8 @@
 // rows 75 TFLOP/s; gemm_f32_lds_kernel, which shares them, 97).  Before, one workgroup per 64 x 64 results with vector
 // instructions: a 0.5B decode step of four requests 23.9 ms (2.4 with this kernel, 1.56 with attention_f32.hip as
 // well), a 509-token prompt 42.6 ms (18.9, 6.5; 5.4 with operands shared); the logits' error against 64 bits 6.4e-7 (2.5e-7).
+#include <type_traits>
+
 #include "api.h"
 #include "common.h"
 #include "gemm_wide.h"
@@ -32,6 +34,22 @@ namespace shk {
 typedef float mf4 __attribute__((ext_vector_type(4)));
 
 constexpr int kF32Segments = 16, kF32Group = 4;
+
+// act(gate) * up as act_mul_kernel forms it
+struct F32Gate {
+  int act;
+  float limit, up_shift;
+};
+__device__ __forceinline__ float f32_gate(float g, float u, F32Gate gate) {
+  if (gate.limit > 0.f) {
+    g = fminf(g, gate.limit);
+    u = fminf(fmaxf(u, -gate.limit), gate.limit);
+  }
+  u += gate.up_shift;
+  if (gate.act == 3) return fmaxf(g, 0.f) * u;
+  const float x = gate.act == 2 ? 2.f * 0.7978845608028654f * (g + 0.044715f * g * g * g) : gate.act == 4 ? 1.702f * g : g;
+  return g / (1.f + expf(-x)) * u;
+}
 constexpr int kDies = 8;
 
 // Four consecutive k of one row.  VEC: k and the rows are multiples of 16 bytes.
@@ -212,6 +230,117 @@ __global__ void __launch_bounds__(kWave * KW * MW * NW)
   }
 }
 
+// The same product, in the same order, for up to 16 rows, tiled weights and a k in whole steps of 16.  A workgroup's KW
+// wavefronts take a segment each (16), a group each (4), or with GROUPS the segments of the group blockIdx.y, whose sum is then
+// one of four parts [group][n][m] that the reader adds in order.  C > 0: a wavefront has at most C steps, all asked for at
+// once; 0: batches of five, two in flight.  ROWS = 8: a workgroup for half a block of features, where whole blocks leave
+// compute units idle.  GATED: w holds a gate matrix and behind it the other factor, m rows each (a multiple of 16); a workgroup
+// forms a block of both and stores what act_mul_kernel would of the two.
+// What bounds it: one round trip to memory and what a compute unit takes in (about 50 GB/s a workgroup).  Weights cold, us at 1 /
+// 4 / 16 rows: 896 x 896 4.8 / 5.0 / 6.4 in the kernel above, 3.7 / 3.8 / 4.9 here, 9728 x 896 11.1 / 10.5 / 13.0 and 8.6 / 8.7 / 11.4,
+// 3584 x 3584 28 / 29 / 39 and 12 / 12 / 15; 896 x 4864 13.0 / 13.3 / 18.8 and, in one workgroup a half block, 11.4 / 11.8 / 18.2.
+template <int KW, int ROWS, int C, bool GATED, bool GROUPS>
+__global__ void __launch_bounds__(kWave* KW)
+    gemm_f32_few_kernel(const float* __restrict__ a, const float* __restrict__ w, const float* __restrict__ bias,
+                        float* __restrict__ out, int n, int m, int k, int lda, int ldo, int accumulate, F32Gate gate) {
+  constexpr int RB = GATED ? 2 : 1, kMine = GROUPS ? 1 : kF32Segments / KW, kSteps = C > 0 ? C : 5;
+  static_assert(!GROUPS || (KW == kF32Group && !GATED), "a workgroup holds one group");
+  __shared__ mf4 sums[KW][RB][kWave];
+  const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int i = lane % 16, kg = lane / 16;
+  const int f = blockIdx.x * ROWS + i % ROWS, ktiles = k / 16;
+  const mf4* wr[RB];
+#pragma unroll
+  for (int r = 0; r < RB; ++r)
+    wr[r] = reinterpret_cast<const mf4*>(w) + static_cast<size_t>(f / 16 + r * (m / 16)) * ktiles * kWave + kg * 16 + f % 16;
+  const float* ar = a + static_cast<size_t>(min(i, n - 1)) * lda + kg * 4;
+
+  const int seg_steps = (k + 16 * kF32Segments - 1) / (16 * kF32Segments);
+  const int first = (GROUPS ? blockIdx.y * kF32Group : 0) + wave * kMine;
+  const int begin = min(first * seg_steps, ktiles), steps = min(begin + kMine * seg_steps, ktiles) - begin;
+  mf4 acc[RB], group[RB];
+#pragma unroll
+  for (int r = 0; r < RB; ++r) acc[r] = group[r] = mf4{0.f, 0.f, 0.f, 0.f};
+  struct Batch {
+    mf4 w[kSteps][RB], a[kSteps];
+  };
+  auto load = [&](Batch& b, int s0) {  // (unconditional: a step beyond the last is the matrix's last)
+#pragma unroll
+    for (int u = 0; u < kSteps; ++u) {
+      const int s = min(begin + s0 + u, ktiles - 1);
+#pragma unroll
+      for (int r = 0; r < RB; ++r) b.w[u][r] = __builtin_nontemporal_load(wr[r] + static_cast<size_t>(s) * kWave);
+      b.a[u] = *reinterpret_cast<const mf4*>(ar + s * 16);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  int in_seg = 0;
+  auto multiply = [&](const Batch& b, int s0) {
+#pragma unroll
+    for (int u = 0; u < kSteps; ++u) {
+      // (beyond the last step: zeros times zeros, which leave a sum that began at zero as it is; a branch would take
+      // the loads with it)
+      const bool have = s0 + u < steps;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float x = have ? b.a[u][j] : 0.f;
+#pragma unroll
+        for (int r = 0; r < RB; ++r) acc[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(have ? b.w[u][r][j] : 0.f, x, acc[r], 0, 0, 0);
+      }
+      if (kMine > 1 && ++in_seg == seg_steps) {  // a segment ends
+        in_seg = 0;
+#pragma unroll
+        for (int r = 0; r < RB; ++r) group[r] += acc[r], acc[r] = mf4{0.f, 0.f, 0.f, 0.f};
+      }
+    }
+  };
+  Batch ping;
+  load(ping, 0);
+  if constexpr (C > 0) {
+    multiply(ping, 0);
+  } else {
+    Batch pong;
+    for (int s = 0; s < steps; s += 2 * kSteps) {
+      load(pong, s + kSteps);
+      multiply(ping, s);
+      load(ping, s + 2 * kSteps);
+      multiply(pong, s + kSteps);
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < RB; ++r) sums[wave][r][lane] = kMine > 1 ? group[r] + acc[r] : acc[r];
+  __syncthreads();
+  // element (feature, row): the wavefronts' shares in order
+  const int row = threadIdx.x / ROWS, at = threadIdx.x % ROWS, col = blockIdx.x * ROWS + at;
+  if (row >= n || col >= m) return;
+  float v[RB];
+#pragma unroll
+  for (int r = 0; r < RB; ++r) {
+    const float* p = reinterpret_cast<const float*>(&sums[0][r][at / 4 * 16 + row]) + at % 4;
+    constexpr int kNext = RB * kWave * 4;
+    v[r] = 0.f;
+    if (KW > 4) {
+#pragma unroll
+      for (int g = 0; g < KW; g += KW / 4) {
+        float s = 0.f;
+#pragma unroll
+        for (int x = 0; x < KW / 4; ++x) s += p[(g + x) * kNext];
+        v[r] += s;
+      }
+    } else {
+#pragma unroll
+      for (int x = 0; x < KW; ++x) v[r] += p[x * kNext];
+    }
+  }
+  float* dst = out + (GROUPS ? static_cast<size_t>(blockIdx.y) * n + row : static_cast<size_t>(row)) * ldo + col;
+  if constexpr (GATED) {
+    *dst = f32_gate(v[0], v[1], gate);
+  } else {
+    if (bias) v[0] += bias[col];
+    *dst = accumulate ? v[0] + *dst : v[0];
+  }
+}
+
 // The same product, in the same order, for many rows and more than 256 of k in whole stages of 32: four wavefronts, 2 x 2 of
 // RT x CT tiles, share their operands through LDS, loaded straight into it two stages ahead.  A wavefront walks all of
 // k, the tiles' sums of segment, group and all in its registers.  The operands of an instruction's 32 cycles are then a
@@ -371,6 +500,37 @@ static void launch_f32_lds(const F32Product& p, hipStream_t s) {
                                                                                     p.ldo, p.accumulate, vec_out);
 }
 
+// Whether gemm_f32_few_kernel takes a product of tiled weights.  (151936 x 896: 98 / 107 us at 4 / 16 rows in gemm_f32_kernel's
+// two blocks a wavefront, 90 / 121 here.)
+static bool f32_few(const F32Product& p) {
+  return p.n <= 16 && (p.m <= 32768 || p.n <= 8) && p.k % 16 == 0 && p.lda % 4 == 0 && reinterpret_cast<uintptr_t>(p.a) % 16 == 0;
+}
+
+// fn with the steps of a wavefront rounded up to one of a few constants, 0 for more than MOST.
+template <int MOST, typename Fn>
+static void with_steps(int steps, Fn fn) {
+  if (steps <= 2) fn(std::integral_constant<int, 2>{});
+  else if (steps <= 4) fn(std::integral_constant<int, 4>{});
+  else if (steps <= 6) fn(std::integral_constant<int, 6>{});
+  else if (steps <= MOST) fn(std::integral_constant<int, MOST>{});
+  else fn(std::integral_constant<int, 0>{});
+}
+
+// Half blocks of features and a segment a wavefront up to 2,048 features, the segments also for a k of up to 1,024, else a group
+// a wavefront: 9728 x 896 at 4 rows 8.7 us by segments, 10.0 by groups, 3584 x 3584 15.5 and 12.2, 3584 x 18944 at 16 rows 70 and 61.
+static void launch_f32_few(const F32Product& p, hipStream_t s) {
+  const int seg_steps = (p.k + 16 * kF32Segments - 1) / (16 * kF32Segments);
+  const auto go = [&](auto kernel, int waves, int rows) {
+    kernel<<<(p.m + rows - 1) / rows, waves * kWave, 0, s>>>(p.a, p.w, p.bias, p.out, p.n, p.m, p.k, p.lda, p.ldo, p.accumulate, F32Gate{});
+  };
+  if (p.m <= 2048)
+    with_steps<10>(seg_steps, [&](auto c) { go(gemm_f32_few_kernel<16, 8, c.value, false, false>, 16, 8); });
+  else if (p.k <= 1024)
+    with_steps<10>(seg_steps, [&](auto c) { go(gemm_f32_few_kernel<16, 16, c.value, false, false>, 16, 16); });
+  else
+    with_steps<16>(4 * seg_steps, [&](auto c) { go(gemm_f32_few_kernel<4, 16, c.value, false, false>, 4, 16); });
+}
+
 // The shape of the kernel for a size (results are the same bits in all of them).  Measured on the 0.5B
 // model's matrices, tiled weights, microseconds:
 //   up to 16 rows: 896 x 896 5 in one-tile workgroups of 16 segments (9 with four row blocks and four groups of
@@ -395,7 +555,9 @@ static void run_f32(const F32Product& p, hipStream_t s) {
   // whole stages of aligned rows, offsets within a tile of 32 bits
   const bool staged = TILED && p.batch == 1 && p.k % 32 == 0 && p.k > 256 && p.k <= 1 << 20 && p.lda % 4 == 0 && p.lda <= 1 << 20 &&
                       reinterpret_cast<uintptr_t>(p.a) % 16 == 0;
-  if (p.n <= 16) {
+  if (TILED && f32_few(p)) {
+    launch_f32_few(p, s);
+  } else if (p.n <= 16) {
     if (p.m <= 2048)
       launch_f32<1, 1, 16, 1, 1, 2, TILED>(p, s);
     else if (p.m <= 32768)
@@ -460,6 +622,52 @@ extern "C" int shk_retile_f32(const void* w, int m, int k, void* wt, void* strea
   retile_f32_kernel<<<static_cast<unsigned>((quads + 255) / 256), 256, 0, static_cast<hipStream_t>(stream)>>>(
       static_cast<const float*>(w), m, k, static_cast<float*>(wt), quads);
   SHK_LAUNCH_CHECK("retile_f32");
+  return 0;
+}
+
+// Groups in which shk_gemm_f32_groups leaves a product for its reader (1: it is formed whole): four where a long k would
+// be walked in few workgroups: with the norm that adds its output 896 x 4864 at 1 / 4 / 16 rows 13.7 / 14.1 / 20.7 us whole, 10.0 /
+// 10.2 / 13.2 in groups, 1536 x 8960 22.4 / 22.9 / 34.5 and 18.9 / 19.5 / 27.7.
+extern "C" int shk_gemm_f32_splits(int n, int m, int k) {
+  return n <= 16 && m <= 2048 && m % 4 == 0 && k >= 2048 && k % 16 == 0 ? kF32Segments / kF32Group : 1;
+}
+
+extern "C" int shk_gemm_f32_groups(const void* a, const void* wt, void* out, int n, int m, int k, int lda, void* stream) {
+  SHK_REQUIRE(n >= 0 && n <= 16 && m > 0 && k > 0 && k % 16 == 0 && lda >= k && lda % 4 == 0,
+              "gemm_f32_groups: bad sizes n=%d m=%d k=%d lda=%d", n, m, k, lda);
+  if (n == 0) return 0;
+  SHK_REQUIRE(a && wt && out && reinterpret_cast<uintptr_t>(wt) % 16 == 0 && reinterpret_cast<uintptr_t>(a) % 16 == 0,
+              "gemm_f32_groups: null or misaligned pointer");
+  with_steps<10>((k + 16 * kF32Segments - 1) / (16 * kF32Segments), [&](auto c) {
+    gemm_f32_few_kernel<4, 8, c.value, false, true><<<dim3((m + 7) / 8, kF32Segments / kF32Group), 4 * kWave, 0, static_cast<hipStream_t>(stream)>>>(
+        static_cast<const float*>(a), static_cast<const float*>(wt), nullptr, static_cast<float*>(out), n, m, k, lda, m, 0, F32Gate{});
+  });
+  SHK_LAUNCH_CHECK("gemm_f32_groups");
+  return 0;
+}
+
+// Whether shk_gemm_f32_gated takes a product of 2 m features, gate and other factor.
+extern "C" int shk_gemm_f32_gated_takes(int n, int m, int k) { return n <= 16 && m > 0 && m % 16 == 0 && k > 0 && k % 16 == 0; }
+
+extern "C" int shk_gemm_f32_gated(const void* a, const void* wt, void* out, int n, int m, int k, int lda, int act, float limit,
+                                  float up_shift, void* stream) {
+  SHK_REQUIRE(n >= 0 && n <= 16 && m > 0 && m % 16 == 0 && k > 0 && k % 16 == 0 && lda >= k && lda % 4 == 0,
+              "gemm_f32_gated: bad sizes n=%d m=%d k=%d lda=%d", n, m, k, lda);
+  SHK_REQUIRE(act >= 1 && act <= 4 && limit >= 0.f, "gemm_f32_gated: unknown gate");
+  if (n == 0) return 0;
+  SHK_REQUIRE(a && wt && out && reinterpret_cast<uintptr_t>(wt) % 16 == 0 && reinterpret_cast<uintptr_t>(a) % 16 == 0,
+              "gemm_f32_gated: null or misaligned pointer");
+  const int seg_steps = (k + 16 * kF32Segments - 1) / (16 * kF32Segments);
+  const F32Gate gate = {act, limit, up_shift};
+  const auto go = [&](auto kernel, int waves) {
+    kernel<<<m / 16, waves * kWave, 0, static_cast<hipStream_t>(stream)>>>(static_cast<const float*>(a), static_cast<const float*>(wt), nullptr,
+                                                                           static_cast<float*>(out), n, m, k, lda, m, 0, gate);
+  };
+  if (k <= 1024)  // (up to four steps a segment)
+    go(seg_steps <= 2 ? gemm_f32_few_kernel<16, 16, 2, true, false> : gemm_f32_few_kernel<16, 16, 4, true, false>, 16);
+  else
+    with_steps<16>(4 * seg_steps, [&](auto c) { go(gemm_f32_few_kernel<4, 16, c.value, true, false>, 4); });
+  SHK_LAUNCH_CHECK("gemm_f32_gated");
   return 0;
 }
 

@@ -149,7 +149,8 @@ class StepContext:
     # what the parts' prepare() added: device arrays, and host-side decisions
     extras: dict = field(default_factory=dict)
     notes: dict = field(default_factory=dict)
-    # (HiddenState, norm): the stream that a sublayer's last product may add to, leaving the norm's rows (Runtime.linear_onto)
+    # (HiddenState, norm, scaled): the stream that a sublayer's last product joins (Runtime.linear_onto), the norm that comes
+    # next, and whether the product may add to the stream and leave the norm's rows for the norm's reader to divide
     onto: tuple | None = None
     # everything a step's launches may depend on, for parts that say launches_follow_shape
     shape_key: tuple = ()

@@ -67,6 +67,10 @@ class Runtime:
         if w.tiled is not None:
             ops.gemm_tiled_weight(x, w.tiled, w.rows, w.cols, out, gated=activation, gate_args=w.gate_args)
             return
+        inter = w.rows // 2
+        if ops.gemm_f32_gated_takes(x.shape[0], inter, w.cols) and ops.f32_rows_aligned(x) and out.is_contiguous():
+            ops.gemm_f32_gated(x, w.tiled_f32, inter, w.cols, out, activation, limit, up_shift)
+            return
         gate_up = ctx.buffer("ffn_gate_up", (x.shape[0], w.rows), self.dtype)
         self.linear(x, w, gate_up)
         ops.act_mul(gate_up, out, activation, limit, up_shift)
@@ -88,12 +92,19 @@ class Runtime:
     def linear_onto(self, ctx, name: str, x, w: LinearWeight, bias=None):
         """linear_deferred() for a sublayer's last product.  Where the block has said which stream it joins and which norm
         comes next (ctx.onto) and the tokens are few, the product adds to the stream itself and leaves the norm's rows
-        in hidden.scaled, and nothing is pending: None."""
+        in hidden.scaled, and nothing is pending: None.  In float32, where a norm's rows keep their bits, it may leave parts
+        for the norm to add."""
         count = self.onto_sums(ctx, w) if x.dim() == 3 or ops.rows_aligned(x) else 0
         target, ctx.onto = ctx.onto, None
         if not count:
+            n = x.shape[0]
+            if target is not None and w.tiled is None and bias is None and w.rows <= 8192 and ops.f32_rows_aligned(x) \
+                    and ops.gemm_f32_splits(n, w.rows, w.cols) > 1:
+                parts = ctx.buffer(name + "_parts", (ops.gemm_f32_splits(n, w.rows, w.cols), n, w.rows), torch.float32)
+                ops.gemm_f32_groups(x, w.tiled_f32, w.rows, w.cols, parts)
+                return ops.SplitSum(parts)
             return self.linear_deferred(ctx, name, x, w, bias=bias)
-        hidden, norm = target
+        hidden, norm, _ = target
         n = hidden.resid.shape[0]
         rows = ctx.buffer("stream_rows", (w.rows // 8, n, 8), self.dtype)
         sums = ctx.buffer("stream_sums", (count, n), torch.float32)
@@ -104,7 +115,7 @@ class Runtime:
 
     def onto_sums(self, ctx, w: LinearWeight) -> int:
         """Groups of sums that linear_onto() leaves of its product with `w` in this step, 0 where it leaves it pending."""
-        if ctx.onto is None or w.tiled is None:
+        if ctx.onto is None or not ctx.onto[2] or w.tiled is None:
             return 0
         return ops.few_stream_sums(ctx.num_tokens, w.rows, w.cols)
 

@@ -372,6 +372,45 @@ def gemm_f32_tiled_weight(a, wt, m: int, k: int, out, bias=None, accumulate=Fals
         a.stride(0), out.stride(0), int(bool(accumulate)), _stream()))
 
 
+def gemm_f32_splits(n: int, m: int, k: int) -> int:
+    """Parts in which gemm_f32_groups leaves an [n, k] x [m, k]^T product (1: it is better formed whole)."""
+    return int(load().shk_gemm_f32_splits(n, m, k))
+
+
+def gemm_f32_gated_takes(n: int, m: int, k: int) -> bool:
+    """Whether gemm_f32_gated takes n rows and two [m, k] matrices."""
+    return bool(load().shk_gemm_f32_gated_takes(n, m, k))
+
+
+def f32_rows_aligned(x) -> bool:
+    """Whether the rows of a float32 matrix begin at multiples of 16 bytes."""
+    return x.data_ptr() % 16 == 0 and x.stride(0) % 4 == 0
+
+
+def gemm_f32_groups(a, wt, m: int, k: int, out) -> None:
+    """out [4, n, m]: parts whose sum in order has the bits of gemm_f32_tiled_weight()."""
+    _rows(a, "gemm_f32_groups a")
+    n = a.shape[0]
+    if a.shape[1] != k or tuple(out.shape) != (4, n, m) or not out.is_contiguous():
+        raise KernelError(f"gemm_f32_groups: out must be contiguous [4, {n}, {m}] for rows of {k}")
+    if wt.numel() != -(-m // 16) * -(-k // 16) * 256 or not wt.is_contiguous():
+        raise KernelError(f"gemm_f32_groups: the tiled weights do not belong to a [{m}, {k}] matrix")
+    check(load().shk_gemm_f32_groups(_dev(a, "a", torch.float32), _dev(wt, "wt", torch.float32), _dev(out, "out", torch.float32), n,
+                                     m, k, a.stride(0), _stream()))
+
+
+def gemm_f32_gated(a, wt, m: int, k: int, out, activation, limit=None, up_shift: float = 0.0) -> None:
+    """out [n, m] = act_mul() of gemm_f32_tiled_weight()'s [n, 2 m], the same bits; up to 16 rows."""
+    _rows(a, "gemm_f32_gated a")
+    n = a.shape[0]
+    if a.shape[1] != k or tuple(out.shape) != (n, m) or not out.is_contiguous():
+        raise KernelError(f"gemm_f32_gated: out must be contiguous [{n}, {m}] for rows of {k}")
+    if wt.numel() != 2 * m // 16 * -(-k // 16) * 256 or not wt.is_contiguous():
+        raise KernelError(f"gemm_f32_gated: the tiled weights do not belong to two [{m}, {k}] matrices")
+    check(load().shk_gemm_f32_gated(_dev(a, "a", torch.float32), _dev(wt, "wt", torch.float32), _dev(out, "out", torch.float32), n, m,
+                                    k, a.stride(0), activation_code(activation), float(limit or 0.0), float(up_shift), _stream()))
+
+
 def tiled_numel(m: int, k: int) -> int:
     """bfloat16 elements of the tiled layout of an [m, k] matrix."""
     return -(-m // 16) * -(-k // 32) * 512

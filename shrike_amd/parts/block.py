@@ -62,9 +62,9 @@ class PreNormResidualBlock(Block):
     def _onto(ctx, hidden, scale, part, norm, reader):
         """What `part`'s last product may add to (StepContext.onto): the stream, where the next norm and its reader take
         what such a product leaves."""
-        if scale != 1.0 or norm is None or not part.ends_onto or not norm.leaves_scaled or not reader.takes_scaled(ctx):
+        if scale != 1.0 or norm is None or not part.ends_onto or not norm.leaves_scaled:
             return None
-        return hidden, norm
+        return hidden, norm, reader.takes_scaled(ctx)
 
 
 register_block("prenorm_residual", PreNormResidualBlock)
