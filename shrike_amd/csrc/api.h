@@ -585,6 +585,17 @@ int shk_moe_experts_grouped(const void* x, const int32_t* chosen, const float* w
                             int identity, int act, float limit, float shift, int tiled,
                             void* stream);
 
+// The same for up to 16 tokens, at most 8 choices each, gated experts and matrices in tiles, with the shared expert in the same
+// launches: shared_gate_up an interleaved gate/up pair, shared_down a matrix in tiles (shk_interleave_gate_up, shk_retile_weight;
+// null: none, shared_ff 0), added times sigmoid(add_gate[t * gate_ld]) where that is given.  act_buf [n * top][ff], shared_act
+// [n][shared_ff], pair_out float32 [(n * top + n)][width] (n * top without a shared expert).
+int shk_moe_few_takes(int n, int top);
+int shk_moe_few(const void* x, const int32_t* chosen, const float* weights, const void* w_gate, const void* w_up,
+                const void* w_down, const void* shared_gate_up, const void* shared_down, const float* add_gate, int gate_ld,
+                void* act_buf, void* shared_act, float* pair_out, void* out, int n, int width, int ff, int shared_ff,
+                int experts, int top, int identity, int act, float limit, float shift, float shared_limit, void* stream);
+
+
 // out = a_pos z^2 + z / 2 where z > 0, a_neg (exp(z) - 1 - z) + z / 2 elsewhere; elementwise.
 int shk_xielu(const void* x, void* out, int dtype, long long numel, float a_pos, float a_neg, void* stream);
 

@@ -108,6 +108,7 @@ const Launcher kLaunchers[] = {
     SHK_LAUNCHER(shk_moe_route),
     SHK_LAUNCHER(shk_moe_experts),
     SHK_LAUNCHER(shk_moe_experts_grouped),
+    SHK_LAUNCHER(shk_moe_few),
     SHK_LAUNCHER(shk_embed_pairs),
     SHK_LAUNCHER(shk_postnorm),
     SHK_LAUNCHER(shk_cast_rows),

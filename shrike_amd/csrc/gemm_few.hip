@@ -22,9 +22,7 @@
 // 17.2.  few_gated against the product without the division: 9728 x 896 5.6 / 6.2 / 6.9 -> 5.9 / 6.1 / 6.4, 37888 x 3584 40.6 /
 // 40.6 / 45.1 -> 40.9 / 40.9 / 42.1.  Steps: 0.5B at 1 / 4 / 16 sequences 755 / 814 / 917 -> 653 / 692 / 757, 7B at 1 / 8 / 16
 // 2,883 / 3,174 / 3,366 -> 2,686 / 3,000 / 3,158.
-#include <type_traits>
-
-#include "gemm_bf16.h"
+#include "gemm_few.h"
 
 namespace shk {
 
@@ -38,6 +36,18 @@ __device__ __forceinline__ int few_first() {
 struct FewRows {
   const bf16* a;
   int token_step, col_step, n, k;
+};
+
+template <int NB>
+struct FewTokens {
+  const FewRows& x;
+  __device__ __forceinline__ void operator()(const bf16* (&arow)[NB]) const {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      const int token = few_first<NB>() + b * 16 + static_cast<int>(threadIdx.x % 16);
+      arow[b] = x.a + static_cast<size_t>(min(token, x.n - 1)) * x.token_step;
+    }
+  }
 };
 
 // What divides them: the squares' sums [count][n], null for rows that are normed already.
@@ -78,93 +88,7 @@ struct FewSquares {
   }
 };
 
-// A wavefront asks for everything before it waits for anything: its k-tiles at once where they fit its registers.
-// acc += the wavefront's k-tiles (wave, wave + waves, ...) of RB blocks of 16 weight rows by NB blocks of 16 tokens.  wrow[]: the lane's
-// weight row at its piece of the first tile.  C > 0: a wavefront has at most C tiles, which are all asked for at once;
-// C = 0: batches of B tiles, two in flight.  Addresses are clamped into the matrices and what lies beyond k is
-// zeroed when it is used: no load stands under a condition.
-template <int C, int B, int RB, int NB, typename Between>
-__device__ __forceinline__ void few_multiply(f32x4 (&acc)[RB][NB], const u32x4* const (&wrow)[RB], const FewRows& x, int ktiles, int wave,
-                                             int waves, Between between) {
-  const int lane = threadIdx.x % kWave, j = lane % 16, kg = lane / 16;
-  const bf16* arow[NB];
-#pragma unroll
-  for (int b = 0; b < NB; ++b) arow[b] = x.a + static_cast<size_t>(min(few_first<NB>() + b * 16 + j, x.n - 1)) * x.token_step;
-  constexpr int kTiles = C > 0 ? C : B;
-  struct Batch {
-    u32x4 w[kTiles][RB], x[kTiles][NB];
-    uint32_t keep[kTiles];
-  };
-  auto load = [&](Batch& b, int t) {
-#pragma unroll
-    for (int u = 0; u < kTiles; ++u) {
-      const int tt = t + u * waves, col = tt * 32 + kg * 8;
-#pragma unroll
-      for (int r = 0; r < RB; ++r)
-        b.w[u][r] = __builtin_nontemporal_load(wrow[r] + static_cast<size_t>(tt < ktiles ? tt : ktiles - 1) * kWave);
-      const bool inside = col < x.k;
-      b.keep[u] = inside ? ~0u : 0u;
-#pragma unroll
-      for (int c = 0; c < NB; ++c)
-        b.x[u][c] = *reinterpret_cast<const u32x4*>(arow[c] + (inside ? static_cast<size_t>(col) * x.col_step : 0));
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  auto multiply = [&](const Batch& b) {
-#pragma unroll
-    for (int u = 0; u < kTiles; ++u)
-#pragma unroll
-      for (int c = 0; c < NB; ++c) {
-        const u32x4 v = b.x[u][c] & b.keep[u];
-#pragma unroll
-        for (int r = 0; r < RB; ++r)
-          acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, b.w[u][r]), __builtin_bit_cast(bf16x8, v),
-                                                              acc[r][c], 0, 0, 0);
-      }
-  };
-#pragma unroll
-  for (int r = 0; r < RB; ++r)
-#pragma unroll
-    for (int c = 0; c < NB; ++c) acc[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-  Batch ping;
-  load(ping, wave);
-  if constexpr (C > 0) {
-    between();
-    multiply(ping);
-  } else {
-    Batch pong;
-    const int step = B * waves, batches = (ktiles + step - 1) / step;
-    load(pong, wave + step);
-    between();
-    int b = 0;
-    for (; b + 3 < batches; b += 2) {
-      multiply(ping);
-      load(ping, wave + (b + 2) * step);
-      multiply(pong);
-      load(pong, wave + (b + 3) * step);
-    }
-    multiply(ping);
-    if (b + 2 < batches) {
-      load(ping, wave + (b + 2) * step);
-      multiply(pong);
-      multiply(ping);
-    } else {
-      multiply(pong);
-    }
-  }
-}
-
 constexpr int kFewWaves = 9;  // wavefronts of a workgroup at most
-constexpr int kFewTiles = 10, kFewPairs = 7;  // k-tiles of a wavefront that are held at once: of one block of weight rows, of two
-
-// Element (row, token) of the 16 x 16 results that `waves` wavefronts have left in LDS, added in their order.
-__device__ __forceinline__ float few_sum(const f32x4* red, int stride, int row, int token, int waves) {
-  const float* p = reinterpret_cast<const float*>(red + row / 4 * 16 + token) + row % 4;
-  float v = 0.f;
-#pragma unroll 4
-  for (int w = 0; w < waves; ++w) v += p[static_cast<size_t>(w) * stride * 4];
-  return v;
-}
 
 // ROWS = 16: a workgroup for a block of 16 weight rows.  ROWS = 8: for half of one (a tile's pieces of 8 rows are whole
 // lines of 128 bytes), where whole blocks leave compute units idle; the other half of the matrix instruction does the same again.
@@ -193,7 +117,7 @@ __global__ void __launch_bounds__(kFewWaves* kWave)
   }
   const u32x4* const wrow[1] = {wt + static_cast<size_t>(wr / 16) * ktiles * kWave + wr % 16 + lane / 16 * 16};
   f32x4 acc[1][NB];
-  few_multiply<C, 4, 1, NB>(acc, wrow, x, ktiles, wave, waves, [] {});
+  few_multiply<C, 4, 1, NB>(acc, wrow, FewTokens<NB>{x}, x.col_step, x.k, ktiles, wave, waves, [] {});
 #pragma unroll
   for (int c = 0; c < NB; ++c) red[(wave * NB + c) * kWave + lane] = acc[0][c];
   __syncthreads();
@@ -225,7 +149,7 @@ __global__ void __launch_bounds__(kFewWaves* kWave)
   const u32x4* first = wt + static_cast<size_t>(blockIdx.x) * 2 * ktiles * kWave + lane;
   const u32x4* const wrow[2] = {first, first + static_cast<size_t>(ktiles) * kWave};
   f32x4 acc[2][NB];
-  few_multiply<C, 2, 2, NB>(acc, wrow, x, ktiles, wave, waves, [&] { squares.leave(part); });
+  few_multiply<C, 2, 2, NB>(acc, wrow, FewTokens<NB>{x}, x.col_step, x.k, ktiles, wave, waves, [&] { squares.leave(part); });
 #pragma unroll
   for (int c = 0; c < NB; ++c) {
     red[(wave * 2 * NB + c) * kWave + lane] = acc[0][c];
@@ -293,7 +217,7 @@ __global__ void __launch_bounds__(kFewWaves* kWave)
     const int wr = lane % 16 < 8 ? first + lane % 16 : second + lane % 16 - 8;
     const u32x4* const wrow[1] = {wt + static_cast<size_t>(wr / 16) * ktiles * kWave + wr % 16 + lane / 16 * 16};
     f32x4 acc[1][1];
-    few_multiply<C, 4, 1, 1>(acc, wrow, x, ktiles, wave, waves, [&] { if (LOADS) squares.leave(part); });
+    few_multiply<C, 4, 1, 1>(acc, wrow, FewTokens<1>{x}, x.col_step, x.k, ktiles, wave, waves, [&] { if (LOADS) squares.leave(part); });
     red[wave * kWave + lane] = acc[0][0];
   }
   const int inside = threadIdx.x / 8, token = few_first<1>() + inside, i = threadIdx.x % 8;
@@ -334,33 +258,7 @@ static bool few_rows_of(FewRows* x, const void* a, int lda, int n, int k) {
   return n >= 0 && n <= 64 && k > 0 && k % 8 == 0 && (pieces || (lda >= k && lda % 8 == 0));
 }
 
-// Wavefronts that share k: where four to eight of them hold all their tiles at once, the number that holds the fewest
-// beyond k, else four or five.  Few, because each more is another sum to add at the end: 896 x 896 with one token 2.97 us in 4,
-// 3.10 in 7, 3.21 in 15; 3584 x 18944 at 1 / 8 / 16 tokens 22.2 / 23.2 / 27.0 in 4, 22.0 / 24.1 / 28.4 in 5, 23.1 / 24.5 / 27.8
-// in 16; 1536 x 8960, whose 280 tiles five share without loads beyond k, 9.7 / 9.8 / 10.6 in 4 and 9.0 / 9.2 / 11.0 in 5.
-// (Whatever the tokens: a row's bits do not depend on those beside it.)
-static int few_waves(int ktiles, int most) {
-  int best = 0, least = 0;
-  for (int waves = 4; waves <= 8; ++waves) {
-    const int tiles = (ktiles + waves - 1) / waves;
-    if (tiles <= most && (!best || tiles * waves < least)) best = waves, least = tiles * waves;
-  }
-  const auto whole = [&](int waves) { return (ktiles + 4 * waves - 1) / (4 * waves) * 4 * waves; };
-  return best ? best : whole(5) <= whole(4) ? 5 : 4;
-}
-
-// fn with the number of k-tiles of a wavefront as a constant, 0 for more than MOST.
-template <int MOST, int C = 1, typename Fn>
-static void with_tiles(int tiles, Fn fn) {
-  if constexpr (C > MOST) {
-    fn(std::integral_constant<int, 0>{});
-  } else {
-    if (tiles == C) fn(std::integral_constant<int, C>{});
-    else with_tiles<MOST, C + 1>(tiles, fn);
-  }
-}
-
-// and with the loads of a thread that adds up squares
+// fn with the loads of a thread that adds up squares as a constant
 template <typename Fn>
 static void with_loads(int count, int threads, Fn fn) {
   const int loads = (count + threads / 16 - 1) / (threads / 16);

@@ -33,8 +33,8 @@
 
 namespace shk {
 
-constexpr int kMaxExpertsPerLane = 8;  // experts <= 512
-
+// kMaxExpertsPerLane: 1 for up to 64 outputs, 8 for up to 512.
+template <int kMaxExpertsPerLane>
 __global__ void __launch_bounds__(256)
     moe_route_kernel(const float* __restrict__ logits, int ld, const float* __restrict__ correction, int experts,
                      int top, int groups, int keep, float scale, int32_t* __restrict__ chosen,
@@ -860,7 +860,7 @@ using namespace shk;
 
 extern "C" int shk_moe_route(const float* logits, int ld, const float* correction, int experts, int top,
                              int groups, int keep, float scale, int32_t* chosen, float* weights, int n, void* stream) {
-  SHK_REQUIRE(n >= 0 && experts > 0 && experts <= kMaxExpertsPerLane * kWave && top >= 1 && top <= experts &&
+  SHK_REQUIRE(n >= 0 && experts > 0 && experts <= 8 * kWave && top >= 1 && top <= experts &&
                   top <= kWave && ld >= experts,
               "moe_route: bad sizes n=%d experts=%d top=%d", n, experts, top);
   SHK_REQUIRE(groups >= 1 && groups <= kWave && experts % groups == 0 && keep >= 1 && keep <= groups &&
@@ -868,8 +868,9 @@ extern "C" int shk_moe_route(const float* logits, int ld, const float* correctio
               "moe_route: %d of %d experts cannot be chosen from %d of %d groups", top, experts, keep, groups);
   if (n == 0) return 0;
   SHK_REQUIRE(logits && chosen && weights, "moe_route: null pointer");
-  moe_route_kernel<<<(n + 3) / 4, 256, 0, static_cast<hipStream_t>(stream)>>>(logits, ld, correction, experts, top,
-                                                                              groups, keep, scale, chosen, weights, n);
+  const auto kernel = experts <= kWave ? moe_route_kernel<1> : moe_route_kernel<8>;
+  kernel<<<(n + 3) / 4, 256, 0, static_cast<hipStream_t>(stream)>>>(logits, ld, correction, experts, top, groups, keep, scale, chosen,
+                                                                    weights, n);
   SHK_LAUNCH_CHECK("moe_route");
   return 0;
 }

@@ -1503,6 +1503,47 @@ def moe_experts(x, chosen, weights, w_gate, w_up, w_down, act_buf, out, activati
                                  top, *form, _stream()))
 
 
+def moe_few_takes(n: int, top: int) -> bool:
+    """Whether moe_few takes a step of n tokens with `top` choices each."""
+    return bool(load().shk_moe_few_takes(n, top))
+
+
+def moe_few(x, chosen, weights, w_gate, w_up, w_down, act_buf, pair_out, out, activation: str = "silu", shared=None, shared_act=None,
+            add_gate=None, identity: int = 0, limit: float | None = None, up_shift: float = 0.0,
+            shared_limit: float | None = None) -> None:
+    """moe_experts() of up to 16 tokens for gated experts in tiles (tile_experts), the shared expert in the same launches: shared =
+    (interleave_gate_up() of its first matrices, retile_weight() of the last, its features), its output not rounded before it is added.
+    act_buf [n * top, ff], shared_act [n, features]; pair_out float32 [n * top, width], with a shared expert n rows more."""
+    n, width = x.shape
+    experts, ff, _ = w_gate.shape
+    top = chosen.shape[1]
+    gate_up, down, features = shared if shared is not None else (None, None, 0)
+    tensors = (x, w_gate, w_up, w_down, act_buf, out, *(() if shared is None else (gate_up, down, shared_act)))
+    if any(t.dtype != torch.bfloat16 or not t.is_contiguous() for t in tensors):
+        raise KernelError("moe_few: tensors must be contiguous and bfloat16")
+    if tuple(w_gate.shape) != (experts, ff, width) or tuple(w_up.shape) != (experts, ff, width) or tuple(w_down.shape) != (experts, width, ff) \
+            or tuple(out.shape) != (n, width) or act_buf.numel() < n * top * ff or tuple(weights.shape) != (n, top) \
+            or tuple(chosen.shape) != (n, top) or not chosen.is_contiguous() or not weights.is_contiguous():
+        raise KernelError("moe_few: mismatched shapes")
+    if shared is not None and (gate_up.numel() != 2 * tiled_numel(features, width) or down.numel() != tiled_numel(width, features)
+                               or shared_act.numel() < n * features):
+        raise KernelError("moe_few: the shared expert's matrices do not fit")
+    if not pair_out.is_contiguous() or pair_out.numel() < (n * top + (n if shared is not None else 0)) * width:
+        raise KernelError("moe_few: pair_out is too small")
+    gate_ptr, gate_ld = None, 0
+    if add_gate is not None:
+        if shared is None or add_gate.dtype != torch.float32 or add_gate.dim() != 1 or add_gate.shape[0] != n:
+            raise KernelError("moe_few: add_gate is a float32 column of n numbers and needs a shared expert")
+        gate_ptr, gate_ld = _dev(add_gate, "add_gate"), max(1, add_gate.stride(0))
+    check(load().shk_moe_few(
+        _dev(x, "x"), _dev(chosen, "chosen", torch.int32), _dev(weights, "weights", torch.float32), _dev(w_gate, "w_gate"),
+        _dev(w_up, "w_up"), _dev(w_down, "w_down"), None if shared is None else _dev(gate_up, "gate_up"),
+        None if shared is None else _dev(down, "down"), gate_ptr, gate_ld, _dev(act_buf, "act_buf"),
+        None if shared is None else _dev(shared_act, "shared_act"), _dev(pair_out, "pair_out", torch.float32), _dev(out, "out"), n, width, ff,
+        int(features), experts, top, int(identity), activation_code(activation), float(limit or 0.0), float(up_shift),
+        float(shared_limit or 0.0), _stream()))
+
+
 def xielu(x, out, a_pos: float, a_neg: float) -> None:
     """out = a_pos x^2 + x / 2 where x > 0, a_neg (exp(x) - 1 - x) + x / 2 elsewhere."""
     if x.shape != out.shape or x.dtype != out.dtype or not x.is_contiguous() or not out.is_contiguous():

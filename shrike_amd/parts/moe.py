@@ -117,6 +117,8 @@ class MixtureOfExperts(FeedForward):
         elif s.shared_size is not None:
             self.shared = (runtime.weight(tensors[f"{self.name}.shared.up"]),
                            runtime.weight(tensors[f"{self.name}.shared.down"]))
+        # whether steps of few tokens take the shared expert beside the others (ops.moe_few)
+        self.few = self.tiled and self.gated and (s.shared_size is None or s.shared_size % 32 == 0)
         self.linear = runtime.linear
         self.gated_linear = runtime.gated_linear
 
@@ -129,6 +131,18 @@ class MixtureOfExperts(FeedForward):
         weights = ctx.buffer("moe_weights", (n, s.top), torch.float32)
         ops.moe_route(logits[:, : self.choices], self.correction, s.top, chosen, weights, groups=s.groups,
                       scale=s.router_scale)
+        if self.few and ops.moe_few_takes(n, s.top):
+            act = ctx.buffer("moe_act", (n * s.top, s.expert_size), ctx.dtype)
+            pair_out = ctx.buffer("moe_pair_out", (n * s.top + (n if self.shared is not None else 0), self.width), torch.float32)
+            out = ctx.buffer("moe_out", (n, self.width), ctx.dtype)
+            shared = shared_act = None
+            if self.shared is not None:
+                shared = (self.shared[0].tiled, self.shared[1].tiled, s.shared_size)
+                shared_act = ctx.buffer("moe_shared_act", (n, s.shared_size), ctx.dtype)
+            ops.moe_few(x, chosen, weights, self.w_gate, self.w_up, self.w_down, act, pair_out, out, self.activation, shared=shared,
+                        shared_act=shared_act, add_gate=logits[:, self.choices] if self.shared_gate else None, identity=s.identity,
+                        limit=s.limit, up_shift=s.up_shift, shared_limit=s.shared_limit)
+            return out
         shared_out = None
         if self.shared is not None:
             act = ctx.buffer("moe_shared_act", (n, s.shared_size), ctx.dtype)
