@@ -312,7 +312,8 @@ __global__ void __launch_bounds__(kPromptWaves* kWave) __attribute__((amdgpu_wav
     if (col_ok && d0 < key_dim) qf[ks].u = *reinterpret_cast<const uint4*>(qrow + d0);
   }
   // what lies behind a row's elements stays zero for the whole kernel
-  for (int i = tid; i < 2 * kRows / 8; i += kThreads) reinterpret_cast<uint4*>(rows0)[i] = make_uint4(0, 0, 0, 0);
+  if (key_dim < KS * 32)
+    for (int i = tid; i < 2 * kRows / 8; i += kThreads) reinterpret_cast<uint4*>(rows0)[i] = make_uint4(0, 0, 0, 0);
   if (tid < 2) unsafe[tid] = 0;
   __syncthreads();
 
@@ -501,28 +502,38 @@ __global__ void __launch_bounds__(kPromptWaves* kWave) __attribute__((amdgpu_wav
   }
 }
 
-// out[row][:] = sum_z 2^(m_z - M) O_z / sum_z 2^(m_z - M) l_z, shares in order; one wavefront a row.
-__global__ void __launch_bounds__(kWave)
+// out[row][:] = sum_z 2^(m_z - M) O_z / sum_z 2^(m_z - M) l_z, shares in order; a thread an element, eight shares asked for at once
+// (one wavefront a row and one share after the other: attention of eight tokens over 850 rows in eight shares 38.0 us with it, 33.7 so;
+// in sixteen 34.3 and 26.5).
+__global__ void __launch_bounds__(256)
     latent_merge_kernel(const float* __restrict__ partial, bf16* __restrict__ out, int nsplit, int v_dim) {
-  __shared__ float weight[64];
   const size_t all_rows = gridDim.x, row = blockIdx.x;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x % kWave, d = blockIdx.y * blockDim.x + threadIdx.x;
   const float* ml = partial + all_rows * nsplit * v_dim + row * nsplit * 2;
+  const float* src = partial + row * nsplit * v_dim + (d < v_dim ? d : 0);
   float mz = -INFINITY, lz = 0.f;
   if (lane < nsplit) mz = ml[lane * 2], lz = ml[lane * 2 + 1];
   const float mx = wave_max(mz);
   const float w = mz == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mz - mx);
-  weight[lane] = w;
-  __syncthreads();
-  float den = 0.f;
-  for (int zz = 0; zz < nsplit; ++zz) den += __shfl(w * lz, zz, kWave);
-  const float inv = 1.f / den;
-  const float* src = partial + row * nsplit * v_dim;
-  for (int d = lane; d < v_dim; d += kWave) {
-    float acc = 0.f;
-    for (int zz = 0; zz < nsplit; ++zz) acc += weight[zz] * src[static_cast<size_t>(zz) * v_dim + d];
-    out[row * v_dim + d] = from_float<bf16>(acc * inv);
+  float den = 0.f, acc = 0.f;
+  for (int z0 = 0; z0 < nsplit; z0 += 8) {
+    float v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = src[static_cast<size_t>(z0 + u < nsplit ? z0 + u : nsplit - 1) * v_dim];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (z0 + u < nsplit) {
+        den += __shfl(w * lz, z0 + u, kWave);
+        acc += __shfl(w, z0 + u, kWave) * v[u];
+      }
   }
+  if (d < v_dim) out[row * v_dim + d] = from_float<bf16>(acc * (1.f / den));
+}
+
+// Its launch: whole wavefronts for the elements of a row.
+static void launch_latent_merge(hipStream_t s, const float* partial, bf16* out, size_t rows, int nsplit, int v_dim) {
+  const int threads = v_dim <= 64 ? 64 : v_dim <= 128 ? 128 : 256;
+  latent_merge_kernel<<<dim3(static_cast<unsigned>(rows), (v_dim + threads - 1) / threads), threads, 0, s>>>(partial, out, nsplit, v_dim);
 }
 
 template <int KS, int DB>
@@ -573,16 +584,24 @@ extern "C" int shk_latent_prompt_bf16(const void* q, void* out, int n, int heads
   };
   using std::integral_constant;
   const int ks = (key_dim + 31) / 32, db = (v_dim + 15) / 16;
+  auto columns = [&](auto ks_of, auto dbw, auto most_columns) {
+    // (few tokens a workgroup: no multiplications for columns that none of them has.  One token of 28 heads a workgroup, rows of 512, eight
+    // at 850 in 16 shares: 27.2 us with seven columns and the merge as it was, 17.4; latent_attention_mfma_kernel 34.3 and 26.5)
+    if (tpw * heads <= 32)
+      go(ks_of, dbw, integral_constant<int, 2>{});
+    else
+      go(ks_of, dbw, most_columns);
+  };
   if (ks <= 8 && db <= 8)
-    go(integral_constant<int, 8>{}, integral_constant<int, 1>{}, integral_constant<int, 8>{});
+    columns(integral_constant<int, 8>{}, integral_constant<int, 1>{}, integral_constant<int, 8>{});
   else if (ks <= 8)
-    go(integral_constant<int, 8>{}, integral_constant<int, 2>{}, integral_constant<int, 8>{});
+    columns(integral_constant<int, 8>{}, integral_constant<int, 2>{}, integral_constant<int, 8>{});
   else if (db <= 16)
-    go(integral_constant<int, 16>{}, integral_constant<int, 2>{}, integral_constant<int, 8>{});
+    columns(integral_constant<int, 16>{}, integral_constant<int, 2>{}, integral_constant<int, 8>{});
   else
-    go(integral_constant<int, 16>{}, integral_constant<int, 4>{}, integral_constant<int, 7>{});
+    columns(integral_constant<int, 16>{}, integral_constant<int, 4>{}, integral_constant<int, 7>{});
   if (nsplit > 1)
-    latent_merge_kernel<<<static_cast<unsigned>(n) * heads, kWave, 0, s>>>(partial, static_cast<bf16*>(out), nsplit, v_dim);
+    launch_latent_merge(s, partial, static_cast<bf16*>(out), static_cast<size_t>(n) * heads, nsplit, v_dim);
   SHK_LAUNCH_CHECK("latent_prompt_bf16");
   return 0;
 }
@@ -628,7 +647,7 @@ extern "C" int shk_latent_attention_bf16(const void* q, void* out, int n, int he
   else { if (db <= 32) SHK_LATENT(20, 32); else SHK_LATENT(20, 40); }
 #undef SHK_LATENT
   if (nsplit > 1)
-    latent_merge_kernel<<<static_cast<unsigned>(n) * heads, kWave, 0, s>>>(partial, static_cast<bf16*>(out), nsplit, v_dim);
+    launch_latent_merge(s, partial, static_cast<bf16*>(out), static_cast<size_t>(n) * heads, nsplit, v_dim);
   SHK_LAUNCH_CHECK("latent_attention_bf16");
   return 0;
 }

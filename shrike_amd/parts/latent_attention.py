@@ -74,6 +74,12 @@ class LatentAttention(Mixer):
         if s.window is not None and s.window < 1:
             raise ValueError(f"{self.name}: window must be positive, got {s.window}")
 
+    @property
+    def single_in_prompt(self) -> bool:
+        """Whether single tokens take the prompt portions' kernel too, one a workgroup: the same bits, 0.5 to 0.8 of the time (14 heads
+        over rows of 176, 28 over rows of 512; 60 to 1,500 rows, 1 to 16 tokens)."""
+        return bool(self.prompt_tokens) and self.spec.num_heads >= 4
+
     def prepare(self, shape) -> None:
         """Among how many workgroups each token's rows are shared on the matrix-instruction
         path: few tokens with thousands of rows each (single tokens of long sequences) would
@@ -99,6 +105,17 @@ class LatentAttention(Mixer):
                 tokens *= 2
             return max(1, min(2 * compute_units() // tokens, most_shares(rows)))
 
+        def single_shares(tokens_of, rows):
+            """The same for a step of single tokens in the prompt portions' kernel: shares of 64 rows, as long as there is a compute unit for
+            each (28 heads over rows of 512, eight tokens at 850: 20.3 us in 8 shares, 17.4 in 16; 16 at 1,500 28.3 in 8, 23.9
+            in 16, 35.1 in 32)."""
+            tokens, keys = 1, 64
+            while tokens < tokens_of:
+                tokens *= 2
+            while keys < min([rows, *bounds]):
+                keys *= 2
+            return max(shares(tokens_of, rows), max(1, min(compute_units() // tokens, keys // 64, 64)))
+
         # prompt portions in a kernel of their own where it takes the shape; else every token alike
         # (neighbouring tokens of a step with portions may share a workgroup and what it stages)
         nsplit, group, first, prompt_split, tokens = 1, 1, shape.num_tokens, 1, 0
@@ -118,6 +135,8 @@ class LatentAttention(Mixer):
                 prompt_split = shares(-(-count // tokens), longest)
                 if first:
                     nsplit = shares(first, int(shape.ctx_lens[:first].max()))
+            elif self.single_in_prompt and shape.num_decode == shape.num_seqs:
+                nsplit = single_shares(shape.num_tokens, int(shape.ctx_lens.max()))
             else:
                 nsplit = shares(shape.num_tokens, int(shape.ctx_lens.max()))
                 group = 1 if shape.num_decode == shape.num_seqs else 4
@@ -188,7 +207,9 @@ class LatentAttention(Mixer):
                        cache.pools["latent"], cache.page_size, s.window, s.scale, chunk=s.chunk, partial=partial, nsplit=shares,
                        **more)
 
-            if first:
+            if first and self.single_in_prompt and first == ctx.num_decode:
+                attend(ops.latent_prompt, 0, first, nsplit, tokens=1)
+            elif first:
                 attend(ops.latent_attention_mfma, 0, first, nsplit, tokens_per_group=group)
             if first < n:
                 attend(ops.latent_prompt, first, n, prompt_split, tokens=tokens)
