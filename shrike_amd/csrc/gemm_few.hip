@@ -1,5 +1,5 @@
-// Products of up to 16 tokens, with small matrices of up to 64, that finish what the kernels between two products would do, so that a decode step has
-// fewer dependent kernels: five a layer instead of eight.  A step of a small model is a chain of kernels of 2.5 to 6 us each,
+// Products of up to 16 tokens, with small matrices of more (64, projections to heads 512), that finish what the kernels between
+// two products would do, so that a decode step has fewer dependent kernels: five a layer instead of eight.  A step of a small model is a chain of kernels of 2.5 to 6 us each,
 // most of which start, wait for memory once and end (weights already in the caches make the 7B output projection 6.3 us
 // instead of 6.8).
 //
@@ -252,10 +252,12 @@ __global__ void __launch_bounds__(kFewWaves* kWave)
 
 using namespace shk;
 
-static bool few_rows_of(FewRows* x, const void* a, int lda, int n, int k) {
+constexpr int kFewTokens = 64, kFewHeadsTokens = 512;
+
+static bool few_rows_of(FewRows* x, const void* a, int lda, int n, int k, int most) {
   const bool pieces = lda == 0;  // [k / 8][n][8]
   *x = FewRows{static_cast<const bf16*>(a), pieces ? 8 : lda, pieces ? n : 1, n, k};
-  return n >= 0 && n <= 64 && k > 0 && k % 8 == 0 && (pieces || (lda >= k && lda % 8 == 0));
+  return n >= 0 && n <= most && k > 0 && k % 8 == 0 && (pieces || (lda >= k && lda % 8 == 0));
 }
 
 // fn with the loads of a thread that adds up squares as a constant
@@ -280,8 +282,14 @@ static int few_stream_rows(int m) { return m <= 2048 ? 8 : 16; }
 // that it spares: 9728 x 896 7.2 / 7.4 / 10.0 -> 7.5 / 7.9 / 10.4, 17920 x 1536 12.9 / 13.5 / 16.8 -> 13.7 / 15.0 / 23.2.
 constexpr long long kFewStreamMost = 5 * 1000 * 1000, kFewHeadsMost = 6 * 1000 * 1000, kFewGatedMost = 10 * 1000 * 1000;
 
+// Heads of more tokens, which spare the position kernel of so many rows: as long as what all blocks of 16 tokens read together
+// stays below this.  Cold weights, product and position kernel against this, at 65 / 128 / 256 / 384 / 512 tokens: 512 x 256
+// 9.1 / 9.2 / 9.4 / 9.4 / 9.7 -> 3.2 / 3.6 / 4.0 / 4.4 / 4.7 us, 1152 x 896 9.9 / 10.0 / 12.2 / 12.5 / 13.4 -> 5.3 / 6.6 / 8.8 /
+// 11.8 / 14.4 (the line lies at 400), 2048 x 1536 12.3 / 13.3 / 18.5 -> 9.2 / 12.7 / 20.6 (at 128), 2560 x 2048 15.7 / 16.8 -> 14.0 / 20.7.
+constexpr long long kFewHeadsRead = 26 * 1000 * 1000;
+
 static bool few_takes(int n, int m, int k, long long most) {
-  return n <= 16 || (n <= 64 && static_cast<long long>(m) * k <= most);
+  return n <= 16 || (n <= kFewTokens && static_cast<long long>(m) * k <= most);
 }
 
 // Not where a second round of workgroups would be nearly empty: 320 of them (5120 x 5120 at 8 tokens 14.3 us for product in shares
@@ -293,12 +301,16 @@ extern "C" int shk_few_stream_sums(int n, int m, int k) {
 // `m` rows of the gate and as many of the other matrix; the k columns may come with as many sums as few_stream leaves.
 extern "C" int shk_few_gated_takes(int n, int m, int k) { return m > 0 && k > 0 && k % 8 == 0 && few_takes(n, 2 * m, k, kFewGatedMost); }
 
-extern "C" int shk_few_heads_takes(int n, int m, int k) { return m > 0 && k > 0 && k % 8 == 0 && few_takes(n, m, k, kFewHeadsMost); }
+extern "C" int shk_few_heads_takes(int n, int m, int k) {
+  if (m <= 0 || k <= 0 || k % 8) return 0;
+  if (few_takes(n, m, k, kFewHeadsMost)) return 1;
+  return n <= kFewHeadsTokens && (counted_tokens(n) + 15LL) / 16 * m * k <= kFewHeadsRead;
+}
 
 extern "C" int shk_few_stream(const void* a, int lda, int n, int k, const void* wt, int m, const float* bias, float* resid,
                               const float* weight, void* rows, float* sums, void* stream) {
   FewRows x;
-  SHK_REQUIRE(few_rows_of(&x, a, lda, n, k) && m > 0 && m % 16 == 0, "few_stream: bad sizes n=%d m=%d k=%d lda=%d", n, m, k, lda);
+  SHK_REQUIRE(few_rows_of(&x, a, lda, n, k, kFewTokens) && m > 0 && m % 16 == 0, "few_stream: bad sizes n=%d m=%d k=%d lda=%d", n, m, k, lda);
   if (n == 0) return 0;
   SHK_REQUIRE(a && wt && resid && weight && rows && sums, "few_stream: null pointer");
   SHK_REQUIRE(reinterpret_cast<uintptr_t>(a) % 16 == 0, "few_stream: rows are not 16-byte aligned");
@@ -319,7 +331,7 @@ extern "C" int shk_few_stream(const void* a, int lda, int n, int k, const void* 
 extern "C" int shk_few_gated(const void* a, int lda, int n, int k, const void* wt, const float* sums, int count, float eps,
                              const float* args, void* out, int m, int ldo, int gated, void* stream) {
   FewRows x;
-  SHK_REQUIRE(few_rows_of(&x, a, lda, n, k) && m > 0 && (ldo ? ldo >= m : m % 8 == 0),
+  SHK_REQUIRE(few_rows_of(&x, a, lda, n, k, kFewTokens) && m > 0 && (ldo ? ldo >= m : m % 8 == 0),
               "few_gated: bad sizes n=%d m=%d k=%d lda=%d ldo=%d", n, m, k, lda, ldo);
   SHK_REQUIRE(gated > 0 && gated <= kActQuickGelu, "few_gated: unknown gate activation %d", gated);
   SHK_REQUIRE(sums && count > 0 && eps > 0.f, "few_gated: rows come with the sums of their squares");
@@ -350,7 +362,7 @@ extern "C" int shk_few_heads(const void* a, int lda, int n, int k, const void* w
                              void* k_pool, void* v_pool, int page_size, int num_pages, int write_kv, float magnitude,
                              void* stream) {
   FewRows x;
-  SHK_REQUIRE(few_rows_of(&x, a, lda, n, k), "few_heads: bad sizes n=%d k=%d lda=%d", n, k, lda);
+  SHK_REQUIRE(few_rows_of(&x, a, lda, n, k, kFewHeadsTokens), "few_heads: bad sizes n=%d k=%d lda=%d", n, k, lda);
   SHK_REQUIRE(heads > 0 && kv_heads > 0 && head_dim > 0 && head_dim % 16 == 0, "few_heads: bad heads %d %d %d", heads, kv_heads, head_dim);
   if (n == 0) return 0;
   SHK_REQUIRE(a && wt && out && inv_freq && positions, "few_heads: null pointer");

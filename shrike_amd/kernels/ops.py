@@ -547,7 +547,7 @@ class ScaledRows:
         return (self.rows.shape[1], 8 * self.rows.shape[0])
 
 
-FEW_TOKENS = 64  # the most that few_stream, few_gated and few_heads take
+FEW_TOKENS, FEW_HEADS_TOKENS = 64, 512  # the most that few_stream and few_gated take, and few_heads
 
 
 def few_stream_sums(n: int, m: int, k: int) -> int:
@@ -566,7 +566,7 @@ def few_heads_takes(n: int, m: int, k: int) -> bool:
     return bool(load().shk_few_heads_takes(n, m, k))
 
 
-def _few_rows(who, x, k, wt, numel):
+def _few_rows(who, x, k, wt, numel, most=FEW_TOKENS):
     """(address, row stride, tokens) of rows [n, k], or [k / 8, n, 8] with the stride 0."""
     pieces = x.dim() == 3
     if pieces:
@@ -575,8 +575,8 @@ def _few_rows(who, x, k, wt, numel):
         _rows(x, f"{who} rows")
         fits = x.shape[1] == k
     n = x.shape[1] if pieces else x.shape[0]
-    if not fits or x.dtype != torch.bfloat16 or n > FEW_TOKENS:
-        raise KernelError(f"{who}: rows must be bfloat16 [up to {FEW_TOKENS}, {k}] or pieces of them, got {tuple(x.shape)}")
+    if not fits or x.dtype != torch.bfloat16 or n > most:
+        raise KernelError(f"{who}: rows must be bfloat16 [up to {most}, {k}] or pieces of them, got {tuple(x.shape)}")
     if wt.numel() != numel or wt.dtype != torch.bfloat16:
         raise KernelError(f"{who}: the tiled weights do not belong to the product")
     return _dev(x, "rows"), 0 if pieces else x.stride(0), n
@@ -625,11 +625,11 @@ def few_gated(x: ScaledRows, wt, m: int, k: int, out, activation, gate_args=None
 
 def few_heads(x, wt, k: int, out, heads, kv_heads, head_dim, inv_freq, positions, token_seq, tables, k_pool, v_pool,
               page_size, write_kv=True, bias=None, magnitude: float = 1.0) -> None:
-    """The projections of up to 64 rows (normed, or ScaledRows) to queries, keys and values, rotated whole as in
+    """The projections of up to 512 rows (normed, or ScaledRows) to queries, keys and values, rotated whole as in
     rope_kv_store: queries into out's query columns, keys and values into their pages."""
     rows, sums, count, eps = _few_sums("few_heads", x)
     width = (heads + 2 * kv_heads) * head_dim
-    p, lda, n = _few_rows("few_heads", rows, k, wt, tiled_numel(width, k))
+    p, lda, n = _few_rows("few_heads", rows, k, wt, tiled_numel(width, k), FEW_HEADS_TOKENS)
     if tuple(out.shape) != (n, width) or not out.is_contiguous() or out.dtype != torch.bfloat16:
         raise KernelError(f"few_heads: out must be contiguous bfloat16 [{n}, {width}]")
     if bias is not None and bias.numel() != width:

@@ -1,5 +1,5 @@
-"""Products of up to 64 tokens that add to the stream, divide by a row's root mean square, or rotate and store what they
-form, at the edges of tiles, batches and layouts, against float64."""
+"""Products of few tokens that add to the stream, divide by a row's root mean square, or rotate and store what they form,
+at the edges of tiles, batches and layouts, against float64."""
 
 import pytest
 import torch
@@ -94,7 +94,7 @@ def test_a_gated_product_of_rows_that_are_still_to_be_divided(m, k, groups, n):
         assert torch.equal(rows(inside), out[:, :m])
 
 
-@pytest.mark.parametrize("n", [1, 7, 16, 17, 50])
+@pytest.mark.parametrize("n", [1, 7, 16, 17, 50, 65, 400, 512])
 @pytest.mark.parametrize("heads, kv_heads, head_dim, k", [(14, 2, 64, 896), (3, 1, 16, 8), (4, 4, 128, 1000), (2, 1, 48, 3584)])
 @pytest.mark.parametrize("scaled, write_kv", [(True, True), (False, True), (True, False)])
 def test_projections_that_are_rotated_and_stored(heads, kv_heads, head_dim, k, n, scaled, write_kv):
