@@ -105,7 +105,8 @@ int shk_retile_f32(const void* w, int m, int k, void* wt, void* stream);
 int shk_gemm_f32_tiled_weight(const void* a, const void* wt, const float* bias, void* out, int n, int m, int k, int lda,
                               int ldo, int accumulate, void* stream);
 
-// Up to 16 rows (16-byte aligned, k a multiple of 16), the same bits.  shk_gemm_f32_groups: out [4][n][m] receives the sum's four
+// The same bits, rows 16-byte aligned, k a multiple of 16; of more than 16 rows k a multiple of 32, at least 288 (groups 768), the
+// matrix less than 2^30 elements, lda up to 2^20.  shk_gemm_f32_groups: out [4][n][m] receives the sum's four
 // groups, whose sum in order is the product (shk_add_rmsnorm adds them); shk_gemm_f32_splits: 4 where that is worth it, else 1.
 // shk_gemm_f32_gated: out[n, m] = act(g) * (u + up_shift) of the product [g | u] with 2 m features, as shk_act_mul forms it
 // (m a multiple of 16).

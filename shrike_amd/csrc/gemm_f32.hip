@@ -349,35 +349,44 @@ __global__ void __launch_bounds__(kWave* KW)
 // rows meet no bank conflicts.
 // What bounds it: the matrix units where workgroups fill the chip several times (3584 x 3584 at 1,501 rows 119 TFLOP/s of
 // the 150 that the instruction reaches alone, 9728 x 896 at 509 97).  64 x 64, 128 x 64 and 128 x 128 results a workgroup
-// were 4 % slower to twice as slow: fewer wavefronts to cover each other's barriers.
-template <int RT, int CT>
+// were 4 % slower to twice as slow: fewer wavefronts to cover each other's barriers.  In groups 896 x 4864 at 509 rows, with the norm
+// that adds them, 48.6 us, 56.4 whole in gemm_f32_kernel; the gate's two kernels become one, 4864 x 896 at 509 88.1 and 83.2.
+// GROUPS: a workgroup forms group blockIdx.y of the sum alone and leaves it in out[blockIdx.y].  GATED: its two blocks of features
+// are the gate's and the other factor's, `m` features each.
+template <int RT, int CT, bool GATED, bool GROUPS>
 __global__ void __launch_bounds__(4 * kWave)
     gemm_f32_lds_kernel(const float* __restrict__ a, const float* __restrict__ w, const float* __restrict__ bias,
-                        float* __restrict__ out, int n, int m, int k, int lda, int ldo, int accumulate, int vec_out) {
+                        float* __restrict__ out, int n, int m, int k, int lda, int ldo, int accumulate, int vec_out, F32Gate gate) {
+  static_assert(!GATED || (RT == 1 && !GROUPS), "a block of the gate, a block of the other factor");
   constexpr int kRing = 3, kW = 4 * RT, kA = 4 * CT;  // stages; KiB of a stage's weights and rows
   __shared__ mf4 mem[kRing * (kW + kA)][kWave];
   const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int mw = wave / 2, nw = wave % 2, i = lane % 16, kg = lane / 16;
   // workgroup -> tile as in gemm_f32_kernel
-  const int rows = (n + 32 * CT - 1) / (32 * CT), cols = (m + 32 * RT - 1) / (32 * RT);
+  constexpr int kBlocks = GATED ? 1 : 2 * RT;  // of 16 results a row
+  const int rows = (n + 32 * CT - 1) / (32 * CT), cols = (m + 16 * kBlocks - 1) / (16 * kBlocks);
   const int per_die = (rows * cols + kDies - 1) / kDies;
   const int tile = blockIdx.x % kDies * per_die + blockIdx.x / kDies;
   if (blockIdx.x / kDies >= per_die || tile >= rows * cols) return;
-  const int f0 = tile / rows * 2 * RT, t0 = tile % rows * 32 * CT;  // first block of 16 features, first row
-  const int ktiles = k / 16, stages = k / 32, blocks = (m + 15) / 16;
+  const int f0 = tile / rows * kBlocks, t0 = tile % rows * 32 * CT;  // first block of 16 features, first row
+  const int seg_steps = (k + 16 * kF32Segments - 1) / (16 * kF32Segments);
+  const int ktiles = k / 16, blocks = (m + 15) / 16;
+  // (a group is a whole number of stages; no group of what comes in groups is empty)
+  const int first = GROUPS ? blockIdx.y * (kF32Group / 2) * seg_steps : 0;
+  const int stages = GROUPS ? min(k / 32 - first, kF32Group / 2 * seg_steps) : k / 32;
 
   // what a wavefront loads: units wave, wave + 4, ..; rows beyond the last are read as the last and not stored
   unsigned woff[RT], aoff[CT];
 #pragma unroll
   for (int u = 0; u < RT; ++u) {
-    const int unit = wave + 4 * u, block = min(f0 + unit / 2, blocks - 1) - f0;
+    const int unit = wave + 4 * u, block = GATED ? unit / 2 * blocks : min(f0 + unit / 2, blocks - 1) - f0;
     woff[u] = (static_cast<unsigned>(block) * ktiles + unit % 2) * 1024u + lane * 16u;
   }
 #pragma unroll
   for (int u = 0; u < CT; ++u)
     aoff[u] = static_cast<unsigned>(min(t0 + (wave + 4 * u) * 8 + lane / 8, n - 1) - t0) * lda * 4u + ((lane % 8) ^ (wave % 2 * 4 + lane / 16)) * 16u;
-  const char* wsrc = reinterpret_cast<const char*>(w) + static_cast<size_t>(f0) * ktiles * 1024;
-  const char* asrc = reinterpret_cast<const char*>(a) + static_cast<size_t>(t0) * lda * 4;
+  const char* wsrc = reinterpret_cast<const char*>(w) + (static_cast<size_t>(f0) * ktiles + 2 * first) * 1024;
+  const char* asrc = reinterpret_cast<const char*>(a) + static_cast<size_t>(t0) * lda * 4 + static_cast<size_t>(first) * 128;
   const unsigned base =
       static_cast<unsigned>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)&mem[0][0])) + wave * 1024;
   auto load = [&](int slot, int stage) {
@@ -393,7 +402,6 @@ __global__ void __launch_bounds__(4 * kWave)
   for (int r = 0; r < RT; ++r)
 #pragma unroll
     for (int c = 0; c < CT; ++c) acc[r][c] = group[r][c] = total[r][c] = mf4{0.f, 0.f, 0.f, 0.f};
-  const int seg_steps = (k + 16 * kF32Segments - 1) / (16 * kF32Segments);
   int in_seg = 0, in_group = 0;
   load(0, 0);
   load(1, 1);
@@ -445,6 +453,21 @@ __global__ void __launch_bounds__(4 * kWave)
   }
   SHK_WAIT_LOADS(0);  // no load may arrive in LDS that the workgroup has given back
 
+  if constexpr (GATED) {
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < CT; ++c) mem[(mw * 2 + nw) * CT + c][lane] = total[0][c] + (group[0][c] + acc[0][c]);
+    __syncthreads();
+    const int row = threadIdx.x / 4, quad = threadIdx.x % 4;  // four neighbouring threads a row's 64 bytes
+    if (row >= 32 * CT || t0 + row >= n) return;
+    const mf4 g = mem[row / 16][quad * 16 + row % 16], up = mem[2 * CT + row / 16][quad * 16 + row % 16];
+    mf4 v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = f32_gate(g[e], up[e], gate);
+    *reinterpret_cast<mf4*>(out + static_cast<size_t>(t0 + row) * ldo + f0 * 16 + quad * 4) = v;
+    return;
+  }
+  if (GROUPS) out += static_cast<size_t>(blockIdx.y) * n * ldo;
 #pragma unroll
   for (int c = 0; c < CT; ++c) {
     const int row = t0 + (nw * CT + c) * 16 + i;  // the matrix instruction's columns
@@ -492,12 +515,14 @@ static void launch_f32(const F32Product& p, hipStream_t s) {
                                                p.a_batch, p.w_batch, p.out_batch);
 }
 
-template <int RT, int CT>
-static void launch_f32_lds(const F32Product& p, hipStream_t s) {
-  const int tiles = (p.m + 32 * RT - 1) / (32 * RT) * ((p.n + 32 * CT - 1) / (32 * CT));
+template <int RT, int CT, bool GATED = false, bool GROUPS = false>
+static void launch_f32_lds(const F32Product& p, hipStream_t s, F32Gate gate = F32Gate{}) {
+  constexpr int F = GATED ? 16 : 32 * RT;
+  const int tiles = (p.m + F - 1) / F * ((p.n + 32 * CT - 1) / (32 * CT));
   const int vec_out = p.ldo % 4 == 0 && reinterpret_cast<uintptr_t>(p.out) % 16 == 0;
-  gemm_f32_lds_kernel<RT, CT><<<(tiles + kDies - 1) / kDies * kDies, 4 * kWave, 0, s>>>(p.a, p.w, p.bias, p.out, p.n, p.m, p.k, p.lda,
-                                                                                    p.ldo, p.accumulate, vec_out);
+  const dim3 grid((tiles + kDies - 1) / kDies * kDies, GROUPS ? kF32Segments / kF32Group : 1);
+  gemm_f32_lds_kernel<RT, CT, GATED, GROUPS><<<grid, 4 * kWave, 0, s>>>(p.a, p.w, p.bias, p.out, p.n, p.m, p.k, p.lda, p.ldo, p.accumulate,
+                                                                        vec_out, gate);
 }
 
 // Whether gemm_f32_few_kernel takes a product of tiled weights.  (151936 x 896: 98 / 107 us at 4 / 16 rows in gemm_f32_kernel's
@@ -625,33 +650,53 @@ extern "C" int shk_retile_f32(const void* w, int m, int k, void* wt, void* strea
   return 0;
 }
 
+// Sizes for which gemm_f32_lds_kernel forms groups (from a k of 768 on: none of them is empty) and gated products: whole stages, a
+// matrix's offsets of 32 bits.
+static bool f32_staged(int m, int k, int lda) {
+  return k % 32 == 0 && k > 256 && lda <= 1 << 20 && static_cast<long long>(m) * k < 1LL << 30;
+}
+
 // Groups in which shk_gemm_f32_groups leaves a product for its reader (1: it is formed whole): four where a long k would
 // be walked in few workgroups: with the norm that adds its output 896 x 4864 at 1 / 4 / 16 rows 13.7 / 14.1 / 20.7 us whole, 10.0 /
-// 10.2 / 13.2 in groups, 1536 x 8960 22.4 / 22.9 / 34.5 and 18.9 / 19.5 / 27.7.
+// 10.2 / 13.2 in groups, 1536 x 8960 22.4 / 22.9 / 34.5 and 18.9 / 19.5 / 27.7.  The same of more rows: 896 x 4864 at 33 / 64 / 128 / 509 /
+// 1,024 / 2,000 rows 19.5 / 21.1 / 27.6 / 56.4 / 92.3 / 170 and 20.3 / 20.2 / 20.7 / 48.6 / 85.2 / 174, 1536 x 8960 at 64 / 509 / 700 /
+// 1,024 44 / 174 / 222 / 239 and 32 / 126 / 176 / 244: up to 640 workgroups a group.  A short k gains nothing: 512 x 2048 at 64 / 320
+// rows 11.2 / 16.8 and 11.9 / 16.8.
 extern "C" int shk_gemm_f32_splits(int n, int m, int k) {
-  return n <= 16 && m <= 2048 && m % 4 == 0 && k >= 2048 && k % 16 == 0 ? kF32Segments / kF32Group : 1;
+  const long long tiles = (m + 31LL) / 32 * ((n + 63) / 64);
+  const bool few = n <= 16 && m <= 2048 && k >= 2048 && k % 16 == 0, more = n >= 64 && k >= 4096 && tiles <= 640 && f32_staged(m, k, k);
+  return m % 4 == 0 && (few || more) ? kF32Segments / kF32Group : 1;
 }
 
 extern "C" int shk_gemm_f32_groups(const void* a, const void* wt, void* out, int n, int m, int k, int lda, void* stream) {
-  SHK_REQUIRE(n >= 0 && n <= 16 && m > 0 && k > 0 && k % 16 == 0 && lda >= k && lda % 4 == 0,
+  SHK_REQUIRE(n >= 0 && m > 0 && k > 0 && k % 16 == 0 && lda >= k && lda % 4 == 0 && (n <= 16 || (k >= 768 && f32_staged(m, k, lda))),
               "gemm_f32_groups: bad sizes n=%d m=%d k=%d lda=%d", n, m, k, lda);
   if (n == 0) return 0;
   SHK_REQUIRE(a && wt && out && reinterpret_cast<uintptr_t>(wt) % 16 == 0 && reinterpret_cast<uintptr_t>(a) % 16 == 0,
               "gemm_f32_groups: null or misaligned pointer");
-  with_steps<10>((k + 16 * kF32Segments - 1) / (16 * kF32Segments), [&](auto c) {
-    gemm_f32_few_kernel<4, 8, c.value, false, true><<<dim3((m + 7) / 8, kF32Segments / kF32Group), 4 * kWave, 0, static_cast<hipStream_t>(stream)>>>(
-        static_cast<const float*>(a), static_cast<const float*>(wt), nullptr, static_cast<float*>(out), n, m, k, lda, m, 0, F32Gate{});
-  });
+  const F32Product p{static_cast<const float*>(a), static_cast<const float*>(wt), nullptr, static_cast<float*>(out), n, m, k, lda, m, 0, 1, 0, 0, 0};
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  if (n <= 16)
+    with_steps<10>((k + 16 * kF32Segments - 1) / (16 * kF32Segments), [&](auto c) {
+      gemm_f32_few_kernel<4, 8, c.value, false, true><<<dim3((m + 7) / 8, kF32Segments / kF32Group), 4 * kWave, 0, s>>>(
+          p.a, p.w, nullptr, p.out, n, m, k, lda, m, 0, F32Gate{});
+    });
+  else
+    launch_f32_lds<1, 2, false, true>(p, s);
   SHK_LAUNCH_CHECK("gemm_f32_groups");
   return 0;
 }
 
-// Whether shk_gemm_f32_gated takes a product of 2 m features, gate and other factor.
-extern "C" int shk_gemm_f32_gated_takes(int n, int m, int k) { return n <= 16 && m > 0 && m % 16 == 0 && k > 0 && k % 16 == 0; }
+// Whether shk_gemm_f32_gated takes a product of 2 m features, gate and other factor.  Product and gate against it, more than 16
+// rows: 4864 x 896 at 17 / 64 / 128 / 509 / 2,000 16.5 / 20.6 / 29.5 / 88.1 / 356 -> 14.2 / 17.8 / 26.9 / 83.2 / 346 us, 8960 x 1536 at
+// 17 / 509 49.6 / 250 -> 30.7 / 247, 512 x 288 6.2 / 9.3 -> 5.4 / 7.0.
+extern "C" int shk_gemm_f32_gated_takes(int n, int m, int k) {
+  return m > 0 && m % 16 == 0 && k > 0 && k % 16 == 0 && (n <= 16 || f32_staged(m, k, k));
+}
 
 extern "C" int shk_gemm_f32_gated(const void* a, const void* wt, void* out, int n, int m, int k, int lda, int act, float limit,
                                   float up_shift, void* stream) {
-  SHK_REQUIRE(n >= 0 && n <= 16 && m > 0 && m % 16 == 0 && k > 0 && k % 16 == 0 && lda >= k && lda % 4 == 0,
+  SHK_REQUIRE(n >= 0 && m > 0 && m % 16 == 0 && k > 0 && k % 16 == 0 && lda >= k && lda % 4 == 0 && (n <= 16 || f32_staged(m, k, lda)),
               "gemm_f32_gated: bad sizes n=%d m=%d k=%d lda=%d", n, m, k, lda);
   SHK_REQUIRE(act >= 1 && act <= 4 && limit >= 0.f, "gemm_f32_gated: unknown gate");
   if (n == 0) return 0;
@@ -659,6 +704,15 @@ extern "C" int shk_gemm_f32_gated(const void* a, const void* wt, void* out, int 
               "gemm_f32_gated: null or misaligned pointer");
   const int seg_steps = (k + 16 * kF32Segments - 1) / (16 * kF32Segments);
   const F32Gate gate = {act, limit, up_shift};
+  if (n > 16) {
+    const F32Product p{static_cast<const float*>(a), static_cast<const float*>(wt), nullptr, static_cast<float*>(out), n, m, k, lda, m, 0, 1, 0, 0, 0};
+    if (m / 16 * ((n + 63LL) / 64) >= 1536)  // (as for the product whole)
+      launch_f32_lds<1, 2, true>(p, static_cast<hipStream_t>(stream), gate);
+    else
+      launch_f32_lds<1, 1, true>(p, static_cast<hipStream_t>(stream), gate);
+    SHK_LAUNCH_CHECK("gemm_f32_gated");
+    return 0;
+  }
   const auto go = [&](auto kernel, int waves) {
     kernel<<<m / 16, waves * kWave, 0, static_cast<hipStream_t>(stream)>>>(static_cast<const float*>(a), static_cast<const float*>(wt), nullptr,
                                                                            static_cast<float*>(out), n, m, k, lda, m, 0, gate);

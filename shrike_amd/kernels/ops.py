@@ -383,8 +383,8 @@ def gemm_f32_gated_takes(n: int, m: int, k: int) -> bool:
 
 
 def f32_rows_aligned(x) -> bool:
-    """Whether the rows of a float32 matrix begin at multiples of 16 bytes."""
-    return x.data_ptr() % 16 == 0 and x.stride(0) % 4 == 0
+    """Whether the rows of a float32 matrix begin at multiples of 16 bytes, not too far apart for gemm_f32_groups and _gated."""
+    return x.data_ptr() % 16 == 0 and x.stride(0) % 4 == 0 and x.stride(0) <= 1 << 20
 
 
 def gemm_f32_groups(a, wt, m: int, k: int, out) -> None:
@@ -400,7 +400,7 @@ def gemm_f32_groups(a, wt, m: int, k: int, out) -> None:
 
 
 def gemm_f32_gated(a, wt, m: int, k: int, out, activation, limit=None, up_shift: float = 0.0) -> None:
-    """out [n, m] = act_mul() of gemm_f32_tiled_weight()'s [n, 2 m], the same bits; up to 16 rows."""
+    """out [n, m] = act_mul() of gemm_f32_tiled_weight()'s [n, 2 m], the same bits."""
     _rows(a, "gemm_f32_gated a")
     n = a.shape[0]
     if a.shape[1] != k or tuple(out.shape) != (n, m) or not out.is_contiguous():

@@ -1,5 +1,5 @@
 """float32 products of up to 16 rows: the bits of the same rows among more of them, whole, in groups and with the gate,
-at the edges of segments, batches of steps and blocks of features."""
+at the edges of segments, batches of steps and blocks of features; groups and gate of more rows against the whole product."""
 
 import pytest
 import torch
@@ -62,7 +62,7 @@ def test_groups_that_the_norm_adds(m, k, n):
 def test_a_gate_in_the_product(m, k, n, activation, limit, shift):
     from shrike_amd.kernels import ops
 
-    assert ops.gemm_f32_gated_takes(n, m, k) and not ops.gemm_f32_gated_takes(17, m, k)
+    assert ops.gemm_f32_gated_takes(n, m, k)
     a, w = operands(2 * m, k)
     wt = ops.retile_f32(w)
     both, want = torch.empty(n, 2 * m, device="cuda"), torch.empty(n, m, device="cuda")
@@ -70,4 +70,34 @@ def test_a_gate_in_the_product(m, k, n, activation, limit, shift):
     ops.act_mul(both, want, activation, limit, shift)
     out = torch.empty(n, m, device="cuda")
     ops.gemm_f32_gated(a[:n], wt, m, k, out, activation, limit, shift)
+    assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("n", [64, 65, 200, 509])
+@pytest.mark.parametrize("m, k", [(896, 4864), (20, 4096), (1004, 4128), (64, 8992)])
+def test_groups_of_more_rows(m, k, n):
+    from shrike_amd.kernels import ops
+
+    assert ops.gemm_f32_splits(n, m, k) == 4 and ops.gemm_f32_splits(2000, 896, 4864) == ops.gemm_f32_splits(n, m, k + 16) == 1
+    torch.manual_seed(m + k + n)
+    a, w = torch.randn(n, k + 4, device="cuda")[:, :k], torch.randn(m, k, device="cuda") / k**0.5
+    wt, whole, parts = ops.retile_f32(w), torch.empty(n, m, device="cuda"), torch.full((4, n, m), 7.0, device="cuda")
+    ops.gemm_f32_tiled_weight(a, wt, m, k, whole)
+    ops.gemm_f32_groups(a, wt, m, k, parts)
+    assert torch.equal(((parts[0] + parts[1]) + parts[2]) + parts[3], whole)
+
+
+@pytest.mark.parametrize("n", [17, 32, 33, 64, 65, 509])
+@pytest.mark.parametrize("m, k", [(16, 288), (48, 512), (4864, 896), (304, 1056), (64, 4896)])
+def test_a_gate_in_the_product_of_more_rows(m, k, n):
+    from shrike_amd.kernels import ops
+
+    assert ops.gemm_f32_gated_takes(n, m, k) and not ops.gemm_f32_gated_takes(n, m, 256)
+    torch.manual_seed(m + k + n)
+    a, w = torch.randn(n, k + 4, device="cuda")[:, :k], torch.randn(2 * m, k, device="cuda") / k**0.5
+    wt = ops.retile_f32(w)
+    both, want, out = torch.empty(n, 2 * m, device="cuda"), torch.empty(n, m, device="cuda"), torch.empty(n, m, device="cuda")
+    ops.gemm_f32_tiled_weight(a, wt, 2 * m, k, both)
+    ops.act_mul(both, want, "gelu_tanh", 0.5, 1.0)
+    ops.gemm_f32_gated(a, wt, m, k, out, "gelu_tanh", 0.5, 1.0)
     assert torch.equal(out, want)
