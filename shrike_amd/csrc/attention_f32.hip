@@ -14,8 +14,8 @@
 // product's operand as it stands: weights never pass through LDS.  What bounds it: a block is 64 + 64
 // instructions of 32 cycles per wavefront (head size 64: 4,096 cycles) and three barriers.  14 heads of 64
 // over 2, 509 tokens: 560 us a layer in the general kernel, whose one workgroup per query head had one key
-// per thread, 39 here; four single tokens at about 400: 50 us, here 12 and 4.4 for the join (whole passes: a
-// prompt of 24 such layers 18.9 ms then, 6.5 now; a decode step of four requests 2.43 ms, 1.56 now).  A
+// per thread, 38 with a workgroup a token, 24 with one for two (kPair: most of the 16 columns then hold a head); four single tokens at about 400: 50 us, here 12 and 4.4 for the join (whole passes: a
+// prompt of 24 such layers 18.9 ms then, 6.5 with a workgroup a token; a decode step of four requests 2.43 ms, 1.56 now).  A
 // single token's block is one chain from the page numbers over keys and values to the join, so all page
 // numbers are read first, without a branch, then as many steps' keys and values as registers hold before the
 // first product (head size 64: all of them; with each step's loads next to its products 16 us for the 12).  A
@@ -51,20 +51,38 @@ __device__ __forceinline__ float keys_share(float M, float& L, const float* sink
   return share;
 }
 
-// D: sixteens of the larger of head_dim and v_dim
-template <int D, bool kSplit>
-__global__ void __launch_bounds__(kWave * kBlockWaves) attention_f32_kernel(F32Attention p) {
+// D: sixteens of the larger of head_dim and v_dim.  kPair: up to eight query heads a key/value head, whose columns two
+// neighbouring tokens of one sequence share, the first in columns 0 to 7.
+template <int D, bool kSplit, bool kPair>
+__global__ void __launch_bounds__(kWave * kBlockWaves) attention_f32_kernel(F32Attention p, int n) {
   __shared__ af4 sums[kBlockWaves][D][kWave];
   __shared__ float tops[kBlockWaves][16], weights[kBlockWaves][16];
   const int lane = threadIdx.x % kWave, i = lane % 16, kg = lane / 16;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int per = p.heads / p.kv_heads, parts = (per + 15) / 16;
-  const int kvh = blockIdx.x / parts, in_group = blockIdx.x % parts * 16 + i;
-  const bool row = in_group < per;
-  const int head = kvh * per + (row ? in_group : 0);
-  const int t = blockIdx.y;
-  const int pos = p.positions[t], lo = first_key(pos, p.window, p.chunk);
-  const int32_t* table = p.tables + static_cast<size_t>(p.token_seq[t]) * p.table_stride;
+  const int kvh = blockIdx.x / parts, in_group = kPair ? i % 8 : blockIdx.x % parts * 16 + i;
+  // (pairs first, the last of the prompt's before the others, then the tokens that most often are a pair's second: in the order
+  // of the tokens every other workgroup would have nothing to do, and with two key/value heads so would four of the eight dies)
+  const int pairs = (n + 1) / 2, y = blockIdx.y;
+  const int t0 = !kPair ? y : y < pairs ? 2 * (pairs - 1 - y) : 2 * (y - pairs) + 1, seq = p.token_seq[t0];
+  const int pos0 = p.positions[t0];
+  int t1 = t0, pos1 = pos0;  // the token of columns 8 to 15
+  if constexpr (kPair) {
+    // (the other token of a pair; read without a condition, so that these loads travel together)
+    const int other = min(t0 ^ 1, n - 1), beside = p.positions[other];
+    const bool same = other != t0 && p.token_seq[other] == seq;
+    if (same && t0 % 2) return;
+    if (same) t1 = other, pos1 = beside;
+  }
+  const int lo0 = first_key(pos0, p.window, p.chunk), lo1 = kPair ? first_key(pos1, p.window, p.chunk) : lo0;
+  const bool later = kPair && i >= 8;  // this column's token is t1
+  const int t = later ? t1 : t0;
+  const bool row = in_group < per && (!later || t1 != t0);
+  const int head = kvh * per + (kPair ? min(in_group, per - 1) : row ? in_group : 0);
+  // keys of either token, of this column's
+  const int pos = kPair ? max(pos0, pos1) : pos0, lo = kPair ? min(lo0, lo1) : lo0;
+  const int mine_to = later ? pos1 : pos0, mine_from = later ? lo1 : lo0;
+  const int32_t* table = p.tables + static_cast<size_t>(seq) * p.table_stride;
   int first = lo / kKeyBlock, last = pos / kKeyBlock, step = 1;
   if (kSplit) {
     first += blockIdx.z;
@@ -173,8 +191,8 @@ __global__ void __launch_bounds__(kWave * kBlockWaves) attention_f32_kernel(F32A
         const int key = key0 + 16 * u + 4 * kg + e;
         float x = s[u][e] * p.scale;
         if (p.softcap > 0.f) x = p.softcap * tanhf(x / p.softcap);
-        const bool have = key >= lo && key <= pos && v_at[u] >= 0;
-        if (p.dist_bias && have) x += p.dist_bias[static_cast<size_t>(head) * p.bias_rows + min(pos - key, p.bias_rows - 1)];
+        const bool have = key >= mine_from && key <= mine_to && v_at[u] >= 0;
+        if (p.dist_bias && have) x += p.dist_bias[static_cast<size_t>(head) * p.bias_rows + min(mine_to - key, p.bias_rows - 1)];
         s[u][e] = have ? x : -INFINITY;
         top = fmaxf(top, s[u][e]);
       }
@@ -199,6 +217,30 @@ __global__ void __launch_bounds__(kWave * kBlockWaves) attention_f32_kernel(F32A
         if (u >= kAhead && u % kAhead == 0)
 #pragma unroll
           for (int ahead = u; ahead < u + kAhead; ++ahead) load_values(ahead);
+        // what one of two tokens may read and the other may not must not meet the other's weight of 0 (it may be infinite)
+        const int step0 = key0 + 16 * u;
+        if (kPair && ((pos0 != pos1 && step0 <= pos && step0 + 15 > min(pos0, pos1)) ||
+                      (lo0 != lo1 && step0 < max(lo0, lo1) && step0 + 15 >= lo))) {
+          af4 other[D];
+#pragma unroll
+          for (int x = 0; x < D; ++x) other[x] = acc[x];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int key = step0 + 4 * kg + e;
+            const bool have0 = key >= lo0 && key <= pos0 && v_at[u] >= 0, have1 = key >= lo1 && key <= pos1 && v_at[u] >= 0;
+            const float w = (i < 8 ? have0 : have1) ? expf(s[u][e] - origin) : 0.f;
+            l += w;
+#pragma unroll
+            for (int x = 0; x < D; ++x) {
+              acc[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(have0 ? vv[u % kAhead][x][e] : 0.f, w, acc[x], 0, 0, 0);
+              other[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(have1 ? vv[u % kAhead][x][e] : 0.f, w, other[x], 0, 0, 0);
+            }
+          }
+#pragma unroll
+          for (int x = 0; x < D; ++x)
+            if (i >= 8) acc[x] = other[x];
+          continue;
+        }
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int key = key0 + 16 * u + 4 * kg + e;
@@ -282,10 +324,16 @@ static void launch(const F32Attention& p, int n, int splits, hipStream_t s) {
   const int per = p.heads / p.kv_heads;
   const dim3 grid(p.kv_heads * ((per + 15) / 16), n, splits);
   if (splits > 1) {
-    attention_f32_kernel<D, true><<<grid, kWave * kBlockWaves, 0, s>>>(p);
+    attention_f32_kernel<D, true, false><<<grid, kWave * kBlockWaves, 0, s>>>(p, n);
     attention_f32_join_kernel<<<dim3(p.heads, n), (p.v_dim + kWave - 1) / kWave * kWave, 0, s>>>(p);
   } else {
-    attention_f32_kernel<D, false><<<grid, kWave * kBlockWaves, 0, s>>>(p);
+    // Pairs where tokens by themselves would be workgroups for the chip one and a half times (heads of 64: two workgroups fit on a
+    // compute unit) or three times (128: one does), else two tokens' chain of work is the longer one.  14 heads of 64 over 2,
+    // at 165 / 200 / 509 / 2,000 tokens 11.3 / 14.1 / 37.7 / 366 us by themselves, 12.3 / 12.8 / 24.4 / 198 in pairs, 28 of 128 over 4 at
+    // 130 / 200 / 509 / 2,000 31.6 / 38.8 / 114 / 1,237 and 35.1 / 36.6 / 98.8 / 955.  (Heads of more than 128 fill the registers.)
+    constexpr bool kPairs = D <= 8;
+    const auto kernel = per <= 8 && p.kv_heads * n > (D <= 6 ? 384 : 768) ? attention_f32_kernel<D, false, kPairs> : attention_f32_kernel<D, false, false>;
+    kernel<<<grid, kWave * kBlockWaves, 0, s>>>(p, n);
   }
 }
 
