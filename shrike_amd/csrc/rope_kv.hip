@@ -140,12 +140,82 @@ __global__ void __launch_bounds__(kRopeThreads)
 // The same for bfloat16 rows that are rotated whole (rot_dim == head_dim, a
 // multiple of 16): one workgroup per token, a thread moves 8 neighbouring
 // elements at a time (16 bytes; a rotated pair is two such runs, head_dim / 2
-// apart), so that queries and keys travel in whole vectors.  Values go to
-// their transposed pages element by element.  Arithmetic as above.
+// apart), so that queries and keys travel in whole vectors.  Values have
+// workgroups of their own, the first of the grid.  Arithmetic as above.
 constexpr int kVecItems = 4;  // runs (or pairs of runs) per thread at most
 // from this many tokens on; fewer (decode steps) are a matter of latency, which the
 // kernel above with its ten workgroups per token and eight parts in flight handles better
 constexpr int kVecMinTokens = 65;
+
+// Values of kValueTokens neighbouring tokens of a step into their pages [head_dim][page_size]: a thread moves one element of
+// each, so that what lies side by side in a page is written by one thread, in one piece where the tokens are neighbours
+// there too.  Token by token sixteen workgroups on all dies wrote two bytes each of the same 32.
+// The whole kernel, us, token by token and so: 40 heads of 128 over 8 at 512 / 1,119 / 2,048 tokens 13.3 / 24.3 / 22.3 -> 10.5 / 19.3 /
+// 16.9, 28 over 4 9.4 / 15.0 / 15.5 -> 8.0 / 11.9 / 12.2 (portions that begin inside a piece 15.5 -> 13.9), 14 of 64 over 2 5.5 / 8.8 /
+// 9.0 -> 5.6 / 7.9 / 8.4.  Every thread looking up all eight pages itself: 10.9 / 20.1 / 18.6, 7.9 / 12.4 / 13.3, 5.7 / 8.0 / 8.6.
+constexpr int kValueTokens = 8;
+
+__device__ __forceinline__ void store_values(int first, int col, int n, int width, int values, int kv_heads, int head_dim,
+                                             const bf16* __restrict__ qkv, const int32_t* __restrict__ positions,
+                                             const int32_t* __restrict__ token_seq, const int32_t* __restrict__ tables, int table_stride,
+                                             bf16* __restrict__ v_pool, int page_size, int num_pages,
+                                             const float* __restrict__ parts, int splits, const float* __restrict__ bias) {
+  // a lane looks up one token's page and slot for its wavefront
+  const int mine = first + static_cast<int>(threadIdx.x) % kValueTokens, token = min(mine, n - 1), pos = positions[token];
+  int my_page = tables[static_cast<size_t>(token_seq[token]) * table_stride + pos / page_size];
+  if (mine >= n || my_page < 0 || my_page >= num_pages) my_page = -1;  // (none, or a host bug: never dereferenced)
+  const int my_slot = pos % page_size;
+  const bool inside = col < kv_heads * head_dim;
+  if (!inside) col = 0;
+  float x[kValueTokens];
+  if (splits == 0) {
+    bf16 raw[kValueTokens];
+#pragma unroll
+    for (int g = 0; g < kValueTokens; ++g) raw[g] = qkv[static_cast<size_t>(min(first + g, n - 1)) * width + values + col];
+#pragma unroll
+    for (int g = 0; g < kValueTokens; ++g) x[g] = to_float(raw[g]);
+  } else {
+#pragma unroll
+    for (int g = 0; g < kValueTokens; ++g) x[g] = 0.f;
+    for (int z0 = 0; z0 < splits; z0 += 2) {  // two parts in flight, added in order
+      float v[2][kValueTokens];
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int g = 0; g < kValueTokens; ++g)
+          v[u][g] = parts[(static_cast<size_t>(min(z0 + u, splits - 1)) * n + min(first + g, n - 1)) * width + values + col];
+#pragma unroll
+      for (int g = 0; g < kValueTokens; ++g) x[g] += v[0][g], x[g] += z0 + 1 < splits ? v[1][g] : 0.f;
+    }
+    if (bias) {
+      const float add = bias[values + col];
+#pragma unroll
+      for (int g = 0; g < kValueTokens; ++g) x[g] += add;
+    }
+  }
+  int page[kValueTokens], slot[kValueTokens];
+  bool neighbours = true;
+#pragma unroll
+  for (int g = 0; g < kValueTokens; ++g) {
+    page[g] = __builtin_amdgcn_readlane(my_page, g);
+    slot[g] = __builtin_amdgcn_readlane(my_slot, g);
+    neighbours &= page[g] >= 0 && page[g] == page[0] && slot[g] == slot[0] + g;
+  }
+  const size_t row = static_cast<size_t>(kv_heads) * page_size * head_dim, at = static_cast<size_t>(col) * page_size;
+  if (!inside) return;
+  if (neighbours && slot[0] % 8 == 0 && page_size % 8 == 0 && reinterpret_cast<uintptr_t>(v_pool) % 16 == 0) {
+    uint4 out;
+    out.x = bf16_bits(x[0]) | (static_cast<uint32_t>(bf16_bits(x[1])) << 16);
+    out.y = bf16_bits(x[2]) | (static_cast<uint32_t>(bf16_bits(x[3])) << 16);
+    out.z = bf16_bits(x[4]) | (static_cast<uint32_t>(bf16_bits(x[5])) << 16);
+    out.w = bf16_bits(x[6]) | (static_cast<uint32_t>(bf16_bits(x[7])) << 16);
+    *reinterpret_cast<uint4*>(v_pool + page[0] * row + at + slot[0]) = out;
+    return;
+  }
+#pragma unroll
+  for (int g = 0; g < kValueTokens; ++g)
+    if (page[g] >= 0) v_pool[page[g] * row + at + slot[g]] = from_float<bf16>(x[g]);
+}
 
 __global__ void __launch_bounds__(kRopeThreads)
     rope_kv_store_vec_kernel(bf16* __restrict__ qkv, int n, int heads, int kv_heads, int head_dim,
@@ -155,17 +225,22 @@ __global__ void __launch_bounds__(kRopeThreads)
                              const int32_t* __restrict__ tables, int table_stride,
                              bf16* __restrict__ k_pool, bf16* __restrict__ v_pool, int page_size,
                              int num_pages, int write_kv, const float* __restrict__ parts, int splits,
-                             const float* __restrict__ bias, float magnitude) {
+                             const float* __restrict__ bias, float magnitude, unsigned value_blocks) {
   __shared__ float cs[kMaxHalf];
   __shared__ float sn[kMaxHalf];
-  const int t = blockIdx.x;
-  const int pos = positions[t];
   const int half = head_dim / 2;
   const int width = (heads + 2 * kv_heads) * head_dim;
+  if (blockIdx.x < value_blocks) {
+    const int per = (kv_heads * head_dim + kRopeThreads - 1) / kRopeThreads;
+    store_values(blockIdx.x / per * kValueTokens, blockIdx.x % per * kRopeThreads + threadIdx.x, n, width, (heads + kv_heads) * head_dim,
+                 kv_heads, head_dim, qkv, positions, token_seq, tables, table_stride, v_pool, page_size, num_pages, parts, splits, bias);
+    return;
+  }
+  const int t = blockIdx.x - value_blocks;
+  const int pos = positions[t];
   bf16* row = qkv + static_cast<size_t>(t) * width;
   const int per_head = half / 8;                      // pairs of runs in a rotated head
   const int n_pairs = (heads + kv_heads) * per_head;  // queries, then keys
-  const int n_values = kv_heads * (head_dim / 8);
   const size_t split_stride = static_cast<size_t>(n) * width;
 
   // 8 elements from column `col` on: the row itself, or the sum of its parts and the bias
@@ -223,8 +298,6 @@ __global__ void __launch_bounds__(kRopeThreads)
       const int col = (item / per_head) * head_dim + (item % per_head) * 8;
       fetch(col, a[u]);
       fetch(col + half, b[u]);
-    } else if (item < n_pairs + n_values) {
-      fetch((heads + kv_heads) * head_dim + (item - n_pairs) * 8, a[u]);
     }
   }
 
@@ -267,11 +340,6 @@ __global__ void __launch_bounds__(kRopeThreads)
         *reinterpret_cast<uint4*>(dst + key_offset(slot, i, page_size, head_dim)) = pack(lo);
         *reinterpret_cast<uint4*>(dst + key_offset(slot, i + half, page_size, head_dim)) = pack(hi);
       }
-    } else if (item < n_pairs + n_values && page >= 0) {
-      const int d0 = (item - n_pairs) * 8;  // kv head * head_dim + element
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        v_pool[page_base + static_cast<size_t>(d0 + e) * page_size + slot] = from_float<bf16>(a[u][e]);
     }
   }
 }
@@ -450,10 +518,12 @@ extern "C" int shk_rope_kv_store(void* qkv, int dtype, int n, int heads, int kv_
       vec_items <= kVecItems * kRopeThreads && reinterpret_cast<uintptr_t>(qkv) % 16 == 0 &&
       (!write_kv || reinterpret_cast<uintptr_t>(k_pool) % 16 == 0) &&
       (!parts || reinterpret_cast<uintptr_t>(parts) % 16 == 0)) {
-    rope_kv_store_vec_kernel<<<n, kRopeThreads, 0, s>>>(
+    const int per = (kv_heads * head_dim + kRopeThreads - 1) / kRopeThreads;
+    const unsigned value_blocks = write_kv ? static_cast<unsigned>((n + kValueTokens - 1) / kValueTokens) * per : 0;
+    rope_kv_store_vec_kernel<<<n + value_blocks, kRopeThreads, 0, s>>>(
         static_cast<bf16*>(qkv), n, heads, kv_heads, head_dim, inv_freq, positions, token_seq, tables,
         table_stride, static_cast<bf16*>(k_pool), static_cast<bf16*>(v_pool), page_size, num_pages,
-        write_kv, parts, splits, bias, magnitude);
+        write_kv, parts, splits, bias, magnitude, value_blocks);
     SHK_LAUNCH_CHECK("rope_kv_store");
     return 0;
   }
