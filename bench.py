@@ -314,6 +314,28 @@ def measure_peaks(device="cuda:0") -> dict:
     return out
 
 
+# the functions of shrike_amd.kernels.ops that launch a step's kernels
+TIMED_OPS = ("embed", "add_rmsnorm", "act_mul", "gemm", "gemm_f32_tiled_weight", "gemm_f32_groups", "gemm_f32_gated", "latent_prompt",
+             "gemm_tiled_weight", "few_stream", "few_gated", "few_heads", "rope_kv_store", "attention",
+             "attention_decode", "attention_prefill", "attention_prefill_shared", "argmax", "sample",
+             "add_deltas", "add_normed_rmsnorm", "act_mul_rows", "add_rows", "embed_pairs", "qkv_store",
+             "latent_prepare", "rotate_heads", "latent_attention", "latent_attention_mfma", "gemm_batched", "mlstm_scan", "headnorm_gate",
+             "xielu", "add_layernorm", "attention_talking", "attention_talking_mfma", "short_conv", "dt_softplus", "selective_scan",
+             "rotate_half_rows", "retention_scan", "retention_chunk", "moe_route", "moe_experts", "moe_few", "mix_history",
+             "scale_softcap", "postnorm", "cast_rows", "activate", "gate_mul", "add_dynamic_tanh", "conv_store", "diff_attention",
+             "diff_attention_decode", "diff_attention_prefill", "rglru", "gla_chunk")
+
+
+def timed_label(name: str, args, kwargs) -> str:
+    """What a call of one of TIMED_OPS is listed under: products are told apart by their matrix [m, k]."""
+    if name in ("gemm_tiled_weight", "few_stream", "few_gated", "gemm_f32_groups", "gemm_f32_gated"):
+        kind = "gemm" if name == "gemm_tiled_weight" else name
+        return f"{kind} {args[2]}x{args[3]}" + (" gated" if kwargs.get("gated") else "")
+    if name == "few_heads":  # (rows, weights, k, out, ..): out is as wide as the matrix has rows
+        return f"few_heads {args[3].shape[1]}x{args[2]}"
+    return name
+
+
 def kernel_breakdown(engine, steps: int = 3, before_step=None) -> dict:
     """Microseconds per step by kernel: the running requests' next steps run kernel by
     kernel (no graph) with an event before and after every launch.  `before_step()` is
@@ -322,28 +344,16 @@ def kernel_breakdown(engine, steps: int = 3, before_step=None) -> dict:
 
     from shrike_amd.kernels import ops
 
-    names = ["embed", "add_rmsnorm", "act_mul", "gemm", "gemm_f32_tiled_weight", "latent_prompt", "gemm_tiled_weight", "rope_kv_store", "attention",
-             "attention_decode", "attention_prefill", "attention_prefill_shared", "argmax", "sample",
-             "add_deltas", "add_normed_rmsnorm", "act_mul_rows", "add_rows", "embed_pairs", "qkv_store",
-             "latent_prepare", "rotate_heads", "latent_attention", "latent_attention_mfma", "gemm_batched", "mlstm_scan", "headnorm_gate",
-             "xielu", "layernorm", "add_layernorm", "attention_talking", "attention_talking_mfma", "short_conv", "dt_softplus", "selective_scan",
-             "rotate_half_rows", "retention_scan", "retention_chunk", "moe_route", "moe_experts", "mix_history", "scale_softcap",
-             "postnorm", "cast_rows", "activate", "gate_mul", "add_dynamic_tanh", "conv_store", "diff_attention",
-             "diff_attention_decode", "diff_attention_prefill", "rglru", "gla_chunk"]
-    names = [n for n in names if hasattr(ops, n)]
     spans: list[tuple[str, object, object]] = []
-    saved = {n: getattr(ops, n) for n in names}
+    saved = {n: getattr(ops, n) for n in TIMED_OPS}
 
     def wrap(name, fn):
         def timed(*args, **kwargs):
-            label = name
-            if name == "gemm_tiled_weight":  # told apart by the matrix: [m, k]
-                label = f"gemm {args[2]}x{args[3]}" + (" gated" if kwargs.get("gated") else "")
             a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
             a.record()
             out = fn(*args, **kwargs)
             b.record()
-            spans.append((label, a, b))
+            spans.append((timed_label(name, args, kwargs), a, b))
             return out
         return timed
 
