@@ -464,7 +464,13 @@ __global__ void __launch_bounds__(4 * kWave)
     mf4 v;
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] = f32_gate(g[e], up[e], gate);
-    *reinterpret_cast<mf4*>(out + static_cast<size_t>(t0 + row) * ldo + f0 * 16 + quad * 4) = v;
+    float* dst = out + static_cast<size_t>(t0 + row) * ldo + f0 * 16 + quad * 4;
+    if (vec_out) {
+      *reinterpret_cast<mf4*>(dst) = v;
+    } else {  // (out does not begin at a multiple of 16 bytes)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) dst[e] = v[e];
+    }
     return;
   }
   if (GROUPS) out += static_cast<size_t>(blockIdx.y) * n * ldo;
