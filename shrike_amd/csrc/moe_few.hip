@@ -50,9 +50,11 @@ struct MoeFewList {
       if (k < top && pick[k] == e) hit = k;
     const unsigned long long votes = __ballot(lane < n && hit >= 0);
     count = __popcll(votes);
-    // the r-th hit's pair to lane r, through LDS of this wavefront's own
+    // the r-th hit's pair to lane r, through LDS of this wavefront's own; the fences order one lane's write and another's read
     if (lane < n && hit >= 0) place[__popcll(votes & ((1ull << lane) - 1ull))] = lane * top + hit;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     mine = place[lane < 16 ? lane : 0];
   }
 };
