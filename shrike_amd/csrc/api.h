@@ -223,12 +223,14 @@ int shk_rope_kv_store(void* qkv, int dtype, int n, int heads, int kv_heads, int 
 // partial (or null) and splits: float32 heads of a multiple of 4 elements with pages of a multiple of 4 tokens may form
 // a token's blocks of 256 keys in up to `splits` workgroups; partial holds n * heads * ceil(table_stride * page_size /
 // 256) * (v_dim + 2) floats.  The result is the same bits.
+// pairs: two neighbouring tokens of a sequence share a workgroup of float32 attention where there are enough of them (1), or
+// each token has its own (0); -1: pairs for heads of up to 96.  The result is the same bits.
 int shk_attention(const void* q, int q_stride, void* out, int dtype, int n, int heads,
                   int kv_heads, int head_dim, const int32_t* positions, const int32_t* token_seq,
                   const int32_t* tables, int table_stride, int num_seqs, const void* k_pool,
                   const void* v_pool, int page_size, int num_pages, int window, int chunk, float scale,
                   int v_dim, float softcap, const float* sinks, const float* dist_bias, int bias_rows,
-                  float* partial, int splits, void* stream);
+                  float* partial, int splits, int pairs, void* stream);
 
 // Cache write for attention without rotation.  qkv is [n, heads * head_dim + kv_heads *
 // (head_dim + v_dim)]: queries, keys, values.  q_every > 0: the queries of the token at

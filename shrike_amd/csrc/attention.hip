@@ -129,7 +129,7 @@ extern "C" int shk_attention(const void* q, int q_stride, void* out, int dtype, 
                              int num_seqs, const void* k_pool, const void* v_pool, int page_size,
                              int num_pages, int window, int chunk, float scale, int v_dim, float softcap,
                              const float* sinks, const float* dist_bias, int bias_rows, float* partial, int splits,
-                             void* stream) {
+                             int pairs, void* stream) {
   SHK_REQUIRE(dtype == kF32 || dtype == kBF16, "attention: unknown dtype %d", dtype);
   SHK_REQUIRE(!dist_bias || bias_rows > 0, "attention: a distance bias needs a table of at least one row");
   SHK_REQUIRE(n >= 0 && heads > 0 && kv_heads > 0 && heads % kv_heads == 0,
@@ -158,7 +158,7 @@ extern "C" int shk_attention(const void* q, int q_stride, void* out, int dtype, 
                    dist_bias, static_cast<float*>(out), partial, positions, token_seq, tables, q_stride, heads, kv_heads,
                    head_dim, v_dim, table_stride, page_size, num_pages, window, chunk, bias_rows, static_cast<int>(blocks),
                    scale, softcap},
-                  n, partial ? splits : 1, s);
+                  n, partial ? splits : 1, pairs, s);
   } else if (dtype == kF32)
     attention_generic_kernel<float><<<grid, kAttnThreads, 0, s>>>(
         static_cast<const float*>(q), q_stride, static_cast<float*>(out), heads, kv_heads, head_dim, v_dim,

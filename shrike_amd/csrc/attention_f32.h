@@ -17,6 +17,7 @@ struct F32Attention {
 };
 
 bool attention_f32_takes(int head_dim, int v_dim, int page_size, const void* k_pool, const void* v_pool);
-void attention_f32(const F32Attention& p, int n, int splits, hipStream_t s);
+// pairs: shk_attention's
+void attention_f32(const F32Attention& p, int n, int splits, int pairs, hipStream_t s);
 
 }  // namespace shk

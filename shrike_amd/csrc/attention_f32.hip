@@ -320,7 +320,7 @@ bool attention_f32_takes(int head_dim, int v_dim, int page_size, const void* k_p
 }
 
 template <int D>
-static void launch(const F32Attention& p, int n, int splits, hipStream_t s) {
+static void launch(const F32Attention& p, int n, int splits, int pairs, hipStream_t s) {
   const int per = p.heads / p.kv_heads;
   const dim3 grid(p.kv_heads * ((per + 15) / 16), n, splits);
   if (splits > 1) {
@@ -331,27 +331,31 @@ static void launch(const F32Attention& p, int n, int splits, hipStream_t s) {
     // compute unit) or three times (128: one does), else two tokens' chain of work is the longer one.  14 heads of 64 over 2,
     // at 165 / 200 / 509 / 2,000 tokens 11.3 / 14.1 / 37.7 / 366 us by themselves, 12.3 / 12.8 / 24.4 / 198 in pairs, 28 of 128 over 4 at
     // 130 / 200 / 509 / 2,000 31.6 / 38.8 / 114 / 1,237 and 35.1 / 36.6 / 98.8 / 955.  (Heads of more than 128 fill the registers.)
+    // A token without a neighbour is the slower in that kernel, and so are heads of more than 96 over few keys (whole steps of
+    // them: f32_pairs() in parts/attention.py), which only the caller knows of.
     constexpr bool kPairs = D <= 8;
-    const auto kernel = per <= 8 && p.kv_heads * n > (D <= 6 ? 384 : 768) ? attention_f32_kernel<D, false, kPairs> : attention_f32_kernel<D, false, false>;
+    const bool wanted = pairs > 0 || (pairs < 0 && D <= 6);
+    const auto kernel = wanted && per <= 8 && p.kv_heads * n > (D <= 6 ? 384 : 768) ? attention_f32_kernel<D, false, kPairs>
+                                                                                    : attention_f32_kernel<D, false, false>;
     kernel<<<grid, kWave * kBlockWaves, 0, s>>>(p, n);
   }
 }
 
-void attention_f32(const F32Attention& p, int n, int splits, hipStream_t s) {
+void attention_f32(const F32Attention& p, int n, int splits, int pairs, hipStream_t s) {
   const int d = p.head_dim > p.v_dim ? p.head_dim : p.v_dim;
   // (heads of 40 in the kernel for 64, of 96 in that for 128: 500 tokens 34.7 us and 35.0 instead of 29.8 and 28.9)
   if (d <= 32)
-    launch<2>(p, n, splits, s);
+    launch<2>(p, n, splits, pairs, s);
   else if (d <= 48)
-    launch<3>(p, n, splits, s);
+    launch<3>(p, n, splits, pairs, s);
   else if (d <= 64)
-    launch<4>(p, n, splits, s);
+    launch<4>(p, n, splits, pairs, s);
   else if (d <= 96)
-    launch<6>(p, n, splits, s);
+    launch<6>(p, n, splits, pairs, s);
   else if (d <= 128)
-    launch<8>(p, n, splits, s);
+    launch<8>(p, n, splits, pairs, s);
   else
-    launch<16>(p, n, splits, s);
+    launch<16>(p, n, splits, pairs, s);
 }
 
 }  // namespace shk

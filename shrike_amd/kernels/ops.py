@@ -726,10 +726,12 @@ def rope_kv_store(qkv, heads, kv_heads, head_dim, rot_dim, inv_freq, positions, 
 
 def attention(q, out, heads, kv_heads, head_dim, positions, token_seq, tables, k_pool, v_pool,
               page_size, window, scale, chunk=None, v_dim=None, softcap=None, sinks=None, dist_bias=None, partial=None,
-              splits=1) -> None:
+              splits=1, pairs=None) -> None:
     """q: [n, >= heads*head_dim] rows (a view into qkv is fine); out [n, heads*v_dim].
     partial: float32 scratch of attention_partial_floats() with which float32 attention may form a token's
     blocks of 256 keys in up to `splits` workgroups (the same bits).
+    pairs: whether two neighbouring tokens of a sequence share a workgroup of float32 attention where sizes allow it (the
+    same bits; None: for heads of up to 96).
     v_dim: size of a value (None: head_dim); softcap: scores become cap * tanh(score / cap);
     sinks: float32 [heads], one more term exp(sinks[h]) in each head's softmax denominator;
     dist_bias: float32 [heads, rows], dist_bias[h, min(i - j, rows - 1)] joins the (capped) score."""
@@ -754,7 +756,8 @@ def attention(q, out, heads, kv_heads, head_dim, positions, token_seq, tables, k
             float(softcap or 0.0), None if sinks is None else _dev(sinks, "sinks", torch.float32),
             None if dist_bias is None else _dev(dist_bias, "dist_bias", torch.float32),
             0 if dist_bias is None else dist_bias.shape[1],
-            None if partial is None else _dev(partial, "partial", torch.float32), int(splits), _stream(),
+            None if partial is None else _dev(partial, "partial", torch.float32), int(splits),
+            -1 if pairs is None else int(bool(pairs)), _stream(),
         )
     )
 

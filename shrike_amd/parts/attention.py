@@ -113,6 +113,30 @@ def f32_split_floats(rows: int, heads: int, kv_heads: int, value_dim: int, keys:
     return 0 if blocks <= 1 or rows * kv_heads >= 2 * compute_units() or 4 * floats > F32_SPLIT_SCRATCH else floats
 
 
+def f32_pairs(num_decode: int, q_lens, starts, kv_heads: int, dim: int, reach: int) -> bool:
+    """Whether neighbouring tokens of a sequence share a workgroup of float32 attention in this step, which has to have enough
+    tokens for that (attention_f32.hip).  A token without a neighbour is the slower there: 256 single tokens at 900 keys 52 us by themselves and 57 in that
+    kernel (2 key/value heads of 64), 210 and 258 (4 of 128), so at most half of the step's tokens may be such, an eighth with heads of
+    more than 96.  Over few keys two tokens' chain of work outweighs what they share: 4 heads of 128 at 12 / 25 / 100 / 150 keys on
+    average 58.6 / 107 / 123 / 221 us by themselves, 68.9 / 122 / 127 / 204 in pairs; 2 of 64, 200 tokens at 12 / 100 keys 11.2 /
+    13.9 and 13.0 / 12.7, but 400 at 12 20.0 and 16.6."""
+    q_lens, starts = np.asarray(q_lens, dtype=np.int64), np.asarray(starts, dtype=np.int64)
+    n = int(q_lens.sum())
+    if kv_heads * n <= (384 if dim <= 96 else 768):
+        return False
+    ends = np.cumsum(q_lens)
+    # pairs are tokens 2 i and 2 i + 1 of the step
+    pairs = int((ends // 2 - (ends - q_lens + 1) // 2).sum())
+    if pairs == 0:
+        return False
+    portions, first = q_lens[num_decode:], starts[num_decode:]
+    keys = float((portions * np.minimum(first + (portions + 1) / 2, reach)).sum()) / max(1, int(portions.sum()))
+    alone = n - 2 * pairs
+    if dim <= 96:
+        return 2 * alone <= n and (kv_heads * n > 768 or keys >= 96)
+    return 8 * alone <= n and keys >= 128
+
+
 def decode_streams(num_seqs: int, kv_heads: int, head_dim: int, max_ctx: int, window: int | None = None) -> bool:
     """Whether a decode launch reads so many keys and values that non-temporal
     loads pay (measured with 4 key/value heads of 128: a tenth faster from 64
@@ -133,6 +157,7 @@ class AttentionPlan:
     nsplit: int = 1  # key splits of the single-token rows
     waves: int = 4  # wavefronts of their workgroups
     blocks_apart: bool = False  # float32: workgroups of their own for a single token's blocks of keys
+    pairs: bool = False  # float32: neighbouring tokens of a sequence share a workgroup
     streaming: bool = False  # single-token rows: non-temporal loads of keys and values
     kernel: str = ""  # for prompt portions: "shared", "tiles" or "" (none in the step)
     small: int = 0  # "shared" with half as many wavefronts per workgroup (1), with 32 rows a wavefront (2)
@@ -503,7 +528,9 @@ class PagedAttention(Mixer):
             # the general kernels take every token alike, but float32 single tokens of more than one block of keys
             # (a longer step's launches serve them side by side and join them: two kernels instead of one)
             plan.blocks_apart = self.dtype == torch.float32 and shape.max_decode_ctx > ops.ATTENTION_KEY_BLOCK
-            shape.launch_key.append((key, plan.blocks_apart))
+            plan.pairs = self.dtype == torch.float32 and f32_pairs(shape.num_decode, shape.q_lens, shape.starts, hkv,
+                                                                   max(d, self.value_dim), reach)
+            shape.launch_key.append((key, plan.blocks_apart, plan.pairs))
             return
         if shape.num_decode:
             plan.nsplit, plan.waves = decode_shares(shape.num_decode, hkv, d, min(shape.max_decode_ctx, reach))
@@ -574,7 +601,7 @@ class PagedAttention(Mixer):
             ops.attention(q, out, h, hkv, d, ctx.positions, ctx.token_seq, tables, cache.pools["k"],
                           cache.pools["v"], cache.page_size, s.window, s.scale, chunk=s.chunk,
                           v_dim=self.value_dim, softcap=getattr(s, "softcap", None), sinks=self.sinks,
-                          dist_bias=self.dist_bias, partial=partial, splits=splits)
+                          dist_bias=self.dist_bias, partial=partial, splits=splits, pairs=plan.pairs)
             return
         if ctx.num_decode:
             partial = ctx.buffer("attn_partial", (ctx.num_decode * h * plan.nsplit * (d + 2),),
