@@ -439,7 +439,9 @@ long long shk_selective_scan_state_floats(int inner, int states, int taps);
 int shk_short_conv(const void* x, int ldx, const float* taps, const float* bias, int num_taps, int inner,
                    const int32_t* positions, const int32_t* token_seq, const int32_t* cu_q,
                    const int32_t* slots, const float* state, long long slot_stride, int states, int silu, void* y,
-                   int dtype, int n, void* stream);
+                   int dtype, int n, int num_seqs, void* stream);
+// whether tokens of num_seqs sequences move through it as vectors (bfloat16, four taps, aligned rows; the same bits)
+int shk_short_conv_in_vectors(int n, int inner, int num_seqs);
 int shk_dt_softplus(const float* low, int ld, const float* w, const float* b, int rank, int inner,
                     float sign, float mult, float* dt, int n, void* stream);
 int shk_selective_scan(const float* dt, const void* x, const float* bc, int ld_bc, int b_off, int c_off,

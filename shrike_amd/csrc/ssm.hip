@@ -91,6 +91,16 @@ constexpr int kConvTokens = 8, kConvThreads = 64;
 // Results from which on it is taken: 3,584 channels at 128 / 256 / 512 tokens 4.2 / 6.6 / 10.9 us above and 6.6 / 7.0 / 7.2 here, 896 at 512 /
 // 1,024 / 2,048 4.6 / 7.1 / 12.1 and 6.7 / 7.0 / 7.5.
 constexpr long long kConvMinResults = 1 << 20;
+// A sequence's first three tokens take inputs from its slot, one token after the other: sequences have to be so long on average.
+// Above and here, sequences of 1 / 2 / 3 / 4 / 5 / 8 / 24 tokens: 600 tokens of 3,584 channels 14.0 / 13.7 / 13.6 / 12.6 / 12.8 / 12.3 / 12.1 us
+// and 20.4 / 16.9 / 15.5 / 13.0 / 11.7 / 10.4 / 9.7, 2,048 of 896 13.8 / 13.3 / 12.4 / 11.9 / 11.7 / 11.8 / 12.0 and 17.7 / 15.0 / 13.3 /
+// 12.0 / 10.9 / 9.6 / 8.5; 600 of 2,048 7.5 / 7.5 / 7.7 / 7.9 / 7.8 / 7.9 / 7.9 and 15.9 / 13.8 / 12.4 / 11.4 / 10.4 / 9.3 / 8.3; 2,048 of 2,048
+// 26.4 / 26.5 / 24.2 and 26.7 / 24.0 / 19.9, of 3,584 43.4 / 44.3 / 44.9 and 44.2 / 37.9 / 32.4.
+static bool conv_in_vectors(int n, int inner, int num_seqs) {
+  const long long results = static_cast<long long>(n) * inner;
+  const int least = results < 3 << 19 ? 64 : results < 1 << 22 ? 5 : 2;
+  return results >= kConvMinResults && n >= static_cast<long long>(least) * num_seqs;
+}
 
 __global__ void __launch_bounds__(kConvThreads)
     short_conv_rows_kernel(const bf16* __restrict__ x, int ldx, const float* __restrict__ taps, const float* __restrict__ bias, int inner,
@@ -460,12 +470,14 @@ extern "C" long long shk_selective_scan_state_floats(int inner, int states, int 
   return static_cast<long long>(inner) * states + static_cast<long long>(taps > 1 ? taps - 1 : 0) * inner;
 }
 
+extern "C" int shk_short_conv_in_vectors(int n, int inner, int num_seqs) { return conv_in_vectors(n, inner, num_seqs); }
+
 extern "C" int shk_short_conv(const void* x, int ldx, const float* taps, const float* bias, int num_taps, int inner,
                              const int32_t* positions, const int32_t* token_seq, const int32_t* cu_q,
                              const int32_t* slots, const float* state, long long slot_stride, int states, int silu,
-                              void* y, int dtype, int n, void* stream) {
+                              void* y, int dtype, int n, int num_seqs, void* stream) {
   SHK_REQUIRE(dtype == kF32 || dtype == kBF16, "short_conv: unknown dtype %d", dtype);
-  SHK_REQUIRE(n >= 0 && inner > 0 && num_taps >= 1 && num_taps <= 64 && ldx >= inner && states > 0,
+  SHK_REQUIRE(n >= 0 && inner > 0 && num_seqs >= 0 && num_taps >= 1 && num_taps <= 64 && ldx >= inner && states > 0,
               "short_conv: bad sizes n=%d inner=%d taps=%d", n, inner, num_taps);
   SHK_REQUIRE(slot_stride >= shk_selective_scan_state_floats(inner, states, num_taps),
               "short_conv: a slot of %lld floats does not hold the state", slot_stride);
@@ -476,7 +488,8 @@ extern "C" int shk_short_conv(const void* x, int ldx, const float* taps, const f
   dim3 grid((inner + 255) / 256, n);
   const long long tail_off = static_cast<long long>(inner) * states;
   const auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
-  if (dtype == kBF16 && num_taps == 4 && static_cast<long long>(n) * inner >= kConvMinResults && inner % 8 == 0 && ldx % 8 == 0 && aligned(x) && aligned(y) && aligned(taps)) {
+  if (dtype == kBF16 && num_taps == 4 && conv_in_vectors(n, inner, num_seqs) && inner % 8 == 0 && ldx % 8 == 0 && aligned(x) && aligned(y) &&
+      aligned(taps)) {
     short_conv_rows_kernel<<<dim3((inner + 8 * kConvThreads - 1) / (8 * kConvThreads), (n + kConvTokens - 1) / kConvTokens), kConvThreads, 0, s>>>(
         static_cast<const bf16*>(x), ldx, taps, bias, inner, positions, token_seq, cu_q, slots, state, slot_stride, tail_off,
         static_cast<bf16*>(y), silu, n);

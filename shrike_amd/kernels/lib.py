@@ -84,7 +84,8 @@ _SIGNATURES = {
                               _P, _I, _F, _P, _I, _P],
     "shk_attention_talking_bf16": [_P, _I, _P, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _I, _P, _P, _I, _I, _I,
                                    _I, _F, _P, _P, _P, _I, _F, _P, _I, _P],
-    "shk_short_conv": [_P, _I, _P, _P, _I, _I, _P, _P, _P, _P, _P, c_longlong, _I, _I, _P, _I, _I, _P],
+    "shk_short_conv": [_P, _I, _P, _P, _I, _I, _P, _P, _P, _P, _P, c_longlong, _I, _I, _P, _I, _I, _I, _P],
+    "shk_short_conv_in_vectors": [_I, _I, _I],
     "shk_dt_softplus": [_P, _I, _P, _P, _I, _I, _F, _F, _P, _I, _P],
     "shk_selective_scan": [_P, _P, _P, _I, _I, _I, _P, _I, _P, _P, _I, _I, _I, _P, _I, _P, _P, _P, _P, c_longlong,
                            _P, _I, _I, _P],

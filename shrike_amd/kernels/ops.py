@@ -1217,7 +1217,12 @@ def short_conv(x, taps, bias, positions, token_seq, cu_q, slots, state, states: 
                                _dev(positions, "positions", torch.int32), _dev(token_seq, "token_seq", torch.int32),
                                _dev(cu_q, "cu_q", torch.int32), _dev(slots, "slots", torch.int32), _dev(state, "state"),
                                state.stride(0), states, int(activation == "silu"), _dev(y, "y"), dtype_code(y.dtype), n,
-                                _stream()))
+                               cu_q.shape[0] - 1, _stream()))
+
+
+def short_conv_in_vectors(n: int, inner: int, num_seqs: int) -> bool:
+    """Whether short_conv() of n bfloat16 tokens of num_seqs sequences moves aligned rows as vectors (the same bits)."""
+    return bool(load().shk_short_conv_in_vectors(n, inner, num_seqs))
 
 
 def dt_softplus(low, w, b, dt, sign: float = 1.0, mult: float = 1.0) -> None:
