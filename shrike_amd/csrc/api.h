@@ -104,6 +104,8 @@ int shk_gemm(const void* a, const void* w, const float* bias, void* out, int n, 
 int shk_retile_f32(const void* w, int m, int k, void* wt, void* stream);
 int shk_gemm_f32_tiled_weight(const void* a, const void* wt, const float* bias, void* out, int n, int m, int k, int lda,
                               int ldo, int accumulate, void* stream);
+// whether it asks for all of a wavefront's k at once (up to 16 aligned rows; the same bits)
+int shk_gemm_f32_few(int n, int m, int k);
 
 // The same bits, rows 16-byte aligned, k a multiple of 16; of more than 16 rows k a multiple of 32, at least 288 (groups 768), the
 // matrix less than 2^30 elements, lda up to 2^20.  shk_gemm_f32_groups: out [4][n][m] receives the sum's four

@@ -238,7 +238,7 @@ __global__ void __launch_bounds__(kWave * KW * MW * NW)
 // forms a block of both and stores what act_mul_kernel would of the two.
 // What bounds it: one round trip to memory and what a compute unit takes in (about 50 GB/s a workgroup).  Weights cold, us at 1 /
 // 4 / 16 rows: 896 x 896 4.8 / 5.0 / 6.4 in the kernel above, 3.7 / 3.8 / 4.9 here, 9728 x 896 11.1 / 10.5 / 13.0 and 8.6 / 8.7 / 11.4,
-// 3584 x 3584 28 / 29 / 39 and 12 / 12 / 15; 896 x 4864 13.0 / 13.3 / 18.8 and, in one workgroup a half block, 11.4 / 11.8 / 18.2.
+// 3584 x 3584 28 / 29 / 39 and 12 / 12 / 15.
 template <int KW, int ROWS, int C, bool GATED, bool GROUPS>
 __global__ void __launch_bounds__(kWave* KW)
     gemm_f32_few_kernel(const float* __restrict__ a, const float* __restrict__ w, const float* __restrict__ bias,
@@ -531,19 +531,28 @@ static void launch_f32_lds(const F32Product& p, hipStream_t s, F32Gate gate = F3
                                                                         vec_out, gate);
 }
 
-// Whether gemm_f32_few_kernel takes a product of tiled weights.  (151936 x 896: 98 / 107 us at 4 / 16 rows in gemm_f32_kernel's
-// two blocks a wavefront, 90 / 121 here.)
-static bool f32_few(const F32Product& p) {
-  return p.n <= 16 && (p.m <= 32768 || p.n <= 8) && p.k % 16 == 0 && p.lda % 4 == 0 && reinterpret_cast<uintptr_t>(p.a) % 16 == 0;
+// Sizes for which gemm_f32_few_kernel is the faster one.  Weights cold, gemm_f32_kernel and it, us at 1 / 8 / 16 rows: half blocks and
+// segments as long as a wavefront holds its steps (2048 x 2048 7.7 / 8.6 / 10.3 and 7.0 / 7.1 / 8.8, x 4096 11.7 / 12.3 / 14.7 and 14.9 / 16.6 /
+// 19.6); up to 8,192 features (8192 x 4096 32.5 / 33.4 / 42.0 and 26.5 / 27.3 / 32.2); with more of them whole blocks of a long k are a part of
+// a second round (11008 x 2048 19.0 / 19.7 / 23.7 and 21.4 / 23.5 / 28.0, 32000 x 2048 40.7 / 40.2 / 43.9 and 52.3 / 60.0 / 71.4; x 1024 11.8 /
+// 12.3 / 14.5 and 9.6 / 10.4 / 12.3), and with still more the kernel above has rounds enough (16384 x 512 8.9 / 9.1 / 10.3 and 8.9 / 9.2 / 10.3,
+// x 896 12.8 / 13.0 / 14.4 and 12.2 / 12.4 / 15.8, 50000 x 256 12.6 / 12.7 / 13.7 and 18.7 / 20.8 / -, x 1024 35.6 / 35.8 / 36.1 and 32.1 /
+// 34.2 / -; 151936 x 896 98 / - / 107 and 90 / - / 121).
+static bool f32_few(int n, int m, int k) {
+  if (n > 16 || k % 16) return false;
+  if (m <= 2048) return k <= 2560;
+  if (m <= 8192) return true;
+  if (m <= 12288) return k <= 1024;
+  return n <= 8 && k >= 896 && k <= 1024;
 }
 
-// fn with the steps of a wavefront rounded up to one of a few constants, 0 for more than MOST.
-template <int MOST, typename Fn>
+// fn with the steps of a wavefront rounded up to one of a few constants, 0 for more than ten.
+template <typename Fn>
 static void with_steps(int steps, Fn fn) {
   if (steps <= 2) fn(std::integral_constant<int, 2>{});
   else if (steps <= 4) fn(std::integral_constant<int, 4>{});
   else if (steps <= 6) fn(std::integral_constant<int, 6>{});
-  else if (steps <= MOST) fn(std::integral_constant<int, MOST>{});
+  else if (steps <= 10) fn(std::integral_constant<int, 10>{});
   else fn(std::integral_constant<int, 0>{});
 }
 
@@ -554,17 +563,22 @@ static void launch_f32_few(const F32Product& p, hipStream_t s) {
   const auto go = [&](auto kernel, int waves, int rows) {
     kernel<<<(p.m + rows - 1) / rows, waves * kWave, 0, s>>>(p.a, p.w, p.bias, p.out, p.n, p.m, p.k, p.lda, p.ldo, p.accumulate, F32Gate{});
   };
-  if (p.m <= 2048)
-    with_steps<10>(seg_steps, [&](auto c) { go(gemm_f32_few_kernel<16, 8, c.value, false, false>, 16, 8); });
-  else if (p.k <= 1024)
-    with_steps<10>(seg_steps, [&](auto c) { go(gemm_f32_few_kernel<16, 16, c.value, false, false>, 16, 16); });
+  if (p.m <= 2048)  // (a k of up to 2,560: ten steps)
+    go(seg_steps <= 2   ? gemm_f32_few_kernel<16, 8, 2, false, false>
+       : seg_steps <= 4 ? gemm_f32_few_kernel<16, 8, 4, false, false>
+       : seg_steps <= 6 ? gemm_f32_few_kernel<16, 8, 6, false, false>
+                        : gemm_f32_few_kernel<16, 8, 10, false, false>,
+       16, 8);
+  else if (p.k <= 1024)  // (four steps)
+    go(seg_steps <= 2 ? gemm_f32_few_kernel<16, 16, 2, false, false> : gemm_f32_few_kernel<16, 16, 4, false, false>, 16, 16);
   else
-    with_steps<16>(4 * seg_steps, [&](auto c) { go(gemm_f32_few_kernel<4, 16, c.value, false, false>, 4, 16); });
+    go(gemm_f32_few_kernel<4, 16, 0, false, false>, 4, 16);
 }
 
 // The shape of the kernel for a size (results are the same bits in all of them).  Measured on the 0.5B
 // model's matrices, tiled weights, microseconds:
-//   up to 16 rows: 896 x 896 5 in one-tile workgroups of 16 segments (9 with four row blocks and four groups of
+//   up to 16 rows (what f32_few() leaves; 896 x 896 and 9728 x 896 are here for rows that are not aligned, or a k that is no multiple of
+//     16): 896 x 896 5 in one-tile workgroups of 16 segments (9 with four row blocks and four groups of
 //     k), 896 x 4864 13 (37); 9728 x 896 10.7 with four row blocks (12), 151936 x 896 98 with eight (113);
 //   more: the largest tile that still leaves the 256 compute units evenly loaded.  896 x 896 at 64 / 128 / 509 /
 //     1024 rows 5.7 / 7.3 / 17 / 26 (16 x 16, 32 x 16, 32 x 64, 64 x 64), 9728 x 896 at 64 / 509 25 / 124
@@ -586,7 +600,8 @@ static void run_f32(const F32Product& p, hipStream_t s) {
   // whole stages of aligned rows, offsets within a tile of 32 bits
   const bool staged = TILED && p.batch == 1 && p.k % 32 == 0 && p.k > 256 && p.k <= 1 << 20 && p.lda % 4 == 0 && p.lda <= 1 << 20 &&
                       reinterpret_cast<uintptr_t>(p.a) % 16 == 0;
-  if (TILED && f32_few(p)) {
+  const bool few = TILED && f32_few(p.n, p.m, p.k) && p.lda % 4 == 0 && reinterpret_cast<uintptr_t>(p.a) % 16 == 0;
+  if (few) {
     launch_f32_few(p, s);
   } else if (p.n <= 16) {
     if (p.m <= 2048)
@@ -683,7 +698,7 @@ extern "C" int shk_gemm_f32_groups(const void* a, const void* wt, void* out, int
   const F32Product p{static_cast<const float*>(a), static_cast<const float*>(wt), nullptr, static_cast<float*>(out), n, m, k, lda, m, 0, 1, 0, 0, 0};
   const hipStream_t s = static_cast<hipStream_t>(stream);
   if (n <= 16)
-    with_steps<10>((k + 16 * kF32Segments - 1) / (16 * kF32Segments), [&](auto c) {
+    with_steps((k + 16 * kF32Segments - 1) / (16 * kF32Segments), [&](auto c) {
       gemm_f32_few_kernel<4, 8, c.value, false, true><<<dim3((m + 7) / 8, kF32Segments / kF32Group), 4 * kWave, 0, s>>>(
           p.a, p.w, nullptr, p.out, n, m, k, lda, m, 0, F32Gate{});
     });
@@ -726,10 +741,12 @@ extern "C" int shk_gemm_f32_gated(const void* a, const void* wt, void* out, int 
   if (k <= 1024)  // (up to four steps a segment)
     go(seg_steps <= 2 ? gemm_f32_few_kernel<16, 16, 2, true, false> : gemm_f32_few_kernel<16, 16, 4, true, false>, 16);
   else
-    with_steps<16>(4 * seg_steps, [&](auto c) { go(gemm_f32_few_kernel<4, 16, c.value, true, false>, 4); });
+    go(gemm_f32_few_kernel<4, 16, 0, true, false>, 4);
   SHK_LAUNCH_CHECK("gemm_f32_gated");
   return 0;
 }
+
+extern "C" int shk_gemm_f32_few(int n, int m, int k) { return f32_few(n, m, k); }
 
 extern "C" int shk_gemm_f32_tiled_weight(const void* a, const void* wt, const float* bias, void* out, int n, int m, int k,
                                          int lda, int ldo, int accumulate, void* stream) {

@@ -372,6 +372,11 @@ def gemm_f32_tiled_weight(a, wt, m: int, k: int, out, bias=None, accumulate=Fals
         a.stride(0), out.stride(0), int(bool(accumulate)), _stream()))
 
 
+def gemm_f32_few(n: int, m: int, k: int) -> bool:
+    """Whether gemm_f32_tiled_weight of n aligned rows and an [m, k] matrix runs in the kernel for few of them (the same bits)."""
+    return bool(load().shk_gemm_f32_few(n, m, k))
+
+
 def gemm_f32_splits(n: int, m: int, k: int) -> int:
     """Parts in which gemm_f32_groups leaves an [n, k] x [m, k]^T product (1: it is better formed whole)."""
     return int(load().shk_gemm_f32_splits(n, m, k))
