@@ -115,6 +115,7 @@ int shk_gemm_f32_few(int n, int m, int k);
 int shk_gemm_f32_splits(int n, int m, int k);
 int shk_gemm_f32_groups(const void* a, const void* wt, void* out, int n, int m, int k, int lda, void* stream);
 int shk_gemm_f32_gated_takes(int n, int m, int k);
+int shk_gemm_f32_gated_faster(int n, int m, int k);  // than the product and shk_act_mul
 int shk_gemm_f32_gated(const void* a, const void* wt, void* out, int n, int m, int k, int lda, int act, float limit,
                        float up_shift, void* stream);
 

@@ -708,12 +708,30 @@ extern "C" int shk_gemm_f32_groups(const void* a, const void* wt, void* out, int
   return 0;
 }
 
-// Whether shk_gemm_f32_gated takes a product of 2 m features, gate and other factor.  Product and gate against it, more than 16
-// rows: 4864 x 896 at 17 / 64 / 128 / 509 / 2,000 16.5 / 20.6 / 29.5 / 88.1 / 356 -> 14.2 / 17.8 / 26.9 / 83.2 / 346 us, 8960 x 1536 at
-// 17 / 509 49.6 / 250 -> 30.7 / 247, 512 x 288 6.2 / 9.3 -> 5.4 / 7.0.
+// Whether shk_gemm_f32_gated takes a product of 2 m features, gate and other factor.
 extern "C" int shk_gemm_f32_gated_takes(int n, int m, int k) {
   return m > 0 && m % 16 == 0 && k > 0 && k % 16 == 0 && (n <= 16 || f32_staged(m, k, k));
 }
+
+// Whether it is faster than product and gate in two kernels.  Weights cold, us, two kernels -> one.
+// Up to 16 rows, at 1 / 16: a k of up to 1,024 (segments a wavefront) always, 4864 x 896 13.0 / 15.7 -> 11.3 / 13.5, 256 x 896 6.3 / 7.8 -> 5.4 /
+// 7.1.  A longer one is walked in four groups, by one workgroup a compute unit: up to 1,024 features the product alone has half blocks and
+// sixteen segments (768 x 2048 9.0 / 10.5 -> 12.1 / 14.2), up to 4,096 it has not (1040 x 2048 19.9 / 24.7 -> 12.7 / 14.5, 4096 x 2048 21.0 /
+// 25.8 -> 15.9 / 18.6); from there on whole blocks are a part of a second round (4480 x 2048 21.0 / 25.6 -> 24.0 / 28.6, 8192 x 2048 24.8 / 26.6 ->
+// 28.3 / 31.8) until it is the product that begins its second (8448 x 2048 38.3 / 45.1 -> 33.9 / 41.8, 11008 x 4096 80.5 / 95.9 -> 66.7 / 77.2;
+// 12288 x 2048 39.0 / 45.5 -> 40.8 / 46.2, 13056 x 2048 39.4 / 46.0 -> 48.4 / 55.8).
+// More rows, whose k one workgroup walks whole where the product shares it among wavefronts: as many workgroups of 32 rows as compute
+// units, unless k is shorter.  4864 x 896 at 17 / 64 / 128 / 509 / 2,000 16.5 / 20.6 / 29.5 / 88.1 / 356 -> 14.2 / 17.8 / 26.9 / 83.2 / 346, 8960 x 1536
+// at 17 / 509 49.6 / 250 -> 30.7 / 247, 512 x 288 6.2 / 9.3 -> 5.4 / 7.0; 768 x 2048 at 17 / 128 10.8 / 16.7 -> 18.6 / 19.2, at 256 28.1 -> 26.4;
+// 2816 x 2048 at 17 / 33 17.3 / 31.0 -> 19.5 / 26.8; 256 x 512 at 17 8.1 -> 7.7, 768 x 896 at 128 11.3 -> 10.5, at 65 9.7 -> 10.6.
+static bool f32_gated_faster(int n, int m, int k) {
+  if (!shk_gemm_f32_gated_takes(n, m, k)) return false;
+  if (n <= 16) return k <= 1024 || (m > 1024 && m <= 4096) || (m > 8192 && m <= 11264);
+  const long long groups = m / 16 * ((n + 31LL) / 32);
+  return k <= 512 || groups > 256 || (k <= 896 && groups >= 176);
+}
+
+extern "C" int shk_gemm_f32_gated_faster(int n, int m, int k) { return f32_gated_faster(n, m, k); }
 
 extern "C" int shk_gemm_f32_gated(const void* a, const void* wt, void* out, int n, int m, int k, int lda, int act, float limit,
                                   float up_shift, void* stream) {
@@ -727,7 +745,11 @@ extern "C" int shk_gemm_f32_gated(const void* a, const void* wt, void* out, int 
   const F32Gate gate = {act, limit, up_shift};
   if (n > 16) {
     const F32Product p{static_cast<const float*>(a), static_cast<const float*>(wt), nullptr, static_cast<float*>(out), n, m, k, lda, m, 0, 1, 0, 0, 0};
-    if (m / 16 * ((n + 63LL) / 64) >= 1536)  // (as for the product whole)
+    const long long tiles = m / 16 * ((n + 63LL) / 64);
+    // (as for the product whole, but for a long k only where the last round of two workgroups a compute unit is at least half full: 32 and 64
+    // rows a workgroup, 1536 x 4096 at 512 rows (768 tiles of 64) 122 and 116 us, 14336 x 2048 at 64 (896) 78 and 70, 4864 x 2048 at 128 (608)
+    // 52 and 57, 8960 x 2048 at 64 (560) 51 and 57)
+    if (tiles >= 1536 || (k > 1024 && n > 32 && tiles >= 440 && (tiles + 256) % 512 <= 256))
       launch_f32_lds<1, 2, true>(p, static_cast<hipStream_t>(stream), gate);
     else
       launch_f32_lds<1, 1, true>(p, static_cast<hipStream_t>(stream), gate);

@@ -68,7 +68,7 @@ class Runtime:
             ops.gemm_tiled_weight(x, w.tiled, w.rows, w.cols, out, gated=activation, gate_args=w.gate_args)
             return
         inter = w.rows // 2
-        if ops.gemm_f32_gated_takes(x.shape[0], inter, w.cols) and ops.f32_rows_aligned(x) and out.is_contiguous():
+        if ops.gemm_f32_gated_faster(x.shape[0], inter, w.cols) and ops.f32_rows_aligned(x) and out.is_contiguous():
             ops.gemm_f32_gated(x, w.tiled_f32, inter, w.cols, out, activation, limit, up_shift)
             return
         gate_up = ctx.buffer("ffn_gate_up", (x.shape[0], w.rows), self.dtype)

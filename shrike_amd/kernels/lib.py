@@ -46,6 +46,7 @@ _SIGNATURES = {
     "shk_gemm_f32_splits": [_I, _I, _I],
     "shk_gemm_f32_groups": [_P, _P, _P, _I, _I, _I, _I, _P],
     "shk_gemm_f32_gated_takes": [_I, _I, _I],
+    "shk_gemm_f32_gated_faster": [_I, _I, _I],
     "shk_gemm_f32_gated": [_P, _P, _P, _I, _I, _I, _I, _I, _F, _F, _P],
     "shk_retile_weight": [_P, _I, _I, _P, _P],
     "shk_interleave_gate_up": [_P, _P, _I, _I, _P, _P],

@@ -387,6 +387,11 @@ def gemm_f32_gated_takes(n: int, m: int, k: int) -> bool:
     return bool(load().shk_gemm_f32_gated_takes(n, m, k))
 
 
+def gemm_f32_gated_faster(n: int, m: int, k: int) -> bool:
+    """Whether gemm_f32_gated takes n rows and two [m, k] matrices, and sooner than a product and act_mul()."""
+    return bool(load().shk_gemm_f32_gated_faster(n, m, k))
+
+
 def f32_rows_aligned(x) -> bool:
     """Whether the rows of a float32 matrix begin at multiples of 16 bytes, not too far apart for gemm_f32_groups and _gated."""
     return x.data_ptr() % 16 == 0 and x.stride(0) % 4 == 0 and x.stride(0) <= 1 << 20
