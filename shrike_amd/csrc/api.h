@@ -109,10 +109,11 @@ int shk_gemm_f32_few(int n, int m, int k);
 
 // The same bits, rows 16-byte aligned, k a multiple of 16; of more than 16 rows k a multiple of 32, at least 288 (groups 768), the
 // matrix less than 2^30 elements, lda up to 2^20.  shk_gemm_f32_groups: out [4][n][m] receives the sum's four
-// groups, whose sum in order is the product (shk_add_rmsnorm adds them); shk_gemm_f32_splits: 4 where that is worth it, else 1.
+// groups, whose sum in order is the product (shk_add_rmsnorm adds them); shk_gemm_f32_splits: 4 for a long k and few workgroups, else 1.
 // shk_gemm_f32_gated: out[n, m] = act(g) * (u + up_shift) of the product [g | u] with 2 m features, as shk_act_mul forms it
 // (m a multiple of 16).
 int shk_gemm_f32_splits(int n, int m, int k);
+int shk_gemm_f32_groups_faster(int n, int m, int k);  // with the norm that adds them, than the product whole and the norm
 int shk_gemm_f32_groups(const void* a, const void* wt, void* out, int n, int m, int k, int lda, void* stream);
 int shk_gemm_f32_gated_takes(int n, int m, int k);
 int shk_gemm_f32_gated_faster(int n, int m, int k);  // than the product and shk_act_mul

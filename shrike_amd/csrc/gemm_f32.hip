@@ -677,16 +677,27 @@ static bool f32_staged(int m, int k, int lda) {
   return k % 32 == 0 && k > 256 && lda <= 1 << 20 && static_cast<long long>(m) * k < 1LL << 30;
 }
 
-// Groups in which shk_gemm_f32_groups leaves a product for its reader (1: it is formed whole): four where a long k would
-// be walked in few workgroups: with the norm that adds its output 896 x 4864 at 1 / 4 / 16 rows 13.7 / 14.1 / 20.7 us whole, 10.0 /
-// 10.2 / 13.2 in groups, 1536 x 8960 22.4 / 22.9 / 34.5 and 18.9 / 19.5 / 27.7.  The same of more rows: 896 x 4864 at 33 / 64 / 128 / 509 /
-// 1,024 / 2,000 rows 19.5 / 21.1 / 27.6 / 56.4 / 92.3 / 170 and 20.3 / 20.2 / 20.7 / 48.6 / 85.2 / 174, 1536 x 8960 at 64 / 509 / 700 /
-// 1,024 44 / 174 / 222 / 239 and 32 / 126 / 176 / 244: up to 640 workgroups a group.  A short k gains nothing: 512 x 2048 at 64 / 320
-// rows 11.2 / 16.8 and 11.9 / 16.8.
+// Groups in which shk_gemm_f32_groups may leave a product for its reader (1: only whole): four where a long k would be walked in few
+// workgroups.
 extern "C" int shk_gemm_f32_splits(int n, int m, int k) {
   const long long tiles = (m + 31LL) / 32 * ((n + 63) / 64);
   const bool few = n <= 16 && m <= 2048 && k >= 2048 && k % 16 == 0, more = n >= 64 && k >= 4096 && tiles <= 640 && f32_staged(m, k, k);
   return m % 4 == 0 && (few || more) ? kF32Segments / kF32Group : 1;
+}
+
+// Whether the groups and a norm that adds them are faster than the product whole and the norm.  Weights cold, us, whole -> in groups.
+// Up to 16 rows, at 1 / 8 / 16: 896 x 4864 14.8 / 16.1 / 18.3 -> 11.4 / 12.0 / 13.9, 1024 x 16384 34.7 / 36.3 / 42.6 -> 24.0 / 24.7 / 31.6; with more features the
+// product has workgroups enough but for steps that its wavefronts hold at once: 1536 x 2560 9.5 / 9.9 / 12.0 -> 9.1 / 9.4 / 11.0, x 2576 11.3 / 12.0 /
+// 12.5 -> 13.0 / 13.8 / 16.9, x 8960 23.3 / 24.6 / 28.0 -> 22.6 / 24.9 / 29.1, 2048 x 2048 9.9 / 10.2 / 11.9 -> 10.2 / 10.6 / 12.4, x 5632 17.2 / 18.2 /
+// 21.0 -> 21.7 / 22.3 / 29.1 (1024 x 2576 10.9 / 11.6 / 12.0 -> 10.4 / 10.9 / 13.0).
+// More rows, at 64 / 100 / 256 / 512 / 1,000 / 2,000: 896 x 4864 19.3 / 27.2 / 33.5 / 58.4 / 97 / 179 -> 20.2 / 20.9 / 30.7 / 49.5 / 83 / 171, 1536 x 8960
+// 42.9 / 53.7 / 94.7 / 173 / 251 / 484 -> 32.3 / 48.5 / 67.8 / 123 / 233 / 479 (up to 640 workgroups a group); tiles of 16 x 16 that the chip holds at once share
+// k among sixteen wavefronts: 256 x 4096 at 64 / 256 / 512 15.7 / 16.0 / 22.9 -> 17.2 / 17.7 / 18.6.  A short k gains nothing: 512 x 2048 at 64 / 320
+// 11.2 / 16.8 -> 11.9 / 16.8.
+extern "C" int shk_gemm_f32_groups_faster(int n, int m, int k) {
+  if (shk_gemm_f32_splits(n, m, k) == 1) return 0;
+  if (n <= 16) return m <= 1024 ? k <= 2560 || k >= 4096 : m <= 1536 && k <= 2560;
+  return (m + 15LL) / 16 * ((n + 15) / 16) > 256;
 }
 
 extern "C" int shk_gemm_f32_groups(const void* a, const void* wt, void* out, int n, int m, int k, int lda, void* stream) {

@@ -99,7 +99,7 @@ class Runtime:
         if not count:
             n = x.shape[0]
             if target is not None and w.tiled is None and bias is None and w.rows <= 8192 and ops.f32_rows_aligned(x) \
-                    and ops.gemm_f32_splits(n, w.rows, w.cols) > 1:
+                    and ops.gemm_f32_groups_faster(n, w.rows, w.cols):
                 parts = ctx.buffer(name + "_parts", (ops.gemm_f32_splits(n, w.rows, w.cols), n, w.rows), torch.float32)
                 ops.gemm_f32_groups(x, w.tiled_f32, w.rows, w.cols, parts)
                 return ops.SplitSum(parts)

@@ -44,6 +44,7 @@ _SIGNATURES = {
     "shk_gemm_f32_tiled_weight": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
     "shk_gemm_f32_few": [_I, _I, _I],
     "shk_gemm_f32_splits": [_I, _I, _I],
+    "shk_gemm_f32_groups_faster": [_I, _I, _I],
     "shk_gemm_f32_groups": [_P, _P, _P, _I, _I, _I, _I, _P],
     "shk_gemm_f32_gated_takes": [_I, _I, _I],
     "shk_gemm_f32_gated_faster": [_I, _I, _I],

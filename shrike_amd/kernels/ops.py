@@ -378,8 +378,13 @@ def gemm_f32_few(n: int, m: int, k: int) -> bool:
 
 
 def gemm_f32_splits(n: int, m: int, k: int) -> int:
-    """Parts in which gemm_f32_groups leaves an [n, k] x [m, k]^T product (1: it is better formed whole)."""
+    """Parts in which gemm_f32_groups may leave an [n, k] x [m, k]^T product (1: only whole)."""
     return int(load().shk_gemm_f32_splits(n, m, k))
+
+
+def gemm_f32_groups_faster(n: int, m: int, k: int) -> bool:
+    """Whether those parts and a norm that adds them are formed sooner than the product whole and the norm."""
+    return bool(load().shk_gemm_f32_groups_faster(n, m, k))
 
 
 def gemm_f32_gated_takes(n: int, m: int, k: int) -> bool:
