@@ -294,8 +294,15 @@ static bool few_takes(int n, int m, int k, long long most) {
 
 // Not where a second round of workgroups would be nearly empty: 320 of them (5120 x 5120 at 8 tokens 14.3 us for product in shares
 // and norm, 15.1 here; 5120 x 13824 28.0 and 31.4).  256 are a round: 4096 x 14336 23.7 -> 20.0.
+// Nor where few workgroups walk a long k, which shares of it spread over the chip.  Product and norm against this at 1 / 8 / 16 tokens: 512 x 5120
+// 6.6 / 7.2 / 7.3 -> 6.0 / 6.0 / 6.9, x 8192 7.7 / 8.0 / 8.4 -> 8.7 / 8.8 / 9.4, 256 x 18944 8.4 / 9.0 / 9.4 -> 17.1 / 17.1 / 18.5, 1536 x 6144 10.1 / 10.5 /
+// 11.2 -> 7.8 / 7.8 / 8.3, x 8960 10.3 / 11.2 / 12.5 -> 11.5 / 11.5 / 11.6, x 18944 14.6 / 16.7 / 19.2 -> 21.4 / 18.7 / 20.3, 2048 x 8192 11.6 / 12.0 /
+// 12.0 -> 11.4 / 11.4 / 10.8, x 14336 15.1 / 15.3 / 16.5 -> 17.9 / 15.0 / 16.3, 2304 x 9216 12.3 / 13.2 / 14.5 -> 12.5 / 13.6 / 15.9, 2560 x 8192 12.1 / 12.1 / 13.1 -> 11.5 / 10.8 / 12.7, x 13824 16.3 / 15.8 /
+// 17.7 -> 17.6 / 16.3 / 19.3; 192 workgroups and more at any k: 3072 x 18944 23.9 / 24.8 / 27.7 -> 23.0 / 22.4 / 26.3, 4096 x 24576 36.3 / 37.8 / 41.0 -> 33.9 /
+// 32.7 / 35.9; 64 tokens, 256 x 6144 8.6 -> 10.0, 512 x 5120 10.6 -> 9.4, x 8192 11.0 -> 12.8.
 extern "C" int shk_few_stream_sums(int n, int m, int k) {
-  return m > 0 && m <= 4096 && m % 16 == 0 && k > 0 && k % 8 == 0 && few_takes(n, m, k, kFewStreamMost) ? m / few_stream_rows(m) : 0;
+  const bool near = m >= 3072 || k <= 5120 || (m <= 2048 ? k <= 4 * m : 2 * k <= 7 * m);
+  return m > 0 && m <= 4096 && m % 16 == 0 && k > 0 && k % 8 == 0 && near && few_takes(n, m, k, kFewStreamMost) ? m / few_stream_rows(m) : 0;
 }
 
 // `m` rows of the gate and as many of the other matrix; the k columns may come with as many sums as few_stream leaves.
