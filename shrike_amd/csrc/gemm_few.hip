@@ -287,6 +287,10 @@ constexpr long long kFewStreamMost = 5 * 1000 * 1000, kFewHeadsMost = 6 * 1000 *
 // 9.1 / 9.2 / 9.4 / 9.4 / 9.7 -> 3.2 / 3.6 / 4.0 / 4.4 / 4.7 us, 1152 x 896 9.9 / 10.0 / 12.2 / 12.5 / 13.4 -> 5.3 / 6.6 / 8.8 /
 // 11.8 / 14.4 (the line lies at 400), 2048 x 1536 12.3 / 13.3 / 18.5 -> 9.2 / 12.7 / 20.6 (at 128), 2560 x 2048 15.7 / 16.8 -> 14.0 / 20.7.
 constexpr long long kFewHeadsRead = 26 * 1000 * 1000;
+// Of 17 to 64 tokens, whose product's own kernel reads the weights once, at 17 / 32: 4608 x 1536 11.6 / 13.3 -> 11.5 / 12.3, 3584 x 2560 11.9 /
+// 13.6 -> 11.7 / 12.0, 4096 x 2304 11.6 / 12.8 -> 11.0 / 11.6, but 4096 x 2560 11.9 / 13.3 -> 12.3 / 12.7, 4608 x 2304 11.8 / 13.0 -> 13.7 / 14.5,
+// 6144 x 2048 12.9 / 13.9 -> 15.2 / 15.6.
+constexpr long long kFewHeadsReadFew = 20 * 1000 * 1000;
 
 static bool few_takes(int n, int m, int k, long long most) {
   return n <= 16 || (n <= kFewTokens && static_cast<long long>(m) * k <= most);
@@ -311,7 +315,7 @@ extern "C" int shk_few_gated_takes(int n, int m, int k) { return m > 0 && k > 0 
 extern "C" int shk_few_heads_takes(int n, int m, int k) {
   if (m <= 0 || k <= 0 || k % 8) return 0;
   if (few_takes(n, m, k, kFewHeadsMost)) return 1;
-  return n <= kFewHeadsTokens && (counted_tokens(n) + 15LL) / 16 * m * k <= kFewHeadsRead;
+  return n <= kFewHeadsTokens && (counted_tokens(n) + 15LL) / 16 * m * k <= (n <= kFewTokens ? kFewHeadsReadFew : kFewHeadsRead);
 }
 
 extern "C" int shk_few_stream(const void* a, int lda, int n, int k, const void* wt, int m, const float* bias, float* resid,
