@@ -599,6 +599,8 @@ int shk_moe_experts_grouped(const void* x, const int32_t* chosen, const float* w
 // null: none, shared_ff 0), added times sigmoid(add_gate[t * gate_ld]) where that is given.  act_buf [n * top][ff], shared_act
 // [n][shared_ff], pair_out float32 [(n * top + n)][width] (n * top without a shared expert).
 int shk_moe_few_takes(int n, int top);
+// whether they are the faster way for a layer of these sizes
+int shk_moe_few_faster(int width, int ff, int shared_ff, int experts, int top, int identity);
 int shk_moe_few(const void* x, const int32_t* chosen, const float* weights, const void* w_gate, const void* w_up,
                 const void* w_down, const void* shared_gate_up, const void* shared_down, const float* add_gate, int gate_ld,
                 void* act_buf, void* shared_act, float* pair_out, void* out, int n, int width, int ff, int shared_ff,

@@ -5,6 +5,8 @@
 // What bounds it is the weights' stream.  Eight tokens, two of eight experts of 4736 over a width of 3584 beside a shared one of 9472: lists
 // 4.6 us, experts 88 and 47, shared 26 and 23, join 4.8 in moe.hip's kernels for short lists and the plain products; a step of 28 such layers
 // 7,570 us so, 6,490 here, one token 4,918 and 3,970, sixteen 8,615 and 7,246.
+#include <cmath>
+
 #include "gemm_few.h"
 
 namespace shk {
@@ -181,6 +183,27 @@ __global__ void __launch_bounds__(256)
 using namespace shk;
 
 extern "C" int shk_moe_few_takes(int n, int top) { return n <= 16 && top <= kMoeFewTop; }
+
+// Whether a layer's steps of up to 16 tokens are faster here than in moe.hip's kernels for short lists and the shared expert's own products.
+// What they save is one launch, with a shared expert four, and that weights stream side by side; what they cost is a workgroup for every block of
+// every expert, chosen or not, and more of them than the other kernels where a block has pairs.  An estimate in microseconds, fitted to 1,755
+// measured steps (2 to 512 experts of 64 x 64 to 7168 x 2048, shared ones of none to 9,472 features, 1 to 8 choices, 1 to 16 tokens): of the
+// 755 that it takes, three are more than 2 % slower (up to 9), the others take 0.53 to 1.02 of the time.  Us at 1 / 4 / 16 tokens, there -> here, said
+// to be faster: 8 experts of 3584 x 4736, two chosen, and a shared one of 9472 95 / 151 / 205 -> 76 / 124 / 165, of 896 x 1216 and 2432 25.3 / 28.2 / 32.1 ->
+// 15.9 / 18.4 / 22.8, 16 of 512 x 512 and 512 18.8 / 19.4 / 20.7 -> 11.9 / 15.1 / 17.7, 8 of 64 x 64 alone 12.1 / 12.4 / 12.6 -> 9.5 / 9.9 / 10.6; not: 64 of 896 x
+// 1216 and 2432 26.0 / 33.6 / 50.3 -> 27.6 / 35.1 / 54.9, 128 of 2048 x 768, eight chosen, 34.0 / 60.3 / 141 -> 49.2 / 87.6 / 180, 512 of them 41.5 / 68.0 / 191 ->
+// 133 / 173 / 348, 16 of 512 x 512 alone 12.8 / 13.2 / 13.6 -> 12.0 / 14.4 / 15.9.  One answer for all numbers of tokens, which a recorded step stands for.
+extern "C" int shk_moe_few_faster(int width, int ff, int shared_ff, int experts, int top, int identity) {
+  if (experts < 1 || top < 1 || top > kMoeFewTop || top > experts + identity) return 0;
+  const bool shared = shared_ff > 0;
+  const double places = (experts + (shared ? 1 : 0)) * ((ff > shared_ff ? ff : shared_ff) + static_cast<double>(width)) / 16e3;
+  for (int n : {1, 16}) {
+    const double chosen = experts * (1.0 - std::pow(1.0 - static_cast<double>(top) / (experts + identity), n));
+    const double blocks = chosen * (ff + static_cast<double>(width)) / 16e3, megabytes = 6e-6 * width * ff * chosen, beside = 6e-6 * width * shared_ff;
+    if (2.0 + (shared ? 5.0 : 0.0) + 0.05 * megabytes + 0.11 * beside <= 0.9 * places + (4.0 + 0.07 * n) * blocks) return 0;
+  }
+  return 1;
+}
 
 extern "C" int shk_moe_few(const void* x, const int32_t* chosen, const float* weights, const void* w_gate, const void* w_up,
                            const void* w_down, const void* shared_gate_up, const void* shared_down, const float* add_gate, int gate_ld,

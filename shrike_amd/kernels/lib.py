@@ -117,6 +117,7 @@ _SIGNATURES = {
     "shk_moe_experts_plan": [_I, _I, _I, _I, _I, _I, _I, _I],
     "shk_moe_experts_grouped": [_P, _P, _P, _P, _P, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _F, _I, _P],
     "shk_moe_few_takes": [_I, _I],
+    "shk_moe_few_faster": [_I, _I, _I, _I, _I, _I],
     "shk_moe_few": [_P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _F, _F, _F, _P],
     "shk_xielu": [_P, _P, _I, c_longlong, _F, _F, _P],
     "shk_embed_pairs": [_P, _P, _I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],

@@ -14,7 +14,8 @@ class MixtureOfExperts(FeedForward):
     matrices are stacked [experts, ...] when the weights are loaded and every (token, chosen
     expert) pair is multiplied by its own expert's rows on the device, chosen there: nothing of
     the routing is read on the host, so steps are recorded into graphs.  The shared expert is
-    the framework's dense gated product; its output is the sum's first term.  From a few
+    the framework's dense gated product, its output the sum's first term (in steps of few tokens that run in
+    ops.moe_few, one more expert of the launch and the last).  From a few
     tokens on, bfloat16 steps list each expert's pairs on the device and run the two products
     per expert on the matrix units, so that an expert's matrices are read once a step."""
 
@@ -118,7 +119,8 @@ class MixtureOfExperts(FeedForward):
             self.shared = (runtime.weight(tensors[f"{self.name}.shared.up"]),
                            runtime.weight(tensors[f"{self.name}.shared.down"]))
         # whether steps of few tokens take the shared expert beside the others (ops.moe_few)
-        self.few = self.tiled and self.gated and (s.shared_size is None or s.shared_size % 32 == 0)
+        self.few = (self.tiled and self.gated and (s.shared_size is None or s.shared_size % 32 == 0)
+                    and ops.moe_few_faster(self.width, s.expert_size, s.experts, s.top, s.shared_size or 0, s.identity))
         self.linear = runtime.linear
         self.gated_linear = runtime.gated_linear
 
