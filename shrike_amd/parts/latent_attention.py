@@ -76,9 +76,15 @@ class LatentAttention(Mixer):
 
     @property
     def single_in_prompt(self) -> bool:
-        """Whether single tokens take the prompt portions' kernel too, one a workgroup: the same bits, 0.5 to 0.8 of the time (14 heads
-        over rows of 176, 28 over rows of 512; 60 to 1,500 rows, 1 to 16 tokens)."""
-        return bool(self.prompt_tokens) and self.spec.num_heads >= 4
+        """Whether single tokens take the prompt portions' kernel too, one a workgroup: the same bits, most often 0.4 to 0.9 of the time (4
+        to 112 heads, rows of 96 to 512, 1 to 128 tokens at 60 to 20,000 rows: 8 tokens at 1,000 15.4 -> 10.9 us with 4 heads over rows of 96,
+        25.9 -> 14.9 with 28 over 264, 128 at 3,000 188 -> 121 with 16 over 264).  Not for latents of up to 64, which the kernel for single tokens
+        holds in fewer registers (rows of 72, 64 tokens at 1,500: 15.3 -> 17.5; 128 at 400: 12.1 -> 14.5), nor for 33 to 64 heads over latents of more
+        than 128 in rows of up to 256, where eight blocks of columns are multiplied for half as many (33 heads over 176, 64 tokens at 1,500 35.0 ->
+        40.0, 128 at 3,000 89.8 -> 112; 100 heads 66.7 -> 49.3 and 176 -> 126)."""
+        heads, latent = self.spec.num_heads, self.spec.kv_rank
+        return (bool(self.prompt_tokens) and heads >= 4 and latent > 64
+                and (not 32 < heads <= 64 or latent <= 128 or latent + self.spec.rot_dim > 256))
 
     def prepare(self, shape) -> None:
         """Among how many workgroups each token's rows are shared on the matrix-instruction
