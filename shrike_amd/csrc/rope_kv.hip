@@ -153,6 +153,10 @@ constexpr int kVecMinTokens = 65;
 // The whole kernel, us, token by token and so: 40 heads of 128 over 8 at 512 / 1,119 / 2,048 tokens 13.3 / 24.3 / 22.3 -> 10.5 / 19.3 /
 // 16.9, 28 over 4 9.4 / 15.0 / 15.5 -> 8.0 / 11.9 / 12.2 (portions that begin inside a piece 15.5 -> 13.9), 14 of 64 over 2 5.5 / 8.8 /
 // 9.0 -> 5.6 / 7.9 / 8.4.  Every thread looking up all eight pages itself: 10.9 / 20.1 / 18.6, 7.9 / 12.4 / 13.3, 5.7 / 8.0 / 8.6.
+// Where that would be 128 workgroups or fewer, they are of one wavefront each, so that four times as many compute units store:
+// single tokens, whose values lie apart, 28 heads of 128 over 4 at 256 / 512 5.1 / 6.8 us token by token, 5.7 / 6.9 in whole workgroups, 5.1 / 6.5
+// so, 40 over 8 at 256 6.7, 7.1 and 6.6, 14 of 64 over 2 at 256 4.2, 4.3 and 4.1; a prompt's 256 of 28 over 4 4.9, 4.6 and 4.3.  (Up
+// to 128 tokens, and 16 over 16, gain nothing: at 128 6.7, 5.1 and 5.3.)
 constexpr int kValueTokens = 8;
 
 __device__ __forceinline__ void store_values(int first, int col, int n, int width, int values, int kv_heads, int head_dim,
@@ -225,14 +229,15 @@ __global__ void __launch_bounds__(kRopeThreads)
                              const int32_t* __restrict__ tables, int table_stride,
                              bf16* __restrict__ k_pool, bf16* __restrict__ v_pool, int page_size,
                              int num_pages, int write_kv, const float* __restrict__ parts, int splits,
-                             const float* __restrict__ bias, float magnitude, unsigned value_blocks) {
+                             const float* __restrict__ bias, float magnitude, unsigned value_blocks, int value_threads) {
   __shared__ float cs[kMaxHalf];
   __shared__ float sn[kMaxHalf];
   const int half = head_dim / 2;
   const int width = (heads + 2 * kv_heads) * head_dim;
   if (blockIdx.x < value_blocks) {
-    const int per = (kv_heads * head_dim + kRopeThreads - 1) / kRopeThreads;
-    store_values(blockIdx.x / per * kValueTokens, blockIdx.x % per * kRopeThreads + threadIdx.x, n, width, (heads + kv_heads) * head_dim,
+    const int per = (kv_heads * head_dim + value_threads - 1) / value_threads;
+    if (static_cast<int>(threadIdx.x) >= value_threads) return;
+    store_values(blockIdx.x / per * kValueTokens, blockIdx.x % per * value_threads + threadIdx.x, n, width, (heads + kv_heads) * head_dim,
                  kv_heads, head_dim, qkv, positions, token_seq, tables, table_stride, v_pool, page_size, num_pages, parts, splits, bias);
     return;
   }
@@ -518,12 +523,14 @@ extern "C" int shk_rope_kv_store(void* qkv, int dtype, int n, int heads, int kv_
       vec_items <= kVecItems * kRopeThreads && reinterpret_cast<uintptr_t>(qkv) % 16 == 0 &&
       (!write_kv || reinterpret_cast<uintptr_t>(k_pool) % 16 == 0) &&
       (!parts || reinterpret_cast<uintptr_t>(parts) % 16 == 0)) {
-    const int per = (kv_heads * head_dim + kRopeThreads - 1) / kRopeThreads;
+    const int wide = (kv_heads * head_dim + kRopeThreads - 1) / kRopeThreads, groups = (n + kValueTokens - 1) / kValueTokens;
+    const int value_threads = n > 128 && wide <= 4 && groups * wide <= 128 ? kWave : kRopeThreads;
+    const int per = (kv_heads * head_dim + value_threads - 1) / value_threads;
     const unsigned value_blocks = write_kv ? static_cast<unsigned>((n + kValueTokens - 1) / kValueTokens) * per : 0;
     rope_kv_store_vec_kernel<<<n + value_blocks, kRopeThreads, 0, s>>>(
         static_cast<bf16*>(qkv), n, heads, kv_heads, head_dim, inv_freq, positions, token_seq, tables,
         table_stride, static_cast<bf16*>(k_pool), static_cast<bf16*>(v_pool), page_size, num_pages,
-        write_kv, parts, splits, bias, magnitude, value_blocks);
+        write_kv, parts, splits, bias, magnitude, value_blocks, value_threads);
     SHK_LAUNCH_CHECK("rope_kv_store");
     return 0;
   }
