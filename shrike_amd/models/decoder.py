@@ -35,11 +35,13 @@ class DecoderModel:
         # every run's result is kept and the stream that goes on is a weighted sum of them
         self._averaged = bool(spec.schedule) and spec.schedule[0].depth_average is not None
         self.depth_coefficients: list = []
-        # of every run, (norm, mixer) that the next one begins with, where nothing comes between them
+        # of every run, (norm, mixer) that the next one begins with, where nothing comes between them (a block derived from
+        # the pre-norm one may do more with the stream, before its parts or after them)
         self._following: list = [None] * len(spec.schedule)
         for pos, entry in enumerate(spec.schedule[1:]):
             block = self.blocks[entry.block]
-            if type(block).forward is PreNormResidualBlock.forward and not entry.add_embedding and entry.add_vector is None:
+            plain = all(type(b).forward is PreNormResidualBlock.forward for b in (self.blocks[spec.schedule[pos].block], block))
+            if plain and not entry.add_embedding and entry.add_vector is None:
                 self._following[pos] = (block.mixer_norm, block.mixer)
         # the parts whose prepare() does something, in the order they run
         self._preparers = [p for p in self.parts() if type(p).prepare is not Part.prepare]
