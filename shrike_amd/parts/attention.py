@@ -642,9 +642,10 @@ class PagedAttention(Mixer):
         return type(self).forward is PagedAttention.forward
 
     def takes_scaled(self, ctx) -> bool:
-        """Whether the step's projections, their rotation and the cache write are one kernel (ops.few_heads)."""
+        """Whether the step's projections, their rotation and the cache write are one kernel (ops.few_heads).  It leaves the
+        queries alone beside the cache, so not for an attend() of another class, which may read the step's keys and values too."""
         s = self.spec
-        if not self.ends_onto or self.plain_store or s.values_from_keys or self.position is None or getattr(self.position, "adjacent_pairs", False):
+        if not self.ends_onto or type(self).attend is not PagedAttention.attend or self.plain_store or s.values_from_keys or self.position is None or getattr(self.position, "adjacent_pairs", False):
             return False
         table = self.position.rotary_table()
         return (table is not None and table[1] == s.head_dim and s.head_dim % 16 == 0 and self.w_qkv.tiled is not None
