@@ -260,12 +260,11 @@ static bool few_rows_of(FewRows* x, const void* a, int lda, int n, int k, int mo
   return n >= 0 && n <= most && k > 0 && k % 8 == 0 && (pieces || (lda >= k && lda % 8 == 0));
 }
 
-// fn with the loads of a thread that adds up squares as a constant
+// fn with the loads of a thread that adds up squares (at least one) as a constant
 template <typename Fn>
 static void with_loads(int count, int threads, Fn fn) {
   const int loads = (count + threads / 16 - 1) / (threads / 16);
-  if (loads == 0) fn(std::integral_constant<int, 0>{});
-  else if (loads <= 4) fn(std::integral_constant<int, 4>{});
+  if (loads <= 4) fn(std::integral_constant<int, 4>{});
   else if (loads <= 8) fn(std::integral_constant<int, 8>{});
   else fn(std::integral_constant<int, 16>{});
 }
@@ -326,12 +325,14 @@ extern "C" int shk_few_stream(const void* a, int lda, int n, int k, const void* 
   SHK_REQUIRE(a && wt && resid && weight && rows && sums, "few_stream: null pointer");
   SHK_REQUIRE(reinterpret_cast<uintptr_t>(a) % 16 == 0, "few_stream: rows are not 16-byte aligned");
   const int kt = (k + 31) / 32, waves = few_waves(kt, kFewTiles), rows_each = few_stream_rows(m);
-  // two blocks of tokens in a workgroup where many tokens would have a long k read four times over (896 x 4864 at 64
-  // tokens 10.4 us in one, 9.5; at 32 6.6 in one, 10.0)
-  const int nb = n > 32 && kt > kFewTiles * waves ? 2 : 1;
   with_tiles<kFewTiles>((kt + waves - 1) / waves, [&](auto c) {
-    const auto kernel = nb == 2 ? rows_each == 8 ? few_stream_kernel<c.value, 8, 2> : few_stream_kernel<c.value, 16, 2>
-                        : rows_each == 8 ? few_stream_kernel<c.value, 8, 1> : few_stream_kernel<c.value, 16, 1>;
+    auto kernel = rows_each == 8 ? few_stream_kernel<c.value, 8, 1> : few_stream_kernel<c.value, 16, 1>;
+    int nb = 1;
+    if constexpr (c.value == 0) {
+      // two blocks of tokens in a workgroup where many tokens would have a long k read four times over (896 x 4864 at 64
+      // tokens 10.4 us in one, 9.5; at 32 6.6 in one, 10.0)
+      if (n > 32 && rows_each == 8) kernel = few_stream_kernel<0, 8, 2>, nb = 2;
+    }
     kernel<<<dim3(m / rows_each, (n + 16 * nb - 1) / (16 * nb)), waves * kWave, nb * waves * kWave * sizeof(f32x4), static_cast<hipStream_t>(stream)>>>(
         x, static_cast<const u32x4*>(wt), kt, m, bias, resid, weight, static_cast<bf16*>(rows), sums);
   });
@@ -388,7 +389,7 @@ extern "C" int shk_few_heads(const void* a, int lda, int n, int k, const void* w
   const int groups = (heads + 2 * kv_heads) * (head_dim / 16);
   const int kt = (k + 31) / 32, waves = few_waves(kt, kFewTiles);
   SHK_REQUIRE(!sums || count <= kFewMostLoads * (waves + 1) * 4, "few_heads: too many sums (%d)", count);
-  with_loads(sums ? count : 0, (waves + 1) * kWave, [&](auto loads) {
+  const auto go = [&](auto loads) {
     with_tiles<kFewTiles>((kt + waves - 1) / waves, [&](auto c) {
       const size_t lds = waves * kWave * sizeof(f32x4) + (waves + 1) * 16 * sizeof(float);
       few_heads_kernel<c.value, loads.value><<<dim3(groups, (n + 15) / 16), (waves + 1) * kWave, lds, static_cast<hipStream_t>(stream)>>>(
@@ -396,7 +397,11 @@ extern "C" int shk_few_heads(const void* a, int lda, int n, int k, const void* w
           token_seq, tables, table_stride, static_cast<bf16*>(k_pool), static_cast<bf16*>(v_pool), page_size, num_pages, write_kv,
           magnitude);
     });
-  });
+  };
+  if (sums)
+    with_loads(count, (waves + 1) * kWave, go);
+  else
+    go(std::integral_constant<int, 0>{});
   SHK_LAUNCH_CHECK("few_heads");
   return 0;
 }
