@@ -517,9 +517,13 @@ extern "C" int shk_rope_kv_store(void* qkv, int dtype, int n, int heads, int kv_
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
   // whole vectors where the layout allows: bfloat16, rows rotated whole, 16-byte alignment
-  const int vec_items = (heads + kv_heads) * (head_dim / 16) + kv_heads * (head_dim / 8);
+  // pairs of runs of queries and keys (values have workgroups of their own).  Where every thread has its four, few tokens' workgroups
+  // are too long: 112 heads of 128 over 8 at 65 / 128 / 300 / 1,024 tokens 5.2 / 7.8 / 14.6 / 40.8 us element by element, 7.0 / 7.8 / 8.8 / 15.2 in
+  // vectors; 64 over 64 8.7 / 15.3 / 27.6 / 77.1 and 7.6 / 14.3 / 11.6 / 25.3.
+  const int vec_items = (heads + kv_heads) * (head_dim / 16);
+  const bool full = vec_items + kv_heads * (head_dim / 8) > kVecItems * kRopeThreads;
   if (dtype == kBF16 && pairing == 0 && !v_from_k && rot_dim == head_dim && head_dim % 16 == 0 &&
-      n >= kVecMinTokens &&
+      n >= (full ? 2 * kVecMinTokens - 2 : kVecMinTokens) &&
       vec_items <= kVecItems * kRopeThreads && reinterpret_cast<uintptr_t>(qkv) % 16 == 0 &&
       (!write_kv || reinterpret_cast<uintptr_t>(k_pool) % 16 == 0) &&
       (!parts || reinterpret_cast<uintptr_t>(parts) % 16 == 0)) {
