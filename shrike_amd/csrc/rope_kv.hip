@@ -523,7 +523,7 @@ extern "C" int shk_rope_kv_store(void* qkv, int dtype, int n, int heads, int kv_
   const int vec_items = (heads + kv_heads) * (head_dim / 16);
   const bool full = vec_items + kv_heads * (head_dim / 8) > kVecItems * kRopeThreads;
   if (dtype == kBF16 && pairing == 0 && !v_from_k && rot_dim == head_dim && head_dim % 16 == 0 &&
-      n >= (full ? 2 * kVecMinTokens - 2 : kVecMinTokens) &&
+      n >= (full ? 128 : kVecMinTokens) &&
       vec_items <= kVecItems * kRopeThreads && reinterpret_cast<uintptr_t>(qkv) % 16 == 0 &&
       (!write_kv || reinterpret_cast<uintptr_t>(k_pool) % 16 == 0) &&
       (!parts || reinterpret_cast<uintptr_t>(parts) % 16 == 0)) {
