@@ -160,8 +160,8 @@ int shk_gemm_bf16_parts(int n, int m, int k, int gated);
 // tiles of a product of more than 64 tokens: their number (0: not served in tiles), (weight rows, tokens) of up to two
 int shk_gemm_bf16_tiles(int n, int m, int k, int gated, int ksplit, int aligned, int* sizes);
 
-// Products of up to 64 tokens (bfloat16, rows 16-byte aligned, k a multiple of 8) that spare the kernels around them; the
-// queries say for which sizes they are the faster ones (shk_few_stream_sums: 0 where not).  lda 0: the rows come as [k / 8][n][8].
+// Products of up to 64 tokens (shk_few_heads: 512; bfloat16, rows 16-byte aligned, k a multiple of 8) that spare the kernels around them;
+// the queries say for which sizes they are the faster ones (shk_few_stream_sums: 0 where not).  lda 0: the rows come as [k / 8][n][8].
 // shk_few_stream: resid[n, m] += a @ w^T + bias (float32 [m] or null); rows [m / 8][n][8] = the new resid * weight in
 // bfloat16 and sums[shk_few_stream_sums(n, m, k)][n] its squares summed by workgroup: what the next two calls take in the place of
 // normed rows, dividing by sqrt(mean(resid^2) + eps) what they form.  m a multiple of 16.

@@ -6,7 +6,9 @@ order of summation whatever the number of rows), weights in tiles of 16 x 16.  b
 operand layout; products with at most 16 rows stream them once through the
 skinny kernel, up to 64 through the streaming one, more rows run the LDS-staged one; from 17 rows on matrices of 256 to 2,048
 weight rows (as far as they are quicker so) run without staging, and from 65 on matrices of up to 64 weight rows in the
-skinny kernel, 16 rows a workgroup.  What a mixer
+skinny kernel, 16 rows a workgroup.  With at most 16 rows, of small matrices 64, a sublayer's last product may add to the
+stream itself, and the products that read the stream then divide by its root mean square (linear_onto, ops.few_stream,
+ops.few_gated, ops.few_heads).  What a mixer
 does between its products is the mixer's own business.
 """
 
