@@ -23,8 +23,6 @@
 // rows 75 TFLOP/s; gemm_f32_lds_kernel, which shares them, 97).  Before, one workgroup per 64 x 64 results with vector
 // instructions: a 0.5B decode step of four requests 23.9 ms (2.4 with this kernel, 1.56 with attention_f32.hip as
 // well), a 509-token prompt 42.6 ms (18.9, 6.5; 5.4 with operands shared); the logits' error against 64 bits 6.4e-7 (2.5e-7).
-#include <type_traits>
-
 #include "api.h"
 #include "common.h"
 #include "gemm_wide.h"
@@ -546,16 +544,6 @@ static bool f32_few(int n, int m, int k) {
   return n <= 8 && k >= 896 && k <= 1024;
 }
 
-// fn with the steps of a wavefront rounded up to one of a few constants, 0 for more than ten.
-template <typename Fn>
-static void with_steps(int steps, Fn fn) {
-  if (steps <= 2) fn(std::integral_constant<int, 2>{});
-  else if (steps <= 4) fn(std::integral_constant<int, 4>{});
-  else if (steps <= 6) fn(std::integral_constant<int, 6>{});
-  else if (steps <= 10) fn(std::integral_constant<int, 10>{});
-  else fn(std::integral_constant<int, 0>{});
-}
-
 // Half blocks of features and a segment a wavefront up to 2,048 features, the segments also for a k of up to 1,024, else a group
 // a wavefront: 9728 x 896 at 4 rows 8.7 us by segments, 10.0 by groups, 3584 x 3584 15.5 and 12.2, 3584 x 18944 at 16 rows 70 and 61.
 static void launch_f32_few(const F32Product& p, hipStream_t s) {
@@ -688,7 +676,7 @@ extern "C" int shk_gemm_f32_splits(int n, int m, int k) {
 // Whether the groups and a norm that adds them are faster than the product whole and the norm.  Weights cold, us, whole -> in groups.
 // Up to 16 rows, at 1 / 8 / 16: 896 x 4864 14.8 / 16.1 / 18.3 -> 11.4 / 12.0 / 13.9, 1024 x 16384 34.7 / 36.3 / 42.6 -> 24.0 / 24.7 / 31.6; with more features the
 // product has workgroups enough but for steps that its wavefronts hold at once: 1536 x 2560 9.5 / 9.9 / 12.0 -> 9.1 / 9.4 / 11.0, x 2576 11.3 / 12.0 /
-// 12.5 -> 13.0 / 13.8 / 16.9, x 8960 23.3 / 24.6 / 28.0 -> 22.6 / 24.9 / 29.1, 2048 x 2048 9.9 / 10.2 / 11.9 -> 10.2 / 10.6 / 12.4, x 5632 17.2 / 18.2 /
+// 12.5 -> 13.0 / 13.8 / 16.9, x 8960 23.3 / 24.6 / 28.0 -> 22.2 / 24.3 / 29.1, 2048 x 2048 9.9 / 10.2 / 11.9 -> 10.2 / 10.6 / 12.4, x 5632 17.2 / 18.2 /
 // 21.0 -> 21.7 / 22.3 / 29.1 (1024 x 2576 10.9 / 11.6 / 12.0 -> 10.4 / 10.9 / 13.0).
 // More rows, at 64 / 100 / 256 / 512 / 1,000 / 2,000: 896 x 4864 19.3 / 27.2 / 33.5 / 58.4 / 97 / 179 -> 20.2 / 20.9 / 30.7 / 49.5 / 83 / 171, 1536 x 8960
 // 42.9 / 53.7 / 94.7 / 173 / 251 / 484 -> 32.3 / 48.5 / 67.8 / 123 / 233 / 479 (up to 640 workgroups a group); tiles of 16 x 16 that the chip holds at once share
@@ -696,7 +684,7 @@ extern "C" int shk_gemm_f32_splits(int n, int m, int k) {
 // 11.2 / 16.8 -> 11.9 / 16.8.
 extern "C" int shk_gemm_f32_groups_faster(int n, int m, int k) {
   if (shk_gemm_f32_splits(n, m, k) == 1) return 0;
-  if (n <= 16) return m <= 1024 ? k <= 2560 || k >= 4096 : m <= 1536 && k <= 2560;
+  if (n <= 16) return m <= 1536 && (k <= 2560 || (k >= 4096 && (m <= 1024 || n <= 8)));
   return (m + 15LL) / 16 * ((n + 15) / 16) > 256;
 }
 
@@ -708,13 +696,12 @@ extern "C" int shk_gemm_f32_groups(const void* a, const void* wt, void* out, int
               "gemm_f32_groups: null or misaligned pointer");
   const F32Product p{static_cast<const float*>(a), static_cast<const float*>(wt), nullptr, static_cast<float*>(out), n, m, k, lda, m, 0, 1, 0, 0, 0};
   const hipStream_t s = static_cast<hipStream_t>(stream);
-  if (n <= 16)
-    with_steps((k + 16 * kF32Segments - 1) / (16 * kF32Segments), [&](auto c) {
-      gemm_f32_few_kernel<4, 8, c.value, false, true><<<dim3((m + 7) / 8, kF32Segments / kF32Group), 4 * kWave, 0, s>>>(
-          p.a, p.w, nullptr, p.out, n, m, k, lda, m, 0, F32Gate{});
-    });
-  else
+  if (n <= 16) {  // (ten steps a segment are asked for at once, which is a k of 2,560)
+    const auto kernel = k <= 2560 ? gemm_f32_few_kernel<4, 8, 10, false, true> : gemm_f32_few_kernel<4, 8, 0, false, true>;
+    kernel<<<dim3((m + 7) / 8, kF32Segments / kF32Group), 4 * kWave, 0, s>>>(p.a, p.w, nullptr, p.out, n, m, k, lda, m, 0, F32Gate{});
+  } else {
     launch_f32_lds<1, 2, false, true>(p, s);
+  }
   SHK_LAUNCH_CHECK("gemm_f32_groups");
   return 0;
 }
