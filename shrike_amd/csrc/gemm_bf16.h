@@ -60,60 +60,58 @@ __device__ __forceinline__ float gate_times_up(float g, float u, int act, const 
 constexpr int kDies = 8;        // accelerator dies (XCDs), each with an L2 of its own
 constexpr int kDieUnits = 32;  // compute units per die
 
+// How the tiles of a large product (tiles_x along the weight rows, tiles_y along the tokens, `shares` of k) are dealt out: in one row,
+// share by share, within a share in `strips` runs of neighbouring token tiles, within a strip weight tile by weight tile.
+struct TileOrder {
+  int tiles_x, tiles_y, shares, strips;
+};
+
 // The tile of a workgroup of the large kernels; false: none (the grid is padded).
-__device__ __forceinline__ bool big_tile(int tiles_x, int tiles_y, int by_die, int& tile_x, int& tile_y) {
-  // Which tile: workgroups are handed to the chip's eight dies (each with its own
-  // L2) in turn, workgroup p to die p % 8.  The tiles are therefore dealt out in
-  // blocks of 32 (up to 8 token tiles of 32 / that many weight tiles) and block B goes to
-  // die B % 8, whose 32 compute units then work on tiles that share their
-  // operands: the die's L2 serves most of their loads.
-  // With fewer tiles (by_die == 2 * dx) the grid of tiles is cut into dx x 8/dx
-  // rectangles, one for each die, where the numbers of tiles allow that; else
-  // (by_die == 0) the tiles are taken in plain order.
-  tile_x = blockIdx.x % tiles_x, tile_y = blockIdx.x / tiles_x;
-  if (by_die > 1) {
-    const int die = blockIdx.x % kDies, turn = blockIdx.x / kDies;
-    const int dx = by_die / 2, wide = tiles_x / dx, high = tiles_y / (kDies / dx);
-    tile_x = (die % dx) * wide + turn % wide;
-    tile_y = (die / dx) * high + turn / wide;
-  } else if (by_die) {
-    const int die = blockIdx.x % kDies, turn = blockIdx.x / kDies;
-    const int block_y = tiles_y < 8 ? tiles_y : 8, block_x = kDieUnits / block_y;
-    const int blocks_x = (tiles_x + block_x - 1) / block_x;
-    const int block = (turn / kDieUnits) * kDies + die, within = turn % kDieUnits;
-    tile_x = (block % blocks_x) * block_x + within / block_y;
-    tile_y = (block / blocks_x) * block_y + within % block_y;
-    if (within >= block_x * block_y) return false;
-  }
-  return tile_x < tiles_x && tile_y < tiles_y;
+// Workgroups are handed to the chip's eight dies (each with its own L2) in turn, workgroup p to die p % 8.  Die d takes the d-th
+// eighth of the row of tiles, in order: what its 32 compute units work on at a time is a run of neighbours that share operands, so that
+// its L2 serves most of their loads, whatever the numbers of tiles.  All dies together draw 10 TB/s from beyond their L2s, 40 GB/s a
+// compute unit, which takes in 130 to 150 from its L2.  Against rectangles for the dies where the numbers divided, and every eighth tile on a
+// die where not, weights cold: 896 x 4864 at 700 / 1,119 / 2,048 tokens 19.0 / 25.1 / 34.3 us -> 15.1 / 19.2 / 28.6, 3584 x 18944 at 512
+// 76.3 -> 73.2, gate and up of 18944 x 3584 at 300 117 -> 102; whole prompts of the 7B sizes at 2,048 tokens 26.6 -> 26.1 ms.
+__device__ __forceinline__ bool big_tile(const TileOrder& t, int& tile_x, int& tile_y, int& share) {
+  const int per_share = t.tiles_x * t.tiles_y;
+  const long long all = static_cast<long long>(per_share) * t.shares;
+  const int die = blockIdx.x % kDies;
+  int i = static_cast<int>(all * die / kDies) + blockIdx.x / kDies;
+  if (i >= static_cast<int>(all * (die + 1) / kDies)) return false;
+  share = t.shares > 1 ? i / per_share : 0;
+  i -= share * per_share;
+  // strip s holds the token tiles tiles_y * s / strips up to the next one's first
+  const int strip = ((i / t.tiles_x + 1) * t.strips - 1) / t.tiles_y;
+  const int first = t.tiles_y * strip / t.strips, high = t.tiles_y * (strip + 1) / t.strips - first;
+  i -= t.tiles_x * first;
+  tile_x = i / high, tile_y = first + i % high;
+  return true;
 }
 
-// The grid of the large kernels: how big_tile() is to deal out the tiles, and the number of workgroups.
-inline unsigned big_grid(int tiles_x, int tiles_y, int tile_rows, int tile_tokens, int* by_die) {
-  // one-dimensional, in whole rounds of the eight dies' blocks of 32 tiles
-  const int block_y = tiles_y < 8 ? tiles_y : 8, block_x = kDieUnits / block_y;
-  const long long blocks = static_cast<long long>((tiles_x + block_x - 1) / block_x) * ((tiles_y + block_y - 1) / block_y);
-  // worth it from four rounds of workgroups on: below that, whole dies would stay idle
-  *by_die = static_cast<long long>(tiles_x) * tiles_y >= 4 * kDies * kDieUnits;
-  if (*by_die) return static_cast<unsigned>((blocks + kDies - 1) / kDies * kDies * kDieUnits);
-  // one rectangle of tiles per die, cut so that a die's tiles share the most
-  // operands (the fewest rows of weights and activations to read per die)
+// The grid of the large kernels, and the strips with which the tiles that a die works on at a time (`units`: workgroups on the whole
+// chip) need the fewest rows of weights and activations.
+inline unsigned big_grid(int tiles_x, int tiles_y, int shares, int tile_rows, int tile_tokens, int units, TileOrder* order) {
+  const long long all = static_cast<long long>(tiles_x) * tiles_y * shares, each = (all + kDies - 1) / kDies;
+  const int at_once = static_cast<int>(each < units / kDies ? each : units / kDies);
+  *order = TileOrder{tiles_x, tiles_y, shares, 1};
   long long least = 0;
-  for (int dx = 1; dx <= kDies; dx *= 2) {
-    const int dy = kDies / dx;
-    if (tiles_x % dx || tiles_y % dy) continue;
-    const long long rows = static_cast<long long>(tiles_x / dx) * tile_rows + static_cast<long long>(tiles_y / dy) * tile_tokens;
-    if (!least || rows < least) least = rows, *by_die = 2 * dx;
+  for (int strips = 1; strips <= tiles_y; ++strips) {
+    const int high = (tiles_y + strips - 1) / strips, wide = (at_once + high - 1) / high;
+    const long long rows = static_cast<long long>(wide < tiles_x ? wide : tiles_x) * tile_rows +
+                           static_cast<long long>(wide < tiles_x ? high : (at_once + tiles_x - 1) / tiles_x) * tile_tokens;
+    if (!least || rows < least) least = rows, order->strips = strips;
+    if (high * high * tile_tokens < tile_rows) break;  // (flatter ones only need more)
   }
-  return static_cast<unsigned>(tiles_x * tiles_y);
+  return static_cast<unsigned>(each * kDies);
 }
 
-// Weight rows and tokens that the tiles of each die need, summed over the dies, where the tiles are taken in plain order (every
-// eighth one on a die); 0 in the other orders, whose dies share.
+// Weight rows and tokens that the tiles of each die need, summed over the dies, with every eighth tile on a die; 0 where the dies
+// can have rectangles of the grid of tiles.  (What wide_fetch() of gemm_wide.hip prices.)
 inline double big_operands(int tiles_x, int tiles_y, int tile_rows, int tile_tokens) {
-  int by_die;
-  big_grid(tiles_x, tiles_y, tile_rows, tile_tokens, &by_die);
-  if (by_die) return 0.0;
+  if (static_cast<long long>(tiles_x) * tiles_y >= 4 * kDies * kDieUnits) return 0.0;
+  for (int dx = 1; dx <= kDies; dx *= 2)
+    if (tiles_x % dx == 0 && tiles_y % (kDies / dx) == 0) return 0.0;
   const double tiles = static_cast<double>(tiles_x) * tiles_y, dies = tiles < kDies ? tiles : kDies, each = tiles / dies;
   const int columns = tiles_x / (tiles_x % 4 == 0 ? 4 : tiles_x % 2 == 0 ? 2 : 1);  // of tiles that a die meets
   return dies * ((each < columns ? each : columns) * tile_rows + (each < tiles_y ? each : tiles_y) * tile_tokens);

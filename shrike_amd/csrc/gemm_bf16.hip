@@ -497,7 +497,7 @@ __global__ void __launch_bounds__(GM* GN* kWave)
     gemm_big_kernel(const bf16* __restrict__ a, int lda, int n, int k,
                     const uint4* __restrict__ wt, int ktiles, int m,
                     const float* __restrict__ bias, void* __restrict__ out, int ldo, int out_f32,
-                    int accumulate, int vec, int ksplit, int tiles_x, int tiles_y, int by_die) {
+                    int accumulate, int vec, TileOrder order) {
   constexpr int kWaves = GM * GN;
   constexpr int kWFrags = GM * WM * KS, kAFrags = GN * WN * KS;  // fragments per stage
   constexpr int kFrags = kWFrags + kAFrags;
@@ -505,17 +505,17 @@ __global__ void __launch_bounds__(GM* GN* kWave)
   auto stage = [&](int buf, int frag) -> uint4* { return stage_mem + (buf * kFrags + frag) * kWave; };
   const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
   const int wm = wave / GN, wn = wave % GN;  // place of the wavefront in the workgroup's tile
-  int tile_x, tile_y;
-  if (!big_tile(tiles_x, tiles_y, by_die, tile_x, tile_y)) return;
+  int tile_x, tile_y, share;
+  if (!big_tile(order, tile_x, tile_y, share)) return;
+  const int ksplit = order.shares;
   const int mb0 = tile_x * (GM * WM);  // first block of 16 weight rows
   const int tok0 = tile_y * (16 * GN * WN);
   // blocks of 16 weight rows; a gated weight has two per 16 output rows
   const int mblocks = (GATED ? 2 : 1) * ((m + 15) / 16);
-  // blockIdx.y: which share of the k stages (ksplit workgroups per tile leave float32
-  // partial sums [ksplit][n][m] that the reading kernel adds up)
+  // ksplit workgroups per tile leave float32 partial sums [ksplit][n][m] that the reading kernel adds up
   const int all_stages = (ktiles + KS - 1) / KS;
   const int per_split = (all_stages + ksplit - 1) / ksplit;
-  const int st_first = blockIdx.y * per_split;
+  const int st_first = share * per_split;
   const int nstages = st_first + per_split < all_stages ? st_first + per_split : all_stages;
 
   f32x4 acc[WM][WN];
@@ -589,7 +589,7 @@ __global__ void __launch_bounds__(GM* GN* kWave)
   }
 
   big_store<WM, WN, GATED>(acc, lane, tok0 + wn * WN * 16, mb0 + wm * WM, n, m, bias, out, ldo, out_f32,
-                           accumulate, blockIdx.y);
+                           accumulate, share);
 }
 
 // gemm_direct_kernel: for small matrices (cached by the time that a few hundred wavefronts ask for them) and
@@ -994,22 +994,22 @@ static void launch_big(hipStream_t s, const bf16* ap, int lda, int n, int k, con
                        int gated, int wblocks, int ksplit) {
   constexpr int lds = 2 * (GM * WM + GN * WN) * KS * kWave * 16;
   const int tiles_x = (wblocks + GM * WM - 1) / (GM * WM), tiles_y = (n + 16 * GN * WN - 1) / (16 * GN * WN);
-  int by_die;
-  const dim3 grid(big_grid(tiles_x, tiles_y, 16 * GM * WM, 16 * GN * WN, &by_die), ksplit);
+  TileOrder order;
+  const unsigned grid = big_grid(tiles_x, tiles_y, ksplit, 16 * GM * WM, 16 * GN * WN, kDies * kDieUnits, &order);
   if (gated) {
     auto kernel = gemm_big_kernel<GM, GN, WM, WN, KS, true>;
     if (lds > 65536)
       hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                           hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     kernel<<<grid, GM * GN * kWave, lds, s>>>(ap, lda, n, k, wp, kt, m, bias, out, ldo, of, accumulate,
-                                              vec, ksplit, tiles_x, tiles_y, by_die);
+                                              vec, order);
   } else {
     auto kernel = gemm_big_kernel<GM, GN, WM, WN, KS, false>;
     if (lds > 65536)
       hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                           hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     kernel<<<grid, GM * GN * kWave, lds, s>>>(ap, lda, n, k, wp, kt, m, bias, out, ldo, of, accumulate,
-                                              vec, ksplit, tiles_x, tiles_y, by_die);
+                                              vec, order);
   }
 }
 

@@ -23,23 +23,24 @@ template <int GM, int GN, int RM, int RN, bool GATED, bool WHOLE>
 __global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per_eu(GM * GN / 4, GM * GN / 4)))
     gemm_wide_kernel(const bf16* __restrict__ a, int lda, int n, int k, const uint4* __restrict__ wt, int ktiles, int m,
                      const float* __restrict__ bias, void* __restrict__ out, int ldo, int out_f32, int accumulate, int pieces,
-                     int ksplit, int tiles_x, int tiles_y, int by_die) {
+                     TileOrder order) {
   using S = WideShape<GM, GN, RM, RN>;
   constexpr int WL = S::kWLoads, XL = S::kXLoads;
   __shared__ u32x4 mem[S::kLds / 16];
   const int tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int wm = wave / GN, wn = wave % GN;
-  int tile_x, tile_y;
-  if (!big_tile(tiles_x, tiles_y, by_die, tile_x, tile_y)) return;
+  int tile_x, tile_y, share;
+  if (!big_tile(order, tile_x, tile_y, share)) return;
+  const int ksplit = order.shares;
   const int mb0 = tile_x * S::kTiles, tok0 = tile_y * (32 * GN * RN);
   // blocks of 16 weight rows; a gated weight has two per 16 output rows
   const int mblocks = (GATED ? 2 : 1) * ((m + 15) / 16);
   // this share's stages of k; the last stage of k may be half a one
   const int all = (ktiles + 1) / 2;
-  const int first = static_cast<int>(static_cast<long long>(all) * blockIdx.y / ksplit);
-  const int stages = static_cast<int>(static_cast<long long>(all) * (blockIdx.y + 1) / ksplit) - first;
+  const int first = static_cast<int>(static_cast<long long>(all) * share / ksplit);
+  const int stages = static_cast<int>(static_cast<long long>(all) * (share + 1) / ksplit) - first;
   if (stages == 0) {  // more shares than stages: zeros
-    float* o = static_cast<float*>(out) + static_cast<size_t>(blockIdx.y) * n * ldo;
+    float* o = static_cast<float*>(out) + static_cast<size_t>(share) * n * ldo;
     for (int i = tid; i < 32 * GN * RN * 16 * S::kTiles; i += S::kWaves * kWave) {
       const int token = tok0 + i / (16 * S::kTiles), row = mb0 * 16 + i % (16 * S::kTiles);
       if (token < n && row < m) o[static_cast<size_t>(token) * ldo + row] = 0.f;
@@ -77,7 +78,7 @@ __global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per
   constexpr int kRows = (GATED ? 16 : 32) * RM;  // output rows of a wavefront
   const int half = lane / 32, j = lane % 32;
   const int row0 = (GATED ? mb0 / 2 : mb0) * 16 + wm * kRows, tok = tok0 + wn * RN * 32;
-  const size_t plane = static_cast<size_t>(blockIdx.y) * n;
+  const size_t plane = static_cast<size_t>(share) * n;
   if (row0 >= m) return;  // (no barrier follows)
   char* mine = reinterpret_cast<char*>(&mem[0]) + wave * (32 * (32 * RM * 4 + 16));
   if constexpr (WHOLE) {
@@ -264,11 +265,11 @@ __global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per
   }
 }
 
-// The least time that the dies' fetches take, at 7 TB/s, where tiles are taken in plain order (big_grid): each die then needs most
-// operands of every share.  896 x 18944 at 2,048 tokens with its norm: 128 us in three shares of 128 x 192 tiles (8.4 MB a stage),
-// which wide_time() alone prefers, 75 in four of 128 x 256.  One or two rows of tiles read their weights as often in any order; with
-// less than 8,192 of k the shares' start and end weigh more (896 x 4864 at 1,119 tokens in a prompt: 25 us in the three
-// shares of 128 x 128 without this, 31 in the two of 128 x 192 that it would take).
+// The least time that the dies' fetches take, at 7 TB/s, where the tiles' numbers do not divide among the dies: a price of
+// shares that few rows of a long k were given while every eighth tile was a die's (896 x 18944 at 2,048 tokens with its norm: 128 us in
+// three shares of 128 x 192 tiles, which wide_time() alone prefers, 75 in four of 128 x 256).  In runs of neighbours (big_tile) the four
+// take 63 us, three of 128 x 256 77.  With less than 8,192 of k the shares' start and end weigh more (896 x 4864 at 1,119 tokens
+// in a prompt: 25 us in the three shares of 128 x 128 without this, 31 in the two of 128 x 192 that it would take; 19 in runs).
 static double wide_fetch(const WideTile& t, int n, int wblocks, int k) {
   const int tiles_x = (wblocks * 16 + t.rows - 1) / t.rows, tiles_y = (n + t.tokens - 1) / t.tokens;
   if (tiles_y <= 2 || k < 8192) return 0.0;
@@ -360,8 +361,8 @@ static void launch_wide(hipStream_t s, const bf16* a, int lda, int n, int k, con
                         void* out, int ldo, int out_f32, int accumulate, int gated, int ksplit) {
   using S = WideShape<GM, GN, RM, RN>;
   const int tiles_x = (wblocks + S::kTiles - 1) / S::kTiles, tiles_y = (n + 32 * GN * RN - 1) / (32 * GN * RN);
-  int by_die;
-  const unsigned groups = big_grid(tiles_x, tiles_y, 16 * S::kTiles, 32 * GN * RN, &by_die);
+  TileOrder order;
+  const unsigned groups = big_grid(tiles_x, tiles_y, ksplit, 16 * S::kTiles, 32 * GN * RN, S::kLds <= 80 * 1024 ? 512 : 256, &order);
   const int per = out_f32 ? 4 : 8;  // values of 16 bytes
   const int pieces = ldo % per == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
   const bool whole = pieces && m % per == 0 && reinterpret_cast<uintptr_t>(bias) % 16 == 0 &&
@@ -369,8 +370,8 @@ static void launch_wide(hipStream_t s, const bf16* a, int lda, int n, int k, con
   const int ktiles = (k + 31) / 32;
   const auto kernel = gated ? (whole ? gemm_wide_kernel<GM, GN, RM, RN, true, true> : gemm_wide_kernel<GM, GN, RM, RN, true, false>)
                             : (whole ? gemm_wide_kernel<GM, GN, RM, RN, false, true> : gemm_wide_kernel<GM, GN, RM, RN, false, false>);
-  kernel<<<dim3(groups, ksplit), S::kWaves * kWave, 0, s>>>(a, lda, n, k, wt, ktiles, m, bias, out, ldo, out_f32, accumulate, pieces,
-                                                            ksplit, tiles_x, tiles_y, by_die);
+  kernel<<<groups, S::kWaves * kWave, 0, s>>>(a, lda, n, k, wt, ktiles, m, bias, out, ldo, out_f32, accumulate, pieces,
+                                                            order);
 }
 
 void wide_product(hipStream_t s, const bf16* a, int lda, int n, int k, const uint4* wt, int m, const float* bias, void* out,
