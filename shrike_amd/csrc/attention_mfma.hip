@@ -18,6 +18,8 @@
 // in a fixed order.  Head sizes: multiples of 32 up to 256; page sizes:
 // multiples of 16; up to 16 query heads per key/value head.  Other shapes are
 // served by the general kernel.
+#include <type_traits>
+
 #include "api.h"
 #include "attention_rows.h"
 #include "common.h"
@@ -287,11 +289,20 @@ __device__ __forceinline__ void attend_tile(const TileArgs& ta, const AFrag (&qf
 
 // ------------------------------------------------------------------- decode
 // grid (kv_heads, sequences, splits), WAVES wavefronts per workgroup.  A
-// single wavefront needs about 1,700 cycles for a chunk of 32 keys whatever the
+// single wavefront needs some 0.6 us for a chunk of 32 keys of 128 elements whatever the
 // memory does, so a workgroup's key range is dealt out to its wavefronts chunk
 // by chunk, and their results are combined through LDS before anything is
 // written.  Four wavefronts, or eight for up to 512 keys of a short context
 // that would else be two splits (the caller's rule).
+//
+// What bounds it is that chain of instructions; loads through LDS in whole lines, with twice as much on the way, were slower (one
+// sequence of 2,048 keys, 28 heads over 4, unsplit: 18.8 us in registers, 21.0).  What shortened it, keys cold, us before and now: the
+// wavefronts' results added by all of them, each its part of the elements, not all by the first; a chunk's pages asked for while
+// the chunk before is fetched; PAGE = 16: a page's size known when this is compiled, so that a chunk's loads share one address (100
+// instructions of 200 form addresses else).  One sequence of 2,048 keys 18.8 -> 15.5, 4 of 500 to 700 10.2 -> 8.2, 64 of 61 to 1,203 21.9 -> 20.6;
+// 14 heads of 64 over 2: one of 333 in eight wavefronts 5.5 -> 4.7, of 2,000 14.2 -> 10.0, 16 of 200 to 900 9.2 -> 6.9, 64 of 40 to 140 5.8 ->
+// 4.9.  The last workgroup of a sequence's splits joining them in the same launch, through agent-scope stores and a counter, took 0.5 to 1 us
+// more than the second kernel.
 //
 // The two products are formed transposed, so that a lane owns one query head
 // throughout and nothing passes through LDS:
@@ -318,22 +329,23 @@ struct DecodeChunk {
   AFrag v[D / 16];
 };
 
-template <int D, bool NT, int WAVES>
+template <int D, bool NT, int WAVES, int PAGE>
 __global__ void __launch_bounds__(WAVES* kWave)
     attention_decode_kernel(const bf16* __restrict__ q, int q_stride, bf16* __restrict__ out,
                             int heads, int kv_heads, const int32_t* __restrict__ positions,
                             const int32_t* __restrict__ tables, int table_stride,
                             const bf16* __restrict__ k_pool, const bf16* __restrict__ v_pool,
-                            int page_size, uint32_t page_magic, int window, int block, float scale,
+                            int any_page_size, uint32_t page_magic, int window, int block, float scale,
                             float* __restrict__ partial, int nsplit, ScoreOpts so) {
   constexpr int NBUF = 2;  // chunk buffers: one computed, one in flight
   constexpr int kStep = 32 * WAVES;  // keys between two chunks of one wavefront
   __shared__ float m_lds[WAVES][16], l_lds[WAVES][16];
-  __shared__ float4 o_lds[WAVES - 1][D / 16][kWave];
+  __shared__ float4 o_lds[WAVES][D / 16][kWave];
   const int kvh = blockIdx.x, seq = blockIdx.y, z = blockIdx.z;
-  const int wave = threadIdx.x / kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int lane = threadIdx.x % kWave, j = lane % 16, g = lane / 16;
   const int group = heads / kv_heads;
+  const int page_size = PAGE ? PAGE : any_page_size;
   const PageDiv pd{page_size, page_magic};
   // decode sequences come first in the step: token index == sequence index
   const int pos = positions[seq];
@@ -369,41 +381,44 @@ __global__ void __launch_bounds__(WAVES* kWave)
     // what of a load's address belongs to the lane: its row inside a half chunk
     // of 16 keys and whether it reads the first or the second half
     const bool k_second = j >= 8;
-    int k_lane[2];
-#pragma unroll
-    for (int t = 0; t < 2; ++t) k_lane[t] = (8 * ((j / 4) % 2) + 4 * t + j % 4) * 32 + g * 8;
+    const int k_lane = (8 * ((j / 4) % 2) + j % 4) * 32 + g * 8;  // (+ 4 * 32 for the second tile)
     const bool v_second = g >= 2;
     const int v_lane = j * page_size + 8 * (g % 2);
     const size_t head_elems = static_cast<size_t>(page_size) * D;  // one kv head of one page
 
-    auto fetch = [&](DecodeChunk<D>& c, int kb) {
-      // pages of the two halves (wave-uniform), clamped into the range the sequence holds
+    // Pages of a chunk's two halves (wave-uniform), clamped into the range the sequence holds: scalar loads, which are counted apart
+    // from the vector loads in flight, asked for a chunk before they are needed.
+    struct Pages {
+      int a, c;
+    };
+    auto find = [&](int kb) {
       int ka = kb < lo ? lo : kb, kc = kb + 16 < lo ? lo : kb + 16;
       ka = ka > pos ? pos : ka;
       kc = kc > pos ? pos : kc;
-      // scalar loads: they are counted apart from the vector loads in flight
-      const int page_a = table[__builtin_amdgcn_readfirstlane(pd.div(ka))];
-      const int page_c = table[__builtin_amdgcn_readfirstlane(pd.div(kc))];
-      const size_t head_a = (static_cast<size_t>(page_a) * kv_heads + kvh) * head_elems;
-      const size_t head_c = (static_cast<size_t>(page_c) * kv_heads + kvh) * head_elems;
-      const int slot_a = pd.mod(kb), slot_c = pd.mod(kb + 16);
+      return Pages{table[__builtin_amdgcn_readfirstlane(PAGE ? ka / (PAGE ? PAGE : 1) : pd.div(ka))],
+                   table[__builtin_amdgcn_readfirstlane(PAGE ? kc / (PAGE ? PAGE : 1) : pd.div(kc))]};
+    };
+    auto fetch = [&](DecodeChunk<D>& c, int kb, const Pages& pages) {
+      const size_t head_a = (static_cast<size_t>(pages.a) * kv_heads + kvh) * head_elems;
+      const size_t head_c = (static_cast<size_t>(pages.c) * kv_heads + kvh) * head_elems;
+      // (a chunk begins at a multiple of 32: pages of 16 hold a half each)
+      const int slot_a = PAGE == 16 ? 0 : pd.mod(kb), slot_c = PAGE == 16 ? 0 : pd.mod(kb + 16);
       // keys lie in slabs of 32 elements, [D / 32][page_size][32]
       const bf16* krow = k_pool + (k_second ? head_c + static_cast<size_t>(slot_c) * 32
-                                            : head_a + static_cast<size_t>(slot_a) * 32);
+                                            : head_a + static_cast<size_t>(slot_a) * 32) + k_lane;
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int ds = 0; ds < D / 32; ++ds)
-          c.k[t][ds].v = NT ? __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(
-                                  krow + k_lane[t] + static_cast<size_t>(ds) * page_size * 32))
-                            : *reinterpret_cast<const bf16x8*>(krow + k_lane[t] +
-                                                              static_cast<size_t>(ds) * page_size * 32);
+        for (int ds = 0; ds < D / 32; ++ds) {
+          const bf16x8* from = reinterpret_cast<const bf16x8*>(krow + t * 128 + ds * page_size * 32);
+          c.k[t][ds].v = NT ? __builtin_nontemporal_load(from) : *from;
+        }
       const bf16* vcol = v_pool + (v_second ? head_c + slot_c : head_a + slot_a) + v_lane;
 #pragma unroll
-      for (int db = 0; db < D / 16; ++db)
-        c.v[db].v = NT ? __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(
-                             vcol + static_cast<size_t>(db) * 16 * page_size))
-                       : *reinterpret_cast<const bf16x8*>(vcol + static_cast<size_t>(db) * 16 * page_size);
+      for (int db = 0; db < D / 16; ++db) {
+        const bf16x8* from = reinterpret_cast<const bf16x8*>(vcol + db * 16 * page_size);
+        c.v[db].v = NT ? __builtin_nontemporal_load(from) : *from;
+      }
     };
 
     auto attend_chunk = [&](const DecodeChunk<D>& c, int kb, auto edge_tag) {
@@ -491,18 +506,17 @@ __global__ void __launch_bounds__(WAVES* kWave)
     // without loads would make the compiler wait for all loads in flight at each step.
     const int last_kb = key_begin + (key_end - 1 - key_begin) / kStep * kStep;
     DecodeChunk<D> buf[NBUF];
-#pragma unroll
-    for (int u = 0; u < NBUF - 1; ++u) {
-      const int kb = key_begin + kStep * u;
-      fetch(buf[u], kb < last_kb ? kb : last_kb);
-    }
+    auto clamped = [&](int kb) { return kb < last_kb ? kb : last_kb; };
+    static_assert(NBUF == 2, "the pages of one chunk are on the way");
+    fetch(buf[0], key_begin, find(key_begin));
+    Pages next = find(clamped(key_begin + kStep));
     for (int kb0 = key_begin; kb0 < key_end; kb0 += kStep * NBUF) {
 #pragma unroll
       for (int u = 0; u < NBUF; ++u) {
         const int kb = kb0 + kStep * u;
         if (kb >= key_end) break;
-        const int ahead = kb + kStep * (NBUF - 1);
-        fetch(buf[(u + NBUF - 1) % NBUF], ahead < last_kb ? ahead : last_kb);
+        fetch(buf[(u + 1) % NBUF], clamped(kb + kStep), next);
+        next = find(clamped(kb + 2 * kStep));
         attend(buf[u], kb);
       }
     }
@@ -526,48 +540,45 @@ __global__ void __launch_bounds__(WAVES* kWave)
   const float mine = __builtin_amdgcn_exp2f(m - m_ref);
   m = m_all;
 #pragma unroll
-  for (int db = 0; db < D / 16; ++db) o[db] *= mine;
-  if (wave > 0) {
-#pragma unroll
-    for (int db = 0; db < D / 16; ++db)
-      o_lds[wave - 1][db][lane] = make_float4(o[db][0], o[db][1], o[db][2], o[db][3]);
-  }
+  for (int db = 0; db < D / 16; ++db)
+    o_lds[wave][db][lane] = make_float4(o[db][0] * mine, o[db][1] * mine, o[db][2] * mine, o[db][3] * mine);
   __syncthreads();
-  if (wave > 0 || j >= group) return;
-#pragma unroll
-  for (int w = 0; w < WAVES - 1; ++w)
-#pragma unroll
-    for (int db = 0; db < D / 16; ++db) {
-      const float4 x = o_lds[w][db][lane];
-      o[db][0] += x.x;
-      o[db][1] += x.y;
-      o[db][2] += x.z;
-      o[db][3] += x.w;
-    }
-
+  if (j >= group) return;
   const int head = kvh * group + j;
+  // each wavefront finishes the elements db * 16 + 4 * g .. + 3 of its own db
+  auto each = [&](auto leave) {
+#pragma unroll
+    for (int i = 0; i < (D / 16 + WAVES - 1) / WAVES; ++i) {
+      const int db = wave + i * WAVES;
+      if (D / 16 % WAVES && db >= D / 16) break;
+      float4 v = o_lds[0][db][lane];
+#pragma unroll
+      for (int w = 1; w < WAVES; ++w) {
+        const float4 x = o_lds[w][db][lane];
+        v.x += x.x, v.y += x.y, v.z += x.z, v.w += x.w;
+      }
+      leave(db, v);
+    }
+  };
   if (nsplit == 1) {
-    // the whole range in one wavefront: normalise and write the output row
+    // the whole range in one workgroup: normalise and write the output row
     if (so.sinks) l += __builtin_amdgcn_exp2f(so.sinks[head] * 1.4426950408889634f - m_ref);
     const float inv = 1.f / l;
     bf16* dst = out + (static_cast<size_t>(seq) * heads + head) * D + 4 * g;
-#pragma unroll
-    for (int db = 0; db < D / 16; ++db) {
+    each([&](int db, const float4& v) {
       uint2 packed;
-      packed.x = bf16_bits(o[db][0] * inv) | (static_cast<uint32_t>(bf16_bits(o[db][1] * inv)) << 16);
-      packed.y = bf16_bits(o[db][2] * inv) | (static_cast<uint32_t>(bf16_bits(o[db][3] * inv)) << 16);
+      packed.x = bf16_bits(v.x * inv) | (static_cast<uint32_t>(bf16_bits(v.y * inv)) << 16);
+      packed.y = bf16_bits(v.z * inv) | (static_cast<uint32_t>(bf16_bits(v.w * inv)) << 16);
       *reinterpret_cast<uint2*>(dst + db * 16) = packed;
-    }
+    });
     return;
   }
   // partial: O [seq][head][split][D], then (max, sum) [seq][head][split][2]
   const size_t rows = static_cast<size_t>(gridDim.y) * heads * nsplit;
   const size_t row = (static_cast<size_t>(seq) * heads + head) * nsplit + z;
   float* dst = partial + row * D + 4 * g;
-#pragma unroll
-  for (int db = 0; db < D / 16; ++db)
-    *reinterpret_cast<float4*>(dst + db * 16) = make_float4(o[db][0], o[db][1], o[db][2], o[db][3]);
-  if (g == 0) *reinterpret_cast<float2*>(partial + rows * D + row * 2) = make_float2(m, l);
+  each([&](int db, const float4& v) { *reinterpret_cast<float4*>(dst + db * 16) = v; });
+  if (wave == 0 && g == 0) *reinterpret_cast<float2*>(partial + rows * D + row * 2) = make_float2(m, l);
 }
 
 // out[seq][head][:] = sum_z 2^(m_z - M) O_z / sum_z 2^(m_z - M) l_z, splits in
@@ -1003,9 +1014,13 @@ static void launch_decode(dim3 grid, hipStream_t s, const bf16* q, int q_stride,
                           int window, int block, float scale, float* partial, int nsplit, int streaming,
                           int waves, ScoreOpts so) {
   const uint32_t magic = static_cast<uint32_t>(((1ull << 32) + page_size - 1) / page_size);
-  auto kernel = streaming ? attention_decode_kernel<D, true, 4> : attention_decode_kernel<D, false, 4>;
-  if constexpr (D <= 64)
-    if (waves == 8) kernel = attention_decode_kernel<D, false, 8>;  // (contexts too short to stream)
+  const auto pick = [&](auto page) {
+    constexpr int P = decltype(page)::value;
+    if constexpr (D <= 64)
+      if (waves == 8) return attention_decode_kernel<D, false, 8, P>;  // (contexts too short to stream)
+    return streaming ? attention_decode_kernel<D, true, 4, P> : attention_decode_kernel<D, false, 4, P>;
+  };
+  const auto kernel = page_size == 16 ? pick(std::integral_constant<int, 16>{}) : pick(std::integral_constant<int, 0>{});
   kernel<<<grid, waves * kWave, 0, s>>>(q, q_stride, out, heads, kv_heads, positions, tables, table_stride, k_pool, v_pool,
                                         page_size, magic, window, block, scale, partial, nsplit, so);
   if (nsplit > 1)
