@@ -27,6 +27,8 @@
 #include "common.h"
 #include "gemm_wide.h"
 
+#include <type_traits>
+
 namespace shk {
 
 typedef float mf4 __attribute__((ext_vector_type(4)));
@@ -228,22 +230,44 @@ __global__ void __launch_bounds__(kWave * KW * MW * NW)
   }
 }
 
+struct F32Product {
+  const float *a, *w, *bias;
+  float* out;
+  int n, m, k, lda, ldo, accumulate, batch;
+  long long a_batch, w_batch, out_batch;
+};
+
 // The same product, in the same order, for up to 16 rows, tiled weights and a k in whole steps of 16.  A workgroup's KW
 // wavefronts take a segment each (16), a group each (4), or with GROUPS the segments of the group blockIdx.y, whose sum is then
 // one of four parts [group][n][m] that the reader adds in order.  C > 0: a wavefront has at most C steps, all asked for at
 // once; 0: batches of five, two in flight.  ROWS = 8: a workgroup for half a block of features, where whole blocks leave
 // compute units idle.  GATED: w holds a gate matrix and behind it the other factor, m rows each (a multiple of 16); a workgroup
 // forms a block of both and stores what act_mul_kernel would of the two.
-// What bounds it: one round trip to memory and what a compute unit takes in (about 50 GB/s a workgroup).  Weights cold, us at 1 /
-// 4 / 16 rows: 896 x 896 4.8 / 5.0 / 6.4 in the kernel above, 3.7 / 3.8 / 4.9 here, 9728 x 896 11.1 / 10.5 / 13.0 and 8.6 / 8.7 / 11.4,
+// What bounds it: one round trip to memory, then the matrix instructions (32 cycles each, 16 columns for however few rows).  Weights cold, us at 1 /
+// 4 / 16 rows: 896 x 896 4.8 / 5.0 / 6.4 in the kernel above, 3.8 / 3.9 / 4.5 here, 9728 x 896 11.1 / 10.5 / 13.0 and 8.8 / 8.9 / 10.2,
 // 3584 x 3584 28 / 29 / 39 and 12 / 12 / 15.
-template <int KW, int ROWS, int C, bool GATED, bool GROUPS>
+// A wavefront's part of the rows is loaded in whole lines and handed to the lanes that multiply it through LDS, in a place of the wavefront's own:
+// straight from memory neighbouring lanes lie on different rows, which a compute unit takes in at a quarter of its rate.  At 4 / 8 / 16 rows: 1152 x 896
+// 4.1 / 4.4 / 5.1 -> 4.0 / 4.1 / 4.5, gate and up of 4864 x 896 10.2 / 10.8 / 12.5 -> 10.0 / 10.3 / 11.4, 896 x 4864 in groups 7.7 / 8.1 / 10.4 -> 7.1 / 7.6 /
+// 9.1.  Not where a wavefront walks a group in batches (C = 0, whole): 3584 x 18944 at 4 / 9 50.5 / 51.5 -> 52.0 / 59.2.
+// NR: rows that a wavefront holds in LDS (at least n), 0: none.
+template <int KW, int ROWS, int C, bool GATED, bool GROUPS, int NR>
+struct F32Few {
+  static constexpr int kBlocks = GATED ? 2 : 1, kSteps = C > 0 ? C : 5, kParts = kSteps > 6 ? 2 : 1, kHeld = kSteps / kParts;
+  static constexpr int kPieces = 4 * kHeld, kPitch = kPieces + 1;  // 16 bytes each: of a row in the steps held at a time; with a place beside them
+  static constexpr int kRegion = NR * kPitch > kBlocks * kWave ? NR * kPitch : kBlocks * kWave;  // of a wavefront: its rows, then its sums
+  static constexpr int kLds = KW * kRegion * 16;
+  static_assert(kLds <= 160 * 1024 && kHeld * kParts == kSteps);
+};
+template <int KW, int ROWS, int C, bool GATED, bool GROUPS, int NR>
 __global__ void __launch_bounds__(kWave* KW)
     gemm_f32_few_kernel(const float* __restrict__ a, const float* __restrict__ w, const float* __restrict__ bias,
                         float* __restrict__ out, int n, int m, int k, int lda, int ldo, int accumulate, F32Gate gate) {
-  constexpr int RB = GATED ? 2 : 1, kMine = GROUPS ? 1 : kF32Segments / KW, kSteps = C > 0 ? C : 5;
+  using F = F32Few<KW, ROWS, C, GATED, GROUPS, NR>;
+  constexpr int RB = F::kBlocks, kMine = GROUPS ? 1 : kF32Segments / KW, kSteps = F::kSteps, kHeld = F::kHeld;
+  constexpr int kLoads = NR ? (NR * F::kPieces + kWave - 1) / kWave : kHeld;  // of a wavefront's rows, for the steps held at a time
   static_assert(!GROUPS || (KW == kF32Group && !GATED), "a workgroup holds one group");
-  __shared__ mf4 sums[KW][RB][kWave];
+  extern __shared__ mf4 mem[];  // [KW][kRegion]
   const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int i = lane % 16, kg = lane / 16;
   const int f = blockIdx.x * ROWS + i % ROWS, ktiles = k / 16;
@@ -251,7 +275,17 @@ __global__ void __launch_bounds__(kWave* KW)
 #pragma unroll
   for (int r = 0; r < RB; ++r)
     wr[r] = reinterpret_cast<const mf4*>(w) + static_cast<size_t>(f / 16 + r * (m / 16)) * ktiles * kWave + kg * 16 + f % 16;
-  const float* ar = a + static_cast<size_t>(min(i, n - 1)) * lda + kg * 4;
+  // the rows' pieces that this lane loads, for whichever lane multiplies them
+  mf4* held = mem + wave * F::kRegion;
+  const float* ar[kLoads];
+  int ahead[kLoads], place[kLoads];
+#pragma unroll
+  for (int t = 0; t < kLoads; ++t) {
+    const int at = min(lane + t * kWave, NR * F::kPieces - 1), row = NR ? at / F::kPieces : i, piece = NR ? at % F::kPieces : 4 * t + kg;
+    ar[t] = a + static_cast<size_t>(min(row, n - 1)) * lda + piece % 4 * 4;
+    ahead[t] = piece / 4, place[t] = row * F::kPitch + piece;
+  }
+  const mf4* mine = held + (NR ? min(i, min(n, NR) - 1) * F::kPitch + kg : 0);
 
   const int seg_steps = (k + 16 * kF32Segments - 1) / (16 * kF32Segments);
   const int first = (GROUPS ? blockIdx.y * kF32Group : 0) + wave * kMine;
@@ -260,35 +294,59 @@ __global__ void __launch_bounds__(kWave* KW)
 #pragma unroll
   for (int r = 0; r < RB; ++r) acc[r] = group[r] = mf4{0.f, 0.f, 0.f, 0.f};
   struct Batch {
-    mf4 w[kSteps][RB], a[kSteps];
+    mf4 w[kSteps][RB], a[F::kParts][kLoads];
   };
   auto load = [&](Batch& b, int s0) {  // (unconditional: a step beyond the last is the matrix's last)
+#pragma unroll
+    for (int part = 0; part < F::kParts; ++part)
+#pragma unroll
+      for (int t = 0; t < kLoads; ++t)
+        b.a[part][t] = *reinterpret_cast<const mf4*>(ar[t] + min(begin + s0 + part * kHeld + ahead[t], ktiles - 1) * 16);
 #pragma unroll
     for (int u = 0; u < kSteps; ++u) {
       const int s = min(begin + s0 + u, ktiles - 1);
 #pragma unroll
       for (int r = 0; r < RB; ++r) b.w[u][r] = __builtin_nontemporal_load(wr[r] + static_cast<size_t>(s) * kWave);
-      b.a[u] = *reinterpret_cast<const mf4*>(ar + s * 16);
     }
     __builtin_amdgcn_sched_barrier(0);
   };
   int in_seg = 0;
   auto multiply = [&](const Batch& b, int s0) {
 #pragma unroll
-    for (int u = 0; u < kSteps; ++u) {
-      // (beyond the last step: zeros times zeros, which leave a sum that began at zero as it is; a branch would take
-      // the loads with it)
-      const bool have = s0 + u < steps;
+    for (int part = 0; part < F::kParts; ++part) {
+      mf4 av[kHeld];
+      if constexpr (NR > 0) {
+        // (the wavefront's own place: its lanes' writes and reads are in order)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float x = have ? b.a[u][j] : 0.f;
+        for (int t = 0; t < kLoads; ++t) held[place[t]] = b.a[part][t];
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
-        for (int r = 0; r < RB; ++r) acc[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(have ? b.w[u][r][j] : 0.f, x, acc[r], 0, 0, 0);
+        for (int u = 0; u < kHeld; ++u) av[u] = mine[u * 4];
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+      } else {
+#pragma unroll
+        for (int u = 0; u < kHeld; ++u) av[u] = b.a[part][u];
       }
-      if (kMine > 1 && ++in_seg == seg_steps) {  // a segment ends
-        in_seg = 0;
 #pragma unroll
-        for (int r = 0; r < RB; ++r) group[r] += acc[r], acc[r] = mf4{0.f, 0.f, 0.f, 0.f};
+      for (int x = 0; x < kHeld; ++x) {
+        const int u = part * kHeld + x;
+        // (beyond the last step: zeros times zeros, which leave a sum that began at zero as it is; a branch would take
+        // the loads with it)
+        const bool have = s0 + u < steps;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float v = have ? av[x][j] : 0.f;
+#pragma unroll
+          for (int r = 0; r < RB; ++r) acc[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(have ? b.w[u][r][j] : 0.f, v, acc[r], 0, 0, 0);
+        }
+        if (kMine > 1 && ++in_seg == seg_steps) {  // a segment ends
+          in_seg = 0;
+#pragma unroll
+          for (int r = 0; r < RB; ++r) group[r] += acc[r], acc[r] = mf4{0.f, 0.f, 0.f, 0.f};
+        }
       }
     }
   };
@@ -306,7 +364,7 @@ __global__ void __launch_bounds__(kWave* KW)
     }
   }
 #pragma unroll
-  for (int r = 0; r < RB; ++r) sums[wave][r][lane] = kMine > 1 ? group[r] + acc[r] : acc[r];
+  for (int r = 0; r < RB; ++r) held[r * kWave + lane] = kMine > 1 ? group[r] + acc[r] : acc[r];
   __syncthreads();
   // element (feature, row): the wavefronts' shares in order
   const int row = threadIdx.x / ROWS, at = threadIdx.x % ROWS, col = blockIdx.x * ROWS + at;
@@ -314,8 +372,8 @@ __global__ void __launch_bounds__(kWave* KW)
   float v[RB];
 #pragma unroll
   for (int r = 0; r < RB; ++r) {
-    const float* p = reinterpret_cast<const float*>(&sums[0][r][at / 4 * 16 + row]) + at % 4;
-    constexpr int kNext = RB * kWave * 4;
+    const float* p = reinterpret_cast<const float*>(mem + r * kWave + at / 4 * 16 + row) + at % 4;
+    constexpr int kNext = F::kRegion * 4;
     v[r] = 0.f;
     if (KW > 4) {
 #pragma unroll
@@ -336,6 +394,27 @@ __global__ void __launch_bounds__(kWave* KW)
   } else {
     if (bias) v[0] += bias[col];
     *dst = accumulate ? v[0] + *dst : v[0];
+  }
+}
+
+template <int KW, int ROWS, int C, bool GATED, bool GROUPS>
+static void run_f32_few(const F32Product& p, hipStream_t s, F32Gate gate = F32Gate{}) {
+  const auto go = [&](auto kernel, int lds) {
+    if (lds > 65536) hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    kernel<<<dim3((p.m + ROWS - 1) / ROWS, GROUPS ? kF32Segments / kF32Group : 1), KW * kWave, lds, s>>>(p.a, p.w, p.bias, p.out, p.n, p.m, p.k, p.lda, p.ldo,
+                                                                                                        p.accumulate, gate);
+  };
+  const auto rows = [&](auto r) {
+    using F = F32Few<KW, ROWS, C, GATED, GROUPS, r.value>;
+    go(gemm_f32_few_kernel<KW, ROWS, C, GATED, GROUPS, r.value>, F::kLds);
+  };
+  if constexpr (C == 0 && !GROUPS) {
+    rows(std::integral_constant<int, 0>{});
+  } else {
+    if (p.n <= 4) rows(std::integral_constant<int, 4>{});
+    else if (p.n <= 8) rows(std::integral_constant<int, 8>{});
+    else if (p.n <= 12) rows(std::integral_constant<int, 12>{});
+    else rows(std::integral_constant<int, 16>{});
   }
 }
 
@@ -499,13 +578,6 @@ __global__ void __launch_bounds__(4 * kWave)
   }
 }
 
-struct F32Product {
-  const float *a, *w, *bias;
-  float* out;
-  int n, m, k, lda, ldo, accumulate, batch;
-  long long a_batch, w_batch, out_batch;
-};
-
 template <int RT, int CT, int KW, int MW, int NW, int U, bool TILED>
 static void launch_f32(const F32Product& p, hipStream_t s) {
   constexpr int F = 16 * RT * MW, T = 16 * CT * NW;
@@ -548,19 +620,17 @@ static bool f32_few(int n, int m, int k) {
 // a wavefront: 9728 x 896 at 4 rows 8.7 us by segments, 10.0 by groups, 3584 x 3584 15.5 and 12.2, 3584 x 18944 at 16 rows 70 and 61.
 static void launch_f32_few(const F32Product& p, hipStream_t s) {
   const int seg_steps = (p.k + 16 * kF32Segments - 1) / (16 * kF32Segments);
-  const auto go = [&](auto kernel, int waves, int rows) {
-    kernel<<<(p.m + rows - 1) / rows, waves * kWave, 0, s>>>(p.a, p.w, p.bias, p.out, p.n, p.m, p.k, p.lda, p.ldo, p.accumulate, F32Gate{});
-  };
-  if (p.m <= 2048)  // (a k of up to 2,560: ten steps)
-    go(seg_steps <= 2   ? gemm_f32_few_kernel<16, 8, 2, false, false>
-       : seg_steps <= 4 ? gemm_f32_few_kernel<16, 8, 4, false, false>
-       : seg_steps <= 6 ? gemm_f32_few_kernel<16, 8, 6, false, false>
-                        : gemm_f32_few_kernel<16, 8, 10, false, false>,
-       16, 8);
-  else if (p.k <= 1024)  // (four steps)
-    go(seg_steps <= 2 ? gemm_f32_few_kernel<16, 16, 2, false, false> : gemm_f32_few_kernel<16, 16, 4, false, false>, 16, 16);
-  else
-    go(gemm_f32_few_kernel<4, 16, 0, false, false>, 4, 16);
+  if (p.m <= 2048) {  // (a k of up to 2,560: ten steps)
+    if (seg_steps <= 2) run_f32_few<16, 8, 2, false, false>(p, s);
+    else if (seg_steps <= 4) run_f32_few<16, 8, 4, false, false>(p, s);
+    else if (seg_steps <= 6) run_f32_few<16, 8, 6, false, false>(p, s);
+    else run_f32_few<16, 8, 10, false, false>(p, s);
+  } else if (p.k <= 1024) {  // (four steps)
+    if (seg_steps <= 2) run_f32_few<16, 16, 2, false, false>(p, s);
+    else run_f32_few<16, 16, 4, false, false>(p, s);
+  } else {
+    run_f32_few<4, 16, 0, false, false>(p, s);
+  }
 }
 
 // The shape of the kernel for a size (results are the same bits in all of them).  Measured on the 0.5B
@@ -697,8 +767,8 @@ extern "C" int shk_gemm_f32_groups(const void* a, const void* wt, void* out, int
   const F32Product p{static_cast<const float*>(a), static_cast<const float*>(wt), nullptr, static_cast<float*>(out), n, m, k, lda, m, 0, 1, 0, 0, 0};
   const hipStream_t s = static_cast<hipStream_t>(stream);
   if (n <= 16) {  // (ten steps a segment are asked for at once, which is a k of 2,560)
-    const auto kernel = k <= 2560 ? gemm_f32_few_kernel<4, 8, 10, false, true> : gemm_f32_few_kernel<4, 8, 0, false, true>;
-    kernel<<<dim3((m + 7) / 8, kF32Segments / kF32Group), 4 * kWave, 0, s>>>(p.a, p.w, nullptr, p.out, n, m, k, lda, m, 0, F32Gate{});
+    if (k <= 2560) run_f32_few<4, 8, 10, false, true>(p, s);
+    else run_f32_few<4, 8, 0, false, true>(p, s);
   } else {
     launch_f32_lds<1, 2, false, true>(p, s);
   }
@@ -754,14 +824,11 @@ extern "C" int shk_gemm_f32_gated(const void* a, const void* wt, void* out, int 
     SHK_LAUNCH_CHECK("gemm_f32_gated");
     return 0;
   }
-  const auto go = [&](auto kernel, int waves) {
-    kernel<<<m / 16, waves * kWave, 0, static_cast<hipStream_t>(stream)>>>(static_cast<const float*>(a), static_cast<const float*>(wt), nullptr,
-                                                                           static_cast<float*>(out), n, m, k, lda, m, 0, gate);
-  };
-  if (k <= 1024)  // (up to four steps a segment)
-    go(seg_steps <= 2 ? gemm_f32_few_kernel<16, 16, 2, true, false> : gemm_f32_few_kernel<16, 16, 4, true, false>, 16);
-  else
-    go(gemm_f32_few_kernel<4, 16, 0, true, false>, 4);
+  const F32Product p{static_cast<const float*>(a), static_cast<const float*>(wt), nullptr, static_cast<float*>(out), n, m, k, lda, m, 0, 1, 0, 0, 0};
+  const hipStream_t few = static_cast<hipStream_t>(stream);
+  if (k > 1024) run_f32_few<4, 16, 0, true, false>(p, few, gate);
+  else if (seg_steps <= 2) run_f32_few<16, 16, 2, true, false>(p, few, gate);
+  else run_f32_few<16, 16, 4, true, false>(p, few, gate);  // (up to four steps a segment)
   SHK_LAUNCH_CHECK("gemm_f32_gated");
   return 0;
 }
