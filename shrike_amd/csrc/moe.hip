@@ -31,6 +31,8 @@
 #include "common.h"
 #include "gemm_wide.h"
 
+#include <type_traits>
+
 namespace shk {
 
 // kMaxExpertsPerLane: 1 for up to 64 outputs, 8 for up to 512.
@@ -594,8 +596,8 @@ __global__ void __launch_bounds__(256)
 // p / 8-th tile of die p % 8's share of all live tiles, counted expert by expert, features outside, the
 // expert's pairs inside, so that the 32 compute units of a die read a matrix from memory once and its pairs'
 // rows stay in the die's L2.
-// What bounds it: as the loop, the multiplications' power limit, and the pairs that a list's last tile lacks.  1,501 tokens, two of
-// eight experts of 4736 features and width 3584: gate/up 232 us, down 101 (262 and 157 with 16 x 16 multiplications and
+// What bounds it: as the loop, the multiplications' power limit, the pairs that a list's last tile lacks, and the last round.  1,501 tokens, two of
+// eight experts of 4736 features and width 3584: gate/up 213 us, down 99 (262 and 157 with 16 x 16 multiplications and
 // a pair's row per lane; 360 and 227 in the kernel above; with row-major weights that loop took 350 and 213).  Pairs'
 // rows laid out in tiles first (19 us a layer) changed nothing, nor did leaving out the multiplications
 // for the empty half of a list's last tile.
@@ -629,30 +631,23 @@ __device__ __forceinline__ bool moe_tile(const int32_t* counts, int experts, int
   return false;
 }
 
+constexpr int kDieRound = 32;  // workgroups at a time on a die: one a compute unit
 enum MoeProduct : int { kMoeGated = 0, kMoeSingle = 1, kMoeDown = 2 };
 
+// One tile of 32 * GM * RM weight rows x 32 * GN * RN pairs of expert e: features f0 and on, the pairs of its list from row0 on.
 template <int PRODUCT, int GM, int GN, int RM, int RN>
-__global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per_eu(GM * GN / 4, GM * GN / 4)))
-    moe_big_mfma_kernel(const bf16* __restrict__ a, const int32_t* __restrict__ order,
-                        const int32_t* __restrict__ counts, const bf16* __restrict__ w0, const bf16* __restrict__ w1,
-                        bf16* __restrict__ act_out, float* __restrict__ pair_out, int n, int k, int m, int experts, int top,
-                        GateForm form) {
+__device__ __forceinline__ void moe_big_tile(u32x4* mem, int* pairs, int e, int f0, int row0, int count, const bf16* __restrict__ a,
+                                             const int32_t* __restrict__ list, const bf16* __restrict__ w0,
+                                             const bf16* __restrict__ w1, bf16* __restrict__ act_out,
+                                             float* __restrict__ pair_out, int n, int k, int m, int top, GateForm form) {
   using S = WideShape<GM, GN, RM, RN>;
   constexpr int kRows = 32 * GM * RM, kPairs = 32 * GN * RN, kFeatures = PRODUCT == kMoeGated ? kRows / 2 : kRows;
   static_assert(PRODUCT != kMoeGated || S::kWaves % 2 == 0, "a wavefront loads tiles of one of the two matrices");
-  __shared__ u32x4 mem[S::kLds / 16];
   const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const int features = (m + kFeatures - 1) / kFeatures;
-  int total, e, within, row_tiles;
-  moe_tile<kPairs>(counts, experts, n, features, -1, lane, total, e, within, row_tiles);
-  const int per_die = (total + 7) / 8, turn = blockIdx.x / 8;
-  if (turn >= per_die) return;
-  if (!moe_tile<kPairs>(counts, experts, n, features, blockIdx.x % 8 * per_die + turn, lane, total, e, within, row_tiles)) return;
-  e = __builtin_amdgcn_readfirstlane(e);
-  within = __builtin_amdgcn_readfirstlane(within);
-  row_tiles = __builtin_amdgcn_readfirstlane(row_tiles);
-  const int count = min(counts[e], n), row0 = within % row_tiles * kPairs, f0 = within / row_tiles * kFeatures;
-  const int32_t* list = order + static_cast<size_t>(e) * n;
+  if (threadIdx.x < kPairs) {  // (read behind the loop's barriers)
+    const int at = row0 + threadIdx.x;
+    pairs[threadIdx.x] = at < count ? min(max(list[at], 0), n * top - 1) : -1;
+  }
 
   // What this wavefront loads: weight tiles and units of 8 pairs wave, wave + kWaves, ..; rows beyond either matrix are read as its
   // last (their products are not stored).  Gated: even tiles are the gate's features, odd ones the same features of up.
@@ -675,11 +670,38 @@ __global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per
                         reinterpret_cast<const char*>(a), xoff, 0u, -1, k / 32, k / 64);
 
   // Register g * 4 + r of lane (j, half) of a tile of 32 x 32 holds weight row g * 8 + half * 4 + r for pair j.  32 pairs'
-  // sums at a time go through LDS and leave in 16-byte pieces along the pairs' rows.
+  // sums at a time go through LDS and leave in 16-byte pieces along the pairs' rows, several pieces of a lane at a time: a
+  // wavefront is alone on its SIMD, so one by one every piece waits for all that it asks for.
   constexpr int kMine = kFeatures / GM;  // output features of a wavefront
   constexpr int kPitch = 32 * RM * 4 + 16, kValues = PRODUCT == kMoeDown ? 4 : 8, kPieces = kMine / kValues;
   const int half = lane / 32, j = lane % 32, first = f0 + wave / GN * kMine;
   char* mine = reinterpret_cast<char*>(mem) + wave * 32 * kPitch;
+  auto leave = [&](int jn, auto act) {
+#pragma unroll 4
+    for (int i = 0; i < 32 * kPieces / kWave; ++i) {
+      const int q = i * kWave + lane, t = q / kPieces, row = q % kPieces * kValues, f = first + row;
+      const int pair = pairs[(wave % GN * RN + jn) * 32 + t];
+      const bool stored = pair >= 0 && f < m;  // (m is a multiple of 64: a piece is inside or outside as a whole)
+      const size_t to = static_cast<size_t>(pair) * m + f;
+      const float* sums = reinterpret_cast<const float*>(mine + t * kPitch);
+      if constexpr (PRODUCT == kMoeDown) {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(sums + row);
+        if (stored) *reinterpret_cast<f32x4*>(pair_out + to) = v;
+      } else {
+        const f32x4* gate = reinterpret_cast<const f32x4*>(sums + (PRODUCT == kMoeGated ? row / 16 * 32 + row % 16 : row));
+        constexpr int kApart = PRODUCT == kMoeGated ? 4 : 0;
+        const GateForm same = {decltype(act)::value, form.limit, form.shift};
+        bf16x8 v;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const f32x4 g = gate[h], u = gate[kApart + h];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) v[4 * h + r] = static_cast<__bf16>(gate_times_up(g[r], u[r], same));
+        }
+        if (stored) *reinterpret_cast<bf16x8*>(act_out + to) = v;
+      }
+    }
+  };
 #pragma unroll
   for (int jn = 0; jn < RN; ++jn) {
 #pragma unroll
@@ -689,28 +711,55 @@ __global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per
         *reinterpret_cast<f32x4*>(mine + j * kPitch + (i * 32 + g * 8 + half * 4) * 4) =
             f32x4{acc[i][jn][g * 4], acc[i][jn][g * 4 + 1], acc[i][jn][g * 4 + 2], acc[i][jn][g * 4 + 3]};
     SHK_LDS_DONE();
-#pragma unroll 1
-    for (int q = lane; q < 32 * kPieces; q += kWave) {
-      const int t = q / kPieces, row = q % kPieces * kValues, at = row0 + (wave % GN * RN + jn) * 32 + t, f = first + row;
-      if (at >= count || f >= m) continue;  // (m is a multiple of 64: a piece is inside or outside as a whole)
-      const size_t pair = min(max(list[at], 0), n * top - 1);
-      const float* sums = reinterpret_cast<const float*>(mine + t * kPitch);
-      if (PRODUCT == kMoeDown) {
-        *reinterpret_cast<f32x4*>(pair_out + pair * m + f) = *reinterpret_cast<const f32x4*>(sums + row);
-      } else {
-        const float* gate = sums + (PRODUCT == kMoeGated ? row / 16 * 32 + row % 16 : row);
-        u32x4 v;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int apart = PRODUCT == kMoeGated ? 16 : 0;
-          v[r] = bf16_bits(gate_times_up(gate[2 * r], gate[2 * r + apart], form)) |
-                 static_cast<uint32_t>(bf16_bits(gate_times_up(gate[2 * r + 1], gate[2 * r + 1 + apart], form))) << 16;
-        }
-        *reinterpret_cast<u32x4*>(act_out + pair * m + f) = v;
-      }
-    }
+    if (PRODUCT == kMoeDown)
+      leave(jn, std::integral_constant<int, 0>{});
+    else if (form.act == 4)
+      leave(jn, std::integral_constant<int, 4>{});
+    else if (form.act == 3)
+      leave(jn, std::integral_constant<int, 3>{});
+    else if (form.act == 2)
+      leave(jn, std::integral_constant<int, 2>{});
+    else
+      leave(jn, std::integral_constant<int, 1>{});
     SHK_LDS_DONE();
   }
+}
+
+// Tiles beyond a die's last whole round of 32 that fill no more than half of one run as two halves of their weight rows each, which take
+// little more than half as long: 1,036 tiles of gate and up (1,501 tokens, two of eight experts of 4736 features and width 3584) 231 us ->
+// 213, of five rounds; 999 tiles, four rounds with 29 of 32 compute units in the last, 187 either way.
+template <int PRODUCT, int GM, int GN, int RM, int RN>
+__global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per_eu(GM * GN / 4, GM * GN / 4)))
+    moe_big_mfma_kernel(const bf16* __restrict__ a, const int32_t* __restrict__ order,
+                        const int32_t* __restrict__ counts, const bf16* __restrict__ w0, const bf16* __restrict__ w1,
+                        bf16* __restrict__ act_out, float* __restrict__ pair_out, int n, int k, int m, int experts, int top,
+                        GateForm form) {
+  constexpr int kPairs = 32 * GN * RN, kFeatures = 32 * GM * RM / (PRODUCT == kMoeGated ? 2 : 1);
+  __shared__ u32x4 mem[WideShape<GM, GN, RM, RN>::kLds / 16];
+  __shared__ int pairs[kPairs];  // of the tile; -1: beyond the list
+  const int lane = threadIdx.x % kWave;
+  const int features = (m + kFeatures - 1) / kFeatures;
+  int total, e, within, row_tiles;
+  moe_tile<kPairs>(counts, experts, n, features, -1, lane, total, e, within, row_tiles);
+  total = __builtin_amdgcn_readfirstlane(total);
+  const int die = blockIdx.x % 8, per_die = (total + 7) / 8, first = die * per_die;
+  const int mine = min(per_die, total - first), whole = 2 * (mine % kDieRound) <= kDieRound ? mine / kDieRound * kDieRound : mine;
+  int turn = blockIdx.x / 8, half = 0;
+  const bool halved = turn >= whole;
+  if (halved) half = (turn - whole) % 2, turn = whole + (turn - whole) / 2;
+  if (turn >= mine) return;
+  if (!moe_tile<kPairs>(counts, experts, n, features, first + turn, lane, total, e, within, row_tiles)) return;
+  e = __builtin_amdgcn_readfirstlane(e);
+  within = __builtin_amdgcn_readfirstlane(within);
+  row_tiles = __builtin_amdgcn_readfirstlane(row_tiles);
+  const int count = min(counts[e], n), row0 = within % row_tiles * kPairs;
+  const int f0 = within / row_tiles * kFeatures + half * (kFeatures / 2);
+  if (f0 >= m) return;
+  const int32_t* list = order + static_cast<size_t>(e) * n;
+  if (halved)
+    moe_big_tile<PRODUCT, GM, GN, RM / 2, RN>(mem, pairs, e, f0, row0, count, a, list, w0, w1, act_out, pair_out, n, k, m, top, form);
+  else
+    moe_big_tile<PRODUCT, GM, GN, RM, RN>(mem, pairs, e, f0, row0, count, a, list, w0, w1, act_out, pair_out, n, k, m, top, form);
 }
 
 template <int PRODUCT, int GM, int GN, int RM, int RN>
@@ -719,15 +768,17 @@ static void launch_big(const bf16* a, const int32_t* order, const int32_t* count
   constexpr int kPairs = 32 * GN * RN, kFeatures = 32 * GM * RM / (PRODUCT == kMoeGated ? 2 : 1);
   const long long features = (m + kFeatures - 1) / kFeatures, pairs = static_cast<long long>(n) * top;
   const long long tiles = features * (pairs / kPairs + (experts < pairs ? experts : pairs));  // live ones at most
-  moe_big_mfma_kernel<PRODUCT, GM, GN, RM, RN><<<static_cast<unsigned>((tiles + 7) / 8 * 8), GM * GN * kWave, 0, s>>>(
+  const long long groups = (tiles + 7) / 8 * 8 + 8 * (kDieRound / 2);  // (with the second halves of each die's last tiles)
+  moe_big_mfma_kernel<PRODUCT, GM, GN, RM, RN><<<static_cast<unsigned>(groups), GM * GN * kWave, 0, s>>>(
       a, order, counts, static_cast<const bf16*>(w0), static_cast<const bf16*>(w1), act_out, pair_out, n, k, m, experts, top,
       form);
 }
 
 // A product per expert in the tile that wide_time() expects to be done first, as far as that can be known here: every
 // list ends in half a tile, and `identity` of the router's outputs take their share of the pairs.  (Which tile makes no
-// difference to the sums.)  A lane's values of the activation take 0.12 us each.  8 experts of 3584 x 4736, 1,501 tokens
-// of two choices in 256 x 128, 256 x 192, 128 x 192: gate and up 232 / 254 / 260 us, down 142 / 105 / 122.
+// difference to the sums.)  A lane's values of the activation take 0.12 us each (measured while pieces left one by one).  8 experts of
+// 3584 x 4736, 1,501 tokens of two choices in 256 x 128, 256 x 192, 128 x 192, before tiles were halved: gate and up 231 / 228 / 237 us,
+// down 143 / 103 / 123; 231 became 213.
 constexpr int kBigTiles[] = {4, 1, 6};  // of kWide: 256 x 128, 256 x 192, 128 x 192
 static int big_tile_of(int product, int n, int k, int m, int experts, int identity, int top) {
   const double pairs = static_cast<double>(n) * top * experts / (experts + identity);
