@@ -5,6 +5,8 @@
 // value: 2 to 5 us a workgroup, 20 to 30 where every value was tested and stored for itself.  Other epilogues and rows that are no
 // whole pieces finish eight rows at a time: 4864 x 896 at 1,119 tokens with bounded gates 33 us in the kernel before, 46 one value at a
 // time, 29 so; 4737 x 896 at 2,048 47, 63, 36; added to 9472 x 3584 float32 results at 2,048 199, 256, 142.
+// Gates other than SiLU, or with constants, leave from registers too: 9472 x 3584 at 1,501 tokens in two launches 102.7 and 82.3 us behind
+// that loop, 99.1 and 78.0 so.
 // Against the kernel before (16 wavefronts, tiles of 16 x 16, 256 x 256, 256 x 128 and 128 x 128), both in the passes of whole models on
 // one card: 7B at 2,048 tokens QKV 100 us -> 67, output and down 168 -> 146 on average, gate/up 507 -> 462 (1.20 PFLOP/s); at 512
 // QKV 46 -> 26, output 33 -> 25, gate/up 156 -> 133 (two launches), down 104 -> 78; 14B at 512 QKV 64 -> 58, output and down
@@ -17,9 +19,10 @@
 
 namespace shk {
 
-// WHOLE: rows in whole 16-byte pieces and at most a bias or SiLU's gate, finished in registers.  Anything else is a kernel of its
-// own, which keeps both short.  pieces: its results leave in 16-byte pieces too.
-template <int GM, int GN, int RM, int RN, bool GATED, bool WHOLE>
+// WHOLE: rows in whole 16-byte pieces, finished in registers: at most a bias or SiLU's gate, or (kWholeGates) bfloat16 rows of any gate,
+// its constants in `bias`.  Anything else is a kernel of its own, which keeps all short.  pieces: its results leave in 16-byte pieces too.
+constexpr int kWholeGates = 2;
+template <int GM, int GN, int RM, int RN, bool GATED, int WHOLE>
 __global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per_eu(GM * GN / 4, GM * GN / 4)))
     gemm_wide_kernel(const bf16* __restrict__ a, int lda, int n, int k, const uint4* __restrict__ wt, int ktiles, int m,
                      const float* __restrict__ bias, void* __restrict__ out, int ldo, int out_f32, int accumulate, int pieces,
@@ -82,7 +85,15 @@ __global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per
   if (row0 >= m) return;  // (no barrier follows)
   char* mine = reinterpret_cast<char*>(&mem[0]) + wave * (32 * (32 * RM * 4 + 16));
   if constexpr (WHOLE) {
-    auto finish = [&](auto f32, auto biased) {
+    const float limit = WHOLE == kWholeGates && bias ? bias[0] : 0.f, shift = WHOLE == kWholeGates && bias ? bias[1] : 0.f;
+    auto gated = [&](float g, float u, auto act) {
+      if constexpr (WHOLE == kWholeGates) {
+        g = limit > 0.f ? fminf(g, limit) : g, u = limit > 0.f ? fminf(fmaxf(u, -limit), limit) : u;
+        u = bias ? u + shift : u;
+      }
+      return gate_times_up(g, u, decltype(act)::value, nullptr);
+    };
+    auto finish = [&](auto f32, auto biased, auto act) {
       constexpr bool F32 = decltype(f32)::value, BIASED = decltype(biased)::value;
       // (asked for together: one by one, each group of rows waits for its own)
       f32x4 add[RM][4];
@@ -103,7 +114,7 @@ __global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per
           f32x4 v;
 #pragma unroll
           for (int r = 0; r < 4; ++r)
-            v[r] = GATED ? gate_times_up(c[jn][g * 4 + r], c[jn][(GATED ? 8 : 0) + g * 4 + r], kActSilu, nullptr) : c[jn][g * 4 + r];
+            v[r] = GATED ? gated(c[jn][g * 4 + r], c[jn][(GATED ? 8 : 0) + g * 4 + r], act) : c[jn][g * 4 + r];
           if constexpr (BIASED) v += add[i][g];
           if constexpr (F32) {
             *reinterpret_cast<f32x4*>(mine + j * kPitch + row * 4) = v;
@@ -132,16 +143,28 @@ __global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per
         SHK_LDS_DONE();
       }
     };
+    constexpr std::integral_constant<int, kActSilu> silu;
     auto leave = [&](auto f32) {
       if (!GATED && bias)
-        finish(f32, std::bool_constant<!GATED>{});
+        finish(f32, std::bool_constant<!GATED>{}, silu);
       else
-        finish(f32, std::false_type{});
+        finish(f32, std::false_type{}, silu);
     };
-    if (out_f32)
+    if constexpr (WHOLE == kWholeGates) {
+      const std::false_type no;
+      if (accumulate == kActQuickGelu)
+        finish(no, no, std::integral_constant<int, kActQuickGelu>{});
+      else if (accumulate == kActGeluTanh)
+        finish(no, no, std::integral_constant<int, kActGeluTanh>{});
+      else if (accumulate == kActRelu)
+        finish(no, no, std::integral_constant<int, kActRelu>{});
+      else
+        finish(no, no, silu);
+    } else if (out_f32) {
       leave(std::true_type{});
-    else
+    } else {
       leave(std::false_type{});
+    }
     return;
   }
   // Anything else: the sums go through LDS as they are; a lane finishes eight neighbouring rows of a token at a time, so that
@@ -365,11 +388,13 @@ static void launch_wide(hipStream_t s, const bf16* a, int lda, int n, int k, con
   const unsigned groups = big_grid(tiles_x, tiles_y, ksplit, 16 * S::kTiles, 32 * GN * RN, S::kLds <= 80 * 1024 ? 512 : 256, &order);
   const int per = out_f32 ? 4 : 8;  // values of 16 bytes
   const int pieces = ldo % per == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
-  const bool whole = pieces && m % per == 0 && reinterpret_cast<uintptr_t>(bias) % 16 == 0 &&
-                     (gated ? accumulate == kActSilu && !bias : accumulate == 0);
+  const bool rows = pieces && m % per == 0;
+  const bool whole = rows && reinterpret_cast<uintptr_t>(bias) % 16 == 0 && (gated ? accumulate == kActSilu && !bias : accumulate == 0);
   const int ktiles = (k + 31) / 32;
-  const auto kernel = gated ? (whole ? gemm_wide_kernel<GM, GN, RM, RN, true, true> : gemm_wide_kernel<GM, GN, RM, RN, true, false>)
-                            : (whole ? gemm_wide_kernel<GM, GN, RM, RN, false, true> : gemm_wide_kernel<GM, GN, RM, RN, false, false>);
+  const auto kernel = gated ? (whole                ? gemm_wide_kernel<GM, GN, RM, RN, true, 1>
+                               : rows && !out_f32 ? gemm_wide_kernel<GM, GN, RM, RN, true, kWholeGates>
+                                                  : gemm_wide_kernel<GM, GN, RM, RN, true, 0>)
+                            : (whole ? gemm_wide_kernel<GM, GN, RM, RN, false, 1> : gemm_wide_kernel<GM, GN, RM, RN, false, 0>);
   kernel<<<groups, S::kWaves * kWave, 0, s>>>(a, lda, n, k, wt, ktiles, m, bias, out, ldo, out_f32, accumulate, pieces,
                                                             order);
 }
