@@ -8,6 +8,7 @@
 namespace shk {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 // 16 bytes as the compiler's own vector type: copies of it are loads and stores,
 // where copies of HIP's uint4 struct can end up as memcpy through scratch memory

@@ -716,7 +716,7 @@ __global__ void __launch_bounds__(16 * kWave)
     gemm_stream_kernel(const bf16* __restrict__ a, int lda, int n, int k,
                        const uint4* __restrict__ wt, int ktiles, int m,
                        const float* __restrict__ bias, void* __restrict__ out, int ldo,
-                       int out_f32, int accumulate, int ksplit) {
+                       int out_f32, int accumulate, int ksplit, int pieces) {
   constexpr int KT = kStreamTiles;
   constexpr int kFrags = NB * KT;      // activation fragments per stage
   constexpr int kLoads = APER + KT;    // loads per wavefront and stage
@@ -851,13 +851,63 @@ __global__ void __launch_bounds__(16 * kWave)
         }
       }
     }
-    if (wave & 1) return;
     ob = wb / 2;
   }
-  if (!have_rows) return;
 
+  // Whole rows: 16 tokens' results at a time go through LDS and leave as pieces of 16 bytes, neighbouring lanes along a token's row.  Straight
+  // from the registers a store touches 16 rows, 4 bytes a lane: weights cold, float32 rows of 151936 x 896 at 17 / 32 tokens 55.9 / 64.6 us,
+  // 53.5 / 58.6 so; 152064 x 3584 at 64 227, 217 so.
   // lane (j, kg) of accumulator b: token b*16 + j, rows ob*16 + kg*4 + r
   const int row0 = ob * 16 + kg * 4;
+  const bool f32 = out_f32 || ksplit > 1;
+  if (pieces && (f32 ? 4 : 2) * waves <= (GATED ? 8 : 4) * kFrags) {
+    const int each = f32 ? 4 : 8;                                                 // values of a piece
+    const int across = (GATED ? waves / 2 : waves) * 16 / each, turn = f32 ? 3 : 1;  // pieces of a token; they lie rotated by its number
+    const int mine = (GATED ? wave / 2 : wave) * 16 + kg * 4, first = (GATED ? blockIdx.x * waves / 2 : blockIdx.x * waves) * 16;
+    auto put = [&](u32x4 (&buf)[kFrags][kWave], const f32x4& sums) {
+      if (GATED && (wave & 1)) return;
+      f32x4 v = sums;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        if (!GATED && bias) v[r] += bias[row0 + r < m ? row0 + r : m - 1];
+        if (!GATED) v[r] = plain_act(v[r], accumulate, row0 + r);
+      }
+      u32x4* at = &buf[0][0] + j * across + ((mine / each) ^ (j & turn));
+      if (f32) {
+        *reinterpret_cast<f32x4*>(at) = v;
+      } else {
+        bf16x4 o;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[r] = static_cast<__bf16>(v[r]);
+        reinterpret_cast<bf16x4*>(at)[mine / 4 % 2] = o;
+      }
+    };
+    auto leave = [&](const u32x4 (&buf)[kFrags][kWave], int b) {
+      for (int q = tid; q < 16 * across; q += waves * kWave) {
+        const int t = q / across, p = q % across, token = b * 16 + t, row = first + p * each;
+        const u32x4 v = (&buf[0][0])[t * across + (p ^ (t & turn))];
+        if (token >= n || row >= m) continue;
+        const size_t idx = (static_cast<size_t>(ksplit > 1 ? blockIdx.y : 0) * n + token) * ldo + row;
+        *reinterpret_cast<u32x4*>(static_cast<char*>(out) + idx * (f32 ? 4 : 2)) = v;
+      }
+    };
+    __syncthreads();  // the stage buffers are read no more
+    put(stage0, acc[0]);
+    put(stage1, acc[1]);
+    if constexpr (NB > 2) put(stage2, acc[2]);
+    __syncthreads();
+    leave(stage0, 0);
+    leave(stage1, 1);
+    if constexpr (NB > 2) {
+      leave(stage2, 2);
+      __syncthreads();
+      put(stage0, acc[3]);
+      __syncthreads();
+      leave(stage0, 3);
+    }
+    return;
+  }
+  if (!have_rows || (GATED && (wave & 1))) return;
 #pragma unroll
   for (int b = 0; b < NB; ++b) {
     const int token = b * 16 + j;
@@ -1349,14 +1399,16 @@ extern "C" int shk_gemm_bf16_tiled_weight(const void* a, const void* wt, const f
     const int nb = n <= 32 ? 2 : 4;
     const int aper = (nb * kStreamTiles + waves - 1) / waves;  // 1 to 4
     dim3 sgrid((wblocks + waves - 1) / waves, ksplit);
+    const int per = of || ksplit > 1 ? 4 : 8;  // values of 16 bytes
+    const int pieces = ldo % per == 0 && m % per == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0 && (gated || accumulate != 1);
 #define SHK_STREAM(NB, APER)                                                         \
   do {                                                                               \
     if (gated)                                                                       \
       gemm_stream_kernel<NB, APER, true><<<sgrid, waves * kWave, 0, s>>>(            \
-          ap, lda, n, k, wp, kt, m, bias, out, ldo, of, accumulate, ksplit);         \
+          ap, lda, n, k, wp, kt, m, bias, out, ldo, of, accumulate, ksplit, pieces); \
     else                                                                             \
       gemm_stream_kernel<NB, APER, false><<<sgrid, waves * kWave, 0, s>>>(           \
-          ap, lda, n, k, wp, kt, m, bias, out, ldo, of, accumulate, ksplit);         \
+          ap, lda, n, k, wp, kt, m, bias, out, ldo, of, accumulate, ksplit, pieces); \
   } while (0)
     if (nb == 2) {
       if (aper == 1) SHK_STREAM(2, 1); else SHK_STREAM(2, 2);
