@@ -6,6 +6,7 @@
 // fallback of the bfloat16 path.  float32 operands go to gemm_f32.hip.
 #include "api.h"
 #include "common.h"
+#include "to_lds.h"
 
 namespace shk {
 
@@ -160,7 +161,7 @@ extern "C" int shk_gemm(const void* a, const void* w, const float* bias, void* o
 // multiplied.  k in multiples of 8 and 16-byte aligned rows; sums run over k in ascending order in every
 // shape, so a row's result depends neither on the shape nor on what else is in the step.
 // What bounds it is the compute units' intake: 64 x 64 a wavefront needs 8 KiB for 16 instructions.
-// 28 heads, 1,501 rows: k = 128 to 448 features 74 us with 16 x 64 a wavefront, no load ahead and 2-byte
+// 28 heads, 1,501 rows (which the next kernel takes now): k = 128 to 448 features 74 us with 16 x 64 a wavefront, no load ahead and 2-byte
 // stores, 41 so; k = 448 to 128 features 58, now 35; 14 blocks of 256 to 512 float32 68, now 35.  Eight rows: 6.0,
 // 11.7 and 7.5 us with 64-row workgroups, 5.0, 5.9 and 4.7 now.
 typedef __bf16 gbf16x8 __attribute__((ext_vector_type(8)));
@@ -259,8 +260,107 @@ __global__ void __launch_bounds__(kWave* RW* CW)
   }
 }
 
+// The same for many rows and k in whole stages of 64: both operands go straight into LDS in whole cache lines, 8 rows x 128 bytes a
+// load (a compute unit takes in loads of 16 rows x 64 bytes at a quarter of its rate, and a workgroup's four wavefronts asked for
+// everything twice), and results leave through LDS in whole pieces along the rows.  128 rows x 128 features a workgroup, two
+// of which share a compute unit; two stages in LDS, one in flight while the other is multiplied.  The same instructions in the
+// same order of k: the same bits.  28 heads, 1,501 rows, in prompts: k = 128 to 448 features 42.4 us in the kernel above, 26.8 so, k = 448 to
+// 128 features 36.3, 17.3; 14 blocks of 256 to 512 float32 35.7, 19.9.  What bounds it now: the results, 38 to 43 MB but for the second.
+constexpr int kLinesK = 64, kLinesRows = 128;
+
+template <typename TO>
+__global__ void __launch_bounds__(4 * kWave)
+    gemm_batched_lines_kernel(const bf16* __restrict__ a, const bf16* __restrict__ w, TO* __restrict__ out, int n, int m, int k,
+                              int lda, int ldo, long long a_batch, long long w_batch, long long out_batch) {
+  constexpr int kUnits = kLinesRows / 8, kLoads = 2 * kUnits / 4;  // units of 8 rows of an operand's stage; a wavefront's loads of a stage
+  __shared__ gu32x4 mem[2 * 2 * kUnits * kWave];                    // stages, each rows then features
+  const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int i = lane % 16, kg = lane / 16;
+  const int row0 = blockIdx.y * kLinesRows, col0 = blockIdx.x * kLinesRows, stages = k / kLinesK;
+  const char* asrc = reinterpret_cast<const char*>(a + blockIdx.z * a_batch + static_cast<size_t>(row0) * lda);
+  const char* wsrc = reinterpret_cast<const char*>(w + blockIdx.z * w_batch + static_cast<size_t>(col0) * k);
+  const unsigned base = static_cast<unsigned>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)mem));
+  // Lane l of a unit loads piece (l % 8) ^ (l / 8) of row l / 8: reads of 16 rows at one piece then meet no bank conflicts.
+  // Rows beyond either matrix are read as its last and not stored.
+  unsigned aoff[kLoads / 2], woff[kLoads / 2];
+#pragma unroll
+  for (int u = 0; u < kLoads / 2; ++u) {
+    const int row = (wave + 4 * u) * 8 + lane / 8;
+    const unsigned piece = ((lane % 8) ^ (lane / 8)) * 16u;
+    aoff[u] = static_cast<unsigned>(min(row, n - 1 - row0)) * lda * 2u + piece;
+    woff[u] = static_cast<unsigned>(min(row, m - 1 - col0)) * k * 2u + piece;
+  }
+  auto load = [&](int st) {  // (a stage beyond the last: the last again, never multiplied)
+    const size_t at = static_cast<size_t>(min(st, stages - 1)) * (kLinesK * 2);
+    const unsigned to = base + (st % 2 * 2 * kUnits + wave) * 1024;
+#pragma unroll
+    for (int u = 0; u < kLoads / 2; ++u) SHK_LOAD_TO_LDS(to + u * 4096, aoff[u], asrc + at);
+#pragma unroll
+    for (int u = 0; u < kLoads / 2; ++u) SHK_LOAD_TO_LDS(to + kUnits * 1024 + u * 4096, woff[u], wsrc + at);
+  };
+  gf32x4 acc[4][4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) acc[r][c] = gf32x4{0.f, 0.f, 0.f, 0.f};
+  const int arow = wave / 2 * 64, wrow = wave % 2 * 64;
+  load(0);
+  load(1);
+  for (int st = 0; st < stages; ++st) {
+    SHK_MEET_WITH_LOADS(kLoads);  // (the stage has landed for every wavefront)
+    const char* lds = reinterpret_cast<const char*>(mem) + st % 2 * 2 * kUnits * 1024;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int piece = ((4 * h + kg) ^ (i % 8)) * 16;
+      gu32x4 av[4], wv[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) av[r] = *reinterpret_cast<const gu32x4*>(lds + (arow + r * 16 + i) * 128 + piece);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) wv[c] = *reinterpret_cast<const gu32x4*>(lds + (kLinesRows + wrow + c * 16 + i) * 128 + piece);
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gbf16x8, wv[c]), __builtin_bit_cast(gbf16x8, av[r]),
+                                                              acc[r][c], 0, 0, 0);
+    }
+    SHK_MEET_WITH_LOADS(kLoads);  // (nobody reads the stage any more; only the next one's loads are in flight)
+    load(st + 2);
+  }
+  SHK_WAIT_LOADS(0);
+  __syncthreads();
+  // A lane has features 4 kg + 0..3 of a tile for row i.  Sixteen rows of a wavefront at a time, in two places by turns.
+  constexpr int E = sizeof(TO), kPitch = 64 * E + 16, kPieces = 64 * E / 16;
+  static_assert(4 * 2 * 16 * kPitch <= sizeof(mem), "the results of sixteen rows a wavefront fit LDS twice");
+  char* mine = reinterpret_cast<char*>(mem) + wave * 2 * 16 * kPitch;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    char* place = mine + r % 2 * 16 * kPitch;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      char* to = place + i * kPitch + (t * 16 + 4 * kg) * E;
+      if constexpr (E == 4) {
+        *reinterpret_cast<gf32x4*>(to) = acc[r][t];
+      } else {
+        const uint32_t lo = bf16_bits(acc[r][t][0]) | static_cast<uint32_t>(bf16_bits(acc[r][t][1])) << 16;
+        const uint32_t hi = bf16_bits(acc[r][t][2]) | static_cast<uint32_t>(bf16_bits(acc[r][t][3])) << 16;
+        *reinterpret_cast<uint2*>(to) = make_uint2(lo, hi);
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int q = 0; q < 16 * kPieces / kWave; ++q) {
+      const int t = (q * kWave + lane) / kPieces, p = (q * kWave + lane) % kPieces;
+      const int row = row0 + arow + r * 16 + t, col = col0 + wrow + p * (16 / E);
+      const gu32x4 v = *reinterpret_cast<const gu32x4*>(place + t * kPitch + p * 16);
+      if (row < n && col < m) *reinterpret_cast<gu32x4*>(out + blockIdx.z * out_batch + static_cast<size_t>(row) * ldo + col) = v;
+    }
+  }
+}
+
 // Shapes: up to 16 rows 16 x 16 a wavefront, side by side along the features (the weights' latency is all
-// there is); 64 x 64 a wavefront where such workgroups fill the compute units, else 32 x 32.  A k of one or two steps
+// there is); 64 x 64 a wavefront where such workgroups fill the compute units, through LDS where k and the results are whole lines and
+// pieces, else 32 x 32.  A k of one or two steps
 // is loaded a step at a time: eight steps' loads, most of them the last step's again, took 4.1 us for 8 products
 // of 256 x 64 at 16 rows, two 2.4 (3.1 with 64-row workgroups).
 template <typename TO>
@@ -270,7 +370,13 @@ static void launch_batched_mfma(const bf16* a, const bf16* w, TO* out, int n, in
   auto grid = [&](int rows, int cols) { return dim3((m + cols - 1) / cols, (n + rows - 1) / rows, batch); };
   const dim3 large = grid(128, 128);
   const bool short_k = k <= 64;
-  if (n <= 16 && short_k)
+  const int per = 16 / sizeof(TO);  // values of a piece
+  // whole stages and whole pieces everywhere, offsets within a workgroup's rows in 32 bits
+  const bool lines = k >= kLinesK && k % kLinesK == 0 && m % per == 0 && ldo % per == 0 && out_batch % per == 0 && w_batch % 8 == 0 &&
+                     reinterpret_cast<uintptr_t>(out) % 16 == 0 && lda <= 1 << 22 && k <= 1 << 22;
+  if (lines && static_cast<long long>(large.x) * large.y * batch >= 256)
+    gemm_batched_lines_kernel<TO><<<large, 256, 0, s>>>(a, w, out, n, m, k, lda, ldo, a_batch, w_batch, out_batch);
+  else if (n <= 16 && short_k)
     gemm_batched_mfma_kernel<1, 1, 1, 4, 1, TO>
         <<<grid(16, 64), 256, 0, s>>>(a, w, out, n, m, k, lda, ldo, vec_out, a_batch, w_batch, out_batch);
   else if (n <= 16)
