@@ -16,7 +16,7 @@
 // 7.8 so; 3584 x 18944 at 8 tokens 25.7, 23.2).
 //
 // Weights cold, chains of one kind of call, us at 1 / 8 / 16 tokens.  Product and norm against few_stream: 896 x 896
-// 5.6 / 6.0 / 6.4 -> 3.0 / 3.3 / 3.7, 896 x 4864 6.9 / 7.3 / 7.5 -> 4.9 / 5.6 / 6.7, 3584 x 3584 9.6 / 9.5 / 10.4 -> 6.1 / 7.4 / 8.3,
+// 5.6 / 6.0 / 6.4 -> 2.9 / 3.0 / 3.0, 896 x 4864 6.9 / 7.3 / 7.5 -> 5.3 / 5.9 / 5.8, 3584 x 3584 9.6 / 9.5 / 10.4 -> 6.1 / 7.4 / 8.3,
 // 3584 x 18944 26.4 / 26.7 / 29.6 -> 21.9 / 24.1 / 27.0.  Projections, rotation and cache write against few_heads: 1152 x 896
 // 5.5 / 6.1 / 6.4 -> 4.1 / 4.3 / 4.4, 4608 x 3584 10.7 / 11.1 / 12.2 -> 10.4 / 11.2 / 12.3, 7168 x 5120 16.4 / 16.2 / 18.2 -> 14.2 / 15.4 /
 // 17.2.  few_gated against the product without the division: 9728 x 896 5.6 / 6.2 / 6.9 -> 5.9 / 6.1 / 6.4, 37888 x 3584 40.6 /
@@ -89,6 +89,7 @@ struct FewSquares {
 };
 
 constexpr int kFewWaves = 9;  // wavefronts of a workgroup at most
+constexpr int kFewHalfWaves = 4, kFewHalfTiles = 8;  // of one for half a block and 8 tokens; its tiles of a batch
 
 // What a workgroup of few_stream's kernels does with the sum of weight row `row` and a token: it joins the stream, goes out times the next norm's
 // weight, and its square with those of the ROWS rows beside it (neighbouring lanes) is their group's sum.
@@ -104,107 +105,85 @@ __device__ __forceinline__ void few_join(float v, float w, int row, int token, b
   if (row % ROWS == 0) sums[static_cast<size_t>(row / ROWS) * n + token] = square;
 }
 
-// A workgroup for a block of 16 weight rows and 16 tokens.
-template <int C>
+// ROWS = 16: a workgroup for a block of 16 weight rows.  ROWS = 8: for half of one (a tile's pieces of 8 rows are whole
+// lines of 128 bytes), where whole blocks leave compute units idle; the other half of the matrix instruction does the same again.
+template <int C, int ROWS, int NB>
 __global__ void __launch_bounds__(kFewWaves* kWave)
     few_stream_kernel(FewRows x, const u32x4* __restrict__ wt, int ktiles, int m, const float* __restrict__ bias,
                       float* __restrict__ resid, const float* __restrict__ weight, bf16* __restrict__ rows,
                       float* __restrict__ sums) {
-  extern __shared__ f32x4 red[];  // [waves][64]
-  const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), waves = blockDim.x / kWave;
-  const int inside = threadIdx.x / 16, r = threadIdx.x % 16, row = blockIdx.x * 16 + r, token = few_first<1>() + inside;
-  const bool mine = inside < 16 && token < x.n;
-  float old = 0.f, w = 0.f;
-  if (mine) {
-    old = resid[static_cast<size_t>(token) * m + row];
-    w = weight[row];
-    if (bias) old += bias[row];
-  }
-  const u32x4* const wrow[1] = {wt + static_cast<size_t>(blockIdx.x) * ktiles * kWave + lane};
-  f32x4 acc[1][1];
-  few_multiply<C, 4, 1, 1>(acc, wrow, FewTokens<1>{x}, x.col_step, x.k, ktiles, wave, waves, [] {});
-  red[wave * kWave + lane] = acc[0][0];
-  __syncthreads();
-  if (inside >= 16) return;
-  few_join<16>(few_sum(red, kWave, r, inside, waves) + old, w, row, token, mine, x.n, m, resid, rows, sums);
-}
-
-// A workgroup for half a block, 8 weight rows (a tile's pieces of 8 rows are whole lines of 128 bytes), and NB times 8 tokens.  An operand of
-// 16 rows holds these 8 of two neighbouring k-tiles, the tokens' operand 8 tokens of both, and two diagonal quarters of the results are
-// the two tiles' sums (the others mix tiles and are left).  What bounds it otherwise: a compute unit takes in 64 bytes a clock, and
-// with the 8 rows in both halves of the operand half of what it took was the same again.  Chains with cold weights, us at 1 / 8 / 16 / 32 tokens:
-// 896 x 4864 6.1 / 6.1 / 7.0 / 6.7 -> 4.9 / 5.6 / 6.7 / 6.4, 1536 x 8960 9.2 / 9.2 / 11.1 -> 7.2 / 8.5 / 11.0, 2048 x 11008 11.9 /
-// 11.9 / 13.0 -> 9.2 / 10.4 / 13.2.
-template <int C, int NB>
-__global__ void __launch_bounds__(kFewWaves* kWave)
-    few_stream_half_kernel(FewRows x, const u32x4* __restrict__ wt, int ktiles, int m, const float* __restrict__ bias,
-                           float* __restrict__ resid, const float* __restrict__ weight, bf16* __restrict__ rows,
-                           float* __restrict__ sums) {
   extern __shared__ f32x4 red[];  // [waves][NB][64]
   const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), waves = blockDim.x / kWave;
-  const int inside = threadIdx.x / 8, r = threadIdx.x % 8, row = blockIdx.x * 8 + r, first = blockIdx.y * 8 * NB, token = first + inside;
-  const bool mine = inside < 8 * NB && token < x.n;
-  float old = 0.f, w = 0.f;
-  if (mine) {
-    old = resid[static_cast<size_t>(token) * m + row];
+  const int wr = blockIdx.x * ROWS + lane % ROWS;
+  const int inside = threadIdx.x / ROWS, r = threadIdx.x % ROWS, row = blockIdx.x * ROWS + r;
+  float old[NB], w = 0.f;
+#pragma unroll
+  for (int c = 0; c < NB; ++c) {
+    const int token = few_first<NB>() + c * 16 + inside;
+    old[c] = inside < 16 && token < x.n ? resid[static_cast<size_t>(token) * m + row] : 0.f;
+  }
+  if (inside < 16) {
+    w = weight[row];
+    if (bias) {
+      const float add = bias[row];
+#pragma unroll
+      for (int c = 0; c < NB; ++c) old[c] += add;
+    }
+  }
+  const u32x4* const wrow[1] = {wt + static_cast<size_t>(wr / 16) * ktiles * kWave + wr % 16 + lane / 16 * 16};
+  f32x4 acc[1][NB];
+  few_multiply<C, 4, 1, NB>(acc, wrow, FewTokens<NB>{x}, x.col_step, x.k, ktiles, wave, waves, [] {});
+#pragma unroll
+  for (int c = 0; c < NB; ++c) red[(wave * NB + c) * kWave + lane] = acc[0][c];
+  __syncthreads();
+  if (inside >= 16) return;
+#pragma unroll
+  for (int c = 0; c < NB; ++c) {
+    const int token = few_first<NB>() + c * 16 + inside;
+    const float v = few_sum(red + c * kWave, NB * kWave, r, inside, waves) + old[c];
+    few_join<ROWS>(v, w, row, token, token < x.n, x.n, m, resid, rows, sums);
+  }
+}
+
+struct FewHalfTokens {  // the same 8 tokens for both halves of an operand
+  const FewRows& x;
+  __device__ __forceinline__ void operator()(const bf16* (&arow)[1]) const {
+    arow[0] = x.a + static_cast<size_t>(min(static_cast<int>(blockIdx.y * 8 + threadIdx.x % 8), x.n - 1)) * x.token_step;
+  }
+};
+
+// The same for half a block and 8 tokens.  The `walks` sums that a whole block's wavefronts form, each of every walks-th k-tile, go two to a
+// wavefront: an operand of 16 rows holds these 8 of a tile of one walk and of a tile of the other, the tokens' operand 8 tokens of both, and two
+// diagonal quarters of the results are the two sums (the others mix walks and are left).  So a row's bits are those that the kernel above gives.
+// What bounds that one: a compute unit takes in 64 bytes a clock, half of them the same 8 rows again.  Chains with cold weights, us at 1 / 8 / 16
+// tokens, above and here: 896 x 896 3.0 / 3.1 / 3.2 -> 2.9 / 3.0 / 3.0, 896 x 4864 6.0 / 6.1 / 7.0 -> 5.3 / 5.9 / 5.8, 1024 x 4096 5.6 / 5.7 / 6.0 -> 4.6 /
+// 5.1 / 5.0, 2048 x 8192 at 1 / 8 11.1 / 11.1 -> 8.4 / 9.4.  Batches of 4, 12 or 16 tiles in place of 8: 896 x 4864 at one token 5.7, 5.8, 5.5.  (Two
+// neighbouring tiles of one walk in an operand, which lets eight wavefronts share k: 4.9 / 5.6 / 6.7, but other sums than a whole block's.)
+template <int C>
+__global__ void __launch_bounds__(kFewHalfWaves* kWave)
+    few_stream_half_kernel(FewRows x, const u32x4* __restrict__ wt, int ktiles, int m, const float* __restrict__ bias,
+                           float* __restrict__ resid, const float* __restrict__ weight, bf16* __restrict__ rows,
+                           float* __restrict__ sums, int walks) {
+  extern __shared__ f32x4 red[];  // [waves][64]
+  const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int inside = threadIdx.x / 8, r = threadIdx.x % 8, row = blockIdx.x * 8 + r, token = blockIdx.y * 8 + inside;
+  const bool mine = inside < 8 && token < x.n;
+  float old = mine ? resid[static_cast<size_t>(token) * m + row] : 0.f, w = 0.f;
+  if (inside < 8) {
     w = weight[row];
     if (bias) old += bias[row];
   }
-  const int second = lane % 16 / 8, kg = lane / 16;  // which tile of a pair the lane reads, and which 8 of its k
-  const u32x4* const wrow = wt + static_cast<size_t>(blockIdx.x / 2) * ktiles * kWave + blockIdx.x % 2 * 8 + lane % 8 + kg * 16;
-  const bf16* arow[NB];
-#pragma unroll
-  for (int b = 0; b < NB; ++b) arow[b] = x.a + static_cast<size_t>(min(first + b * 8 + lane % 8, x.n - 1)) * x.token_step;
-  constexpr int kPairs = C > 0 ? C : NB > 2 ? 2 : 4;
-  struct Batch {
-    u32x4 w[kPairs], x[kPairs][NB];
-    uint32_t keep[kPairs];
-  };
-  auto load = [&](Batch& q, int t) {  // (addresses are clamped and what lies beyond k is zeroed, as in few_multiply)
-#pragma unroll
-    for (int u = 0; u < kPairs; ++u) {
-      const int tile = 2 * (t + u * waves) + second, col = tile * 32 + kg * 8;
-      q.w[u] = __builtin_nontemporal_load(wrow + static_cast<size_t>(tile < ktiles ? tile : ktiles - 1) * kWave);
-      const bool in = col < x.k;
-      q.keep[u] = in ? ~0u : 0u;
-#pragma unroll
-      for (int b = 0; b < NB; ++b)
-        q.x[u][b] = *reinterpret_cast<const u32x4*>(arow[b] + (in ? static_cast<size_t>(col) * x.col_step : 0));
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  f32x4 acc[NB];
-#pragma unroll
-  for (int b = 0; b < NB; ++b) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
-  auto multiply = [&](const Batch& q) {
-#pragma unroll
-    for (int u = 0; u < kPairs; ++u) {
-      const bf16x8 wv = __builtin_bit_cast(bf16x8, q.w[u] & q.keep[u]);
-#pragma unroll
-      for (int b = 0; b < NB; ++b)
-        acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv, __builtin_bit_cast(bf16x8, q.x[u][b] & q.keep[u]), acc[b], 0, 0, 0);
-    }
-  };
-  Batch ping;
-  load(ping, wave);
-  if constexpr (C > 0) {
-    multiply(ping);
-  } else {
-    Batch pong;
-    const int step = kPairs * waves, batches = ((ktiles + 1) / 2 + step - 1) / step;
-    for (int i = 0; i < batches; i += 2) {
-      load(pong, wave + (i + 1) * step);
-      multiply(ping);
-      load(ping, wave + (i + 2) * step);
-      multiply(pong);
-    }
-  }
-#pragma unroll
-  for (int b = 0; b < NB; ++b) red[(wave * NB + b) * kWave + lane] = acc[b];
+  const u32x4* const wrow[1] = {wt + static_cast<size_t>(blockIdx.x / 2) * ktiles * kWave + blockIdx.x % 2 * 8 + lane % 8 + lane / 16 * 16};
+  const int walk = 2 * wave + lane % 16 / 8;  // (an odd number of them: the last one's neighbour is none, all zeros)
+  f32x4 acc[1][1];
+  few_multiply<C, kFewHalfTiles, 1, 1>(acc, wrow, FewHalfTokens{x}, x.col_step, x.k, ktiles, walk < walks ? walk : ktiles, walks, [] {});
+  red[wave * kWave + lane] = acc[0][0];
   __syncthreads();
-  if (inside >= 8 * NB) return;
-  const f32x4* part = red + inside / 8 * kWave;
-  const float v = few_sum(part, NB * kWave, r, inside % 8, waves) + few_sum(part, NB * kWave, r + 8, inside % 8 + 8, waves);
+  if (inside >= 8) return;
+  // element (r, token) of an even walk, (r + 8, token + 8) of an odd one, added in their order
+  const float* p = reinterpret_cast<const float*>(red + r / 4 * 16 + inside) + r % 4;
+  float v = 0.f;
+  for (int t = 0; t < walks; ++t) v += p[(t / 2 * kWave + t % 2 * (2 * 16 + 8)) * 4];
   few_join<8>(v + old, w, row, token, mine, x.n, m, resid, rows, sums);
 }
 
@@ -342,9 +321,13 @@ static void with_loads(int count, int threads, Fn fn) {
 }
 constexpr int kFewMostLoads = 16;
 
-// Half blocks where whole ones would be one for every second compute unit or fewer: 896 x 4864 at 8 tokens 6.6 us whole, 5.6 in
-// halves, 2048 x 11008 12.7 and 10.4; 3584 x 18944 23.2 and 32.1.
+// Half blocks where whole ones would be one for every second compute unit or fewer: 896 x 4864 at 8 tokens 6.6 us whole, 5.9 in
+// halves, 2048 x 11008 12.7 and 11.8; 3584 x 18944 23.2 and 32.1.
 static int few_stream_rows(int m) { return m <= 2048 ? 8 : 16; }
+
+// Half blocks of 8 tokens, whose wavefronts take two walks of k each: up to 8 tokens, and as long as all of them are at work at once.  At 16 / 32
+// tokens in blocks of 16 and of 8: 896 x 4864 7.0 / 6.6 and 5.8 / 8.9 us, 512 x 2048 4.1 / 4.0 and 3.4 / 3.5, 1536 x 1536 4.0 / 5.0 and 4.3 / 5.2.
+static bool few_stream_paired(int n, int m) { return n <= 8 || (n + 7LL) / 8 * (m / 8) <= kDies * kDieUnits; }
 
 // The most rows * k for which 17 to 64 tokens go this way: every 16 of them read the weights again, from the caches.
 // At 17 / 32 / 64 tokens, with the norm: 896 x 896 7.6 / 7.6 / 7.6 -> 3.6 / 3.6 / 4.7, 896 x 4864 10.3 / 11.0 / 12.2 -> 6.3 / 6.6 / 9.5,
@@ -369,14 +352,14 @@ static bool few_takes(int n, int m, int k, long long most) {
 
 // Not where a second round of workgroups would be nearly empty: 320 of them (5120 x 5120 at 8 tokens 14.3 us for product in shares
 // and norm, 15.1 here; 5120 x 13824 28.0 and 31.4).  256 are a round: 4096 x 14336 23.7 -> 20.0.
-// Nor where few workgroups walk a long k, which shares of it spread over the chip.  Product and norm against this at 1 / 8 / 16 tokens: 512 x 5120
-// 6.6 / 7.2 / 7.3 -> 6.0 / 6.0 / 6.9, x 8192 7.7 / 8.0 / 8.4 -> 8.7 / 8.8 / 9.4, 256 x 18944 8.4 / 9.0 / 9.4 -> 17.1 / 17.1 / 18.5, 1536 x 6144 10.1 / 10.5 /
-// 11.2 -> 7.8 / 7.8 / 8.3, x 8960 10.3 / 11.2 / 12.5 -> 11.5 / 11.5 / 11.6, x 18944 14.6 / 16.7 / 19.2 -> 21.4 / 18.7 / 20.3, 2048 x 8192 11.6 / 12.0 /
-// 12.0 -> 11.4 / 11.4 / 10.8, x 14336 15.1 / 15.3 / 16.5 -> 17.9 / 15.0 / 16.3, 2304 x 9216 12.3 / 13.2 / 14.5 -> 12.5 / 13.6 / 15.9, 2560 x 8192 12.1 / 12.1 / 13.1 -> 11.5 / 10.8 / 12.7, x 13824 16.3 / 15.8 /
-// 17.7 -> 17.6 / 16.3 / 19.3; 192 workgroups and more at any k: 3072 x 18944 23.9 / 24.8 / 27.7 -> 23.0 / 22.4 / 26.3, 4096 x 24576 36.3 / 37.8 / 41.0 -> 33.9 /
-// 32.7 / 35.9; 64 tokens, 256 x 6144 8.6 -> 10.0, 512 x 5120 10.6 -> 9.4, x 8192 11.0 -> 12.8.
-// (Half blocks have become faster since these lines were drawn, 256 x 18944 10.7 / 13.5 / 18.3, 1536 x 8960 7.2 / 8.6 / 10.9, 2048 x 14336 10.7 / 12.4 / 16.0;
-// the lines stand, so that sizes keep the sums that they had.)
+// Nor where few workgroups walk a long k, which shares of it spread over the chip.  Product and norm against this at 1 / 8 / 16 tokens: 1024 x 5120
+// 7.3 / 7.3 / 7.9 -> 5.7 / 6.2 / 6.0, 512 x 8192 7.6 / 8.1 / 8.4 -> 6.4 / 7.3 / 7.1, 256 x 18944 8.3 / 8.7 / 9.1 -> 11.8 / 13.5 / 13.1, 1536 x 6144 10.4 /
+// 11.0 / 11.1 -> 6.5 / 7.5 / 8.7, x 8960 10.1 / 10.9 / 13.2 -> 8.7 / 10.9 / 12.4, x 18944 15.1 / 17.0 / 21.7 -> 15.2 / 18.5 / 22.7, 2048 x 8192 11.4 / 11.8 /
+// 12.7 -> 8.4 / 9.4 / 11.7, x 14336 15.7 / 16.4 / 17.6 -> 12.8 / 14.5 / 19.6; whole blocks, 2304 x 9216 12.3 / 13.2 / 14.5 -> 12.5 / 13.6 / 15.9, 2560 x 8192
+// 12.1 / 12.1 / 13.1 -> 11.5 / 10.8 / 12.7, x 13824 16.3 / 15.8 / 17.7 -> 17.6 / 16.3 / 19.3; 192 workgroups and more at any k: 3072 x 18944 23.9 / 24.8 / 27.7 -> 23.0 /
+// 22.4 / 26.3, 4096 x 24576 36.3 / 37.8 / 41.0 -> 33.9 / 32.7 / 35.9; 64 tokens, 256 x 6144 8.6 -> 10.0, 512 x 5120 10.6 -> 9.4, x 8192 11.0 -> 12.8.
+// (Half blocks' line was drawn while a wavefront took one walk, 512 x 8192 8.7 / 8.8 / 9.4, 1536 x 8960 11.5 / 11.5 / 11.6, 2048 x 14336 17.9 / 15.0 / 16.3.  It
+// stands there, so that the sizes between keep the order in which shares and norm add them up.)
 extern "C" int shk_few_stream_sums(int n, int m, int k) {
   const bool near = m >= 3072 || k <= 5120 || (m <= 2048 ? k <= 4 * m : 2 * k <= 7 * m);
   return m > 0 && m <= 4096 && m % 16 == 0 && k > 0 && k % 8 == 0 && near && few_takes(n, m, k, kFewStreamMost) ? m / few_stream_rows(m) : 0;
@@ -398,27 +381,20 @@ extern "C" int shk_few_stream(const void* a, int lda, int n, int k, const void* 
   if (n == 0) return 0;
   SHK_REQUIRE(a && wt && resid && weight && rows && sums, "few_stream: null pointer");
   SHK_REQUIRE(reinterpret_cast<uintptr_t>(a) % 16 == 0, "few_stream: rows are not 16-byte aligned");
-  const int kt = (k + 31) / 32, half = few_stream_rows(m) == 8, steps = half ? (kt + 1) / 2 : kt;
-  int waves = few_waves(steps, kFewTiles);
-  if (half) {
-    // as few as hold their pairs of tiles at once, else four (896 x 896 at 1 / 16 tokens 2.95 / 3.73 us in four, 3.07 / 3.85 in seven;
-    // 1536 x 8960 at 8 / 16 8.5 / 11.0 in four, 9.2 / 12.0 in five)
-    for (waves = 4; waves <= 8 && (steps + waves - 1) / waves > kFewTiles;) ++waves;
-    if (waves > 8) waves = 4;
-  }
-  const auto go = [&](auto kernel, int rows_each, int nb) {
-    kernel<<<dim3(m / rows_each, (n + nb - 1) / nb), waves * kWave, (half ? nb / 8 : 1) * waves * kWave * sizeof(f32x4), static_cast<hipStream_t>(stream)>>>(
-        x, static_cast<const u32x4*>(wt), kt, m, bias, resid, weight, static_cast<bf16*>(rows), sums);
-  };
-  with_tiles<kFewTiles>((steps + waves - 1) / waves, [&](auto c) {
-    if (!half)
-      go(few_stream_kernel<c.value>, 16, 16);
-    else if (n <= 8)
-      go(few_stream_half_kernel<c.value, 1>, 8, 8);
-    else if (n <= 32 || (c.value > 0 && c.value <= 5))
-      go(few_stream_half_kernel<c.value, 2>, 8, 16);
-    else  // (many tokens would have a long k read four times over: 896 x 4864 at 64 10.8 us in blocks of 16; 896 x 896 5.1 so, 4.8)
-      go(few_stream_half_kernel<0, 4>, 8, 32);
+  const int kt = (k + 31) / 32, waves = few_waves(kt, kFewTiles), rows_each = few_stream_rows(m);
+  with_tiles<kFewTiles>((kt + waves - 1) / waves, [&](auto c) {
+    const auto go = [&](auto kernel, int tokens, int wavefronts, auto... more) {
+      kernel<<<dim3(m / rows_each, (n + tokens - 1) / tokens), wavefronts * kWave, (tokens + 15) / 16 * wavefronts * kWave * sizeof(f32x4), static_cast<hipStream_t>(stream)>>>(
+          x, static_cast<const u32x4*>(wt), kt, m, bias, resid, weight, static_cast<bf16*>(rows), sums, more...);
+    };
+    if (rows_each == 16) return go(few_stream_kernel<c.value, 16, 1>, 16, waves);
+    if (few_stream_paired(n, m)) return go(few_stream_half_kernel<c.value>, 8, (waves + 1) / 2, waves);
+    if constexpr (c.value == 0) {
+      // two blocks of tokens in a workgroup where many tokens would have a long k read four times over (896 x 4864 at 64
+      // tokens 10.4 us in one, 9.5; at 32 6.6 in one, 10.0)
+      if (n > 32) return go(few_stream_kernel<0, 8, 2>, 32, waves);
+    }
+    go(few_stream_kernel<c.value, 8, 1>, 16, waves);
   });
   SHK_LAUNCH_CHECK("few_stream");
   return 0;
