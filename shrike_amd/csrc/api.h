@@ -356,6 +356,8 @@ int shk_latent_prompt_bf16(const void* q, void* out, int n, int heads, int key_d
 // a_b = a + b * a_batch (rows lda apart), w_b = w + b * w_batch (contiguous), out_b = out + b *
 // out_batch (rows ldo apart); operands of `dtype`, out of out_dtype (the same or float32), float32
 // accumulation in ascending k.
+// (shk_gemm_batched_lines: whether aligned bfloat16 operands take the kernel for many rows; f32: results of float32.)
+int shk_gemm_batched_lines(int n, int m, int k, int batch, int f32);
 int shk_gemm_batched(const void* a, const void* w, void* out, int n, int m, int k, int lda, int ldo,
                      int batch, long long a_batch, long long w_batch, long long out_batch, int dtype,
                      int out_dtype, void* stream);

@@ -344,7 +344,7 @@ __global__ void __launch_bounds__(WAVES* kWave)
   const int kvh = blockIdx.x, seq = blockIdx.y, z = blockIdx.z;
   // Heads of 128 elements: a lane's own number, with which the compiler keeps to 232 registers, so that two workgroups share a compute unit; with the
   // wavefront's it needs 261.  One workgroup a compute unit and two, 256 sequences of 300 keys: 28 heads over 4 41.3 and 35.8 us, 40 over 8 77.0 and 68.0,
-  // 16 over 16 141 and 126; 64 of 61 to 1,203, which end one by one, 28 over 4 21.9 and 21.8, 40 over 8 38.6 and 40.6; one of 2,048 in eight splits 8.5 and 8.6.
+  // 16 over 16 141 and 126; 64 of 61 to 1,203, which end one by one, 28 over 4 21.9 and 21.8, 40 over 8 38.6 and 40.6; one of 2,048 in eight splits 8.6 and 8.7.
   const int own = threadIdx.x / kWave, wave = D == 128 ? own : __builtin_amdgcn_readfirstlane(own);
   const int lane = threadIdx.x % kWave, j = lane % 16, g = lane / 16;
   const int group = heads / kv_heads;

@@ -265,7 +265,9 @@ __global__ void __launch_bounds__(kWave* RW* CW)
 // everything twice), and results leave through LDS in whole pieces along the rows.  128 rows x 128 features a workgroup, two
 // of which share a compute unit; two stages in LDS, one in flight while the other is multiplied.  The same instructions in the
 // same order of k: the same bits.  28 heads, 1,501 rows, in prompts: k = 128 to 448 features 42.4 us in the kernel above, 26.8 so, k = 448 to
-// 128 features 36.3, 17.3; 14 blocks of 256 to 512 float32 35.7, 19.9.  What bounds it now: the results, 38 to 43 MB but for the second.
+// 128 features 36.3, 17.3; 14 blocks of 256 to 512 float32 35.7, 19.9.  What bounds it now: a workgroup's chain of two to seven stages' latency and four
+// turns of its results through LDS, which only one other workgroup on the compute unit covers; the results alone, 38 to 43 MB but for the second, would
+// take a third to a half of that at a copy's rate.
 constexpr int kLinesK = 64, kLinesRows = 128;
 
 template <typename TO>
@@ -358,9 +360,27 @@ __global__ void __launch_bounds__(4 * kWave)
   }
 }
 
+// The fewest rows of whole lines and pieces for which gemm_batched_lines_kernel is the faster one, where its workgroups fill the compute units: each
+// loads 128 rows and forms 128 features, however few there are, and rounds them all where the results are bfloat16.  Weights cold, us at 1 / 8 / 16 / 17 / 48 /
+// 64 rows in the other kernels and in this one.  256 products of 64 x 128: bfloat16 3.7 / 4.0 / 4.5 / 5.7 / 7.1 / 8.2 and 5.8 / 5.9 / 6.1 / 6.1 / 6.9 / 7.3,
+// float32 3.6 / 4.1 / 4.7 / 4.9 / 6.5 / 7.2 and 4.1 / 4.3 / 4.7 / 4.9 / 6.0 / 6.6; 128 of 128 x 256: 6.0 / 7.1 / 8.1 / 7.5 / 9.0 / 10.1 and 6.9 / 7.0 / 7.1 / 7.1 / 7.8 /
+// 8.3, float32 6.1 / 7.1 / 8.3 / 6.6 / 8.2 / 9.0 and 5.3 / 5.5 / 5.7 / 5.8 / 6.9 / 7.7; 256 of 192 x 128: 6.2 / 7.3 / 8.6 / 9.2 / 10.9 / 12.3 and 7.6 / 7.9 / 8.1 / 8.2 / 9.1 /
+// 9.7; 128 of 512 x 256: 10.1 / 11.3 / 13.1 / 16.9 / 19.1 / 20.8 and 12.9 / 12.9 / 12.9 / 13.0 / 14.3 / 15.1.  With up to 64 features half of it is idle: 256 of 128 x 64 a
+// quarter to a half slower up to 16 rows, 7 % at 17 to 32, 14 % faster from 49 on.
+static int batched_lines_from(int m, int k, bool f32) {
+  if (k < 128 || (m <= 64 && k < 192)) return 49;
+  if (m <= 64) return 17;
+  return f32 && k < 256 ? 1 : (k < 256 ? k : 256) / 16 + 1;
+}
+
+static bool batched_lines(int n, int m, int k, int batch, bool f32) {
+  const long long groups = static_cast<long long>((m + kLinesRows - 1) / kLinesRows) * ((n + kLinesRows - 1) / kLinesRows) * batch;
+  return k % kLinesK == 0 && k <= 1 << 22 && groups >= 256 && n >= batched_lines_from(m, k, f32);
+}
+
 // Shapes: up to 16 rows 16 x 16 a wavefront, side by side along the features (the weights' latency is all
-// there is); 64 x 64 a wavefront where such workgroups fill the compute units, through LDS where k and the results are whole lines and
-// pieces, else 32 x 32.  A k of one or two steps
+// there is); 64 x 64 a wavefront where such workgroups fill the compute units, else 32 x 32; through LDS where batched_lines() says so and k and
+// the results are whole lines and pieces.  A k of one or two steps
 // is loaded a step at a time: eight steps' loads, most of them the last step's again, took 4.1 us for 8 products
 // of 256 x 64 at 16 rows, two 2.4 (3.1 with 64-row workgroups).
 template <typename TO>
@@ -372,9 +392,8 @@ static void launch_batched_mfma(const bf16* a, const bf16* w, TO* out, int n, in
   const bool short_k = k <= 64;
   const int per = 16 / sizeof(TO);  // values of a piece
   // whole stages and whole pieces everywhere, offsets within a workgroup's rows in 32 bits
-  const bool lines = k >= kLinesK && k % kLinesK == 0 && m % per == 0 && ldo % per == 0 && out_batch % per == 0 && w_batch % 8 == 0 &&
-                     reinterpret_cast<uintptr_t>(out) % 16 == 0 && lda <= 1 << 22 && k <= 1 << 22;
-  if (lines && static_cast<long long>(large.x) * large.y * batch >= 256)
+  const bool whole = m % per == 0 && ldo % per == 0 && out_batch % per == 0 && w_batch % 8 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0 && lda <= 1 << 22;
+  if (whole && batched_lines(n, m, k, batch, sizeof(TO) == 4))
     gemm_batched_lines_kernel<TO><<<large, 256, 0, s>>>(a, w, out, n, m, k, lda, ldo, a_batch, w_batch, out_batch);
   else if (n <= 16 && short_k)
     gemm_batched_mfma_kernel<1, 1, 1, 4, 1, TO>
@@ -392,6 +411,9 @@ static void launch_batched_mfma(const bf16* a, const bf16* w, TO* out, int n, in
     gemm_batched_mfma_kernel<2, 2, 2, 2, 2, TO>
         <<<grid(64, 64), 256, 0, s>>>(a, w, out, n, m, k, lda, ldo, vec_out, a_batch, w_batch, out_batch);
 }
+
+// Whether bfloat16 operands in whole lines whose results are whole pieces (`f32`: of float32) go through LDS.
+extern "C" int shk_gemm_batched_lines(int n, int m, int k, int batch, int f32) { return n > 0 && m > 0 && k > 0 && batch > 0 && batched_lines(n, m, k, batch, f32); }
 
 // A batch of products of one shape (one per head, say): product b reads a + b * a_batch
 // (rows lda apart), w + b * w_batch ([m, k] contiguous) and writes out + b * out_batch.

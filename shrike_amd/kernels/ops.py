@@ -969,6 +969,12 @@ def latent_prompt(q, out, heads, key_dim, v_dim, positions, token_seq, tables, p
         _dev(partial, "partial", torch.float32) if nsplit > 1 else None, int(nsplit), int(tokens), _stream()))
 
 
+def gemm_batched_lines(n: int, m: int, k: int, batch: int, f32: bool = False) -> bool:
+    """Whether gemm_batched of n bfloat16 rows runs in the kernel for many of them, where operands and results (`f32`: float32) are
+    16-byte aligned."""
+    return bool(load().shk_gemm_batched_lines(n, m, k, batch, int(f32)))
+
+
 def gemm_batched(a, w, out, batch: int, a_step: int, out_step: int) -> None:
     """out[:, b*out_step : b*out_step + m] = a[:, b*a_step : b*a_step + k] @ w[b].T for b < batch;
     w [batch, m, k] contiguous; a and out 2-d with unit inner stride; all of one dtype, or out float32."""
