@@ -900,6 +900,7 @@ __global__ void __launch_bounds__(16 * kWave)
     leave(stage1, 1);
     if constexpr (NB > 2) {
       leave(stage2, 2);
+      if (n <= 48) return;  // (the same for the whole launch)
       __syncthreads();
       put(stage0, acc[3]);
       __syncthreads();
