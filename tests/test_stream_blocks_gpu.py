@@ -11,4 +11,4 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("n", [34, 47, 48, 49, 63])
 @pytest.mark.parametrize("m, k, form", [(200, 136, "float32"), (1032, 520, "bfloat16"), (200, 136, "gated"), (516, 2056, "shares"), (20004, 72, "float32")])
 def test_the_last_block_of_tokens(m, k, form, n):
-    rows.test_rows_leave_whole(m, k, form, n)
+    rows.test_rows_leave_whole(n=n, m=m, k=k, form=form)
