@@ -74,11 +74,11 @@ struct TileOrder {
 // compute unit, which takes in 130 to 150 from its L2.  Against rectangles for the dies where the numbers divided, and every eighth tile on a
 // die where not, weights cold: 896 x 4864 at 700 / 1,119 / 2,048 tokens 19.0 / 25.1 / 34.3 us -> 15.1 / 19.2 / 28.6, 3584 x 18944 at 512
 // 76.3 -> 73.2, gate and up of 18944 x 3584 at 300 117 -> 102; whole prompts of the 7B sizes at 2,048 tokens 26.6 -> 26.1 ms.
-__device__ __forceinline__ bool big_tile(const TileOrder& t, int& tile_x, int& tile_y, int& share) {
+__host__ __device__ __forceinline__ bool tile_of(const TileOrder& t, unsigned group, int& tile_x, int& tile_y, int& share) {
   const int per_share = t.tiles_x * t.tiles_y;
   const long long all = static_cast<long long>(per_share) * t.shares;
-  const int die = blockIdx.x % kDies;
-  int i = static_cast<int>(all * die / kDies) + blockIdx.x / kDies;
+  const int die = group % kDies;
+  int i = static_cast<int>(all * die / kDies) + group / kDies;
   if (i >= static_cast<int>(all * (die + 1) / kDies)) return false;
   share = t.shares > 1 ? i / per_share : 0;
   i -= share * per_share;
@@ -88,6 +88,10 @@ __device__ __forceinline__ bool big_tile(const TileOrder& t, int& tile_x, int& t
   i -= t.tiles_x * first;
   tile_x = i / high, tile_y = first + i % high;
   return true;
+}
+
+__device__ __forceinline__ bool big_tile(const TileOrder& t, int& tile_x, int& tile_y, int& share) {
+  return tile_of(t, blockIdx.x, tile_x, tile_y, share);
 }
 
 // The grid of the large kernels, and the strips with which the tiles that a die works on at a time (`units`: workgroups on the whole
@@ -102,7 +106,7 @@ inline unsigned big_grid(int tiles_x, int tiles_y, int shares, int tile_rows, in
     const long long rows = static_cast<long long>(wide < tiles_x ? wide : tiles_x) * tile_rows +
                            static_cast<long long>(wide < tiles_x ? high : (at_once + tiles_x - 1) / tiles_x) * tile_tokens;
     if (!least || rows < least) least = rows, order->strips = strips;
-    if (high * high * tile_tokens < tile_rows) break;  // (flatter ones only need more)
+    if (static_cast<long long>(high) * high * tile_tokens < tile_rows) break;  // (flatter ones only need more)
   }
   return static_cast<unsigned>(each * kDies);
 }
