@@ -63,12 +63,12 @@ constexpr int kDieUnits = 32;  // compute units per die
 
 // How the tiles of a large product (tiles_x along the weight rows, tiles_y along the tokens, `shares` of k) are dealt out: in one row,
 // share by share (or, with one row of token tiles, tile by tile), within a share in `strips` runs of neighbouring token tiles, within a strip weight tile by
-// weight tile.
+// weight tile.  in_turn: dies take 32 of them at a time, in turn, else an eighth of the row each.
 struct TileOrder {
-  int tiles_x, tiles_y, shares, strips;
+  int tiles_x, tiles_y, shares, strips, in_turn;
 };
 
-// The tile of a workgroup of the large kernels; false: none (the grid is padded).
+// The tile of workgroup `group` of the large kernels; false: none (the grid is padded).
 // Workgroups are handed to the chip's eight dies (each with its own L2) in turn, workgroup p to die p % 8.  Die d takes the d-th
 // eighth of the row of tiles, in order: what its 32 compute units work on at a time is a run of neighbours that share operands, so that
 // its L2 serves most of their loads, whatever the numbers of tiles.  All dies together draw 10 TB/s from beyond their L2s, 40 GB/s a
@@ -78,9 +78,9 @@ struct TileOrder {
 __host__ __device__ __forceinline__ bool tile_of(const TileOrder& t, unsigned group, int& tile_x, int& tile_y, int& share) {
   const int per_share = t.tiles_x * t.tiles_y;
   const long long all = static_cast<long long>(per_share) * t.shares;
-  const int die = group % kDies;
-  int i = static_cast<int>(all * die / kDies) + group / kDies;
-  if (i >= static_cast<int>(all * (die + 1) / kDies)) return false;
+  const int die = group % kDies, turn = group / kDies;
+  int i = t.in_turn ? (turn / kDieUnits * kDies + die) * kDieUnits + turn % kDieUnits : static_cast<int>(all * die / kDies) + turn;
+  if (i >= static_cast<int>(t.in_turn ? all : all * (die + 1) / kDies)) return false;
   // One row of token tiles: no two tiles of a share have weights in common, and a die that walks one share after the other asks for all of a moment's
   // weights from the same part of every row of tiles.  So a tile's shares follow each other: 4096 x 4096 in four at 65 / 100 / 128 tokens 15.6 /
   // 16.5 / 17.1 us share by share, 14.8 / 15.5 / 16.0 so, 2048 x 4096 10.6 / 10.9 / 11.0 and 10.3 / 10.6 / 10.6.
@@ -103,11 +103,15 @@ __device__ __forceinline__ bool big_tile(const TileOrder& t, int& tile_x, int& t
 }
 
 // The grid of the large kernels, and the strips with which the tiles that a die works on at a time (`units`: workgroups on the whole
-// chip) need the fewest rows of weights and activations.
-inline unsigned big_grid(int tiles_x, int tiles_y, int shares, int tile_rows, int tile_tokens, int units, TileOrder* order) {
+// chip) need the fewest rows of weights and activations.  In turn from four rounds of tiles on with up to 2,048 of k: all dies then work on one strip, and
+// a die meets the same few weight tiles in every strip, which with so short a k stay in its L2.  An eighth each and in turn: 8192 x 1024 at 8,192 / 16,384
+// tokens 131 / 268 us and 125 / 244, 16384 x 1024 at 4,096 / 16,384 130 / 525 and 124 / 486, 9728 x 896 at 16,384 281 and 262; with longer k, gate and up of
+// 18944 x 3584 at 2,048 / 4,096 435 / 862 and 449 / 880.
+inline unsigned big_grid(int tiles_x, int tiles_y, int shares, int tile_rows, int tile_tokens, int k, int units, TileOrder* order) {
   const long long all = static_cast<long long>(tiles_x) * tiles_y * shares, each = (all + kDies - 1) / kDies;
-  const int at_once = static_cast<int>(each < units / kDies ? each : units / kDies);
-  *order = TileOrder{tiles_x, tiles_y, shares, 1};
+  const int in_turn = static_cast<long long>(tiles_x) * tiles_y >= 4 * kDies * kDieUnits && k <= 2048;
+  const int most = in_turn ? kDieUnits : units / kDies, at_once = static_cast<int>(each < most ? each : most);
+  *order = TileOrder{tiles_x, tiles_y, shares, 1, in_turn};
   long long least = 0;
   for (int strips = 1; strips <= tiles_y; ++strips) {
     const int high = (tiles_y + strips - 1) / strips, wide = (at_once + high - 1) / high;
@@ -116,7 +120,7 @@ inline unsigned big_grid(int tiles_x, int tiles_y, int shares, int tile_rows, in
     if (!least || rows < least) least = rows, order->strips = strips;
     if (static_cast<long long>(high) * high * tile_tokens < tile_rows) break;  // (flatter ones only need more)
   }
-  return static_cast<unsigned>(each * kDies);
+  return static_cast<unsigned>((in_turn ? (each + kDieUnits - 1) / kDieUnits * kDieUnits : each) * kDies);
 }
 
 // Weight rows and tokens that the tiles of each die need, summed over the dies, with every eighth tile on a die; 0 where the dies

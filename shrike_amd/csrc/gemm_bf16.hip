@@ -1046,7 +1046,7 @@ static void launch_big(hipStream_t s, const bf16* ap, int lda, int n, int k, con
   constexpr int lds = 2 * (GM * WM + GN * WN) * KS * kWave * 16;
   const int tiles_x = (wblocks + GM * WM - 1) / (GM * WM), tiles_y = (n + 16 * GN * WN - 1) / (16 * GN * WN);
   TileOrder order;
-  const unsigned grid = big_grid(tiles_x, tiles_y, ksplit, 16 * GM * WM, 16 * GN * WN, kDies * kDieUnits, &order);
+  const unsigned grid = big_grid(tiles_x, tiles_y, ksplit, 16 * GM * WM, 16 * GN * WN, k, kDies * kDieUnits, &order);
   if (gated) {
     auto kernel = gemm_big_kernel<GM, GN, WM, WN, KS, true>;
     if (lds > 65536)

@@ -385,7 +385,7 @@ static void launch_wide(hipStream_t s, const bf16* a, int lda, int n, int k, con
   using S = WideShape<GM, GN, RM, RN>;
   const int tiles_x = (wblocks + S::kTiles - 1) / S::kTiles, tiles_y = (n + 32 * GN * RN - 1) / (32 * GN * RN);
   TileOrder order;
-  const unsigned groups = big_grid(tiles_x, tiles_y, ksplit, 16 * S::kTiles, 32 * GN * RN, S::kLds <= 80 * 1024 ? 512 : 256, &order);
+  const unsigned groups = big_grid(tiles_x, tiles_y, ksplit, 16 * S::kTiles, 32 * GN * RN, k, S::kLds <= 80 * 1024 ? 512 : 256, &order);
   const int per = out_f32 ? 4 : 8;  // values of 16 bytes
   const int pieces = ldo % per == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
   const bool rows = pieces && m % per == 0;

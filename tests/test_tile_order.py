@@ -18,9 +18,10 @@ int main() {
   for (int x : xs)
     for (int y : ys)
       for (int shares : {1, 2, 3, 7})
-        for (int units : {256, 512}) {
+        for (int units : {256, 512})
+         for (int k : {1024, 4096}) {
           TileOrder order;
-          const unsigned groups = big_grid(x, y, shares, 256, 128, units, &order);
+          const unsigned groups = big_grid(x, y, shares, 256, 128, k, units, &order);
           std::vector<int> seen(static_cast<size_t>(x) * y * shares, 0);
           for (unsigned g = 0; g < groups; ++g) {
             int tx = -1, ty = -1, share = -1;
@@ -32,9 +33,10 @@ int main() {
             if (times != 1) return printf("%d x %d tiles, %d shares: one is dealt out %d times\n", x, y, shares, times), 1;
         }
   // 32 tiles at a time on a die: of 64 x 2,000 or more they are 6 x 6 or so, not 32 x 1
-  for (int y : {16, 100, 2000, 2897, 3500, 6000, 20000}) {
+  for (int k : {1024, 4096})
+   for (int y : {16, 100, 2000, 2897, 3500, 6000, 20000}) {
     TileOrder order;
-    big_grid(64, y, 1, 256, 256, 256, &order);
+    big_grid(64, y, 1, 256, 256, k, 256, &order);
     const int high = (y + order.strips - 1) / order.strips;
     if (high < 4 || high > 8) return printf("64 x %d tiles in %d strips\n", y, order.strips), 1;
   }
