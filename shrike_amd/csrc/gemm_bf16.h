@@ -123,8 +123,8 @@ inline unsigned big_grid(int tiles_x, int tiles_y, int shares, int tile_rows, in
   return static_cast<unsigned>((in_turn ? (each + kDieUnits - 1) / kDieUnits * kDieUnits : each) * kDies);
 }
 
-// Weight rows and tokens that the tiles of each die need, summed over the dies, with every eighth tile on a die; 0 where the dies
-// can have rectangles of the grid of tiles.  (What wide_fetch() of gemm_wide.hip prices.)
+// Weight rows and tokens that the tiles of each die would need, summed over the dies, with every eighth tile on a die; 0 where the dies could have
+// rectangles of the grid of tiles.  No launch deals tiles out in either way: it is what wide_fetch() of gemm_wide.hip prices, and why is said there.
 inline double big_operands(int tiles_x, int tiles_y, int tile_rows, int tile_tokens) {
   if (static_cast<long long>(tiles_x) * tiles_y >= 4 * kDies * kDieUnits) return 0.0;
   for (int dx = 1; dx <= kDies; dx *= 2)

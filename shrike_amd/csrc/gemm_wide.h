@@ -167,8 +167,8 @@ __device__ __forceinline__ void wide_loop(f32x16 (&acc)[RM][RN], u32x4* mem, con
 // The tiles, and what they were measured to take: a workgroup's start and end, a stage of 64 of k with the chip nearly
 // empty (its loads' latency) and what is added when all its compute units work (the power limit), in us; workgroups that
 // fit on the chip.  From 13 products of 512 to 8,192 tokens in one to three shares: within 15 % of nearly all.  Over 2,568 of 100 to
-// 4,000 tokens, 384 to 5,120 rows and up to eleven shares, weights in cache, 0.71 to 1.29 of the time in nine of ten; most of
-// those below are what wide_fetch() of gemm_wide.hip prices.
+// 4,000 tokens, 384 to 5,120 rows and up to eleven shares, weights in cache, 0.71 to 1.29 of the time in nine of ten.  (Both while tiles were dealt
+// out in another order, see tile_of: products of few shares and many tokens then took up to half as long again.)
 struct WideTile {
   int rows, tokens, units;
   double ends, alone, full;

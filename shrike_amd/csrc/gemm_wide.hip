@@ -288,11 +288,15 @@ __global__ void __launch_bounds__(GM* GN* kWave) __attribute__((amdgpu_waves_per
   }
 }
 
-// The least time that the dies' fetches take, at 7 TB/s, where the tiles' numbers do not divide among the dies: a price of
-// shares that few rows of a long k were given while every eighth tile was a die's (896 x 18944 at 2,048 tokens with its norm: 128 us in
-// three shares of 128 x 192 tiles, which wide_time() alone prefers, 75 in four of 128 x 256).  In runs of neighbours (big_tile) the four
-// take 63 us, three of 128 x 256 77.  With less than 8,192 of k the shares' start and end weigh more (896 x 4864 at 1,119 tokens
-// in a prompt: 25 us in the three shares of 128 x 128 without this, 31 in the two of 128 x 192 that it would take; 19 in runs).
+// A price of few shares of a long k: the least time, at 7 TB/s, of the dies' fetches in an order in which tiles are no longer dealt out (every eighth
+// tile a die's, rectangles where the numbers divide).  In the present order (tile_of) fetches bound none of these sizes, and whether numbers
+// divide changes nothing but this price.  It stays because the choices that it makes are not the worse ones: with the shares that it gives and with those that
+// wide_time() gives alone, product without its reader, 896 x 18944 at 2,048 tokens 4 shares 64.6 us and 3 69.3, at 2,112 5 71.3 and 3 73.7, at 2,752 4
+// 90.4 and 2 93.4, 640 x 18944 at 2,048 6 47.8 and 4 52.3, 1152 x 18944 3 83.6 and 2 96.5, 896 x 9472 4 36.3 and 3 36.6; against it 896 x 18944 at 3,712, two shares
+// in tiles of 256 x 128 123.9 and 128 x 256 112.9, and 2304 x 9472 at 777 2 46.8 and 4 38.6.  The jumps at 3584 x 18944 (one share at 1,700, two at 1,792, one at
+// 1,793: 216, 210, 225 us, 210, 221, 214 with the other number) are wide_time()'s own.  With less than 8,192 of k the shares' start and end weigh more
+// (896 x 4864 at 1,119 tokens in a prompt, in the old order: 25 us in the three shares of 128 x 128 without this, 31 in the two of 128 x 192 that it would take;
+// 19 now).
 static double wide_fetch(const WideTile& t, int n, int wblocks, int k) {
   const int tiles_x = (wblocks * 16 + t.rows - 1) / t.rows, tiles_y = (n + t.tokens - 1) / t.tokens;
   if (tiles_y <= 2 || k < 8192) return 0.0;

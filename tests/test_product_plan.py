@@ -388,12 +388,13 @@ def test_a_deferred_product_is_planned_for_the_rows_that_it_gets(monkeypatch):
 
 
 def test_shares_of_few_rows_and_a_long_k_are_priced_with_what_the_dies_fetch():
-    """Tiles in plain order on the dies, with the reading norm: 896 x 18944 at 2,048 tokens 128 us in three shares of 128 x 192,
-    75 in four of 128 x 256; 640 x 18944 93 in four of 128 x 192, 58; 1152 x 18944 146 in two of 128 x 192, 95."""
+    """The price is that of an order in which every eighth tile was a die's (with the reading norm, 896 x 18944 at 2,048 tokens 128 us in three shares of
+    128 x 192, 75 in four of 128 x 256).  In runs of neighbours, the products alone: 896 x 18944 69 in three and 65 in four, 640 x 18944 52 in four
+    of 128 x 192 and 48 in six, 1152 x 18944 97 in two of 128 x 192 and 84 in three."""
     for n, m, k, old in ((2048, 896, 18944, (3, (128, 192))), (2048, 640, 18944, (4, (128, 192))), (2048, 1152, 18944, (2, (128, 192))),
                          (2048, 896, 9472, (3, (128, 192))), (777, 2304, 9472, (4, (256, 128)))):
         splits = ops.gemm_splits(n, m, k)
         assert (splits, *ops.gemm_tiles(n, m, k, False, splits)) != old, (n, m, k)
-    # tiles that the dies share, one or two rows of them, a shorter k: as without that price
+    # numbers of tiles that divide among the dies, one or two rows of them, a shorter k: as without that price
     assert ops.gemm_splits(512, 3584, 18944) == 3 and ops.gemm_splits(128, 3584, 18944) == 9 and ops.gemm_splits(2048, 3584, 18944) == 1
     assert ops.gemm_splits(1119, 896, 4864) == 3
