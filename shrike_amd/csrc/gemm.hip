@@ -361,12 +361,15 @@ __global__ void __launch_bounds__(4 * kWave)
 }
 
 // The fewest rows of whole lines and pieces for which gemm_batched_lines_kernel is the faster one, where its workgroups fill the compute units: each
-// loads 128 rows and forms 128 features, however few there are, and rounds them all where the results are bfloat16.  Weights cold, us at 1 / 8 / 16 / 17 / 48 /
-// 64 rows in the other kernels and in this one.  256 products of 64 x 128: bfloat16 3.7 / 4.0 / 4.5 / 5.7 / 7.1 / 8.2 and 5.8 / 5.9 / 6.1 / 6.1 / 6.9 / 7.3,
-// float32 3.6 / 4.1 / 4.7 / 4.9 / 6.5 / 7.2 and 4.1 / 4.3 / 4.7 / 4.9 / 6.0 / 6.6; 128 of 128 x 256: 6.0 / 7.1 / 8.1 / 7.5 / 9.0 / 10.1 and 6.9 / 7.0 / 7.1 / 7.1 / 7.8 /
-// 8.3, float32 6.1 / 7.1 / 8.3 / 6.6 / 8.2 / 9.0 and 5.3 / 5.5 / 5.7 / 5.8 / 6.9 / 7.7; 256 of 192 x 128: 6.2 / 7.3 / 8.6 / 9.2 / 10.9 / 12.3 and 7.6 / 7.9 / 8.1 / 8.2 / 9.1 /
-// 9.7; 128 of 512 x 256: 10.1 / 11.3 / 13.1 / 16.9 / 19.1 / 20.8 and 12.9 / 12.9 / 12.9 / 13.0 / 14.3 / 15.1.  With up to 64 features half of it is idle: 256 of 128 x 64 a
-// quarter to a half slower up to 16 rows, 7 % at 17 to 32, 14 % faster from 49 on.
+// loads 128 rows and forms 128 features, however few there are, and rounds them all where the results are bfloat16.  Weights cold, us at 1 / 8 / 16 /
+// 17 / 48 / 64 rows in the other kernels and in this one:
+//   256 of k = 64 to 128 features   bfloat16 3.7 / 4.0 / 4.5 / 5.7 / 7.1 / 8.2 and 5.8 / 5.9 / 6.1 / 6.1 / 6.9 / 7.3,
+//                                   float32 3.6 / 4.1 / 4.7 / 4.9 / 6.5 / 7.2 and 4.1 / 4.3 / 4.7 / 4.9 / 6.0 / 6.6
+//   128 of 128 to 256               bfloat16 6.0 / 7.1 / 8.1 / 7.5 / 9.0 / 10.1 and 6.9 / 7.0 / 7.1 / 7.1 / 7.8 / 8.3,
+//                                   float32 6.1 / 7.1 / 8.3 / 6.6 / 8.2 / 9.0 and 5.3 / 5.5 / 5.7 / 5.8 / 6.9 / 7.7
+//   256 of 192 to 128               bfloat16 6.2 / 7.3 / 8.6 / 9.2 / 10.9 / 12.3 and 7.6 / 7.9 / 8.1 / 8.2 / 9.1 / 9.7
+//   128 of 512 to 256               bfloat16 10.1 / 11.3 / 13.1 / 16.9 / 19.1 / 20.8 and 12.9 / 12.9 / 12.9 / 13.0 / 14.3 / 15.1
+// With up to 64 features half of it is idle: 256 of 128 to 64 a quarter to a half slower up to 16 rows, 7 % at 17 to 32, 14 % faster from 49 on.
 static int batched_lines_from(int m, int k, bool f32) {
   if (k < 128 || (m <= 64 && k < 192)) return 49;
   if (m <= 64) return 17;
@@ -413,7 +416,9 @@ static void launch_batched_mfma(const bf16* a, const bf16* w, TO* out, int n, in
 }
 
 // Whether bfloat16 operands in whole lines whose results are whole pieces (`f32`: of float32) go through LDS.
-extern "C" int shk_gemm_batched_lines(int n, int m, int k, int batch, int f32) { return n > 0 && m > 0 && k > 0 && batch > 0 && batched_lines(n, m, k, batch, f32); }
+extern "C" int shk_gemm_batched_lines(int n, int m, int k, int batch, int f32) {
+  return n > 0 && m > 0 && k > 0 && batch > 0 && batched_lines(n, m, k, batch, f32);
+}
 
 // A batch of products of one shape (one per head, say): product b reads a + b * a_batch
 // (rows lda apart), w + b * w_batch ([m, k] contiguous) and writes out + b * out_batch.
