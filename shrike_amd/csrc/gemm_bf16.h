@@ -90,10 +90,13 @@ __host__ __device__ __forceinline__ bool tile_of(const TileOrder& t, unsigned gr
   }
   share = t.shares > 1 ? i / per_share : 0;
   i -= share * per_share;
-  // strip s holds the token tiles tiles_y * s / strips up to the next one's first
-  const int strip = ((i / t.tiles_x + 1) * t.strips - 1) / t.tiles_y;
-  const int first = t.tiles_y * strip / t.strips, high = t.tiles_y * (strip + 1) / t.strips - first;
-  i -= t.tiles_x * first;
+  int first = 0, high = t.tiles_y;
+  if (t.strips > 1) {  // (its divisions are 0.1 us of a workgroup's start)
+    // strip s holds the token tiles tiles_y * s / strips up to the next one's first
+    const int strip = ((i / t.tiles_x + 1) * t.strips - 1) / t.tiles_y;
+    first = t.tiles_y * strip / t.strips, high = t.tiles_y * (strip + 1) / t.strips - first;
+    i -= t.tiles_x * first;
+  }
   tile_x = i / high, tile_y = first + i % high;
   return true;
 }
