@@ -61,11 +61,28 @@ __device__ __forceinline__ float gate_times_up(float g, float u, int act, const 
 constexpr int kDies = 8;        // accelerator dies (XCDs), each with an L2 of its own
 constexpr int kDieUnits = 32;  // compute units per die
 
+// i / by for i < 2^31 and a number `by` that the host knows: the upper half of a product, exact since times exceeds 2^(31 + shift) / by by less
+// than one and 2^shift is at least `by`.  (A division by a number known at run time only is a chain of some 25 instructions.)
+struct Divisor {
+  unsigned times, shift;
+};
+inline Divisor divisor(unsigned by) {
+  unsigned shift = 0;
+  while (1ull << shift < by) ++shift;
+  return Divisor{static_cast<unsigned>(((1ull << (31 + shift)) + by - 1) / by), shift};
+}
+__host__ __device__ __forceinline__ int divided(int i, const Divisor& d) {
+  return static_cast<int>(static_cast<unsigned>(static_cast<unsigned long long>(2u * static_cast<unsigned>(i)) * d.times >> 32) >> d.shift);
+}
+
 // How the tiles of a large product (tiles_x along the weight rows, tiles_y along the tokens, `shares` of k) are dealt out: in one row,
-// share by share (or, with one row of token tiles, tile by tile), within a share in `strips` runs of neighbouring token tiles, within a strip weight tile by
-// weight tile.  in_turn: dies take 32 of them at a time, in turn, else an eighth of the row each.
+// share by share (or, with one row of token tiles, tile by tile), within a share in `strips` runs of neighbouring token tiles, the taller ones first, within a
+// strip weight tile by weight tile.  in_turn: dies take 32 of them at a time, in turn, else an eighth of the row each.
 struct TileOrder {
   int tiles_x, tiles_y, shares, strips, in_turn;
+  // Tiles of all shares and of one; token tiles (with one row of them: shares) of a low strip, of all taller ones, and those ones' tiles.
+  int all, each, low, tall_rows, tall_tiles;
+  Divisor by_each, by_strip[2], by_high[2];  // (of low strips and of taller ones)
 };
 
 // The tile of workgroup `group` of the large kernels; false: none (the grid is padded).
@@ -75,29 +92,26 @@ struct TileOrder {
 // compute unit, which takes in 130 to 150 from its L2.  Against rectangles for the dies where the numbers divided, and every eighth tile on a
 // die where not, weights cold: 896 x 4864 at 700 / 1,119 / 2,048 tokens 19.0 / 25.1 / 34.3 us -> 15.1 / 19.2 / 28.6, 3584 x 18944 at 512
 // 76.3 -> 73.2, gate and up of 18944 x 3584 at 300 117 -> 102; whole prompts of the 7B sizes at 2,048 tokens 26.6 -> 26.1 ms.
+// Nothing of a workgroup can begin before this is known, so it holds no divisions and nothing to branch on but the padding: 896 x 896 at 777 / 1,119 /
+// 2,048 tokens 8.8 / 8.8 / 9.0 us with both, 8.5 / 8.5 / 8.7 so, 4096 10.4 and 9.9; 1152 x 896 at 512 8.7 and 8.4; 896 x 4864 at 1,119 16.3 and 15.9.
+// One row of token tiles: no two tiles of a share have weights in common, and a die that walks one share after the other asks for all of a moment's
+// weights from the same part of every row of tiles.  So a tile's shares follow each other, as its token tiles would: 4096 x 4096 in four at 65 / 100 / 128
+// tokens 15.6 / 16.5 / 17.1 us share by share, 14.8 / 15.5 / 16.0 so, 2048 x 4096 10.6 / 10.9 / 11.0 and 10.3 / 10.6 / 10.6.
 __host__ __device__ __forceinline__ bool tile_of(const TileOrder& t, unsigned group, int& tile_x, int& tile_y, int& share) {
-  const int per_share = t.tiles_x * t.tiles_y;
-  const long long all = static_cast<long long>(per_share) * t.shares;
   const int die = group % kDies, turn = group / kDies;
-  int i = t.in_turn ? (turn / kDieUnits * kDies + die) * kDieUnits + turn % kDieUnits : static_cast<int>(all * die / kDies) + turn;
-  if (i >= static_cast<int>(t.in_turn ? all : all * (die + 1) / kDies)) return false;
-  // One row of token tiles: no two tiles of a share have weights in common, and a die that walks one share after the other asks for all of a moment's
-  // weights from the same part of every row of tiles.  So a tile's shares follow each other: 4096 x 4096 in four at 65 / 100 / 128 tokens 15.6 /
-  // 16.5 / 17.1 us share by share, 14.8 / 15.5 / 16.0 so, 2048 x 4096 10.6 / 10.9 / 11.0 and 10.3 / 10.6 / 10.6.
-  if (t.tiles_y == 1) {
-    share = i % t.shares, tile_x = i / t.shares, tile_y = 0;
-    return true;
-  }
-  share = t.shares > 1 ? i / per_share : 0;
-  i -= share * per_share;
-  int first = 0, high = t.tiles_y;
-  if (t.strips > 1) {  // (its divisions are 0.1 us of a workgroup's start)
-    // strip s holds the token tiles tiles_y * s / strips up to the next one's first
-    const int strip = ((i / t.tiles_x + 1) * t.strips - 1) / t.tiles_y;
-    first = t.tiles_y * strip / t.strips, high = t.tiles_y * (strip + 1) / t.strips - first;
-    i -= t.tiles_x * first;
-  }
-  tile_x = i / high, tile_y = first + i % high;
+  const int eighth = static_cast<unsigned>(t.all) / kDies, over = static_cast<unsigned>(t.all) % kDies;
+  const int begin = eighth * die + over * die / kDies, end = eighth * (die + 1) + over * (die + 1) / kDies;
+  int i = t.in_turn ? (turn / kDieUnits * kDies + die) * kDieUnits + turn % kDieUnits : begin + turn;
+  if (i >= (t.in_turn ? t.all : end)) return false;
+  share = divided(i, t.by_each);
+  i -= share * t.each;
+  const bool tall = i < t.tall_tiles;
+  i -= tall ? 0 : t.tall_tiles;
+  const int high = t.low + tall, strip = divided(i, tall ? t.by_strip[1] : t.by_strip[0]);
+  i -= strip * high * t.tiles_x;
+  tile_x = divided(i, tall ? t.by_high[1] : t.by_high[0]);
+  tile_y = (tall ? 0 : t.tall_rows) + strip * high + i - tile_x * high;
+  if (t.tiles_y == 1) share = tile_y, tile_y = 0;
   return true;
 }
 
@@ -114,15 +128,18 @@ inline unsigned big_grid(int tiles_x, int tiles_y, int shares, int tile_rows, in
   const long long all = static_cast<long long>(tiles_x) * tiles_y * shares, each = (all + kDies - 1) / kDies;
   const int in_turn = static_cast<long long>(tiles_x) * tiles_y >= 4 * kDies * kDieUnits && k <= 2048;
   const int most = in_turn ? kDieUnits : units / kDies, at_once = static_cast<int>(each < most ? each : most);
-  *order = TileOrder{tiles_x, tiles_y, shares, 1, in_turn};
+  int best = 1;
   long long least = 0;
   for (int strips = 1; strips <= tiles_y; ++strips) {
     const int high = (tiles_y + strips - 1) / strips, wide = (at_once + high - 1) / high;
     const long long rows = static_cast<long long>(wide < tiles_x ? wide : tiles_x) * tile_rows +
                            static_cast<long long>(wide < tiles_x ? high : (at_once + tiles_x - 1) / tiles_x) * tile_tokens;
-    if (!least || rows < least) least = rows, order->strips = strips;
+    if (!least || rows < least) least = rows, best = strips;
     if (static_cast<long long>(high) * high * tile_tokens < tile_rows) break;  // (flatter ones only need more)
   }
+  const int rows = tiles_y > 1 ? tiles_y : shares, low = rows / best, tall = rows % best;  // (tall: how many strips are taller)
+  *order = TileOrder{tiles_x, tiles_y, shares, best, in_turn, static_cast<int>(all), tiles_x * rows, low, tall * (low + 1), tall * (low + 1) * tiles_x,
+                     divisor(tiles_x * rows), {divisor(tiles_x * low), divisor(tiles_x * (low + 1))}, {divisor(low), divisor(low + 1)}};
   return static_cast<unsigned>((in_turn ? (each + kDieUnits - 1) / kDieUnits * kDieUnits : each) * kDies);
 }
 

@@ -14,6 +14,17 @@ PROGRAM = r"""
 using namespace shk;
 
 int main() {
+  // divisions by numbers that the host knows, on both sides of every multiple near either end
+  for (unsigned by = 1; by < 70000; by += by < 300 ? 1 : by / 7) {
+    const Divisor d = divisor(by);
+    for (long long base : {0ll, 65536ll, (1ll << 31) - 1 - 5ll * by})
+      for (int m = 0; m < 5; ++m)
+        for (int off = -1; off <= 1; ++off) {
+          const long long i = (base / by + m) * by + off;
+          if (i >= 0 && i < 1ll << 31 && divided(static_cast<int>(i), d) != i / by) return printf("%lld / %u\n", i, by), 1;
+        }
+    if (divided(2147483647, d) != 2147483647 / static_cast<int>(by)) return printf("the last / %u\n", by), 1;
+  }
   const int xs[] = {1, 2, 3, 7, 8, 14, 56, 297}, ys[] = {1, 2, 5, 8, 9, 16, 33, 100};
   for (int x : xs)
     for (int y : ys)
