@@ -94,10 +94,9 @@ __device__ __forceinline__ float few_sum(const f32x4* red, int stride, int row, 
   return v;
 }
 
-// Wavefronts that share k (or walks, where a wavefront takes two; the figures are with one each): where four to eight of them hold all their tiles at
-// once, the number that holds the fewest
-// beyond k, else four or five.  Few, because each more is another sum to add at the end: 896 x 896 with one token 2.97 us in 4,
-// 3.10 in 7, 3.21 in 15; 3584 x 18944 at 1 / 8 / 16 tokens 22.2 / 23.2 / 27.0 in 4, 22.0 / 24.1 / 28.4 in 5, 23.1 / 24.5 / 27.8
+// Wavefronts that share k (or walks of it, where a wavefront takes two; the figures are with one each): where four to eight of them hold
+// all their tiles at once, the number that holds the fewest beyond k, else four or five.  Few, because each more is another sum to add
+// at the end: 896 x 896 with one token 2.97 us in 4, 3.10 in 7, 3.21 in 15; 3584 x 18944 at 1 / 8 / 16 tokens 22.2 / 23.2 / 27.0 in 4, 22.0 / 24.1 / 28.4 in 5, 23.1 / 24.5 / 27.8
 // in 16; 1536 x 8960, whose 280 tiles five share without loads beyond k, 9.7 / 9.8 / 10.6 in 4 and 9.0 / 9.2 / 11.0 in 5.
 // (Whatever the tokens: a row's bits do not depend on those beside it.)
 inline int few_waves(int ktiles, int most) {
